@@ -141,6 +141,10 @@ typedef struct {
 } infllm_attn_args;
 int infllm_attn_stage(const infllm_attn_args *a, void *stream);
 
+/* How many key splits a stage's argument block is best cut into (its nsplit and partial buffers are not read): the number
+ * for which an estimate of rounds of workgroups, tiles per workgroup and the merge is smallest, 1..max_splits; < 0 on error. */
+int infllm_attn_stage_splits(const infllm_attn_args *a, int32_t max_splits);
+
 /* Joint softmax across stages/splits (torch_impl.py:15-36):
  * o = sum_p 2^(lse_p - LSE) o_p, LSE = log2 sum_p 2^lse_p.
  * d_o_part fp16 [P,B,H,Lq,128], d_lse_part [P,B,H,Lq] -> d_out bf16 [B,H,Lq,128]
@@ -150,6 +154,10 @@ int infllm_attn_merge(const uint16_t *d_o_part, const float *d_lse_part, int32_t
                       int32_t B, int32_t H, int32_t Lq,
                       void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
                       float *d_lse, void *stream);
+/* The same over two sets of partials in buffers of their own (P2 = 0: the first alone). */
+int infllm_attn_merge_pair(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2, const float *d_lse_part2,
+                           int32_t P2, int32_t B, int32_t H, int32_t Lq, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse,
+                           void *stream);
 /* The operator's whole forward in one call (attn.append(local...), attn.append(global..., end=True),
  * attn.get_result(): context_manager.py:486-489, 526-533): the local stage over a ring or tensor, the global
  * stage over a page table (either may be NULL), and their merge into d_out / d_lse.  The stages keep their own
@@ -181,6 +189,51 @@ int infllm_attn_stages_fused(const infllm_attn_args *local, const infllm_attn_ar
 #define INFLLM_NOALLOC_MAX_PART_ROWS 65536
 int infllm_attn_fwd_noalloc(const infllm_attn_args *local, const infllm_attn_args *global,
                             void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse, void *stream);
+
+/* ---------------------------------------------------------------------------
+ * One call of an attention type that keeps a plain cache: attention sinks + sliding window (stream_llm.py:6-111,
+ * infinite_lm.py:6-100) or causal attention over everything (origin.py:4-79).  From the projections' rows to the
+ * output rows: rotary embedding of the new queries and keys at their stream positions, the new cache, both stages of
+ * the attention under one softmax, the output in the caller's layout.
+ *
+ * kind: 0 causal (no sinks), 1 sinks rotated at their own positions ("stream-llm"), 2 sinks un-rotated at one distance
+ * ("infinite-lm").  The cache holds rotated keys and values as rows of `dim` elements, row stride dim, any batch and head
+ * strides (multiples of 8): rows_old rows before the call (all tokens, or n_init sinks followed by the tail) and
+ * rows_new after it (old rows [0, n_init) and the last rows_new - n_init of all rows when the cache is cut; otherwise all
+ * of them).  d_cache_k == d_old_k with the same strides continues the cache in place: the rows that are there stay, the
+ * new ones are written behind them.
+ * d_all_k / d_all_v: room for rows_old + n_new rows [B, Hkv, .., dim] that the attention reads, when the cut cache does not
+ * hold every key the call sees (n_q > 1 and the cache is cut); else NULL, and the attention reads the new cache.
+ * d_raw: the un-rotated sinks (kind 2): raw_old of them in d_raw_old [B, Hkv, raw_old, dim], raw_new in d_raw (the same
+ * pointer and counts when nothing is added).
+ * d_work: scratch, work_bytes long: 2 * B * H * n_q * dim bf16 for the rotated queries (once for kind 0), the rest, if any, for
+ * partial rows (more of it allows more key splits, up to 64 * B * H * n_q rows of 2 * dim + 4 bytes). */
+typedef struct {
+    const void *d_q, *d_k, *d_v;            /* [B,H,n_q,dim], [B,Hkv,n_new,dim] */
+    int64_t q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;
+    int32_t B, H, Hkv, dim;                 /* dim 64 or 128 */
+    int32_t n_q, n_new, kind, n_init;
+    int64_t n_local;
+    int64_t seen;                           /* tokens before this call */
+    const float *d_inv_freq;                /* [dim / 2] */
+    double distance_scale;
+    const void *d_old_k, *d_old_v;
+    int64_t ok_sb, ok_sh, ov_sb, ov_sh;
+    void *d_cache_k, *d_cache_v;
+    int64_t ck_sb, ck_sh, cv_sb, cv_sh;
+    int32_t rows_old, rows_new;
+    void *d_all_k, *d_all_v;
+    const void *d_raw_old;
+    void *d_raw;
+    int32_t raw_old, raw_new;
+    void *d_work;
+    int64_t work_bytes;
+    void *d_out;                            /* bf16 rows [b, h, i] at b*o_sb + h*o_sh + i*o_sl */
+    int64_t o_sb, o_sh, o_sl;
+    float softmax_scale;                    /* 1/sqrt(dim) of the model (dim itself may be a wider row) */
+    int32_t reserved;
+} infllm_window_args;
+int infllm_window_forward(const infllm_window_args *a, void *stream);
 
 /* ---------------------------------------------------------------------------
  * Column sums of the final probabilities of one linear stage

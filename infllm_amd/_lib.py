@@ -60,6 +60,24 @@ class ScoreArgs(C.Structure):
     ]
 
 
+class WindowArgs(C.Structure):
+    _fields_ = [
+        ("d_q", c_vp), ("d_k", c_vp), ("d_v", c_vp),
+        ("q_sb", c_i64), ("q_sh", c_i64), ("q_sl", c_i64), ("k_sb", c_i64), ("k_sh", c_i64), ("k_sl", c_i64),
+        ("v_sb", c_i64), ("v_sh", c_i64), ("v_sl", c_i64),
+        ("B", c_i32), ("H", c_i32), ("Hkv", c_i32), ("dim", c_i32),
+        ("n_q", c_i32), ("n_new", c_i32), ("kind", c_i32), ("n_init", c_i32),
+        ("n_local", c_i64), ("seen", c_i64),
+        ("d_inv_freq", c_vp), ("distance_scale", c_f64),
+        ("d_old_k", c_vp), ("d_old_v", c_vp), ("ok_sb", c_i64), ("ok_sh", c_i64), ("ov_sb", c_i64), ("ov_sh", c_i64),
+        ("d_cache_k", c_vp), ("d_cache_v", c_vp), ("ck_sb", c_i64), ("ck_sh", c_i64), ("cv_sb", c_i64), ("cv_sh", c_i64),
+        ("rows_old", c_i32), ("rows_new", c_i32),
+        ("d_all_k", c_vp), ("d_all_v", c_vp), ("d_raw_old", c_vp), ("d_raw", c_vp), ("raw_old", c_i32), ("raw_new", c_i32),
+        ("d_work", c_vp), ("work_bytes", c_i64), ("d_out", c_vp), ("o_sb", c_i64), ("o_sh", c_i64), ("o_sl", c_i64),
+        ("softmax_scale", c_f32), ("reserved", c_i32),
+    ]
+
+
 class LayerDesc(C.Structure):
     _fields_ = [
         ("B", c_i32), ("H", c_i32), ("Hkv", c_i32),
@@ -139,9 +157,12 @@ SYMBOLS = {
     "infllm_rope_rows": (c_i32, [c_vp, c_i64, c_i64, c_i64, c_i32, c_i32, c_i32, c_i64, c_i32, c_vp, C.c_double, c_vp, c_vp]),
     "infllm_attn_stage": (c_i32, [C.POINTER(AttnArgs), c_vp]),
     "infllm_attn_merge": (c_i32, [c_vp, c_vp, c_i32, c_i32, c_i32, c_i32, c_vp, c_i64, c_i64, c_i64, c_vp, c_vp]),
+    "infllm_attn_stage_splits": (c_i32, [C.POINTER(AttnArgs), c_i32]),
+    "infllm_attn_merge_pair": (c_i32, [c_vp, c_vp, c_i32, c_vp, c_vp, c_i32, c_i32, c_i32, c_i32, c_vp, c_i64, c_i64, c_i64, c_vp, c_vp]),
     "infllm_attn_fwd": (c_i32, [C.POINTER(AttnArgs), C.POINTER(AttnArgs), c_vp, c_i64, c_i64, c_i64, c_vp, c_vp]),
     "infllm_attn_stages_fused": (c_i32, [C.POINTER(AttnArgs), C.POINTER(AttnArgs), c_vp]),
     "infllm_attn_fwd_noalloc": (c_i32, [C.POINTER(AttnArgs), C.POINTER(AttnArgs), c_vp, c_i64, c_i64, c_i64, c_vp, c_vp]),
+    "infllm_window_forward": (c_i32, [c_vp, c_vp]),      # infllm_window_args: WindowArgs by reference, or its bytes
     "infllm_local_score": (c_i32, [C.POINTER(ScoreArgs), c_vp]),
     "infllm_unit_scores": (c_i32, [c_vp, c_i64, c_i32, c_i32, c_i32, c_vp, c_vp, c_vp]),
     "infllm_topk": (c_i32, [c_vp, c_i32, c_i32, c_vp, c_vp]),

@@ -1,6 +1,6 @@
 """Shared body of the attention types that keep attention sinks plus a sliding window
 ("stream-llm", "infinite-lm": inf_llm/attention/stream_llm.py:6-111, infinite_lm.py:6-100) and of
-plain causal attention ("origin": origin.py:4-79), on the multi-stage HIP operator.
+plain causal attention ("origin": origin.py:4-79): one native call per layer call (infllm_window_forward).
 
 The reference re-rotates the whole cached window on every call (positions relative to the window).
 Here every key is rotated once, at its absolute stream position, when it arrives, and the cache keeps
@@ -13,121 +13,176 @@ tables produce.  The sink stage uses one fixed query angle:
 A sink key j is visible to the query at stream position p in that stage iff p - j >= n_local (otherwise it
 is still inside the window and the local stage sees it).  The cache tuple keeps the reference's first three
 fields (keys, values, tokens seen); a fourth holds the un-rotated sink keys when the type needs them.
+
+A cache that still holds every token grows in place: its tensors are the filled part of buffers with room behind it
+(a quarter more), and the next call writes its rows there instead of copying everything - when the cache it is given is
+the newest one of those buffers.  An older one (a second continuation of the same prompt) gets buffers of its own.
 """
+import math
+import struct
+import threading
+
 import torch
 
-from .. import ops
+from .. import _lib
+from ..ops import HEAD_DIM, _stream
 from ._rows import check_head_dim, narrow, wide_inv_freq, widen
-from .dot_production_attention import get_multi_stage_dot_production_attention
+
+_KINDS = {"origin": 0, "stream-llm": 1, "infinite-lm": 2}
+_ARGS = struct.Struct("@3P9q8i2qPd2P4q2P4q2i4P2iPqP3qf4x")        # infllm_window_args
+_SPLIT_ROWS = 131072                # partial rows that key splits of a call of several queries may take
+
+
+class _Room:
+    """Buffers [B, Hkv, capacity, dim] of which the first `used` rows are a cache."""
+    __slots__ = ("k", "v", "used", "lock")
+
+    def __init__(self, k, v, used):
+        self.k, self.v, self.used, self.lock = k, v, used, threading.Lock()
+
+    def claim(self, past_k, past_v, n_new):
+        """Whether this call may write the n_new rows behind the given cache."""
+        rows = past_k.size(2)
+        if (past_k.data_ptr() != self.k.data_ptr() or past_v.data_ptr() != self.v.data_ptr() or past_k.stride() != self.k.stride()
+                or past_v.stride() != self.v.stride() or past_k.shape[:2] != self.k.shape[:2] or rows + n_new > self.k.size(2)):
+            return False
+        with self.lock:
+            if self.used != rows:                              # another call went on from this cache already
+                return False
+            self.used = rows + n_new
+        return True
+
+
+def _rows16(t):
+    """rows the kernels can read: unit stride inside a row, 16-byte alignment"""
+    s = t.stride()
+    return t if s[-1] == 1 and not any(x % 8 for x in s[:-1]) and t.data_ptr() % 16 == 0 else t.contiguous()
+
+
+def _cache_rows(t):
+    """a cached tensor as the native call takes it: rows next to each other"""
+    t = _rows16(t)
+    return t if t.stride(2) == t.size(3) else t.contiguous()
 
 
 def _heads(x, batch, length, heads, dim):
-    return x.view(batch, length, heads, dim).permute(0, 2, 1, 3)
+    """(tensor that is kept alive, batch, head and row strides) of projected rows [batch, length, heads * dim]"""
+    if x.dim() != 3 or x.size(2) != heads * dim:
+        x = x.view(batch, length, heads * dim)
+    x = _rows16(x)
+    return x, x.stride(0), dim, x.stride(1)
 
 
-def _rope_args(position_bias, device):
-    return wide_inv_freq(position_bias.inv_freq, device), float(position_bias.distance_scale)
+def _wide_heads(x, batch, length, heads, dim):
+    x = widen(x.view(batch, length, heads, dim), dim)
+    return x, x.stride(0), x.stride(2), x.stride(1)
 
 
-def _rope(x, inv_freq, scale, pos0, consecutive=True):
-    """rows rotated at pos0 + r (or all at pos0); narrower heads take the way through a 128-wide row"""
-    d = x.shape[-1]
-    if d == ops.HEAD_DIM:
-        return ops.rope_rows(x, inv_freq, scale, pos0, consecutive)
-    check_head_dim(d)
-    return narrow(ops.rope_rows(widen(x, d), inv_freq, scale, pos0, consecutive), d).contiguous()
+def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_q, project_k, project_v, dim_head, num_heads, num_heads_kv):
+    """Output rows [batch, len_q, heads * dim] and the new (keys, values, tokens seen, un-rotated sinks)."""
+    batch, len_q, n_new = query.size(0), query.size(1), key_value.size(1)
+    xq, xk, xv = project_q(query), project_k(key_value), project_v(key_value)
+    for x in (xq, xk, xv):
+        if x.dtype != torch.bfloat16:
+            raise TypeError(f"the HIP attention path computes in bfloat16, got {x.dtype}")
+    check_head_dim(dim_head)
+    dev = xq.device
+    native = dim_head in (64, HEAD_DIM)                        # other widths travel in rows of 128
+    dim = dim_head if native else HEAD_DIM
+    split = _heads if native else _wide_heads
+    q, q_sb, q_sh, q_sl = split(xq, batch, len_q, num_heads, dim_head)
+    k, k_sb, k_sh, k_sl = split(xk, batch, n_new, num_heads_kv, dim_head)
+    v, v_sb, v_sh, v_sl = split(xv, batch, n_new, num_heads_kv, dim_head)
+    inv_freq = position_bias.inv_freq
+    if inv_freq.device != dev or inv_freq.dtype != torch.float32 or inv_freq.numel() != dim // 2 or not inv_freq.is_contiguous():
+        inv_freq = inv_freq.to(device=dev, dtype=torch.float32).contiguous() if native else wide_inv_freq(inv_freq, dev)
+    if inv_freq.numel() != dim // 2:
+        raise ValueError(f"the rotary embedding is built for head_dim {2 * position_bias.inv_freq.numel()}, the heads have {dim_head}")
+
+    old_k = old_v = raw_old = None
+    seen = rows_old = raw_rows = 0
+    if past is not None:
+        old_k, old_v, seen, raw_old = past
+        rows_old = old_k.size(2)
+        if native:
+            cached_k, cached_v = _cache_rows(old_k), _cache_rows(old_v)
+        else:
+            cached_k, cached_v = widen(old_k, dim_head).contiguous(), widen(old_v, dim_head).contiguous()
+            raw_old = None if raw_old is None else widen(raw_old, dim_head)
+        if raw_old is not None:
+            raw_old = raw_old.contiguous()
+            raw_rows = raw_old.size(2)
+    rows_all, len_k = rows_old + n_new, seen + n_new
+    bf = dict(dtype=torch.bfloat16, device=dev)
+    cut = kind and len_k > n_local + n_init and rows_all > n_local + n_init
+    raw, raw_new = raw_old, raw_rows
+    if kind == 2 and raw_rows < n_init and seen == raw_rows:   # un-rotated copies of the first n_init keys
+        raw_new = min(n_init, len_k)
+        raw = torch.empty((batch, num_heads_kv, raw_new, dim), **bf)
+    all_kv = None
+    if cut:
+        rows_new = n_init + n_local
+        cache = torch.empty((2, batch, num_heads_kv, rows_new, dim), **bf)
+        new_k, new_v = buf_k, buf_v = cache.unbind(0)
+        if len_q > 1 or n_new > 1:
+            all_kv = torch.empty((2, batch, num_heads_kv, rows_all, dim), **bf)
+    else:
+        rows_new = rows_all
+        room = getattr(old_k, "_infllm_room", None) if past is not None and native else None
+        if room is None or not room.claim(old_k, old_v, n_new):
+            cap = rows_all + max(256, rows_all // 4)
+            if kind:
+                cap = max(rows_all, min(cap, n_local + n_init))
+            both = torch.empty((2, batch, num_heads_kv, cap, dim), **bf)
+            room = _Room(both[0], both[1], rows_all)
+        buf_k, buf_v = room.k, room.v
+        new_k, new_v = buf_k.narrow(2, 0, rows_all), buf_v.narrow(2, 0, rows_all)
+        new_k._infllm_room = room
+
+    rows_q = batch * num_heads * len_q
+    q_bytes = (2 if kind else 1) * rows_q * dim * 2
+    part_rows = 64 * rows_q if rows_q <= 2048 else _SPLIT_ROWS if 2 * rows_q <= _SPLIT_ROWS else 0
+    work = torch.empty((q_bytes + part_rows * (2 * dim + 4),), dtype=torch.uint8, device=dev)
+    out = torch.empty((batch, len_q, num_heads * dim), **bf)
+    okp = ovp = 0
+    ok_sb = ok_sh = ov_sb = ov_sh = 0
+    if rows_old:
+        okp, ovp = cached_k.data_ptr(), cached_v.data_ptr()
+        ok_sb, ok_sh, ov_sb, ov_sh = cached_k.stride(0), cached_k.stride(1), cached_v.stride(0), cached_v.stride(1)
+    args = _ARGS.pack(q.data_ptr(), k.data_ptr(), v.data_ptr(), q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl, batch, num_heads, num_heads_kv, dim,
+                      len_q, n_new, kind, n_init, n_local, seen, inv_freq.data_ptr(), float(position_bias.distance_scale), okp, ovp, ok_sb, ok_sh, ov_sb,
+                      ov_sh, buf_k.data_ptr(), buf_v.data_ptr(), buf_k.stride(0), buf_k.stride(1), buf_v.stride(0), buf_v.stride(1), rows_old, rows_new,
+                      all_kv[0].data_ptr() if all_kv is not None else 0, all_kv[1].data_ptr() if all_kv is not None else 0,
+                      raw_old.data_ptr() if raw_old is not None else 0, raw.data_ptr() if raw is not None else 0, raw_rows, raw_new, work.data_ptr(),
+                      work.numel(), out.data_ptr(), out.stride(0), dim, out.stride(1), 1.0 / math.sqrt(dim_head))
+    _lib.check(_lib.load().infllm_window_forward(args, _stream()), "infllm_window_forward")
+    if not native:
+        out = narrow(out.view(batch, len_q, num_heads, dim), dim_head).reshape(batch, len_q, num_heads * dim_head)
+        new_k, new_v = narrow(new_k, dim_head), narrow(new_v, dim_head)
+        raw = None if raw is None else narrow(raw, dim_head)
+    return out, (new_k, new_v, len_k, raw)
 
 
 def sink_window_forward(kind, n_local, n_init, fattn=False):
     assert kind in ("stream-llm", "infinite-lm")
-    Attn, _ = get_multi_stage_dot_production_attention(fattn)
-    sink_query_pos = n_local - 1 if kind == "infinite-lm" else n_local + n_init - 1
-    raw_sinks = kind == "infinite-lm"
+    code = _KINDS[kind]
 
     def forward(self, query, key_value, position_bias, use_cache, past_key_value, project_q, project_k, project_v,
                 attention_out, dim_head, num_heads, num_heads_kv):
-        batch, len_q, len_new = query.size(0), query.size(1), key_value.size(1)
-        q = _heads(project_q(query), batch, len_q, num_heads, dim_head)
-        k = _heads(project_k(key_value), batch, len_new, num_heads_kv, dim_head)
-        v = _heads(project_v(key_value), batch, len_new, num_heads_kv, dim_head)
-        if q.dtype != torch.bfloat16:
-            raise TypeError(f"the HIP attention path computes in bfloat16, got {q.dtype}")
-        inv_freq, scale = _rope_args(position_bias, q.device)
-
-        seen = past_key_value[2] if past_key_value is not None else 0
-        len_k = seen + len_new
-        q_loc = _rope(q, inv_freq, scale, len_k - len_q)
-        k_rot = _rope(k, inv_freq, scale, seen)
-        v_all = v
-        sinks = None
-        if past_key_value is not None:
-            k_rot = torch.cat((past_key_value[0], k_rot), dim=2)
-            v_all = torch.cat((past_key_value[1], v), dim=2)
-            sinks = past_key_value[3]
-        if raw_sinks:                                       # un-rotated copies of the first n_init keys
-            have = 0 if sinks is None else sinks.size(2)
-            if have < n_init and seen == have:
-                fresh = k[:, :, :n_init - have]
-                sinks = fresh.contiguous() if sinks is None else torch.cat((sinks, fresh), dim=2)
-
-        rows = k_rot.size(2)                                # all tokens, or n_init sinks followed by the tail
-        if use_cache:
-            if len_k <= n_local + n_init:
-                cache = (k_rot, v_all, len_k, sinks)
-            else:
-                cut = max(0, rows - n_local)
-                cache = (torch.cat((k_rot[:, :, :n_init], k_rot[:, :, cut:]), dim=2),
-                         torch.cat((v_all[:, :, :n_init], v_all[:, :, cut:]), dim=2), len_k, sinks)
-        else:
-            cache = None
-
-        first = max(0, rows - len_q - n_local)              # the local stage never needs more than this tail
-        attn = Attn(q_loc.shape, q_loc.dtype, q_loc.device)
-        attn.append(q_loc, k_rot[:, :, first:], v_all[:, :, first:], sliding_window=n_local)
-        if len_k > n_local:
-            q_sink = _rope(q, inv_freq, scale, sink_query_pos, consecutive=False)
-            k_sink = sinks if raw_sinks and sinks is not None else k_rot[:, :, :n_init]
-            v_sink = v_all[:, :, :n_init]
-        else:
-            q_sink = q.contiguous()
-            k_sink = k_rot[:, :, :0]
-            v_sink = v_all[:, :, :0]
-        attn.append(q_sink, k_sink, v_sink, end=True, sliding_window=(len_k - len_q, n_local),
-                    complement_sliding_window=True)
-        o, _ = attn.get_result()
-
-        o = o.view(batch, num_heads, len_q, dim_head).permute(0, 2, 1, 3).reshape(batch, len_q, num_heads * dim_head)
-        o = attention_out(o)
-        return (o, cache) if use_cache else o
+        out, cache = _call(code, n_local, n_init, query, key_value, position_bias, past_key_value, project_q, project_k, project_v, dim_head, num_heads,
+                           num_heads_kv)
+        out = attention_out(out)
+        return (out, cache) if use_cache else out
 
     return forward
 
 
 def causal_forward(fattn=False):
-    Attn, _ = get_multi_stage_dot_production_attention(fattn)
-
     def forward(self, query, key_value, position_bias, use_cache, past_key_value, project_q, project_k, project_v,
                 attention_out, dim_head, num_heads, num_heads_kv):
         assert use_cache                                                           # origin.py:18
-        batch, len_q, len_new = query.size(0), query.size(1), key_value.size(1)
-        q = _heads(project_q(query), batch, len_q, num_heads, dim_head)
-        k = _heads(project_k(key_value), batch, len_new, num_heads_kv, dim_head)
-        v = _heads(project_v(key_value), batch, len_new, num_heads_kv, dim_head)
-        if q.dtype != torch.bfloat16:
-            raise TypeError(f"the HIP attention path computes in bfloat16, got {q.dtype}")
-        inv_freq, scale = _rope_args(position_bias, q.device)
-        seen = past_key_value[0].size(2) if past_key_value is not None else 0
-        len_k = seen + len_new
-        q_rot = _rope(q, inv_freq, scale, len_k - len_q)
-        k_rot = _rope(k, inv_freq, scale, seen)
-        v_all = v.contiguous()
-        if past_key_value is not None:
-            k_rot = torch.cat((past_key_value[0], k_rot), dim=2)
-            v_all = torch.cat((past_key_value[1], v_all), dim=2)
-        attn = Attn(q_rot.shape, q_rot.dtype, q_rot.device)
-        attn.append(q_rot, k_rot, v_all, sliding_window=len_k, end=True)          # window >= everything: causal
-        o, _ = attn.get_result()
-        o = o.view(batch, num_heads, len_q, dim_head).permute(0, 2, 1, 3).reshape(batch, len_q, dim_head * num_heads)
-        return attention_out(o), (k_rot, v_all)
+        past = None if past_key_value is None else (past_key_value[0], past_key_value[1], past_key_value[0].size(2), None)
+        out, cache = _call(0, 0, 0, query, key_value, position_bias, past, project_q, project_k, project_v, dim_head, num_heads, num_heads_kv)
+        return attention_out(out), cache[:2]
 
     return forward

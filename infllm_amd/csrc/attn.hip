@@ -19,7 +19,9 @@
 #include <cstdlib>
 
 #include "common.h"
+#include "decode.h"
 
+#include <algorithm>
 #include <atomic>
 #include <cstddef>
 #include <cstring>
@@ -76,6 +78,10 @@ struct StageGeom {
     int32_t out_exc;
     int64_t out_block_rows;
     FastDiv out_exc_div;
+    // A launch with one key split whose result nothing else joins (out != NULL) writes the finished bf16 rows itself:
+    // row [b, h, i] at b * o_sb + h * o_sh + i * o_sl; no partial rows, no merge.
+    bf16_t *out;
+    int64_t o_sb, o_sh, o_sl;
 };
 
 // LDS layouts.  Tiles go from global memory straight into LDS (global_load_lds_dwordx4: lane l of a
@@ -94,7 +100,13 @@ struct StageGeom {
 //                          supplies the address of 4 consecutive d of key j, and lane i receives element
 //                          i of keys j = 0..3, i.e. 4 consecutive keys at one d.
 __device__ __forceinline__ int k_lds_row(int key) { return (key & ~12) | ((key & 4) << 1) | ((key & 8) >> 1); }
-__device__ __forceinline__ int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+// Heads of 64: a row is 128 bytes (8 chunks), two rows share a 256-byte line.  16 consecutive rows, one chunk each, hit 16
+// different places when the row pairs use 8 different positions; the four row pairs' bit that decides the upper or lower
+// four chunks is the pair's lowest, so that the transposing read's 4 rows x 4 chunks x 2 halves are 32 different slots.
+template <int D>
+__device__ __forceinline__ int swz(int row) {
+    return D == 128 ? ((row & 3) << 2) | ((row >> 2) & 3) : (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
+}
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ s16x4 lds_read_tr(const bf16_t *p) {
@@ -113,7 +125,8 @@ __device__ __forceinline__ void load_to_lds16(const bf16_t *g, bf16_t *lds_wave_
                  : "memory");
 }
 
-constexpr int kTileBytes = kTile * kD * 2;        // one K (or V) tile in LDS
+template <int D>
+constexpr int kTileBytes = kTile * D * 2;         // one K (or V) tile in LDS
 constexpr float kLazyLog2 = 8.f;                  // the running max may lag the true max by 2^8
 
 template <int N>
@@ -123,8 +136,10 @@ struct IntC {
 
 // MODE: what the launch walks.  kLinear: the linear source of `a`; kPaged: the page table of `a`; kBoth: the linear
 // source of `a`, then the page table of `a2` with `a2`'s queries - both stages of the operator in one launch, as ONE
-// list of tiles that the key splits divide between them (one set of partials, one fixed cost instead of two).
-enum { kLinear = 0, kPaged = 1, kBoth = 2 };
+// list of tiles that the key splits divide between them (one set of partials, one fixed cost instead of two).  kSinks:
+// the linear source of `a`, then the first j_hi rows of the linear source of `a2` (rows of D elements, no ring) under the
+// complement mask with `a2`'s queries - the sliding window and the attention sinks of the sink + window types.
+enum { kLinear = 0, kPaged = 1, kBoth = 2, kSinks = 3 };
 
 // The page table can ride in the launch itself (INLINE): the host passes up to kInlinePages entries by value, and the
 // kernel reads them where they lie in its argument segment - scalar loads through the constant address space, like the
@@ -141,13 +156,14 @@ struct KernargLayout {                     // the arguments as the launch lays t
     InlinePages pages;
 };
 
-template <int MODE, bool INLINE = false>
+template <int D, int MODE, bool INLINE = false>
 __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_args a, infllm_attn_args a2, StageGeom geo,
                                                                  std::conditional_t<INLINE, InlinePages, NoInlinePages>) {
-    constexpr bool HAS_LIN = MODE != kPaged, HAS_PAG = MODE != kLinear;
-    const infllm_attn_args &ap = MODE == kBoth ? a2 : a;                 // the paged stage's arguments
+    constexpr bool HAS_LIN = MODE != kPaged, HAS_PAG = MODE != kLinear, TWO = MODE == kBoth || MODE == kSinks;
+    constexpr int kRow = D * 2, kTB = kTileBytes<D>;                     // bytes of a row, of a tile
+    const infllm_attn_args &ap = TWO ? a2 : a;                 // the paged stage's arguments
     extern __shared__ __attribute__((aligned(16))) char lds_dyn[];      // kStages K tiles, then kStages V tiles
-    char *const Ks = lds_dyn, *const Vs = lds_dyn + kStages * kTileBytes;
+    char *const Ks = lds_dyn, *const Vs = lds_dyn + kStages * kTB;
     __shared__ int wg_lo[kWaves], wg_hi[kWaves];
 
     // the wave index is the same in every lane: said so, what derives from it (the wave's queries, tile range, mask
@@ -169,6 +185,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
             bz = (int)fdiv(rest, geo.gy);
             by = rest - bz * gy;
         }
+        // a causal launch of more workgroups than the chip holds starts with the last queries, which see the most keys:
+        // the short ones fill the end (7,904 causal keys, 512 workgroups: 281 -> 232 us)
+        if (HAS_LIN && a.mask == INFLLM_MASK_WINDOW) bx = gx - 1 - bx;
     }
     const int b = (int)fdiv(by, geo.hkv), g = by - b * a.Hkv;
     const int split = bz;
@@ -203,7 +222,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
     }
     if (lin_t1 <= lin_t0) lin_t0 = lin_t1 = 0;
     // The unified tile list: u in [0, n_lin) is linear tile lin_t0 + u, u in [n_lin, n_lin + n_pag) is page u - n_lin.
-    const int n_lin = lin_t1 - lin_t0, n_pag = HAS_PAG ? ap.n_pages : 0;
+    const int n_lin = lin_t1 - lin_t0, n_pag = MODE == kSinks ? ((int)ap.j_hi + kTile - 1) >> 6 : HAS_PAG ? ap.n_pages : 0;
     int g_t0, g_t1;                      // this split's share of the list
     {
         // n / nsplit tiles each; the n % nsplit left over go one each to a run of splits in the middle: the first and
@@ -218,35 +237,36 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
     }
     const int wu0 = w_t0 - lin_t0, wu1 = w_t1 - lin_t0;     // this wave's linear tiles in list indices
 
-    bf16x8 qreg[kD / 16];                     // Q as the B operand: lane = (query col, k-group); loaded behind the first tiles
+    bf16x8 qreg[D / 16];                     // Q as the B operand: lane = (query col, k-group); loaded behind the first tiles
 
     // ---- per-lane LDS byte offsets of the MFMA operands (inside one tile buffer)
-    uint32_t k_off[kD / 16];                  // K operand kk of sub-tile 0 (sub-tile 1: + 32 rows)
+    uint32_t k_off[D / 16];                  // K operand kk of sub-tile 0 (sub-tile 1: + 32 rows)
 #pragma unroll
-    for (int kk = 0; kk < kD / 16; ++kk) k_off[kk] = col * 256 + (((kk * 2 + grp) ^ swz(col)) * 16);
-    uint32_t v_off[kD / 32][2];               // V^T operand of d-tile dt, key half e, of 16-key step 0 (step gi: + 16*gi rows)
+    for (int kk = 0; kk < D / 16; ++kk) k_off[kk] = col * kRow + (((kk * 2 + grp) ^ swz<D>(col)) * 16);
+    uint32_t v_off[D / 32][2];               // V^T operand of d-tile dt, key half e, of 16-key step 0 (step gi: + 16*gi rows)
     {
         const int lam = lane & 15, g16 = lane >> 4;
         const int vr = 8 * (g16 >> 1) + (lam >> 2);              // lane 4*j + q addresses key j ...
         const int vc = 2 * (g16 & 1) + ((lam & 3) >> 1);         // ... at 4 consecutive d: 16-byte chunk
         const int vh = 8 * (lam & 1);                            //     and byte offset inside it
 #pragma unroll
-        for (int dt = 0; dt < kD / 32; ++dt)
+        for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
-            for (int e = 0; e < 2; ++e) v_off[dt][e] = (vr + 4 * e) * 256 + (((dt * 4 + vc) ^ swz(vr + 4 * e)) * 16) + vh;
+            for (int e = 0; e < 2; ++e) v_off[dt][e] = (vr + 4 * e) * kRow + (((dt * 4 + vc) ^ swz<D>(vr + 4 * e)) * 16) + vh;
     }
 
-    // ---- tile loads: wave w, instruction i fills LDS rows 8*w + 4*i .. +3; lane -> (row, position).
+    // ---- tile loads: an instruction fills 1024 bytes of LDS (4 rows of 128 elements or 8 of 64); wave w fills the 8 rows
+    //      from 8*w on; lane -> (row, position).
     //      The wave-uniform tile base advances with the loop; the per-lane offsets are loop invariant.
-    constexpr int kLd = kTile / (4 * kWaves);  // load instructions per wave and tile, for K and for V
+    constexpr int kRowsPerLd = 1024 / kRow, kLd = kTile / (kRowsPerLd * kWaves);  // load instructions per wave and tile, for K and for V
     uint32_t gk_off[kLd], gv_off[kLd];        // element offsets inside a linear tile
-    uint32_t pk_off[kLd], pv_off[kLd];        // ... inside a page (rows of kD elements)
+    uint32_t pk_off[kLd], pv_off[kLd];        // ... inside a page (rows of D elements)
     int gk_row[kLd], gv_row[kLd];
     {
-        const int ld_pos = lane & 15, ld_sub = lane >> 4;
+        const int ld_pos = lane & (D / 8 - 1), ld_sub = lane / (D / 8);
 #pragma unroll
         for (int i = 0; i < kLd; ++i) {
-            const int R = 4 * kLd * wave + 4 * i + ld_sub, chunk = ld_pos ^ swz(R);
+            const int R = kRowsPerLd * (kLd * wave + i) + ld_sub, chunk = ld_pos ^ swz<D>(R);
             gk_row[i] = k_lds_row(R);
             gv_row[i] = R;
             if (HAS_LIN) {
@@ -254,8 +274,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
                 gv_off[i] = (uint32_t)(R * a.v_sl + chunk * 8);
             }
             if (HAS_PAG) {
-                pk_off[i] = (uint32_t)(gk_row[i] * kD + chunk * 8);
-                pv_off[i] = (uint32_t)(R * kD + chunk * 8);
+                pk_off[i] = (uint32_t)(gk_row[i] * D + chunk * 8);
+                pv_off[i] = (uint32_t)(R * D + chunk * 8);
             }
         }
     }
@@ -280,8 +300,14 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
     auto load_tile = [&](int u, int buf) {     // list index; linear tiles are requested in ascending order
         const bf16_t *kbase, *vbase;
         int row_lo, row_hi;                   // valid rows of this tile: [row_lo, row_hi)
-        const bool paged = MODE == kPaged || (MODE == kBoth && u >= n_lin);
-        if (paged) {
+        const bool paged = MODE == kPaged || (TWO && u >= n_lin);
+        if (MODE == kSinks && paged) {
+            const int64_t j0 = (int64_t)(u - n_lin) * kTile;
+            kbase = (const bf16_t *)ap.d_k + (int64_t)b * ap.k_sb + (int64_t)g * ap.k_sh + j0 * D;
+            vbase = (const bf16_t *)ap.d_v + (int64_t)b * ap.v_sb + (int64_t)g * ap.v_sh + j0 * D;
+            row_lo = 0;
+            row_hi = (int)min((int64_t)kTile, ap.j_hi - j0);
+        } else if (paged) {
             const __attribute__((address_space(4))) infllm_page *entry = page_table + (u - n_lin);
             const int64_t hs = entry->head_stride;
             kbase = (const bf16_t *)entry->k + (int64_t)g * hs;
@@ -297,7 +323,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
             row_lo = (int)max((int64_t)0, a.j_lo - j0);
             row_hi = (int)min((int64_t)kTile, a.j_hi - j0);
         }
-        char *kdst = Ks + buf * kTileBytes + wave * (kLd * 1024), *vdst = Vs + buf * kTileBytes + wave * (kLd * 1024);
+        char *kdst = Ks + buf * kTB + wave * (kLd * 1024), *vdst = Vs + buf * kTB + wave * (kLd * 1024);
         if (row_lo == 0 && row_hi == kTile) {          // the common case: no per-lane predicate
 #pragma unroll
             for (int i = 0; i < kLd; ++i) {
@@ -318,9 +344,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
 
     // ---- running softmax state of this lane's query (max kept in raw logit units, allowed to lag)
     float m_run = -INFINITY, l_run = 0.f, neg_ms = 0.f;
-    f32x16 oacc[kD / 32];
+    f32x16 oacc[D / 32];
 #pragma unroll
-    for (int dt = 0; dt < kD / 32; ++dt)
+    for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
 
@@ -328,7 +354,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
     const float lazy = kLazyLog2 / scale;
 
     auto tile_math = [&](int buf, int t) {
-        const char *kb = Ks + buf * kTileBytes, *vb = Vs + buf * kTileBytes;
+        const char *kb = Ks + buf * kTB, *vb = Vs + buf * kTB;
         f32x16 s[2];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
@@ -337,16 +363,17 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
         {
             // 16 K operands in groups of 4 (kk pair x both sub-tiles): a group is requested from LDS while the
             // MFMAs of the previous one run; scheduling fences keep the compiler from serialising read -> MFMA
-            bf16x8 ka[4][4];
+            constexpr int NG = D / 32;                 // (16 K operands of heads of 128, 8 of heads of 64)
+            bf16x8 ka[NG][4];
             auto k_operand = [&](int i) {          // i = kk * 2 + ks
-                return *(const bf16x8 *)(kb + (i & 1) * 32 * 256 + k_off[i >> 1]);
+                return *(const bf16x8 *)(kb + (i & 1) * 32 * kRow + k_off[i >> 1]);
             };
 #pragma unroll
             for (int j = 0; j < 4; ++j) ka[0][j] = k_operand(j);
 #pragma unroll
-            for (int gi = 0; gi < 4; ++gi) {
+            for (int gi = 0; gi < NG; ++gi) {
                 __builtin_amdgcn_sched_barrier(0);
-                if (gi < 3) {
+                if (gi < NG - 1) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) ka[gi + 1][j] = k_operand((gi + 1) * 4 + j);
                     __builtin_amdgcn_sched_barrier(0);
@@ -363,8 +390,13 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
         bool need_mask;
         int row_lo = 0, row_hi = kTile;
         int d0 = 0;                            // dist of (this lane's query, key 0 of the tile)
-        const bool paged = MODE == kPaged || (MODE == kBoth && t >= n_lin);
-        if (paged) {
+        const bool paged = MODE == kPaged || (TWO && t >= n_lin);
+        if (MODE == kSinks && paged) {
+            const int64_t j0 = (int64_t)(t - n_lin) * kTile, e0 = (int64_t)i0 + ap.offset - j0;
+            row_hi = (int)min((int64_t)kTile, ap.j_hi - j0);
+            need_mask = row_hi < kTile || e0 - (kTile - 1) < ap.window;
+            d0 = (int)min(max(e0, (int64_t)-kBig), (int64_t)kBig) + col;
+        } else if (paged) {
             row_hi = page_table[t - n_lin].n_valid;
             need_mask = row_hi < kTile;
         } else {
@@ -381,7 +413,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
             d0 = (int)min(max(e0, (int64_t)-kBig), (int64_t)kBig) + col;
         }
         if (need_mask) {
-            const int win = (int)min(a.window, (int64_t)2 * kBig);
+            const int win = (int)min(MODE == kSinks && paged ? ap.window : a.window, (int64_t)2 * kBig);
             const int lo_l = row_lo - 8 * grp, hi_l = row_hi - 8 * grp;      // bounds on kc for this lane
             const int dl = d0 - 8 * grp;                                       // dist = dl - kc
 #pragma unroll
@@ -395,6 +427,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
                     if (!paged) {
                         if (a.mask == INFLLM_MASK_WINDOW) vis = vis && (kc <= dl) && (kc > dl - win);
                         if (a.mask == INFLLM_MASK_COMPLEMENT) vis = vis && (kc <= dl - win);
+                    } else if (MODE == kSinks) {
+                        vis = vis && (kc <= dl - win);
                     }
                     s[ks][r] = vis ? s[ks][r] : -INFINITY;
                 }
@@ -414,7 +448,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
             const float al = moved ? alpha : 1.f;
             l_run *= al;
 #pragma unroll
-            for (int dt = 0; dt < kD / 32; ++dt)
+            for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) oacc[dt][r] *= al;
             m_run = m_new;
@@ -440,12 +474,12 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
             // 4 steps of 16 keys, 4 MFMAs each; the V^T operands of a step are requested from LDS while the
             // MFMAs of the previous step run
             typedef short s16x8 __attribute__((ext_vector_type(8)));
-            s16x8 va[2][kD / 32];
+            s16x8 va[2][D / 32];
             auto v_operands = [&](int gi, s16x8 *dst) {
 #pragma unroll
-                for (int dt = 0; dt < kD / 32; ++dt) {
-                    dst[dt].lo = lds_read_tr((const bf16_t *)(vb + gi * 16 * 256 + v_off[dt][0]));
-                    dst[dt].hi = lds_read_tr((const bf16_t *)(vb + gi * 16 * 256 + v_off[dt][1]));
+                for (int dt = 0; dt < D / 32; ++dt) {
+                    dst[dt].lo = lds_read_tr((const bf16_t *)(vb + gi * 16 * kRow + v_off[dt][0]));
+                    dst[dt].hi = lds_read_tr((const bf16_t *)(vb + gi * 16 * kRow + v_off[dt][1]));
                 }
             };
             v_operands(0, va[0]);
@@ -464,11 +498,11 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
                 // exponentials of the tile's second half go between the MFMAs of its first half.
                 if (gi < 2) exps(1, 8 * gi, 8 * gi + 8);
 #pragma unroll
-                for (int dt = 0; dt < kD / 32; ++dt)
+                for (int dt = 0; dt < D / 32; ++dt)
                     oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va[gi & 1][dt]), pb, oacc[dt], 0, 0, 0);
                 if (gi < 2) {
 #pragma unroll
-                    for (int dt = 0; dt < kD / 32; ++dt) {
+                    for (int dt = 0; dt < D / 32; ++dt) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // one MFMA
                         __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);      // multiply-adds, rounding, row sum
                         __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);      // two exponentials
@@ -492,14 +526,14 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
         const bool ok = live && qi < src.Lq;
         const bf16_t *qrow = (const bf16_t *)src.d_q + (int64_t)b * src.q_sb + (int64_t)h * src.q_sh + (int64_t)qi * src.q_sl;
 #pragma unroll
-        for (int kk = 0; kk < kD / 16; ++kk) {
+        for (int kk = 0; kk < D / 16; ++kk) {
             u32x4 raw = ok ? *(const u32x4 *)(qrow + kk * 16 + grp * 8) : u32x4{0, 0, 0, 0};
             qreg[kk] = __builtin_bit_cast(bf16x8, raw);
         }
     };
     // the queries of the stage this split starts in; a split that crosses from the linear tiles into the pages swaps
     // them for the paged stage's queries at its first page (once per workgroup: that wait also covers the tiles in flight)
-    bool q_paged = MODE == kPaged || (MODE == kBoth && g_t0 >= n_lin);
+    bool q_paged = MODE == kPaged || (TWO && g_t0 >= n_lin);
     load_q(q_paged ? ap : a);
 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -507,10 +541,13 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
     // asm makes it place its own wait for them HERE rather than in front of their first use inside the loop,
     // where a vmcnt(0) would wait for the tiles in flight.
 #pragma unroll
-    for (int kk = 0; kk < kD / 16; ++kk) asm volatile("" : "+v"(qreg[kk]));
+    for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(qreg[kk]));
     __syncthreads();
     // does this wave see tile u at all?  (pages: every live wave; linear tiles: the wave's own visible range)
-    auto mine = [&](int u) { return (HAS_PAG && u >= n_lin) ? live : (u >= wu0 && u < wu1); };
+    auto mine = [&](int u) {
+        if (MODE == kSinks && u >= n_lin) return live && (int64_t)i1 + ap.offset - ap.window >= (int64_t)(u - n_lin) * kTile;
+        return (HAS_PAG && u >= n_lin) ? live : (u >= wu0 && u < wu1);
+    };
     for (int t = g_t0; t < g_t1; t += 2) {
         const int buf = (t - g_t0) & 3;                          // 0 or 2
         if (t + 2 < g_t1) load_tile(t + 2, buf ^ 2);
@@ -519,7 +556,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
         for (int e = 0; e < 2; ++e) {                            // wave-uniform conditions; barriers stay outside
             const int u = t + e;
             if (u >= g_t1) break;
-            if (MODE == kBoth && u >= n_lin && !q_paged) {
+            if (TWO && u >= n_lin && !q_paged) {
                 load_q(ap);
                 q_paged = true;
             }
@@ -545,27 +582,49 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
         rows_left = n_blk - in_blk;
     }
     const int64_t row = row0 + col;
+    char *stage = lds_dyn + wave * (kQTile * kRow);
+    constexpr int kChunks = D / 8;                                                 // 16-byte chunks of a row
+    constexpr int kRowsPerSt = 64 / kChunks;                                       // rows a wave stores per instruction
+    if (geo.out) {                                                                 // the finished rows, rounded to bf16 once
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+                const u32x2 o4{pack_bf16x2(oacc[dt][4 * q4] * inv, oacc[dt][4 * q4 + 1] * inv),
+                               pack_bf16x2(oacc[dt][4 * q4 + 2] * inv, oacc[dt][4 * q4 + 3] * inv)};
+                const int chunk = dt * 4 + q4;
+                *(u32x2 *)(stage + col * kRow + ((chunk ^ col) & (kChunks - 1)) * 16 + grp * 8) = o4;
+            }
+        const int piece = lane & (kChunks - 1);
+        bf16_t *dst = geo.out + (int64_t)b * geo.o_sb + (int64_t)h * geo.o_sh + (int64_t)i0 * geo.o_sl + piece * 8;
+#pragma unroll
+        for (int k4 = 0; k4 < kQTile / kRowsPerSt; ++k4) {
+            const int qr = kRowsPerSt * k4 + lane / kChunks;
+            const u32x4 o8 = *(const u32x4 *)(stage + qr * kRow + ((piece ^ qr) & (kChunks - 1)) * 16);
+            if (qr < rows_left) *(u32x4 *)(dst + (int64_t)qr * geo.o_sl) = o8;
+        }
+        return;
+    }
     {
         // fp16 keeps 11 bits of a value that ends up rounded to bf16's 8, and halves what the partials cost in HBM
         // (with few tiles per workgroup their write is a tenth of the kernel); staged rows are 256 bytes, a lane's
         // 4-value piece is 8 bytes, and 16-byte chunks are swizzled by the row
-        char *stage = lds_dyn + wave * (kQTile * kD * 2);
 #pragma unroll
-        for (int dt = 0; dt < kD / 32; ++dt)
+        for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
             for (int q4 = 0; q4 < 4; ++q4) {
                 const f16x4 o4{(_Float16)(oacc[dt][4 * q4] * inv), (_Float16)(oacc[dt][4 * q4 + 1] * inv),
                                (_Float16)(oacc[dt][4 * q4 + 2] * inv), (_Float16)(oacc[dt][4 * q4 + 3] * inv)};
                 const int chunk = dt * 4 + q4;                                     // 16-byte chunk of the row; grp picks its half
-                *(f16x4 *)(stage + col * (kD * 2) + ((chunk ^ col) & 15) * 16 + grp * 8) = o4;
+                *(f16x4 *)(stage + col * kRow + ((chunk ^ col) & (kChunks - 1)) * 16 + grp * 8) = o4;
             }
-        const int piece = lane & 15;
+        const int piece = lane & (kChunks - 1);
         _Float16 *o_part = (_Float16 *)a.d_o_part;
 #pragma unroll
-        for (int k4 = 0; k4 < kQTile / 4; ++k4) {
-            const int qr = 4 * k4 + (lane >> 4);
-            const u32x4 o8 = *(const u32x4 *)(stage + qr * (kD * 2) + ((piece ^ qr) & 15) * 16);
-            if (qr < rows_left) *(u32x4 *)(o_part + (row0 + qr) * kD + piece * 8) = o8;
+        for (int k4 = 0; k4 < kQTile / kRowsPerSt; ++k4) {
+            const int qr = kRowsPerSt * k4 + lane / kChunks;
+            const u32x4 o8 = *(const u32x4 *)(stage + qr * kRow + ((piece ^ qr) & (kChunks - 1)) * 16);
+            if (qr < rows_left) *(u32x4 *)(o_part + (row0 + qr) * D + piece * 8) = o8;
         }
     }
     if (qi >= a.Lq) return;
@@ -573,7 +632,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
 }
 
 // one thread per (row, 8 dims): P fp16 partials -> bf16 output row + final lse (merge_piece, common.h)
-__global__ __launch_bounds__(256) void attn_merge_kernel(MergeJob job) { merge_piece(job, (int64_t)blockIdx.x * 256 + threadIdx.x); }
+template <int D>
+__global__ __launch_bounds__(256) void attn_merge_kernel(MergeJob job) { merge_piece<D>(job, (int64_t)blockIdx.x * 256 + threadIdx.x); }
 
 // the log-sum-exp half of the merge alone: one thread per row
 __global__ __launch_bounds__(256) void attn_merge_lse_kernel(const float *lse_part, int P, int64_t rows, float *lse_out, PartSets ps) {
@@ -610,14 +670,16 @@ __device__ __forceinline__ float group16_sum(float v) {
     return v;
 }
 
+template <int D>
 __global__ __launch_bounds__(256) void attn_merge_wide_kernel(const _Float16 *o_part, const float *lse_part, int P, int B, int H,
                                                               int Lq, bf16_t *out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
                                                               float *lse_out, PartSets ps) {
     const int64_t rows = (int64_t)B * H * Lq;
     const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 4;       // (row, 8 dims)
     const int pl = threadIdx.x & 15;
-    const int64_t row = e >> 4;
-    const int c = (int)(e & 15);
+    constexpr int kPieces = D / 8;
+    const int64_t row = e / kPieces;
+    const int c = (int)(e % kPieces);
     if (row >= rows) return;                                                 // whole 16-lane groups leave together
     constexpr int kMine = 8;                                                 // partials per lane: P <= 128
     float l[kMine];
@@ -628,7 +690,7 @@ __global__ __launch_bounds__(256) void attn_merge_wide_kernel(const _Float16 *o_
         const int p = pl + 16 * i;
         const bool on = p < P;
         l[i] = on ? lse_part[ps.l(p, rows) + row] : -INFINITY;
-        o[i] = on ? *(const f16x8 *)(o_part + (ps.l(p, rows) + row) * kD + ps.o(p) + c * 8) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        o[i] = on ? *(const f16x8 *)(o_part + (ps.l(p, rows) + row) * D + ps.o(p) + c * 8) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
         m = fmaxf(m, l[i]);
     }
     m = group16_max(m);
@@ -708,51 +770,59 @@ int check_common(const infllm_attn_args *a) {
     return 0;
 }
 
-// mode: kLinear (a), kPaged (a), kBoth (a = linear stage, a2 = paged stage); h_pages: NULL, or the paged stage's table
-// [B, n_pages] in HOST memory, B * n_pages <= kInlinePages, which then travels in the launch (d_pages is not read)
+// Where a launch's rows go besides the argument block's partial buffers: see StageGeom
+struct StageOut {
+    int out_exc = 0;
+    int64_t out_block_rows = 0;
+    bf16_t *out = nullptr;
+    int64_t o_sb = 0, o_sh = 0, o_sl = 0;
+};
+
+template <int D, int MODE, bool INLINE, typename Pages>
+int launch_mode(dim3 grid, const infllm_attn_args &a, const infllm_attn_args &a2, const StageGeom &geo, const Pages &pages, void *stream) {
+    constexpr size_t lds_bytes = 2 * kStages * kTileBytes<D>;
+    static std::atomic<bool> lds_set{false};                  // dynamic LDS above 64 KiB must be enabled once per kernel
+    if (!lds_set.load(std::memory_order_acquire)) {
+        const hipError_t e = hipFuncSetAttribute((const void *)attn_stage_kernel<D, MODE, INLINE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+        if (e != hipSuccess) return infllm_fail(-2, "attn_stage: %s", hipGetErrorString(e));
+        lds_set.store(true, std::memory_order_release);
+    }
+    hipLaunchKernelGGL((attn_stage_kernel<D, MODE, INLINE>), grid, dim3(kThreads), lds_bytes, (hipStream_t)stream, a, a2, geo, pages);
+    INFLLM_CHECK_LAUNCH("attn_stage");
+    return 0;
+}
+
+// mode: kLinear (a), kPaged (a), kBoth / kSinks (a = linear stage, a2 = the other stage); h_pages: NULL, or the paged
+// stage's table [B, n_pages] in HOST memory, B * n_pages <= kInlinePages, which then travels in the launch (d_pages is
+// not read)
+template <int D = kD>
 int launch_stage(int mode, const infllm_attn_args *a, const infllm_attn_args *a2, void *stream, const infllm_page *h_pages = nullptr,
-                 int out_exc = 0, int64_t out_block_rows = 0) {
+                 const StageOut &so = StageOut()) {
     const int G = a->H / a->Hkv;
     const int n_tasks = ((a->Lq + kQTile - 1) / kQTile) * G;
     dim3 grid((n_tasks + kWaves - 1) / kWaves, a->B * a->Hkv, a->nsplit);
     INFLLM_REQUIRE((int64_t)grid.x * grid.y * grid.z < (1ll << 31), "attn_stage: grid too large");
     StageGeom geo{fast_div(grid.x), fast_div(grid.y), fast_div((uint32_t)a->Hkv), fast_div((uint32_t)G),
-                  fast_div((uint32_t)a->nsplit), fast_div(1), n_tasks, out_exc, out_block_rows, fast_div((uint32_t)(out_exc > 0 ? out_exc : 1))};
+                  fast_div((uint32_t)a->nsplit), fast_div(1), n_tasks, so.out_exc, so.out_block_rows,
+                  fast_div((uint32_t)(so.out_exc > 0 ? so.out_exc : 1)), so.out, so.o_sb, so.o_sh, so.o_sl};
     // tile indices stay below 2^30, so any ring of 2^31 tiles or more never wraps: one divisor stands for all of them
     if (mode != kPaged) geo.cap_tiles = fast_div((uint32_t)std::min<int64_t>(a->cap / kTile, 1ll << 31));
-    constexpr size_t lds_bytes = 2 * kStages * kTileBytes;
-    static bool lds_set[3] = {false, false, false};           // dynamic LDS above 64 KiB must be enabled once per kernel
     const infllm_attn_args &second = a2 ? *a2 : *a;
     if (h_pages) {
         const infllm_attn_args &pg = mode == kBoth ? second : *a;
-        INFLLM_REQUIRE(mode != kLinear && pg.n_pages >= 0 && (int64_t)pg.B * pg.n_pages <= kInlinePages,
+        INFLLM_REQUIRE((mode == kPaged || mode == kBoth) && pg.n_pages >= 0 && (int64_t)pg.B * pg.n_pages <= kInlinePages,
                        "attn_stage: %d x %d pages do not fit a launch", pg.B, pg.n_pages);
-        static bool lds_set_inline[3] = {false, false, false};
-        const void *fn = mode == kPaged ? (const void *)attn_stage_kernel<kPaged, true> : (const void *)attn_stage_kernel<kBoth, true>;
-        if (!lds_set_inline[mode]) {
-            hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-            if (e != hipSuccess) return infllm_fail(-2, "attn_stage: %s", hipGetErrorString(e));
-            lds_set_inline[mode] = true;
-        }
         InlinePages table;
         memcpy(table.p, h_pages, sizeof(infllm_page) * pg.B * pg.n_pages);
-        if (mode == kPaged) hipLaunchKernelGGL((attn_stage_kernel<kPaged, true>), grid, dim3(kThreads), lds_bytes, (hipStream_t)stream, *a, second, geo, table);
-        else hipLaunchKernelGGL((attn_stage_kernel<kBoth, true>), grid, dim3(kThreads), lds_bytes, (hipStream_t)stream, *a, second, geo, table);
-        INFLLM_CHECK_LAUNCH("attn_stage");
-        return 0;
+        return mode == kPaged ? launch_mode<D, kPaged, true>(grid, *a, second, geo, table, stream)
+                              : launch_mode<D, kBoth, true>(grid, *a, second, geo, table, stream);
     }
-    const void *fn = mode == kLinear ? (const void *)attn_stage_kernel<kLinear>
-                     : mode == kPaged ? (const void *)attn_stage_kernel<kPaged> : (const void *)attn_stage_kernel<kBoth>;
-    if (!lds_set[mode]) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-        if (e != hipSuccess) return infllm_fail(-2, "attn_stage: %s", hipGetErrorString(e));
-        lds_set[mode] = true;
+    switch (mode) {
+        case kLinear: return launch_mode<D, kLinear, false>(grid, *a, second, geo, NoInlinePages{}, stream);
+        case kPaged: return launch_mode<D, kPaged, false>(grid, *a, second, geo, NoInlinePages{}, stream);
+        case kBoth: return launch_mode<D, kBoth, false>(grid, *a, second, geo, NoInlinePages{}, stream);
+        default: return launch_mode<D, kSinks, false>(grid, *a, second, geo, NoInlinePages{}, stream);
     }
-    if (mode == kLinear) hipLaunchKernelGGL(attn_stage_kernel<kLinear>, grid, dim3(kThreads), lds_bytes, (hipStream_t)stream, *a, second, geo, NoInlinePages{});
-    else if (mode == kPaged) hipLaunchKernelGGL(attn_stage_kernel<kPaged>, grid, dim3(kThreads), lds_bytes, (hipStream_t)stream, *a, second, geo, NoInlinePages{});
-    else hipLaunchKernelGGL(attn_stage_kernel<kBoth>, grid, dim3(kThreads), lds_bytes, (hipStream_t)stream, *a, second, geo, NoInlinePages{});
-    INFLLM_CHECK_LAUNCH("attn_stage");
-    return 0;
 }
 
 }  // namespace
@@ -767,7 +837,42 @@ extern "C" int infllm_attn_stage(const infllm_attn_args *a, void *stream) {
         return launch_stage(kPaged, a, nullptr, stream);
     }
     rc = check_linear_stage(a);
-    return rc ? rc : launch_stage(kLinear, a, nullptr, stream);
+    if (rc) return rc;
+    if (a->Lq == 1 && a->k_sl == kD && a->v_sl == kD) {
+        // One query: what it sees is a range of keys, at most two runs of ring rows - the streaming kernel, which reads a
+        // kv head's rows once for its query heads (4097 ring rows, 32 splits: 9.6 -> 5 us).
+        int64_t lo = a->j_lo, hi = a->j_hi;
+        if (a->mask == INFLLM_MASK_WINDOW) lo = std::max(lo, a->offset - a->window + 1), hi = std::min(hi, a->offset + 1);
+        else if (a->mask == INFLLM_MASK_COMPLEMENT) hi = std::min(hi, a->offset - a->window + 1);
+        DecodeJob d{};
+        d.q[0] = d.q[1] = (const bf16_t *)a->d_q;
+        d.q_sb = a->q_sb; d.q_sh = a->q_sh;
+        d.B = a->B; d.H = a->H; d.Hkv = a->Hkv;
+        d.scale = a->softmax_scale;
+        d.nsplit = a->nsplit;
+        d.o_part = a->d_o_part; d.lse_part = a->d_lse_part;
+        for (int64_t pos = lo; pos < hi;) {
+            const int64_t row = pos % a->cap, n = std::min(hi - pos, a->cap - row);
+            INFLLM_REQUIRE(n < (1ll << 31), "attn_stage: key range too long");
+            d.seg[d.n_seg++] = DecodeSeg{(const bf16_t *)a->d_k + row * kD, (const bf16_t *)a->d_v + row * kD, a->k_sb, a->k_sh, a->v_sb, a->v_sh, (int32_t)n,
+                                         0, 0, nullptr};
+            pos += n;
+        }
+        if (d.n_seg == 0) d.n_seg = 1;                 // nothing visible: empty partials
+        return infllm_decode_attn(&d, kD, stream);
+    }
+    return launch_stage(kLinear, a, nullptr, stream);
+}
+
+int infllm_attn_splits(int64_t wgs, int64_t tiles, int32_t max_parts);
+extern "C" int infllm_attn_stage_splits(const infllm_attn_args *a, int32_t max_splits) {
+    INFLLM_REQUIRE(a && a->B > 0 && a->H > 0 && a->Hkv > 0 && a->H % a->Hkv == 0 && a->Lq > 0 && max_splits >= 1, "attn_stage_splits: bad arguments");
+    int64_t keys = a->d_pages ? (int64_t)a->n_pages * kTile : a->j_hi - a->j_lo;
+    if (!a->d_pages && a->mask == INFLLM_MASK_WINDOW) keys = std::min<int64_t>(keys, a->window + kTile);
+    keys = std::max<int64_t>(keys, 1);
+    if (a->Lq == 1 && !a->d_pages) return infllm_decode_splits(a->B, a->H, a->Hkv, (keys + kDecodeBlock - 1) / kDecodeBlock, std::min(max_splits, 64));
+    const int64_t wgs = ((int64_t)((a->Lq + kQTile - 1) / kQTile) * (a->H / a->Hkv) + kWaves - 1) / kWaves * a->Hkv * a->B;
+    return infllm_attn_splits(wgs, (keys + kTile - 1) / kTile, std::min(max_splits, 64));
 }
 
 // library-internal: a linear stage over the queries of several consecutive execution blocks of `exc` rows (the last
@@ -780,7 +885,11 @@ int infllm_attn_stage_blocked(const infllm_attn_args *a, int32_t exc, int64_t bl
     int rc = check_common(a);
     if (rc) return rc;
     rc = check_linear_stage(a);
-    return rc ? rc : launch_stage(kLinear, a, nullptr, stream, nullptr, exc, block_rows);
+    if (rc) return rc;
+    StageOut so;
+    so.out_exc = exc;
+    so.out_block_rows = block_rows;
+    return launch_stage(kLinear, a, nullptr, stream, nullptr, so);
 }
 
 // library-internal: the paged stage (local == NULL) or both stages in one launch, with the page table [B, n_pages]
@@ -902,13 +1011,14 @@ extern "C" int infllm_attn_fwd_noalloc(const infllm_attn_args *local, const infl
 }
 
 // library-internal: the description of a merge over two sets of partials, P1 behind (d_o_part, d_lse_part) and P2
-// behind (d_o_part2, d_lse_part2), in that order; P2 == 0 is the plain merge
+// behind (d_o_part2, d_lse_part2), in that order; P2 == 0 is the plain merge.  dim: elements of a row, 128 or 64.
 int infllm_merge_job(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2, const float *d_lse_part2,
                      int32_t P2, int32_t B, int32_t H, int32_t Lq, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse,
-                     MergeJob *job) {
+                     MergeJob *job, int32_t dim) {
     INFLLM_REQUIRE(d_o_part && d_lse_part && job, "attn_merge: null pointer");
     INFLLM_REQUIRE(P1 >= 1 && P2 >= 0 && (P2 == 0 || (d_o_part2 && d_lse_part2)), "attn_merge: bad partial sets %d + %d", P1, P2);
     INFLLM_REQUIRE(B > 0 && H > 0 && Lq > 0, "attn_merge: bad sizes B=%d H=%d Lq=%d", B, H, Lq);
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "attn_merge: rows of %d elements", dim);
     INFLLM_REQUIRE((o_sl % 8 | o_sh % 8 | o_sb % 8) == 0, "attn_merge: output strides must be multiples of 8");
     PartSets ps{P1 + P2, 0, 0};
     if (P2 > 0) {
@@ -916,7 +1026,7 @@ int infllm_merge_job(const uint16_t *d_o_part, const float *d_lse_part, int32_t 
         ps.n_first = P1;
         // index (p * rows + row) of the first buffers -> index ((p - P1) * rows + row) of the second
         ps.skip_l = (int64_t)(((intptr_t)d_lse_part2 - (intptr_t)d_lse_part) / (intptr_t)sizeof(float)) - (int64_t)P1 * rows_;
-        ps.skip_o = (int64_t)(((intptr_t)d_o_part2 - (intptr_t)d_o_part) / 2) - (int64_t)P1 * rows_ * kD - ps.skip_l * kD;
+        ps.skip_o = (int64_t)(((intptr_t)d_o_part2 - (intptr_t)d_o_part) / 2) - (int64_t)P1 * rows_ * dim - ps.skip_l * dim;
     }
     *job = MergeJob{(const _Float16 *)d_o_part, d_lse_part, P1 + P2, B, H, Lq, (bf16_t *)d_out, o_sb, o_sh, o_sl, d_lse, ps};
     return 0;
@@ -925,9 +1035,9 @@ int infllm_merge_job(const uint16_t *d_o_part, const float *d_lse_part, int32_t 
 // library-internal: the merge over two sets of partials
 int infllm_attn_merge2(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2,
                        const float *d_lse_part2, int32_t P2, int32_t B, int32_t H, int32_t Lq, void *d_out, int64_t o_sb,
-                       int64_t o_sh, int64_t o_sl, float *d_lse, void *stream) {
+                       int64_t o_sh, int64_t o_sl, float *d_lse, void *stream, int32_t dim) {
     MergeJob job;
-    const int jrc = infllm_merge_job(d_o_part, d_lse_part, P1, d_o_part2, d_lse_part2, P2, B, H, Lq, d_out, o_sb, o_sh, o_sl, d_lse, &job);
+    const int jrc = infllm_merge_job(d_o_part, d_lse_part, P1, d_o_part2, d_lse_part2, P2, B, H, Lq, d_out, o_sb, o_sh, o_sl, d_lse, &job, dim);
     if (jrc) return jrc;
     const int32_t P = P1 + P2;
     const PartSets ps = job.ps;
@@ -945,13 +1055,13 @@ int infllm_attn_merge2(const uint16_t *d_o_part, const float *d_lse_part, int32_
         INFLLM_CHECK_LAUNCH("attn_merge (lse)");
         return 0;
     }
-    const int64_t threads = (int64_t)B * H * Lq * 16;
+    const int64_t threads = (int64_t)B * H * Lq * (dim / 8);
     if (wide)
-        hipLaunchKernelGGL(attn_merge_wide_kernel, dim3((unsigned)((threads * 16 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                           (const _Float16 *)d_o_part, d_lse_part, P, B, H, Lq, (bf16_t *)d_out, o_sb, o_sh, o_sl, d_lse, ps);
+        hipLaunchKernelGGL((dim == 64 ? attn_merge_wide_kernel<64> : attn_merge_wide_kernel<128>), dim3((unsigned)((threads * 16 + 255) / 256)),
+                           dim3(256), 0, (hipStream_t)stream, (const _Float16 *)d_o_part, d_lse_part, P, B, H, Lq, (bf16_t *)d_out, o_sb, o_sh, o_sl, d_lse, ps);
     else
-        hipLaunchKernelGGL(attn_merge_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                           job);
+        hipLaunchKernelGGL((dim == 64 ? attn_merge_kernel<64> : attn_merge_kernel<128>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                           (hipStream_t)stream, job);
     INFLLM_CHECK_LAUNCH("attn_merge");
     return 0;
 }
@@ -959,5 +1069,40 @@ int infllm_attn_merge2(const uint16_t *d_o_part, const float *d_lse_part, int32_
 extern "C" int infllm_attn_merge(const uint16_t *d_o_part, const float *d_lse_part, int32_t P, int32_t B, int32_t H,
                                  int32_t Lq, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse,
                                  void *stream) {
-    return infllm_attn_merge2(d_o_part, d_lse_part, P, nullptr, nullptr, 0, B, H, Lq, d_out, o_sb, o_sh, o_sl, d_lse, stream);
+    return infllm_attn_merge2(d_o_part, d_lse_part, P, nullptr, nullptr, 0, B, H, Lq, d_out, o_sb, o_sh, o_sl, d_lse, stream, kD);
+}
+
+extern "C" int infllm_attn_merge_pair(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2, const float *d_lse_part2,
+                                      int32_t P2, int32_t B, int32_t H, int32_t Lq, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse,
+                                      void *stream) {
+    return infllm_attn_merge2(d_o_part, d_lse_part, P1, d_o_part2, d_lse_part2, P2, B, H, Lq, d_out, o_sb, o_sh, o_sl, d_lse, stream, kD);
+}
+
+// library-internal: a linear stage and (sinks != NULL) the rows of a second source under the complement mask, under one
+// softmax, as rows of `dim` elements (128 or 64) in the caller's layout; local->nsplit key splits of the joint tile list,
+// with partial rows at local->d_o_part / d_lse_part when there is more than one
+int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, int32_t dim, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
+                       void *stream) {
+    INFLLM_REQUIRE(local && d_out && (dim == 128 || dim == 64), "attn_window: bad arguments");
+    int rc = check_common(local);
+    if (rc) return rc;
+    rc = check_linear_stage(local);
+    if (rc) return rc;
+    if (sinks) {
+        INFLLM_REQUIRE(sinks->d_q && sinks->d_k && sinks->d_v && sinks->j_lo == 0 && sinks->j_hi >= 0 && sinks->k_sl == dim && sinks->v_sl == dim,
+                       "attn_window: bad sink rows");
+        INFLLM_REQUIRE(sinks->q_sl == local->q_sl && sinks->q_sh == local->q_sh && sinks->q_sb == local->q_sb && sinks->Lq == local->Lq,
+                       "attn_window: the two stages disagree");
+    }
+    StageOut so;
+    if (local->nsplit == 1) {
+        so.out = (bf16_t *)d_out;
+        so.o_sb = o_sb; so.o_sh = o_sh; so.o_sl = o_sl;
+    } else
+        INFLLM_REQUIRE(local->d_o_part && local->d_lse_part, "attn_window: splits without partial rows");
+    const int mode = sinks ? kSinks : kLinear;
+    rc = dim == 128 ? launch_stage<128>(mode, local, sinks, stream, nullptr, so) : launch_stage<64>(mode, local, sinks, stream, nullptr, so);
+    if (rc || local->nsplit == 1) return rc;
+    return infllm_attn_merge2(local->d_o_part, local->d_lse_part, local->nsplit, nullptr, nullptr, 0, local->B, local->H, local->Lq, d_out, o_sb, o_sh, o_sl,
+                              nullptr, stream, dim);
 }

@@ -84,15 +84,17 @@ struct MergeJob {
     PartSets ps;
 };
 
-// thread e of the merge: (row, 8 dims) = (e / 16, e % 16).  (inf_llm/attention/dot_production_attention/torch_impl.py:15-36)
+// thread e of the merge: (row, 8 dims) = (e / 16, e % 16) for rows of 128 elements, (e / 8, e % 8) for rows of 64.  (inf_llm/attention/dot_production_attention/torch_impl.py:15-36)
+template <int D = kD>
 __device__ __forceinline__ void merge_piece(const MergeJob &mj, int64_t e) {
     const _Float16 *o_part = mj.o_part;
     const float *lse_part = mj.lse_part;
     const PartSets ps = mj.ps;
     const int P = mj.P, H = mj.H, Lq = mj.Lq;
     const int64_t rows = (int64_t)mj.B * H * Lq;
-    const int64_t row = e >> 4;
-    const int c = (int)(e & 15);
+    constexpr int kPieces = D / 8;
+    const int64_t row = e / kPieces;
+    const int c = (int)(e % kPieces);
     if (row >= rows) return;
     // partials in batches of 8 so that the loads of a batch are in flight together (decode-sized blocks merge
     // dozens of partials of very few rows: a chain of dependent loads would be all latency)
@@ -116,7 +118,7 @@ __device__ __forceinline__ void merge_piece(const MergeJob &mj, int64_t e) {
             for (int i = 0; i < 8; ++i) {
                 const bool on = p0 + i < P;
                 l8[i] = on ? lse_part[ps.l(p0 + i, rows) + row] : -INFINITY;
-                o8[i] = on ? *(const f16x8 *)(o_part + (ps.l(p0 + i, rows) + row) * kD + ps.o(p0 + i) + c * 8) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+                o8[i] = on ? *(const f16x8 *)(o_part + (ps.l(p0 + i, rows) + row) * D + ps.o(p0 + i) + c * 8) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
             }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {

@@ -1,0 +1,283 @@
+// Attention of ONE query per head over a list of key ranges: the decode step of every attention type
+// (inf_llm/attention/dot_production_attention/torch_impl.py:39-96 for one query; stages joined by the merge).
+//
+// One query per head makes the step a read of K and V (2 FLOP per byte): bound by HBM, or for short ranges by the
+// latency of two dependent round trips.  So nothing is staged: every wave streams blocks of 16 keys of one kv head
+// straight from memory into registers, the next block's rows in flight while the current one is used, and the query
+// heads that share the kv head (up to four) are handled together, so that K and V are read once for all of them.
+//   S[key, head] = K . q^T by v_mfma_f32_16x16x32_bf16 (keys as rows, heads as columns): lane (head = lane & 15, row group
+//   rg = lane >> 4) receives the logits of keys 4 * rg + 0..3 of its head;
+//   the softmax runs per lane over those (its own running maximum and sum, no exchange between lanes);
+//   O[head, d] += p[key] * v[key, d] on the vector units in fp32: a row group reads its own four keys' value rows
+//   (16 lanes x 16 bytes), and a head's probability reaches the row's lanes by a DPP row broadcast.
+// The states of all row groups and waves are joined through LDS at the end, the splits by the merge kernels.
+// 32,768 keys x 8 kv heads (134 MB): 648 us with the tile kernel of attn.hip at one split, 33 us here.
+#include "decode.h"
+
+#include <type_traits>
+
+namespace {
+
+constexpr int kDecWaves = 4;
+constexpr float kLazyDec = 8.f;                    // the running maximum may lag the true one by 2^8
+
+template <int N>
+__device__ __forceinline__ float row_bcast(float x) {      // lane N of every row of 16 lanes, to the whole row
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x150 + N, 0xf, 0xf, true));
+}
+
+template <int NG, int H0 = 0, typename F>
+__device__ __forceinline__ void each_head(F &&f) {
+    if constexpr (H0 < NG) {
+        f(std::integral_constant<int, H0>{});
+        each_head<NG, H0 + 1>(f);
+    }
+}
+
+// D: head dimension (128 or 64); NG: query heads handled together (columns of the MFMA; heads beyond the group's last are
+// zero queries whose results are not written)
+template <int D, int NG, bool LOGITS>
+__global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(DecodeJob j) {
+    constexpr int KK = D / 32;                     // k-steps of the first MFMA
+    constexpr int LPR = D / 8;                     // lanes that hold a value row, 16 bytes each
+    constexpr int VL = kDecodeBlock * LPR / 64;    // value loads per block: 4 (D = 128) or 2 (D = 64)
+    constexpr int GRP = 64 / LPR;                  // value rows of one load: one (D = 128) or two (D = 64) per row group
+    __shared__ float red[kDecWaves][GRP][NG][D];
+    __shared__ float sm[kDecWaves][4][NG], sl[kDecWaves][4][NG];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int col = lane & 15, rg = lane >> 4;
+    const int G = j.H / j.Hkv, chunks = (G + NG - 1) / NG;
+    const int split = blockIdx.x, g = blockIdx.y / chunks, c = blockIdx.y % chunks, b = blockIdx.z;
+    const int h0 = g * G + c * NG, nh = min(NG, G - c * NG);
+    const float scale = j.scale * 1.4426950408889634f;
+    const float lazy = kLazyDec / scale;
+
+    // ---- the list of blocks: every range rounded up to whole blocks (units: every unit by itself)
+    int n_blocks = 0;
+    for (int s = 0; s < j.n_seg; ++s) n_blocks += (j.seg[s].rows + kDecodeBlock - 1) / kDecodeBlock * (j.seg[s].ids ? j.seg[s].n_ids : 1);
+    const int b_lo = (int)((int64_t)n_blocks * split / gridDim.x), b_hi = (int)((int64_t)n_blocks * (split + 1) / gridDim.x);
+
+    struct Block {
+        const bf16_t *k, *v;
+        int valid, q, row;                         // rows of the block, which query, first row (ranges) or -1
+    };
+    auto find = [&](int blk) {                     // wave-uniform
+        Block r{nullptr, nullptr, 0, 0, -1};
+        for (int s = 0; s < j.n_seg; ++s) {
+            const DecodeSeg &sg = j.seg[s];
+            const int per = (sg.rows + kDecodeBlock - 1) / kDecodeBlock, n = sg.ids ? per * sg.n_ids : per;
+            if (blk >= n) {
+                blk -= n;
+                continue;
+            }
+            r.q = sg.q;
+            if (sg.ids) {
+                const int i = blk / per, r0 = (blk - i * per) * kDecodeBlock;
+                const int u = __builtin_amdgcn_readfirstlane(sg.ids[(int64_t)b * sg.n_ids + i]);
+                const int ch = u / j.per_chunk;
+                const bf16_t *base = (const bf16_t *)(uintptr_t)j.chunk[ch] + (int64_t)(u - ch * j.per_chunk) * j.unit_elems + (int64_t)b * j.row_elems +
+                                     (int64_t)g * j.unit_sh + (int64_t)r0 * D;
+                r.k = base;
+                r.v = base + j.unit_v_off;
+                r.valid = min(kDecodeBlock, sg.rows - r0);
+            } else {
+                const int r0 = blk * kDecodeBlock;
+                r.k = sg.k + (int64_t)b * sg.k_sb + (int64_t)g * sg.k_sh + (int64_t)r0 * D;
+                r.v = sg.v + (int64_t)b * sg.v_sb + (int64_t)g * sg.v_sh + (int64_t)r0 * D;
+                r.valid = min(kDecodeBlock, sg.rows - r0);
+                if (s == 0) r.row = r0;
+            }
+            return r;
+        }
+        return r;
+    };
+
+    u32x4 kbuf[2][KK], vbuf[2][VL];
+    auto load = [&](const Block &bl, int buf) {    // rows beyond the range: its last row again, masked below
+        const bf16_t *kr = bl.k + min(col, bl.valid - 1) * D + rg * 8;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) kbuf[buf][kk] = __builtin_nontemporal_load((const u32x4 *)(kr + kk * 32));
+#pragma unroll
+        for (int i = 0; i < VL; ++i) {
+            const int key = D == 128 ? 4 * rg + i : 4 * rg + 2 * i + (col >> 3);
+            vbuf[buf][i] = __builtin_nontemporal_load((const u32x4 *)(bl.v + min(key, bl.valid - 1) * D + (lane & (LPR - 1)) * 8));
+        }
+    };
+
+    bf16x8 qreg[KK];
+    auto load_q = [&](int which) {
+        const bf16_t *q = j.q[which] + (int64_t)b * j.q_sb + (int64_t)(h0 + min(col, nh - 1)) * j.q_sh + rg * 8;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+            const u32x4 raw = *(const u32x4 *)(q + kk * 32);
+            qreg[kk] = __builtin_bit_cast(bf16x8, col < nh ? raw : u32x4{0, 0, 0, 0});
+        }
+    };
+
+    float m = -INFINITY, l = 0.f, neg_ms = 0.f;
+    float acc[NG][8];
+#pragma unroll
+    for (int h = 0; h < NG; ++h)
+#pragma unroll
+        for (int d = 0; d < 8; ++d) acc[h][d] = 0.f;
+
+    auto step = [&](const Block &bl, int buf) {
+        f32x4 s{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kbuf[buf][kk]), qreg[kk], s, 0, 0, 0);
+        if (LOGITS && bl.row >= 0 && col < nh) {
+            float *dst = j.logits + ((int64_t)b * j.H + h0 + col) * j.logit_stride + bl.row + 4 * rg;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (4 * rg + r < bl.valid) dst[r] = s[r] * scale;
+        }
+        if (bl.valid < kDecodeBlock) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[r] = 4 * rg + r < bl.valid ? s[r] : -INFINITY;
+        }
+        const float t = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+        const bool moved = t > m + lazy;
+        if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+            const float mn = moved ? t : m;
+            const float al = moved ? __builtin_amdgcn_exp2f((m - mn) * scale) : 1.f;
+            l *= al;
+            each_head<NG>([&](auto hc) {
+                constexpr int h = decltype(hc)::value;
+                const float a = row_bcast<h>(al);
+#pragma unroll
+                for (int d = 0; d < 8; ++d) acc[h][d] *= a;
+            });
+            m = mn;
+            neg_ms = m == -INFINITY ? 0.f : -m * scale;
+        }
+        float p[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale, neg_ms));
+        l += (p[0] + p[1]) + (p[2] + p[3]);
+#pragma unroll
+        for (int i = 0; i < VL; ++i) {
+            float v[8];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) v[2 * w] = bf16_bits_to_f32(vbuf[buf][i][w] & 0xffffu), v[2 * w + 1] = __uint_as_float(vbuf[buf][i][w] & 0xffff0000u);
+            each_head<NG>([&](auto hc) {
+                constexpr int h = decltype(hc)::value;
+                float pb;
+                if constexpr (D == 128) pb = row_bcast<h>(p[i]);
+                else {
+                    const float lo = row_bcast<h>(p[2 * i]), hi = row_bcast<h>(p[2 * i + 1]);
+                    pb = (col >> 3) ? hi : lo;
+                }
+#pragma unroll
+                for (int d = 0; d < 8; ++d) acc[h][d] = __builtin_fmaf(pb, v[d], acc[h][d]);
+            });
+        }
+    };
+
+    int q_now = -1, blk = b_lo + wave;
+    if (blk < b_hi) {
+        Block cur = find(blk);
+        load(cur, 0);
+        load_q(cur.q);
+        q_now = cur.q;
+        for (int buf = 0; blk < b_hi; blk += 2 * kDecWaves) {        // two blocks per turn, so that the buffers are fixed registers
+            Block nxt{};
+            const bool more = blk + kDecWaves < b_hi;
+            if (more) {
+                nxt = find(blk + kDecWaves);
+                load(nxt, 1);
+            }
+            if (cur.q != q_now) load_q(q_now = cur.q);
+            step(cur, 0);
+            if (!more) break;
+            if (blk + 2 * kDecWaves < b_hi) {
+                cur = find(blk + 2 * kDecWaves);
+                load(cur, 0);
+            }
+            if (nxt.q != q_now) load_q(q_now = nxt.q);
+            step(nxt, 1);
+        }
+    }
+
+    // ---- join the row groups and waves
+    if (col < NG) {
+        sm[wave][rg][col] = m;
+        sl[wave][rg][col] = l;
+    }
+    __syncthreads();
+    const int vg = lane / LPR;                     // this lane's group of value rows: its own row group, or half of it
+    each_head<NG>([&](auto hc) {
+        constexpr int h = decltype(hc)::value;
+        float mx = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < kDecWaves; ++w)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sm[w][r][h]);
+        const float own = sm[wave][rg][h];
+        const float f = own == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((own - mx) * scale);
+        float *dst = &red[wave][vg][h][(lane & (LPR - 1)) * 8];
+        *(f32x4 *)dst = f32x4{acc[h][0] * f, acc[h][1] * f, acc[h][2] * f, acc[h][3] * f};
+        *(f32x4 *)(dst + 4) = f32x4{acc[h][4] * f, acc[h][5] * f, acc[h][6] * f, acc[h][7] * f};
+    });
+    __syncthreads();
+    for (int e = threadIdx.x; e < nh * D; e += kDecWaves * kWave) {
+        const int h = e / D, d = e % D;
+        float mx = -INFINITY, den = 0.f, o = 0.f;
+#pragma unroll
+        for (int w = 0; w < kDecWaves; ++w)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sm[w][r][h]);
+#pragma unroll
+        for (int w = 0; w < kDecWaves; ++w)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) den += sm[w][r][h] == -INFINITY ? 0.f : sl[w][r][h] * __builtin_amdgcn_exp2f((sm[w][r][h] - mx) * scale);
+#pragma unroll
+        for (int w = 0; w < kDecWaves; ++w)
+#pragma unroll
+            for (int r = 0; r < GRP; ++r) o += red[w][r][h][d];
+        const int64_t row = ((int64_t)split * j.B + b) * j.H + h0 + h;
+        ((_Float16 *)j.o_part)[row * D + d] = (_Float16)(den > 0.f ? o / den : 0.f);
+        if (d == 0) j.lse_part[row] = den > 0.f ? mx * scale + log2f(den) : -INFINITY;
+    }
+}
+
+template <int D, bool LOGITS>
+int launch(const DecodeJob *job, void *stream) {
+    const int G = job->H / job->Hkv;
+    const int NG = G >= 3 ? 4 : G;
+    const dim3 grid(job->nsplit, job->Hkv * ((G + NG - 1) / NG), job->B);
+    if (NG == 1) hipLaunchKernelGGL((decode_attn_kernel<D, 1, LOGITS>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
+    else if (NG == 2) hipLaunchKernelGGL((decode_attn_kernel<D, 2, LOGITS>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
+    else hipLaunchKernelGGL((decode_attn_kernel<D, 4, LOGITS>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
+    INFLLM_CHECK_LAUNCH("decode_attn");
+    return 0;
+}
+
+}  // namespace
+
+// Key splits of a decode step over `blocks` blocks of 16 keys: two workgroups per CU where there are blocks for them (a
+// wave then has one or two blocks of its own in flight), never fewer than one block per wave, at most max_splits.
+int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int64_t blocks, int32_t max_splits) {
+    const int G = H / Hkv, NG = G >= 3 ? 4 : G;
+    const int64_t wgs = (int64_t)B * Hkv * ((G + NG - 1) / NG);
+    int64_t s = (2 * 256 + wgs - 1) / wgs;
+    if (s > blocks / kDecWaves) s = blocks / kDecWaves;
+    if (s > max_splits) s = max_splits;
+    return s < 1 ? 1 : (int)s;
+}
+
+int infllm_decode_attn(const DecodeJob *job, int32_t dim, void *stream) {
+    INFLLM_REQUIRE(job && job->q[0] && job->q[1] && job->o_part && job->lse_part, "decode_attn: null pointer");
+    INFLLM_REQUIRE(job->B > 0 && job->H > 0 && job->Hkv > 0 && job->H % job->Hkv == 0 && job->B <= 65535, "decode_attn: bad geometry B=%d H=%d Hkv=%d", job->B,
+                   job->H, job->Hkv);
+    INFLLM_REQUIRE(job->n_seg >= 1 && job->n_seg <= kDecodeSegs && job->nsplit >= 1 && job->nsplit <= 128, "decode_attn: %d ranges, %d splits", job->n_seg,
+                   job->nsplit);
+    for (int s = 0; s < job->n_seg; ++s) {
+        const DecodeSeg &sg = job->seg[s];
+        INFLLM_REQUIRE(sg.rows >= 0 && (sg.q == 0 || sg.q == 1), "decode_attn: bad range");
+        if (sg.ids) INFLLM_REQUIRE(job->chunk && job->per_chunk > 0 && sg.n_ids >= 0, "decode_attn: units without an arena");
+        else INFLLM_REQUIRE(sg.rows == 0 || (sg.k && sg.v), "decode_attn: null range");
+    }
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "decode_attn: head_dim %d", dim);
+    if (job->logits) return dim == 128 ? launch<128, true>(job, stream) : launch<64, true>(job, stream);
+    return dim == 128 ? launch<128, false>(job, stream) : launch<64, false>(job, stream);
+}

@@ -1,53 +1,22 @@
 // Prologue of the streaming path: RoPE of new tokens and their staging into the
 // per-layer rings (inf_llm/attention/rope.py:89-112,
 // inf_llm/attention/context_manager.py:719-747, 373-375).
-#include "common.h"
+#include "rope.h"
 
 namespace {
 
-constexpr int kPosPerBlock = 16;   // stream positions handled by one workgroup
 constexpr int kHalf = kD / 2;      // 64 rotation pairs per head
-
-struct Rot8 {
-    u32x4 lo, hi;
-};
-
-// rotate 8 pairs (lo[i], hi[i]) by (c[i], s[i]); fp32 math, one rounding to bf16.  `raw` (optional) receives the 16
-// rotated values before that rounding: lo pairs first, then hi pairs.
-__device__ __forceinline__ Rot8 rotate8(u32x4 xlo, u32x4 xhi, const float2 *cs, float *raw = nullptr) {
-    Rot8 r;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        float a0 = bf16_bits_to_f32(xlo[w] & 0xffffu), a1 = bf16_bits_to_f32(xlo[w] >> 16);
-        float b0 = bf16_bits_to_f32(xhi[w] & 0xffffu), b1 = bf16_bits_to_f32(xhi[w] >> 16);
-        float2 c0 = cs[2 * w], c1 = cs[2 * w + 1];
-        // x*cos + rotate_half(x)*sin, rotate_half = (-hi, lo)
-        const float l0 = a0 * c0.x - b0 * c0.y, l1 = a1 * c1.x - b1 * c1.y;
-        const float h0 = b0 * c0.x + a0 * c0.y, h1 = b1 * c1.x + a1 * c1.y;
-        r.lo[w] = pack_bf16x2(l0, l1);
-        r.hi[w] = pack_bf16x2(h0, h1);
-        if (raw) {
-            raw[2 * w] = l0, raw[2 * w + 1] = l1;
-            raw[8 + 2 * w] = h0, raw[8 + 2 * w + 1] = h1;
-        }
-    }
-    return r;
-}
 
 // grid = (position tiles of 16, batch rows, kv heads): a workgroup rotates the query heads of one
 // kv-head group plus that group's key head, copies its value head, and leaves the sum of its
 // rotated-to-one-position queries over its positions in d_qpart (for the block's mean query; summed
 // before the rounding to bf16, so the mean query carries no rounding of its own).
 //
-// Angles.  cos / sin of (position x frequency) are needed for 16 positions x 64 frequencies per workgroup.
-// Only the workgroup's FIRST position and the step of one position are evaluated (fp64 sincos, one call
-// per thread for 128 threads); the other 15 positions follow by the angle-addition recurrence in fp64,
-// whose error after 15 steps is a few 1e-16 - far below the fp32 value the rotation consumes.  The rows
-// the workgroup will rotate are requested from memory BEFORE that arithmetic, so the two overlap.
+// Angles (rope_angles): the rows the workgroup will rotate are requested from memory BEFORE that arithmetic, so the
+// two overlap.
 __global__ __launch_bounds__(256) void ingest_kernel(infllm_ingest_args a) {
     __shared__ float2 cs_pos[kPosPerBlock][kHalf];
     __shared__ float2 cs_glb[kHalf];
-    __shared__ double2 cs_step[kHalf];                // (cos, sin) of one position's step per frequency
     __shared__ float red[4][kPosPerBlock][kD];        // q_glb of 4 heads x 16 positions, for the partial sums
     const int tid = threadIdx.x;
     const int b = blockIdx.y, g = blockIdx.z;
@@ -88,30 +57,7 @@ __global__ __launch_bounds__(256) void ingest_kernel(infllm_ingest_args a) {
     if (tid < np * 16) v_row = *(const u32x4 *)(v + (int64_t)(p0 + (tid >> 4)) * a.v_sl + (tid & 15) * 8);
 
     // ---- angles
-    if (tid < kHalf) {
-        const double w = a.distance_scale * (double)a.d_inv_freq[tid];
-        double s, c;
-        sincos((double)(a.pos0 + p0) * w, &s, &c);
-        cs_pos[0][tid] = make_float2((float)c, (float)s);
-        cs_step[tid] = make_double2(c, s);            // parked here until the step values arrive
-    } else if (tid < 2 * kHalf) {
-        const int f = tid - kHalf;
-        double s, c;
-        sincos((double)a.glb_pos * a.distance_scale * (double)a.d_inv_freq[f], &s, &c);
-        cs_glb[f] = make_float2((float)c, (float)s);
-    }
-    double2 step = make_double2(1.0, 0.0);
-    if (tid < kHalf) {
-        double s, c;
-        sincos(a.distance_scale * (double)a.d_inv_freq[tid], &s, &c);
-        step = make_double2(c, s);
-        double2 cur = cs_step[tid];
-        for (int p = 1; p < kPosPerBlock; ++p) {      // (cos, sin)(x + w) from (cos, sin)(x)
-            const double c2 = cur.x * step.x - cur.y * step.y, s2 = cur.y * step.x + cur.x * step.y;
-            cur = make_double2(c2, s2);
-            cs_pos[p][tid] = make_float2((float)c2, (float)s2);
-        }
-    }
+    rope_angles<kHalf>(a.pos0 + p0, np, a.glb_pos, a.distance_scale, a.d_inv_freq, cs_pos, cs_glb);
     __syncthreads();
 
     // query heads of the group, 4 at a time: 8 threads per (head, position) row

@@ -1,0 +1,336 @@
+// One call of an attention type with a plain cache - attention sinks + sliding window (inf_llm/attention/stream_llm.py:6-111,
+// infinite_lm.py:6-100) or causal attention (origin.py:4-79) - in two or three launches: the new tokens' rows (rotary
+// embedding, cache), the attention, and the merge of its key splits where it has any.
+#include <algorithm>
+
+#include "decode.h"
+#include "rope.h"
+
+int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, int32_t dim, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
+                       void *stream);
+int infllm_attn_merge2(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2, const float *d_lse_part2,
+                       int32_t P2, int32_t B, int32_t H, int32_t Lq, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse,
+                       void *stream, int32_t dim);
+
+namespace {
+
+// rows [0, n) of a source to a destination, for every (batch row, kv head); rows are D elements apart on both sides
+struct RowCopy {
+    const bf16_t *src;
+    bf16_t *dst;
+    int64_t s_sb, s_sh, d_sb, d_sh;
+    int32_t n;
+};
+constexpr int kCopies = 6;
+constexpr int kCopyRows = 64;                  // rows a copying workgroup moves
+
+struct StageJob {
+    const bf16_t *q, *k, *v;                   // new rows
+    int64_t q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;
+    int32_t B, H, Hkv, n;                      // n: rows of the q (or k / v) part
+    int32_t do_q, do_kv;
+    int64_t pos0, glb_pos;                     // position of row 0; the one angle of the sinks' queries
+    const float *inv_freq;
+    double distance_scale;
+    bf16_t *q_loc, *q_glb;                     // [B, H, n, D]; q_glb NULL: no sinks
+    bf16_t *dk, *dv;                           // where row 0 of head 0 goes, rotated / as it is
+    int64_t dk_sb, dk_sh, dv_sb, dv_sh;
+    bf16_t *raw;                               // where un-rotated row 0 goes, rows [0, n_raw)
+    int64_t raw_sb, raw_sh;
+    int32_t n_raw;
+    int32_t tiles;                             // workgroups along x that stage rows; the rest copy
+    RowCopy copy[kCopies];
+};
+
+// Bound by HBM for a prompt (a row read, one to three written), by the latency of the fp64 angles for a step.  grid =
+// (position tiles of 16, then pieces of the row copies; batch rows; kv heads): a workgroup rotates the query heads of a
+// kv head's group and its key head at 16 positions.  (One wave per row with its own sincos, a launch for every tensor and
+// angle, and torch.cat for the cache: 13 launches and 2.1 x the bytes per call.)
+template <int D>
+__global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
+    constexpr int HALF = D / 2, C2 = D / 16;           // chunk pairs of a row
+    __shared__ float2 cs_pos[kPosPerBlock][HALF];
+    __shared__ float2 cs_glb[HALF];
+    const int tid = threadIdx.x, b = blockIdx.y, g = blockIdx.z;
+    if ((int)blockIdx.x >= j.tiles) {
+        int piece = (int)blockIdx.x - j.tiles;
+        for (int c = 0; c < kCopies; ++c) {
+            const RowCopy &rc = j.copy[c];
+            const int n = (rc.n + kCopyRows - 1) / kCopyRows;
+            if (piece >= n) {
+                piece -= n;
+                continue;
+            }
+            const int r0 = piece * kCopyRows, m = min(kCopyRows, rc.n - r0) * (D / 8);
+            const u32x4 *src = (const u32x4 *)(rc.src + (int64_t)b * rc.s_sb + (int64_t)g * rc.s_sh + (int64_t)r0 * D);
+            u32x4 *dst = (u32x4 *)(rc.dst + (int64_t)b * rc.d_sb + (int64_t)g * rc.d_sh + (int64_t)r0 * D);
+            constexpr int U = kCopyRows * (D / 8) / 256;
+            u32x4 x[U];
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+                if (tid + 256 * i < m) x[i] = src[tid + 256 * i];
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+                if (tid + 256 * i < m) dst[tid + 256 * i] = x[i];
+            return;
+        }
+        return;
+    }
+    const int G = j.H / j.Hkv;
+    const int p0 = blockIdx.x * kPosPerBlock, np = min(kPosPerBlock, j.n - p0);
+    // ---- requests first: up to four query heads, the key head, the value head
+    constexpr int kItems = 4 * kPosPerBlock * C2 / 256;                  // 2 (D = 128) or 1 (D = 64)
+    u32x4 q_lo[kItems], q_hi[kItems], k_lo, k_hi, v_row;
+    const bf16_t *q = j.q + (int64_t)b * j.q_sb;
+    if (j.do_q) {
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            const int e = tid + i * 256, c = e % C2, p = e / C2 % kPosPerBlock, hl = e / C2 / kPosPerBlock;
+            if (hl < min(4, G) && p < np) {
+                const bf16_t *src = q + (int64_t)(g * G + hl) * j.q_sh + (int64_t)(p0 + p) * j.q_sl;
+                q_lo[i] = *(const u32x4 *)(src + c * 8);
+                q_hi[i] = *(const u32x4 *)(src + HALF + c * 8);
+            }
+        }
+    }
+    const int kc = tid % C2, kp = tid / C2, vc = tid % (D / 8), vp = tid / (D / 8);
+    if (j.do_kv) {
+        if (kp < np) {
+            const bf16_t *src = j.k + (int64_t)b * j.k_sb + (int64_t)g * j.k_sh + (int64_t)(p0 + kp) * j.k_sl;
+            k_lo = *(const u32x4 *)(src + kc * 8);
+            k_hi = *(const u32x4 *)(src + HALF + kc * 8);
+        }
+        if (vp < np) v_row = *(const u32x4 *)(j.v + (int64_t)b * j.v_sb + (int64_t)g * j.v_sh + (int64_t)(p0 + vp) * j.v_sl + vc * 8);
+    }
+    rope_angles<HALF>(j.pos0 + p0, np, j.glb_pos, j.distance_scale, j.inv_freq, cs_pos, cs_glb);
+    __syncthreads();
+    if (j.do_q) {
+        for (int hg0 = 0; hg0 < G; hg0 += 4) {
+#pragma unroll
+            for (int i = 0; i < kItems; ++i) {
+                const int e = tid + i * 256, c = e % C2, p = e / C2 % kPosPerBlock, hl = e / C2 / kPosPerBlock;
+                if (hl >= min(4, G - hg0) || p >= np) continue;
+                const int h = g * G + hg0 + hl;
+                u32x4 lo = q_lo[i], hi = q_hi[i];
+                if (hg0 > 0) {
+                    const bf16_t *src = q + (int64_t)h * j.q_sh + (int64_t)(p0 + p) * j.q_sl;
+                    lo = *(const u32x4 *)(src + c * 8), hi = *(const u32x4 *)(src + HALF + c * 8);
+                }
+                const int64_t o = (((int64_t)b * j.H + h) * j.n + p0 + p) * D;
+                Rot8 r = rotate8(lo, hi, &cs_pos[p][c * 8]);
+                *(u32x4 *)(j.q_loc + o + c * 8) = r.lo;
+                *(u32x4 *)(j.q_loc + o + HALF + c * 8) = r.hi;
+                if (j.q_glb) {
+                    r = rotate8(lo, hi, &cs_glb[c * 8]);
+                    *(u32x4 *)(j.q_glb + o + c * 8) = r.lo;
+                    *(u32x4 *)(j.q_glb + o + HALF + c * 8) = r.hi;
+                }
+            }
+        }
+    }
+    if (j.do_kv) {
+        if (kp < np) {
+            bf16_t *dst = j.dk + (int64_t)b * j.dk_sb + (int64_t)g * j.dk_sh + (int64_t)(p0 + kp) * D;
+            const Rot8 r = rotate8(k_lo, k_hi, &cs_pos[kp][kc * 8]);
+            *(u32x4 *)(dst + kc * 8) = r.lo;
+            *(u32x4 *)(dst + HALF + kc * 8) = r.hi;
+            if (p0 + kp < j.n_raw) {
+                bf16_t *raw = j.raw + (int64_t)b * j.raw_sb + (int64_t)g * j.raw_sh + (int64_t)(p0 + kp) * D;
+                *(u32x4 *)(raw + kc * 8) = k_lo;
+                *(u32x4 *)(raw + HALF + kc * 8) = k_hi;
+            }
+        }
+        if (vp < np) *(u32x4 *)(j.dv + (int64_t)b * j.dv_sb + (int64_t)g * j.dv_sh + (int64_t)(p0 + vp) * D + vc * 8) = v_row;
+    }
+}
+
+int launch_stage_rows(StageJob &j, int dim, void *stream) {
+    int pieces = 0;
+    for (const RowCopy &c : j.copy) pieces += (c.n + kCopyRows - 1) / kCopyRows;
+    j.tiles = j.do_q || j.do_kv ? (j.n + kPosPerBlock - 1) / kPosPerBlock : 0;
+    if (j.tiles + pieces == 0) return 0;
+    const dim3 grid(j.tiles + pieces, j.B, j.Hkv);
+    if (dim == 128) hipLaunchKernelGGL(stage_rows_kernel<128>, grid, dim3(256), 0, (hipStream_t)stream, j);
+    else hipLaunchKernelGGL(stage_rows_kernel<64>, grid, dim3(256), 0, (hipStream_t)stream, j);
+    INFLLM_CHECK_LAUNCH("stage_rows");
+    return 0;
+}
+
+}  // namespace
+
+// Key splits of a launch over `wgs` workgroups of `tiles` key tiles each.  A workgroup costs about 6 us to start and drain
+// plus 1.9 us per tile (a CU holds one), 256 of them run at a time, and splits cost a merge of 5 us; the smallest
+// estimate wins.  max_parts: splits that the partial rows have room for.
+int infllm_attn_splits(int64_t wgs, int64_t tiles, int32_t max_parts) {
+    int best = 1;
+    double best_us = 0;
+    for (int s = 1; s <= std::min(max_parts, 32) && (s == 1 || tiles / s >= 2); ++s) {
+        const int64_t rounds = (wgs * s + 255) / 256;
+        const double us = (double)rounds * (6.0 + 1.9 * (double)((tiles + s - 1) / s)) + (s > 1 ? 5.0 : 0.0);
+        if (s == 1 || us < best_us) best = s, best_us = us;
+    }
+    return best;
+}
+
+extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) {
+    INFLLM_REQUIRE(a != nullptr, "window_forward: null argument block");
+    INFLLM_REQUIRE(a->dim == 128 || a->dim == 64, "window_forward: head_dim %d is not 64 or 128", a->dim);
+    INFLLM_REQUIRE(a->B > 0 && a->H > 0 && a->Hkv > 0 && a->H % a->Hkv == 0 && a->B <= 65535 && a->Hkv <= 65535, "window_forward: bad geometry B=%d H=%d Hkv=%d",
+                   a->B, a->H, a->Hkv);
+    INFLLM_REQUIRE(a->n_q > 0 && a->n_new > 0 && a->kind >= 0 && a->kind <= 2 && a->n_init >= 0 && a->seen >= 0, "window_forward: bad sizes");
+    INFLLM_REQUIRE(a->d_q && a->d_k && a->d_v && a->d_inv_freq && a->d_cache_k && a->d_cache_v && a->d_work && a->d_out, "window_forward: null pointer");
+    INFLLM_REQUIRE(((a->q_sb | a->q_sh | a->q_sl | a->k_sb | a->k_sh | a->k_sl | a->v_sb | a->v_sh | a->v_sl | a->ok_sb | a->ok_sh | a->ov_sb | a->ov_sh |
+                     a->ck_sb | a->ck_sh | a->cv_sb | a->cv_sh | a->o_sb | a->o_sh | a->o_sl) & 7) == 0,
+                   "window_forward: strides must be multiples of 8 elements");
+    const bool causal = a->kind == 0, inplace = a->d_old_k == a->d_cache_k && a->rows_old > 0;
+    const int64_t rows_all = (int64_t)a->rows_old + a->n_new, len_k = a->seen + a->n_new;
+    const bool cut = a->rows_new < rows_all;
+    INFLLM_REQUIRE(a->rows_old >= 0 && a->rows_new > 0 && a->rows_new <= rows_all && (a->rows_old == 0 || (a->d_old_k && a->d_old_v)), "window_forward: bad cache rows");
+    INFLLM_REQUIRE(a->rows_old <= a->seen && a->n_q <= rows_all, "window_forward: more cached rows or queries than tokens");
+    INFLLM_REQUIRE(!cut || (!causal && a->rows_new >= a->n_init && a->rows_new - a->n_init >= std::min<int64_t>(a->n_local, rows_all)), "window_forward: cut cache too short");
+    INFLLM_REQUIRE(!cut || a->d_all_k || (a->n_q == 1 && a->n_new == 1), "window_forward: a cut cache does not hold what several queries see");
+    INFLLM_REQUIRE(!inplace || (!cut && a->ok_sb == a->ck_sb && a->ok_sh == a->ck_sh && a->d_old_v == a->d_cache_v && a->ov_sb == a->cv_sb && a->ov_sh == a->cv_sh),
+                   "window_forward: in place needs the same strides and an uncut cache");
+    INFLLM_REQUIRE((a->d_all_k != nullptr) == (a->d_all_v != nullptr), "window_forward: all_k without all_v");
+    INFLLM_REQUIRE(a->softmax_scale > 0.f, "window_forward: softmax scale");
+    const int D = a->dim;
+    const int64_t q_elems = (int64_t)a->B * a->H * a->n_q * D;
+    const bool sink_stage = !causal && len_k > a->n_local && a->n_init > 0;
+    const int n_sink = sink_stage ? (int)std::min<int64_t>(a->n_init, rows_all) : 0;
+    INFLLM_REQUIRE(!sink_stage || a->kind != 2 || (a->d_raw && a->raw_new >= n_sink), "window_forward: un-rotated sinks missing");
+    const int64_t q_bytes = (causal ? 1 : 2) * q_elems * 2;
+    INFLLM_REQUIRE(a->work_bytes >= q_bytes, "window_forward: scratch of %lld bytes for %lld", (long long)a->work_bytes, (long long)q_bytes);
+    bf16_t *q_loc = (bf16_t *)a->d_work, *q_sink = causal ? nullptr : q_loc + q_elems;
+
+    // ---- where the attention reads its keys: everything, or the new cache
+    const bool all = a->d_all_k != nullptr;
+    bf16_t *bk = (bf16_t *)(all ? a->d_all_k : a->d_cache_k), *bv = (bf16_t *)(all ? a->d_all_v : a->d_cache_v);
+    const int64_t bk_sh = all ? rows_all * D : a->ck_sh, bk_sb = all ? bk_sh * a->Hkv : a->ck_sb;
+    const int64_t bv_sh = all ? rows_all * D : a->cv_sh, bv_sb = all ? bv_sh * a->Hkv : a->cv_sb;
+    const int64_t rows_base = all ? rows_all : a->rows_new;
+
+    StageJob j{};
+    j.B = a->B; j.H = a->H; j.Hkv = a->Hkv;
+    j.q = (const bf16_t *)a->d_q; j.k = (const bf16_t *)a->d_k; j.v = (const bf16_t *)a->d_v;
+    j.q_sb = a->q_sb; j.q_sh = a->q_sh; j.q_sl = a->q_sl;
+    j.k_sb = a->k_sb; j.k_sh = a->k_sh; j.k_sl = a->k_sl;
+    j.v_sb = a->v_sb; j.v_sh = a->v_sh; j.v_sl = a->v_sl;
+    j.glb_pos = a->kind == 2 ? a->n_local - 1 : a->n_local + a->n_init - 1;
+    j.inv_freq = a->d_inv_freq; j.distance_scale = a->distance_scale;
+    j.q_loc = q_loc; j.q_glb = sink_stage ? q_sink : nullptr;
+    j.dk = bk + (rows_base - a->n_new) * D; j.dv = bv + (rows_base - a->n_new) * D;
+    j.dk_sb = bk_sb; j.dk_sh = bk_sh; j.dv_sb = bv_sb; j.dv_sh = bv_sh;
+    const int64_t raw_sh = (int64_t)a->raw_new * D;
+    if (a->raw_new > a->raw_old) {
+        INFLLM_REQUIRE(a->d_raw && a->raw_old == a->seen && a->raw_new - a->raw_old <= a->n_new && (a->raw_old == 0 || a->d_raw_old), "window_forward: bad sink rows");
+        j.raw = (bf16_t *)a->d_raw + (int64_t)a->raw_old * D;
+        j.raw_sh = raw_sh; j.raw_sb = raw_sh * a->Hkv;
+        j.n_raw = a->raw_new - a->raw_old;
+    }
+    int nc = 0;
+    auto copy = [&](const void *src, int64_t ss_b, int64_t ss_h, int64_t s_row, void *dst, int64_t ds_b, int64_t ds_h, int64_t d_row, int64_t n) {
+        if (n > 0) j.copy[nc++] = RowCopy{(const bf16_t *)src + s_row * D, (bf16_t *)dst + d_row * D, ss_b, ss_h, ds_b, ds_h, (int32_t)n};
+    };
+    if (all || !cut) {
+        if (!inplace) {
+            copy(a->d_old_k, a->ok_sb, a->ok_sh, 0, bk, bk_sb, bk_sh, 0, a->rows_old);
+            copy(a->d_old_v, a->ov_sb, a->ov_sh, 0, bv, bv_sb, bv_sh, 0, a->rows_old);
+        }
+    } else {                                    // one new row: the sinks, and the tail without its oldest rows
+        const int64_t tail = a->rows_new - a->n_init - a->n_new, from = a->rows_old - tail;
+        copy(a->d_old_k, a->ok_sb, a->ok_sh, 0, bk, bk_sb, bk_sh, 0, a->n_init);
+        copy(a->d_old_v, a->ov_sb, a->ov_sh, 0, bv, bv_sb, bv_sh, 0, a->n_init);
+        copy(a->d_old_k, a->ok_sb, a->ok_sh, from, bk, bk_sb, bk_sh, a->n_init, tail);
+        copy(a->d_old_v, a->ov_sb, a->ov_sh, from, bv, bv_sb, bv_sh, a->n_init, tail);
+    }
+    if (j.n_raw > 0 && a->raw_old > 0)
+        copy(a->d_raw_old, (int64_t)a->raw_old * D * a->Hkv, (int64_t)a->raw_old * D, 0, a->d_raw, raw_sh * a->Hkv, raw_sh, 0, a->raw_old);
+    int rc;
+    if (a->n_q == a->n_new) {
+        j.do_q = j.do_kv = 1;
+        j.n = a->n_q;
+        j.pos0 = a->seen;
+        rc = launch_stage_rows(j, D, stream);
+        if (rc) return rc;
+    } else {                                    // queries and keys at different positions: a launch for each
+        j.do_kv = 1;
+        j.n = a->n_new;
+        j.pos0 = a->seen;
+        rc = launch_stage_rows(j, D, stream);
+        if (rc) return rc;
+        j.do_q = 1;
+        j.do_kv = 0;
+        j.n = a->n_q;
+        j.pos0 = len_k - a->n_q;
+        for (RowCopy &c : j.copy) c.n = 0;
+        rc = launch_stage_rows(j, D, stream);
+        if (rc) return rc;
+    }
+    if (all) {                                  // the new cache out of everything: all of it, or the sinks and the tail
+        StageJob c{};
+        c.B = a->B; c.H = a->H; c.Hkv = a->Hkv;
+        const int64_t head = cut ? a->n_init : a->rows_new, tail = a->rows_new - head;
+        c.copy[0] = RowCopy{bk, (bf16_t *)a->d_cache_k, bk_sb, bk_sh, a->ck_sb, a->ck_sh, (int32_t)head};
+        c.copy[1] = RowCopy{bv, (bf16_t *)a->d_cache_v, bv_sb, bv_sh, a->cv_sb, a->cv_sh, (int32_t)head};
+        c.copy[2] = RowCopy{bk + (rows_all - tail) * D, (bf16_t *)a->d_cache_k + head * D, bk_sb, bk_sh, a->ck_sb, a->ck_sh, (int32_t)tail};
+        c.copy[3] = RowCopy{bv + (rows_all - tail) * D, (bf16_t *)a->d_cache_v + head * D, bv_sb, bv_sh, a->cv_sb, a->cv_sh, (int32_t)tail};
+        rc = launch_stage_rows(c, D, stream);
+        if (rc) return rc;
+    }
+
+    // ---- attention
+    const int64_t rows_q = (int64_t)a->B * a->H * a->n_q;
+    const int64_t part_rows = (a->work_bytes - q_bytes) / (2 * D + 4);
+    int max_parts = (int)std::min<int64_t>(part_rows / rows_q, 64);
+    const bf16_t *sk = a->kind == 2 ? (const bf16_t *)a->d_raw : bk;
+    const int64_t sk_sh = a->kind == 2 ? raw_sh : bk_sh, sk_sb = a->kind == 2 ? raw_sh * a->Hkv : bk_sb;
+    const float scale = a->softmax_scale;
+    if (a->n_q == 1 && max_parts >= 1) {
+        DecodeJob d{};
+        d.q[0] = q_loc; d.q[1] = sink_stage ? q_sink : q_loc;
+        d.q_sb = (int64_t)a->H * D; d.q_sh = D;
+        d.B = a->B; d.H = a->H; d.Hkv = a->Hkv;
+        d.scale = scale;
+        const int64_t near = causal ? rows_base : std::min<int64_t>(rows_base, a->n_local);       // the last rows
+        d.seg[0] = DecodeSeg{bk + (rows_base - near) * D, bv + (rows_base - near) * D, bk_sb, bk_sh, bv_sb, bv_sh, (int32_t)near, 0, 0, nullptr};
+        d.n_seg = 1;
+        // sink j is seen from a distance of at least n_local: j <= position - n_local
+        const int64_t far = std::min<int64_t>(n_sink, len_k - a->n_local);
+        if (far > 0) d.seg[d.n_seg++] = DecodeSeg{sk, bv, sk_sb, sk_sh, bv_sb, bv_sh, (int32_t)far, 1, 0, nullptr};
+        const int64_t blocks = (near + kDecodeBlock - 1) / kDecodeBlock + (far > 0 ? (far + kDecodeBlock - 1) / kDecodeBlock : 0);
+        d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, blocks, max_parts);
+        d.o_part = (uint16_t *)((char *)a->d_work + q_bytes);
+        d.lse_part = (float *)((char *)a->d_work + q_bytes + part_rows * 2 * D);
+        rc = infllm_decode_attn(&d, D, stream);
+        if (rc) return rc;
+        return infllm_attn_merge2(d.o_part, d.lse_part, d.nsplit, nullptr, nullptr, 0, a->B, a->H, 1, a->d_out, a->o_sb, a->o_sh, a->o_sl, nullptr, stream, D);
+    }
+    infllm_attn_args l{}, s{};
+    l.d_q = q_loc;
+    l.q_sl = D; l.q_sh = (int64_t)a->n_q * D; l.q_sb = (int64_t)a->H * a->n_q * D;
+    l.B = a->B; l.H = a->H; l.Hkv = a->Hkv; l.Lq = a->n_q;
+    l.d_k = bk; l.d_v = bv;
+    l.k_sl = l.v_sl = D;
+    l.k_sh = bk_sh; l.k_sb = bk_sb; l.v_sh = bv_sh; l.v_sb = bv_sb;
+    l.cap = 1ll << 40;
+    l.mask = INFLLM_MASK_WINDOW;
+    l.offset = rows_base - a->n_q;
+    l.window = causal ? rows_base : a->n_local;
+    l.j_lo = std::max<int64_t>(0, rows_base - a->n_q - l.window + 1);
+    l.j_hi = rows_base;
+    l.softmax_scale = scale;
+    if (sink_stage) {
+        s = l;
+        s.d_q = q_sink;
+        s.d_k = sk; s.k_sh = sk_sh; s.k_sb = sk_sb;
+        s.j_lo = 0; s.j_hi = n_sink;
+        s.mask = INFLLM_MASK_COMPLEMENT;
+        s.offset = len_k - a->n_q; s.window = a->n_local;
+    }
+    const int64_t wgs = ((int64_t)((a->n_q + 31) / 32) * (a->H / a->Hkv) + 7) / 8 * a->Hkv * a->B;
+    const int64_t tiles = (std::min<int64_t>(l.window + 64, l.j_hi - l.j_lo) + kTile - 1) / kTile + (n_sink + kTile - 1) / kTile;
+    l.nsplit = infllm_attn_splits(wgs, tiles, max_parts);
+    l.d_o_part = (uint16_t *)((char *)a->d_work + q_bytes);
+    l.d_lse_part = (float *)((char *)a->d_work + q_bytes + part_rows * 2 * D);
+    return infllm_attn_window(&l, sink_stage ? &s : nullptr, D, a->d_out, a->o_sb, a->o_sh, a->o_sl, stream);
+}
