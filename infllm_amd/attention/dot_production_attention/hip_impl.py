@@ -8,7 +8,9 @@ values and sliding-window mask; ``end=True`` closes the joint softmax;
 ``get_result()`` returns the output and, per stage, the column sums of the
 final probabilities (or None).  Each stage is one launch of infllm_attn_stage
 that leaves a partial (o, lse); the merge kernel joins them, and the scores
-are computed afterwards from the final lse (infllm_local_score).  Scores are
+are computed afterwards from the final lse (infllm_local_score).  A stage of few
+queries is cut into as many key splits as fill the chip (infllm_attn_stage_splits),
+with partial rows for each.  Scores are
 returned in fp32.  Heads narrower than 128 are padded with zeros to the kernels'
 width (the softmax scale stays 1/sqrt of the real head_dim) and the result is cut
 back.
@@ -49,9 +51,7 @@ class HipMultiStageDotProductionAttention(MultiStageDotProductionAttention):
                 sliding_window = (len_k - Lq, sliding_window)
             offset, window = int(sliding_window[0]), int(sliding_window[1])
             mask = ops.MASK_COMPLEMENT if complement_sliding_window else ops.MASK_WINDOW
-        o_part = torch.empty((1, B, H, Lq, D), dtype=torch.float16, device=q.device)
-        lse_part = torch.empty((1, B, H, Lq), dtype=torch.float32, device=q.device)
-        ops.attn_stage_linear(q, k, v, o_part, lse_part, j_lo=0, j_hi=len_k, mask=mask, offset=offset, window=window, softmax_scale=scale)
+        o_part, lse_part = ops.attn_stage_split(q, k, v, j_lo=0, j_hi=len_k, mask=mask, offset=offset, window=window, softmax_scale=scale)
         self._o_parts.append(o_part)
         self._lse_parts.append(lse_part)
         self._stages.append((q, k, mask, offset, window, get_score, scale))
@@ -62,20 +62,20 @@ class HipMultiStageDotProductionAttention(MultiStageDotProductionAttention):
         self.end = True
         B, H, Lq, d = self.q_shape
         D = max(d, ops.HEAD_DIM)
-        P = len(self._stages)
-        o_all = torch.cat(self._o_parts, dim=0) if P > 1 else self._o_parts[0]
-        lse_all = torch.cat(self._lse_parts, dim=0) if P > 1 else self._lse_parts[0]
-        dev = o_all.device
+        dev = self._o_parts[0].device
+        if len(self._o_parts) > 2:                             # the merge takes two sets of partials
+            self._o_parts = [self._o_parts[0], torch.cat(self._o_parts[1:], dim=0)]
+            self._lse_parts = [self._lse_parts[0], torch.cat(self._lse_parts[1:], dim=0)]
         self.ret = torch.empty((B, H, Lq, D), dtype=torch.bfloat16, device=dev)
         self.lse = torch.empty((B, H, Lq), dtype=torch.float32, device=dev)
-        ops.attn_merge(o_all, lse_all, P, self.ret, self.lse)
+        ops.attn_merge_sets(self._o_parts, self._lse_parts, self.ret, self.lse)
         if d < D:
             self.ret = self.ret[..., :d].contiguous()
         for q, k, mask, offset, window, want, scale in self._stages:
             if not want:
                 self.score_list.append(None)
                 continue
-            score = torch.zeros((B, H, k.shape[2]), dtype=torch.float32, device=dev)
+            score = torch.empty((B, H, k.shape[2]), dtype=torch.float32, device=dev)       # every cell is written
             if k.shape[2] > 0:
                 ops.local_score(q, k, self.lse, score, j_lo=0, j_hi=k.shape[2], mask=mask, offset=offset,
                                 window=window, accumulate=False, softmax_scale=scale)

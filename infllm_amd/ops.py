@@ -142,6 +142,24 @@ def attn_stage_linear(q, k, v, o_part, lse_part, **kw):
     check(_lib.load().infllm_attn_stage(linear_stage_args(q, k, v, o_part, lse_part, **kw), _stream()), "infllm_attn_stage")
 
 
+def attn_stage_split(q, k, v, max_splits=64, **kw):
+    """One stage over a linear key source, cut into as many key splits as pay (infllm_attn_stage_splits); returns its
+    partials (o [splits,B,H,Lq,D] fp16, lse [splits,B,H,Lq] fp32)."""
+    B, H, Lq, D = q.shape
+    lib = _lib.load()
+    o_part = torch.empty((0,), dtype=torch.float16, device=q.device)
+    lse_part = torch.empty((0,), dtype=torch.float32, device=q.device)
+    a = linear_stage_args(q, k, v, o_part, lse_part, **kw)
+    n = lib.infllm_attn_stage_splits(a, max_splits)
+    if n < 1:
+        check(n, "infllm_attn_stage_splits")
+    o_part = torch.empty((n, B, H, Lq, D), dtype=torch.float16, device=q.device)
+    lse_part = torch.empty((n, B, H, Lq), dtype=torch.float32, device=q.device)
+    a.nsplit, a.d_o_part, a.d_lse_part = n, o_part.data_ptr(), lse_part.data_ptr()
+    check(lib.infllm_attn_stage(a, _stream()), "infllm_attn_stage")
+    return o_part, lse_part
+
+
 def attn_stage_paged(q, pages_dev, n_pages, Hkv, o_part, lse_part, **kw):
     """One stage over a device page table (see paged_stage_args)."""
     check(_lib.load().infllm_attn_stage(paged_stage_args(q, pages_dev, n_pages, Hkv, o_part, lse_part, **kw), _stream()),
@@ -179,6 +197,17 @@ def attn_merge(o_part, lse_part, P, out, lse):
     check(_lib.load().infllm_attn_merge(o_part.data_ptr(), lse_part.data_ptr(), P, B, H, Lq,
                                         out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
                                         lse.data_ptr() if lse is not None else None, _stream()), "infllm_attn_merge")
+
+
+def attn_merge_sets(o_parts, lse_parts, out, lse):
+    """attn_merge over one or two sets of partials in buffers of their own."""
+    B, H, Lq, D = out.shape
+    _need(out.stride(-1) == 1 and out.dtype == torch.bfloat16 and 1 <= len(o_parts) <= 2, "bad merge arguments")
+    two = len(o_parts) == 2
+    check(_lib.load().infllm_attn_merge_pair(o_parts[0].data_ptr(), lse_parts[0].data_ptr(), o_parts[0].shape[0], o_parts[1].data_ptr() if two else None,
+                                             lse_parts[1].data_ptr() if two else None, o_parts[1].shape[0] if two else 0, B, H, Lq, out.data_ptr(),
+                                             out.stride(0), out.stride(1), out.stride(2), lse.data_ptr() if lse is not None else None, _stream()),
+          "infllm_attn_merge_pair")
 
 
 def local_score(q, k, lse, score, *, cap=None, j_lo=0, j_hi=None, mask=MASK_NONE, offset=0, window=0,
