@@ -68,6 +68,9 @@ typedef struct {
     float *d_qpart;                /* optional fp32 [B, ceil(n/16), H*128]: sums of q_glb over each run of 16 positions */
 } infllm_ingest_args;
 int infllm_ingest(const infllm_ingest_args *a, void *stream);
+/* The same for heads of 64 (dim 64: every row holds 64 elements) or 128.  d_qbar (optional, n <= 16): the mean global query
+ * [B, H*dim]; d_qpart is then not written. */
+int infllm_ingest_dim(const infllm_ingest_args *a, int32_t dim, float *d_qbar, void *stream);
 
 /* out[b,c] = scale * sum_p parts[b,p,c] (p ascending): turns the d_qpart sums of infllm_ingest into
  * the mean global query of a block (context_manager.py:373-375) with scale = 1/n. */
@@ -627,6 +630,80 @@ int infllm_layer_path_counts(void *layer, int64_t *counts /* [6] */);
  * of the selections, the candidates a guess fetched that were not selected after all, and what a wrong guess's
  * repair brought back - the host-to-device traffic of MemoryUnit.load (context_manager.py:76-91) in units. */
 int64_t infllm_layer_fetched_units(void *layer);
+
+/* ---------------------------------------------------------------------------
+ * The streaming memory with every unit resident in HBM: a whole append() call (context_manager.py:474-545, 614-679,
+ * 682-813) enqueued by one native call, without the host in between.  The ranking kernel turns a block's selection into
+ * the global stage's page table on the device; selections travel to a pinned log, from which the residency bookkeeping
+ * (which unit would sit in the max_cached_block slots of CudaCache, context_manager.py:6-26, 495-515: hit, miss and
+ * eviction counts, infllm_cache_*) is done as they arrive.  Same kernels, same results as the block-by-block calls above.
+ *
+ * Buffers are the caller's.  dim: 128 or 64; every row buffer holds rows of dim elements.
+ *   units       chunks of units_per_chunk units [.., B, 2, Hkv, block_size, dim]; h_chunks / d_chunks: their addresses, as
+ *               the host and as the device reads them
+ *   d_log       log_slots x (B * topk + 1) ints of pinned memory, device and host view
+ *   d_ids       [B, topk]; d_iota: 0, 1, .. topk - 1; d_pages: [B, max_pages]
+ *   h_caches    [B] policy objects (infllm_cache_create, lru or fifo) */
+typedef struct {
+    int32_t B, H, Hkv, dim;
+    int32_t n_local, n_init, block_size, exc, topk, repr_topk, max_cached;
+    int32_t max_splits, num_cus, call_tokens, group_blocks, max_pages, units_per_chunk, log_slots;
+    int64_t ring_cap, init_cap;
+    void *d_ring_k_raw, *d_ring_k_rot, *d_ring_v;
+    float *d_ring_score;
+    void *d_init_kv;
+    infllm_page *d_pages;
+    int32_t *d_ids;
+    const int32_t *d_iota;
+    int32_t *d_log;
+    const int32_t *h_log;
+    void *const *h_caches;
+    const float *d_inv_freq;
+    double distance_scale;
+    float softmax_scale;
+    int32_t first_seq;                                /* the log's sequence numbers go on from here (0 for a cleared log) */
+} infllm_resident_desc;
+/* 1: the geometry and knobs have this path (topk <= 64, exc_block_size a multiple of 32, at most 64 units carved by a block
+ * and 256 by a call, H * dim <= 8192), 0: they do not */
+int infllm_resident_fits(const infllm_resident_desc *d);
+void *infllm_resident_create(const infllm_resident_desc *d);
+int infllm_resident_destroy(void *handle);                       /* the stream's work with the buffers is the caller's to wait for */
+int infllm_resident_set_state(void *handle, int64_t length, int64_t cursor, int32_t init_len, int32_t n_units);
+typedef struct {
+    const void *d_q, *d_k, *d_v;                      /* [B,H,n,dim], [B,Hkv,n,dim] */
+    int64_t q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;
+    void *d_out;                                      /* bf16 rows [b, h, i] at b*o_sb + h*o_sh + i*o_sl */
+    int64_t o_sb, o_sh, o_sl;
+    int64_t n;                                        /* tokens of the call */
+    int32_t call_tokens, max_tokens;                  /* tokens prepared in one go (0: one block); tokens the buffers hold */
+    void *d_reps;                                     /* [B, rep_rows, H*dim] */
+    int64_t rep_sb, rep_su;
+    int32_t rep_rows, n_chunks;
+    float *d_unit_scores;                             /* [B, >= units] */
+    int64_t unit_scores_sb;
+    const uint64_t *h_chunks, *d_chunks;
+    /* workspaces, dead between calls: any caller of the same stream may share them */
+    void *d_q_loc, *d_q_glb;                          /* [B,H,max_tokens,dim] */
+    float *d_qpart, *d_qbar;                          /* [B, ceil(max_tokens/16), H*dim], [blocks, B, H*dim] */
+    uint16_t *d_o_part;                               /* [part_rows, dim]: partial rows of the local stage, of a decode step */
+    float *d_lse_part;
+    int64_t part_rows;
+    uint16_t *d_o_part2;                              /* [part_rows2, dim]: of the global stage (infllm_resident_part_rows) */
+    float *d_lse_part2;
+    int64_t part_rows2;
+    float *d_lse;                                     /* [B,H,exc] */
+    float *d_logits;                                  /* [B,H,n_local] */
+    float *d_call_scores;                             /* [blocks, B, scores_cols], scores_cols >= the units after the call */
+    int64_t scores_cols;
+    int32_t *d_base;                                  /* [blocks, B, topk] */
+} infllm_resident_call;
+int infllm_resident_append(void *handle, const infllm_resident_call *a, void *stream);
+int64_t infllm_resident_part_rows(const infllm_resident_desc *d);
+/* out[10]: length, carving cursor, init tokens, units; blocks worked off; hits, misses, evictions of the bookkeeping done so
+ * far (wait != 0: all of it, waiting for the stream); selections ranked from a call's lists; last sequence number */
+int infllm_resident_state(void *handle, int32_t wait, int64_t *out);
+int infllm_resident_timing(void *handle, int32_t capacity, int32_t stride);              /* as infllm_layer_timing */
+int infllm_resident_read_timing(void *handle, int32_t which, float *ms, int32_t *n_queries, int32_t *n_keys, int32_t capacity);
 
 /* Event timing of the two attention stages (for benchmarks): enable with a record
  * capacity and a stride (every stride-th launch of each stage is bracketed by two events; an event pair

@@ -96,6 +96,30 @@ class LayerDesc(C.Structure):
     ]
 
 
+class ResidentDesc(C.Structure):
+    _fields_ = [(n, c_i32) for n in ("B", "H", "Hkv", "dim", "n_local", "n_init", "block_size", "exc", "topk", "repr_topk", "max_cached", "max_splits",
+                                     "num_cus", "call_tokens", "group_blocks", "max_pages", "units_per_chunk", "log_slots")] + [
+        ("ring_cap", c_i64), ("init_cap", c_i64),
+        ("d_ring_k_raw", c_vp), ("d_ring_k_rot", c_vp), ("d_ring_v", c_vp), ("d_ring_score", c_vp), ("d_init_kv", c_vp), ("d_pages", c_vp),
+        ("d_ids", c_vp), ("d_iota", c_vp), ("d_log", c_vp), ("h_log", c_vp), ("h_caches", c_vp), ("d_inv_freq", c_vp),
+        ("distance_scale", c_f64), ("softmax_scale", c_f32), ("first_seq", c_i32),
+    ]
+
+
+class ResidentCall(C.Structure):
+    _fields_ = [
+        ("d_q", c_vp), ("d_k", c_vp), ("d_v", c_vp),
+        ("q_sb", c_i64), ("q_sh", c_i64), ("q_sl", c_i64), ("k_sb", c_i64), ("k_sh", c_i64), ("k_sl", c_i64),
+        ("v_sb", c_i64), ("v_sh", c_i64), ("v_sl", c_i64),
+        ("d_out", c_vp), ("o_sb", c_i64), ("o_sh", c_i64), ("o_sl", c_i64), ("n", c_i64), ("call_tokens", c_i32), ("max_tokens", c_i32),
+        ("d_reps", c_vp), ("rep_sb", c_i64), ("rep_su", c_i64), ("rep_rows", c_i32), ("n_chunks", c_i32),
+        ("d_unit_scores", c_vp), ("unit_scores_sb", c_i64), ("h_chunks", c_vp), ("d_chunks", c_vp),
+        ("d_q_loc", c_vp), ("d_q_glb", c_vp), ("d_qpart", c_vp), ("d_qbar", c_vp), ("d_o_part", c_vp), ("d_lse_part", c_vp), ("part_rows", c_i64),
+        ("d_o_part2", c_vp), ("d_lse_part2", c_vp), ("part_rows2", c_i64), ("d_lse", c_vp), ("d_logits", c_vp),
+        ("d_call_scores", c_vp), ("scores_cols", c_i64), ("d_base", c_vp),
+    ]
+
+
 class FrontArgs(C.Structure):
     _fields_ = [
         ("d_q", c_vp), ("d_k", c_vp), ("d_v", c_vp),
@@ -151,6 +175,7 @@ SYMBOLS = {
     "infllm_version": (c_i32, []),
     "infllm_last_error": (C.c_char_p, []),
     "infllm_ingest": (c_i32, [C.POINTER(IngestArgs), c_vp]),
+    "infllm_ingest_dim": (c_i32, [C.POINTER(IngestArgs), c_i32, c_vp, c_vp]),
     "infllm_reduce_partials": (c_i32, [c_vp, c_i32, c_i32, c_i32, c_f32, c_vp, c_vp]),
     "infllm_block_mean": (c_i32, [c_vp, c_i32, c_i32, c_i32, c_i32, c_vp, c_vp]),
     "infllm_chunk_qbar": (c_i32, [c_vp, c_i64, c_i64, c_i64, c_i32, c_i32, c_i32, c_i32, c_vp, C.c_double, c_i64, c_vp, c_vp]),
@@ -203,6 +228,15 @@ SYMBOLS = {
     "infllm_block_prefetch": (c_i32, [c_vp, C.POINTER(SelectArgs), c_vp, c_vp]),
     "infllm_layer_prefetch_stats": (c_i32, [c_vp, c_vp, c_vp]),
     "infllm_layer_last_selection": (c_i32, [c_vp, c_vp, c_i32]),
+    "infllm_resident_fits": (c_i32, [C.POINTER(ResidentDesc)]),
+    "infllm_resident_part_rows": (c_i64, [C.POINTER(ResidentDesc)]),
+    "infllm_resident_create": (c_vp, [C.POINTER(ResidentDesc)]),
+    "infllm_resident_destroy": (c_i32, [c_vp]),
+    "infllm_resident_set_state": (c_i32, [c_vp, c_i64, c_i64, c_i32, c_i32]),
+    "infllm_resident_append": (c_i32, [c_vp, C.POINTER(ResidentCall), c_vp]),
+    "infllm_resident_state": (c_i32, [c_vp, c_i32, c_vp]),
+    "infllm_resident_timing": (c_i32, [c_vp, c_i32, c_i32]),
+    "infllm_resident_read_timing": (c_i32, [c_vp, c_i32, c_vp, c_vp, c_vp, c_i32]),
     "infllm_layer_timing": (c_i32, [c_vp, c_i32, c_i32]),
     "infllm_layer_read_timing": (c_i32, [c_vp, c_i32, c_vp, c_vp, c_vp, c_i32]),
 }

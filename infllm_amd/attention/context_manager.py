@@ -14,41 +14,98 @@ stream positions and device-resident rings instead of torch.cat/trim:
 * both stages leave partials that the merge kernel joins into the joint
   softmax; the local score (probability column sums) is a third kernel that
   needs the merged log-sum-exp;
-* memory units live in pinned host memory (always) and in a slab of
+* memory units live in HBM where there is room for them (``resident_bytes``):
+  a whole append() call is then enqueued by one native call
+  (infllm_resident_append), the selections become page tables on the device,
+  and the host only keeps the residency policy's books from a pinned log;
+* otherwise - beyond that budget, with the lru-s policy, with retrieval in
+  chunks, and while selections are recorded or stepped through - the host
+  drives every block: units live in pinned host memory and in a slab of
   ``max_cached_block`` device slots managed by the reference's lru / lru-s
   policy (plus fifo; native, infllm_cache_*); the misses of a block are moved
   by the DMA engines (short blocks: read from the pinned pages by one kernel
   on a side stream), for lru / fifo starting from the selection's candidates a
   block ahead of the selection itself (``fetch_ahead``).
 
-This module keeps the state machine, in absolute positions
-(context_manager.py:614-679 restated): ``cursor`` is the first token not yet
-carved, tokens [0, init_len) are the attention sinks, unit u is tokens
-[n_init + u*bs, n_init + (u+1)*bs).  The device work of one execution block is
-issued by three native calls: infllm_block_front, infllm_block_select (the one
-host wait, for the retrieved unit ids, which overlaps the local stage; then
-cache policy and fetch) and infllm_block_back, plus infllm_block_prefetch for
-the next block.
+The state machine is in absolute positions (context_manager.py:614-679
+restated): ``cursor`` is the first token not yet carved, tokens [0, init_len)
+are the attention sinks, unit u is tokens [n_init + u*bs, n_init + (u+1)*bs).
+Driven by the host, the device work of one execution block is issued by three
+native calls: infllm_block_front, infllm_block_select (the one host wait, for
+the retrieved unit ids, which overlaps the local stage; then cache policy and
+fetch) and infllm_block_back, plus infllm_block_prefetch for the next block.
 """
 import ctypes
 import os
+import threading
+import weakref
 
 import torch
 
 from .. import _lib
-from .._lib import BackArgs, FrontArgs, LayerDesc, check
+from .._lib import BackArgs, FrontArgs, LayerDesc, ResidentCall, ResidentDesc, check
 from ..ops import HEAD_DIM, KEY_TILE
 
 from ._rows import check_head_dim, narrow as _narrow, wide_inv_freq, widen as _widen
 
 _SIDE_STREAM = None          # one process-wide side stream, like GLOBAL_STREAM (context_manager.py:193)
-_CALL_BUFFERS = {}           # (device, stream, geometry) -> the buffers of a call prepared in one go, see _bind_call_buffers
+# (device, stream, geometry) -> the buffers of a call prepared in one go, shared by the managers that are alive
+_CALL_BUFFERS = weakref.WeakValueDictionary()
 _HOST_CHUNK_UNITS = 64       # units per pinned host allocation
+_UNIT_CHUNK = 64             # units per allocation of their home in HBM
+_LOG_SLOTS = 256             # selections whose bookkeeping may be outstanding
 _MAX_SPLITS = 16             # key splits of one attention stage
 _NUM_CUS = 256               # MI355X
 _PAGE_SLOTS = 4
 _CARVE_SLOTS = 4             # staging slots of the carve, used in turn (more of them serve more misses on the device - 16: 18 %,
                              # 64: 57 % of the benchmark stream's - but the stream is no faster for it, measured)
+
+
+class _Buffers(dict):
+    """dict that can be referenced weakly"""
+
+
+class _Units:
+    """What the resident units of all managers take of a device's memory, and the pinned logs between managers."""
+    lock = threading.Lock()
+    used = {}                 # device index -> bytes
+    logs = {}                 # (device index, ints) -> [(log, last sequence number written or on its way)]
+    max_logs = 64             # logs kept per size
+
+    @classmethod
+    def take(cls, dev, n, limit):
+        with cls.lock:
+            total = cls.used.get(dev, 0) + n
+            if total > limit:
+                return False
+            cls.used[dev] = total
+        return True
+
+    @classmethod
+    def give(cls, dev, n):
+        with cls.lock:
+            cls.used[dev] = cls.used.get(dev, 0) - n
+
+    @classmethod
+    def take_log(cls, dev, stride):
+        """A pinned log and the sequence number to go on from: one whose last selection has arrived, or a new one."""
+        n = _LOG_SLOTS * stride
+        with cls.lock:
+            pool = cls.logs.setdefault((dev, n), [])
+            for i, (log, seq) in enumerate(pool):
+                if seq == 0 or int(log[(seq % _LOG_SLOTS) * stride + stride - 1]) == seq:
+                    del pool[i]
+                    return log, seq
+        return torch.zeros((n,), dtype=torch.int32, pin_memory=True), 0
+
+    @classmethod
+    def give_log(cls, dev, log, seq):
+        with cls.lock:
+            pool = cls.logs.setdefault((dev, log.numel()), [])
+            if seq < 1 << 30 and len(pool) < cls.max_logs:
+                pool.append((log, seq))
+                return
+        torch.cuda.synchronize(dev)               # kernels may still be on their way to it
 
 
 class CachePolicy:
@@ -125,7 +182,10 @@ class ContextManager:
     call_tokens = 8192          # tokens of an append() call prepared in one go (prologue, mean queries and the local
                                 # stage of all their blocks: infllm_call_front); 0: every block runs its own.
                                 # INFLLM_CALL_TOKENS overrides it.  Needs exc_block_size to be a multiple of 32.
-    local_group_blocks = 2      # blocks of a prepared call per launch of the local stage (INFLLM_LOCAL_GROUP overrides it)
+    local_group_blocks = None   # blocks of a prepared call per launch of the local stage (INFLLM_LOCAL_GROUP overrides it);
+                                # None: two where the host drives, else as many as pay
+    resident_bytes = None       # HBM that the units of all managers of this process may take together on a device; None: a
+                                # quarter of it.  0 keeps units in pinned host memory (so does INFLLM_NO_RESIDENT=1).
 
     def __init__(self, position_embedding, n_init, n_local, block_size, max_cached_block, topk, exc_block_size,
                  score_decay=None, fattn=False, repr_topk=1, cache_strategy="lru", chunk_topk_calc=None,
@@ -155,8 +215,11 @@ class ContextManager:
         self.trace_blocks, self.trace_units = [], []
         self._call_scores = None      # [blocks of a call, B, units]: scores of every unit under every block's mean query
         self._host_copies_open = False
-        self.stats = dict(blocks=0, hits=0, misses=0, evictions=0)
+        self._stats = dict(blocks=0, hits=0, misses=0, evictions=0)
+        self._policy = []
         self._layer = None
+        self._resident = None         # native handle while the units are resident in HBM
+        self._base_stats = None
         self._timing_cap, self._timing_stride = 0, 1
         self._mass_units = None                # lru-s: selections of the block whose unit masses are still on the device
         global _SIDE_STREAM
@@ -165,56 +228,297 @@ class ContextManager:
 
     def __del__(self):
         layer, self._layer = getattr(self, "_layer", None), None
-        if layer:
-            try:
+        try:
+            if layer:
                 _lib.load().infllm_layer_destroy(layer)       # waits for this layer's own work, not for the device
-            except Exception:
-                pass
+            self._drop_resident()
+        except Exception:
+            pass
 
     # ------------------------------------------------------------------ setup
-    def _init(self, q, k):
-        B, H, _, D = q.shape
+    def _wants_resident(self):
+        """Whether the units may live in HBM: nothing asks for the host between a block's selection and its fetch."""
+        return not (self.record_trace or self.select_in_steps or not self.fetch_ahead)
+
+    def _init(self, q, k, resident=None):
+        """q, k: rows of the heads' own width.  resident: None to choose."""
+        B, H = q.shape[0], q.shape[1]
         Hkv = k.shape[1]
         dev = q.device
-        assert D == HEAD_DIM                                    # rows arrive widened (see _widen)
         if self.topk > self.max_cached_block:
             raise ValueError("topk must not exceed max_cached_block")
         if self.topk > 64:
             raise ValueError("this build selects at most 64 units per block (topk <= 64)")
         if self.repr_topk > self.block_size:
             raise ValueError("repr_topk must not exceed block_size")
+        if self.position_embedding.inv_freq.numel() != self.dim_head // 2:
+            raise ValueError(f"the rotary embedding is built for head_dim {2 * self.position_embedding.inv_freq.numel()}, "
+                             f"the heads have {self.dim_head}")
         self.batch_size = self.num_units = B
         self.num_heads = self.unit_size = H
         self.num_heads_kv = self.unit_size_kv = Hkv
-        self.head_width = D                                     # of the rows the kernels see; self.dim_head is the caller's
         self.dtype = q.dtype
         self.device = dev
+        self._dev_index = dev.index if dev.index is not None else torch.cuda.current_device()
+        self._lib = _lib.load()
         bs, exc, topk = self.block_size, self.exc_block_size, self.topk
         ct = int(os.environ.get("INFLLM_CALL_TOKENS", self.call_tokens))
         self._call_tokens = min(ct, 16 * exc) // exc * exc if (ct >= exc and exc % 32 == 0) else 0
+        group = os.environ.get("INFLLM_LOCAL_GROUP", self.local_group_blocks)
         # the rings hold the local window, the remainder that waits to fill a unit, and what is prepared ahead of the
         # block being attended: one block, or the rest of a call prepared in one go
         cap = self.n_local + exc + bs + max(exc, self._call_tokens)
-        self.ring_cap = cap = (cap + KEY_TILE - 1) // KEY_TILE * KEY_TILE + KEY_TILE
-        bf = dict(dtype=torch.bfloat16, device=dev)
-        f32 = dict(dtype=torch.float32, device=dev)
-        self.ring_k_raw = torch.zeros((B, Hkv, cap, D), **bf)
-        self.ring_k_rot = torch.zeros((B, Hkv, cap, D), **bf)
-        self.ring_v = torch.zeros((B, Hkv, cap, D), **bf)
-        self.ring_score = torch.zeros((B, H, cap), **f32)
-        self.init_kv = torch.zeros((B, 2, Hkv, max(self.n_init, 1), D), **bf)
-        self.slab = torch.zeros((B, self.max_cached_block, 2, Hkv, bs, D), **bf)
-        self.reps = torch.zeros((B, 16, H * D), **bf)
-        self.unit_scores = torch.empty((B, 16), **f32)
-        self.host_chunks, self._host_base, self._host_dev_base = [], [], []
-        self._chunk_base = (ctypes.c_uint64 * 64)()           # device-visible chunk addresses, as the native side reads them
-        self.policy = [CachePolicy(self.max_cached_block, self.cache_strategy, self.score_decay) for _ in range(B)]
-        if self.record_trace:
-            for pol in self.policy:
-                pol.evicted_log = []
+        self.ring_cap = (cap + KEY_TILE - 1) // KEY_TILE * KEY_TILE + KEY_TILE
+        tiles_per_unit = (bs + KEY_TILE - 1) // KEY_TILE
+        self.max_pages = topk * tiles_per_unit + (self.n_init + KEY_TILE - 1) // KEY_TILE + (exc + bs) // KEY_TILE + 3
         self.cursor = 0
         self.init_len = 0
         self.num_global_block = 0
+        self._policy = [CachePolicy(self.max_cached_block, self.cache_strategy, self.score_decay) for _ in range(B)]
+        if self.record_trace:
+            for pol in self._policy:
+                pol.evicted_log = []
+        if resident is None:
+            resident = self._can_be_resident()
+        # Blocks per launch of the local stage.  With the host between the blocks two: a launch covers the wait for a fetch.
+        # Without it as many as a call has: the launch's fixed cost once.
+        self._local_group = int(group) if group is not None else 16 if resident else 2
+        # rows of 64 are the kernels' own width where the units are resident; everything else travels in rows of 128
+        self.head_width = D = 64 if resident and self.dim_head == 64 else HEAD_DIM
+        bf = dict(dtype=torch.bfloat16, device=dev)
+        f32 = dict(dtype=torch.float32, device=dev)
+        self.ring_k_raw, self.ring_k_rot, self.ring_v = torch.empty((3, B, Hkv, self.ring_cap, D), **bf).unbind(0)
+        self.ring_score = torch.empty((B, H, self.ring_cap), **f32)
+        self.init_kv = torch.empty((B, 2, Hkv, max(self.n_init, 1), D), **bf)
+        self.reps = torch.empty((B, 16, H * D), **bf)
+        self.unit_scores = torch.empty((B, 16), **f32)
+        self.inv_freq = (self.position_embedding.inv_freq.to(device=dev, dtype=torch.float32).contiguous() if D == self.dim_head
+                         else wide_inv_freq(self.position_embedding.inv_freq, dev))
+        self.slot_bytes = 2 * Hkv * bs * D * 2              # one unit of one batch row
+        self.unit_bytes = B * self.slot_bytes               # one unit, all batch rows
+        self._init_resident() if resident else self._init_host()
+        self._call_stream = None               # stream the call buffers were taken for (they are bound at the first append)
+        self.initialized = True
+
+    # ------------------------------------------------------ units resident in HBM
+    def _resident_limit(self):
+        if os.environ.get("INFLLM_NO_RESIDENT", "0") not in ("", "0"):
+            return 0
+        if self.resident_bytes is not None:
+            return self.resident_bytes
+        return torch.cuda.get_device_properties(self._dev_index).total_memory // 4
+
+    def _resident_desc(self, D):
+        d = ResidentDesc()
+        d.B, d.H, d.Hkv, d.dim = self.num_units, self.unit_size, self.unit_size_kv, D
+        d.n_local, d.n_init, d.block_size, d.exc = self.n_local, self.n_init, self.block_size, self.exc_block_size
+        d.topk, d.repr_topk, d.max_cached = self.topk, self.repr_topk, self.max_cached_block
+        d.max_splits, d.num_cus, d.call_tokens, d.group_blocks = _MAX_SPLITS, _NUM_CUS, self._call_tokens, getattr(self, "_local_group", 1)
+        d.max_pages, d.units_per_chunk, d.log_slots = self.max_pages, _UNIT_CHUNK, _LOG_SLOTS
+        d.ring_cap, d.init_cap = self.ring_cap, max(self.n_init, 1)
+        return d
+
+    def _can_be_resident(self):
+        if not self._wants_resident() or self.cache_strategy == "lru-s" or self.chunk_topk_calc is not None or self.topk < 1:
+            return False
+        # the switches that choose between ways of the host-driven path ask for that path
+        if any(name in os.environ for name in ("INFLLM_FETCH_AHEAD_ALWAYS", "INFLLM_NO_DMA_FETCH", "INFLLM_NO_DMA_ENGINE", "INFLLM_NO_STAGING_COPY",
+                                               "INFLLM_NO_CALL_LISTS", "INFLLM_CALL_LISTS_ROOM", "INFLLM_PAGE_TABLE_KERNEL", "INFLLM_SCORE_MERGE_APART")):
+            return False
+        limit = self._resident_limit()
+        if not limit or _Units.used.get(self._dev_index, 0) >= limit:
+            return False
+        return self._lib.infllm_resident_fits(ctypes.byref(self._resident_desc(64 if self.dim_head == 64 else HEAD_DIM))) == 1
+
+    def _init_resident(self):
+        dev, B, topk = self.device, self.num_units, self.topk
+        i32 = dict(dtype=torch.int32, device=dev)
+        self._chunks = []                       # homes of the units: [_UNIT_CHUNK, B, 2, Hkv, bs, D] each
+        self._chunk_bytes = _UNIT_CHUNK * self.unit_bytes
+        self._chunk_host = (ctypes.c_uint64 * 16)()
+        self._chunk_dev = torch.empty((16,), dtype=torch.int64, device=dev)
+        self._ids = torch.empty((B, topk), **i32)
+        self._iota = torch.arange(topk, **i32)
+        self._pages = torch.empty((B * self.max_pages * ctypes.sizeof(_lib.Page),), dtype=torch.uint8, device=dev)
+        self._log, seq = _Units.take_log(self._dev_index, B * topk + 1)
+        self._caches = (ctypes.c_void_p * B)(*[pol.handle for pol in self._policy])
+        d = self._resident_desc(self.head_width)
+        d.d_ring_k_raw, d.d_ring_k_rot = self.ring_k_raw.data_ptr(), self.ring_k_rot.data_ptr()
+        d.d_ring_v, d.d_ring_score, d.d_init_kv = self.ring_v.data_ptr(), self.ring_score.data_ptr(), self.init_kv.data_ptr()
+        d.d_pages, d.d_ids, d.d_iota = self._pages.data_ptr(), self._ids.data_ptr(), self._iota.data_ptr()
+        d.d_log, d.h_log = self._lib.infllm_host_device_pointer(self._log.data_ptr()), self._log.data_ptr()
+        d.h_caches, d.d_inv_freq = ctypes.addressof(self._caches), self.inv_freq.data_ptr()
+        d.distance_scale, d.softmax_scale = float(self.position_embedding.distance_scale), 1.0 / (self.dim_head ** 0.5)
+        d.first_seq = seq
+        self._part_rows2 = int(self._lib.infllm_resident_part_rows(ctypes.byref(d)))
+        self._resident = self._lib.infllm_resident_create(ctypes.byref(d))
+        if not self._resident:
+            raise _lib.InfLLMHipError("infllm_resident_create failed: " + (self._lib.infllm_last_error() or b"").decode())
+        if self._timing_cap:
+            check(self._lib.infllm_resident_timing(self._resident, self._timing_cap, self._timing_stride), "infllm_resident_timing")
+        self._state = (ctypes.c_int64 * 10)()
+        self._streams = {torch.cuda.current_stream(dev).cuda_stream}
+        self._rc = ResidentCall()
+        self._rc_ref = ctypes.byref(self._rc)
+        self._rc.h_chunks, self._rc.d_chunks = ctypes.addressof(self._chunk_host), self._chunk_dev.data_ptr()
+        self._rc.call_tokens = self._call_tokens
+        self._rc.max_tokens = max(self._call_tokens, self.exc_block_size)
+        self._bind_resident_reps()
+
+    def _bind_resident_reps(self):
+        rc = self._rc
+        rc.d_reps, rc.rep_sb, rc.rep_su, rc.rep_rows = self.reps.data_ptr(), self.reps.stride(0), self.reps.stride(1), self.reps.shape[1]
+        rc.d_unit_scores, rc.unit_scores_sb = self.unit_scores.data_ptr(), self.unit_scores.stride(0)
+
+    def _add_chunks(self, n_units):
+        """Homes for n_units units; False when the budget or the memory does not have them."""
+        while len(self._chunks) * _UNIT_CHUNK < n_units:
+            if not _Units.take(self._dev_index, self._chunk_bytes, self._resident_limit()):
+                return False
+            try:
+                t = torch.empty((_UNIT_CHUNK, self.num_units, 2, self.unit_size_kv, self.block_size, self.head_width), dtype=torch.bfloat16,
+                                device=self.device)
+            except torch.OutOfMemoryError:
+                _Units.give(self._dev_index, self._chunk_bytes)
+                return False
+            n = len(self._chunks)
+            self._chunks.append(t)
+            if n == len(self._chunk_host):
+                grown = (ctypes.c_uint64 * (2 * n))()
+                grown[:n] = self._chunk_host[:]
+                table = torch.empty((2 * n,), dtype=torch.int64, device=self.device)
+                table[:n] = self._chunk_dev
+                self._chunk_host, self._chunk_dev = grown, table
+                self._rc.h_chunks, self._rc.d_chunks = ctypes.addressof(grown), table.data_ptr()
+            self._chunk_host[n] = t.data_ptr()
+            self._chunk_dev[n].fill_(t.data_ptr())
+        self._rc.n_chunks = len(self._chunks)
+        return True
+
+    def _drop_resident(self):
+        handle, self._resident = getattr(self, "_resident", None), None
+        if not handle:
+            return
+        self._lib.infllm_resident_state(handle, 0, self._state)
+        _Units.give_log(self._dev_index, self._log, int(self._state[9]))
+        _Units.give(self._dev_index, len(self._chunks) * self._chunk_bytes)
+        self._lib.infllm_resident_destroy(handle)
+        if len(self._streams) > 1:              # buffers go back to the allocator for the stream they were made on
+            torch.cuda.synchronize(self.device)
+        self._chunks, self._log = [], None
+
+    def _resident_books(self, wait):
+        """The bookkeeping of the selections so far (wait: of all of them) into the counters."""
+        check(self._lib.infllm_resident_state(self._resident, 1 if wait else 0, self._state), "infllm_resident_state")
+        st, base = self._state, self._base_stats
+        for i, name in ((4, "blocks"), (5, "hits"), (6, "misses"), (7, "evictions")):
+            self._stats[name] = int(st[i]) + (base[name] if base else 0)
+
+    @property
+    def stats(self):
+        """Blocks worked off and the residency counters: hits, misses and evictions of the unit cache of max_cached_block
+        slots (of the books, where the units are resident and nothing has to move)."""
+        if self._resident:
+            self._resident_books(True)
+        return self._stats
+
+    @property
+    def policy(self):
+        if self._resident:
+            self._resident_books(True)
+        return self._policy
+
+    def _leave_resident(self):
+        """From here on the host drives (selections are to be recorded, or the units outgrew their budget): the state moves
+        over as export_state / load_state move it, the policies stay, and the slots they hand out are filled."""
+        policy, stats, length, timing = self.policy, self.stats, self.length, (self._timing_cap, self._timing_stride)
+        units, n = self._chunks, self.num_global_block
+        state = self.export_state(with_units=False)
+        state["units"] = None
+        self._drop_resident()
+        self.initialized, self.length = False, 0
+        self._load(state, resident=False, unit_at=lambda u: units[u // _UNIT_CHUNK][u % _UNIT_CHUNK])
+        self._policy, self._stats = policy, stats
+        for u, pol in enumerate(policy):
+            if self.record_trace and pol.evicted_log is None:
+                pol.evicted_log = []
+            self._caches[u] = pol.handle
+            for unit, slot in pol.slot_of.items():
+                self.slab[u, slot] = _widen(units[unit // _UNIT_CHUNK][unit % _UNIT_CHUNK, u], self.dim_head) if self.head_width != units[0].shape[-1] \
+                    else units[unit // _UNIT_CHUNK][unit % _UNIT_CHUNK, u]
+        torch.cuda.synchronize(self.device)
+        assert self.length == length and self.num_global_block == n
+
+    def _append_resident(self, q, k, v, n):
+        """One append() call on resident units; None when the units no longer fit (nothing has been done then)."""
+        rc, length = self._rc, self.length
+        units = max(0, (length + n - self.n_init - self.n_local) // self.block_size)
+        if units > len(self._chunks) * _UNIT_CHUNK and not self._add_chunks(units):
+            return None
+        if units > self.reps.shape[1]:
+            self._grow_reps(units)
+        stream = torch.cuda.current_stream().cuda_stream
+        if self._call_stream != stream:
+            self._bind_resident_buffers(stream)
+        if n > 1 and units > self.topk and (self._call_scores is None or self._call_scores.shape[2] < units):
+            cols = max(-(-units // 256) * 256, 2 * (self._call_scores.shape[2] if self._call_scores is not None else 0))
+            self._call_scores = torch.empty((-(-rc.max_tokens // self.exc_block_size), self.num_units, cols), dtype=torch.float32, device=self.device)
+            rc.d_call_scores, rc.scores_cols = self._call_scores.data_ptr(), cols
+        B, H, D = self.num_units, self.unit_size, self.head_width
+        # rows of a token next to each other, as the layer's output projection takes them
+        out = torch.empty((B, n, H, D), dtype=torch.bfloat16, device=q.device)
+        rc.d_q, rc.d_k, rc.d_v, rc.d_out, rc.n = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), n
+        rc.q_sb, rc.q_sh, rc.q_sl, _ = q.stride()
+        rc.k_sb, rc.k_sh, rc.k_sl, _ = k.stride()
+        rc.v_sb, rc.v_sh, rc.v_sl, _ = v.stride()
+        rc.o_sb, rc.o_sl, rc.o_sh = n * H * D, H * D, D
+        status = self._lib.infllm_resident_append(self._resident, self._rc_ref, stream)
+        if status:
+            check(status, "infllm_resident_append")
+        self.length = length + n
+        self.num_global_block = units
+        self.init_len = min(self.n_init, max(self.length - self.n_local, 0))
+        self.cursor = self.init_len + units * self.block_size
+        if self.cache_strategy == "lru":
+            self.load_count += -(-n // self.exc_block_size)
+        return out.permute(0, 2, 1, 3)
+
+    def _bind_resident_buffers(self, stream):
+        """Workspaces of a call: dead between append() calls, so the managers that work on one stream (one after the
+        other, as the layers of a model do) share one set."""
+        B, H, D, exc, T = self.num_units, self.unit_size, self.head_width, self.exc_block_size, self._rc.max_tokens
+        blocks = -(-T // exc)
+        part_rows = max(8, 2 * min(self._local_group, blocks)) * B * H * exc       # (at most two key splits of several blocks)
+        key = ("resident", self._dev_index, stream, B, H, D, T, exc, self.n_local, self.topk, part_rows, self._part_rows2)
+        buf = _CALL_BUFFERS.get(key)
+        if buf is None:
+            bf = dict(dtype=torch.bfloat16, device=self.device)
+            f32 = dict(dtype=torch.float32, device=self.device)
+            f16 = dict(dtype=torch.float16, device=self.device)
+            buf = _Buffers(q_loc=torch.empty((B * H * T * D,), **bf), q_glb=torch.empty((B * H * T * D,), **bf),
+                           qpart=torch.empty((B * ((T + 15) // 16) * H * D,), **f32), qbar=torch.empty((blocks * B * H * D,), **f32),
+                           o_part=torch.empty((part_rows * D,), **f16), lse_part=torch.empty((part_rows,), **f32),
+                           o_part2=torch.empty((self._part_rows2 * D,), **f16), lse_part2=torch.empty((self._part_rows2,), **f32),
+                           lse=torch.empty((B * H * exc,), **f32), logits=torch.empty((B * H * self.n_local,), **f32),
+                           base=torch.empty((blocks * B * self.topk,), dtype=torch.int32, device=self.device))
+            _CALL_BUFFERS[key] = buf
+        self._call_buf = buf
+        rc = self._rc
+        for name, t in buf.items():
+            setattr(rc, "d_" + name, t.data_ptr())
+        rc.part_rows, rc.part_rows2 = part_rows, self._part_rows2
+        self._call_stream = stream
+        self._streams.add(stream)
+
+    # -------------------------------------------------------- the host drives
+    def _init_host(self):
+        B, H, Hkv, D, dev, cap = self.num_units, self.unit_size, self.unit_size_kv, self.head_width, self.device, self.ring_cap
+        bs, exc, topk = self.block_size, self.exc_block_size, self.topk
+        bf = dict(dtype=torch.bfloat16, device=dev)
+        f32 = dict(dtype=torch.float32, device=dev)
+        self.slab = torch.empty((B, self.max_cached_block, 2, Hkv, bs, D), **bf)
+        self.host_chunks, self._host_base, self._host_dev_base = [], [], []
+        self._chunk_base = (ctypes.c_uint64 * 64)()           # device-visible chunk addresses, as the native side reads them
         # workspaces of one execution block
         self.q_loc = torch.empty((2, B * H * exc * D), **bf)        # two slots: this block / the one prepared ahead
         self.q_glb = torch.empty((2, B * H * exc * D), **bf)
@@ -226,19 +530,11 @@ class ContextManager:
         self.lse = torch.empty((B * H * exc,), **f32)
         self.topk_idx = torch.zeros((B, max(topk, 1)), dtype=torch.int32, device=dev)
         self.topk_idx_host = torch.zeros((B, max(topk, 1)), dtype=torch.int32, pin_memory=True)
-        tiles_per_unit = (bs + KEY_TILE - 1) // KEY_TILE
-        self.max_pages = topk * tiles_per_unit + (self.n_init + KEY_TILE - 1) // KEY_TILE + (exc + bs) // KEY_TILE + 3
         page_bytes = ctypes.sizeof(_lib.Page)
         self.pages_dev = torch.empty((B * self.max_pages * page_bytes,), dtype=torch.uint8, device=dev)
         self.pages_host = torch.empty((_PAGE_SLOTS * B * self.max_pages * page_bytes,), dtype=torch.uint8, pin_memory=True)
         self.max_carve = (exc + self.n_init) // bs + 2
         self.carve_stage = torch.empty((_CARVE_SLOTS, self.max_carve, B, 2, Hkv, bs, D), **bf)
-        if self.position_embedding.inv_freq.numel() != self.dim_head // 2:
-            raise ValueError(f"the rotary embedding is built for head_dim {2 * self.position_embedding.inv_freq.numel()}, "
-                             f"the heads have {self.dim_head}")
-        self.inv_freq = wide_inv_freq(self.position_embedding.inv_freq, dev)
-        self.slot_bytes = 2 * Hkv * bs * D * 2              # one unit of one batch row
-        self.unit_bytes = B * self.slot_bytes               # one unit, all batch rows
 
         d = LayerDesc()
         d.B, d.H, d.Hkv = B, H, Hkv
@@ -251,7 +547,6 @@ class ContextManager:
         d.d_q_loc, d.d_q_glb, d.d_qbar = self.q_loc.data_ptr(), self.q_glb.data_ptr(), self.qbar.data_ptr()
         d.d_qpart = self.qpart.data_ptr()
         d.d_o_part, d.d_lse_part, d.d_lse = self.o_part.data_ptr(), self.lse_part.data_ptr(), self.lse.data_ptr()
-        self._lib = _lib.load()
         # the top-k kernel writes the ids straight into pinned host memory (no copy in the chain)
         d.d_topk_idx = self._lib.infllm_host_device_pointer(self.topk_idx_host.data_ptr())
         d.h_topk_idx = None
@@ -267,13 +562,11 @@ class ContextManager:
         d.d_inv_freq = self.inv_freq.data_ptr()
         d.distance_scale = float(self.position_embedding.distance_scale)
         d.softmax_scale = 1.0 / (self.dim_head ** 0.5)
-        self._lib = _lib.load()
         self._layer = self._lib.infllm_layer_create(ctypes.byref(d))
         if not self._layer:
             raise _lib.InfLLMHipError("infllm_layer_create failed: " + (self._lib.infllm_last_error() or b"").decode())
         if self._timing_cap:
             check(self._lib.infllm_layer_timing(self._layer, self._timing_cap, self._timing_stride), "infllm_layer_timing")
-        self._call_stream = None               # stream the call buffers were taken for (they are bound at the first append)
         # argument blocks and host arrays reused by every block
         self._fa, self._ba = FrontArgs(), BackArgs()
         self._sel_slots = (ctypes.c_int32 * (B * max(topk, 1)))()
@@ -300,7 +593,7 @@ class ContextManager:
         self._sel_ids = (ctypes.c_int32 * n_ids)()
         self._evicted = (ctypes.c_int32 * n_ids)()
         self._n_evicted, self._n_miss_row = (ctypes.c_int32 * B)(), (ctypes.c_int32 * B)()
-        self._caches = (ctypes.c_void_p * B)(*[pol.handle for pol in self.policy])
+        self._caches = (ctypes.c_void_p * B)(*[pol.handle for pol in self._policy])
         sa = self._sa = _lib.SelectArgs()
         sa.caches = ctypes.addressof(self._caches)
         sa.h_chunk_base, sa.n_chunks, sa.units_per_chunk = ctypes.addressof(self._chunk_base), 0, _HOST_CHUNK_UNITS
@@ -311,26 +604,26 @@ class ContextManager:
                                                       ctypes.addressof(self._n_miss_row))
         self._sa_ref = ctypes.byref(sa)
         self._fa_ref, self._ba_ref = ctypes.byref(self._fa), ctypes.byref(self._ba)
-        self.initialized = True
+        self._bind_reps()
 
     def _bind_call_buffers(self, stream):
         """Buffers of a call prepared in one go: the rotated queries of up to call_tokens tokens, the blocks' mean
         queries and the local stage's partial rows.  They are dead between append() calls, so the layers that work on
         one stream (one after the other, as the layers of a model do) share one set."""
         B, H, D, exc, T = self.num_units, self.unit_size, self.head_width, self.exc_block_size, self._call_tokens
-        group = int(os.environ.get("INFLLM_LOCAL_GROUP", self.local_group_blocks))
+        group = self._local_group
         blocks = max(8, 4 * group)            # partial rows: two groups of blocks, up to two key splits each
-        dev = self.device.index if self.device.index is not None else torch.cuda.current_device()
-        key = (dev, stream, B, H, D, T, exc, blocks)
+        key = (self._dev_index, stream, B, H, D, T, exc, blocks)
         buf = _CALL_BUFFERS.get(key)
         if buf is None:
             bf = dict(dtype=torch.bfloat16, device=self.device)
             f32 = dict(dtype=torch.float32, device=self.device)
-            buf = _CALL_BUFFERS[key] = dict(
+            buf = _Buffers(
                 q_loc=torch.empty((B, H, T, D), **bf), q_glb=torch.empty((B, H, T, D), **bf),
                 qpart=torch.empty((B, (T + 15) // 16, H * D), **f32), qbar=torch.empty((T // exc, B, H * D), **f32),
                 o_part=torch.empty((blocks * B * H * exc, D), dtype=torch.float16, device=self.device),
                 lse_part=torch.empty((blocks * B * H * exc,), **f32))
+            _CALL_BUFFERS[key] = buf
         self._call_buf = buf
         bd = _lib.BatchDesc()
         bd.d_q_loc, bd.d_q_glb = buf["q_loc"].data_ptr(), buf["q_glb"].data_ptr()
@@ -377,15 +670,23 @@ class ContextManager:
             self._host_copies_open = False
 
     def host_unit(self, unit):
-        """Pinned host tensor [B, 2, Hkv, bs, D] of a carved unit (K at index 0, V at 1); for heads narrower than 128 a
-        copy with the real dimensions picked out."""
+        """Pinned host tensor [B, 2, Hkv, bs, D] of a carved unit (K at index 0, V at 1); a copy where the unit is resident in
+        HBM, and for heads narrower than 128 one with the real dimensions picked out."""
+        if self._resident:
+            t = self._chunks[unit // _UNIT_CHUNK][unit % _UNIT_CHUNK]
+            host = torch.empty(t.shape, dtype=t.dtype, pin_memory=True)
+            return _narrow(host.copy_(t), self.dim_head) if t.shape[-1] != self.dim_head else host.copy_(t)
         self._finish_host_copies()
         return _narrow(self._host_unit_rows(unit), self.dim_head)
 
     def rep_rows(self, row, lo, hi):
         """Representatives of units [lo, hi) of batch row `row` as a CPU fp32 tensor [hi - lo, H * D]."""
         r = self.reps[row, lo:hi].view(hi - lo, self.unit_size, self.head_width)
-        return _narrow(r, self.dim_head).reshape(hi - lo, -1).float().cpu()
+        return self._own_width(r).reshape(hi - lo, -1).float().cpu()
+
+    def _own_width(self, t):
+        """rows of head_width elements -> rows of the heads' own width"""
+        return t if t.shape[-1] == self.dim_head else _narrow(t, self.dim_head)
 
     # ----------------------------------------------------------------- timing
     def enable_timing(self, capacity, stride=1):
@@ -393,6 +694,8 @@ class ContextManager:
         self._timing_cap, self._timing_stride = capacity, stride
         if self._layer:
             check(self._lib.infllm_layer_timing(self._layer, capacity, stride), "infllm_layer_timing")
+        if self._resident:
+            check(self._lib.infllm_resident_timing(self._resident, capacity, stride), "infllm_resident_timing")
 
     def prefetch_stats(self):
         """(guesses made, guesses that turned out to be the selection) of the fetch ahead of the selection."""
@@ -411,6 +714,9 @@ class ContextManager:
         counts = (ctypes.c_int64 * 6)()
         if self._layer:
             check(self._lib.infllm_layer_path_counts(self._layer, counts), "infllm_layer_path_counts")
+        if self._resident:
+            self._resident_books(False)
+            counts[5] = self._state[8]
         return dict(zip(("tables_inline", "tables_kernel", "tables_upload", "score_merged", "score_apart", "call_ranked"),
                         (int(c) for c in counts)))
 
@@ -422,7 +728,8 @@ class ContextManager:
         """[(ms, n_queries, n_keys)] of the timed launches; which = 0 local stage, 1 global stage."""
         cap = self._timing_cap
         ms, nq, nk = (ctypes.c_float * cap)(), (ctypes.c_int32 * cap)(), (ctypes.c_int32 * cap)()
-        n = self._lib.infllm_layer_read_timing(self._layer, which, ms, nq, nk, cap)
+        n = (self._lib.infllm_resident_read_timing(self._resident, which, ms, nq, nk, cap) if self._resident
+             else self._lib.infllm_layer_read_timing(self._layer, which, ms, nq, nk, cap))
         if n < 0:
             check(n, "infllm_layer_read_timing")
         return [(ms[i], nq[i], nk[i]) for i in range(n)]
@@ -450,12 +757,12 @@ class ContextManager:
         # ---- retrieval result (context_manager.py:366-383) -> cache policy (495-515) -> fetch, in one native call:
         #      this stretch is on the chain from one block's selection to the next, the rest of the host's work is not
         sa = self._sa
-        stats = self.stats
+        stats = self._stats
         if self._mass_units is not None:                     # lru-s: the previous block's masses decide this eviction
             check(lib.infllm_layer_wait_mass(layer), "infllm_layer_wait_mass")
             masses = self.mass_host.tolist()
             for u in range(B):
-                self.policy[u].add_scores(self._mass_units[u], masses[u][:len(self._mass_units[u])])
+                self._policy[u].add_scores(self._mass_units[u], masses[u][:len(self._mass_units[u])])
             self._mass_units = None
         # ---- state machine after the block (context_manager.py:614-679): it does not depend on the selection, so the
         #      arguments of the block's second half are ready before the host waits for the ids
@@ -516,8 +823,8 @@ class ContextManager:
                 selected = [self._sel_ids[u * n_sel:(u + 1) * n_sel] for u in range(B)]
             stats["evictions"] += sum(self._n_evicted[:B])
             for u in range(B):
-                if self.policy[u].evicted_log is not None:
-                    self.policy[u].evicted_log.append(list(self._evicted[u * n_sel:u * n_sel + self._n_evicted[u]]))
+                if self._policy[u].evicted_log is not None:
+                    self._policy[u].evicted_log.append(list(self._evicted[u * n_sel:u * n_sel + self._n_evicted[u]]))
         stats["hits"] += B * n_sel - n_miss
         stats["misses"] += n_miss
         if self.cache_strategy == "lru":
@@ -552,9 +859,9 @@ class ContextManager:
             selected = self.topk_idx_host.tolist()
         n_sel, n_miss = len(selected[0]), 0
         for u in range(B):
-            pol = self.policy[u]
+            pol = self._policy[u]
             misses, evicted = pol.touch(selected[u])
-            self.stats["evictions"] += len(evicted)
+            self._stats["evictions"] += len(evicted)
             slot_of = pol.slot_of
             for i, unit in enumerate(selected[u]):
                 self._sel_slots[u * n_sel + i] = slot_of[unit]
@@ -599,12 +906,12 @@ class ContextManager:
     def _grow_reps(self, need):
         B, N = self.num_units, self.num_global_block
         rows = max(2 * self.reps.shape[1], need)
-        grown = torch.zeros((B, rows, self.reps.shape[2]), dtype=torch.bfloat16, device=self.device)
+        grown = torch.empty((B, rows, self.reps.shape[2]), dtype=torch.bfloat16, device=self.device)
         grown[:, :N] = self.reps[:, :N]
         scores = torch.empty((B, rows), dtype=torch.float32, device=self.device)
         scores[:, :N] = self.unit_scores[:, :N]          # scores prepared ahead for the next block
         self.reps, self.unit_scores = grown, scores
-        self._bind_reps()
+        self._bind_resident_reps() if self._resident else self._bind_reps()
 
     def _bind_reps(self):
         fa, ba = self._fa, self._ba
@@ -639,16 +946,26 @@ class ContextManager:
             check_head_dim(self.dim_head)
         if q.size(3) != self.dim_head:
             raise ValueError(f"head_dim changed from {self.dim_head} to {q.size(3)}")
-        q, k, v = _widen(q, self.dim_head), _widen(k, self.dim_head), _widen(v, self.dim_head)
         if not self.initialized:
             self._init(q, k)
-            self._bind_reps()
+        if self._resident and not self._wants_resident():
+            self._leave_resident()
+        if self.head_width != self.dim_head:
+            q, k, v = _widen(q, self.dim_head), _widen(k, self.dim_head), _widen(v, self.dim_head)
         assert q.shape[:2] == (self.num_units, self.unit_size) and k.shape[1] == self.unit_size_kv
 
         def rows16(t):          # rows must be contiguous and 16-byte aligned for the vector loads
             ok = t.stride(-1) == 1 and not any(s % 8 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0
             return t if ok else t.contiguous()
         q, k, v = rows16(q), rows16(k), rows16(v)
+        if self._resident:
+            out = self._append_resident(q, k, v, input_length)
+            if out is not None:
+                out = self._own_width(out)
+                return out.reshape(batch_size, heads, input_length, -1) if self.perhead else out
+            self._leave_resident()
+            if self.head_width != q.shape[-1]:
+                q, k, v = (_widen(t, self.dim_head) for t in (q, k, v))
         out = torch.empty((self.num_units, self.unit_size, input_length, self.head_width), dtype=torch.bfloat16, device=q.device)
         fa, ba = self._fa, self._ba
         fa.q_sb, fa.q_sh, fa.q_sl = q.stride(0), q.stride(1), q.stride(2)
@@ -706,7 +1023,7 @@ class ContextManager:
         # (the last carved units go on to their pinned home in the background: _finish_host_copies before reading them)
         check(self._lib.infllm_layer_end_call(self._layer, self._copy_raw), "infllm_layer_end_call")
         self._host_copies_open = True
-        out = _narrow(out, self.dim_head)
+        out = self._own_width(out)
         if self.perhead:
             out = out.view(batch_size, heads, input_length, -1)
         return out
@@ -721,15 +1038,19 @@ class ContextManager:
         torch.cuda.synchronize()
         T, cur, cap = self.length, self.cursor, self.ring_cap
         rows = torch.arange(cur, T, device=self.device) % cap
-        units = [self.host_unit(u).clone() for u in range(self.num_global_block)] if with_units else []
-        d, n = self.dim_head, self.num_global_block
-        reps = _narrow(self.reps[:, :n].view(self.num_units, n, self.unit_size, self.head_width), d).reshape(self.num_units, n, -1)
+        if with_units and self._resident and self.num_global_block:
+            units = self._own_width(torch.cat([c.cpu() for c in self._chunks])[:self.num_global_block])
+        else:
+            units = [self.host_unit(u).clone() for u in range(self.num_global_block)] if with_units else []
+            units = torch.stack(units) if units else None
+        own, n = self._own_width, self.num_global_block
+        reps = own(self.reps[:, :n].view(self.num_units, n, self.unit_size, self.head_width)).reshape(self.num_units, n, -1)
         return dict(length=T, n_units=n, init_len=self.init_len,
-                    tail_k=_narrow(self.ring_k_raw[:, :, rows], d).clone(), tail_v=_narrow(self.ring_v[:, :, rows], d).clone(),
+                    tail_k=own(self.ring_k_raw[:, :, rows]).clone(), tail_v=own(self.ring_v[:, :, rows]).clone(),
                     tail_score=self.ring_score[:, :, rows].clone(),
-                    init_k=_narrow(self.init_kv[:, 0, :, :self.init_len], d).clone(),
-                    init_v=_narrow(self.init_kv[:, 1, :, :self.init_len], d).clone(),
-                    units=torch.stack(units) if units else None, reps=reps.clone())
+                    init_k=own(self.init_kv[:, 0, :, :self.init_len]).clone(),
+                    init_v=own(self.init_kv[:, 1, :, :self.init_len]).clone(),
+                    units=units, reps=reps.clone())
 
     def load_state(self, state):
         """Start from a prepared memory.  ``state``: length T; tail_k/tail_v [B,Hkv,T-cursor,D] (un-rotated,
@@ -737,46 +1058,61 @@ class ContextManager:
         init_k/init_v [B,Hkv,init_len,D]; units [n_units,B,2,Hkv,bs,D] (any device) or None; reps
         [B,n_units,H*D].  The counts must satisfy the stream's closed forms (context_manager.py:614-679):
         init_len = min(n_init, max(T-n_local, 0)), n_units = max(0, (T-n_init-n_local)//block_size)."""
+        return self._load(state)
+
+    def _load(self, state, resident=None, unit_at=None):
+        """load_state; unit_at(u): a unit in rows of any width, in place of state["units"]."""
         from .. import ops
         assert not self.initialized and self.length == 0, "load_state needs a fresh ContextManager"
         tail_k, tail_v = state["tail_k"], state["tail_v"]
         T = int(state["length"])
         B, Hkv, n_tail, D = tail_k.shape
         reps = state["reps"]
-        H = reps.shape[2] // D if reps is not None and reps.numel() else state["num_heads"]
+        H = reps.shape[2] // D if reps is not None and reps.numel() else state["tail_score"].shape[1] if state.get("tail_score") is not None else state["num_heads"]
         init_len = min(self.n_init, max(T - self.n_local, 0))
         n_units = max(0, (T - self.n_init - self.n_local) // self.block_size)
         cursor = init_len + n_units * self.block_size
         assert n_tail == T - cursor, f"tail holds {n_tail} tokens, the stream state needs {T - cursor}"
-        assert state["init_k"].shape[2] == init_len and (n_units == 0 or state["units"].shape[0] == n_units)
+        assert state["init_k"].shape[2] == init_len and (n_units == 0 or unit_at is not None or state["units"].shape[0] == n_units)
         check_head_dim(D)
         self.dim_head = D
-        tail_k, tail_v = _widen(tail_k, D), _widen(tail_v, D)
-        q_like = torch.empty((B, H, 1, HEAD_DIM), dtype=torch.bfloat16, device=tail_k.device)
-        self._init(q_like, tail_k[:, :, :1])
-        self._bind_reps()
+        q_like = torch.empty((B, H, 1, D), dtype=torch.bfloat16, device=tail_k.device)
+        self._init(q_like, tail_k[:, :, :1], resident)
+        if self._resident and n_units and not self._add_chunks(n_units):
+            self._drop_resident()
+            self._init(q_like, tail_k[:, :, :1], False)
+        W = self.head_width
+        wide = lambda t: t if t.shape[-1] == W else _widen(t, t.shape[-1])
         self.length, self.cursor, self.init_len = T, cursor, init_len
         if init_len:
-            self.init_kv[:, 0, :, :init_len] = _widen(state["init_k"], D)
-            self.init_kv[:, 1, :, :init_len] = _widen(state["init_v"], D)
+            self.init_kv[:, 0, :, :init_len] = wide(state["init_k"])
+            self.init_kv[:, 1, :, :init_len] = wide(state["init_v"])
         if n_units:
             self._grow_reps(n_units) if n_units > self.reps.shape[1] else None
-            self.reps[:, :n_units] = _widen(reps.view(B, n_units, H, D), D).reshape(B, n_units, -1)
-            for u in range(n_units):
-                self._host_unit_addr(u)                        # allocates the pinned chunk
-                self._host_unit_rows(u).copy_(_widen(state["units"][u], D))
+            self.reps[:, :n_units] = wide(reps.view(B, n_units, H, D)).reshape(B, n_units, -1)
+            if self._resident:
+                for u in range(0, n_units, _UNIT_CHUNK):
+                    n = min(_UNIT_CHUNK, n_units - u)
+                    self._chunks[u // _UNIT_CHUNK][:n] = wide(state["units"][u:u + n])
+            else:
+                for u in range(n_units):
+                    self._host_unit_addr(u)                        # allocates the pinned chunk
+                    self._host_unit_rows(u).copy_(wide(state["units"][u] if unit_at is None else unit_at(u)))
             self.num_global_block = n_units
         # tail -> rings (RoPE at the absolute positions) in pieces of one execution block
-        D = HEAD_DIM
-        zq = torch.zeros((B, H, self.exc_block_size, D), dtype=torch.bfloat16, device=self.device)
-        for st in range(0, n_tail, self.exc_block_size):
-            n = min(self.exc_block_size, n_tail - st)
+        tail_k, tail_v = wide(tail_k), wide(tail_v)
+        exc = self.exc_block_size
+        zq = torch.zeros((B, H, exc, W), dtype=torch.bfloat16, device=self.device)
+        for st in range(0, n_tail, exc):
+            n = min(exc, n_tail - st)
             ops.ingest(zq[:, :, :n], tail_k[:, :, st:st + n], tail_v[:, :, st:st + n], cursor + st, self.n_local - 1,
                        self.inv_freq, float(self.position_embedding.distance_scale), self.ring_k_raw, self.ring_k_rot,
-                       self.ring_v, self.ring_score, self.q_loc[0], self.q_glb[0])
+                       self.ring_v, self.ring_score, torch.empty_like(zq), torch.empty_like(zq))
         if state.get("tail_score") is not None:
             rows = torch.arange(cursor, T, device=self.device) % self.ring_cap
             self.ring_score[:, :, rows] = state["tail_score"].to(torch.float32)
+        if self._resident:
+            check(self._lib.infllm_resident_set_state(self._resident, T, cursor, init_len, n_units), "infllm_resident_set_state")
         torch.cuda.synchronize()
         return self
 

@@ -855,7 +855,7 @@ extern "C" int infllm_attn_stage(const infllm_attn_args *a, void *stream) {
             const int64_t row = pos % a->cap, n = std::min(hi - pos, a->cap - row);
             INFLLM_REQUIRE(n < (1ll << 31), "attn_stage: key range too long");
             d.seg[d.n_seg++] = DecodeSeg{(const bf16_t *)a->d_k + row * kD, (const bf16_t *)a->d_v + row * kD, a->k_sb, a->k_sh, a->v_sb, a->v_sh, (int32_t)n,
-                                         0, 0, nullptr};
+                                         0, 0, nullptr, -1};
             pos += n;
         }
         if (d.n_seg == 0) d.n_seg = 1;                 // nothing visible: empty partials
@@ -878,7 +878,7 @@ extern "C" int infllm_attn_stage_splits(const infllm_attn_args *a, int32_t max_s
 // library-internal: a linear stage over the queries of several consecutive execution blocks of `exc` rows (the last
 // may be shorter); block k's partial rows and log-sum-exps start at row k * block_rows of d_o_part / d_lse_part and
 // are laid out [nsplit, B, H, n_k, 128] / [nsplit, B, H, n_k], as infllm_attn_merge takes them for that block.
-int infllm_attn_stage_blocked(const infllm_attn_args *a, int32_t exc, int64_t block_rows, void *stream) {
+int infllm_attn_stage_blocked(const infllm_attn_args *a, int32_t exc, int64_t block_rows, void *stream, int32_t dim) {
     INFLLM_REQUIRE(a && a->d_o_part && a->d_lse_part && !a->d_pages, "attn_stage_blocked: null argument or paged source");
     INFLLM_REQUIRE(exc > 0 && exc % kQTile == 0, "attn_stage_blocked: blocks of %d rows are not whole query tiles", exc);
     INFLLM_REQUIRE(block_rows >= (int64_t)a->nsplit * a->B * a->H * (a->Lq < exc ? a->Lq : exc), "attn_stage_blocked: block stride too small");
@@ -889,7 +889,18 @@ int infllm_attn_stage_blocked(const infllm_attn_args *a, int32_t exc, int64_t bl
     StageOut so;
     so.out_exc = exc;
     so.out_block_rows = block_rows;
-    return launch_stage(kLinear, a, nullptr, stream, nullptr, so);
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "attn_stage_blocked: head_dim %d", dim);
+    return dim == 128 ? launch_stage<128>(kLinear, a, nullptr, stream, nullptr, so) : launch_stage<64>(kLinear, a, nullptr, stream, nullptr, so);
+}
+
+// library-internal: the paged stage over a table in device memory, or (h_pages != NULL, B * n_pages <=
+// infllm_inline_page_limit()) one in host memory that the launch carries, for heads of 128 or 64
+int infllm_attn_paged(const infllm_attn_args *a, const infllm_page *h_pages, void *stream, int32_t dim) {
+    INFLLM_REQUIRE(a && a->d_o_part && a->d_lse_part && (h_pages || a->d_pages) && a->n_pages >= 0, "attn_paged: null argument");
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "attn_paged: head_dim %d", dim);
+    const int rc = check_common(a);
+    if (rc) return rc;
+    return dim == 128 ? launch_stage<128>(kPaged, a, nullptr, stream, h_pages) : launch_stage<64>(kPaged, a, nullptr, stream, h_pages);
 }
 
 // library-internal: the paged stage (local == NULL) or both stages in one launch, with the page table [B, n_pages]

@@ -14,6 +14,7 @@ struct DecodeSeg {
     int32_t rows, q;                       // q: which of the job's two rotations of the query this range is attended with
     int32_t n_ids;
     const int32_t *ids;                    // [B, n_ids] on the device, NULL: a plain range
+    int32_t logit0;                        // row r's scaled logit goes to logits[.., logit0 + r]; -1: not kept
 };
 
 struct DecodeJob {
@@ -29,8 +30,7 @@ struct DecodeJob {
     const uint64_t *chunk;                 // device: address of every chunk of units
     int32_t per_chunk;
     int64_t unit_elems, row_elems, unit_v_off, unit_sh;
-    // scaled logits of seg[0] in base 2 (optional): [B, H, logit_stride], row r of the range at r
-    float *logits;
+    float *logits;                         // optional [B, H, logit_stride]: scaled logits in base 2 (see DecodeSeg)
     int64_t logit_stride;
 };
 

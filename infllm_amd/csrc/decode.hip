@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
 
     struct Block {
         const bf16_t *k, *v;
-        int valid, q, row;                         // rows of the block, which query, first row (ranges) or -1
+        int valid, q, row;                         // rows of the block, which query, where its logits go (-1: nowhere)
     };
     auto find = [&](int blk) {                     // wave-uniform
         Block r{nullptr, nullptr, 0, 0, -1};
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
                 r.k = sg.k + (int64_t)b * sg.k_sb + (int64_t)g * sg.k_sh + (int64_t)r0 * D;
                 r.v = sg.v + (int64_t)b * sg.v_sb + (int64_t)g * sg.v_sh + (int64_t)r0 * D;
                 r.valid = min(kDecodeBlock, sg.rows - r0);
-                if (s == 0) r.row = r0;
+                if (LOGITS && sg.logit0 >= 0) r.row = sg.logit0 + r0;
             }
             return r;
         }

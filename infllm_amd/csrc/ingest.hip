@@ -5,8 +5,6 @@
 
 namespace {
 
-constexpr int kHalf = kD / 2;      // 64 rotation pairs per head
-
 // grid = (position tiles of 16, batch rows, kv heads): a workgroup rotates the query heads of one
 // kv-head group plus that group's key head, copies its value head, and leaves the sum of its
 // rotated-to-one-position queries over its positions in d_qpart (for the block's mean query; summed
@@ -14,10 +12,15 @@ constexpr int kHalf = kD / 2;      // 64 rotation pairs per head
 //
 // Angles (rope_angles): the rows the workgroup will rotate are requested from memory BEFORE that arithmetic, so the
 // two overlap.
-__global__ __launch_bounds__(256) void ingest_kernel(infllm_ingest_args a) {
+//
+// D: head dimension (128 or 64).  qbar (optional): where the mean of the queries goes when the launch has a single
+// position tile (a decode step), whose partial sum is the whole sum.
+template <int D>
+__global__ __launch_bounds__(256) void ingest_kernel(infllm_ingest_args a, float *qbar) {
+    constexpr int kHalf = D / 2, C2 = D / 16;          // rotation pairs of a head; pairs of 16-byte chunks of a row
     __shared__ float2 cs_pos[kPosPerBlock][kHalf];
     __shared__ float2 cs_glb[kHalf];
-    __shared__ float red[4][kPosPerBlock][kD];        // q_glb of 4 heads x 16 positions, for the partial sums
+    __shared__ float red[4][kPosPerBlock][D];        // q_glb of 4 heads x 16 positions, for the partial sums
     const int tid = threadIdx.x;
     const int b = blockIdx.y, g = blockIdx.z;
     const int G = a.H / a.Hkv;
@@ -27,34 +30,34 @@ __global__ __launch_bounds__(256) void ingest_kernel(infllm_ingest_args a) {
     const bf16_t *q = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb;
     const bf16_t *k = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh;
     const bf16_t *v = (const bf16_t *)a.d_v + (int64_t)b * a.v_sb + (int64_t)g * a.v_sh;
-    bf16_t *q_loc = (bf16_t *)a.d_q_loc + (int64_t)b * a.H * a.n * kD;
-    bf16_t *q_glb = (bf16_t *)a.d_q_glb + (int64_t)b * a.H * a.n * kD;
-    const int64_t ring_g = ((int64_t)b * a.Hkv + g) * a.ring_cap * kD;
+    bf16_t *q_loc = (bf16_t *)a.d_q_loc + (int64_t)b * a.H * a.n * D;
+    bf16_t *q_glb = (bf16_t *)a.d_q_glb + (int64_t)b * a.H * a.n * D;
+    const int64_t ring_g = ((int64_t)b * a.Hkv + g) * a.ring_cap * D;
     bf16_t *rk_raw = (bf16_t *)a.d_ring_k_raw + ring_g;
     bf16_t *rk_rot = (bf16_t *)a.d_ring_k_rot + ring_g;
     bf16_t *rv = (bf16_t *)a.d_ring_v + ring_g;
     const int n_tiles = (a.n + kPosPerBlock - 1) / kPosPerBlock;
 
     // ---- requests first: the first group of (up to) 4 query heads, the key head, the value head
-    constexpr int kQItems = 2;                        // 4 heads x 16 positions x 8 chunk pairs = 512 items over 256 threads
+    constexpr int kQItems = 4 * kPosPerBlock * C2 / 256;   // 4 heads x 16 positions x 8 (4) chunk pairs over 256 threads
     u32x4 q_lo[kQItems], q_hi[kQItems], k_lo, k_hi, v_row;
     const int nh0 = min(4, G);
 #pragma unroll
     for (int i = 0; i < kQItems; ++i) {
         const int e = tid + i * 256;
-        if (e < nh0 * np * 8) {
-            const int c = e & 7, p = (e >> 3) % np, hl = (e >> 3) / np;
+        if (e < nh0 * np * C2) {
+            const int c = e % C2, p = e / C2 % np, hl = e / C2 / np;
             const bf16_t *src = q + (int64_t)(g * G + hl) * a.q_sh + (int64_t)(p0 + p) * a.q_sl;
             q_lo[i] = *(const u32x4 *)(src + c * 8);
             q_hi[i] = *(const u32x4 *)(src + kHalf + c * 8);
         }
     }
-    if (tid < np * 8) {
-        const bf16_t *src = k + (int64_t)(p0 + (tid >> 3)) * a.k_sl;
-        k_lo = *(const u32x4 *)(src + (tid & 7) * 8);
-        k_hi = *(const u32x4 *)(src + kHalf + (tid & 7) * 8);
+    if (tid < np * C2) {
+        const bf16_t *src = k + (int64_t)(p0 + tid / C2) * a.k_sl;
+        k_lo = *(const u32x4 *)(src + tid % C2 * 8);
+        k_hi = *(const u32x4 *)(src + kHalf + tid % C2 * 8);
     }
-    if (tid < np * 16) v_row = *(const u32x4 *)(v + (int64_t)(p0 + (tid >> 4)) * a.v_sl + (tid & 15) * 8);
+    if (tid < np * 2 * C2) v_row = *(const u32x4 *)(v + (int64_t)(p0 + tid / (2 * C2)) * a.v_sl + tid % (2 * C2) * 8);
 
     // ---- angles
     rope_angles<kHalf>(a.pos0 + p0, np, a.glb_pos, a.distance_scale, a.d_inv_freq, cs_pos, cs_glb);
@@ -66,15 +69,15 @@ __global__ __launch_bounds__(256) void ingest_kernel(infllm_ingest_args a) {
 #pragma unroll
         for (int i = 0; i < kQItems; ++i) {
             const int e = tid + i * 256;
-            if (e >= nh * np * 8) continue;
-            const int c = e & 7, p = (e >> 3) % np, hl = (e >> 3) / np;
+            if (e >= nh * np * C2) continue;
+            const int c = e % C2, p = e / C2 % np, hl = e / C2 / np;
             const int h = g * G + hg0 + hl;
             u32x4 lo = q_lo[i], hi = q_hi[i];
             if (hg0 > 0) {
                 const bf16_t *src = q + (int64_t)h * a.q_sh + (int64_t)(p0 + p) * a.q_sl;
                 lo = *(const u32x4 *)(src + c * 8), hi = *(const u32x4 *)(src + kHalf + c * 8);
             }
-            int64_t o = ((int64_t)h * a.n + p0 + p) * kD;
+            int64_t o = ((int64_t)h * a.n + p0 + p) * D;
             Rot8 r = rotate8(lo, hi, &cs_pos[p][c * 8]);
             *(u32x4 *)(q_loc + o + c * 8) = r.lo;
             *(u32x4 *)(q_loc + o + kHalf + c * 8) = r.hi;
@@ -82,36 +85,37 @@ __global__ __launch_bounds__(256) void ingest_kernel(infllm_ingest_args a) {
             r = rotate8(lo, hi, &cs_glb[c * 8], raw);
             *(u32x4 *)(q_glb + o + c * 8) = r.lo;
             *(u32x4 *)(q_glb + o + kHalf + c * 8) = r.hi;
-            if (a.d_qpart) {
+            if (a.d_qpart || qbar) {
                 *(f32x4 *)&red[hl][p][c * 8] = f32x4{raw[0], raw[1], raw[2], raw[3]};
                 *(f32x4 *)&red[hl][p][c * 8 + 4] = f32x4{raw[4], raw[5], raw[6], raw[7]};
                 *(f32x4 *)&red[hl][p][kHalf + c * 8] = f32x4{raw[8], raw[9], raw[10], raw[11]};
                 *(f32x4 *)&red[hl][p][kHalf + c * 8 + 4] = f32x4{raw[12], raw[13], raw[14], raw[15]};
             }
         }
-        if (a.d_qpart) {
+        if (a.d_qpart || qbar) {
             __syncthreads();
-            for (int e = tid; e < nh * kD; e += 256) {
-                const int d = e % kD, hl = e / kD;
+            for (int e = tid; e < nh * D; e += 256) {
+                const int d = e % D, hl = e / D;
                 float s = 0.f;
                 for (int p = 0; p < np; ++p) s += red[hl][p][d];          // fixed order
-                a.d_qpart[(((int64_t)b * n_tiles + blockIdx.x) * a.H + g * G + hg0 + hl) * kD + d] = s;
+                if (qbar) qbar[((int64_t)b * a.H + g * G + hg0 + hl) * D + d] = s * (1.f / (float)a.n);
+                else a.d_qpart[(((int64_t)b * n_tiles + blockIdx.x) * a.H + g * G + hg0 + hl) * D + d] = s;
             }
             __syncthreads();
         }
     }
     // key head: raw copy + rotated copy into the rings
-    if (tid < np * 8) {
-        const int c = tid & 7, p = tid >> 3;
-        const int64_t o = ((a.pos0 + p0 + p) % a.ring_cap) * kD;
+    if (tid < np * C2) {
+        const int c = tid % C2, p = tid / C2;
+        const int64_t o = ((a.pos0 + p0 + p) % a.ring_cap) * D;
         *(u32x4 *)(rk_raw + o + c * 8) = k_lo;
         *(u32x4 *)(rk_raw + o + kHalf + c * 8) = k_hi;
         Rot8 r = rotate8(k_lo, k_hi, &cs_pos[p][c * 8]);
         *(u32x4 *)(rk_rot + o + c * 8) = r.lo;
         *(u32x4 *)(rk_rot + o + kHalf + c * 8) = r.hi;
     }
-    // value head: plain copy, 16 threads per row
-    if (tid < np * 16) *(u32x4 *)(rv + ((a.pos0 + p0 + (tid >> 4)) % a.ring_cap) * kD + (tid & 15) * 8) = v_row;
+    // value head: plain copy
+    if (tid < np * 2 * C2) *(u32x4 *)(rv + ((a.pos0 + p0 + tid / (2 * C2)) % a.ring_cap) * D + tid % (2 * C2) * 8) = v_row;
     // the score track of a new token starts at zero (context_manager.py:733-741)
     for (int e = tid; e < G * np; e += 256) {
         const int p = e % np, h = g * G + e / np;
@@ -250,6 +254,7 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(const bf16_t *x, int64_t
 }
 
 // grid.z = B, or 2*B to gather from a second ring (ring2 -> out2, same geometry) in the same launch
+template <int D>
 __global__ __launch_bounds__(256) void gather_rows_kernel(const bf16_t *ring, int64_t ring_cap, int Hkv, int64_t t0,
                                                           int n, int unit_rows, bf16_t *out, int64_t out_sb,
                                                           int64_t out_su, int64_t out_sh, int B, const bf16_t *ring2, bf16_t *out2) {
@@ -259,17 +264,17 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const bf16_t *ring, in
         out = out2;
     }
     const int e = blockIdx.x * 256 + threadIdx.x;      // (row, 16-byte chunk)
-    if (e >= n * 16) return;
-    int r = e >> 4, c = e & 15;
+    if (e >= n * (D / 8)) return;
+    int r = e / (D / 8), c = e % (D / 8);
     int64_t row = (t0 + r) % ring_cap;
-    const bf16_t *src = ring + (((int64_t)b * Hkv + h) * ring_cap + row) * kD + c * 8;
+    const bf16_t *src = ring + (((int64_t)b * Hkv + h) * ring_cap + row) * D + c * 8;
     *(u32x4 *)(out + (int64_t)b * out_sb + (int64_t)(r / unit_rows) * out_su + (int64_t)h * out_sh +
-               (int64_t)(r % unit_rows) * kD + c * 8) = *(const u32x4 *)src;
+               (int64_t)(r % unit_rows) * D + c * 8) = *(const u32x4 *)src;
 }
 
 }  // namespace
 
-extern "C" int infllm_ingest(const infllm_ingest_args *a, void *stream) {
+extern "C" int infllm_ingest_dim(const infllm_ingest_args *a, int32_t dim, float *d_qbar, void *stream) {
     INFLLM_REQUIRE(a != nullptr, "ingest: null argument block");
     INFLLM_REQUIRE(a->d_q && a->d_k && a->d_v && a->d_inv_freq, "ingest: null input pointer");
     INFLLM_REQUIRE(a->d_ring_k_raw && a->d_ring_k_rot && a->d_ring_v && a->d_ring_score && a->d_q_loc && a->d_q_glb,
@@ -282,12 +287,17 @@ extern "C" int infllm_ingest(const infllm_ingest_args *a, void *stream) {
     INFLLM_REQUIRE((a->q_sl % 8 | a->q_sh % 8 | a->q_sb % 8 | a->k_sl % 8 | a->k_sh % 8 | a->k_sb % 8 | a->v_sl % 8 |
                     a->v_sh % 8 | a->v_sb % 8) == 0,
                    "ingest: strides must be multiples of 8 elements (16-byte rows)");
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "ingest: head_dim %d", dim);
+    INFLLM_REQUIRE(!d_qbar || a->n <= kPosPerBlock, "ingest: the mean of %d queries takes more than one tile", a->n);
     if (a->n == 0) return 0;
     dim3 grid((a->n + kPosPerBlock - 1) / kPosPerBlock, a->B, a->Hkv);
-    hipLaunchKernelGGL(ingest_kernel, grid, dim3(256), 0, (hipStream_t)stream, *a);
+    if (dim == 128) hipLaunchKernelGGL(ingest_kernel<128>, grid, dim3(256), 0, (hipStream_t)stream, *a, d_qbar);
+    else hipLaunchKernelGGL(ingest_kernel<64>, grid, dim3(256), 0, (hipStream_t)stream, *a, d_qbar);
     INFLLM_CHECK_LAUNCH("ingest");
     return 0;
 }
+
+extern "C" int infllm_ingest(const infllm_ingest_args *a, void *stream) { return infllm_ingest_dim(a, kD, nullptr, stream); }
 
 extern "C" int infllm_reduce_partials(const float *d_parts, int32_t B, int32_t n_parts, int32_t C, float scale, float *d_out,
                                       void *stream) {
@@ -355,23 +365,25 @@ extern "C" int infllm_gather_rows(const void *d_ring, int64_t ring_cap, int32_t 
     INFLLM_REQUIRE(unit_rows > 0, "gather_rows: unit_rows must be positive");
     INFLLM_REQUIRE((out_sb % 8 | out_su % 8 | out_sh % 8) == 0, "gather_rows: output strides must be multiples of 8");
     if (n == 0) return 0;
-    hipLaunchKernelGGL(gather_rows_kernel, dim3((n * 16 + 255) / 256, Hkv, B), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(gather_rows_kernel<kD>, dim3((n * 16 + 255) / 256, Hkv, B), dim3(256), 0, (hipStream_t)stream,
                        (const bf16_t *)d_ring, ring_cap, Hkv, t0, n, unit_rows, (bf16_t *)d_out, out_sb, out_su, out_sh, B,
                        (const bf16_t *)nullptr, (bf16_t *)nullptr);
     INFLLM_CHECK_LAUNCH("gather_rows");
     return 0;
 }
 
-// internal: the K and the V rows of the same stream positions in one launch (same arguments as infllm_gather_rows)
+// internal: the K and the V rows of the same stream positions in one launch (same arguments as infllm_gather_rows; rows of
+// `dim` elements)
 int infllm_gather_rows_pair(const void *d_ring_a, void *d_out_a, const void *d_ring_b, void *d_out_b, int64_t ring_cap, int32_t B,
                             int32_t Hkv, int64_t t0, int32_t n, int32_t unit_rows, int64_t out_sb, int64_t out_su, int64_t out_sh,
-                            void *stream) {
+                            void *stream, int32_t dim) {
     INFLLM_REQUIRE(d_ring_a && d_out_a && d_ring_b && d_out_b, "gather_rows: null pointer");
     INFLLM_REQUIRE(B > 0 && Hkv > 0 && ring_cap > 0 && n >= 0 && n <= ring_cap && t0 >= 0 && unit_rows > 0, "gather_rows: bad sizes");
     INFLLM_REQUIRE((out_sb % 8 | out_su % 8 | out_sh % 8) == 0, "gather_rows: output strides must be multiples of 8");
     if (n == 0) return 0;
-    hipLaunchKernelGGL(gather_rows_kernel, dim3((n * 16 + 255) / 256, Hkv, 2 * B), dim3(256), 0, (hipStream_t)stream,
-                       (const bf16_t *)d_ring_a, ring_cap, Hkv, t0, n, unit_rows, (bf16_t *)d_out_a, out_sb, out_su, out_sh, B,
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "gather_rows: head_dim %d", dim);
+    hipLaunchKernelGGL((dim == 64 ? gather_rows_kernel<64> : gather_rows_kernel<128>), dim3((n * (dim / 8) + 255) / 256, Hkv, 2 * B), dim3(256), 0,
+                       (hipStream_t)stream, (const bf16_t *)d_ring_a, ring_cap, Hkv, t0, n, unit_rows, (bf16_t *)d_out_a, out_sb, out_su, out_sh, B,
                        (const bf16_t *)d_ring_b, (bf16_t *)d_out_b);
     INFLLM_CHECK_LAUNCH("gather_rows");
     return 0;

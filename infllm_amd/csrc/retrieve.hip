@@ -543,26 +543,28 @@ __device__ __forceinline__ void select_topk_block(const float *scores, int N, in
     }
 }
 
-template <int CPL, int ROWS>
-__global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16_t *reps, int64_t rep_stride, int N, const float *qbar,
+// CPL: 512-element pieces of a row; TAIL: the row is shorter than that (C elements; the lanes beyond it hold zeros)
+template <int CPL, int ROWS, bool TAIL>
+__global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16_t *reps, int64_t rep_stride, int N, int C_, const float *qbar,
                                                                       float *scores, int k, int32_t *idx_out, int32_t *idx_out2,
                                                                       int32_t *flag, int32_t flag_value, int ticket_slot) {
     extern __shared__ float qs[];                                // the mean query
     __shared__ int is_last;
-    constexpr int C = CPL * 512;
+    const int C = TAIL ? C_ : CPL * 512;
     const int lane = threadIdx.x & 63;
     const int waves_per_wg = kRetrThreads / 64;
     const int n_waves = gridDim.x * waves_per_wg;
     int n = blockIdx.x * waves_per_wg + (threadIdx.x >> 6);     // rows n, n + n_waves, ... belong to this wave
+    auto in_row = [&](int j) { return !TAIL || j * 512 + lane * 8 < C; };
     u32x4 w[ROWS][CPL];
 #pragma unroll
     for (int r = 0; r < ROWS; ++r)
         if (n + r * n_waves < N) {
             const bf16_t *row = reps + (int64_t)(n + r * n_waves) * rep_stride + lane * 8;
 #pragma unroll
-            for (int j = 0; j < CPL; ++j) w[r][j] = __builtin_nontemporal_load((const u32x4 *)(row + j * 512));
+            for (int j = 0; j < CPL; ++j) w[r][j] = in_row(j) ? __builtin_nontemporal_load((const u32x4 *)(row + j * 512)) : u32x4{0, 0, 0, 0};
         }
-    for (int e = threadIdx.x * 4; e < C; e += kRetrThreads * 4) *(f32x4 *)(qs + e) = *(const f32x4 *)(qbar + e);
+    for (int e = threadIdx.x * 4; e < CPL * 512; e += kRetrThreads * 4) *(f32x4 *)(qs + e) = e < C ? *(const f32x4 *)(qbar + e) : f32x4{0.f, 0.f, 0.f, 0.f};
     __syncthreads();
     float q[CPL][8];
 #pragma unroll
@@ -589,7 +591,7 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
             if (nxt < N) {
                 const bf16_t *row = reps + (int64_t)nxt * rep_stride + lane * 8;
 #pragma unroll
-                for (int j = 0; j < CPL; ++j) w[r][j] = __builtin_nontemporal_load((const u32x4 *)(row + j * 512));
+                for (int j = 0; j < CPL; ++j) w[r][j] = in_row(j) ? __builtin_nontemporal_load((const u32x4 *)(row + j * 512)) : u32x4{0, 0, 0, 0};
             }
             const float acc = wave_sum(acc0 + acc1);
             if (lane == 0) __hip_atomic_store(scores + cur, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -624,70 +626,100 @@ struct CarveCopy {
     int32_t Hkv, B, n, unit_rows, x_extra;         // n rows from t0 on; x_extra = extra workgroups along x (0: no copy)
 };
 
-// one wave per (query head, unit, batch row); workgroups with blockIdx.x >= H copy
+// One wave per (query head, unit, batch row); workgroups with blockIdx.x >= H copy.  A chain of latencies (scores, repr_topk
+// arg-max steps, the chosen rows), so it is kept short: up to 256 scores live in registers as 64-bit composites (order of
+// the score, lower row first), an arg-max is a wave-wide maximum of those, and the rows of four picks are requested
+// together (four picks of 128: 8.3 -> 5 us with the arg-max through LDS and a row per step before).  Larger units go
+// through LDS.  NaN scores never win; a unit without a finite score still yields valid rows.
+template <int D>
 __global__ __launch_bounds__(64) void repr_keys_kernel(const float *ring_score, const bf16_t *ring_k, int64_t ring_cap,
                                                        int H, int Hkv, int64_t t0, int bs, int repr_topk, bf16_t *rep_out,
                                                        int64_t rep_sb, int64_t rep_su, int32_t *idx_out, CarveCopy cc) {
-    __shared__ float sc[kMaxUnit];
+    extern __shared__ float sc[];                                        // [bs], units beyond 256 rows only
+    constexpr int kChunks = D / 8;
     if ((int)blockIdx.x >= H) {
         const int64_t g = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * cc.x_extra + ((int)blockIdx.x - H);
         const int64_t e = g * 64 + threadIdx.x;                        // (ring, batch row, kv head, row, 16-byte chunk)
-        if (e >= (int64_t)2 * cc.B * cc.Hkv * cc.n * 16) return;
-        const int c = (int)(e & 15);
-        int64_t rest = e >> 4;
-        const int r = (int)(rest % cc.n);
-        rest /= cc.n;
-        const int hk = (int)(rest % cc.Hkv);
-        rest /= cc.Hkv;
-        const int bb = (int)(rest % cc.B);
-        const bool second = rest / cc.B != 0;
-        const bf16_t *src = (second ? cc.ring_b : cc.ring_a) + (((int64_t)bb * cc.Hkv + hk) * cc.ring_cap + (cc.t0 + r) % cc.ring_cap) * kD + c * 8;
+        if (e >= (int64_t)2 * cc.B * cc.Hkv * cc.n * kChunks) return;
+        const int c = (int)(e % kChunks);
+        uint32_t rest = (uint32_t)(e / kChunks);
+        const int r = (int)(rest % (uint32_t)cc.n);
+        rest /= (uint32_t)cc.n;
+        const int hk = (int)(rest % (uint32_t)cc.Hkv);
+        rest /= (uint32_t)cc.Hkv;
+        const int bb = (int)(rest % (uint32_t)cc.B);
+        const bool second = rest / (uint32_t)cc.B != 0;
+        const bf16_t *src = (second ? cc.ring_b : cc.ring_a) + (((int64_t)bb * cc.Hkv + hk) * cc.ring_cap + (cc.t0 + r) % cc.ring_cap) * D + c * 8;
         bf16_t *dst = (second ? cc.out_b : cc.out_a) + (int64_t)bb * cc.out_sb + (int64_t)(r / cc.unit_rows) * cc.out_su +
-                      (int64_t)hk * cc.out_sh + (int64_t)(r % cc.unit_rows) * kD + c * 8;
+                      (int64_t)hk * cc.out_sh + (int64_t)(r % cc.unit_rows) * D + c * 8;
         *(u32x4 *)dst = *(const u32x4 *)src;
         return;
     }
     const int h = blockIdx.x, u = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
     const int n_units = gridDim.y;
     const int g = h / (H / Hkv);
-    const int64_t first = t0 + (int64_t)u * bs;
+    const int64_t first = (t0 + (int64_t)u * bs) % ring_cap;
     const float *srow = ring_score + ((int64_t)b * H + h) * ring_cap;
-    for (int r = lane; r < bs; r += 64) sc[r] = srow[(first + r) % ring_cap];
-    __syncthreads();
-    const bf16_t *kbase = ring_k + ((int64_t)b * Hkv + g) * ring_cap * kD;
-    float a0 = 0.f, a1 = 0.f;
-    for (int it = 0; it < repr_topk; ++it) {
-        float best = -INFINITY;
-        int best_r = INT32_MAX;
-        for (int r = lane; r < bs; r += 64) {
-            float x = sc[r];
-            if (x > best || (x == best && r < best_r)) {     // NaN never wins
-                best = x;
-                best_r = r;
-            }
-        }
-        if (best_r == INT32_MAX && lane < bs) best_r = lane;   // all -inf / NaN: still pick a valid row
+    auto row_of = [&](int r) { return first + r < ring_cap ? first + r : first + r - ring_cap; };
+    const bf16_t *kbase = ring_k + ((int64_t)b * Hkv + g) * ring_cap * D;
+    int32_t *idx = idx_out ? idx_out + (((int64_t)b * n_units + u) * H + h) * repr_topk : nullptr;
+    constexpr int kRegs = 4;
+    const bool in_regs = bs <= 64 * kRegs;
+    // composite of a score: larger is better, equal scores by lower row; 0 only for rows that do not exist or are taken
+    auto composite = [&](float x, int r) { return ((uint64_t)(x == x ? order_key(x) : 1u) << 32) | (uint32_t)~r; };
+    uint64_t key[kRegs];
+    if (in_regs) {
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            float ob = __shfl_xor(best, o, 64);
-            int orr = __shfl_xor(best_r, o, 64);
-            if (ob > best || (ob == best && orr < best_r) || best_r == INT32_MAX) {
-                best = ob;
-                best_r = orr;
-            }
+        for (int i = 0; i < kRegs; ++i) {
+            const int r = lane + 64 * i;
+            key[i] = r < bs ? composite(srow[row_of(r)], r) : 0;
         }
-        if (lane == 0) {
-            sc[best_r] = -INFINITY;
-            if (idx_out) idx_out[(((int64_t)b * n_units + u) * H + h) * repr_topk + it] = best_r;
-        }
-        uint32_t w = *(const uint32_t *)(kbase + ((first + best_r) % ring_cap) * kD + lane * 2);
-        a0 += bf16_bits_to_f32(w & 0xffffu);
-        a1 += bf16_bits_to_f32(w >> 16);
+    } else {
+        for (int r = lane; r < bs; r += 64) sc[r] = srow[row_of(r)];
         __syncthreads();
     }
+    uint64_t last = ~0ull;                                               // LDS form: picks come in descending composite
+    auto pick = [&]() {
+        uint64_t best = 0;
+        if (in_regs) {
+#pragma unroll
+            for (int i = 0; i < kRegs; ++i) best = key[i] > best ? key[i] : best;
+        } else {
+            for (int r = lane; r < bs; r += 64) {
+                const uint64_t c = composite(sc[r], r);
+                best = c < last && c > best ? c : best;
+            }
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint64_t other = shfl_xor_u64(best, o);
+            best = other > best ? other : best;
+        }
+        last = best;
+#pragma unroll
+        for (int i = 0; i < kRegs; ++i) key[i] = in_regs && key[i] == best ? 0 : key[i];
+        return (int)~(uint32_t)best;
+    };
+    float a0 = 0.f, a1 = 0.f;
+    for (int it = 0; it < repr_topk; it += 4) {
+        int r[4];
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            r[i] = it + i < repr_topk ? pick() : r[0];
+            if (idx && lane == 0 && it + i < repr_topk) idx[it + i] = r[i];
+            w[i] = lane * 2 < D ? *(const uint32_t *)(kbase + row_of(r[i]) * D + lane * 2) : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (it + i < repr_topk) {
+                a0 += bf16_bits_to_f32(w[i] & 0xffffu);
+                a1 += bf16_bits_to_f32(w[i] >> 16);
+            }
+    }
     const float inv = 1.f / (float)repr_topk;
-    *(uint32_t *)(rep_out + (int64_t)b * rep_sb + (int64_t)u * rep_su + (int64_t)h * kD + lane * 2) =
-        pack_bf16x2(a0 * inv, a1 * inv);
+    if (lane * 2 < D)
+        *(uint32_t *)(rep_out + (int64_t)b * rep_sb + (int64_t)u * rep_su + (int64_t)h * D + lane * 2) = pack_bf16x2(a0 * inv, a1 * inv);
 }
 
 }  // namespace
@@ -915,11 +947,12 @@ __global__ __launch_bounds__(kRetrThreads) void select_rows_kernel(const float *
 // sit in LDS (QG x C floats), a wave keeps two rows in registers and walks the group's queries over them.  The sums
 // are unit_scores_rows_kernel's, term by term.
 constexpr int kQueryGroup = 8;
-template <int CPL>
-__global__ __launch_bounds__(512) void unit_scores_queries_kernel(const bf16_t *reps, int64_t rep_stride, int N, const float *qbars,
+template <int CPL, bool TAIL>
+__global__ __launch_bounds__(512) void unit_scores_queries_kernel(const bf16_t *reps, int64_t rep_stride, int N, int C_, const float *qbars,
                                                                    int64_t qbar_qs, int n_queries, float *scores, int64_t scores_qs) {
-    extern __shared__ float qs[];                               // [kQueryGroup][C]
-    constexpr int C = CPL * 512;
+    extern __shared__ float qs[];                               // [kQueryGroup][CP]
+    constexpr int CP = CPL * 512;
+    const int C = TAIL ? C_ : CP;
     const int lane = threadIdx.x & 63;
     // Workgroups go to the 8 XCDs round-robin by their id.  The workgroups that walk the same rows for different
     // groups of queries get ids 8 apart: they run on the same XCD at about the same time, and all but the first of
@@ -939,12 +972,12 @@ __global__ __launch_bounds__(512) void unit_scores_queries_kernel(const bf16_t *
             if (first + r * n_waves < N) {
                 const bf16_t *row = reps + (int64_t)(first + r * n_waves) * rep_stride + lane * 8;
 #pragma unroll
-                for (int j = 0; j < CPL; ++j) dst[r][j] = *(const u32x4 *)(row + j * 512);
+                for (int j = 0; j < CPL; ++j) dst[r][j] = !TAIL || j * 512 + lane * 8 < C ? *(const u32x4 *)(row + j * 512) : u32x4{0, 0, 0, 0};
             }
     };
     load_rows(w, n);
-    for (int e = threadIdx.x * 4; e < nq * C; e += 512 * 4)
-        *(f32x4 *)(qs + e) = *(const f32x4 *)(qbars + (int64_t)(q0 + e / C) * qbar_qs + e % C);
+    for (int e = threadIdx.x * 4; e < nq * CP; e += 512 * 4)
+        *(f32x4 *)(qs + e) = !TAIL || e % CP < C ? *(const f32x4 *)(qbars + (int64_t)(q0 + e / CP) * qbar_qs + e % CP) : f32x4{0.f, 0.f, 0.f, 0.f};
     __syncthreads();
     while (n < N) {
         const bool two = n + n_waves < N;
@@ -964,7 +997,7 @@ __global__ __launch_bounds__(512) void unit_scores_queries_kernel(const bf16_t *
 #pragma unroll
             for (int q = 0; q < kQueryGroup; ++q) {
                 if (q >= nq) break;
-                const float *qq = qs + q * C + j * 512 + lane * 8;
+                const float *qq = qs + q * CP + j * 512 + lane * 8;
                 const f32x4 q_lo = *(const f32x4 *)qq, q_hi = *(const f32x4 *)(qq + 4);
                 const float qv[8] = {q_lo[0], q_lo[1], q_lo[2], q_lo[3], q_hi[0], q_hi[1], q_hi[2], q_hi[3]};
 #pragma unroll
@@ -1002,20 +1035,28 @@ extern "C" int infllm_score_topk_queries(const void *d_reps, int64_t rep_stride,
     const int groups = (n_queries + kQueryGroup - 1) / kQueryGroup;
     int wgs = ((N + 15) / 16 + 7) / 8 * 8;                 // two rows per wave and trip; a multiple of the 8 XCDs
     if (wgs > 256) wgs = 256;                              // one workgroup per CU: the queries take most of its LDS
-    static bool lds_set = false;                           // dynamic LDS above 64 KiB must be enabled once per kernel
-    if (!lds_set) {
-        hipError_t e = hipFuncSetAttribute((const void *)unit_scores_queries_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           kQueryGroup * 4096 * (int)sizeof(float));
-        if (e != hipSuccess) return infllm_fail(-2, "score_topk_queries: %s", hipGetErrorString(e));
-        lds_set = true;
+    // rows of up to 9 * 512 elements: eight queries in LDS (147,456 bytes) and four rows of a wave in registers
+    if (C % 8 != 0 || C > 9 * 512) return 1;
+#define QUERIES_CASE(n, tail)                                                                                                                    \
+    {                                                                                                                                            \
+        constexpr size_t lds = (size_t)kQueryGroup * n * 512 * sizeof(float);                                                                    \
+        static std::atomic<bool> lds_set{false};           /* dynamic LDS above 64 KiB must be enabled once per kernel */                        \
+        if (lds > 65536 && !lds_set.load(std::memory_order_acquire)) {                                                                           \
+            hipError_t e = hipFuncSetAttribute((const void *)unit_scores_queries_kernel<n, tail>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+            if (e != hipSuccess) return infllm_fail(-2, "score_topk_queries: %s", hipGetErrorString(e));                                        \
+            lds_set.store(true, std::memory_order_release);                                                                                      \
+        }                                                                                                                                        \
+        hipLaunchKernelGGL((unit_scores_queries_kernel<n, tail>), dim3(wgs * groups), dim3(512), lds, (hipStream_t)stream, rows, rep_stride, N, C, \
+                           d_qbars, qbar_qs, n_queries, d_scores, scores_qs);                                                                    \
     }
-    switch (C % 512 == 0 ? C / 512 : 0) {
-#define QUERIES_CASE(n) case n: hipLaunchKernelGGL(unit_scores_queries_kernel<n>, dim3(wgs * groups), dim3(512), (size_t)kQueryGroup * n * 512 * sizeof(float), \
-                                                    (hipStream_t)stream, rows, rep_stride, N, d_qbars, qbar_qs, n_queries, d_scores, scores_qs); break
-        QUERIES_CASE(1); QUERIES_CASE(2); QUERIES_CASE(4); QUERIES_CASE(8);
+    if (C == 512) QUERIES_CASE(1, false)
+    else if (C == 1024) QUERIES_CASE(2, false)
+    else if (C == 2048) QUERIES_CASE(4, false)
+    else if (C == 4096) QUERIES_CASE(8, false)
+    else if (C < 1024) QUERIES_CASE(2, true)
+    else if (C <= 2560) QUERIES_CASE(5, true)
+    else QUERIES_CASE(9, true)
 #undef QUERIES_CASE
-    default: return 1;
-    }
     INFLLM_CHECK_LAUNCH("score_topk_queries");
     if (N > 32 * kRetrThreads || k > 64) return launch_topk(d_scores, N, k, d_idx, nullptr, nullptr, 0, n_queries, scores_qs, idx_qs, stream);
     if (N <= 16 * kRetrThreads)
@@ -1028,15 +1069,13 @@ extern "C" int infllm_score_topk_queries(const void *d_reps, int64_t rep_stride,
 
 // library-internal: unit scores of all N units and the k best of them in ONE launch (retrieve_fused_kernel), the ids
 // leaving as infllm_topk_publish_pair leaves them.  Returns 1, with nothing launched, where that kernel does not apply
-// (row lengths other than 512 * {1, 2, 4, 8}, more than 16384 units, k > 64): the caller then launches the two steps.
+// (rows of more than 4608 elements or not of whole 16-byte chunks, more than 16384 units, k > 64): the caller then launches the two steps.
 int infllm_retrieve_fused(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar, int32_t k, float *d_scores,
                           int32_t *d_idx, int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, void *stream) {
     INFLLM_REQUIRE(d_reps && d_qbar && d_scores && d_idx, "retrieve: null pointer");
     INFLLM_REQUIRE(N > 0 && k > 0 && k <= N, "retrieve: k=%d with N=%d", k, N);
     INFLLM_REQUIRE(rep_stride >= C && rep_stride % 8 == 0, "retrieve: row stride %lld", (long long)rep_stride);
-    if (N > 16384 || k > 64 || C % 512 != 0) return 1;
-    const int cpl = C / 512;
-    if (cpl != 1 && cpl != 2 && cpl != 4 && cpl != 8) return 1;
+    if (N > 16384 || k > 64 || C % 8 != 0 || C > 9 * 512) return 1;
     static std::atomic<unsigned int> next_slot{0};
     const int slot = (int)(next_slot.fetch_add(1, std::memory_order_relaxed) % kTicketSlots);
     constexpr int waves_per_wg = kRetrThreads / 64;
@@ -1044,19 +1083,21 @@ int infllm_retrieve_fused(const void *d_reps, int64_t rep_stride, int32_t N, int
     const int per_wg = waves_per_wg * (deep ? 2 : 1);
     int wgs = (N + per_wg - 1) / per_wg;
     if (wgs > 256) wgs = 256;
-    const size_t lds = (size_t)C * sizeof(float);
     const bf16_t *reps = (const bf16_t *)d_reps;
     const hipStream_t st = (hipStream_t)stream;
-#define FUSED_CASE(c)                                                                                                              \
-    case c: {                                                                                                                      \
-        auto kern = deep ? retrieve_fused_kernel<c, 2> : retrieve_fused_kernel<c, 1>;                                              \
-        hipLaunchKernelGGL(kern, dim3(wgs), dim3(kRetrThreads), lds, st, reps, rep_stride, N, d_qbar, d_scores, k, d_idx, d_idx2,   \
-                           d_flag, flag_value, slot);                                                                              \
-        break;                                                                                                                     \
+#define FUSED_CASE(c, tail)                                                                                                          \
+    {                                                                                                                                \
+        auto kern = deep ? retrieve_fused_kernel<c, 2, tail> : retrieve_fused_kernel<c, 1, tail>;                                    \
+        hipLaunchKernelGGL(kern, dim3(wgs), dim3(kRetrThreads), (size_t)c * 512 * sizeof(float), st, reps, rep_stride, N, C, d_qbar,  \
+                           d_scores, k, d_idx, d_idx2, d_flag, flag_value, slot);                                                    \
     }
-    switch (cpl) {
-        FUSED_CASE(1) FUSED_CASE(2) FUSED_CASE(4) FUSED_CASE(8)
-    }
+    if (C == 512) FUSED_CASE(1, false)
+    else if (C == 1024) FUSED_CASE(2, false)
+    else if (C == 2048) FUSED_CASE(4, false)
+    else if (C == 4096) FUSED_CASE(8, false)
+    else if (C < 1024) FUSED_CASE(2, true)
+    else if (C <= 2560) FUSED_CASE(5, true)
+    else FUSED_CASE(9, true)
 #undef FUSED_CASE
     INFLLM_CHECK_LAUNCH("retrieve");
     return 0;
@@ -1080,8 +1121,9 @@ extern "C" int infllm_score_topk(const void *d_reps, int64_t rep_stride, int32_t
 int infllm_repr_keys_carve(const float *d_ring_score, const void *d_ring_k_raw, int64_t ring_cap, int32_t B, int32_t H, int32_t Hkv,
                            int64_t t0, int32_t bs, int32_t n_units, int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su,
                            int32_t *d_idx_out, const void *d_ring_v, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
-                           int64_t out_sh, void *stream) {
+                           int64_t out_sh, void *stream, int32_t dim) {
     INFLLM_REQUIRE(d_ring_score && d_ring_k_raw && d_rep_out, "repr_keys: null pointer");
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "repr_keys: head_dim %d", dim);
     INFLLM_REQUIRE(B > 0 && H > 0 && Hkv > 0 && H % Hkv == 0, "repr_keys: bad geometry B=%d H=%d Hkv=%d", B, H, Hkv);
     INFLLM_REQUIRE(bs > 0 && bs <= kMaxUnit, "repr_keys: unit size %d not in 1..%d", bs, kMaxUnit);
     INFLLM_REQUIRE(repr_topk > 0 && repr_topk <= bs, "repr_keys: repr_topk %d not in 1..%d", repr_topk, bs);
@@ -1096,10 +1138,12 @@ int infllm_repr_keys_carve(const float *d_ring_score, const void *d_ring_k_raw, 
         cc.out_a = (bf16_t *)d_out_k; cc.out_b = (bf16_t *)d_out_v;
         cc.ring_cap = ring_cap; cc.t0 = t0; cc.out_sb = out_sb; cc.out_su = out_su; cc.out_sh = out_sh;
         cc.Hkv = Hkv; cc.B = B; cc.n = n_units * bs; cc.unit_rows = bs;
-        const int64_t waves = ((int64_t)2 * B * Hkv * cc.n * 16 + 63) / 64, per_x = (int64_t)n_units * B;
+        INFLLM_REQUIRE((int64_t)2 * B * Hkv * cc.n * (dim / 8) < (1ll << 32), "repr_keys: copy too large");
+        const int64_t waves = ((int64_t)2 * B * Hkv * cc.n * (dim / 8) + 63) / 64, per_x = (int64_t)n_units * B;
         cc.x_extra = (int32_t)((waves + per_x - 1) / per_x);
     }
-    hipLaunchKernelGGL(repr_keys_kernel, dim3(H + cc.x_extra, n_units, B), dim3(64), 0, (hipStream_t)stream, d_ring_score,
+    const size_t lds = bs > 256 ? (size_t)bs * sizeof(float) : 0;
+    hipLaunchKernelGGL((dim == 64 ? repr_keys_kernel<64> : repr_keys_kernel<128>), dim3(H + cc.x_extra, n_units, B), dim3(64), lds, (hipStream_t)stream, d_ring_score,
                        (const bf16_t *)d_ring_k_raw, ring_cap, H, Hkv, t0, bs, repr_topk, (bf16_t *)d_rep_out, rep_sb,
                        rep_su, d_idx_out, cc);
     INFLLM_CHECK_LAUNCH("repr_keys");
@@ -1110,5 +1154,5 @@ extern "C" int infllm_repr_keys(const float *d_ring_score, const void *d_ring_k_
                                 int32_t Hkv, int64_t t0, int32_t bs, int32_t n_units, int32_t repr_topk, void *d_rep_out,
                                 int64_t rep_sb, int64_t rep_su, int32_t *d_idx_out, void *stream) {
     return infllm_repr_keys_carve(d_ring_score, d_ring_k_raw, ring_cap, B, H, Hkv, t0, bs, n_units, repr_topk, d_rep_out, rep_sb, rep_su,
-                                  d_idx_out, nullptr, nullptr, nullptr, 0, 0, 0, stream);
+                                  d_idx_out, nullptr, nullptr, nullptr, 0, 0, 0, stream, kD);
 }

@@ -11,11 +11,13 @@
 // (A operand, shared by the 4 waves, double buffered).  Exactly one lane writes each
 // (head, key) cell, so results are deterministic.
 #include "common.h"
+#include <atomic>
 #include <type_traits>
 
 namespace {
 
-constexpr int kQPad = kD + 8;              // LDS row of Q (bf16 elements): 272 bytes rotates the banks
+template <int D>
+constexpr int kQPad = D + 8;               // LDS row of Q (bf16 elements): 272 (144) bytes rotates the banks
 
 // KS = 32-key halves per wave: 2 for long key ranges; 1 halves the work of a wave per query stage, which is what
 // bounds the short launches that sit on the critical path between two blocks.  QS = queries per LDS stage: a short
@@ -35,7 +37,7 @@ struct ScoreMerge {
 };
 struct NoScoreMerge {};
 
-template <int KS, int QS, bool MERGE = false>
+template <int D, int KS, int QS, bool MERGE = false>
 __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a, std::conditional_t<MERGE, ScoreMerge, NoScoreMerge> sm) {
     constexpr int kWaveKeys = 32 * KS, kKeysPerWg = 4 * kWaveKeys, kQStage = QS;
     int n_tiles = gridDim.y;
@@ -43,14 +45,14 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
     if constexpr (MERGE) {
         n_tiles = sm.score_tiles;
         if ((int)blockIdx.y >= n_tiles) {
-            merge_piece(sm.job, ((int64_t)((int)blockIdx.y - n_tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x);
+            merge_piece<D>(sm.job, ((int64_t)((int)blockIdx.y - n_tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x);
             return;
         }
         lps = sm.job.ps;
     }
     extern __shared__ __attribute__((aligned(16))) char score_lds[];
-    bf16_t(*Qs)[kQStage][kQPad] = (bf16_t(*)[kQStage][kQPad])score_lds;                               // [2][QS][kQPad]
-    float(*Ls)[kQStage] = (float(*)[kQStage])(score_lds + 2 * kQStage * kQPad * sizeof(bf16_t));      // [2][QS]
+    bf16_t(*Qs)[kQStage][kQPad<D>] = (bf16_t(*)[kQStage][kQPad<D>])score_lds;                               // [2][QS][kQPad]
+    float(*Ls)[kQStage] = (float(*)[kQStage])(score_lds + 2 * kQStage * kQPad<D> * sizeof(bf16_t));      // [2][QS]
     [[maybe_unused]] float *Lall = (float *)Ls;                                                        // MERGE: [Lq rounded up to QS]
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -72,7 +74,7 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
     const float scale = a.softmax_scale * 1.4426950408889634f;
 
     // ---- this wave's 64 keys as the B operand (lane = key column)
-    bf16x8 kreg[KS][kD / 16];
+    bf16x8 kreg[KS][D / 16];
     bool jok[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -80,7 +82,7 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
         jok[ks] = j >= a.j_lo && j < a.j_hi;
         const bf16_t *krow = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + (j % a.cap) * a.k_sl;
 #pragma unroll
-        for (int kk = 0; kk < kD / 16; ++kk) {
+        for (int kk = 0; kk < D / 16; ++kk) {
             u32x4 raw = jok[ks] ? *(const u32x4 *)(krow + kk * 16 + grp * 8) : u32x4{0, 0, 0, 0};
             kreg[ks][kk] = __builtin_bit_cast(bf16x8, raw);
         }
@@ -110,14 +112,15 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
 
     const bf16_t *qbase = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh;
     const float *lse = a.d_lse + ((int64_t)b * a.H + h) * a.Lq;
-    const int ld_chunk = tid & 15, ld_row = tid >> 4;
-    u32x4 qbuf[kQStage / 16];
+    constexpr int kChunks = D / 8, kLdRows = 256 / kChunks;        // chunks of a row, rows of Q a pass of the workgroup loads
+    const int ld_chunk = tid % kChunks, ld_row = tid / kChunks;
+    u32x4 qbuf[kQStage / kLdRows];
     float lbuf = 0.f;
     auto load_stage = [&](int s) {
         const int i0 = s * kQStage;
 #pragma unroll
-        for (int i = 0; i < kQStage / 16; ++i) {
-            const int qi = i0 + ld_row + 16 * i;
+        for (int i = 0; i < kQStage / kLdRows; ++i) {
+            const int qi = i0 + ld_row + kLdRows * i;
             qbuf[i] = qi < a.Lq ? *(const u32x4 *)(qbase + (int64_t)qi * a.q_sl + ld_chunk * 8) : u32x4{0, 0, 0, 0};
         }
         if (!MERGE && tid < kQStage) {
@@ -147,7 +150,7 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
     };
     auto store_stage = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < kQStage / 16; ++i) *(u32x4 *)&Qs[buf][ld_row + 16 * i][ld_chunk * 8] = qbuf[i];
+        for (int i = 0; i < kQStage / kLdRows; ++i) *(u32x4 *)&Qs[buf][ld_row + kLdRows * i][ld_chunk * 8] = qbuf[i];
         if (!MERGE && tid < kQStage) Ls[buf][tid] = lbuf;
     };
 
@@ -191,10 +194,10 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
             f32x16 sacc[2][KS];
             f32x4 l4[2][4];
             auto issue = [&](int qs, int pb) {
-                bf16x8 qa[kD / 16];                              // A operand: lane = query row
+                bf16x8 qa[D / 16];                              // A operand: lane = query row
                 const bf16_t *qrow = &Qs[cur][qs * 32 + col][grp * 8];
 #pragma unroll
-                for (int kk = 0; kk < kD / 16; ++kk) qa[kk] = *(const bf16x8 *)(qrow + kk * 16);
+                for (int kk = 0; kk < D / 16; ++kk) qa[kk] = *(const bf16x8 *)(qrow + kk * 16);
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) l4[pb][q4] = *(const f32x4 *)(MERGE ? &Lall[i0 + qs * 32 + 8 * q4 + 4 * grp] : &Ls[cur][qs * 32 + 8 * q4 + 4 * grp]);
 #pragma unroll
@@ -202,7 +205,7 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
 #pragma unroll
                     for (int r = 0; r < 16; ++r) sacc[pb][ks][r] = 0.f;
 #pragma unroll
-                for (int kk = 0; kk < kD / 16; ++kk)
+                for (int kk = 0; kk < D / 16; ++kk)
 #pragma unroll
                     for (int ks = 0; ks < KS; ++ks)
                         sacc[pb][ks] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[kk], kreg[ks][kk], sacc[pb][ks], 0, 0, 0);
@@ -223,10 +226,10 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
                 if (qs + 1 < kSub) {
                     // one MFMA, then its share of the exponentials (16 * KS of each per sub-tile)
 #pragma unroll
-                    for (int i = 0; i < 8 * KS; ++i) {
+                    for (int i = 0; i < D / 16 * KS; ++i) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // MFMA
-                        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);      // VALU
-                        __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);      // transcendental
+                        __builtin_amdgcn_sched_group_barrier(0x002, 512 / D, 0);      // VALU
+                        __builtin_amdgcn_sched_group_barrier(0x400, 256 / D, 0);      // transcendental
                     }
                 }
             }
@@ -236,10 +239,10 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
             for (int qs = 0; qs < kQStage / 32; ++qs) {
                 const int64_t iq = i0 + qs * 32;
                 if (iq >= w_hi || iq + 32 <= w_lo) continue;
-                bf16x8 qa[kD / 16];                              // A operand: lane = query row
+                bf16x8 qa[D / 16];                              // A operand: lane = query row
                 const bf16_t *qrow = &Qs[cur][qs * 32 + col][grp * 8];
 #pragma unroll
-                for (int kk = 0; kk < kD / 16; ++kk) qa[kk] = *(const bf16x8 *)(qrow + kk * 16);
+                for (int kk = 0; kk < D / 16; ++kk) qa[kk] = *(const bf16x8 *)(qrow + kk * 16);
                 f32x4 l4[4];                                     // lse of rows 8*(r>>2) + 4*grp + (r&3)
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) l4[q4] = *(const f32x4 *)(MERGE ? &Lall[i0 + qs * 32 + 8 * q4 + 4 * grp] : &Ls[cur][qs * 32 + 8 * q4 + 4 * grp]);
@@ -250,7 +253,7 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
 #pragma unroll
                     for (int r = 0; r < 16; ++r) sacc2[ks][r] = 0.f;
 #pragma unroll
-                for (int kk = 0; kk < kD / 16; ++kk)
+                for (int kk = 0; kk < D / 16; ++kk)
 #pragma unroll
                     for (int ks = 0; ks < KS; ++ks)
                         sacc2[ks] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[kk], kreg[ks][kk], sacc2[ks], 0, 0, 0);
@@ -323,52 +326,52 @@ int check_score_args(const infllm_score_args *a) {
     return 0;
 }
 
-size_t score_lds_bytes(int qs) { return (size_t)(2 * qs * kQPad * sizeof(bf16_t) + 2 * qs * sizeof(float)); }
+template <int D>
+size_t score_lds_bytes(int qs) { return (size_t)(2 * qs * kQPad<D> * sizeof(bf16_t) + 2 * qs * sizeof(float)); }
 constexpr int kMergedMaxLq = 2048;                     // MERGE: 4 bytes of LDS per query of the launch
-size_t score_lds_bytes_merged(int qs, int lq) { return (size_t)(2 * qs * kQPad * sizeof(bf16_t) + (size_t)((lq + qs - 1) / qs * qs) * sizeof(float)); }
+template <int D>
+size_t score_lds_bytes_merged(int qs, int lq) { return (size_t)(2 * qs * kQPad<D> * sizeof(bf16_t) + (size_t)((lq + qs - 1) / qs * qs) * sizeof(float)); }
 
+template <int D>
 int score_lds_setup() {
-    static bool lds_set = false;                       // dynamic LDS above 64 KiB must be enabled once per kernel
-    if (!lds_set) {
-        hipError_t e = hipFuncSetAttribute((const void *)local_score_kernel<1, 128>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)score_lds_bytes(128));
+    static std::atomic<bool> lds_set{false};           // dynamic LDS above 64 KiB must be enabled once per kernel
+    if (!lds_set.load(std::memory_order_acquire)) {
+        hipError_t e = hipFuncSetAttribute((const void *)local_score_kernel<D, 1, 128>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)score_lds_bytes<D>(128));
         if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)local_score_kernel<2, 128>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)score_lds_bytes(128));
+            e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)score_lds_bytes<D>(128));
         if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)local_score_kernel<2, 128, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)score_lds_bytes_merged(128, kMergedMaxLq));
+            e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)score_lds_bytes_merged<D>(128, kMergedMaxLq));
         if (e != hipSuccess) return infllm_fail(-2, "local_score: %s", hipGetErrorString(e));
-        lds_set = true;
+        lds_set.store(true, std::memory_order_release);
     }
     return 0;
 }
 
-}  // namespace
-
-extern "C" int infllm_local_score(const infllm_score_args *a, void *stream) {
+template <int D>
+int score_launch(const infllm_score_args *a, void *stream) {
     int rc = check_score_args(a);
     if (rc) return rc;
     if (a->j_hi <= a->j_lo) return 0;
-    rc = score_lds_setup();
+    rc = score_lds_setup<D>();
     if (rc) return rc;
     if (a->j_hi - a->j_lo > 1024) {
         const int64_t tiles = (a->j_hi - 1) / 64 - a->j_lo / 64 + 1;
-        hipLaunchKernelGGL((local_score_kernel<2, 128>), dim3(a->B * a->H, (unsigned)((tiles + 3) / 4)), dim3(256), score_lds_bytes(128),
+        hipLaunchKernelGGL((local_score_kernel<D, 2, 128>), dim3(a->B * a->H, (unsigned)((tiles + 3) / 4)), dim3(256), score_lds_bytes<D>(128),
                            (hipStream_t)stream, *a, NoScoreMerge{});
     } else {
         const int64_t tiles = (a->j_hi - 1) / 32 - a->j_lo / 32 + 1;
-        hipLaunchKernelGGL((local_score_kernel<1, 128>), dim3(a->B * a->H, (unsigned)((tiles + 3) / 4)), dim3(256), score_lds_bytes(128),
+        hipLaunchKernelGGL((local_score_kernel<D, 1, 128>), dim3(a->B * a->H, (unsigned)((tiles + 3) / 4)), dim3(256), score_lds_bytes<D>(128),
                            (hipStream_t)stream, *a, NoScoreMerge{});
     }
     INFLLM_CHECK_LAUNCH("local_score");
     return 0;
 }
 
-// library-internal: the local score of a block and the merge of its partial attention outputs in one launch.  The
-// scores are taken against the joint log-sum-exp of the job's partials (a->d_lse and a->n_parts are set from the job);
-// returns 1, with nothing launched, where the one-launch form does not apply (short key ranges).
-int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream) {
+template <int D>
+int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *stream) {
     INFLLM_REQUIRE(a && job, "local_score_merged: null argument");
     INFLLM_REQUIRE(job->out && job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1 && job->P <= 8,
                    "local_score_merged: the merge does not belong to these queries");
@@ -378,15 +381,33 @@ int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, v
     int rc = check_score_args(&sc);
     if (rc) return rc;
     if (sc.j_hi - sc.j_lo <= 1024 || sc.Lq > kMergedMaxLq) return 1;
-    rc = score_lds_setup();
+    rc = score_lds_setup<D>();
     if (rc) return rc;
     const int64_t tiles = (sc.j_hi - 1) / 64 - sc.j_lo / 64 + 1;
     const int score_tiles = (int)((tiles + 3) / 4);
-    const int64_t merge_wgs = ((int64_t)job->B * job->H * job->Lq * 16 + 255) / 256;
+    const int64_t merge_wgs = ((int64_t)job->B * job->H * job->Lq * (D / 8) + 255) / 256;
     const int gx = sc.B * sc.H;
     const int merge_slots = (int)((merge_wgs + gx - 1) / gx);
-    hipLaunchKernelGGL((local_score_kernel<2, 128, true>), dim3(gx, (unsigned)(score_tiles + merge_slots)), dim3(256),
-                       score_lds_bytes_merged(128, sc.Lq), (hipStream_t)stream, sc, ScoreMerge{*job, score_tiles});
+    hipLaunchKernelGGL((local_score_kernel<D, 2, 128, true>), dim3(gx, (unsigned)(score_tiles + merge_slots)), dim3(256),
+                       score_lds_bytes_merged<D>(128, sc.Lq), (hipStream_t)stream, sc, ScoreMerge{*job, score_tiles});
     INFLLM_CHECK_LAUNCH("local_score_merged");
     return 0;
+}
+
+}  // namespace
+
+extern "C" int infllm_local_score(const infllm_score_args *a, void *stream) { return score_launch<kD>(a, stream); }
+
+// library-internal: the same for heads of 128 or 64
+int infllm_local_score_dim(const infllm_score_args *a, int32_t dim, void *stream) {
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "local_score: head_dim %d", dim);
+    return dim == 128 ? score_launch<128>(a, stream) : score_launch<64>(a, stream);
+}
+
+// library-internal: the local score of a block and the merge of its partial attention outputs in one launch.  The
+// scores are taken against the joint log-sum-exp of the job's partials (a->d_lse and a->n_parts are set from the job);
+// returns 1, with nothing launched, where the one-launch form does not apply (short key ranges).
+int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream, int32_t dim) {
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "local_score: head_dim %d", dim);
+    return dim == 128 ? score_launch_merged<128>(a, job, stream) : score_launch_merged<64>(a, job, stream);
 }

@@ -209,8 +209,8 @@ int infllm_copy_units(const void *const *d_src, void *const *d_dst, int32_t n, i
 int infllm_merge_job(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2, const float *d_lse_part2,
                      int32_t P2, int32_t B, int32_t H, int32_t Lq, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse,
                      MergeJob *job, int32_t dim = kD);
-int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream);
-int infllm_attn_stage_blocked(const infllm_attn_args *a, int32_t exc, int64_t block_rows, void *stream);
+int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream, int32_t dim = kD);
+int infllm_attn_stage_blocked(const infllm_attn_args *a, int32_t exc, int64_t block_rows, void *stream, int32_t dim = kD);
 int infllm_attn_merge2(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2, const float *d_lse_part2,
                        int32_t P2, int32_t B, int32_t H, int32_t Lq, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse,
                        void *stream, int32_t dim = kD);
@@ -222,12 +222,9 @@ int infllm_score_new_rank(const void *d_reps, int64_t rep_stride, int32_t C, con
 int infllm_repr_keys_carve(const float *d_ring_score, const void *d_ring_k_raw, int64_t ring_cap, int32_t B, int32_t H, int32_t Hkv,
                            int64_t t0, int32_t bs, int32_t n_units, int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su,
                            int32_t *d_idx_out, const void *d_ring_v, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
-                           int64_t out_sh, void *stream);
+                           int64_t out_sh, void *stream, int32_t dim = kD);
 int infllm_topk_publish_pair(const float *d_scores, int32_t N, int32_t k, int32_t *d_idx, int32_t *d_idx2, int32_t *d_flag,
                              int32_t flag_value, void *stream);
-int infllm_gather_rows_pair(const void *d_ring_a, void *d_out_a, const void *d_ring_b, void *d_out_b, int64_t ring_cap, int32_t B,
-                            int32_t Hkv, int64_t t0, int32_t n, int32_t unit_rows, int64_t out_sb, int64_t out_su, int64_t out_sh,
-                            void *stream);
 int infllm_topk_merge_publish(const float *d_scores, const int32_t *d_cand, int32_t n_cand, int32_t first_new, int32_t n_new, int32_t k,
                               int32_t *d_idx, int32_t *d_flag, int32_t flag_value, void *stream);
 namespace {
@@ -249,6 +246,11 @@ int splits_for(const infllm_layer_desc &d, int n_queries, int n_tiles) {
     if (s > cap) s = cap;
     return s < 1 ? 1 : s;
 }
+
+}  // namespace
+// library-internal: the same rule for the path with resident units (resident.hip), whose results are to be these bit for bit
+int infllm_key_splits(const infllm_layer_desc *d, int32_t n_queries, int32_t n_tiles) { return splits_for(*d, n_queries, n_tiles); }
+namespace {
 
 // ---- page table built on the device from the slot list (no host staging, no copy in the chain)
 constexpr int kPageJobSlots = 64;

@@ -292,11 +292,11 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         d.B = a->B; d.H = a->H; d.Hkv = a->Hkv;
         d.scale = scale;
         const int64_t near = causal ? rows_base : std::min<int64_t>(rows_base, a->n_local);       // the last rows
-        d.seg[0] = DecodeSeg{bk + (rows_base - near) * D, bv + (rows_base - near) * D, bk_sb, bk_sh, bv_sb, bv_sh, (int32_t)near, 0, 0, nullptr};
+        d.seg[0] = DecodeSeg{bk + (rows_base - near) * D, bv + (rows_base - near) * D, bk_sb, bk_sh, bv_sb, bv_sh, (int32_t)near, 0, 0, nullptr, -1};
         d.n_seg = 1;
         // sink j is seen from a distance of at least n_local: j <= position - n_local
         const int64_t far = std::min<int64_t>(n_sink, len_k - a->n_local);
-        if (far > 0) d.seg[d.n_seg++] = DecodeSeg{sk, bv, sk_sb, sk_sh, bv_sb, bv_sh, (int32_t)far, 1, 0, nullptr};
+        if (far > 0) d.seg[d.n_seg++] = DecodeSeg{sk, bv, sk_sb, sk_sh, bv_sb, bv_sh, (int32_t)far, 1, 0, nullptr, -1};
         const int64_t blocks = (near + kDecodeBlock - 1) / kDecodeBlock + (far > 0 ? (far + kDecodeBlock - 1) / kDecodeBlock : 0);
         d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, blocks, max_parts);
         d.o_part = (uint16_t *)((char *)a->d_work + q_bytes);

@@ -45,10 +45,10 @@ def _need(cond, msg):
         raise ValueError(msg)
 
 
-def _bf16_4d(t, name):
+def _bf16_4d(t, name, dims=(HEAD_DIM,)):
     _need(t.is_cuda, f"{name} must be a GPU tensor")
     _need(t.dtype == torch.bfloat16, f"{name} must be bfloat16 (the HIP path computes in bf16), got {t.dtype}")
-    _need(t.dim() == 4 and t.shape[-1] == HEAD_DIM, f"{name} must be [B, heads, len, {HEAD_DIM}], got {tuple(t.shape)}")
+    _need(t.dim() == 4 and t.shape[-1] in dims, f"{name} must be [B, heads, len, {dims[-1]}], got {tuple(t.shape)}")
     if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:-1]):
         t = t.contiguous()
     return t
@@ -57,24 +57,24 @@ def _bf16_4d(t, name):
 def ingest(q, k, v, pos0, glb_pos, inv_freq, distance_scale, ring_k_raw, ring_k_rot, ring_v, ring_score, q_loc, q_glb,
            qpart=None):
     """RoPE + staging of the new tokens; see infllm_ingest."""
-    q, k, v = _bf16_4d(q, "q"), _bf16_4d(k, "k"), _bf16_4d(v, "v")
-    B, H, n, _ = q.shape
+    q, k, v = (_bf16_4d(t, name, (64, HEAD_DIM)) for t, name in ((q, "q"), (k, "k"), (v, "v")))
+    B, H, n, D = q.shape
     Hkv = k.shape[1]
-    _need(k.shape == v.shape == (B, Hkv, n, HEAD_DIM), "k/v shape mismatch")
+    _need(k.shape == v.shape == (B, Hkv, n, D), "k/v shape mismatch")
     cap = ring_k_raw.shape[2]
     for r in (ring_k_raw, ring_k_rot, ring_v):
-        _need(r.is_contiguous() and r.shape == (B, Hkv, cap, HEAD_DIM) and r.dtype == torch.bfloat16, "bad ring")
+        _need(r.is_contiguous() and r.shape == (B, Hkv, cap, D) and r.dtype == torch.bfloat16, "bad ring")
     _need(ring_score.is_contiguous() and ring_score.shape == (B, H, cap) and ring_score.dtype == torch.float32, "bad score ring")
     for o in (q_loc, q_glb):
-        _need(o.is_contiguous() and o.dtype == torch.bfloat16 and o.numel() >= B * H * n * HEAD_DIM, "bad q workspace")
-    _need(inv_freq.dtype == torch.float32 and inv_freq.numel() == HEAD_DIM // 2 and inv_freq.is_cuda, "bad inv_freq")
+        _need(o.is_contiguous() and o.dtype == torch.bfloat16 and o.numel() >= B * H * n * D, "bad q workspace")
+    _need(inv_freq.dtype == torch.float32 and inv_freq.numel() == D // 2 and inv_freq.is_cuda, "bad inv_freq")
     a = IngestArgs(q.data_ptr(), k.data_ptr(), v.data_ptr(),
                    q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
                    v.stride(0), v.stride(1), v.stride(2), B, H, Hkv, n, pos0, glb_pos,
                    inv_freq.data_ptr(), float(distance_scale),
                    ring_k_raw.data_ptr(), ring_k_rot.data_ptr(), ring_v.data_ptr(), ring_score.data_ptr(), cap,
                    q_loc.data_ptr(), q_glb.data_ptr(), qpart.data_ptr() if qpart is not None else None)
-    check(_lib.load().infllm_ingest(a, _stream()), "infllm_ingest")
+    check(_lib.load().infllm_ingest_dim(a, D, None, _stream()), "infllm_ingest")
 
 
 def reduce_partials(parts, scale, out):
