@@ -62,6 +62,15 @@ __device__ __forceinline__ float wave_xor32(float x) {
     return __shfl_xor(x, 32, 64);
 }
 
+__device__ __forceinline__ uint32_t order_key(float f) {
+    uint32_t u = __float_as_uint(f);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);       // larger float <=> larger key
+}
+__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int o) {
+    const uint32_t lo = __shfl_xor((uint32_t)v, o, 64), hi = __shfl_xor((uint32_t)(v >> 32), o, 64);
+    return ((uint64_t)hi << 32) | lo;
+}
+
 // ---- the merge of partial attention outputs, shared by the merge kernels (attn.hip) and by the local-score launch
 //      that carries the merge of its block along (score.hip)
 // The partials of a merge may lie in two places: the first n_first of them behind the pointers the kernel is given,

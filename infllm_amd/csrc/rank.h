@@ -1,0 +1,165 @@
+// A selection and what becomes of it on the device, for units resident in HBM (resident.hip; the local-score launch of
+// score.hip carries it along).
+#pragma once
+#include "common.h"
+
+constexpr int kRankEntries = 320;          // the k <= 64 best of the call's start + 256 units carved since
+constexpr int kRankNew = 64;               // units carved by one block
+
+// The page table of a block: selected units, init tokens, overflow remainder of the ring (the order of the host-built
+// tables of stream.hip).
+struct PageList {
+    infllm_page *out;                      // [B, n_pages]
+    int32_t n_unit_pages, n_init_pages, n_pages, tiles_per_unit;
+    int32_t Hkv, bs, init_len, dim;
+    int64_t cursor, overflow_end, ring_cap, init_cap;
+    const bf16_t *init_kv, *ring_k, *ring_v;
+    const uint64_t *chunk;                 // device: chunks of units, [per_chunk, B, 2, Hkv, bs, dim] each
+    int32_t per_chunk, B;
+};
+
+__device__ __forceinline__ void write_page(const PageList &j, int u, int p, const int32_t *ids) {
+    const int64_t unit_elems = (int64_t)j.Hkv * j.bs * j.dim;
+    infllm_page pg;
+    pg.reserved = 0;
+    if (p < j.n_unit_pages) {
+        const int s = p / j.tiles_per_unit, t0 = (p - s * j.tiles_per_unit) * kTile;
+        const int unit = ids[s], ch = unit / j.per_chunk;
+        const bf16_t *kb = (const bf16_t *)(uintptr_t)j.chunk[ch] + (((int64_t)(unit - ch * j.per_chunk) * j.B + u) * 2) * unit_elems + (int64_t)t0 * j.dim;
+        pg.k = kb;
+        pg.v = kb + unit_elems;
+        pg.head_stride = (int64_t)j.bs * j.dim;
+        pg.n_valid = min(j.bs - t0, kTile);
+    } else if (p < j.n_unit_pages + j.n_init_pages) {
+        const int t0 = (p - j.n_unit_pages) * kTile;
+        const bf16_t *ik = j.init_kv + (int64_t)u * 2 * j.Hkv * j.init_cap * j.dim + (int64_t)t0 * j.dim;
+        pg.k = ik;
+        pg.v = ik + (int64_t)j.Hkv * j.init_cap * j.dim;
+        pg.head_stride = j.init_cap * j.dim;
+        pg.n_valid = min(j.init_len - t0, kTile);
+    } else {
+        const int want = p - j.n_unit_pages - j.n_init_pages;
+        int64_t pos = j.cursor, len = 0;
+        for (int i = 0; i <= want; ++i) {          // runs of <= 64 rows that do not cross the end of the ring
+            pos += len;
+            len = min(min(j.overflow_end - pos, (int64_t)kTile), j.ring_cap - pos % j.ring_cap);
+        }
+        const int64_t row = pos % j.ring_cap;
+        pg.k = j.ring_k + ((int64_t)u * j.Hkv * j.ring_cap + row) * j.dim;
+        pg.v = j.ring_v + ((int64_t)u * j.Hkv * j.ring_cap + row) * j.dim;
+        pg.head_stride = j.ring_cap * j.dim;
+        pg.n_valid = (int)len;
+    }
+    j.out[(int64_t)u * j.n_pages + p] = pg;
+}
+
+// After a block has carved n_new units: workgroup x scores them under the mean query of the call's block j0 + x; the one
+// of block j_sel ranks that block's list of the call's start against all units carved since, and turns the selection into
+// the block's page table.
+struct RankJob {
+    const bf16_t *reps;
+    int64_t rep_sb, rep_su;
+    const float *qbars;                    // [blocks][B][C]
+    float *scores;                         // [blocks][B][cols]
+    int64_t cols;
+    const int32_t *base;                   // [blocks][B][k], n_list entries of a row are filled
+    int32_t B, C, k, n_list, n_base, first_new, n_new, j0, j_sel;
+    int32_t *log;                          // pinned: [B][k] ids, then the sequence number
+    int32_t seq;
+    PageList pages;
+};
+
+struct RankLds {
+    float fresh[kRankNew];
+    uint32_t e_key[kRankEntries];
+    int32_t e_id[kRankEntries], sel[64];
+};
+
+// workgroup x of 256 threads (the sums are unit_scores_rows_kernel's, term by term: a unit's score does not depend on which
+// kernel computed it)
+template <int CPL>
+__device__ __forceinline__ void rank_block(const RankJob &jb, int x, RankLds &lds) {
+    float *fresh = lds.fresh;
+    uint32_t *e_key = lds.e_key;
+    int32_t *e_id = lds.e_id, *sel = lds.sel;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, C = jb.C;
+    const int j = jb.j0 + x;
+    const bool is_sel = j == jb.j_sel;
+    const int n = jb.n_list + jb.first_new + jb.n_new - jb.n_base;
+    for (int u = 0; u < jb.B; ++u) {
+        const float *qbar = jb.qbars + ((int64_t)j * jb.B + u) * C;
+        float *scores = jb.scores + ((int64_t)j * jb.B + u) * jb.cols;
+        // the ranking threads' entries, asked for ahead of the scoring
+        int my_id[2] = {-1, -1};
+        float my_score[2] = {0.f, 0.f};
+        if (is_sel) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int e = tid + 256 * i;
+                if (e >= n) continue;
+                my_id[i] = e < jb.n_list ? jb.base[((int64_t)j * jb.B + u) * jb.k + e] : jb.n_base + (e - jb.n_list);
+                if (my_id[i] < jb.first_new) my_score[i] = scores[my_id[i]];
+            }
+        }
+        if (jb.n_new > 0) {
+            float q[CPL][8];
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) {
+                const bool in = c * 512 + lane * 8 < C;
+                const f32x4 lo = in ? *(const f32x4 *)(qbar + c * 512 + lane * 8) : f32x4{0.f, 0.f, 0.f, 0.f};
+                const f32x4 hi = in ? *(const f32x4 *)(qbar + c * 512 + lane * 8 + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) q[c][i] = lo[i], q[c][4 + i] = hi[i];
+            }
+            for (int r = wave; r < jb.n_new; r += 4) {
+                const bf16_t *row = jb.reps + (int64_t)u * jb.rep_sb + (int64_t)(jb.first_new + r) * jb.rep_su + lane * 8;
+                u32x4 w[CPL];
+#pragma unroll
+                for (int c = 0; c < CPL; ++c) w[c] = c * 512 + lane * 8 < C ? *(const u32x4 *)(row + c * 512) : u32x4{0, 0, 0, 0};
+                float acc0 = 0.f, acc1 = 0.f;
+#pragma unroll
+                for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        acc0 += bf16_bits_to_f32(w[c][i] & 0xffffu) * q[c][2 * i];
+                        acc1 += bf16_bits_to_f32(w[c][i] >> 16) * q[c][2 * i + 1];
+                    }
+                float acc = acc0 + acc1;
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+                if (lane == 0) {
+                    scores[jb.first_new + r] = acc;
+                    fresh[r] = acc;
+                }
+            }
+        }
+        if (!is_sel) continue;                                   // workgroup-uniform
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int e = tid + 256 * i;
+            if (e >= n) continue;
+            e_id[e] = my_id[i];
+            e_key[e] = order_key(my_id[i] >= jb.first_new ? fresh[my_id[i] - jb.first_new] : my_score[i]);
+        }
+        __syncthreads();
+        for (int e = tid; e < n; e += 256) {
+            const uint32_t key = e_key[e];
+            const int id = e_id[e];
+            int rank = 0;
+            for (int o = 0; o < n; ++o) rank += (e_key[o] > key || (e_key[o] == key && e_id[o] < id)) ? 1 : 0;
+            if (rank < jb.k) {
+                sel[rank] = id;
+                jb.log[(int64_t)u * jb.k + rank] = id;
+            }
+        }
+        __syncthreads();
+        for (int p = tid; p < jb.pages.n_pages; p += 256) write_page(jb.pages, u, p, sel);
+        __syncthreads();                                         // the lists are rewritten for the next row
+    }
+    if (is_sel) {
+        __threadfence_system();
+        __syncthreads();
+        if (tid == 0) __hip_atomic_store(jb.log + (int64_t)jb.B * jb.k, jb.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}

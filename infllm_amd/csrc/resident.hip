@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "decode.h"
+#include "rank.h"
 
 int infllm_reduce_partials_blocks(const float *d_parts, int32_t B, int32_t n, int32_t exc, int32_t C, float *d_out, void *stream);
 int infllm_attn_stage_blocked(const infllm_attn_args *a, int32_t exc, int64_t block_rows, void *stream, int32_t dim);
@@ -32,6 +33,10 @@ int infllm_attn_merge2(const uint16_t *d_o_part, const float *d_lse_part, int32_
                        void *stream, int32_t dim);
 int infllm_local_score_dim(const infllm_score_args *a, int32_t dim, void *stream);
 int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream, int32_t dim);
+int infllm_local_score_merged_rank(const infllm_score_args *a, const MergeJob *job, const RankJob *rank, int32_t n_rank, void *stream, int32_t dim);
+int infllm_carve_score(const infllm_score_args *a, const MergeJob *job, const void *d_ring_k_raw, const void *d_ring_v, int64_t t0, int32_t bs, int32_t n_units,
+                       int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
+                       int64_t out_sh, void *stream, int32_t dim);
 int infllm_repr_keys_carve(const float *d_ring_score, const void *d_ring_k_raw, int64_t ring_cap, int32_t B, int32_t H, int32_t Hkv,
                            int64_t t0, int32_t bs, int32_t n_units, int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su,
                            int32_t *d_idx_out, const void *d_ring_v, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
@@ -47,162 +52,10 @@ int infllm_key_splits(const infllm_layer_desc *d, int32_t n_queries, int32_t n_t
 
 namespace {
 
-constexpr int kRankEntries = 320;          // the k <= 64 best of the call's start + 256 units carved since
-constexpr int kRankNew = 64;               // units carved by one block
-
-// The page table of a block: selected units, init tokens, overflow remainder of the ring (the order of the host-built
-// tables of stream.hip).
-struct PageList {
-    infllm_page *out;                      // [B, n_pages]
-    int32_t n_unit_pages, n_init_pages, n_pages, tiles_per_unit;
-    int32_t Hkv, bs, init_len, dim;
-    int64_t cursor, overflow_end, ring_cap, init_cap;
-    const bf16_t *init_kv, *ring_k, *ring_v;
-    const uint64_t *chunk;                 // device: chunks of units, [per_chunk, B, 2, Hkv, bs, dim] each
-    int32_t per_chunk, B;
-};
-
-__device__ __forceinline__ void write_page(const PageList &j, int u, int p, const int32_t *ids) {
-    const int64_t unit_elems = (int64_t)j.Hkv * j.bs * j.dim;
-    infllm_page pg;
-    pg.reserved = 0;
-    if (p < j.n_unit_pages) {
-        const int s = p / j.tiles_per_unit, t0 = (p - s * j.tiles_per_unit) * kTile;
-        const int unit = ids[s], ch = unit / j.per_chunk;
-        const bf16_t *kb = (const bf16_t *)(uintptr_t)j.chunk[ch] + (((int64_t)(unit - ch * j.per_chunk) * j.B + u) * 2) * unit_elems + (int64_t)t0 * j.dim;
-        pg.k = kb;
-        pg.v = kb + unit_elems;
-        pg.head_stride = (int64_t)j.bs * j.dim;
-        pg.n_valid = min(j.bs - t0, kTile);
-    } else if (p < j.n_unit_pages + j.n_init_pages) {
-        const int t0 = (p - j.n_unit_pages) * kTile;
-        const bf16_t *ik = j.init_kv + (int64_t)u * 2 * j.Hkv * j.init_cap * j.dim + (int64_t)t0 * j.dim;
-        pg.k = ik;
-        pg.v = ik + (int64_t)j.Hkv * j.init_cap * j.dim;
-        pg.head_stride = j.init_cap * j.dim;
-        pg.n_valid = min(j.init_len - t0, kTile);
-    } else {
-        const int want = p - j.n_unit_pages - j.n_init_pages;
-        int64_t pos = j.cursor, len = 0;
-        for (int i = 0; i <= want; ++i) {          // runs of <= 64 rows that do not cross the end of the ring
-            pos += len;
-            len = min(min(j.overflow_end - pos, (int64_t)kTile), j.ring_cap - pos % j.ring_cap);
-        }
-        const int64_t row = pos % j.ring_cap;
-        pg.k = j.ring_k + ((int64_t)u * j.Hkv * j.ring_cap + row) * j.dim;
-        pg.v = j.ring_v + ((int64_t)u * j.Hkv * j.ring_cap + row) * j.dim;
-        pg.head_stride = j.ring_cap * j.dim;
-        pg.n_valid = (int)len;
-    }
-    j.out[(int64_t)u * j.n_pages + p] = pg;
-}
-
-// After a block has carved n_new units: workgroup x scores them under the mean query of the call's block j0 + x; the one
-// of block j_sel ranks that block's list of the call's start against all units carved since, and turns the selection into
-// the block's page table.
-struct RankJob {
-    const bf16_t *reps;
-    int64_t rep_sb, rep_su;
-    const float *qbars;                    // [blocks][B][C]
-    float *scores;                         // [blocks][B][cols]
-    int64_t cols;
-    const int32_t *base;                   // [blocks][B][k], n_list entries of a row are filled
-    int32_t B, C, k, n_list, n_base, first_new, n_new, j0, j_sel;
-    int32_t *log;                          // pinned: [B][k] ids, then the sequence number
-    int32_t seq;
-    PageList pages;
-};
-
-// (the sums are unit_scores_rows_kernel's, term by term: a unit's score does not depend on which kernel computed it)
 template <int CPL>
 __global__ __launch_bounds__(256) void rank_kernel(RankJob jb) {
-    __shared__ float fresh[kRankNew];
-    __shared__ uint32_t e_key[kRankEntries];
-    __shared__ int32_t e_id[kRankEntries], sel[64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, C = jb.C;
-    const int j = jb.j0 + (int)blockIdx.x;
-    const bool is_sel = j == jb.j_sel;
-    const int n = jb.n_list + jb.first_new + jb.n_new - jb.n_base;
-    for (int u = 0; u < jb.B; ++u) {
-        const float *qbar = jb.qbars + ((int64_t)j * jb.B + u) * C;
-        float *scores = jb.scores + ((int64_t)j * jb.B + u) * jb.cols;
-        // the ranking threads' entries, asked for ahead of the scoring
-        int my_id[2] = {-1, -1};
-        float my_score[2] = {0.f, 0.f};
-        if (is_sel) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int e = tid + 256 * i;
-                if (e >= n) continue;
-                my_id[i] = e < jb.n_list ? jb.base[((int64_t)j * jb.B + u) * jb.k + e] : jb.n_base + (e - jb.n_list);
-                if (my_id[i] < jb.first_new) my_score[i] = scores[my_id[i]];
-            }
-        }
-        if (jb.n_new > 0) {
-            float q[CPL][8];
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) {
-                const bool in = c * 512 + lane * 8 < C;
-                const f32x4 lo = in ? *(const f32x4 *)(qbar + c * 512 + lane * 8) : f32x4{0.f, 0.f, 0.f, 0.f};
-                const f32x4 hi = in ? *(const f32x4 *)(qbar + c * 512 + lane * 8 + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) q[c][i] = lo[i], q[c][4 + i] = hi[i];
-            }
-            for (int r = wave; r < jb.n_new; r += 4) {
-                const bf16_t *row = jb.reps + (int64_t)u * jb.rep_sb + (int64_t)(jb.first_new + r) * jb.rep_su + lane * 8;
-                u32x4 w[CPL];
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) w[c] = c * 512 + lane * 8 < C ? *(const u32x4 *)(row + c * 512) : u32x4{0, 0, 0, 0};
-                float acc0 = 0.f, acc1 = 0.f;
-#pragma unroll
-                for (int c = 0; c < CPL; ++c)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        acc0 += bf16_bits_to_f32(w[c][i] & 0xffffu) * q[c][2 * i];
-                        acc1 += bf16_bits_to_f32(w[c][i] >> 16) * q[c][2 * i + 1];
-                    }
-                float acc = acc0 + acc1;
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-                if (lane == 0) {
-                    scores[jb.first_new + r] = acc;
-                    fresh[r] = acc;
-                }
-            }
-        }
-        if (!is_sel) continue;                                   // workgroup-uniform
-        __syncthreads();
-        auto order = [](float f) {
-            const uint32_t v = __float_as_uint(f);
-            return (v & 0x80000000u) ? ~v : (v | 0x80000000u);
-        };
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int e = tid + 256 * i;
-            if (e >= n) continue;
-            e_id[e] = my_id[i];
-            e_key[e] = order(my_id[i] >= jb.first_new ? fresh[my_id[i] - jb.first_new] : my_score[i]);
-        }
-        __syncthreads();
-        for (int e = tid; e < n; e += 256) {
-            const uint32_t key = e_key[e];
-            const int id = e_id[e];
-            int rank = 0;
-            for (int o = 0; o < n; ++o) rank += (e_key[o] > key || (e_key[o] == key && e_id[o] < id)) ? 1 : 0;
-            if (rank < jb.k) {
-                sel[rank] = id;
-                jb.log[(int64_t)u * jb.k + rank] = id;
-            }
-        }
-        __syncthreads();
-        for (int p = tid; p < jb.pages.n_pages; p += 256) write_page(jb.pages, u, p, sel);
-        __syncthreads();                                         // the lists are rewritten for the next row
-    }
-    if (is_sel) {
-        __threadfence_system();
-        __syncthreads();
-        if (tid == 0) __hip_atomic_store(jb.log + (int64_t)jb.B * jb.k, jb.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    __shared__ RankLds lds;
+    rank_block<CPL>(jb, blockIdx.x, lds);
 }
 
 // the page table of a selection that is already in memory
@@ -460,9 +313,12 @@ infllm_ingest_args ingest_args(const Resident *R, const infllm_resident_call *a,
     return in;
 }
 
-// init tokens and units that leave the window behind a block ending at b1
-int carve(Resident *R, const infllm_resident_call *a, const Carve &c, hipStream_t st) {
+// Init tokens and units that leave the window behind a block ending at b1.  With sc / job the block's scores of those units
+// have not been added yet: the launch that picks their representatives takes them along where it can (*scored), else
+// nothing is done for the units (1 is returned).
+int carve(Resident *R, const infllm_resident_call *a, const Carve &c, hipStream_t st, const infllm_score_args *sc = nullptr, const MergeJob *job = nullptr) {
     const infllm_resident_desc &d = R->d;
+    if (sc && c.count > 0 && (d.block_size % 32 != 0 || d.block_size > 128 || sc->Lq > 512 || job->P > 8)) return 1;
     if (c.take > 0) {
         INFLLM_REQUIRE(R->init_len + c.take <= d.init_cap, "resident: init overflow");
         bf16_t *ik = (bf16_t *)d.d_init_kv + (int64_t)R->init_len * d.dim;
@@ -478,10 +334,13 @@ int carve(Resident *R, const infllm_resident_call *a, const Carve &c, hipStream_
         const int unit = R->n_units, n = std::min(c.count - done, d.units_per_chunk - unit % d.units_per_chunk);
         INFLLM_REQUIRE(unit + n <= a->n_chunks * d.units_per_chunk && unit + n <= a->rep_rows, "resident: no room for unit %d", unit + n - 1);
         bf16_t *home = unit_home(R, a, unit);
-        const int rc = infllm_repr_keys_carve(d.d_ring_score, d.d_ring_k_raw, d.ring_cap, d.B, d.H, d.Hkv, R->cursor, d.block_size, n, d.repr_topk,
+        const int rc = sc ? infllm_carve_score(sc, job, d.d_ring_k_raw, d.d_ring_v, R->cursor, d.block_size, n, d.repr_topk,
+                                               (bf16_t *)a->d_reps + unit * a->rep_su, a->rep_sb, a->rep_su, home, home + unit_elems, 2 * unit_elems,
+                                               (int64_t)d.B * 2 * unit_elems, (int64_t)d.block_size * d.dim, st, d.dim)
+                          : infllm_repr_keys_carve(d.d_ring_score, d.d_ring_k_raw, d.ring_cap, d.B, d.H, d.Hkv, R->cursor, d.block_size, n, d.repr_topk,
                                               (bf16_t *)a->d_reps + unit * a->rep_su, a->rep_sb, a->rep_su, nullptr, d.d_ring_v, home, home + unit_elems,
                                               2 * unit_elems, (int64_t)d.B * 2 * unit_elems, (int64_t)d.block_size * d.dim, st, d.dim);
-        if (rc) return rc;
+        if (rc) return rc < 0 ? rc : infllm_fail(-2, "resident: no carving kernel after the checks");
         R->cursor += (int64_t)n * d.block_size;
         R->n_units += n;
         done += n;
@@ -722,25 +581,34 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
         sc.mask = INFLLM_MASK_WINDOW; sc.accumulate = 1; sc.offset = b0; sc.window = d.n_local;
         sc.d_lse = a->d_lse; sc.softmax_scale = d.softmax_scale;
         sc.d_score = d.d_ring_score; sc.score_sh = d.ring_cap; sc.score_sb = d.H * d.ring_cap; sc.score_cap = d.ring_cap;
-        rc = parts <= 8 ? infllm_local_score_merged(&sc, &job, st, D) : 1;
+        // What the next block waits for comes first where there is a kernel for it - the scores and representatives of the units
+        // that leave the window now, in one launch -, then the rest of the scores, with the merge and the ranking riding along.
+        const Carve c = carve_after(d, R->cursor, R->init_len, b1);
+        const bool one = parts <= 8 && b1 - lo > 1024;               // (the form that carries them takes long key ranges)
+        rc = one ? carve(R, a, c, st, &sc, &job) : 1;
         if (rc < 0) return rc;
-        if (rc == 1) {
-            rc = infllm_attn_merge2(o_loc, lse_loc, nsplit, ns_g ? a->d_o_part2 : nullptr, ns_g ? a->d_lse_part2 : nullptr, ns_g, B, d.H, nb, out, a->o_sb,
-                                    a->o_sh, a->o_sl, a->d_lse, st, D);
-            if (rc) return rc;
-            rc = infllm_local_score_dim(&sc, D, st);
+        const bool early = rc == 0;
+        if (!early) {
+            rc = one ? infllm_local_score_merged(&sc, &job, st, D) : 1;
+            if (rc < 0) return rc;
+            if (rc == 1) {
+                rc = infllm_attn_merge2(o_loc, lse_loc, nsplit, ns_g ? a->d_o_part2 : nullptr, ns_g ? a->d_lse_part2 : nullptr, ns_g, B, d.H, nb, out,
+                                        a->o_sb, a->o_sh, a->o_sl, a->d_lse, st, D);
+                if (rc) return rc;
+                rc = infllm_local_score_dim(&sc, D, st);
+                if (rc) return rc;
+            }
+            rc = carve(R, a, c, st);
             if (rc) return rc;
         }
-        const Carve c = carve_after(d, R->cursor, R->init_len, b1);
-        rc = carve(R, a, c, st);
-        if (rc) return rc;
         R->length = b1;
         ++R->blocks;
         // ---- the next block's selection and page table
         const int N1 = R->n_units;
-        if (i + 1 < n_blocks && (retrieve && (c.count > 0 || N1 > d.topk))) {
+        const bool rank = i + 1 < n_blocks && retrieve && (c.count > 0 || N1 > d.topk);
+        RankJob jb{};
+        if (rank) {
             const bool select = N1 > d.topk;
-            RankJob jb{};
             jb.reps = (const bf16_t *)a->d_reps; jb.rep_sb = a->rep_sb; jb.rep_su = a->rep_su;
             jb.qbars = a->d_qbar; jb.scores = a->d_call_scores; jb.cols = a->scores_cols; jb.base = a->d_base;
             jb.B = B; jb.C = C; jb.k = d.topk; jb.n_list = n_list; jb.n_base = n0; jb.first_new = N; jb.n_new = N1 - N;
@@ -755,7 +623,25 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
                 j_done = i + 1;
                 ++R->ranked;
             }
-            rc = launch_rank(R, jb, jb.n_new > 0 ? n_blocks - (i + 1) : 1, st);
+        }
+        const int n_rank = jb.n_new > 0 ? n_blocks - (i + 1) : 1;
+        bool ranked = !rank;
+        if (early) {
+            sc.j_lo = std::max(lo, R->cursor);
+            const bool carry = rank && C <= 9 * 512 && b1 - sc.j_lo > 1024;
+            rc = carry ? infllm_local_score_merged_rank(&sc, &job, &jb, n_rank, st, D) : infllm_local_score_merged(&sc, &job, st, D);
+            if (rc < 0) return rc;
+            ranked = ranked || carry;
+            if (rc == 1) {                                           // a short window once the units have left it
+                rc = infllm_attn_merge2(o_loc, lse_loc, nsplit, ns_g ? a->d_o_part2 : nullptr, ns_g ? a->d_lse_part2 : nullptr, ns_g, B, d.H, nb, out,
+                                        a->o_sb, a->o_sh, a->o_sl, a->d_lse, st, D);
+                if (rc) return rc;
+                rc = infllm_local_score_dim(&sc, D, st);
+                if (rc) return rc;
+            }
+        }
+        if (!ranked) {
+            rc = launch_rank(R, jb, n_rank, st);
             if (rc) return rc;
         }
     }

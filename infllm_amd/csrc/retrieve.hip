@@ -3,7 +3,7 @@
 // (inf_llm/attention/context_manager.py:159-163, 268-277, 366-383, 664-670).
 // All three are memory-bound; reductions are wavefront-wide with a fixed order, so the
 // outputs are deterministic.
-#include "common.h"
+#include "carve.h"
 
 #include <algorithm>
 #include <atomic>
@@ -120,11 +120,6 @@ void launch_unit_scores_rows(const bf16_t *reps, int64_t rep_stride, int N, cons
 
 // ---------------------------------------------------------------- top-k (radix select)
 constexpr int kSelThreads = 1024;
-
-__device__ __forceinline__ uint32_t order_key(float f) {
-    uint32_t u = __float_as_uint(f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);       // larger float <=> larger key
-}
 
 // exclusive scan of one int per thread over the workgroup; returns the total in *total
 __device__ int block_exclusive_scan(int v, int *wave_tot, int *total) {
@@ -438,11 +433,6 @@ constexpr int kSurvivorCap = 1024;
 constexpr int kTicketSlots = 64;
 static __device__ unsigned int retrieval_tickets[kTicketSlots];       // zero at load; the last workgroup puts its slot back to zero
 
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int o) {
-    const uint32_t lo = __shfl_xor((uint32_t)v, o, 64), hi = __shfl_xor((uint32_t)(v >> 32), o, 64);
-    return ((uint64_t)hi << 32) | lo;
-}
-
 // the selection by one workgroup of kRetrThreads threads over N <= NB * 16 * kRetrThreads scores; a thread keeps its
 // keys (units tid, tid + kRetrThreads, ...) in registers
 template <int NB>
@@ -617,15 +607,6 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
 // ---------------------------------------------------------------- representative keys
 constexpr int kMaxUnit = 2048;             // largest supported unit (block_size)
 
-// The copy of the same units' K and V rows out of the rings into contiguous staging (what infllm_gather_rows does)
-// can ride in the launch that picks their representatives: independent work, one launch less in the stream.
-struct CarveCopy {
-    const bf16_t *ring_a, *ring_b;
-    bf16_t *out_a, *out_b;
-    int64_t ring_cap, t0, out_sb, out_su, out_sh;
-    int32_t Hkv, B, n, unit_rows, x_extra;         // n rows from t0 on; x_extra = extra workgroups along x (0: no copy)
-};
-
 // One wave per (query head, unit, batch row); workgroups with blockIdx.x >= H copy.  A chain of latencies (scores, repr_topk
 // arg-max steps, the chosen rows), so it is kept short: up to 256 scores live in registers as 64-bit composites (order of
 // the score, lower row first), an arg-max is a wave-wide maximum of those, and the rows of four picks are requested
@@ -636,23 +617,8 @@ __global__ __launch_bounds__(64) void repr_keys_kernel(const float *ring_score, 
                                                        int H, int Hkv, int64_t t0, int bs, int repr_topk, bf16_t *rep_out,
                                                        int64_t rep_sb, int64_t rep_su, int32_t *idx_out, CarveCopy cc) {
     extern __shared__ float sc[];                                        // [bs], units beyond 256 rows only
-    constexpr int kChunks = D / 8;
     if ((int)blockIdx.x >= H) {
-        const int64_t g = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * cc.x_extra + ((int)blockIdx.x - H);
-        const int64_t e = g * 64 + threadIdx.x;                        // (ring, batch row, kv head, row, 16-byte chunk)
-        if (e >= (int64_t)2 * cc.B * cc.Hkv * cc.n * kChunks) return;
-        const int c = (int)(e % kChunks);
-        uint32_t rest = (uint32_t)(e / kChunks);
-        const int r = (int)(rest % (uint32_t)cc.n);
-        rest /= (uint32_t)cc.n;
-        const int hk = (int)(rest % (uint32_t)cc.Hkv);
-        rest /= (uint32_t)cc.Hkv;
-        const int bb = (int)(rest % (uint32_t)cc.B);
-        const bool second = rest / (uint32_t)cc.B != 0;
-        const bf16_t *src = (second ? cc.ring_b : cc.ring_a) + (((int64_t)bb * cc.Hkv + hk) * cc.ring_cap + (cc.t0 + r) % cc.ring_cap) * D + c * 8;
-        bf16_t *dst = (second ? cc.out_b : cc.out_a) + (int64_t)bb * cc.out_sb + (int64_t)(r / cc.unit_rows) * cc.out_su +
-                      (int64_t)hk * cc.out_sh + (int64_t)(r % cc.unit_rows) * D + c * 8;
-        *(u32x4 *)dst = *(const u32x4 *)src;
+        carve_copy<D>(cc, (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * cc.x_extra + ((int)blockIdx.x - H)) * 64 + threadIdx.x);
         return;
     }
     const int h = blockIdx.x, u = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
@@ -665,14 +631,12 @@ __global__ __launch_bounds__(64) void repr_keys_kernel(const float *ring_score, 
     int32_t *idx = idx_out ? idx_out + (((int64_t)b * n_units + u) * H + h) * repr_topk : nullptr;
     constexpr int kRegs = 4;
     const bool in_regs = bs <= 64 * kRegs;
-    // composite of a score: larger is better, equal scores by lower row; 0 only for rows that do not exist or are taken
-    auto composite = [&](float x, int r) { return ((uint64_t)(x == x ? order_key(x) : 1u) << 32) | (uint32_t)~r; };
     uint64_t key[kRegs];
     if (in_regs) {
 #pragma unroll
         for (int i = 0; i < kRegs; ++i) {
             const int r = lane + 64 * i;
-            key[i] = r < bs ? composite(srow[row_of(r)], r) : 0;
+            key[i] = r < bs ? pick_key(srow[row_of(r)], r) : 0;
         }
     } else {
         for (int r = lane; r < bs; r += 64) sc[r] = srow[row_of(r)];
@@ -686,7 +650,7 @@ __global__ __launch_bounds__(64) void repr_keys_kernel(const float *ring_score, 
             for (int i = 0; i < kRegs; ++i) best = key[i] > best ? key[i] : best;
         } else {
             for (int r = lane; r < bs; r += 64) {
-                const uint64_t c = composite(sc[r], r);
+                const uint64_t c = pick_key(sc[r], r);
                 best = c < last && c > best ? c : best;
             }
         }

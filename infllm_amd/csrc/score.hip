@@ -10,7 +10,8 @@
 // (B operand) for the whole kernel, while tiles of 64 or 128 queries stream through LDS
 // (A operand, shared by the 4 waves, double buffered).  Exactly one lane writes each
 // (head, key) cell, so results are deterministic.
-#include "common.h"
+#include "carve.h"
+#include "rank.h"
 #include <atomic>
 #include <type_traits>
 
@@ -35,22 +36,39 @@ struct ScoreMerge {
     MergeJob job;
     int32_t score_tiles;               // blockIdx.y below this scores, from there on merges
 };
+// RANK: the launch also ranks the units for the next block (rank.h), in workgroups of their own that are dispatched first:
+// a chain of latencies that needs next to nothing of the chip, and that the scores do not depend on
+struct ScoreMergeRank : ScoreMerge {
+    RankJob rank;
+    int32_t rank_slots, n_rank;        // rows of the grid in front that rank; workgroups in them with something to do
+};
 struct NoScoreMerge {};
+constexpr int kScore = 0, kScoreMerge = 1, kScoreMergeRank = 2;
 
-template <int D, int KS, int QS, bool MERGE = false>
-__global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a, std::conditional_t<MERGE, ScoreMerge, NoScoreMerge> sm) {
+template <int D, int KS, int QS, int WITH = kScore>
+__global__ __launch_bounds__(256, 2) void local_score_kernel(
+    infllm_score_args a, std::conditional_t<WITH == kScoreMergeRank, ScoreMergeRank, std::conditional_t<WITH == kScoreMerge, ScoreMerge, NoScoreMerge>> sm) {
+    constexpr bool MERGE = WITH != kScore;
     constexpr int kWaveKeys = 32 * KS, kKeysPerWg = 4 * kWaveKeys, kQStage = QS;
-    int n_tiles = gridDim.y;
+    int n_tiles = gridDim.y, slot = blockIdx.y;
     PartSets lps{a.n_parts, 0, 0};
+    extern __shared__ __attribute__((aligned(16))) char score_lds[];
+    if constexpr (WITH == kScoreMergeRank) {
+        slot -= sm.rank_slots;
+        if (slot < 0) {
+            const int x = (int)blockIdx.y * gridDim.x + blockIdx.x;
+            if (x < sm.n_rank) rank_block<9>(sm.rank, x, *(RankLds *)score_lds);
+            return;
+        }
+    }
     if constexpr (MERGE) {
         n_tiles = sm.score_tiles;
-        if ((int)blockIdx.y >= n_tiles) {
-            merge_piece<D>(sm.job, ((int64_t)((int)blockIdx.y - n_tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x);
+        if (slot >= n_tiles) {
+            merge_piece<D>(sm.job, ((int64_t)(slot - n_tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x);
             return;
         }
         lps = sm.job.ps;
     }
-    extern __shared__ __attribute__((aligned(16))) char score_lds[];
     bf16_t(*Qs)[kQStage][kQPad<D>] = (bf16_t(*)[kQStage][kQPad<D>])score_lds;                               // [2][QS][kQPad]
     float(*Ls)[kQStage] = (float(*)[kQStage])(score_lds + 2 * kQStage * kQPad<D> * sizeof(bf16_t));      // [2][QS]
     [[maybe_unused]] float *Lall = (float *)Ls;                                                        // MERGE: [Lq rounded up to QS]
@@ -65,7 +83,6 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
     // Workgroups are dispatched x fastest: all heads of one key tile, then the next tile.  The two tiles at either end
     // of a masked key range see only part of the queries and finish early, so they go last: when the grid is a little
     // more than what the chip holds at once, the workgroups that start late are then the short ones.
-    const int slot = blockIdx.y;
     int tile = slot;
     if (n_tiles >= 6 && a.mask != INFLLM_MASK_NONE)
         tile = slot < n_tiles - 4 ? slot + 2 : slot == n_tiles - 4 ? 1 : slot == n_tiles - 3 ? n_tiles - 2 : slot == n_tiles - 2 ? 0 : n_tiles - 1;
@@ -342,7 +359,10 @@ int score_lds_setup() {
             e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)score_lds_bytes<D>(128));
         if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+            e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128, kScoreMerge>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)score_lds_bytes_merged<D>(128, kMergedMaxLq));
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128, kScoreMergeRank>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)score_lds_bytes_merged<D>(128, kMergedMaxLq));
         if (e != hipSuccess) return infllm_fail(-2, "local_score: %s", hipGetErrorString(e));
         lds_set.store(true, std::memory_order_release);
@@ -371,7 +391,7 @@ int score_launch(const infllm_score_args *a, void *stream) {
 }
 
 template <int D>
-int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *stream) {
+int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *stream, const RankJob *rank = nullptr, int n_rank = 0) {
     INFLLM_REQUIRE(a && job, "local_score_merged: null argument");
     INFLLM_REQUIRE(job->out && job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1 && job->P <= 8,
                    "local_score_merged: the merge does not belong to these queries");
@@ -388,13 +408,201 @@ int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *s
     const int64_t merge_wgs = ((int64_t)job->B * job->H * job->Lq * (D / 8) + 255) / 256;
     const int gx = sc.B * sc.H;
     const int merge_slots = (int)((merge_wgs + gx - 1) / gx);
-    hipLaunchKernelGGL((local_score_kernel<D, 2, 128, true>), dim3(gx, (unsigned)(score_tiles + merge_slots)), dim3(256),
+    if (rank) {
+        INFLLM_REQUIRE(rank->C <= 9 * 512 && rank->C % 8 == 0 && n_rank >= 1, "local_score_merged: no ranking for rows of %d elements", rank->C);
+        ScoreMergeRank sm;
+        sm.job = *job;
+        sm.score_tiles = score_tiles;
+        sm.rank = *rank;
+        sm.n_rank = n_rank;
+        sm.rank_slots = (n_rank + gx - 1) / gx;
+        hipLaunchKernelGGL((local_score_kernel<D, 2, 128, kScoreMergeRank>), dim3(gx, (unsigned)(sm.rank_slots + score_tiles + merge_slots)), dim3(256),
+                           score_lds_bytes_merged<D>(128, sc.Lq), (hipStream_t)stream, sc, sm);
+        INFLLM_CHECK_LAUNCH("local_score_merged");
+        return 0;
+    }
+    hipLaunchKernelGGL((local_score_kernel<D, 2, 128, kScoreMerge>), dim3(gx, (unsigned)(score_tiles + merge_slots)), dim3(256),
                        score_lds_bytes_merged<D>(128, sc.Lq), (hipStream_t)stream, sc, ScoreMerge{*job, score_tiles});
     INFLLM_CHECK_LAUNCH("local_score_merged");
     return 0;
 }
 
+// The keys that leave the window behind this block: the block's share of their scores, added to what the earlier blocks left
+// in the track, and at once the representatives of the units they make up (context_manager.py:268-277) - what the next
+// block's retrieval waits for, in one launch in front of the rest of the scores.  A chain of latencies with little work in
+// it (128 keys x 512 queries per workgroup, half of them outside the window), so a workgroup is 16 waves: each takes 32 of
+// the unit's keys (B operand) and every so many-th sub-tile of 32 queries, read straight from memory, and leaves a sub-tile's
+// column sums in LDS; they are added in the order of the queries, as local_score_kernel adds them (the same bits).
+// Workgroups with blockIdx.x >= H copy the units' rows to their home.  One unit and head: 9.4 us, against 10 for scores of
+// 512 keys in a launch of their own plus 5 for the representatives.
+constexpr int kCarveMaxLq = 512, kCarveMaxUnit = 128;
+struct CarveScore {
+    infllm_score_args s;
+    PartSets lps;
+    const bf16_t *ring_k_raw;
+    int64_t t0;
+    int32_t bs, n_units, repr_topk;
+    bf16_t *rep_out;
+    int64_t rep_sb, rep_su;
+    CarveCopy cc;
+};
+
+template <int D>
+__global__ __launch_bounds__(1024) void carve_score_kernel(CarveScore j) {
+    __shared__ float lse_sh[kCarveMaxLq];
+    __shared__ float sums[kCarveMaxLq / 32][2][kCarveMaxUnit];
+    __shared__ float sc[kCarveMaxUnit];
+    const infllm_score_args &a = j.s;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 31, grp = lane >> 5;
+    if ((int)blockIdx.x >= a.H) {
+        carve_copy<D>(j.cc, (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * j.cc.x_extra + ((int)blockIdx.x - a.H)) * 1024 + tid);
+        return;
+    }
+    const int h = blockIdx.x, u = blockIdx.y, b = blockIdx.z, g = h / (a.H / a.Hkv);
+    const float scale = a.softmax_scale * 1.4426950408889634f;
+    const int64_t first = j.t0 + (int64_t)u * j.bs;
+    const int KG = j.bs / 32, QP = 16 / KG;                       // groups of keys, waves that share one
+    const int kg = wave % KG, qp = wave / KG;
+    const int64_t key = first + kg * 32 + col;
+    bf16x8 kreg[D / 16];
+    {
+        const bf16_t *krow = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + (key % a.cap) * a.k_sl + grp * 8;
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) kreg[kk] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(krow + kk * 16));
+    }
+    float track = 0.f;
+    if (tid < j.bs) track = a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + (first + tid) % a.score_cap];
+    // queries that see any of the unit's keys: i < n_q (they all lie behind the keys)
+    const int n_q = (int)max(min((int64_t)a.Lq, first + j.bs - 1 - a.offset + a.window), (int64_t)0);
+    const int n_sub = (n_q + 31) / 32;
+    const bf16_t *qbase = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh;
+    bf16x8 qa[D / 16];
+    auto load_q = [&](int st) {
+        const bf16_t *row = qbase + (int64_t)min(st * 32 + col, a.Lq - 1) * a.q_sl + grp * 8;
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) qa[kk] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(row + kk * 16));
+    };
+    const bool works = qp < QP;
+    if (works && qp < n_sub) load_q(qp);
+    if (tid < n_sub * 32) {                                      // joined log-sum-exps (local_score_kernel's join)
+        const int64_t rows = (int64_t)a.B * a.H * a.Lq;
+        const float *lse = a.d_lse + ((int64_t)b * a.H + h) * a.Lq;
+        float l8[8], m8 = -INFINITY, den = 0.f;
+#pragma unroll
+        for (int p = 0; p < 8; ++p) l8[p] = tid < a.Lq && p < a.n_parts ? lse[j.lps.l(p, rows) + tid] : -INFINITY;
+#pragma unroll
+        for (int p = 0; p < 8; ++p) m8 = fmaxf(m8, l8[p]);
+        if (m8 != -INFINITY) {
+#pragma unroll
+            for (int p = 0; p < 8; ++p) den += __builtin_amdgcn_exp2f(l8[p] - m8);
+        }
+        lse_sh[tid] = den > 0.f ? m8 + log2f(den) : INFINITY;    // +inf => probability 0
+    }
+    __syncthreads();
+    const int win = (int)min(a.window, (int64_t)(1 << 30));
+    auto sub_tile = [&](int st) {
+        f32x16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[kk], kreg[kk], s, 0, 0, 0);
+        if (st + QP < n_sub) load_q(st + QP);                    // behind the exponentials
+        const int64_t e0 = (int64_t)st * 32 - key + a.offset;    // distance of the sub-tile's first query to this lane's key
+        const int d0 = (int)min(max(e0, (int64_t)-(1 << 29)), (int64_t)(1 << 29));
+        float acc = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int qi = 8 * (r >> 2) + 4 * grp + (r & 3), dist = d0 + qi;
+            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale, -lse_sh[st * 32 + qi]));
+            acc += dist >= 0 && dist < win ? p : 0.f;
+        }
+        sums[st][grp][kg * 32 + col] = acc;
+    };
+    if (works) {
+        for (int st = qp; st < n_sub; st += QP) sub_tile(st);
+    }
+    __syncthreads();
+    if (tid < j.bs) {
+        float lo = 0.f, hi = 0.f;
+        for (int st = 0; st < n_sub; ++st) lo += sums[st][0][tid], hi += sums[st][1][tid];
+        sc[tid] = track + (lo + hi);
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    // ---- the representatives (repr_keys_kernel's picks)
+    uint64_t pick[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) pick[i] = lane + 64 * i < j.bs ? pick_key(sc[lane + 64 * i], lane + 64 * i) : 0;
+    const bf16_t *kraw = j.ring_k_raw + ((int64_t)b * a.Hkv + g) * a.cap * D;
+    float a0 = 0.f, a1 = 0.f;
+    for (int it = 0; it < j.repr_topk; it += 4) {
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            w[i] = 0;
+            if (it + i >= j.repr_topk) continue;
+            uint64_t best = pick[0] > pick[1] ? pick[0] : pick[1];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                const uint64_t other = shfl_xor_u64(best, o);
+                best = other > best ? other : best;
+            }
+#pragma unroll
+            for (int e = 0; e < 2; ++e) pick[e] = pick[e] == best ? 0 : pick[e];
+            if (lane * 2 < D) w[i] = *(const uint32_t *)(kraw + ((first + (int)~(uint32_t)best) % a.cap) * D + lane * 2);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (it + i < j.repr_topk) {
+                a0 += bf16_bits_to_f32(w[i] & 0xffffu);
+                a1 += bf16_bits_to_f32(w[i] >> 16);
+            }
+    }
+    const float inv = 1.f / (float)j.repr_topk;
+    if (lane * 2 < D)
+        *(uint32_t *)(j.rep_out + (int64_t)b * j.rep_sb + (int64_t)u * j.rep_su + (int64_t)h * D + lane * 2) = pack_bf16x2(a0 * inv, a1 * inv);
+}
+
 }  // namespace
+
+// library-internal: scores and representatives of the n_units units of bs tokens from position t0 on, which leave the
+// window behind the block of `a` (whose d_lse / n_parts are set from the job's partials), and their rows to their home (as
+// infllm_repr_keys_carve lays them out).  Returns 1, with nothing launched, for units or blocks the kernel does not take.
+int infllm_carve_score(const infllm_score_args *a, const MergeJob *job, const void *d_ring_k_raw, const void *d_ring_v, int64_t t0, int32_t bs, int32_t n_units,
+                       int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
+                       int64_t out_sh, void *stream, int32_t dim) {
+    INFLLM_REQUIRE(a && job && d_ring_k_raw && d_ring_v && d_rep_out && d_out_k && d_out_v, "carve_score: null pointer");
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "carve_score: head_dim %d", dim);
+    if (n_units == 0) return 0;
+    if (bs % 32 != 0 || bs > kCarveMaxUnit || a->Lq > kCarveMaxLq || job->P > 8 || a->mask != INFLLM_MASK_WINDOW || a->cap != a->score_cap) return 1;
+    CarveScore j{};
+    j.s = *a;
+    j.s.d_lse = job->lse_part;
+    j.s.n_parts = job->P;
+    const int rc = check_score_args(&j.s);
+    if (rc) return rc;
+    INFLLM_REQUIRE(repr_topk >= 1 && repr_topk <= bs && n_units > 0 && t0 >= 0 && (int64_t)n_units * bs <= a->cap && n_units <= 65535 && a->B <= 65535,
+                   "carve_score: bad sizes");
+    INFLLM_REQUIRE(t0 + (int64_t)n_units * bs <= a->offset + 1, "carve_score: the units reach into the block");
+    INFLLM_REQUIRE((rep_sb | rep_su) % 2 == 0 && (out_sb | out_su | out_sh) % 8 == 0, "carve_score: bad strides");
+    j.lps = job->ps;
+    j.ring_k_raw = (const bf16_t *)d_ring_k_raw;
+    j.t0 = t0; j.bs = bs; j.n_units = n_units; j.repr_topk = repr_topk;
+    j.rep_out = (bf16_t *)d_rep_out; j.rep_sb = rep_sb; j.rep_su = rep_su;
+    CarveCopy &cc = j.cc;
+    cc.ring_a = (const bf16_t *)d_ring_k_raw; cc.ring_b = (const bf16_t *)d_ring_v;
+    cc.out_a = (bf16_t *)d_out_k; cc.out_b = (bf16_t *)d_out_v;
+    cc.ring_cap = a->cap; cc.t0 = t0; cc.out_sb = out_sb; cc.out_su = out_su; cc.out_sh = out_sh;
+    cc.Hkv = a->Hkv; cc.B = a->B; cc.n = n_units * bs; cc.unit_rows = bs;
+    const int64_t wgs = ((int64_t)2 * a->B * a->Hkv * cc.n * (dim / 8) + 1023) / 1024, per_x = (int64_t)n_units * a->B;
+    INFLLM_REQUIRE((int64_t)2 * a->B * a->Hkv * cc.n * (dim / 8) < (1ll << 32), "carve_score: copy too large");
+    cc.x_extra = (int32_t)((wgs + per_x - 1) / per_x);
+    const dim3 grid(a->H + cc.x_extra, n_units, a->B);
+    if (dim == 128) hipLaunchKernelGGL(carve_score_kernel<128>, grid, dim3(1024), 0, (hipStream_t)stream, j);
+    else hipLaunchKernelGGL(carve_score_kernel<64>, grid, dim3(1024), 0, (hipStream_t)stream, j);
+    INFLLM_CHECK_LAUNCH("carve_score");
+    return 0;
+}
 
 extern "C" int infllm_local_score(const infllm_score_args *a, void *stream) { return score_launch<kD>(a, stream); }
 
@@ -410,4 +618,9 @@ int infllm_local_score_dim(const infllm_score_args *a, int32_t dim, void *stream
 int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream, int32_t dim) {
     INFLLM_REQUIRE(dim == 128 || dim == 64, "local_score: head_dim %d", dim);
     return dim == 128 ? score_launch_merged<128>(a, job, stream) : score_launch_merged<64>(a, job, stream);
+}
+// ... and with the next block's ranking in n_rank workgroups
+int infllm_local_score_merged_rank(const infllm_score_args *a, const MergeJob *job, const RankJob *rank, int32_t n_rank, void *stream, int32_t dim) {
+    INFLLM_REQUIRE(rank && (dim == 128 || dim == 64), "local_score: bad ranking");
+    return dim == 128 ? score_launch_merged<128>(a, job, stream, rank, n_rank) : score_launch_merged<64>(a, job, stream, rank, n_rank);
 }
