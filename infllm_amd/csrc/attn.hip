@@ -1029,6 +1029,7 @@ int infllm_merge_job(const uint16_t *d_o_part, const float *d_lse_part, int32_t 
     INFLLM_REQUIRE(d_o_part && d_lse_part && job, "attn_merge: null pointer");
     INFLLM_REQUIRE(P1 >= 1 && P2 >= 0 && (P2 == 0 || (d_o_part2 && d_lse_part2)), "attn_merge: bad partial sets %d + %d", P1, P2);
     INFLLM_REQUIRE(B > 0 && H > 0 && Lq > 0, "attn_merge: bad sizes B=%d H=%d Lq=%d", B, H, Lq);
+    INFLLM_REQUIRE((int64_t)B * H * Lq < (1ll << 31), "attn_merge: %lld rows", (long long)B * H * Lq);
     INFLLM_REQUIRE(dim == 128 || dim == 64, "attn_merge: rows of %d elements", dim);
     INFLLM_REQUIRE((o_sl % 8 | o_sh % 8 | o_sb % 8) == 0, "attn_merge: output strides must be multiples of 8");
     PartSets ps{P1 + P2, 0, 0};

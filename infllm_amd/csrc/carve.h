@@ -8,8 +8,9 @@
 struct CarveCopy {
     const bf16_t *ring_a, *ring_b;
     bf16_t *out_a, *out_b;
-    int64_t ring_cap, t0, out_sb, out_su, out_sh;
-    int32_t Hkv, B, n, unit_rows, x_extra;         // n rows from t0 on; x_extra = extra workgroups along x (0: no copy)
+    int64_t out_sb, out_su, out_sh;
+    int32_t ring_cap, slot0;                       // n <= ring_cap rows from ring row slot0 on
+    int32_t Hkv, B, n, unit_rows, x_extra;         // x_extra = extra workgroups along x (0: no copy)
 };
 
 // element e = (ring, batch row, kv head, row, 16-byte chunk)
@@ -25,9 +26,10 @@ __device__ __forceinline__ void carve_copy(const CarveCopy &cc, int64_t e) {
     rest /= (uint32_t)cc.Hkv;
     const int bb = (int)(rest % (uint32_t)cc.B);
     const bool second = rest / (uint32_t)cc.B != 0;
-    const bf16_t *src = (second ? cc.ring_b : cc.ring_a) + (((int64_t)bb * cc.Hkv + hk) * cc.ring_cap + (cc.t0 + r) % cc.ring_cap) * D + c * 8;
-    bf16_t *dst = (second ? cc.out_b : cc.out_a) + (int64_t)bb * cc.out_sb + (int64_t)(r / cc.unit_rows) * cc.out_su +
-                  (int64_t)hk * cc.out_sh + (int64_t)(r % cc.unit_rows) * D + c * 8;
+    const int slot = cc.slot0 + r < cc.ring_cap ? cc.slot0 + r : cc.slot0 + r - cc.ring_cap;
+    const bf16_t *src = (second ? cc.ring_b : cc.ring_a) + (((int64_t)bb * cc.Hkv + hk) * cc.ring_cap + slot) * D + c * 8;
+    bf16_t *dst = (second ? cc.out_b : cc.out_a) + (int64_t)bb * cc.out_sb + (int64_t)((uint32_t)r / (uint32_t)cc.unit_rows) * cc.out_su +
+                  (int64_t)hk * cc.out_sh + (int64_t)((uint32_t)r % (uint32_t)cc.unit_rows) * D + c * 8;
     *(u32x4 *)dst = *(const u32x4 *)src;
 }
 

@@ -100,11 +100,11 @@ __device__ __forceinline__ void merge_piece(const MergeJob &mj, int64_t e) {
     const float *lse_part = mj.lse_part;
     const PartSets ps = mj.ps;
     const int P = mj.P, H = mj.H, Lq = mj.Lq;
-    const int64_t rows = (int64_t)mj.B * H * Lq;
+    const int64_t rows = (int64_t)mj.B * H * Lq;                         // (fewer than 2^31)
     constexpr int kPieces = D / 8;
-    const int64_t row = e / kPieces;
+    if (e >= rows * kPieces) return;
+    const uint32_t row = (uint32_t)(e / kPieces);
     const int c = (int)(e % kPieces);
-    if (row >= rows) return;
     // partials in batches of 8 so that the loads of a batch are in flight together (decode-sized blocks merge
     // dozens of partials of very few rows: a chain of dependent loads would be all latency)
     float m = -INFINITY;
@@ -139,7 +139,7 @@ __device__ __forceinline__ void merge_piece(const MergeJob &mj, int64_t e) {
         }
     }
     const float inv = den > 0.f ? 1.f / den : 0.f;
-    const int i = (int)(row % Lq), h = (int)((row / Lq) % H), b = (int)(row / ((int64_t)Lq * H));
+    const uint32_t bh = row / (uint32_t)Lq, i = row - bh * (uint32_t)Lq, b = bh / (uint32_t)H, h = bh - b * (uint32_t)H;
     u32x4 packed{pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv),
                  pack_bf16x2(acc[4] * inv, acc[5] * inv), pack_bf16x2(acc[6] * inv, acc[7] * inv)};
     *(u32x4 *)(mj.out + (int64_t)b * mj.o_sb + (int64_t)h * mj.o_sh + (int64_t)i * mj.o_sl + c * 8) = packed;

@@ -314,9 +314,9 @@ infllm_ingest_args ingest_args(const Resident *R, const infllm_resident_call *a,
 }
 
 // Init tokens and units that leave the window behind a block ending at b1.  With sc / job the block's scores of those units
-// have not been added yet: the launch that picks their representatives takes them along where it can (*scored), else
-// nothing is done for the units (1 is returned).
-int carve(Resident *R, const infllm_resident_call *a, const Carve &c, hipStream_t st, const infllm_score_args *sc = nullptr, const MergeJob *job = nullptr) {
+// have not been added yet: the launch that picks their representatives takes them along, and the merge of the block's
+// partials, where it can; else nothing is done (1 is returned).
+int carve(Resident *R, const infllm_resident_call *a, const Carve &c, hipStream_t st, const infllm_score_args *sc = nullptr, MergeJob *job = nullptr) {
     const infllm_resident_desc &d = R->d;
     if (sc && c.count > 0 && (d.block_size % 32 != 0 || d.block_size > 128 || sc->Lq > 512 || job->P > 8)) return 1;
     if (c.take > 0) {
@@ -341,6 +341,7 @@ int carve(Resident *R, const infllm_resident_call *a, const Carve &c, hipStream_
                                               (bf16_t *)a->d_reps + unit * a->rep_su, a->rep_sb, a->rep_su, nullptr, d.d_ring_v, home, home + unit_elems,
                                               2 * unit_elems, (int64_t)d.B * 2 * unit_elems, (int64_t)d.block_size * d.dim, st, d.dim);
         if (rc) return rc < 0 ? rc : infllm_fail(-2, "resident: no carving kernel after the checks");
+        if (sc) job->out = nullptr;                               // merged along with the first of them
         R->cursor += (int64_t)n * d.block_size;
         R->n_units += n;
         done += n;
@@ -582,7 +583,8 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
         sc.d_lse = a->d_lse; sc.softmax_scale = d.softmax_scale;
         sc.d_score = d.d_ring_score; sc.score_sh = d.ring_cap; sc.score_sb = d.H * d.ring_cap; sc.score_cap = d.ring_cap;
         // What the next block waits for comes first where there is a kernel for it - the scores and representatives of the units
-        // that leave the window now, in one launch -, then the rest of the scores, with the merge and the ranking riding along.
+        // that leave the window now, in one launch that merges the block's partials along the way -, then the rest of the scores,
+        // with the ranking riding along.
         const Carve c = carve_after(d, R->cursor, R->init_len, b1);
         const bool one = parts <= 8 && b1 - lo > 1024;               // (the form that carries them takes long key ranges)
         rc = one ? carve(R, a, c, st, &sc, &job) : 1;
@@ -633,8 +635,8 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             if (rc < 0) return rc;
             ranked = ranked || carry;
             if (rc == 1) {                                           // a short window once the units have left it
-                rc = infllm_attn_merge2(o_loc, lse_loc, nsplit, ns_g ? a->d_o_part2 : nullptr, ns_g ? a->d_lse_part2 : nullptr, ns_g, B, d.H, nb, out,
-                                        a->o_sb, a->o_sh, a->o_sl, a->d_lse, st, D);
+                rc = job.out ? infllm_attn_merge2(o_loc, lse_loc, nsplit, ns_g ? a->d_o_part2 : nullptr, ns_g ? a->d_lse_part2 : nullptr, ns_g, B, d.H, nb,
+                                                  out, a->o_sb, a->o_sh, a->o_sl, a->d_lse, st, D) : 0;
                 if (rc) return rc;
                 rc = infllm_local_score_dim(&sc, D, st);
                 if (rc) return rc;

@@ -614,7 +614,7 @@ constexpr int kMaxUnit = 2048;             // largest supported unit (block_size
 // through LDS.  NaN scores never win; a unit without a finite score still yields valid rows.
 template <int D>
 __global__ __launch_bounds__(64) void repr_keys_kernel(const float *ring_score, const bf16_t *ring_k, int64_t ring_cap,
-                                                       int H, int Hkv, int64_t t0, int bs, int repr_topk, bf16_t *rep_out,
+                                                       int H, int Hkv, int64_t slot0, int bs, int repr_topk, bf16_t *rep_out,
                                                        int64_t rep_sb, int64_t rep_su, int32_t *idx_out, CarveCopy cc) {
     extern __shared__ float sc[];                                        // [bs], units beyond 256 rows only
     if ((int)blockIdx.x >= H) {
@@ -624,7 +624,8 @@ __global__ __launch_bounds__(64) void repr_keys_kernel(const float *ring_score, 
     const int h = blockIdx.x, u = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
     const int n_units = gridDim.y;
     const int g = h / (H / Hkv);
-    const int64_t first = (t0 + (int64_t)u * bs) % ring_cap;
+    int64_t first = slot0 + (int64_t)u * bs;                             // (all the units fit the ring)
+    first -= first >= ring_cap ? ring_cap : 0;
     const float *srow = ring_score + ((int64_t)b * H + h) * ring_cap;
     auto row_of = [&](int r) { return first + r < ring_cap ? first + r : first + r - ring_cap; };
     const bf16_t *kbase = ring_k + ((int64_t)b * Hkv + g) * ring_cap * D;
@@ -1100,7 +1101,8 @@ int infllm_repr_keys_carve(const float *d_ring_score, const void *d_ring_k_raw, 
         INFLLM_REQUIRE(d_out_k && d_out_v && (out_sb % 8 | out_su % 8 | out_sh % 8) == 0, "repr_keys: bad copy destination");
         cc.ring_a = (const bf16_t *)d_ring_k_raw; cc.ring_b = (const bf16_t *)d_ring_v;
         cc.out_a = (bf16_t *)d_out_k; cc.out_b = (bf16_t *)d_out_v;
-        cc.ring_cap = ring_cap; cc.t0 = t0; cc.out_sb = out_sb; cc.out_su = out_su; cc.out_sh = out_sh;
+        INFLLM_REQUIRE(ring_cap < (1ll << 30), "repr_keys: ring too large");
+        cc.ring_cap = (int32_t)ring_cap; cc.slot0 = (int32_t)(t0 % ring_cap); cc.out_sb = out_sb; cc.out_su = out_su; cc.out_sh = out_sh;
         cc.Hkv = Hkv; cc.B = B; cc.n = n_units * bs; cc.unit_rows = bs;
         INFLLM_REQUIRE((int64_t)2 * B * Hkv * cc.n * (dim / 8) < (1ll << 32), "repr_keys: copy too large");
         const int64_t waves = ((int64_t)2 * B * Hkv * cc.n * (dim / 8) + 63) / 64, per_x = (int64_t)n_units * B;
@@ -1108,7 +1110,7 @@ int infllm_repr_keys_carve(const float *d_ring_score, const void *d_ring_k_raw, 
     }
     const size_t lds = bs > 256 ? (size_t)bs * sizeof(float) : 0;
     hipLaunchKernelGGL((dim == 64 ? repr_keys_kernel<64> : repr_keys_kernel<128>), dim3(H + cc.x_extra, n_units, B), dim3(64), lds, (hipStream_t)stream, d_ring_score,
-                       (const bf16_t *)d_ring_k_raw, ring_cap, H, Hkv, t0, bs, repr_topk, (bf16_t *)d_rep_out, rep_sb,
+                       (const bf16_t *)d_ring_k_raw, ring_cap, H, Hkv, t0 % ring_cap, bs, repr_topk, (bf16_t *)d_rep_out, rep_sb,
                        rep_su, d_idx_out, cc);
     INFLLM_CHECK_LAUNCH("repr_keys");
     return 0;

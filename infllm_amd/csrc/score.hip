@@ -12,6 +12,7 @@
 // (head, key) cell, so results are deterministic.
 #include "carve.h"
 #include "rank.h"
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -393,7 +394,7 @@ int score_launch(const infllm_score_args *a, void *stream) {
 template <int D>
 int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *stream, const RankJob *rank = nullptr, int n_rank = 0) {
     INFLLM_REQUIRE(a && job, "local_score_merged: null argument");
-    INFLLM_REQUIRE(job->out && job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1 && job->P <= 8,
+    INFLLM_REQUIRE(job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1 && job->P <= 8,
                    "local_score_merged: the merge does not belong to these queries");
     infllm_score_args sc = *a;
     sc.d_lse = job->lse_part;
@@ -407,7 +408,7 @@ int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *s
     const int score_tiles = (int)((tiles + 3) / 4);
     const int64_t merge_wgs = ((int64_t)job->B * job->H * job->Lq * (D / 8) + 255) / 256;
     const int gx = sc.B * sc.H;
-    const int merge_slots = (int)((merge_wgs + gx - 1) / gx);
+    const int merge_slots = job->out ? (int)((merge_wgs + gx - 1) / gx) : 0;      // (none: the job has been done by then)
     if (rank) {
         INFLLM_REQUIRE(rank->C <= 9 * 512 && rank->C % 8 == 0 && n_rank >= 1, "local_score_merged: no ranking for rows of %d elements", rank->C);
         ScoreMergeRank sm;
@@ -430,18 +431,18 @@ int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *s
 // The keys that leave the window behind this block: the block's share of their scores, added to what the earlier blocks left
 // in the track, and at once the representatives of the units they make up (context_manager.py:268-277) - what the next
 // block's retrieval waits for, in one launch in front of the rest of the scores.  A chain of latencies with little work in
-// it (128 keys x 512 queries per workgroup, half of them outside the window), so a workgroup is 16 waves: each takes 32 of
-// the unit's keys (B operand) and every so many-th sub-tile of 32 queries, read straight from memory, and leaves a sub-tile's
-// column sums in LDS; they are added in the order of the queries, as local_score_kernel adds them (the same bits).
-// Workgroups with blockIdx.x >= H copy the units' rows to their home.  One unit and head: 9.4 us, against 10 for scores of
-// 512 keys in a launch of their own plus 5 for the representatives.
+// it (a workgroup per unit and head: 128 keys x 512 queries, half of them outside the window), so each step is as short as
+// it can be: a wave per sub-tile of 32 queries, whose rows are requested at once together with everything else the kernel
+// reads; the unit's keys in LDS (every wave needs them all); a sub-tile's column sums added in the order of the queries, as
+// local_score_kernel adds them (the same bits); the picks by counting, all rows at once.  The workgroups behind the heads'
+// copy the units' rows to their home and merge the block's partial outputs: independent work for a chip that is half idle.
 constexpr int kCarveMaxLq = 512, kCarveMaxUnit = 128;
 struct CarveScore {
     infllm_score_args s;
-    PartSets lps;
+    MergeJob merge;
     const bf16_t *ring_k_raw;
-    int64_t t0;
-    int32_t bs, n_units, repr_topk;
+    int32_t slot0, cap, to_first;      // ring row of the first unit; dist of query 0 to the first unit's first key
+    int32_t win, bs, n_units, repr_topk;
     bf16_t *rep_out;
     int64_t rep_sb, rep_su;
     CarveCopy cc;
@@ -449,47 +450,55 @@ struct CarveScore {
 
 template <int D>
 __global__ __launch_bounds__(1024) void carve_score_kernel(CarveScore j) {
+    constexpr int kChunks = D / 8;
+    __shared__ __attribute__((aligned(16))) bf16_t keys[kCarveMaxUnit * D];        // chunk c of row r at c ^ (r mod kChunks)
     __shared__ float lse_sh[kCarveMaxLq];
     __shared__ float sums[kCarveMaxLq / 32][2][kCarveMaxUnit];
-    __shared__ float sc[kCarveMaxUnit];
+    __shared__ uint64_t rank_key[kCarveMaxUnit];
+    __shared__ int32_t chosen[kCarveMaxUnit];
     const infllm_score_args &a = j.s;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 31, grp = lane >> 5;
     if ((int)blockIdx.x >= a.H) {
-        carve_copy<D>(j.cc, (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * j.cc.x_extra + ((int)blockIdx.x - a.H)) * 1024 + tid);
+        const int x = (int)blockIdx.x - a.H;
+        const int64_t wg = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
+        if (x < j.cc.x_extra) carve_copy<D>(j.cc, (wg * j.cc.x_extra + x) * 1024 + tid);
+        else merge_piece<D>(j.merge, (wg * ((int)gridDim.x - a.H - j.cc.x_extra) + (x - j.cc.x_extra)) * 1024 + tid);
         return;
     }
-    const int h = blockIdx.x, u = blockIdx.y, b = blockIdx.z, g = h / (a.H / a.Hkv);
+    const int h = blockIdx.x, u = blockIdx.y, b = blockIdx.z, g = h / (a.H / a.Hkv), bs = j.bs;
     const float scale = a.softmax_scale * 1.4426950408889634f;
-    const int64_t first = j.t0 + (int64_t)u * j.bs;
-    const int KG = j.bs / 32, QP = 16 / KG;                       // groups of keys, waves that share one
-    const int kg = wave % KG, qp = wave / KG;
-    const int64_t key = first + kg * 32 + col;
-    bf16x8 kreg[D / 16];
-    {
-        const bf16_t *krow = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + (key % a.cap) * a.k_sl + grp * 8;
-#pragma unroll
-        for (int kk = 0; kk < D / 16; ++kk) kreg[kk] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(krow + kk * 16));
-    }
-    float track = 0.f;
-    if (tid < j.bs) track = a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + (first + tid) % a.score_cap];
-    // queries that see any of the unit's keys: i < n_q (they all lie behind the keys)
-    const int n_q = (int)max(min((int64_t)a.Lq, first + j.bs - 1 - a.offset + a.window), (int64_t)0);
-    const int n_sub = (n_q + 31) / 32;
-    const bf16_t *qbase = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh;
+    auto slot_of = [&](int r) {                                   // ring row of row r of the unit
+        const int s = j.slot0 + u * bs + r;
+        return s < j.cap ? s : s - j.cap;
+    };
+    // queries that see any of the unit's keys: i < n_q (they all lie behind the keys), one sub-tile of 32 a wave
+    const int d_first = j.to_first - u * bs;                      // distance of query 0 to the unit's first key
+    const int n_q = max(min(a.Lq, j.win + bs - 1 - d_first), 0), n_sub = (n_q + 31) / 32;
+    const bool works = wave < n_sub;
     bf16x8 qa[D / 16];
-    auto load_q = [&](int st) {
-        const bf16_t *row = qbase + (int64_t)min(st * 32 + col, a.Lq - 1) * a.q_sl + grp * 8;
+    if (works) {
+        const bf16_t *row = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)min(wave * 32 + col, a.Lq - 1) * a.q_sl + grp * 8;
 #pragma unroll
         for (int kk = 0; kk < D / 16; ++kk) qa[kk] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(row + kk * 16));
-    };
-    const bool works = qp < QP;
-    if (works && qp < n_sub) load_q(qp);
+    }
+    constexpr int kLoads = kCarveMaxUnit * kChunks / 1024;
+    u32x4 k_in[kLoads], raw_in[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int r = (tid + i * 1024) / kChunks, c = tid % kChunks;
+        if (r >= bs) continue;
+        const int64_t at = (int64_t)slot_of(r);
+        k_in[i] = *(const u32x4 *)((const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + at * a.k_sl + c * 8);
+        raw_in[i] = *(const u32x4 *)(j.ring_k_raw + (((int64_t)b * a.Hkv + g) * j.cap + at) * D + c * 8);
+    }
+    float track = 0.f;
+    if (tid < bs) track = a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + slot_of(tid)];
     if (tid < n_sub * 32) {                                      // joined log-sum-exps (local_score_kernel's join)
         const int64_t rows = (int64_t)a.B * a.H * a.Lq;
         const float *lse = a.d_lse + ((int64_t)b * a.H + h) * a.Lq;
         float l8[8], m8 = -INFINITY, den = 0.f;
 #pragma unroll
-        for (int p = 0; p < 8; ++p) l8[p] = tid < a.Lq && p < a.n_parts ? lse[j.lps.l(p, rows) + tid] : -INFINITY;
+        for (int p = 0; p < 8; ++p) l8[p] = tid < a.Lq && p < a.n_parts ? lse[j.merge.ps.l(p, rows) + tid] : -INFINITY;
 #pragma unroll
         for (int p = 0; p < 8; ++p) m8 = fmaxf(m8, l8[p]);
         if (m8 != -INFINITY) {
@@ -498,76 +507,90 @@ __global__ __launch_bounds__(1024) void carve_score_kernel(CarveScore j) {
         }
         lse_sh[tid] = den > 0.f ? m8 + log2f(den) : INFINITY;    // +inf => probability 0
     }
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int r = (tid + i * 1024) / kChunks, c = tid % kChunks;
+        if (r < bs) *(u32x4 *)&keys[(r * kChunks + (c ^ (r % kChunks))) * 8] = k_in[i];
+    }
     __syncthreads();
-    const int win = (int)min(a.window, (int64_t)(1 << 30));
-    auto sub_tile = [&](int st) {
-        f32x16 s;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = 0.f;
-#pragma unroll
-        for (int kk = 0; kk < D / 16; ++kk) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[kk], kreg[kk], s, 0, 0, 0);
-        if (st + QP < n_sub) load_q(st + QP);                    // behind the exponentials
-        const int64_t e0 = (int64_t)st * 32 - key + a.offset;    // distance of the sub-tile's first query to this lane's key
-        const int d0 = (int)min(max(e0, (int64_t)-(1 << 29)), (int64_t)(1 << 29));
-        float acc = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int qi = 8 * (r >> 2) + 4 * grp + (r & 3), dist = d0 + qi;
-            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale, -lse_sh[st * 32 + qi]));
-            acc += dist >= 0 && dist < win ? p : 0.f;
-        }
-        sums[st][grp][kg * 32 + col] = acc;
-    };
     if (works) {
-        for (int st = qp; st < n_sub; st += QP) sub_tile(st);
-    }
-    __syncthreads();
-    if (tid < j.bs) {
-        float lo = 0.f, hi = 0.f;
-        for (int st = 0; st < n_sub; ++st) lo += sums[st][0][tid], hi += sums[st][1][tid];
-        sc[tid] = track + (lo + hi);
-    }
-    __syncthreads();
-    if (wave != 0) return;
-    // ---- the representatives (repr_keys_kernel's picks)
-    uint64_t pick[2];
+        f32x4 l4[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) pick[i] = lane + 64 * i < j.bs ? pick_key(sc[lane + 64 * i], lane + 64 * i) : 0;
-    const bf16_t *kraw = j.ring_k_raw + ((int64_t)b * a.Hkv + g) * a.cap * D;
-    float a0 = 0.f, a1 = 0.f;
-    for (int it = 0; it < j.repr_topk; it += 4) {
-        uint32_t w[4];
+        for (int q4 = 0; q4 < 4; ++q4) l4[q4] = *(const f32x4 *)&lse_sh[wave * 32 + 8 * q4 + 4 * grp];
+        for (int kg = 0; kg < bs / 32; ++kg) {
+            const bf16_t *krow = &keys[(kg * 32 + col) * D];
+            f32x16 s;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            w[i] = 0;
-            if (it + i >= j.repr_topk) continue;
-            uint64_t best = pick[0] > pick[1] ? pick[0] : pick[1];
+            for (int r = 0; r < 16; ++r) s[r] = 0.f;
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                const uint64_t other = shfl_xor_u64(best, o);
-                best = other > best ? other : best;
+            for (int kk = 0; kk < D / 16; ++kk)
+                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[kk], *(const bf16x8 *)(krow + ((kk * 2 + grp) ^ (col % kChunks)) * 8), s, 0, 0, 0);
+            const int e0 = d_first + wave * 32 - kg * 32;        // distance of the sub-tile's first query to the group's first key
+            float acc = 0.f;
+            if (e0 - 31 >= 0 && e0 + 31 < j.win) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc += __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale, -l4[r >> 2][r & 3]));
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int dist = e0 - col + 8 * (r >> 2) + 4 * grp + (r & 3);
+                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale, -l4[r >> 2][r & 3]));
+                    acc += dist >= 0 && dist < j.win ? p : 0.f;
+                }
             }
-#pragma unroll
-            for (int e = 0; e < 2; ++e) pick[e] = pick[e] == best ? 0 : pick[e];
-            if (lane * 2 < D) w[i] = *(const uint32_t *)(kraw + ((first + (int)~(uint32_t)best) % a.cap) * D + lane * 2);
+            sums[wave][grp][kg * 32 + col] = acc;
         }
+    }
+    __syncthreads();
+    // ---- the representatives: row r's place in the order is the number of rows in front of it; the raw keys take the place
+    //      of the rotated ones meanwhile
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (it + i < j.repr_topk) {
-                a0 += bf16_bits_to_f32(w[i] & 0xffffu);
-                a1 += bf16_bits_to_f32(w[i] >> 16);
+    for (int i = 0; i < kLoads; ++i)
+        if ((tid + i * 1024) / kChunks < bs) *(u32x4 *)&keys[(tid + i * 1024) * 8] = raw_in[i];
+    if (tid < kCarveMaxUnit) {
+        uint64_t key = 0;
+        if (tid < bs) {
+            float lo = 0.f, hi = 0.f;
+            if (n_sub == kCarveMaxLq / 32) {
+#pragma unroll
+                for (int st = 0; st < kCarveMaxLq / 32; ++st) lo += sums[st][0][tid], hi += sums[st][1][tid];
+            } else {
+#pragma unroll 4
+                for (int st = 0; st < n_sub; ++st) lo += sums[st][0][tid], hi += sums[st][1][tid];
             }
+            key = pick_key(track + (lo + hi), tid);
+        }
+        rank_key[tid] = key;
+    }
+    __syncthreads();
+    {
+        const int r = tid >> 3, p = tid & 7;
+        const uint64_t own = rank_key[r];
+        int before = 0;
+#pragma unroll
+        for (int i = 0; i < kCarveMaxUnit / 8; ++i) before += rank_key[i * 8 + p] > own;
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) before += __shfl_xor(before, o, 64);
+        if (p == 0 && r < bs && before < j.repr_topk) chosen[before] = r;
+    }
+    __syncthreads();
+    if (tid * 2 >= D) return;
+    float a0 = 0.f, a1 = 0.f;
+    for (int i = 0; i < j.repr_topk; ++i) {
+        const uint32_t w = *(const uint32_t *)&keys[chosen[i] * D + tid * 2];
+        a0 += bf16_bits_to_f32(w & 0xffffu);
+        a1 += bf16_bits_to_f32(w >> 16);
     }
     const float inv = 1.f / (float)j.repr_topk;
-    if (lane * 2 < D)
-        *(uint32_t *)(j.rep_out + (int64_t)b * j.rep_sb + (int64_t)u * j.rep_su + (int64_t)h * D + lane * 2) = pack_bf16x2(a0 * inv, a1 * inv);
+    *(uint32_t *)(j.rep_out + (int64_t)b * j.rep_sb + (int64_t)u * j.rep_su + (int64_t)h * D + tid * 2) = pack_bf16x2(a0 * inv, a1 * inv);
 }
 
 }  // namespace
 
 // library-internal: scores and representatives of the n_units units of bs tokens from position t0 on, which leave the
-// window behind the block of `a` (whose d_lse / n_parts are set from the job's partials), and their rows to their home (as
-// infllm_repr_keys_carve lays them out).  Returns 1, with nothing launched, for units or blocks the kernel does not take.
+// window behind the block of `a` (whose d_lse / n_parts are set from the job's partials), their rows to their home (as
+// infllm_repr_keys_carve lays them out), and the job itself, the merge of the block's partials (job->out NULL: none).  Returns 1, with nothing
+// launched, for units or blocks the kernel does not take.
 int infllm_carve_score(const infllm_score_args *a, const MergeJob *job, const void *d_ring_k_raw, const void *d_ring_v, int64_t t0, int32_t bs, int32_t n_units,
                        int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
                        int64_t out_sh, void *stream, int32_t dim) {
@@ -585,19 +608,24 @@ int infllm_carve_score(const infllm_score_args *a, const MergeJob *job, const vo
                    "carve_score: bad sizes");
     INFLLM_REQUIRE(t0 + (int64_t)n_units * bs <= a->offset + 1, "carve_score: the units reach into the block");
     INFLLM_REQUIRE((rep_sb | rep_su) % 2 == 0 && (out_sb | out_su | out_sh) % 8 == 0, "carve_score: bad strides");
-    j.lps = job->ps;
+    INFLLM_REQUIRE(job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1, "carve_score: the merge does not belong to these queries");
+    INFLLM_REQUIRE(a->cap < (1ll << 30), "carve_score: ring too large");
+    j.merge = *job;
     j.ring_k_raw = (const bf16_t *)d_ring_k_raw;
-    j.t0 = t0; j.bs = bs; j.n_units = n_units; j.repr_topk = repr_topk;
+    j.slot0 = (int32_t)(t0 % a->cap); j.cap = (int32_t)a->cap; j.bs = bs; j.n_units = n_units; j.repr_topk = repr_topk;
+    j.to_first = (int32_t)std::min<int64_t>(a->offset - t0, 1 << 29);
+    j.win = (int32_t)std::min<int64_t>(a->window, 1 << 28);
     j.rep_out = (bf16_t *)d_rep_out; j.rep_sb = rep_sb; j.rep_su = rep_su;
     CarveCopy &cc = j.cc;
     cc.ring_a = (const bf16_t *)d_ring_k_raw; cc.ring_b = (const bf16_t *)d_ring_v;
     cc.out_a = (bf16_t *)d_out_k; cc.out_b = (bf16_t *)d_out_v;
-    cc.ring_cap = a->cap; cc.t0 = t0; cc.out_sb = out_sb; cc.out_su = out_su; cc.out_sh = out_sh;
+    cc.ring_cap = j.cap; cc.slot0 = j.slot0; cc.out_sb = out_sb; cc.out_su = out_su; cc.out_sh = out_sh;
     cc.Hkv = a->Hkv; cc.B = a->B; cc.n = n_units * bs; cc.unit_rows = bs;
-    const int64_t wgs = ((int64_t)2 * a->B * a->Hkv * cc.n * (dim / 8) + 1023) / 1024, per_x = (int64_t)n_units * a->B;
-    INFLLM_REQUIRE((int64_t)2 * a->B * a->Hkv * cc.n * (dim / 8) < (1ll << 32), "carve_score: copy too large");
-    cc.x_extra = (int32_t)((wgs + per_x - 1) / per_x);
-    const dim3 grid(a->H + cc.x_extra, n_units, a->B);
+    const int64_t per_x = (int64_t)n_units * a->B, elems = (int64_t)2 * a->B * a->Hkv * cc.n * (dim / 8), pieces = (int64_t)a->B * a->H * a->Lq * (dim / 8);
+    INFLLM_REQUIRE(elems < (1ll << 32), "carve_score: copy too large");
+    cc.x_extra = (int32_t)(((elems + 1023) / 1024 + per_x - 1) / per_x);
+    const int32_t x_merge = job->out ? (int32_t)(((pieces + 1023) / 1024 + per_x - 1) / per_x) : 0;
+    const dim3 grid(a->H + cc.x_extra + x_merge, n_units, a->B);
     if (dim == 128) hipLaunchKernelGGL(carve_score_kernel<128>, grid, dim3(1024), 0, (hipStream_t)stream, j);
     else hipLaunchKernelGGL(carve_score_kernel<64>, grid, dim3(1024), 0, (hipStream_t)stream, j);
     INFLLM_CHECK_LAUNCH("carve_score");
