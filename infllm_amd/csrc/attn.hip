@@ -156,8 +156,15 @@ struct KernargLayout {                     // the arguments as the launch lays t
     InlinePages pages;
 };
 
+// Heads of 64 leave room for two workgroups on a CU: half the accumulators and operands fit 128 registers (four waves per
+// SIMD), the tiles 64 KB.  Their arithmetic per tile is bound by the exponentials (32 of 16 cycles a wave against 512 cycles
+// of MFMA), and within one wave the two only add up; with four waves one's MFMAs run under another's exponentials (36 heads,
+// prompt of 24,300 tokens, with the scores' smaller workgroups: 4474 -> 3550 us a pass).
+template <int D, int MODE>
+constexpr int kWgsPerCu = D == 64 && (MODE == kLinear || MODE == kPaged) ? 2 : 1;
+
 template <int D, int MODE, bool INLINE = false>
-__global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_args a, infllm_attn_args a2, StageGeom geo,
+__global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage_kernel(infllm_attn_args a, infllm_attn_args a2, StageGeom geo,
                                                                  std::conditional_t<INLINE, InlinePages, NoInlinePages>) {
     constexpr bool HAS_LIN = MODE != kPaged, HAS_PAG = MODE != kLinear, TWO = MODE == kBoth || MODE == kSinks;
     constexpr int kRow = D * 2, kTB = kTileBytes<D>;                     // bytes of a row, of a tile
@@ -355,6 +362,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
 
     auto tile_math = [&](int buf, int t) {
         const char *kb = Ks + buf * kTB, *vb = Vs + buf * kTB;
+        // Heads of 64: registers are what two workgroups on a CU are short of, so an operand's address is made from the first
+        // one's where it is read: kk flips chunk bits 1 and 2 of a K row.  (Said anew per tile, or the compiler keeps them all.)
+        uint32_t k_base = k_off[0];
+        if (D == 64) asm volatile("" : "+v"(k_base));
         f32x16 s[2];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
@@ -363,24 +374,24 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
         {
             // 16 K operands in groups of 4 (kk pair x both sub-tiles): a group is requested from LDS while the
             // MFMAs of the previous one run; scheduling fences keep the compiler from serialising read -> MFMA
-            constexpr int NG = D / 32;                 // (16 K operands of heads of 128, 8 of heads of 64)
-            bf16x8 ka[NG][4];
+            constexpr int KG = D == 128 ? 4 : 2, NG = D / 8 / KG;      // (heads of 64: 8 operands, in groups of 2)
+            bf16x8 ka[NG][KG];
             auto k_operand = [&](int i) {          // i = kk * 2 + ks
-                return *(const bf16x8 *)(kb + (i & 1) * 32 * kRow + k_off[i >> 1]);
+                return *(const bf16x8 *)(kb + (i & 1) * 32 * kRow + (D == 128 ? k_off[i >> 1] : k_base ^ ((i >> 1) * 32)));
             };
 #pragma unroll
-            for (int j = 0; j < 4; ++j) ka[0][j] = k_operand(j);
+            for (int j = 0; j < KG; ++j) ka[0][j] = k_operand(j);
 #pragma unroll
             for (int gi = 0; gi < NG; ++gi) {
                 __builtin_amdgcn_sched_barrier(0);
                 if (gi < NG - 1) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) ka[gi + 1][j] = k_operand((gi + 1) * 4 + j);
+                    for (int j = 0; j < KG; ++j) ka[gi + 1][j] = k_operand((gi + 1) * KG + j);
                     __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int i = gi * 4 + j;
+                for (int j = 0; j < KG; ++j) {
+                    const int i = gi * KG + j;
                     s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[gi][j], qreg[i >> 1], s[i & 1], 0, 0, 0);
                 }
             }
@@ -474,6 +485,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
             // 4 steps of 16 keys, 4 MFMAs each; the V^T operands of a step are requested from LDS while the
             // MFMAs of the previous step run
             typedef short s16x8 __attribute__((ext_vector_type(8)));
+            constexpr bool AHEAD = D == 128;      // (heads of 64: the SIMD's other waves fill the wait, see kWgsPerCu)
             s16x8 va[2][D / 32];
             auto v_operands = [&](int gi, s16x8 *dst) {
 #pragma unroll
@@ -482,11 +494,12 @@ __global__ __launch_bounds__(kThreads, 2) void attn_stage_kernel(infllm_attn_arg
                     dst[dt].hi = lds_read_tr((const bf16_t *)(vb + gi * 16 * kRow + v_off[dt][1]));
                 }
             };
-            v_operands(0, va[0]);
+            if (AHEAD) v_operands(0, va[0]);
 #pragma unroll
             for (int gi = 0; gi < 4; ++gi) {
                 __builtin_amdgcn_sched_barrier(0);
-                if (gi < 3) {
+                if (!AHEAD) v_operands(gi, va[gi & 1]);
+                if (AHEAD && gi < 3) {
                     v_operands(gi + 1, va[(gi + 1) & 1]);
                     __builtin_amdgcn_sched_barrier(0);
                 }

@@ -436,6 +436,19 @@ int decode_step(Resident *R, const infllm_resident_call *a, int64_t st0, hipStre
     return 0;
 }
 
+// Key splits of the global stage.  Heads of 128: a CU holds one workgroup, the host-driven path's rule (and its bits).  Heads
+// of 64: it holds two, so the chip is full at twice as many workgroups, and a launch of a little more than that would start
+// over for the few; a workgroup keeps four tiles or more.
+int stage_splits(const infllm_resident_desc &d, int n_queries, int n_tiles) {
+    if (d.dim == 64 && n_queries > 32) {
+        const int wgs = (((n_queries + 31) / 32) * (d.H / d.Hkv) + 7) / 8 * d.Hkv * d.B;
+        return std::max(1, std::min({2 * d.num_cus / wgs, n_tiles / 4, d.max_splits}));
+    }
+    infllm_layer_desc geo{};
+    geo.B = d.B; geo.H = d.H; geo.Hkv = d.Hkv; geo.exc = d.exc; geo.max_splits = d.max_splits; geo.num_cus = d.num_cus;
+    return infllm_key_splits(&geo, n_queries, n_tiles);
+}
+
 // n queries, worked off in execution blocks
 int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, hipStream_t st) {
     const infllm_resident_desc &d = R->d;
@@ -555,7 +568,9 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             at.cap = kTile;
             at.d_pages = d.d_pages; at.n_pages = pl.n_pages;
             at.softmax_scale = d.softmax_scale;
-            at.nsplit = ns_g = infllm_key_splits(&geo, nb, pl.n_pages);
+            ns_g = stage_splits(d, nb, pl.n_pages);
+            if (D == 64) ns_g = std::min(ns_g, std::max(1, 8 - nsplit));              // (up to 8 partials are merged along with the scores)
+            at.nsplit = ns_g;
             at.d_o_part = a->d_o_part2; at.d_lse_part = a->d_lse_part2;
             INFLLM_REQUIRE((int64_t)ns_g * B * d.H * nb <= a->part_rows2, "resident: global partial rows do not fit");
             const int tw = timer_begin(R, 2, nb, 0, st);          // (where the stream of the host-driven path waits for missed units)
@@ -665,10 +680,8 @@ extern "C" int infllm_resident_fits(const infllm_resident_desc *d) {
 
 extern "C" int64_t infllm_resident_part_rows(const infllm_resident_desc *d) {
     if (!d || d->B <= 0 || d->H <= 0 || d->Hkv <= 0 || d->H % d->Hkv || d->exc <= 0) return infllm_fail(-1, "resident_part_rows: bad descriptor");
-    infllm_layer_desc geo{};
-    geo.B = d->B; geo.H = d->H; geo.Hkv = d->Hkv; geo.exc = d->exc; geo.max_splits = d->max_splits; geo.num_cus = d->num_cus;
     int64_t rows = 0;
-    for (int n = 1; n <= d->exc; ++n) rows = std::max<int64_t>(rows, (int64_t)infllm_key_splits(&geo, n, d->max_pages) * n);
+    for (int n = 1; n <= d->exc; ++n) rows = std::max<int64_t>(rows, (int64_t)stage_splits(*d, n, d->max_pages) * n);
     return rows * d->B * d->H;
 }
 

@@ -346,6 +346,7 @@ int check_score_args(const infllm_score_args *a) {
 
 template <int D>
 size_t score_lds_bytes(int qs) { return (size_t)(2 * qs * kQPad<D> * sizeof(bf16_t) + 2 * qs * sizeof(float)); }
+constexpr int kScoreCus = 256;
 constexpr int kMergedMaxLq = 2048;                     // MERGE: 4 bytes of LDS per query of the launch
 template <int D>
 size_t score_lds_bytes_merged(int qs, int lq) { return (size_t)(2 * qs * kQPad<D> * sizeof(bf16_t) + (size_t)((lq + qs - 1) / qs * qs) * sizeof(float)); }
@@ -359,16 +360,20 @@ int score_lds_setup() {
         if (e == hipSuccess)
             e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)score_lds_bytes<D>(128));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128, kScoreMerge>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)score_lds_bytes_merged<D>(128, kMergedMaxLq));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128, kScoreMergeRank>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)score_lds_bytes_merged<D>(128, kMergedMaxLq));
+        for (const void *k : {(const void *)local_score_kernel<D, 2, 128, kScoreMerge>, (const void *)local_score_kernel<D, 2, 128, kScoreMergeRank>,
+                              (const void *)local_score_kernel<D, 1, 128, kScoreMerge>, (const void *)local_score_kernel<D, 1, 128, kScoreMergeRank>})
+            if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)score_lds_bytes_merged<D>(128, kMergedMaxLq));
         if (e != hipSuccess) return infllm_fail(-2, "local_score: %s", hipGetErrorString(e));
         lds_set.store(true, std::memory_order_release);
     }
     return 0;
+}
+
+// Keys of a wave, in 32s.  64 keys halve what a workgroup reads of the queries per key, but a launch of fewer than two
+// workgroups per CU is only as fast as one of them: it takes 32 keys a wave and twice the workgroups
+// (1,999-token prompt: 172 -> 162 us; 16,001 tokens, whose first blocks see few keys: 3276 -> 3223).
+inline bool wide_waves(const infllm_score_args &a) {
+    return a.j_hi - a.j_lo > 1024 && (int64_t)a.B * a.H * (((a.j_hi - 1) / 64 - a.j_lo / 64 + 4) / 4) >= 2 * kScoreCus;
 }
 
 template <int D>
@@ -378,7 +383,7 @@ int score_launch(const infllm_score_args *a, void *stream) {
     if (a->j_hi <= a->j_lo) return 0;
     rc = score_lds_setup<D>();
     if (rc) return rc;
-    if (a->j_hi - a->j_lo > 1024) {
+    if (wide_waves(*a)) {
         const int64_t tiles = (a->j_hi - 1) / 64 - a->j_lo / 64 + 1;
         hipLaunchKernelGGL((local_score_kernel<D, 2, 128>), dim3(a->B * a->H, (unsigned)((tiles + 3) / 4)), dim3(256), score_lds_bytes<D>(128),
                            (hipStream_t)stream, *a, NoScoreMerge{});
@@ -404,7 +409,9 @@ int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *s
     if (sc.j_hi - sc.j_lo <= 1024 || sc.Lq > kMergedMaxLq) return 1;
     rc = score_lds_setup<D>();
     if (rc) return rc;
-    const int64_t tiles = (sc.j_hi - 1) / 64 - sc.j_lo / 64 + 1;
+    const bool wide = wide_waves(sc);
+    const int wave_keys = wide ? 64 : 32;
+    const int64_t tiles = (sc.j_hi - 1) / wave_keys - sc.j_lo / wave_keys + 1;
     const int score_tiles = (int)((tiles + 3) / 4);
     const int64_t merge_wgs = ((int64_t)job->B * job->H * job->Lq * (D / 8) + 255) / 256;
     const int gx = sc.B * sc.H;
@@ -417,13 +424,15 @@ int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *s
         sm.rank = *rank;
         sm.n_rank = n_rank;
         sm.rank_slots = (n_rank + gx - 1) / gx;
-        hipLaunchKernelGGL((local_score_kernel<D, 2, 128, kScoreMergeRank>), dim3(gx, (unsigned)(sm.rank_slots + score_tiles + merge_slots)), dim3(256),
-                           score_lds_bytes_merged<D>(128, sc.Lq), (hipStream_t)stream, sc, sm);
+        const auto kern = wide ? local_score_kernel<D, 2, 128, kScoreMergeRank> : local_score_kernel<D, 1, 128, kScoreMergeRank>;
+        hipLaunchKernelGGL(kern, dim3(gx, (unsigned)(sm.rank_slots + score_tiles + merge_slots)), dim3(256), score_lds_bytes_merged<D>(128, sc.Lq),
+                           (hipStream_t)stream, sc, sm);
         INFLLM_CHECK_LAUNCH("local_score_merged");
         return 0;
     }
-    hipLaunchKernelGGL((local_score_kernel<D, 2, 128, kScoreMerge>), dim3(gx, (unsigned)(score_tiles + merge_slots)), dim3(256),
-                       score_lds_bytes_merged<D>(128, sc.Lq), (hipStream_t)stream, sc, ScoreMerge{*job, score_tiles});
+    const auto kern = wide ? local_score_kernel<D, 2, 128, kScoreMerge> : local_score_kernel<D, 1, 128, kScoreMerge>;
+    hipLaunchKernelGGL(kern, dim3(gx, (unsigned)(score_tiles + merge_slots)), dim3(256), score_lds_bytes_merged<D>(128, sc.Lq), (hipStream_t)stream, sc,
+                       ScoreMerge{*job, score_tiles});
     INFLLM_CHECK_LAUNCH("local_score_merged");
     return 0;
 }

@@ -17,6 +17,8 @@ CASES = [
     ("three heads a group, no sinks", [600, 1, 130], 6, 2, 1, dict(SMALL, n_init=0)),
     ("reference", [8192, 1501, 1, 1], 32, 8, 1, dict(REFERENCE)),
     ("heads of 64", [4100, 1, 1], 12, 12, 1, dict(REFERENCE, n_local=1024, dim=64)),
+    # ... the chip full of them at six key splits, scores of 32 keys a wave
+    ("36 heads of 64", [3300, 700, 1], 36, 36, 1, dict(REFERENCE, n_local=1100, dim=64)),
     ("heads of 32", [900, 1, 200], 8, 2, 2, dict(SMALL, dim=32)),
 ]
 
