@@ -691,7 +691,7 @@ typedef struct {
     uint16_t *d_o_part2;                              /* [part_rows2, dim]: of the global stage (infllm_resident_part_rows) */
     float *d_lse_part2;
     int64_t part_rows2;
-    float *d_lse;                                     /* [B,H,exc] */
+    float *d_lse;                                     /* [B,H,max_tokens] */
     float *d_logits;                                  /* [B,H,n_local] */
     float *d_call_scores;                             /* [blocks, B, scores_cols], scores_cols >= the units after the call */
     int64_t scores_cols;

@@ -500,7 +500,7 @@ class ContextManager:
                            qpart=torch.empty((B * ((T + 15) // 16) * H * D,), **f32), qbar=torch.empty((blocks * B * H * D,), **f32),
                            o_part=torch.empty((part_rows * D,), **f16), lse_part=torch.empty((part_rows,), **f32),
                            o_part2=torch.empty((self._part_rows2 * D,), **f16), lse_part2=torch.empty((self._part_rows2,), **f32),
-                           lse=torch.empty((B * H * exc,), **f32), logits=torch.empty((B * H * self.n_local,), **f32),
+                           lse=torch.empty((B * H * max(T, exc),), **f32), logits=torch.empty((B * H * self.n_local,), **f32),
                            base=torch.empty((blocks * B * self.topk,), dtype=torch.int32, device=self.device))
             _CALL_BUFFERS[key] = buf
         self._call_buf = buf

@@ -648,6 +648,18 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
 template <int D>
 __global__ __launch_bounds__(256) void attn_merge_kernel(MergeJob job) { merge_piece<D>(job, (int64_t)blockIdx.x * 256 + threadIdx.x); }
 
+// ... of several execution blocks' partials (infllm_attn_stage_blocked), blockIdx.y one of them
+template <int D>
+__global__ __launch_bounds__(256) void attn_merge_blocked_kernel(MergeJob job, int64_t block_rows, int32_t exc, int32_t n) {
+    const int32_t q0 = (int32_t)blockIdx.y * exc;
+    job.Lq = min(exc, n - q0);
+    job.o_part += blockIdx.y * block_rows * D;
+    job.lse_part += blockIdx.y * block_rows;
+    job.out += q0 * job.o_sl;
+    job.lse_out += q0;
+    merge_piece<D>(job, (int64_t)blockIdx.x * 256 + threadIdx.x);
+}
+
 // the log-sum-exp half of the merge alone: one thread per row
 __global__ __launch_bounds__(256) void attn_merge_lse_kernel(const float *lse_part, int P, int64_t rows, float *lse_out, PartSets ps) {
     const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -1053,7 +1065,23 @@ int infllm_merge_job(const uint16_t *d_o_part, const float *d_lse_part, int32_t 
         ps.skip_l = (int64_t)(((intptr_t)d_lse_part2 - (intptr_t)d_lse_part) / (intptr_t)sizeof(float)) - (int64_t)P1 * rows_;
         ps.skip_o = (int64_t)(((intptr_t)d_o_part2 - (intptr_t)d_o_part) / 2) - (int64_t)P1 * rows_ * dim - ps.skip_l * dim;
     }
-    *job = MergeJob{(const _Float16 *)d_o_part, d_lse_part, P1 + P2, B, H, Lq, (bf16_t *)d_out, o_sb, o_sh, o_sl, d_lse, ps};
+    *job = MergeJob{(const _Float16 *)d_o_part, d_lse_part, P1 + P2, B, H, Lq, (bf16_t *)d_out, o_sb, o_sh, o_sl, d_lse, ps, Lq};
+    return 0;
+}
+
+// library-internal: the merge of the partials that infllm_attn_stage_blocked left for n queries in blocks of exc (P of them a
+// block, blocks block_rows apart), in one launch: rows of all blocks to d_out, their joint log-sum-exps [B, H, n] to d_lse
+int infllm_attn_merge_blocked(const uint16_t *d_o_part, const float *d_lse_part, int32_t P, int32_t B, int32_t H, int32_t n, int32_t exc, int64_t block_rows,
+                              void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse, void *stream, int32_t dim) {
+    INFLLM_REQUIRE(n > 0 && exc > 0 && d_out && d_lse && (n + exc - 1) / exc <= 65535, "attn_merge_blocked: bad arguments");
+    MergeJob job;
+    const int rc = infllm_merge_job(d_o_part, d_lse_part, P, nullptr, nullptr, 0, B, H, std::min(n, exc), d_out, o_sb, o_sh, o_sl, d_lse, &job, dim);
+    if (rc) return rc;
+    job.lse_sh = n;
+    const int64_t threads = (int64_t)B * H * std::min(n, exc) * (dim / 8);
+    hipLaunchKernelGGL((dim == 64 ? attn_merge_blocked_kernel<64> : attn_merge_blocked_kernel<128>), dim3((unsigned)((threads + 255) / 256), (n + exc - 1) / exc),
+                       dim3(256), 0, (hipStream_t)stream, job, block_rows, exc, n);
+    INFLLM_CHECK_LAUNCH("attn_merge_blocked");
     return 0;
 }
 

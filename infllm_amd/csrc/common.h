@@ -89,8 +89,9 @@ struct MergeJob {
     int32_t P, B, H, Lq;
     bf16_t *out;                       // rows [b, h, i] at b * o_sb + h * o_sh + i * o_sl
     int64_t o_sb, o_sh, o_sl;
-    float *lse_out;                    // [B, H, Lq] or NULL
+    float *lse_out;                    // [B, H, Lq] with head rows lse_sh apart, or NULL
     PartSets ps;
+    int32_t lse_sh;
 };
 
 // thread e of the merge: (row, 8 dims) = (e / 16, e % 16) for rows of 128 elements, (e / 8, e % 8) for rows of 64.  (inf_llm/attention/dot_production_attention/torch_impl.py:15-36)
@@ -143,7 +144,7 @@ __device__ __forceinline__ void merge_piece(const MergeJob &mj, int64_t e) {
     u32x4 packed{pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv),
                  pack_bf16x2(acc[4] * inv, acc[5] * inv), pack_bf16x2(acc[6] * inv, acc[7] * inv)};
     *(u32x4 *)(mj.out + (int64_t)b * mj.o_sb + (int64_t)h * mj.o_sh + (int64_t)i * mj.o_sl + c * 8) = packed;
-    if (c == 0 && mj.lse_out) mj.lse_out[row] = den > 0.f ? m + log2f(den) : -INFINITY;
+    if (c == 0 && mj.lse_out) mj.lse_out[(int64_t)bh * mj.lse_sh + i] = den > 0.f ? m + log2f(den) : -INFINITY;
 }
 
 

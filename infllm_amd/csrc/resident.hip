@@ -31,6 +31,8 @@ int infllm_merge_job(const uint16_t *d_o_part, const float *d_lse_part, int32_t 
 int infllm_attn_merge2(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2, const float *d_lse_part2,
                        int32_t P2, int32_t B, int32_t H, int32_t Lq, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse,
                        void *stream, int32_t dim);
+int infllm_attn_merge_blocked(const uint16_t *d_o_part, const float *d_lse_part, int32_t P, int32_t B, int32_t H, int32_t n, int32_t exc, int64_t block_rows,
+                              void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse, void *stream, int32_t dim);
 int infllm_local_score_dim(const infllm_score_args *a, int32_t dim, void *stream);
 int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream, int32_t dim);
 int infllm_local_score_merged_rank(const infllm_score_args *a, const MergeJob *job, const RankJob *rank, int32_t n_rank, void *stream, int32_t dim);
@@ -509,7 +511,22 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
     INFLLM_REQUIRE(a->part_rows / (nsplit * rows_one) >= group, "resident: partial rows do not fit");
     const int64_t block_rows = nsplit * rows_one;
 
+    // the score launch of nq queries from the call's query q0 on, which see the keys [lo, hi)
+    auto score_args = [&](int64_t q0, int nq, int64_t lo, int64_t hi) {
+        infllm_score_args sc{};
+        sc.d_q = (const bf16_t *)a->d_q_loc + q0 * row_elems;
+        sc.q_sl = D; sc.q_sh = (int64_t)n * D; sc.q_sb = (int64_t)d.H * n * D;
+        sc.B = B; sc.H = d.H; sc.Hkv = d.Hkv; sc.Lq = nq;
+        sc.d_k = d.d_ring_k_rot;
+        sc.k_sl = D; sc.k_sh = d.ring_cap * D; sc.k_sb = d.Hkv * d.ring_cap * D;
+        sc.cap = d.ring_cap; sc.j_lo = lo; sc.j_hi = hi;
+        sc.mask = INFLLM_MASK_WINDOW; sc.accumulate = 1; sc.offset = call_b0 + q0; sc.window = d.n_local;
+        sc.d_lse = a->d_lse; sc.softmax_scale = d.softmax_scale;
+        sc.d_score = d.d_ring_score; sc.score_sh = d.ring_cap; sc.score_sb = d.H * d.ring_cap; sc.score_cap = d.ring_cap;
+        return sc;
+    };
     int32_t j_done = -1;                          // the block whose page table is on the device
+    int plain_end = 0;                            // blocks in front of this one are done
     for (int i = 0; i < n_blocks; ++i) {
         const int nb = std::min(exc, n - i * exc);
         const int64_t b0 = call_b0 + (int64_t)i * exc, b1 = b0 + nb, lo = std::max<int64_t>(0, b0 - d.n_local);
@@ -558,6 +575,31 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             jb.pages = pl;
             rc = launch_rank(R, jb, 1, st);
             if (rc) return rc;
+            // Blocks that read nothing but the window and from which nothing leaves (a stream's first n_local tokens) have no
+            // chain from one to the next: their partials are merged and their scores taken in one launch each for all of them
+            // (eight blocks: 16 launches of some 20 us; 4,096 queries at once keep the chip full).
+            int m = 0;
+            for (; i + m < std::min(n_blocks, i + group); ++m) {
+                const int64_t e1 = call_b0 + std::min((i + m + 1) * exc, n);
+                const Carve c = carve_after(d, R->cursor, R->init_len, e1);
+                if (c.take || c.count || page_list(R, a, std::min(N, d.topk), e1).n_pages) break;
+            }
+            if (m >= 2) {
+                const int q0 = i * exc, nq = std::min(m * exc, n - q0);
+                rc = infllm_attn_merge_blocked(a->d_o_part, a->d_lse_part, nsplit, B, d.H, nq, exc, block_rows, (bf16_t *)a->d_out + (st0 + q0) * a->o_sl, a->o_sb,
+                                               a->o_sh, a->o_sl, a->d_lse, st, D);
+                if (rc) return rc;
+                const infllm_score_args sc = score_args(q0, nq, lo, b0 + nq);
+                rc = infllm_local_score_dim(&sc, D, st);
+                if (rc) return rc;
+                plain_end = i + m;
+            }
+        }
+        if (i < plain_end) {
+            R->queue.push_back(Resident::Entry{0, 0, 0});
+            R->length = b1;
+            ++R->blocks;
+            continue;
         }
         int parts = nsplit, ns_g = 0;
         if (pl.n_pages > 0) {
@@ -587,16 +629,7 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
         rc = infllm_merge_job(o_loc, lse_loc, nsplit, ns_g ? a->d_o_part2 : nullptr, ns_g ? a->d_lse_part2 : nullptr, ns_g, B, d.H, nb, out, a->o_sb, a->o_sh,
                               a->o_sl, a->d_lse, &job, D);
         if (rc) return rc;
-        infllm_score_args sc{};
-        sc.d_q = (const bf16_t *)a->d_q_loc + (int64_t)i * exc * row_elems;
-        sc.q_sl = D; sc.q_sh = (int64_t)n * D; sc.q_sb = (int64_t)d.H * n * D;
-        sc.B = B; sc.H = d.H; sc.Hkv = d.Hkv; sc.Lq = nb;
-        sc.d_k = d.d_ring_k_rot;
-        sc.k_sl = D; sc.k_sh = d.ring_cap * D; sc.k_sb = d.Hkv * d.ring_cap * D;
-        sc.cap = d.ring_cap; sc.j_lo = lo; sc.j_hi = b1;
-        sc.mask = INFLLM_MASK_WINDOW; sc.accumulate = 1; sc.offset = b0; sc.window = d.n_local;
-        sc.d_lse = a->d_lse; sc.softmax_scale = d.softmax_scale;
-        sc.d_score = d.d_ring_score; sc.score_sh = d.ring_cap; sc.score_sb = d.H * d.ring_cap; sc.score_cap = d.ring_cap;
+        infllm_score_args sc = score_args((int64_t)i * exc, nb, lo, b1);
         // What the next block waits for comes first where there is a kernel for it - the scores and representatives of the units
         // that leave the window now, in one launch that merges the block's partials along the way -, then the rest of the scores,
         // with the ranking riding along.

@@ -84,8 +84,12 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(
     // Workgroups are dispatched x fastest: all heads of one key tile, then the next tile.  The two tiles at either end
     // of a masked key range see only part of the queries and finish early, so they go last: when the grid is a little
     // more than what the chip holds at once, the workgroups that start late are then the short ones.
+    // Where the queries are (nearly) as many as the keys, a tile's work falls from the first to the last instead: a CU that
+    // takes one of the first half and one of the second gets a long and a short one.
     int tile = slot;
-    if (n_tiles >= 6 && a.mask != INFLLM_MASK_NONE)
+    if (a.mask == INFLLM_MASK_WINDOW && a.Lq >= (a.j_hi - a.j_lo) - (a.j_hi - a.j_lo) / 4)
+        tile = slot < (n_tiles + 1) / 2 ? slot : n_tiles - 1 - (slot - (n_tiles + 1) / 2);
+    else if (n_tiles >= 6 && a.mask != INFLLM_MASK_NONE)
         tile = slot < n_tiles - 4 ? slot + 2 : slot == n_tiles - 4 ? 1 : slot == n_tiles - 3 ? n_tiles - 2 : slot == n_tiles - 2 ? 0 : n_tiles - 1;
     const int64_t jg = (a.j_lo / kWaveKeys + (int64_t)tile * 4) * kWaveKeys;         // first key of the workgroup
     const int64_t j0 = jg + (int64_t)wave * kWaveKeys;                               // first key of this wave

@@ -11,6 +11,8 @@ CASES = [
     # calls that begin inside the window, blocks that end on and off a unit, the first selection over exactly topk units, calls
     # of one token (a step) with and without a unit carved behind it
     ("small", [300, 1, 1, 700, 64, 1, 33], 8, 2, 2, dict(SMALL)),
+    # calls whose blocks read nothing but the window, the last one short: merged and scored together
+    ("inside the window", [200, 47, 900], 8, 2, 2, dict(SMALL, n_local=512)),
     ("fifo, tight cache", [1300, 40, 1, 500], 8, 2, 1, dict(SMALL, max_cached_block=4, cache_strategy="fifo")),
     ("steps", [420] + [1] * 70, 8, 2, 1, dict(SMALL)),
     ("no GQA, perhead", [500, 1, 200], 4, 2, 1, dict(SMALL, perhead=True)),
