@@ -48,8 +48,6 @@ int infllm_gather_rows_pair(const void *d_ring_a, void *d_out_a, const void *d_r
                             void *stream, int32_t dim);
 int infllm_retrieve_fused(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar, int32_t k, float *d_scores,
                           int32_t *d_idx, int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, void *stream);
-int infllm_topk_publish_pair(const float *d_scores, int32_t N, int32_t k, int32_t *d_idx, int32_t *d_idx2, int32_t *d_flag,
-                             int32_t flag_value, void *stream);
 int infllm_key_splits(const infllm_layer_desc *d, int32_t n_queries, int32_t n_tiles);
 
 namespace {
@@ -67,7 +65,11 @@ __global__ __launch_bounds__(256) void pages_kernel(PageList j, const int32_t *i
 }
 
 // The end of a decode step: output rows = the joined splits; the window's score track += the probabilities, from the
-// logits that the attention launch left behind.  grid (B * H, 1 + ceil(window / 1024)): y == 0 joins, the others score.
+// logits that the attention launch left behind; and the step's selection on its way to the host's log, whose write across
+// the bus then runs beside the rest instead of behind the retrieval (which ended 3 us earlier without it).
+// grid (B * H, 1 + ceil(window / 1024)): y == 0 joins, the others score.  A handful of loads per thread and nothing else, so
+// all of them are requested before the first is waited for (32 heads, 64 splits: 11.4 -> 6 us with the splits' rows as
+// 16-byte pieces, one batch instead of a chain of four).
 struct FinishJob {
     const _Float16 *o_part;
     const float *lse_part;
@@ -77,65 +79,89 @@ struct FinishJob {
     const float *logits;                   // [B, H, logit_stride]
     int64_t logit_stride;
     float *score;                          // [B, H, ring_cap]
-    int64_t ring_cap, j_lo;
+    int32_t ring_cap, slot0;               // ring row of the window's first key
     int32_t n;                             // keys of the window
+    const int32_t *ids;                    // the selection [n_ids] and its log slot, a sequence number behind them; log NULL: none
+    int32_t *log;
+    int32_t n_ids, seq;
 };
 
 template <int D>
 __global__ __launch_bounds__(256) void decode_finish_kernel(FinishJob j) {
-    __shared__ float w_sh[128];
-    __shared__ float part[256 / D][D];
+    constexpr int kPieces = D / 8, kGroups = 256 / kPieces, kMaxParts = 64, kMine = kMaxParts / kGroups;
+    __shared__ float w_sh[kMaxParts];
+    __shared__ __attribute__((aligned(16))) float part[kGroups][D];
     const int tid = threadIdx.x, lane = tid & 63, rh = blockIdx.x;
     const int64_t rows = (int64_t)j.B * j.H;
-    constexpr int kPer = 4;
-    float x[kPer] = {0.f, 0.f, 0.f, 0.f};
-    const int y0 = ((int)blockIdx.y - 1) * 1024;
+    const float l0 = lane < j.P ? j.lse_part[lane * rows + rh] : -INFINITY;
+    // joint log-sum-exp: every wave for itself
+    float e0 = 0.f, m = 0.f, den = 0.f;
+    auto join = [&]() {
+        m = l0;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+        e0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(l0 - m);
+        den = e0;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) den += __shfl_xor(den, o, 64);
+    };
     if (blockIdx.y > 0) {
-#pragma unroll
-        for (int i = 0; i < kPer; ++i)
-            if (y0 + i * 256 + tid < j.n) x[i] = j.logits[(int64_t)rh * j.logit_stride + y0 + i * 256 + tid];
-    }
-    // joint log-sum-exp: every wave for itself (P <= 128)
-    const float l0 = lane < j.P ? j.lse_part[lane * rows + rh] : -INFINITY, l1 = lane + 64 < j.P ? j.lse_part[(lane + 64) * rows + rh] : -INFINITY;
-    float m = fmaxf(l0, l1);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-    const float e0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(l0 - m), e1 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(l1 - m);
-    float den = e0 + e1;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) den += __shfl_xor(den, o, 64);
-    if (blockIdx.y > 0) {
-        const float lse = den > 0.f ? m + log2f(den) : INFINITY;
+        constexpr int kPer = 4;
+        const int y0 = ((int)blockIdx.y - 1) * 1024;
+        const float *logit = j.logits + (int64_t)rh * j.logit_stride;
         float *score = j.score + (int64_t)rh * j.ring_cap;
+        float x[kPer], old[kPer];
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const int k = y0 + i * 256 + tid;
-            if (k < j.n) score[(j.j_lo + k) % j.ring_cap] += __builtin_amdgcn_exp2f(x[i] - lse);
+            if (k >= j.n) continue;
+            const int at = j.slot0 + k;
+            x[i] = logit[k];
+            old[i] = score[at < j.ring_cap ? at : at - j.ring_cap];
+        }
+        join();
+        const float lse = den > 0.f ? m + log2f(den) : INFINITY;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int k = y0 + i * 256 + tid, at = j.slot0 + k;
+            if (k < j.n) score[at < j.ring_cap ? at : at - j.ring_cap] = old[i] + __builtin_amdgcn_exp2f(x[i] - lse);
         }
         return;
     }
-    if (tid < 64) w_sh[lane] = e0, w_sh[lane + 64] = e1;
-    __syncthreads();
-    const int d = tid % D, q = tid / D;
-    float acc = 0.f;
-    for (int p0 = q; p0 < j.P; p0 += 8 * (256 / D)) {
-        float o[8];
+    const int c = tid % kPieces, q = tid / kPieces;
+    f16x8 o[kMine];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int p = p0 + i * (256 / D);
-            o[i] = p < j.P ? (float)j.o_part[((int64_t)p * rows + rh) * D + d] * w_sh[p] : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc += o[i];
+    for (int i = 0; i < kMine; ++i) {
+        const int p = q + i * kGroups;
+        o[i] = p < j.P ? *(const f16x8 *)(j.o_part + ((int64_t)p * rows + rh) * D + c * 8) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
-    part[q][d] = acc;
+    const bool logs = rh == 0 && j.log;
+    if (logs)
+        for (int i = tid; i < j.n_ids; i += 256) j.log[i] = j.ids[i];
+    join();
+    if (tid < 64) w_sh[lane] = e0;
+    __syncthreads();
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kMine; ++i) {
+        const float w = w_sh[q + i * kGroups];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += (float)o[i][e] * w;
+    }
+    *(f32x4 *)&part[q][c * 8] = f32x4{acc[0], acc[1], acc[2], acc[3]};
+    *(f32x4 *)&part[q][c * 8 + 4] = f32x4{acc[4], acc[5], acc[6], acc[7]};
     __syncthreads();
     if (tid < D / 2) {
         float lo = 0.f, hi = 0.f;
 #pragma unroll
-        for (int i = 0; i < 256 / D; ++i) lo += part[i][2 * tid], hi += part[i][2 * tid + 1];
+        for (int i = 0; i < kGroups; ++i) lo += part[i][2 * tid], hi += part[i][2 * tid + 1];
         const float inv = den > 0.f ? 1.f / den : 0.f;
         *(uint32_t *)(j.out + (int64_t)(rh / j.H) * j.o_sb + (int64_t)(rh % j.H) * j.o_sh + tid * 2) = pack_bf16x2(lo * inv, hi * inv);
+    }
+    if (logs) {
+        __threadfence_system();
+        __syncthreads();
+        if (tid == 0) __hip_atomic_store(j.log + j.n_ids, j.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -362,22 +388,22 @@ int decode_step(Resident *R, const infllm_resident_call *a, int64_t st0, hipStre
     if (rc) return rc;
     const int n_sel = std::min(N, d.topk);
     const int32_t *ids = d.d_iota;
+    FinishJob f{};
     if (retrieve) {
-        int32_t slot = 0, seq = 0;
-        rc = take_slot(R, &slot, &seq);
+        int32_t slot = 0;
+        rc = take_slot(R, &slot, &f.seq);
         if (rc) return rc;
-        const int stride = B * d.topk + 1;
-        int32_t *log = d.d_log + (int64_t)slot * stride;
+        f.log = d.d_log + (int64_t)slot * (B * d.topk + 1);
+        f.ids = d.d_ids; f.n_ids = B * d.topk;
         ids = d.d_ids;
         for (int u = 0; u < B; ++u) {
             const bf16_t *reps = (const bf16_t *)a->d_reps + (int64_t)u * a->rep_sb;
             float *scores = a->d_unit_scores + (int64_t)u * a->unit_scores_sb;
             const float *qbar = a->d_qbar + (int64_t)u * C;
-            int32_t *flag = u == B - 1 ? log + stride - 1 : nullptr;
-            rc = infllm_retrieve_fused(reps, a->rep_su, N, C, qbar, d.topk, scores, d.d_ids + (int64_t)u * d.topk, log + (int64_t)u * d.topk, flag, seq, st);
+            rc = infllm_retrieve_fused(reps, a->rep_su, N, C, qbar, d.topk, scores, d.d_ids + (int64_t)u * d.topk, nullptr, nullptr, 0, st);
             if (rc == 1) {
                 rc = infllm_unit_scores(reps, a->rep_su, 0, N, C, qbar, scores, st);
-                if (!rc) rc = infllm_topk_publish_pair(scores, N, d.topk, d.d_ids + (int64_t)u * d.topk, log + (int64_t)u * d.topk, flag, seq, st);
+                if (!rc) rc = infllm_topk(scores, N, d.topk, d.d_ids + (int64_t)u * d.topk, st);
             }
             if (rc) return rc;
         }
@@ -421,12 +447,11 @@ int decode_step(Resident *R, const infllm_resident_call *a, int64_t st0, hipStre
     j.logits = a->d_logits; j.logit_stride = d.n_local;
     rc = infllm_decode_attn(&j, d.dim, st);
     if (rc) return rc;
-    FinishJob f{};
     f.o_part = (const _Float16 *)a->d_o_part; f.lse_part = a->d_lse_part;
     f.P = j.nsplit; f.B = B; f.H = d.H;
     f.out = (bf16_t *)a->d_out + st0 * a->o_sl; f.o_sb = a->o_sb; f.o_sh = a->o_sh;
     f.logits = a->d_logits; f.logit_stride = d.n_local;
-    f.score = d.d_ring_score; f.ring_cap = d.ring_cap; f.j_lo = j_lo; f.n = (int32_t)(b1 - j_lo);
+    f.score = d.d_ring_score; f.ring_cap = (int32_t)d.ring_cap; f.slot0 = (int32_t)(j_lo % d.ring_cap); f.n = (int32_t)(b1 - j_lo);
     const dim3 grid(B * d.H, 1 + (f.n + 1023) / 1024);
     if (d.dim == 128) hipLaunchKernelGGL(decode_finish_kernel<128>, grid, dim3(256), 0, st, f);
     else hipLaunchKernelGGL(decode_finish_kernel<64>, grid, dim3(256), 0, st, f);
@@ -550,31 +575,6 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             rc = infllm_attn_stage_blocked(&at, exc, block_rows, st, D);
             timer_end(R, 0, ti, st);
             if (rc) return rc;
-        }
-        const uint16_t *o_loc = a->d_o_part + (int64_t)(i % group) * block_rows * D;
-        const float *lse_loc = a->d_lse_part + (int64_t)(i % group) * block_rows;
-
-        // ---- the block's page table and global stage
-        const int n_sel = std::min(N, d.topk);
-        const PageList pl = page_list(R, a, n_sel, b1);
-        INFLLM_REQUIRE(pl.n_pages <= d.max_pages, "resident: %d pages exceed the table (%d)", pl.n_pages, d.max_pages);
-        const bool all_units = N <= d.topk;
-        if (all_units) R->queue.push_back(Resident::Entry{N, 0, 0});
-        if (all_units && pl.n_pages > 0) {
-            hipLaunchKernelGGL(pages_kernel, dim3((pl.n_pages + 255) / 256, B), dim3(256), 0, st, pl, d.d_iota, 0);
-            INFLLM_CHECK_LAUNCH("pages");
-        } else if (!all_units && j_done != i) {                   // the call's first block (the others' tables came with the previous block)
-            int32_t slot = 0, seq = 0;
-            rc = take_slot(R, &slot, &seq);
-            if (rc) return rc;
-            RankJob jb{};
-            jb.reps = (const bf16_t *)a->d_reps; jb.rep_sb = a->rep_sb; jb.rep_su = a->rep_su;
-            jb.qbars = a->d_qbar; jb.scores = a->d_call_scores; jb.cols = a->scores_cols; jb.base = a->d_base;
-            jb.B = B; jb.C = C; jb.k = d.topk; jb.n_list = n_list; jb.n_base = n0; jb.first_new = N; jb.n_new = 0; jb.j0 = jb.j_sel = i;
-            jb.log = d.d_log + (int64_t)slot * (B * d.topk + 1); jb.seq = seq;
-            jb.pages = pl;
-            rc = launch_rank(R, jb, 1, st);
-            if (rc) return rc;
             // Blocks that read nothing but the window and from which nothing leaves (a stream's first n_local tokens) have no
             // chain from one to the next: their partials are merged and their scores taken in one launch each for all of them
             // (eight blocks: 16 launches of some 20 us; 4,096 queries at once keep the chip full).
@@ -600,6 +600,31 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             R->length = b1;
             ++R->blocks;
             continue;
+        }
+        const uint16_t *o_loc = a->d_o_part + (int64_t)(i % group) * block_rows * D;
+        const float *lse_loc = a->d_lse_part + (int64_t)(i % group) * block_rows;
+
+        // ---- the block's page table and global stage
+        const int n_sel = std::min(N, d.topk);
+        const PageList pl = page_list(R, a, n_sel, b1);
+        INFLLM_REQUIRE(pl.n_pages <= d.max_pages, "resident: %d pages exceed the table (%d)", pl.n_pages, d.max_pages);
+        const bool all_units = N <= d.topk;
+        if (all_units) R->queue.push_back(Resident::Entry{N, 0, 0});
+        if (all_units && pl.n_pages > 0) {
+            hipLaunchKernelGGL(pages_kernel, dim3((pl.n_pages + 255) / 256, B), dim3(256), 0, st, pl, d.d_iota, 0);
+            INFLLM_CHECK_LAUNCH("pages");
+        } else if (!all_units && j_done != i) {                   // the call's first block (the others' tables came with the previous block)
+            int32_t slot = 0, seq = 0;
+            rc = take_slot(R, &slot, &seq);
+            if (rc) return rc;
+            RankJob jb{};
+            jb.reps = (const bf16_t *)a->d_reps; jb.rep_sb = a->rep_sb; jb.rep_su = a->rep_su;
+            jb.qbars = a->d_qbar; jb.scores = a->d_call_scores; jb.cols = a->scores_cols; jb.base = a->d_base;
+            jb.B = B; jb.C = C; jb.k = d.topk; jb.n_list = n_list; jb.n_base = n0; jb.first_new = N; jb.n_new = 0; jb.j0 = jb.j_sel = i;
+            jb.log = d.d_log + (int64_t)slot * (B * d.topk + 1); jb.seq = seq;
+            jb.pages = pl;
+            rc = launch_rank(R, jb, 1, st);
+            if (rc) return rc;
         }
         int parts = nsplit, ns_g = 0;
         if (pl.n_pages > 0) {
