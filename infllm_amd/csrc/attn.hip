@@ -424,23 +424,24 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             d0 = (int)min(max(e0, (int64_t)-kBig), (int64_t)kBig) + col;
         }
         if (need_mask) {
-            const int win = (int)min(MODE == kSinks && paged ? ap.window : a.window, (int64_t)2 * kBig);
-            const int lo_l = row_lo - 8 * grp, hi_l = row_hi - 8 * grp;      // bounds on kc for this lane
-            const int dl = d0 - 8 * grp;                                       // dist = dl - kc
+            // Whatever the mask, a lane's query sees ONE run of the tile's keys: its bounds are found once, and a key costs a
+            // subtraction and a compare (a mask's conditions key by key: 150 branches in the sinks' form of the kernel).
+            // dist = dl - kc; kc is the compile-time part of register r's key, which is kc + 8 * grp
+            const int win = (int)min(MODE == kSinks && paged ? ap.window : a.window, (int64_t)2 * kBig), dl = d0 - 8 * grp;
+            int lo_l = row_lo - 8 * grp, hi_l = row_hi - 8 * grp;
+            if (MODE == kSinks && paged) {
+                hi_l = min(hi_l, dl - win + 1);
+            } else if (!paged) {
+                if (a.mask == INFLLM_MASK_WINDOW) lo_l = max(lo_l, dl - win + 1), hi_l = min(hi_l, dl + 1);
+                if (a.mask == INFLLM_MASK_COMPLEMENT) hi_l = min(hi_l, dl - win + 1);
+            }
+            const uint32_t n_l = (uint32_t)max(hi_l - lo_l, 0);
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    // key of register r: ko = kc + 8*grp with the compile-time part kc; everything is
-                    // expressed relative to the per-lane bases so that no per-register value is kept
                     const int kc = ks * 32 + 16 * (r >> 3) + (r & 7);
-                    bool vis = (kc >= lo_l) && (kc < hi_l);
-                    if (!paged) {
-                        if (a.mask == INFLLM_MASK_WINDOW) vis = vis && (kc <= dl) && (kc > dl - win);
-                        if (a.mask == INFLLM_MASK_COMPLEMENT) vis = vis && (kc <= dl - win);
-                    } else if (MODE == kSinks) {
-                        vis = vis && (kc <= dl - win);
-                    }
+                    const bool vis = MODE == kPaged ? kc < hi_l : (uint32_t)(kc - lo_l) < n_l;      // (a page begins with its rows)
                     s[ks][r] = vis ? s[ks][r] : -INFINITY;
                 }
         }
