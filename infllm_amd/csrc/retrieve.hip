@@ -438,7 +438,7 @@ static __device__ unsigned int retrieval_tickets[kTicketSlots];       // zero at
 template <int NB>
 __device__ __forceinline__ void select_topk_block(const float *scores, int N, int k, int32_t *idx_out, int32_t *idx_out2) {
     __shared__ uint64_t surv[kSurvivorCap + 8];
-    __shared__ __align__(16) uint32_t gmax[64];
+    __shared__ uint32_t gmax[kRetrThreads / 64][64];
     __shared__ int wave_cnt[kRetrThreads / 64];
     __shared__ int s_count;
     constexpr int R = NB * 16;                                   // 16 loads in flight per thread and round trip
@@ -463,23 +463,26 @@ __device__ __forceinline__ void select_topk_block(const float *scores, int N, in
     }
     auto composite = [&](int j) { return ((uint64_t)key[j] << 32) | (uint32_t)(0xffffffffu - (uint32_t)(tid + j * kRetrThreads)); };
     if (tid == 0) s_count = 0;
-    if (tid < 64) gmax[tid] = 0xffffffffu;
-    __syncthreads();
-    // groups of 32, 16 or 8 lanes: 16, 32 or 64 groups; the threshold is on the score's key alone (units that tie with
-    // it all pass, and are told apart by the composites afterwards)
-    const int width = k <= 16 ? 32 : k <= 32 ? 16 : 8;
-    for (int o = 1; o < width; o <<= 1) {
+    // 16, 32 or 64 groups: the threads whose number is the same modulo that, so that all of them have units however few there
+    // are (479 units, 16 best: groups of neighbours left one empty, every unit passed the threshold, and ranking them by
+    // counting made the launch 17.7 us instead of 11).  The threshold is on the score's key alone: units that tie with it all
+    // pass, and are told apart by the composites afterwards.
+    const int groups = k <= 16 ? 16 : k <= 32 ? 32 : 64;
+    for (int o = 32; o >= groups; o >>= 1) {
         const uint32_t other = __shfl_xor(best, o, 64);
         best = other > best ? other : best;
     }
-    if ((lane & (width - 1)) == 0) gmax[tid / width] = best;
+    gmax[wave][lane] = best;                                     // lane: its group's maximum, lane mod groups
     __syncthreads();
-    uint32_t tau = 0xffffffffu;
+    uint32_t tau = 0;
 #pragma unroll
-    for (int g = 0; g < 64; g += 4) {
-        const u32x4 m = *(const u32x4 *)(gmax + g);
-        tau = min(min(tau, m[0]), min(m[1], min(m[2], m[3])));
-    }
+    for (int w = 0; w < kRetrThreads / 64; ++w) tau = max(tau, gmax[w][lane]);
+    // the smallest of them: rows of 16 lanes by rotation, which is the whole of it when the rows are copies of each other
+    tau = min(tau, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)tau, 0x121, 0xf, 0xf, false));
+    tau = min(tau, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)tau, 0x122, 0xf, 0xf, false));
+    tau = min(tau, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)tau, 0x124, 0xf, 0xf, false));
+    tau = min(tau, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)tau, 0x128, 0xf, 0xf, false));
+    for (int o = 16; o < groups; o <<= 1) tau = min(tau, (uint32_t)__shfl_xor(tau, o, 64));
     auto collect = [&](uint64_t thr) {                           // composites >= thr into surv[]; s_count = how many there are
 #pragma unroll
         for (int j = 0; j < R; ++j) {

@@ -459,7 +459,9 @@ def test_topk_on_heavily_tied_scores_is_the_stable_descending_prefix(N, k, level
 
 
 @pytest.mark.parametrize("N,k,pattern", [(6000, 16, "levels"), (16384, 16, "one_group"), (16384, 64, "one_group"), (9000, 16, "falling"),
-                                         (9000, 40, "rising"), (8192, 33, "constant"), (700, 64, "levels"), (16, 16, "falling")])
+                                         (9000, 40, "rising"), (8192, 33, "constant"), (700, 64, "levels"), (16, 16, "falling"),
+                                         # thread groups by the unit's number: few units in each, one unit in some, the best of all in one
+                                         (16384, 16, "one_residue"), (479, 16, "falling"), (300, 32, "rising"), (511, 64, "levels"), (70, 64, "falling")])
 def test_scores_and_selection_in_one_launch_give_the_stable_descending_prefix(N, k, pattern):
     """infllm_score_topk where scoring and selection are ONE launch (rows of 512 elements, k <= 64, N <= 16384), on
     scores made to be exact in fp32 (score = 256 * column 0 + column 1 of small integers): few distinct values, scores
@@ -477,6 +479,8 @@ def test_scores_and_selection_in_one_launch_give_the_stable_descending_prefix(N,
         val = n
     elif pattern == "constant":
         val = torch.full((N,), 7)
+    elif pattern == "one_residue":
+        val = torch.where(n % 16 == 5, 1000 + torch.randint(0, 50, (N,), generator=g), torch.randint(0, 900, (N,), generator=g))
     else:
         val = torch.where(n % 512 < 32, 1000 + torch.randint(0, 50, (N,), generator=g), torch.randint(0, 900, (N,), generator=g))
     reps = torch.zeros((N, 512), dtype=torch.bfloat16)
