@@ -55,8 +55,11 @@ class _Room:
 
 def _rows16(t):
     """rows the kernels can read: unit stride inside a row, 16-byte alignment"""
-    s = t.stride()
-    return t if s[-1] == 1 and not any(x % 8 for x in s[:-1]) and t.data_ptr() % 16 == 0 else t.contiguous()
+    *outer, inner = t.stride()
+    odd = 0
+    for s in outer:
+        odd |= s
+    return t if inner == 1 and not odd & 7 and not t.data_ptr() & 15 else t.contiguous()
 
 
 def _cache_rows(t):

@@ -44,7 +44,7 @@ import torch
 
 from .. import _lib
 from .._lib import BackArgs, FrontArgs, LayerDesc, ResidentCall, ResidentDesc, check
-from ..ops import HEAD_DIM, KEY_TILE
+from ..ops import HEAD_DIM, KEY_TILE, current_stream
 
 from ._rows import check_head_dim, narrow as _narrow, wide_inv_freq, widen as _widen
 
@@ -458,7 +458,7 @@ class ContextManager:
             return None
         if units > self.reps.shape[1]:
             self._grow_reps(units)
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = current_stream()
         if self._call_stream != stream:
             self._bind_resident_buffers(stream)
         if n > 1 and units > self.topk and (self._call_scores is None or self._call_scores.shape[2] < units):
@@ -933,9 +933,10 @@ class ContextManager:
         if q.dtype != torch.bfloat16:
             raise TypeError(f"the HIP path computes in bfloat16; got {q.dtype}")
         assert q.dim() == 4 and q.is_cuda
-        batch_size, input_length = q.size(0), q.size(-2)
-        for t in (q, k, v):
-            assert t.size(0) == batch_size and t.size(2) == input_length and t.size(3) == q.size(3)
+        batch_size, _, input_length, width = q.shape
+        for t in (k, v):
+            t0, _, t2, t3 = t.shape
+            assert t0 == batch_size and t2 == input_length and t3 == width
         if self.perhead:                                        # context_manager.py:690-704
             heads, heads_kv = q.size(1), k.size(1)
             rep = lambda t: (t.reshape(batch_size, heads_kv, 1, input_length, -1)
@@ -956,8 +957,8 @@ class ContextManager:
         assert q.shape[:2] == (self.num_units, self.unit_size) and k.shape[1] == self.unit_size_kv
 
         def rows16(t):          # rows must be contiguous and 16-byte aligned for the vector loads
-            ok = t.stride(-1) == 1 and not any(s % 8 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0
-            return t if ok else t.contiguous()
+            s0, s1, s2, s3 = t.stride()
+            return t if s3 == 1 and not (s0 | s1 | s2) & 7 and not t.data_ptr() & 15 else t.contiguous()
         q, k, v = rows16(q), rows16(k), rows16(v)
         if self._resident:
             out = self._append_resident(q, k, v, input_length)
