@@ -890,7 +890,7 @@ extern "C" int infllm_attn_stage(const infllm_attn_args *a, void *stream) {
     return launch_stage(kLinear, a, nullptr, stream);
 }
 
-int infllm_attn_splits(int64_t wgs, int64_t tiles, int32_t max_parts);
+int infllm_attn_splits(int64_t wgs, int64_t tiles, int32_t max_parts, double mean_tiles);
 extern "C" int infllm_attn_stage_splits(const infllm_attn_args *a, int32_t max_splits) {
     INFLLM_REQUIRE(a && a->B > 0 && a->H > 0 && a->Hkv > 0 && a->H % a->Hkv == 0 && a->Lq > 0 && max_splits >= 1, "attn_stage_splits: bad arguments");
     int64_t keys = a->d_pages ? (int64_t)a->n_pages * kTile : a->j_hi - a->j_lo;
@@ -898,7 +898,8 @@ extern "C" int infllm_attn_stage_splits(const infllm_attn_args *a, int32_t max_s
     keys = std::max<int64_t>(keys, 1);
     if (a->Lq == 1 && !a->d_pages) return infllm_decode_splits(a->B, a->H, a->Hkv, (keys + kDecodeBlock - 1) / kDecodeBlock, std::min(max_splits, 64));
     const int64_t wgs = ((int64_t)((a->Lq + kQTile - 1) / kQTile) * (a->H / a->Hkv) + kWaves - 1) / kWaves * a->Hkv * a->B;
-    return infllm_attn_splits(wgs, (keys + kTile - 1) / kTile, std::min(max_splits, 64));
+    const int64_t tiles = (keys + kTile - 1) / kTile;
+    return infllm_attn_splits(wgs, tiles, std::min(max_splits, 64), (double)tiles);
 }
 
 // library-internal: a linear stage over the queries of several consecutive execution blocks of `exc` rows (the last

@@ -117,3 +117,18 @@ def test_rope_rows_matches_fp64_rotation(pos0, consecutive):
     assert float((got - want).abs().max()) <= 2 ** -7 * float(want.abs().max())      # one bf16 rounding
     empty = ops.rope_rows(x[:, :, :0], rope.inv_freq.float().cuda(), 1.0, 0)
     assert empty.shape == (B, H, 0, D)
+
+
+@pytest.mark.parametrize("kind,T,H,Hkv", [("origin", 1500, 32, 8), ("origin", 2048, 32, 8), ("origin", 705, 12, 4), ("infinite-lm", 1100, 32, 8)])
+def test_key_splits_of_a_prompts_first_call_follow_the_oracle(kind, T, H, Hkv):
+    """A prompt whose longest rows decide how many key splits its first call is cut into (bounds of this file: bf16 outputs)."""
+    from infllm_amd.attention import ATTN_FORWRAD
+    xq, xk, xv = _stream(T, H, Hkv, seed=T)
+    heads = _heads(xq, H), _heads(xk, Hkv), _heads(xv, Hkv)
+    if kind == "origin":
+        got, _ = _drive(ATTN_FORWRAD[kind](False), xq, xk, xv, [T], H, Hkv, 1e4)
+        want = CausalOracle(RopeOracle(D, base=1e4)).append(*heads)
+    else:
+        got, _ = _drive(ATTN_FORWRAD[kind](1024, 64, fattn=False), xq, xk, xv, [T], H, Hkv, 1e4)
+        want = SinkWindowOracle(RopeOracle(D, base=1e4), 1024, 64, kind).append(*heads)
+    _check(got, want)
