@@ -70,7 +70,7 @@ def _cache_rows(t):
 
 def _heads(x, batch, length, heads, dim):
     """(tensor that is kept alive, batch, head and row strides) of projected rows [batch, length, heads * dim]"""
-    if x.dim() != 3 or x.size(2) != heads * dim:
+    if x.shape != (batch, length, heads * dim):
         x = x.view(batch, length, heads * dim)
     x = _rows16(x)
     return x, x.stride(0), dim, x.stride(1)
@@ -81,15 +81,41 @@ def _wide_heads(x, batch, length, heads, dim):
     return x, x.stride(0), x.stride(2), x.stride(1)
 
 
+def _check_rows(x, device):
+    """projected rows: the native call takes them by address and reads bfloat16 on the GPU"""
+    if x.dtype != torch.bfloat16:
+        raise TypeError(f"the HIP attention path computes in bfloat16, got {x.dtype}")
+    if x.device != device or not _on_gpu(x):
+        raise ValueError(f"q, k and v must be on one GPU, got {x.device} beside {device}")
+
+
+def _on_gpu(x):
+    return x.is_cuda
+
+
+def _check_cached(old_k, old_v, raw, batch, heads, dim, device):
+    """A cache that the call's rows can join.  The native call takes addresses and strides and cannot see how far a tensor
+    reaches, so whatever joining the tensors would refuse - another batch, head count, width, type or device - is refused here."""
+    for name, t in (("keys", old_k), ("values", old_v), ("un-rotated sinks", raw)):
+        if t is None and name == "un-rotated sinks":
+            continue
+        shape = (batch, heads, t.size(2) if t.dim() == 4 else -1, dim)
+        if t.shape != shape:
+            raise ValueError(f"cached {name} {tuple(t.shape)} do not fit a call of batch {batch}, {heads} kv heads of {dim}")
+        if t.dtype != torch.bfloat16 or t.device != device:
+            raise ValueError(f"cached {name} must be bfloat16 on {device}, got {t.dtype} on {t.device}")
+    if old_v.size(2) != old_k.size(2):
+        raise ValueError(f"the cache holds {old_k.size(2)} keys and {old_v.size(2)} values")
+
+
 def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_q, project_k, project_v, dim_head, num_heads, num_heads_kv):
     """Output rows [batch, len_q, heads * dim] and the new (keys, values, tokens seen, un-rotated sinks)."""
     batch, len_q, n_new = query.size(0), query.size(1), key_value.size(1)
     xq, xk, xv = project_q(query), project_k(key_value), project_v(key_value)
-    for x in (xq, xk, xv):
-        if x.dtype != torch.bfloat16:
-            raise TypeError(f"the HIP attention path computes in bfloat16, got {x.dtype}")
     check_head_dim(dim_head)
     dev = xq.device
+    for x in (xq, xk, xv):
+        _check_rows(x, dev)
     native = dim_head in (64, HEAD_DIM)                        # other widths travel in rows of 128
     dim = dim_head if native else HEAD_DIM
     split = _heads if native else _wide_heads
@@ -106,6 +132,7 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
     seen = rows_old = raw_rows = 0
     if past is not None:
         old_k, old_v, seen, raw_old = past
+        _check_cached(old_k, old_v, raw_old, batch, num_heads_kv, dim_head, dev)
         rows_old = old_k.size(2)
         if native:
             cached_k, cached_v = _cache_rows(old_k), _cache_rows(old_v)

@@ -1,0 +1,85 @@
+"""CPU-only checks of the sliding-window and causal attention types' host side: what reaches the native call, with a stand-in
+for the library that records it."""
+import pytest
+import torch
+
+from infllm_amd.attention import ATTN_FORWRAD, RotaryEmbeddingESM, _sink_window
+
+H, HKV, D, B = 4, 2, 128, 2
+
+
+class Native:
+    """records the argument blocks of infllm_window_forward instead of launching"""
+
+    def __init__(self):
+        self.calls = []
+
+    def infllm_window_forward(self, args, stream):
+        self.calls.append((_sink_window._ARGS.unpack(args), stream))
+        return 0
+
+
+@pytest.fixture
+def native(monkeypatch):
+    lib = Native()
+    monkeypatch.setattr(_sink_window._lib, "load", lambda: lib)
+    monkeypatch.setattr(_sink_window, "_stream", lambda: 7)
+    monkeypatch.setattr(_sink_window, "_on_gpu", lambda t: True)
+    return lib
+
+
+def layer(kind, past, n, batch=B, q=None, k=None, v=None):
+    fwd = ATTN_FORWRAD[kind](False) if kind == "origin" else ATTN_FORWRAD[kind](64, 8, fattn=False)
+    same = lambda t: t
+    rows = lambda h: torch.zeros((batch, n, h * D), dtype=torch.bfloat16)
+    q, k, v = rows(H) if q is None else q, rows(HKV) if k is None else k, rows(HKV) if v is None else v
+    return fwd(None, torch.zeros((batch, n, 1)), torch.zeros((batch, n, 1)), RotaryEmbeddingESM(D, device="cpu"), True, past, lambda _: q, lambda _: k,
+               lambda _: v, same, D, H, HKV)
+
+
+KINDS = ["origin", "stream-llm", "infinite-lm"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("what", ["batch", "heads", "width", "dtype", "device", "rank", "short values", "values' batch"])
+def test_a_cache_that_does_not_fit_the_call_is_refused(kind, what, native):
+    """(the native call would read, and copy, rows beyond the end of such a cache)"""
+    _, past = layer(kind, None, 30)
+    k, v, rest = past[0], past[1], past[2:]
+    bad = {"batch": lambda t: t[:1], "heads": lambda t: t[:, :1], "width": lambda t: t[..., :64], "dtype": lambda t: t.half(),
+           "device": lambda t: t.to("meta"), "rank": lambda t: t[0], "short values": lambda t: t[:, :, :20], "values' batch": lambda t: t[:1]}[what]
+    if what not in ("short values", "values' batch"):
+        k = bad(k)
+    v = bad(v)
+    n = len(native.calls)
+    with pytest.raises((ValueError, IndexError)):
+        layer(kind, (k, v) + tuple(rest), 1)
+    assert len(native.calls) == n
+
+
+def test_un_rotated_sinks_that_do_not_fit_the_call_are_refused(native):
+    _, past = layer("infinite-lm", None, 30)
+    for bad in (past[3][:1], past[3][:, :1], past[3].float(), past[3].to("meta")):
+        with pytest.raises(ValueError):
+            layer("infinite-lm", past[:3] + (bad,), 1)
+    assert len(native.calls) == 1
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_projections_of_another_length_or_batch_are_refused(kind, native):
+    rows = lambda b, n, h: torch.zeros((b, n, h * D), dtype=torch.bfloat16)
+    for bad in (dict(q=rows(B, 29, H)), dict(k=rows(B - 1, 30, HKV)), dict(v=rows(B, 31, HKV)), dict(v=rows(B, 30, HKV).to("meta"))):
+        with pytest.raises((RuntimeError, ValueError)):
+            layer(kind, None, 30, **bad)
+    assert not native.calls
+    layer(kind, None, 30, q=rows(B, 30, H).view(B * 30, H * D), k=rows(B, 30, HKV).view(B, 30, HKV, D))    # other shapes of the same rows are taken
+    assert len(native.calls) == 1
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_cache_that_fits_is_taken(kind, native):
+    _, past = layer(kind, None, 30)
+    for n in (1, 20, 60, 1):
+        out, past = layer(kind, past, n)
+        assert out.shape == (B, n, H * D)
+    assert len(native.calls) == 5 and past[0].shape == past[1].shape
