@@ -34,17 +34,27 @@ _SPLIT_ROWS = 131072                # partial rows that key splits of a call of 
 
 
 class _Room:
-    """Buffers [B, Hkv, capacity, dim] of which the first `used` rows are a cache."""
-    __slots__ = ("k", "v", "used", "lock")
+    """How far the buffers [B, Hkv, capacity, dim] of a cache are filled: the first `used` rows are the newest cache in them.
 
-    def __init__(self, k, v, used):
-        self.k, self.v, self.used, self.lock = k, v, used, threading.Lock()
+    It hangs on the storage that both buffers share, not on the tensors that are handed out, so that copying, pickling or saving
+    those takes their data and nothing of this.  It keeps numbers only (a tensor here would keep the storage alive)."""
+    __slots__ = ("k_ptr", "v_ptr", "k_shape", "strides", "used", "lock")
+
+    def __init__(self, both, used):
+        k, v = both.unbind(0)
+        self.k_ptr, self.v_ptr, self.k_shape, self.strides = k.data_ptr(), v.data_ptr(), k.shape, k.stride()
+        self.used, self.lock = used, threading.Lock()
+        both.untyped_storage()._infllm_room = self
+
+    @staticmethod
+    def of(t):
+        return getattr(t.untyped_storage(), "_infllm_room", None)
 
     def claim(self, past_k, past_v, n_new):
         """Whether this call may write the n_new rows behind the given cache."""
         rows = past_k.size(2)
-        if (past_k.data_ptr() != self.k.data_ptr() or past_v.data_ptr() != self.v.data_ptr() or past_k.stride() != self.k.stride()
-                or past_v.stride() != self.v.stride() or past_k.shape[:2] != self.k.shape[:2] or rows + n_new > self.k.size(2)):
+        if (past_k.data_ptr() != self.k_ptr or past_v.data_ptr() != self.v_ptr or past_k.stride() != self.strides or past_v.stride() != self.strides
+                or past_k.shape[:2] != self.k_shape[:2] or past_k.size(3) != self.k_shape[3] or rows + n_new > self.k_shape[2]):
             return False
         with self.lock:
             if self.used != rows:                              # another call went on from this cache already
@@ -153,21 +163,22 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
     if cut:
         rows_new = n_init + n_local
         cache = torch.empty((2, batch, num_heads_kv, rows_new, dim), **bf)
-        new_k, new_v = buf_k, buf_v = cache.unbind(0)
+        new_k, new_v = cache.unbind(0)
         if len_q > 1 or n_new > 1:
             all_kv = torch.empty((2, batch, num_heads_kv, rows_all, dim), **bf)
     else:
         rows_new = rows_all
-        room = getattr(old_k, "_infllm_room", None) if past is not None and native else None
-        if room is None or not room.claim(old_k, old_v, n_new):
+        shape = (batch, num_heads_kv, rows_all, dim)
+        room = _Room.of(old_k) if past is not None and native else None
+        if room is not None and room.claim(old_k, old_v, n_new):
+            new_k, new_v = (t.as_strided(shape, t.stride(), t.storage_offset()) for t in (old_k, old_v))
+        else:
             cap = rows_all + max(256, rows_all // 4)
             if kind:
                 cap = max(rows_all, min(cap, n_local + n_init))
             both = torch.empty((2, batch, num_heads_kv, cap, dim), **bf)
-            room = _Room(both[0], both[1], rows_all)
-        buf_k, buf_v = room.k, room.v
-        new_k, new_v = buf_k.narrow(2, 0, rows_all), buf_v.narrow(2, 0, rows_all)
-        new_k._infllm_room = room
+            _Room(both, rows_all)
+            new_k, new_v = both.narrow(3, 0, rows_all).unbind(0)
 
     rows_q = batch * num_heads * len_q
     q_bytes = (2 if kind else 1) * rows_q * dim * 2
@@ -181,7 +192,7 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
         ok_sb, ok_sh, ov_sb, ov_sh = cached_k.stride(0), cached_k.stride(1), cached_v.stride(0), cached_v.stride(1)
     args = _ARGS.pack(q.data_ptr(), k.data_ptr(), v.data_ptr(), q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl, batch, num_heads, num_heads_kv, dim,
                       len_q, n_new, kind, n_init, n_local, seen, inv_freq.data_ptr(), float(position_bias.distance_scale), okp, ovp, ok_sb, ok_sh, ov_sb,
-                      ov_sh, buf_k.data_ptr(), buf_v.data_ptr(), buf_k.stride(0), buf_k.stride(1), buf_v.stride(0), buf_v.stride(1), rows_old, rows_new,
+                      ov_sh, new_k.data_ptr(), new_v.data_ptr(), new_k.stride(0), new_k.stride(1), new_v.stride(0), new_v.stride(1), rows_old, rows_new,
                       all_kv[0].data_ptr() if all_kv is not None else 0, all_kv[1].data_ptr() if all_kv is not None else 0,
                       raw_old.data_ptr() if raw_old is not None else 0, raw.data_ptr() if raw is not None else 0, raw_rows, raw_new, work.data_ptr(),
                       work.numel(), out.data_ptr(), out.stride(0), dim, out.stride(1), 1.0 / math.sqrt(dim_head))

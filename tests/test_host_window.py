@@ -83,3 +83,23 @@ def test_a_cache_that_fits_is_taken(kind, native):
         out, past = layer(kind, past, n)
         assert out.shape == (B, n, H * D)
     assert len(native.calls) == 5 and past[0].shape == past[1].shape
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_cache_can_be_copied_pickled_and_saved(kind, native):
+    """Keeping a prompt's cache for later continuations is a normal use; the copies are caches of their own."""
+    import copy
+    import io
+    import pickle
+    _, past = layer(kind, None, 30)
+    for t in past[:2]:
+        t.normal_()
+    saved = io.BytesIO()
+    torch.save(past, saved)
+    saved.seek(0)
+    for other in (copy.deepcopy(past), pickle.loads(pickle.dumps(past)), torch.load(saved, weights_only=True), tuple(copy.copy(past))):
+        assert all(torch.equal(a, b) for a, b in zip(other[:2], past[:2]))
+        _, new = layer(kind, other, 1)
+        if other[0].data_ptr() != past[0].data_ptr():
+            assert new[0].data_ptr() not in (other[0].data_ptr(), past[0].data_ptr())
+    assert past[0].shape[2] == 30
