@@ -37,23 +37,26 @@ class _Room:
     """How far the buffers [B, Hkv, capacity, dim] of a cache are filled: the first `used` rows are the newest cache in them.
 
     It hangs on the storage that both buffers share, not on the tensors that are handed out, so that copying, pickling or saving
-    those takes their data and nothing of this.  It keeps numbers only (a tensor here would keep the storage alive)."""
-    __slots__ = ("k_ptr", "v_ptr", "k_shape", "strides", "used", "lock")
+    those takes their data and nothing of this.  It keeps numbers only (a tensor here would keep the storage alive).
 
-    def __init__(self, both, used):
+    A call on another stream than the buffers' own takes new ones: what it returns has to be memory of ITS stream, which the
+    allocator gives out again in that stream's order once the caller drops it."""
+    __slots__ = ("k_ptr", "v_ptr", "k_shape", "strides", "used", "stream", "lock")
+
+    def __init__(self, both, used, stream):
         k, v = both.unbind(0)
         self.k_ptr, self.v_ptr, self.k_shape, self.strides = k.data_ptr(), v.data_ptr(), k.shape, k.stride()
-        self.used, self.lock = used, threading.Lock()
+        self.used, self.stream, self.lock = used, stream, threading.Lock()
         both.untyped_storage()._infllm_room = self
 
     @staticmethod
     def of(t):
         return getattr(t.untyped_storage(), "_infllm_room", None)
 
-    def claim(self, past_k, past_v, n_new):
+    def claim(self, past_k, past_v, n_new, stream):
         """Whether this call may write the n_new rows behind the given cache."""
         rows = past_k.size(2)
-        if (past_k.data_ptr() != self.k_ptr or past_v.data_ptr() != self.v_ptr or past_k.stride() != self.strides or past_v.stride() != self.strides
+        if (stream != self.stream or past_k.data_ptr() != self.k_ptr or past_v.data_ptr() != self.v_ptr or past_k.stride() != self.strides or past_v.stride() != self.strides
                 or past_k.shape[:2] != self.k_shape[:2] or past_k.size(3) != self.k_shape[3] or rows + n_new > self.k_shape[2]):
             return False
         with self.lock:
@@ -140,6 +143,7 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
 
     old_k = old_v = raw_old = None
     seen = rows_old = raw_rows = 0
+    stream = _stream()
     if past is not None:
         old_k, old_v, seen, raw_old = past
         _check_cached(old_k, old_v, raw_old, batch, num_heads_kv, dim_head, dev)
@@ -170,14 +174,14 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
         rows_new = rows_all
         shape = (batch, num_heads_kv, rows_all, dim)
         room = _Room.of(old_k) if past is not None and native else None
-        if room is not None and room.claim(old_k, old_v, n_new):
+        if room is not None and room.claim(old_k, old_v, n_new, stream):
             new_k, new_v = (t.as_strided(shape, t.stride(), t.storage_offset()) for t in (old_k, old_v))
         else:
             cap = rows_all + max(256, rows_all // 4)
             if kind:
                 cap = max(rows_all, min(cap, n_local + n_init))
             both = torch.empty((2, batch, num_heads_kv, cap, dim), **bf)
-            _Room(both, rows_all)
+            _Room(both, rows_all, stream)
             new_k, new_v = both.narrow(3, 0, rows_all).unbind(0)
 
     rows_q = batch * num_heads * len_q
@@ -196,7 +200,7 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
                       all_kv[0].data_ptr() if all_kv is not None else 0, all_kv[1].data_ptr() if all_kv is not None else 0,
                       raw_old.data_ptr() if raw_old is not None else 0, raw.data_ptr() if raw is not None else 0, raw_rows, raw_new, work.data_ptr(),
                       work.numel(), out.data_ptr(), out.stride(0), dim, out.stride(1), 1.0 / math.sqrt(dim_head))
-    _lib.check(_lib.load().infllm_window_forward(args, _stream()), "infllm_window_forward")
+    _lib.check(_lib.load().infllm_window_forward(args, stream), "infllm_window_forward")
     if not native:
         out = narrow(out.view(batch, len_q, num_heads, dim), dim_head).reshape(batch, len_q, num_heads * dim_head)
         new_k, new_v = narrow(new_k, dim_head), narrow(new_v, dim_head)

@@ -103,3 +103,16 @@ def test_a_cache_can_be_copied_pickled_and_saved(kind, native):
         if other[0].data_ptr() != past[0].data_ptr():
             assert new[0].data_ptr() not in (other[0].data_ptr(), past[0].data_ptr())
     assert past[0].shape[2] == 30
+
+
+def test_a_call_on_another_stream_gets_buffers_of_its_own(native, monkeypatch):
+    """Buffers belong to the stream they were allocated on: the allocator may hand them out again in that stream's order while
+    another stream still writes them."""
+    _, past = layer("origin", None, 30)
+    _, same = layer("origin", past, 1)
+    assert same[0].data_ptr() == past[0].data_ptr()
+    monkeypatch.setattr(_sink_window, "_stream", lambda: 8)
+    _, other = layer("origin", same, 1)
+    assert other[0].data_ptr() != same[0].data_ptr() and other[1].data_ptr() != same[1].data_ptr() and native.calls[-1][1] == 8
+    _, again = layer("origin", other, 1)
+    assert again[0].data_ptr() == other[0].data_ptr()
