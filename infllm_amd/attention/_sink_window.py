@@ -16,7 +16,8 @@ fields (keys, values, tokens seen); a fourth holds the un-rotated sink keys when
 
 A cache that still holds every token grows in place: its tensors are the filled part of buffers with room behind it
 (a quarter more), and the next call writes its rows there instead of copying everything - when the cache it is given is
-the newest one of those buffers.  An older one (a second continuation of the same prompt) gets buffers of its own.
+the newest one of those buffers.  An older one (a second continuation of the same prompt) gets buffers of its own.  A cache
+and the one it continues then share memory: a caller that writes into a cache's tensors clones them first.
 """
 import math
 import struct
@@ -56,8 +57,9 @@ class _Room:
     def claim(self, past_k, past_v, n_new, stream):
         """Whether this call may write the n_new rows behind the given cache."""
         rows = past_k.size(2)
-        if (stream != self.stream or past_k.data_ptr() != self.k_ptr or past_v.data_ptr() != self.v_ptr or past_k.stride() != self.strides or past_v.stride() != self.strides
-                or past_k.shape[:2] != self.k_shape[:2] or past_k.size(3) != self.k_shape[3] or rows + n_new > self.k_shape[2]):
+        if (stream != self.stream or past_k.data_ptr() != self.k_ptr or past_v.data_ptr() != self.v_ptr or past_k.stride() != self.strides
+                or past_v.stride() != self.strides or past_k.shape[:2] != self.k_shape[:2] or past_k.size(3) != self.k_shape[3]
+                or rows + n_new > self.k_shape[2]):
             return False
         with self.lock:
             if self.used != rows:                              # another call went on from this cache already

@@ -132,3 +132,112 @@ def test_key_splits_of_a_prompts_first_call_follow_the_oracle(kind, T, H, Hkv):
         got, _ = _drive(ATTN_FORWRAD[kind](1024, 64, fattn=False), xq, xk, xv, [T], H, Hkv, 1e4)
         want = SinkWindowOracle(RopeOracle(D, base=1e4), 1024, 64, kind).append(*heads)
     _check(got, want)
+
+
+# ---- a cache that grows in place: its tensors are the filled part of buffers that the next call writes on
+N_LOCAL, N_INIT = 700, 16          # every stream below stays inside: nothing is cut
+
+
+class _Branch:
+    """A stream of one of the types, fed [batch, tokens, heads * D] rows, with the oracle following it."""
+
+    def __init__(self, kind, H, Hkv, past=None, history=()):
+        from infllm_amd.attention import ATTN_FORWRAD
+        self.kind, self.H, self.Hkv, self.past, self.history = kind, H, Hkv, past, list(history)
+        self.forward = ATTN_FORWRAD[kind](False) if kind == "origin" else ATTN_FORWRAD[kind](N_LOCAL, N_INIT, fattn=False)
+
+    def feed(self, rows):
+        from infllm_amd.attention import RotaryEmbeddingESM
+        q, k, v = (t.cuda() for t in rows)
+        same = lambda t: t
+        o, self.past = self.forward(None, q, k, RotaryEmbeddingESM(D, base=1e4, device="cuda"), True, self.past, same, same, lambda _: v, same, D, self.H,
+                                    self.Hkv)
+        self.history.append(rows)
+        return o
+
+    def check(self, o):
+        """the last call's rows against the oracle over the whole history (bounds of this file)"""
+        rope = RopeOracle(D, base=1e4)
+        ora = CausalOracle(rope) if self.kind == "origin" else SinkWindowOracle(rope, N_LOCAL, N_INIT, self.kind)
+        for q, k, v in self.history:
+            want = ora.append(_heads(q, self.H), _heads(k, self.Hkv), _heads(v, self.Hkv))
+        _check(o.cpu(), want)
+
+    def fork(self, past=None, history=None):
+        return _Branch(self.kind, self.H, self.Hkv, self.past if past is None else past, self.history if history is None else history)
+
+    def cut(self, change):
+        """the cache with `change` made to its tensors"""
+        return tuple(change(t) if torch.is_tensor(t) else t for t in self.past)
+
+
+KINDS = ["origin", "stream-llm", "infinite-lm"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("B", [1, 2])
+def test_two_continuations_of_one_prompt(kind, B):
+    """The first one goes on in the prompt's buffers, the second finds them taken and copies; neither sees the other's rows."""
+    H, Hkv = 4, 2
+    prompt = _Branch(kind, H, Hkv)
+    prompt.check(prompt.feed(_stream(300, H, Hkv, 1, B)))
+    kept = [t.clone() for t in prompt.past[:2]]
+    a, b = prompt.fork(), prompt.fork()
+    for i, n in enumerate([1, 1, 40, 1]):
+        a.check(a.feed(_stream(n, H, Hkv, 10 + i, B)))
+        if i == 0:
+            assert a.past[0].data_ptr() == prompt.past[0].data_ptr()
+        b.check(b.feed(_stream(n, H, Hkv, 20 + i, B)))
+        assert a.past[0].data_ptr() != b.past[0].data_ptr() and a.past[0].shape == b.past[0].shape
+    again = prompt.fork()
+    again.check(again.feed(_stream(7, H, Hkv, 30, B)))
+    assert all(torch.equal(x, y) for x, y in zip(kept, prompt.past[:2]))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_changed_caches_continue_in_buffers_of_their_own(kind):
+    """rolled back by some tokens, rows of the batch in another order, one prompt for a whole batch, one row of the batch"""
+    H, Hkv, B = 4, 2, 2
+    base = _Branch(kind, H, Hkv)
+    base.feed(_stream(300, H, Hkv, 1, B))
+    rows = base.history[0]
+    kept = [t.clone() for t in base.past[:2]]
+    seen = lambda past, n: past if kind == "origin" else (past[0], past[1], n, past[3])
+    back = base.fork(seen(tuple(t[:, :, :280] if torch.is_tensor(t) and t.shape[2] == 300 else t for t in base.past), 280), [tuple(t[:, :280] for t in rows)])
+    order = base.fork(base.cut(lambda t: t[[1, 0]]), [tuple(t[[1, 0]] for t in rows)])
+    one = base.fork(base.cut(lambda t: t[1:]), [tuple(t[1:] for t in rows)])
+    many = base.fork(base.cut(lambda t: t[:1].expand(3, -1, -1, -1)), [tuple(t[:1].expand(3, -1, -1) for t in rows)])
+    for i, (branch, batch) in enumerate(((back, B), (order, B), (one, 1), (many, 3))):
+        for n in (1, 30, 1):
+            branch.check(branch.feed(_stream(n, H, Hkv, 40 + 3 * i + n, batch)))
+        assert branch.past[0].data_ptr() != base.past[0].data_ptr()
+    assert all(torch.equal(x, y) for x, y in zip(kept, base.past[:2]))
+    base.check(base.feed(_stream(1, H, Hkv, 60, B)))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_growth_past_the_room(kind):
+    """200 tokens leave room for 256 more; the calls cross its end by one token, exactly, and by many"""
+    H, Hkv = 4, 2
+    for calls in ([200, 255, 1, 1], [200, 256, 1], [200, 250, 20, 1], [200, 1, 400]):
+        s = _Branch(kind, H, Hkv)
+        for i, n in enumerate(calls):
+            o = s.feed(_stream(n, H, Hkv, 70 + i))
+        s.check(o)
+        assert s.past[0].shape[2] == sum(calls)
+
+
+def test_a_dropped_cache_is_given_back():
+    H, Hkv = 4, 2
+    rows = _stream(300, H, Hkv, 1), _stream(1, H, Hkv, 2)
+    s = _Branch("origin", H, Hkv)
+    s.feed(rows[0])
+    del s
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    s = _Branch("origin", H, Hkv)
+    s.feed(rows[0])
+    s.feed(rows[1])
+    assert torch.cuda.memory_allocated() > before
+    del s
+    assert torch.cuda.memory_allocated() == before

@@ -116,3 +116,22 @@ def test_a_call_on_another_stream_gets_buffers_of_its_own(native, monkeypatch):
     assert other[0].data_ptr() != same[0].data_ptr() and other[1].data_ptr() != same[1].data_ptr() and native.calls[-1][1] == 8
     _, again = layer("origin", other, 1)
     assert again[0].data_ptr() == other[0].data_ptr()
+
+
+def test_which_calls_write_behind_the_cache_they_are_given(native):
+    """Only a continuation of the newest cache of the buffers, unchanged, with room behind it; every other call copies."""
+    _, p = layer("origin", None, 30)                                                  # room for 256 more
+    where = lambda past: (past[0].data_ptr(), past[1].data_ptr())
+    _, a = layer("origin", p, 1)
+    _, b = layer("origin", p, 1)
+    assert where(a) == where(p) and where(b) != where(p)
+    for other in ((b[0][:, :, :30], b[1][:, :, :30]), (b[0][[1, 0]], b[1][[1, 0]]), (b[0], a[1]), (a[0], b[1]), (b[1], b[0]),
+                  (b[0][:1].expand(B, -1, -1, -1), b[1][:1].expand(B, -1, -1, -1))):
+        _, c = layer("origin", other, 1)
+        assert where(c)[0] not in (where(a)[0], where(b)[0]) and where(c)[1] not in (where(a)[1], where(b)[1])
+    _, full = layer("origin", b, 256)                                                 # exactly to the end
+    assert where(full) == where(b)
+    _, beyond = layer("origin", full, 1)
+    assert where(beyond) != where(full) and beyond[0].shape[2] == 288
+    _, same = layer("origin", (beyond[0].detach(), beyond[1].detach()), 1)            # another tensor of the same rows
+    assert where(same) == where(beyond)
