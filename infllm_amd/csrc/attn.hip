@@ -720,15 +720,14 @@ __global__ __launch_bounds__(256) void attn_merge_wide_kernel(const _Float16 *o_
         m = fmaxf(m, l[i]);
     }
     m = group16_max(m);
+    if (m == -INFINITY) m = 0.f;                                             // as in merge_piece
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, den = 0.f;
-    if (m > -INFINITY) {
 #pragma unroll
-        for (int i = 0; i < kMine; ++i) {
-            const float w = __builtin_amdgcn_exp2f(l[i] - m);
+    for (int i = 0; i < kMine; ++i) {
+        const float w = __builtin_amdgcn_exp2f(l[i] - m);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] += (float)o[i][j] * w;
-            den += w;
-        }
+        for (int j = 0; j < 8; ++j) acc[j] += (float)o[i][j] * w;
+        den += w;
     }
     den = group16_sum(den);
 #pragma unroll

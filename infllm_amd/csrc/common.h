@@ -116,27 +116,27 @@ __device__ __forceinline__ void merge_piece(const MergeJob &mj, int64_t e) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) m = fmaxf(m, l8[i]);
     }
+    if (m == -INFINITY) m = 0.f;                                         // no partial with a finite sum: every weight is 0
     float acc[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] = 0.f;
     float den = 0.f;
-    if (m > -INFINITY) {
-        for (int p0 = 0; p0 < P; p0 += 8) {
-            float l8[8];
-            f16x8 o8[8];
+    for (int p0 = 0; p0 < P; p0 += 8) {
+        float l8[8];
+        f16x8 o8[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const bool on = p0 + i < P;
-                l8[i] = on ? lse_part[ps.l(p0 + i, rows) + row] : -INFINITY;
-                o8[i] = on ? *(const f16x8 *)(o_part + (ps.l(p0 + i, rows) + row) * D + ps.o(p0 + i) + c * 8) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            }
+        for (int i = 0; i < 8; ++i) {
+            const bool on = p0 + i < P;
+            l8[i] = on ? lse_part[ps.l(p0 + i, rows) + row] : -INFINITY;
+            o8[i] = on ? *(const f16x8 *)(o_part + (ps.l(p0 + i, rows) + row) * D + ps.o(p0 + i) + c * 8) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float w = __builtin_amdgcn_exp2f(l8[i] - m);       // exp2(-inf) = 0: empty partials hold zeros
+        for (int i = 0; i < 8; ++i) {
+            // exp2(-inf) = 0: empty partials hold zeros, those with a logit that was no number NaN, which stays NaN
+            const float w = __builtin_amdgcn_exp2f(l8[i] - m);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) acc[j] += (float)o8[i][j] * w;
-                den += w;
-            }
+            for (int j = 0; j < 8; ++j) acc[j] += (float)o8[i][j] * w;
+            den += w;
         }
     }
     const float inv = den > 0.f ? 1.f / den : 0.f;

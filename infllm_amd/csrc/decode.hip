@@ -11,6 +11,8 @@
 //   O[head, d] += p[key] * v[key, d] on the vector units in fp32: a row group reads its own four keys' value rows
 //   (16 lanes x 16 bytes), and a head's probability reaches the row's lanes by a DPP row broadcast.
 // The states of all row groups and waves are joined through LDS at the end, the splits by the merge kernels.
+// A logit that is NaN or +infinity makes its query's row NaN, as the softmax has it: a lane that saw nothing but NaN still has
+// its maximum at -infinity, so its sum is taken as it is, and a split whose sum is no number writes NaN rather than zeros.
 // 32,768 keys x 8 kv heads (134 MB): 648 us with the tile kernel of attn.hip at one split, 33 us here.
 #include "decode.h"
 
@@ -150,6 +152,11 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
             m = mn;
             neg_ms = m == -INFINITY ? 0.f : -m * scale;
         }
+        if (bl.valid < kDecodeBlock) {                     // the repeated rows: 0 x infinity would be NaN
+#pragma unroll
+            for (int i = 0; i < VL; ++i)
+                if ((D == 128 ? 4 * rg + i : 4 * rg + 2 * i + (col >> 3)) >= bl.valid) vbuf[buf][i] = u32x4{0, 0, 0, 0};
+        }
         float p[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale, neg_ms));
@@ -229,13 +236,13 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
 #pragma unroll
         for (int w = 0; w < kDecWaves; ++w)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) den += sm[w][r][h] == -INFINITY ? 0.f : sl[w][r][h] * __builtin_amdgcn_exp2f((sm[w][r][h] - mx) * scale);
+            for (int r = 0; r < 4; ++r) den += sl[w][r][h] * (sm[w][r][h] == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((sm[w][r][h] - mx) * scale));
 #pragma unroll
         for (int w = 0; w < kDecWaves; ++w)
 #pragma unroll
             for (int r = 0; r < GRP; ++r) o += red[w][r][h][d];
         const int64_t row = ((int64_t)split * j.B + b) * j.H + h0 + h;
-        ((_Float16 *)j.o_part)[row * D + d] = (_Float16)(den > 0.f ? o / den : 0.f);
+        ((_Float16 *)j.o_part)[row * D + d] = (_Float16)(den == 0.f ? 0.f : o / den);
         if (d == 0) j.lse_part[row] = den > 0.f ? mx * scale + log2f(den) : -INFINITY;
     }
 }
