@@ -77,10 +77,13 @@ def _rows16(t):
     return t if inner == 1 and not odd & 7 and not t.data_ptr() & 15 else t.contiguous()
 
 
-def _cache_rows(t):
-    """a cached tensor as the native call takes it: rows next to each other"""
-    t = _rows16(t)
-    return t if t.stride(2) == t.size(3) else t.contiguous()
+def _cache_rows(t, dim):
+    """(a cached tensor as the native call takes it: rows next to each other, its batch and head strides)"""
+    sb, sh, sl, inner = t.stride()
+    if inner != 1 or sl != dim or (sb | sh) & 7 or t.data_ptr() & 15:
+        t = t.contiguous()
+        sb, sh, _, _ = t.stride()
+    return t, sb, sh
 
 
 def _heads(x, batch, length, heads, dim):
@@ -96,41 +99,41 @@ def _wide_heads(x, batch, length, heads, dim):
     return x, x.stride(0), x.stride(2), x.stride(1)
 
 
-def _check_rows(x, device):
-    """projected rows: the native call takes them by address and reads bfloat16 on the GPU"""
-    if x.dtype != torch.bfloat16:
-        raise TypeError(f"the HIP attention path computes in bfloat16, got {x.dtype}")
-    if x.device != device or not _on_gpu(x):
-        raise ValueError(f"q, k and v must be on one GPU, got {x.device} beside {device}")
-
-
 def _on_gpu(x):
     return x.is_cuda
 
 
-def _check_cached(old_k, old_v, raw, batch, heads, dim, device):
-    """A cache that the call's rows can join.  The native call takes addresses and strides and cannot see how far a tensor
-    reaches, so whatever joining the tensors would refuse - another batch, head count, width, type or device - is refused here."""
-    for name, t in (("keys", old_k), ("values", old_v), ("un-rotated sinks", raw)):
-        if t is None and name == "un-rotated sinks":
-            continue
-        shape = (batch, heads, t.size(2) if t.dim() == 4 else -1, dim)
-        if t.shape != shape:
-            raise ValueError(f"cached {name} {tuple(t.shape)} do not fit a call of batch {batch}, {heads} kv heads of {dim}")
-        if t.dtype != torch.bfloat16 or t.device != device:
-            raise ValueError(f"cached {name} must be bfloat16 on {device}, got {t.dtype} on {t.device}")
-    if old_v.size(2) != old_k.size(2):
-        raise ValueError(f"the cache holds {old_k.size(2)} keys and {old_v.size(2)} values")
+def _check_rows(q, k, v):
+    """projected rows: the native call takes them by address and reads bfloat16 on the GPU"""
+    bf, dev = torch.bfloat16, q.device
+    if q.dtype is not bf or k.dtype is not bf or v.dtype is not bf:
+        raise TypeError(f"the HIP attention path computes in bfloat16, got {q.dtype}, {k.dtype}, {v.dtype}")
+    if k.device != dev or v.device != dev or not _on_gpu(q):
+        raise ValueError(f"q, k and v must be on one GPU, got {q.device}, {k.device}, {v.device}")
+
+
+def _check_cached(k, v, raw, batch, heads, dim, device):
+    """The rows of a cache that the call's rows can join.  The native call takes addresses and strides and cannot see how far a
+    tensor reaches, so whatever joining the tensors would refuse - another batch, head count, width, type or device - is refused
+    here."""
+    bf, shape = torch.bfloat16, k.shape
+    rows = shape[2] if len(shape) == 4 else -1
+    if shape != (batch, heads, rows, dim) or v.shape != shape:
+        raise ValueError(f"cached keys {tuple(shape)} and values {tuple(v.shape)} do not fit a call of batch {batch}, {heads} kv heads of {dim}")
+    if k.dtype is not bf or v.dtype is not bf or k.device != device or v.device != device:
+        raise ValueError(f"the cache must be bfloat16 on {device}, got {k.dtype} on {k.device} and {v.dtype} on {v.device}")
+    if raw is not None and (raw.dim() != 4 or raw.shape != (batch, heads, raw.size(2), dim) or raw.dtype is not bf or raw.device != device):
+        raise ValueError(f"un-rotated sinks {tuple(raw.shape)}, {raw.dtype} on {raw.device}, do not fit a call of batch {batch}, {heads} kv heads of {dim}")
+    return rows
 
 
 def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_q, project_k, project_v, dim_head, num_heads, num_heads_kv):
     """Output rows [batch, len_q, heads * dim] and the new (keys, values, tokens seen, un-rotated sinks)."""
-    batch, len_q, n_new = query.size(0), query.size(1), key_value.size(1)
+    (batch, len_q), n_new = query.shape[:2], key_value.size(1)
     xq, xk, xv = project_q(query), project_k(key_value), project_v(key_value)
     check_head_dim(dim_head)
     dev = xq.device
-    for x in (xq, xk, xv):
-        _check_rows(x, dev)
+    _check_rows(xq, xk, xv)
     native = dim_head in (64, HEAD_DIM)                        # other widths travel in rows of 128
     dim = dim_head if native else HEAD_DIM
     split = _heads if native else _wide_heads
@@ -148,12 +151,11 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
     stream = _stream()
     if past is not None:
         old_k, old_v, seen, raw_old = past
-        _check_cached(old_k, old_v, raw_old, batch, num_heads_kv, dim_head, dev)
-        rows_old = old_k.size(2)
+        rows_old = _check_cached(old_k, old_v, raw_old, batch, num_heads_kv, dim_head, dev)
         if native:
-            cached_k, cached_v = _cache_rows(old_k), _cache_rows(old_v)
+            cached_k, cached_v = old_k, old_v
         else:
-            cached_k, cached_v = widen(old_k, dim_head).contiguous(), widen(old_v, dim_head).contiguous()
+            cached_k, cached_v = widen(old_k, dim_head), widen(old_v, dim_head)
             raw_old = None if raw_old is None else widen(raw_old, dim_head)
         if raw_old is not None:
             raw_old = raw_old.contiguous()
@@ -189,19 +191,22 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
     rows_q = batch * num_heads * len_q
     q_bytes = (2 if kind else 1) * rows_q * dim * 2
     part_rows = 64 * rows_q if rows_q <= 2048 else _SPLIT_ROWS if 2 * rows_q <= _SPLIT_ROWS else 0
-    work = torch.empty((q_bytes + part_rows * (2 * dim + 4),), dtype=torch.uint8, device=dev)
+    work_bytes = q_bytes + part_rows * (2 * dim + 4)
+    work = torch.empty((work_bytes,), dtype=torch.uint8, device=dev)
     out = torch.empty((batch, len_q, num_heads * dim), **bf)
     okp = ovp = 0
     ok_sb = ok_sh = ov_sb = ov_sh = 0
     if rows_old:
+        cached_k, ok_sb, ok_sh = _cache_rows(cached_k, dim)
+        cached_v, ov_sb, ov_sh = _cache_rows(cached_v, dim)
         okp, ovp = cached_k.data_ptr(), cached_v.data_ptr()
-        ok_sb, ok_sh, ov_sb, ov_sh = cached_k.stride(0), cached_k.stride(1), cached_v.stride(0), cached_v.stride(1)
+    (nk_sb, nk_sh, _, _), (nv_sb, nv_sh, _, _) = new_k.stride(), new_v.stride()
     args = _ARGS.pack(q.data_ptr(), k.data_ptr(), v.data_ptr(), q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl, batch, num_heads, num_heads_kv, dim,
                       len_q, n_new, kind, n_init, n_local, seen, inv_freq.data_ptr(), float(position_bias.distance_scale), okp, ovp, ok_sb, ok_sh, ov_sb,
-                      ov_sh, new_k.data_ptr(), new_v.data_ptr(), new_k.stride(0), new_k.stride(1), new_v.stride(0), new_v.stride(1), rows_old, rows_new,
+                      ov_sh, new_k.data_ptr(), new_v.data_ptr(), nk_sb, nk_sh, nv_sb, nv_sh, rows_old, rows_new,
                       all_kv[0].data_ptr() if all_kv is not None else 0, all_kv[1].data_ptr() if all_kv is not None else 0,
                       raw_old.data_ptr() if raw_old is not None else 0, raw.data_ptr() if raw is not None else 0, raw_rows, raw_new, work.data_ptr(),
-                      work.numel(), out.data_ptr(), out.stride(0), dim, out.stride(1), 1.0 / math.sqrt(dim_head))
+                      work_bytes, out.data_ptr(), len_q * num_heads * dim, dim, num_heads * dim, 1.0 / math.sqrt(dim_head))
     _lib.check(_lib.load().infllm_window_forward(args, stream), "infllm_window_forward")
     if not native:
         out = narrow(out.view(batch, len_q, num_heads, dim), dim_head).reshape(batch, len_q, num_heads * dim_head)
