@@ -35,6 +35,7 @@ native calls: infllm_block_front, infllm_block_select (the one host wait, for
 the retrieved unit ids, which overlaps the local stage; then cache policy and
 fetch) and infllm_block_back, plus infllm_block_prefetch for the next block.
 """
+import contextlib
 import ctypes
 import os
 import threading
@@ -62,7 +63,12 @@ _CARVE_SLOTS = 4             # staging slots of the carve, used in turn (more of
 
 
 class _Buffers(dict):
-    """dict that can be referenced weakly"""
+    """Workspaces of a call, shared by the managers that work on one stream.  Whoever enqueues launches on them holds the lock
+    until the call's last one is enqueued: the stream orders whole calls, not the launches that two threads enqueue by turns."""
+
+    def __init__(self, **tensors):
+        super().__init__(**tensors)
+        self.lock = threading.Lock()
 
 
 class _Units:
@@ -473,7 +479,8 @@ class ContextManager:
         rc.k_sb, rc.k_sh, rc.k_sl, _ = k.stride()
         rc.v_sb, rc.v_sh, rc.v_sl, _ = v.stride()
         rc.o_sb, rc.o_sl, rc.o_sh = n * H * D, H * D, D
-        status = self._lib.infllm_resident_append(self._resident, self._rc_ref, stream)
+        with self._call_buf.lock:
+            status = self._lib.infllm_resident_append(self._resident, self._rc_ref, stream)
         if status:
             check(status, "infllm_resident_append")
         self.length = length + n
@@ -485,8 +492,8 @@ class ContextManager:
         return out.permute(0, 2, 1, 3)
 
     def _bind_resident_buffers(self, stream):
-        """Workspaces of a call: dead between append() calls, so the managers that work on one stream (one after the
-        other, as the layers of a model do) share one set."""
+        """Workspaces of a call: dead between append() calls, so the managers that work on one stream share one set; the set's
+        lock keeps the launches of two threads' calls apart."""
         B, H, D, exc, T = self.num_units, self.unit_size, self.head_width, self.exc_block_size, self._rc.max_tokens
         blocks = -(-T // exc)
         part_rows = max(8, 2 * min(self._local_group, blocks)) * B * H * exc       # (at most two key splits of several blocks)
@@ -610,7 +617,7 @@ class ContextManager:
     def _bind_call_buffers(self, stream):
         """Buffers of a call prepared in one go: the rotated queries of up to call_tokens tokens, the blocks' mean
         queries and the local stage's partial rows.  They are dead between append() calls, so the layers that work on
-        one stream (one after the other, as the layers of a model do) share one set."""
+        one stream share one set; the set's lock keeps the launches of two threads' calls apart."""
         B, H, D, exc, T = self.num_units, self.unit_size, self.head_width, self.exc_block_size, self._call_tokens
         group = self._local_group
         blocks = max(8, 4 * group)            # partial rows: two groups of blocks, up to two key splits each
@@ -990,37 +997,39 @@ class ContextManager:
             if cuts[-1] < input_length:
                 cuts.append(input_length)
             cut_i, plan, plan_pos = -1, None, 0
-        call_end = 0
-        for st in range(0, input_length, exc):
-            n = min(exc, input_length - st)
-            if self._call_tokens and st == call_end:
-                # the next stretch of the call in one go: prologue, mean queries, first retrieval, local stage
-                call_end = min(st + self._call_tokens, input_length)
-                if self.length + call_end - self.cursor > self.ring_cap:
-                    raise RuntimeError(f"a call of {call_end} tokens at {self.length} does not fit the rings "
-                                       f"({self.ring_cap} rows, carving cursor {self.cursor})")
-                if call_end - st > exc:          # a single block (a decode step) gains nothing from being prepared apart
-                    fa.d_q, fa.d_k, fa.d_v = (self._q_ptr + st * self._q_step, self._k_ptr + st * self._k_step,
-                                              self._v_ptr + st * self._v_step)
-                    fa.n, fa.n_units, fa.b0 = call_end - st, self.num_global_block, self.length + st
-                    fa.flags = _lib.NO_RETRIEVAL if use_chunks else 0
-                    # room for every block's scores of the units there are and of those the call can carve
-                    blocks, cols = -(-self._call_tokens // exc), self.num_global_block + (call_end - st) // self.block_size + 2
-                    if self._call_scores is None or self._call_scores.shape[2] < cols or self._call_scores.shape[0] < blocks:
-                        cols = max(-(-cols // 256) * 256, 2 * (self._call_scores.shape[2] if self._call_scores is not None else 0))
-                        self._call_scores = torch.empty((blocks, self.num_units, cols), dtype=torch.float32, device=self.device)
-                    fa.d_call_scores, fa.call_scores_cols = self._call_scores.data_ptr(), self._call_scores.shape[2]
-                    check(self._lib.infllm_call_front(self._layer, self._fa_ref, self._main_raw), "infllm_call_front")
-            elif not self._call_tokens:
-                call_end = input_length
-            chosen = None
-            if use_chunks:
-                if cuts[cut_i + 1] < st + n:
-                    cut_i += 1
-                    plan, plan_pos = self._chunk_topk(q, cuts[cut_i], cuts[cut_i + 1]), 0
-                chosen = plan[plan_pos]
-                plan_pos += 1
-            self._block(st, n, out_ptr + st * out_step, min(exc, call_end - st - n), chosen)
+        shared = self._call_tokens and input_length > exc       # (a call of one block has workspaces of its own)
+        with self._call_buf.lock if shared else contextlib.nullcontext():
+            call_end = 0
+            for st in range(0, input_length, exc):
+                n = min(exc, input_length - st)
+                if self._call_tokens and st == call_end:
+                    # the next stretch of the call in one go: prologue, mean queries, first retrieval, local stage
+                    call_end = min(st + self._call_tokens, input_length)
+                    if self.length + call_end - self.cursor > self.ring_cap:
+                        raise RuntimeError(f"a call of {call_end} tokens at {self.length} does not fit the rings "
+                                           f"({self.ring_cap} rows, carving cursor {self.cursor})")
+                    if call_end - st > exc:          # a single block (a decode step) gains nothing from being prepared apart
+                        fa.d_q, fa.d_k, fa.d_v = (self._q_ptr + st * self._q_step, self._k_ptr + st * self._k_step,
+                                                  self._v_ptr + st * self._v_step)
+                        fa.n, fa.n_units, fa.b0 = call_end - st, self.num_global_block, self.length + st
+                        fa.flags = _lib.NO_RETRIEVAL if use_chunks else 0
+                        # room for every block's scores of the units there are and of those the call can carve
+                        blocks, cols = -(-self._call_tokens // exc), self.num_global_block + (call_end - st) // self.block_size + 2
+                        if self._call_scores is None or self._call_scores.shape[2] < cols or self._call_scores.shape[0] < blocks:
+                            cols = max(-(-cols // 256) * 256, 2 * (self._call_scores.shape[2] if self._call_scores is not None else 0))
+                            self._call_scores = torch.empty((blocks, self.num_units, cols), dtype=torch.float32, device=self.device)
+                        fa.d_call_scores, fa.call_scores_cols = self._call_scores.data_ptr(), self._call_scores.shape[2]
+                        check(self._lib.infllm_call_front(self._layer, self._fa_ref, self._main_raw), "infllm_call_front")
+                elif not self._call_tokens:
+                    call_end = input_length
+                chosen = None
+                if use_chunks:
+                    if cuts[cut_i + 1] < st + n:
+                        cut_i += 1
+                        plan, plan_pos = self._chunk_topk(q, cuts[cut_i], cuts[cut_i + 1]), 0
+                    chosen = plan[plan_pos]
+                    plan_pos += 1
+                self._block(st, n, out_ptr + st * out_step, min(exc, call_end - st - n), chosen)
         self.length += input_length
         # (the last carved units go on to their pinned home in the background: _finish_host_copies before reading them)
         check(self._lib.infllm_layer_end_call(self._layer, self._copy_raw), "infllm_layer_end_call")

@@ -112,3 +112,24 @@ def test_managers_of_two_threads_and_streams(monkeypatch):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert torch.equal(got[0], alone[0]) and torch.equal(got[1], alone[1])
+
+
+def test_managers_of_two_threads_on_one_stream():
+    """Two threads on the default stream, each with a manager of its own, calls of one token and of several blocks: they share
+    the calls' workspaces, and the stream orders their calls."""
+    import threading
+    calls = [700] + [1] * 40 + [300] + [1] * 40 + [129]
+    data = [tuple(t.cuda() for t in make_stream(sum(calls), 8, 2, 190 + i)) for i in range(2)]
+    alone = [torch.cat(feed(new_manager(1e4, **SMALL), *d, calls), dim=2) for d in data]
+    torch.cuda.synchronize()
+    got, start = [None, None], threading.Barrier(2)
+
+    def work(i):
+        start.wait()
+        got[i] = torch.cat(feed(new_manager(1e4, **SMALL), *data[i], calls), dim=2)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], alone[0]) and torch.equal(got[1], alone[1])

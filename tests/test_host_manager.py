@@ -1,0 +1,66 @@
+"""CPU-only checks of ContextManager's host side: what its native calls may find, with a stand-in for the library."""
+import ctypes
+import threading
+import time
+
+import pytest
+import torch
+
+from infllm_amd._lib import ResidentCall
+from infllm_amd.attention import ContextManager, context_manager
+
+
+class Native:
+    def __init__(self):
+        self.open, self.overlaps, self.calls, self.guard = {}, 0, 0, threading.Lock()
+
+    def infllm_resident_append(self, manager, rc, stream):
+        with self.guard:
+            self.calls += 1
+            key = rc._obj.d_q_loc
+            self.overlaps += self.open.get(key, 0)
+            self.open[key] = self.open.get(key, 0) + 1
+        time.sleep(2e-3)                                   # (another thread runs, as while a native call is under way)
+        with self.guard:
+            self.open[key] -= 1
+        return 0
+
+
+def resident_manager(lib):
+    """a manager of a small geometry as _init leaves it, without the library's own objects"""
+    cm = ContextManager.__new__(ContextManager)
+    cm.n_init, cm.n_local, cm.block_size, cm.topk, cm.exc_block_size, cm.cache_strategy = 4, 64, 16, 2, 32, "lru"
+    cm.num_units, cm.unit_size, cm.unit_size_kv, cm.head_width, cm.dim_head = 1, 2, 1, 64, 64
+    cm.length = cm.load_count = cm.num_global_block = 0
+    cm._lib, cm._resident, cm._dev_index, cm.device, cm._layer = lib, cm, 0, torch.device("cpu"), None
+    cm._local_group, cm._part_rows2, cm._chunks, cm._call_scores, cm._call_stream = 1, 64, [], None, None
+    cm._streams, cm.reps = set(), torch.empty((1, 16, 128), dtype=torch.bfloat16)
+    cm._rc = ResidentCall()
+    cm._rc.max_tokens = 64
+    cm._rc_ref = ctypes.byref(cm._rc)
+    return cm
+
+
+@pytest.fixture
+def one_stream(monkeypatch):
+    monkeypatch.setattr(context_manager, "current_stream", lambda: 7)
+
+
+def test_calls_of_two_threads_on_one_stream_are_enqueued_one_after_the_other(one_stream):
+    """Both managers' launches write the same workspaces; interleaved, one call's prologue would overwrite the queries that
+    the other's attention has yet to read."""
+    lib = Native()
+    managers = [resident_manager(lib) for _ in range(2)]
+    row = lambda h: torch.zeros((1, h, 1, 64), dtype=torch.bfloat16)
+
+    def steps(cm):
+        for _ in range(20):
+            cm._append_resident(row(2), row(1), row(1), 1)
+
+    threads = [threading.Thread(target=steps, args=(cm,)) for cm in managers]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    shared = managers[0]._rc.d_q_loc == managers[1]._rc.d_q_loc
+    for cm in managers:
+        cm._resident = None                                # (nothing to give back)
+    assert shared and lib.calls == 40 and lib.overlaps == 0
