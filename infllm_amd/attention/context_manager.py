@@ -73,7 +73,7 @@ class _Buffers(dict):
 
 class _Units:
     """What the resident units of all managers take of a device's memory, and the pinned logs between managers."""
-    lock = threading.Lock()
+    lock = threading.RLock()  # (a manager that the interpreter collects while it holds the lock gives its share back then)
     used = {}                 # device index -> bytes
     logs = {}                 # (device index, ints) -> [(log, last sequence number written or on its way)]
     max_logs = 64             # logs kept per size
@@ -81,11 +81,11 @@ class _Units:
     @classmethod
     def take(cls, dev, n, limit):
         with cls.lock:
-            total = cls.used.get(dev, 0) + n
-            if total > limit:
-                return False
-            cls.used[dev] = total
-        return True
+            cls.used[dev] = cls.used.get(dev, 0) + n
+            if cls.used[dev] <= limit:
+                return True
+            cls.used[dev] -= n
+        return False
 
     @classmethod
     def give(cls, dev, n):

@@ -57,10 +57,26 @@ def test_calls_of_two_threads_on_one_stream_are_enqueued_one_after_the_other(one
         for _ in range(20):
             cm._append_resident(row(2), row(1), row(1), 1)
 
+    [cm._append_resident(row(2), row(1), row(1), 1) for cm in managers]          # binds them to the stream's workspaces
     threads = [threading.Thread(target=steps, args=(cm,)) for cm in managers]
     [t.start() for t in threads]
     [t.join() for t in threads]
     shared = managers[0]._rc.d_q_loc == managers[1]._rc.d_q_loc
     for cm in managers:
         cm._resident = None                                # (nothing to give back)
-    assert shared and lib.calls == 40 and lib.overlaps == 0
+    assert shared and lib.calls == 42 and lib.overlaps == 0
+
+
+def test_a_manager_may_be_collected_while_the_budget_is_looked_at():
+    """The interpreter runs a collected object's destructor wherever it allocates, also inside the budget's own sections."""
+    units, done = context_manager._Units, threading.Event()
+
+    def inside():
+        with units.lock:
+            units.give(99, 5)
+        done.set()
+
+    thread = threading.Thread(target=inside, daemon=True)
+    assert units.take(99, 5, 5) and not units.take(99, 1, 5)
+    thread.start()
+    assert done.wait(5) and units.used.pop(99) == 0
