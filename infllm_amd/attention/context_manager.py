@@ -77,6 +77,7 @@ class _Units:
     used = {}                 # device index -> bytes
     logs = {}                 # (device index, ints) -> [(log, last sequence number written or on its way)]
     max_logs = 64             # logs kept per size
+    lost = []                 # logs whose launches could not be waited for
 
     @classmethod
     def take(cls, dev, n, limit):
@@ -407,12 +408,20 @@ class ContextManager:
         if not handle:
             return
         self._lib.infllm_resident_state(handle, 0, self._state)
-        _Units.give_log(self._dev_index, self._log, int(self._state[9]))
-        _Units.give(self._dev_index, len(self._chunks) * self._chunk_bytes)
-        self._lib.infllm_resident_destroy(handle)
-        if len(self._streams) > 1:              # buffers go back to the allocator for the stream they were made on
-            torch.cuda.synchronize(self.device)
-        self._chunks, self._log = [], None
+        log, self._log = self._log, None
+        try:
+            # Work on several streams is waited for: the newest selection may be in the log while an older one, on another
+            # stream, is still to be written there; and the buffers go back to the allocator for the stream they were made on.
+            if len(self._streams) > 1:
+                torch.cuda.synchronize(self.device)
+            _Units.give_log(self._dev_index, log, int(self._state[9]))
+        except Exception:
+            _Units.lost.append(log)                        # (launches may still write to it: never handed out or freed)
+            raise
+        finally:
+            _Units.give(self._dev_index, len(self._chunks) * self._chunk_bytes)
+            self._lib.infllm_resident_destroy(handle)
+            self._chunks = []
 
     def _resident_books(self, wait):
         """The bookkeeping of the selections so far (wait: of all of them) into the counters."""

@@ -14,6 +14,12 @@ class Native:
     def __init__(self):
         self.open, self.overlaps, self.calls, self.guard = {}, 0, 0, threading.Lock()
 
+    def infllm_resident_state(self, manager, wait, state):
+        return 0
+
+    def infllm_resident_destroy(self, manager):
+        return 0
+
     def infllm_resident_append(self, manager, rc, stream):
         with self.guard:
             self.calls += 1
@@ -80,3 +86,29 @@ def test_a_manager_may_be_collected_while_the_budget_is_looked_at():
     assert units.take(99, 5, 5) and not units.take(99, 1, 5)
     thread.start()
     assert done.wait(5) and units.used.pop(99) == 0
+
+
+@pytest.mark.parametrize("streams,waits", [({1}, False), ({1, 2}, True)])
+def test_a_log_is_handed_on_when_every_stream_is_done_with_it(streams, waits, monkeypatch):
+    """With two streams the newest selection may have arrived while an older one is still to be written."""
+    order = []
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda dev=None: order.append("wait"))
+    monkeypatch.setattr(context_manager._Units, "give_log", lambda dev, log, seq: order.append((log, seq)))
+    cm = resident_manager(Native())
+    cm._streams, cm._chunk_bytes, cm._log, cm._state = streams, 0, "log", [0] * 9 + [12]
+    cm._drop_resident()
+    assert order == (["wait"] if waits else []) + [("log", 12)] and cm._log is None and cm._resident is None
+
+
+def test_a_log_that_cannot_be_waited_for_is_not_handed_on(monkeypatch):
+    def fails(dev=None):
+        raise RuntimeError("a capture is under way")
+
+    monkeypatch.setattr(torch.cuda, "synchronize", fails)
+    monkeypatch.setattr(context_manager._Units, "give_log", lambda *a: pytest.fail("handed on"))
+    monkeypatch.setattr(context_manager._Units, "lost", [])
+    cm = resident_manager(Native())
+    cm._streams, cm._chunk_bytes, cm._log, cm._state = {1, 2}, 0, "log", [0] * 9 + [12]
+    with pytest.raises(RuntimeError):
+        cm._drop_resident()
+    assert context_manager._Units.lost == ["log"] and cm._resident is None
