@@ -53,7 +53,9 @@ _SIDE_STREAM = None          # one process-wide side stream, like GLOBAL_STREAM 
 # (device, stream, geometry) -> the buffers of a call prepared in one go, shared by the managers that are alive
 _CALL_BUFFERS = weakref.WeakValueDictionary()
 _HOST_CHUNK_UNITS = 64       # units per pinned host allocation
-_UNIT_CHUNK = 64             # units per allocation of their home in HBM
+_UNIT_CHUNK = 64             # units per allocation of their home in HBM, at most ...
+_CHUNK_BYTES = 96 << 20      # ... fewer where that many would take more than this (a batch), but four at least
+_SPARE = 8                   # by default units do not take the last eighth of a device's memory
 _LOG_SLOTS = 256             # selections whose bookkeeping may be outstanding
 _MAX_SPLITS = 16             # key splits of one attention stage
 _NUM_CUS = 256               # MI355X
@@ -192,7 +194,8 @@ class ContextManager:
     local_group_blocks = None   # blocks of a prepared call per launch of the local stage (INFLLM_LOCAL_GROUP overrides it);
                                 # None: two where the host drives, else as many as pay
     resident_bytes = None       # HBM that the units of all managers of this process may take together on a device; None: a
-                                # quarter of it.  0 keeps units in pinned host memory (so does INFLLM_NO_RESIDENT=1).
+                                # quarter of it, and not the last eighth of what is free.  0 keeps units in pinned host
+                                # memory, max_cached_block of them on the device (so does INFLLM_NO_RESIDENT=1).
 
     def __init__(self, position_embedding, n_init, n_local, block_size, max_cached_block, topk, exc_block_size,
                  score_decay=None, fattn=False, repr_topk=1, cache_strategy="lru", chunk_topk_calc=None,
@@ -316,13 +319,33 @@ class ContextManager:
             return self.resident_bytes
         return torch.cuda.get_device_properties(self._dev_index).total_memory // 4
 
+    def _leaves_room(self, n):
+        """Whether the device still has memory for its other users once the units take n bytes more: units that found a home in
+        HBM are not moved out of it when an allocation of the caller fails.  A budget set by the caller is taken at its word."""
+        if self.resident_bytes is not None:
+            return True
+        free, total = torch.cuda.mem_get_info(self._dev_index)
+        if free - n >= total // _SPARE:
+            return True
+        return free + torch.cuda.memory_reserved(self._dev_index) - torch.cuda.memory_allocated(self._dev_index) - n >= total // _SPARE
+
+    @staticmethod
+    def _units_per_chunk(unit_bytes):
+        """The step in which a manager takes memory, also for its first unit (a batch of 8 in 32 layers of the reference's
+        geometry: 2 GiB, where 64 units a step would be 8, and a cache of 32 slots 4)."""
+        n = _UNIT_CHUNK
+        while n > 4 and n * unit_bytes > _CHUNK_BYTES:
+            n //= 2
+        return n
+
     def _resident_desc(self, D):
         d = ResidentDesc()
         d.B, d.H, d.Hkv, d.dim = self.num_units, self.unit_size, self.unit_size_kv, D
         d.n_local, d.n_init, d.block_size, d.exc = self.n_local, self.n_init, self.block_size, self.exc_block_size
         d.topk, d.repr_topk, d.max_cached = self.topk, self.repr_topk, self.max_cached_block
         d.max_splits, d.num_cus, d.call_tokens, d.group_blocks = _MAX_SPLITS, _NUM_CUS, self._call_tokens, getattr(self, "_local_group", 1)
-        d.max_pages, d.units_per_chunk, d.log_slots = self.max_pages, _UNIT_CHUNK, _LOG_SLOTS
+        unit_bytes = 2 * self.num_units * self.unit_size_kv * self.block_size * D * 2
+        d.max_pages, d.units_per_chunk, d.log_slots = self.max_pages, self._units_per_chunk(unit_bytes), _LOG_SLOTS
         d.ring_cap, d.init_cap = self.ring_cap, max(self.n_init, 1)
         return d
 
@@ -341,8 +364,9 @@ class ContextManager:
     def _init_resident(self):
         dev, B, topk = self.device, self.num_units, self.topk
         i32 = dict(dtype=torch.int32, device=dev)
-        self._chunks = []                       # homes of the units: [_UNIT_CHUNK, B, 2, Hkv, bs, D] each
-        self._chunk_bytes = _UNIT_CHUNK * self.unit_bytes
+        self._chunks = []                       # homes of the units: [_chunk_units, B, 2, Hkv, bs, D] each
+        self._chunk_units = self._units_per_chunk(self.unit_bytes)
+        self._chunk_bytes = self._chunk_units * self.unit_bytes
         self._chunk_host = (ctypes.c_uint64 * 16)()
         self._chunk_dev = torch.empty((16,), dtype=torch.int64, device=dev)
         self._ids = torch.empty((B, topk), **i32)
@@ -380,11 +404,11 @@ class ContextManager:
 
     def _add_chunks(self, n_units):
         """Homes for n_units units; False when the budget or the memory does not have them."""
-        while len(self._chunks) * _UNIT_CHUNK < n_units:
-            if not _Units.take(self._dev_index, self._chunk_bytes, self._resident_limit()):
+        while len(self._chunks) * self._chunk_units < n_units:
+            if not self._leaves_room(self._chunk_bytes) or not _Units.take(self._dev_index, self._chunk_bytes, self._resident_limit()):
                 return False
             try:
-                t = torch.empty((_UNIT_CHUNK, self.num_units, 2, self.unit_size_kv, self.block_size, self.head_width), dtype=torch.bfloat16,
+                t = torch.empty((self._chunk_units, self.num_units, 2, self.unit_size_kv, self.block_size, self.head_width), dtype=torch.bfloat16,
                                 device=self.device)
             except torch.OutOfMemoryError:
                 _Units.give(self._dev_index, self._chunk_bytes)
@@ -448,20 +472,20 @@ class ContextManager:
         """From here on the host drives (selections are to be recorded, or the units outgrew their budget): the state moves
         over as export_state / load_state move it, the policies stay, and the slots they hand out are filled."""
         policy, stats, length, timing = self.policy, self.stats, self.length, (self._timing_cap, self._timing_stride)
-        units, n = self._chunks, self.num_global_block
+        units, per, n = self._chunks, self._chunk_units, self.num_global_block
         state = self.export_state(with_units=False)
         state["units"] = None
         self._drop_resident()
         self.initialized, self.length = False, 0
-        self._load(state, resident=False, unit_at=lambda u: units[u // _UNIT_CHUNK][u % _UNIT_CHUNK])
+        self._load(state, resident=False, unit_at=lambda u: units[u // per][u % per])
         self._policy, self._stats = policy, stats
         for u, pol in enumerate(policy):
             if self.record_trace and pol.evicted_log is None:
                 pol.evicted_log = []
             self._caches[u] = pol.handle
             for unit, slot in pol.slot_of.items():
-                self.slab[u, slot] = _widen(units[unit // _UNIT_CHUNK][unit % _UNIT_CHUNK, u], self.dim_head) if self.head_width != units[0].shape[-1] \
-                    else units[unit // _UNIT_CHUNK][unit % _UNIT_CHUNK, u]
+                home = units[unit // per][unit % per, u]
+                self.slab[u, slot] = _widen(home, self.dim_head) if self.head_width != home.shape[-1] else home
         torch.cuda.synchronize(self.device)
         assert self.length == length and self.num_global_block == n
 
@@ -469,7 +493,7 @@ class ContextManager:
         """One append() call on resident units; None when the units no longer fit (nothing has been done then)."""
         rc, length = self._rc, self.length
         units = max(0, (length + n - self.n_init - self.n_local) // self.block_size)
-        if units > len(self._chunks) * _UNIT_CHUNK and not self._add_chunks(units):
+        if units > len(self._chunks) * self._chunk_units and not self._add_chunks(units):
             return None
         if units > self.reps.shape[1]:
             self._grow_reps(units)
@@ -690,7 +714,7 @@ class ContextManager:
         """Pinned host tensor [B, 2, Hkv, bs, D] of a carved unit (K at index 0, V at 1); a copy where the unit is resident in
         HBM, and for heads narrower than 128 one with the real dimensions picked out."""
         if self._resident:
-            t = self._chunks[unit // _UNIT_CHUNK][unit % _UNIT_CHUNK]
+            t = self._chunks[unit // self._chunk_units][unit % self._chunk_units]
             host = torch.empty(t.shape, dtype=t.dtype, pin_memory=True)
             return _narrow(host.copy_(t), self.dim_head) if t.shape[-1] != self.dim_head else host.copy_(t)
         self._finish_host_copies()
@@ -1111,9 +1135,9 @@ class ContextManager:
             self._grow_reps(n_units) if n_units > self.reps.shape[1] else None
             self.reps[:, :n_units] = wide(reps.view(B, n_units, H, D)).reshape(B, n_units, -1)
             if self._resident:
-                for u in range(0, n_units, _UNIT_CHUNK):
-                    n = min(_UNIT_CHUNK, n_units - u)
-                    self._chunks[u // _UNIT_CHUNK][:n] = wide(state["units"][u:u + n])
+                for u in range(0, n_units, self._chunk_units):
+                    n = min(self._chunk_units, n_units - u)
+                    self._chunks[u // self._chunk_units][:n] = wide(state["units"][u:u + n])
             else:
                 for u in range(n_units):
                     self._host_unit_addr(u)                        # allocates the pinned chunk

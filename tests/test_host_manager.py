@@ -39,7 +39,7 @@ def resident_manager(lib):
     cm.num_units, cm.unit_size, cm.unit_size_kv, cm.head_width, cm.dim_head = 1, 2, 1, 64, 64
     cm.length = cm.load_count = cm.num_global_block = 0
     cm._lib, cm._resident, cm._dev_index, cm.device, cm._layer = lib, cm, 0, torch.device("cpu"), None
-    cm._local_group, cm._part_rows2, cm._chunks, cm._call_scores, cm._call_stream = 1, 64, [], None, None
+    cm._chunk_units, cm._local_group, cm._part_rows2, cm._chunks, cm._call_scores, cm._call_stream = 4, 1, 64, [], None, None
     cm._streams, cm.reps = set(), torch.empty((1, 16, 128), dtype=torch.bfloat16)
     cm._rc = ResidentCall()
     cm._rc.max_tokens = 64
@@ -112,3 +112,30 @@ def test_a_log_that_cannot_be_waited_for_is_not_handed_on(monkeypatch):
     with pytest.raises(RuntimeError):
         cm._drop_resident()
     assert context_manager._Units.lost == ["log"] and cm._resident is None
+
+
+@pytest.mark.parametrize("free,reserved,allocated,budget,fits", [
+    (100, 0, 0, None, True), (12, 0, 0, None, False),              # of 100 chunks' memory: enough, and the last eighth of it
+    (2, 30, 5, None, True),                                        # ... with what the allocator holds and does not use
+    (2, 0, 0, 10, True),                                           # a budget of the caller's is taken at its word
+])
+def test_units_leave_memory_to_the_other_users_of_the_device(free, reserved, allocated, budget, fits, monkeypatch):
+    cm = resident_manager(Native())
+    cm._chunk_units, cm._chunk_bytes, cm.resident_bytes = 4, 4 * 2 * 16 * 64 * 2, budget
+    cm._chunk_host, cm._chunk_dev = (ctypes.c_uint64 * 16)(), torch.zeros((16,), dtype=torch.int64)
+    mem = cm._chunk_bytes
+    monkeypatch.setattr(context_manager._Units, "used", {})
+    monkeypatch.setattr(ContextManager, "_resident_limit", lambda self: 10 * mem)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda dev: (free * mem, 100 * mem))
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda dev: reserved * mem)
+    monkeypatch.setattr(torch.cuda, "memory_allocated", lambda dev: allocated * mem)
+    assert cm._add_chunks(7) == fits
+    assert len(cm._chunks) == (2 if fits else 0)
+    assert context_manager._Units.used.get(0, 0) == len(cm._chunks) * mem
+    cm._resident = None
+
+
+def test_a_batch_takes_its_memory_in_smaller_steps():
+    unit = 2 * 8 * 128 * 128 * 2                                    # one row's unit of the reference's geometry: 512 KiB
+    steps = {b: ContextManager._units_per_chunk(b * unit) for b in (1, 2, 8, 64, 1024)}
+    assert steps == {1: 64, 2: 64, 8: 16, 64: 4, 1024: 4}
