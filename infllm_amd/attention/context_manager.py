@@ -197,6 +197,9 @@ class ContextManager:
                                 # quarter of it, and not the last eighth of what is free.  0 keeps units in pinned host
                                 # memory, max_cached_block of them on the device (so does INFLLM_NO_RESIDENT=1).
 
+    rows_by_token = False       # set for the next append() by a caller that takes a token's rows next to each other (the view
+                                # [B, H, n, D] of a tensor [B, n, H, D], where the path has one to give): spares it a copy
+
     def __init__(self, position_embedding, n_init, n_local, block_size, max_cached_block, topk, exc_block_size,
                  score_decay=None, fattn=False, repr_topk=1, cache_strategy="lru", chunk_topk_calc=None,
                  async_global_stream=False, pin_memory=False, faiss=False, perhead=False):
@@ -489,7 +492,7 @@ class ContextManager:
         torch.cuda.synchronize(self.device)
         assert self.length == length and self.num_global_block == n
 
-    def _append_resident(self, q, k, v, n):
+    def _append_resident(self, q, k, v, n, by_token=False):
         """One append() call on resident units; None when the units no longer fit (nothing has been done then)."""
         rc, length = self._rc, self.length
         units = max(0, (length + n - self.n_init - self.n_local) // self.block_size)
@@ -505,13 +508,12 @@ class ContextManager:
             self._call_scores = torch.empty((-(-rc.max_tokens // self.exc_block_size), self.num_units, cols), dtype=torch.float32, device=self.device)
             rc.d_call_scores, rc.scores_cols = self._call_scores.data_ptr(), cols
         B, H, D = self.num_units, self.unit_size, self.head_width
-        # rows of a token next to each other, as the layer's output projection takes them
-        out = torch.empty((B, n, H, D), dtype=torch.bfloat16, device=q.device)
+        out = torch.empty((B, n, H, D) if by_token else (B, H, n, D), dtype=torch.bfloat16, device=q.device)
         rc.d_q, rc.d_k, rc.d_v, rc.d_out, rc.n = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), n
         rc.q_sb, rc.q_sh, rc.q_sl, _ = q.stride()
         rc.k_sb, rc.k_sh, rc.k_sl, _ = k.stride()
         rc.v_sb, rc.v_sh, rc.v_sl, _ = v.stride()
-        rc.o_sb, rc.o_sl, rc.o_sh = n * H * D, H * D, D
+        rc.o_sb, rc.o_sl, rc.o_sh = (n * H * D, H * D, D) if by_token else (n * H * D, D, n * D)
         with self._call_buf.lock:
             status = self._lib.infllm_resident_append(self._resident, self._rc_ref, stream)
         if status:
@@ -522,7 +524,7 @@ class ContextManager:
         self.cursor = self.init_len + units * self.block_size
         if self.cache_strategy == "lru":
             self.load_count += -(-n // self.exc_block_size)
-        return out.permute(0, 2, 1, 3)
+        return out.permute(0, 2, 1, 3) if by_token else out
 
     def _bind_resident_buffers(self, stream):
         """Workspaces of a call: dead between append() calls, so the managers that work on one stream share one set; the set's
@@ -965,6 +967,8 @@ class ContextManager:
 
     # ----------------------------------------------------------------- append
     def append(self, local_q, local_k, local_v, global_q, global_k, global_v):
+        """The next tokens of the stream: their output rows [B, H, n, D], contiguous (unless ``rows_by_token`` was set)."""
+        by_token, self.rows_by_token = self.rows_by_token, False
         if not (global_q is local_q and global_k is local_k and global_v is local_v):
             if not (global_q.data_ptr() == local_q.data_ptr() and global_k.data_ptr() == local_k.data_ptr()
                     and global_v.data_ptr() == local_v.data_ptr()):
@@ -1001,7 +1005,7 @@ class ContextManager:
             return t if s3 == 1 and not (s0 | s1 | s2) & 7 and not t.data_ptr() & 15 else t.contiguous()
         q, k, v = rows16(q), rows16(k), rows16(v)
         if self._resident:
-            out = self._append_resident(q, k, v, input_length)
+            out = self._append_resident(q, k, v, input_length, by_token)
             if out is not None:
                 out = self._own_width(out)
                 return out.reshape(batch_size, heads, input_length, -1) if self.perhead else out

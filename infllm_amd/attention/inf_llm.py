@@ -31,6 +31,7 @@ def inf_llm_forward(n_local, n_init, topk, block_size, max_cached_block, exc_blo
                 score_decay, fattn, repr_topk, cache_strategy, chunk_topk_calc, async_global_stream,
                 pin_memory, faiss, perhead)
 
+        past_key_value.rows_by_token = True        # as the output projection below reads them
         o = past_key_value.append(h_q, h_k, h_v, h_q, h_k, h_v)
 
         o = o.view(batch_size, num_heads, len_q, dim_head).permute(0, 2, 1, 3)

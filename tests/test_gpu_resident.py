@@ -133,3 +133,27 @@ def test_managers_of_two_threads_on_one_stream():
     [t.join() for t in threads]
     torch.cuda.synchronize()
     assert torch.equal(got[0], alone[0]) and torch.equal(got[1], alone[1])
+
+
+@pytest.mark.parametrize("driven", ["resident", "host"])
+@pytest.mark.parametrize("calls,kw", [([500, 1, 130], dict(SMALL)), ([500, 1], dict(SMALL, dim=32)), ([500, 1], dict(SMALL, perhead=True))],
+                         ids=["128", "32", "perhead"])
+def test_append_returns_contiguous_rows_on_either_path(driven, calls, kw, monkeypatch):
+    """[B, H, n, D], which a caller may view with heads and tokens in one; the attention type takes the rows by token and gives
+    the same ones."""
+    from infllm_amd.attention import ContextManager, inf_llm_forward, RotaryEmbeddingESM
+    if driven == "host":
+        monkeypatch.setattr(ContextManager, "resident_bytes", 0)
+    H, Hkv, B, dim = 4, 2, 2, kw.get("dim", 128)
+    q, k, v = (t.cuda() for t in make_stream(sum(calls), H, Hkv, 7, B=B, D=dim))
+    outs = feed(new_manager(1e4, **kw), q, k, v, calls)
+    for n, o in zip(calls, outs):
+        assert o.shape == (B, H, n, dim) and o.is_contiguous() and o.view(B, H * n, dim).shape == (B, H * n, dim)
+    forward = inf_llm_forward(**{n: x for n, x in kw.items() if n != "dim"}, fattn=False)
+    past, pos, same = None, 0, lambda t: t
+    rope = RotaryEmbeddingESM(dim, base=1e4, device="cuda")
+    for n, o in zip(calls, outs):
+        rows = [t[:, :, pos:pos + n].transpose(1, 2).reshape(B, n, -1) for t in (q, k, v)]
+        got, past = forward(None, rows[0], rows[1], rope, True, past, same, same, lambda _: rows[2], same, dim, H, Hkv)
+        assert torch.equal(got, o.transpose(1, 2).reshape(B, n, -1)) and not past.rows_by_token
+        pos += n
