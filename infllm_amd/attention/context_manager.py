@@ -423,12 +423,20 @@ class ContextManager:
                 grown[:n] = self._chunk_host[:]
                 table = torch.empty((2 * n,), dtype=torch.int64, device=self.device)
                 table[:n] = self._chunk_dev
+                self._retire(self._chunk_dev)
                 self._chunk_host, self._chunk_dev = grown, table
                 self._rc.h_chunks, self._rc.d_chunks = ctypes.addressof(grown), table.data_ptr()
             self._chunk_host[n] = t.data_ptr()
             self._chunk_dev[n].fill_(t.data_ptr())
         self._rc.n_chunks = len(self._chunks)
         return True
+
+    @staticmethod
+    def _retire(*buffers):
+        """Buffers that are replaced: a stream other than the one they were made on may still have launches that use them."""
+        for t in buffers:
+            if t is not None and t.is_cuda:
+                t.record_stream(torch.cuda.current_stream(t.device))
 
     def _drop_resident(self):
         handle, self._resident = getattr(self, "_resident", None), None
@@ -505,6 +513,7 @@ class ContextManager:
             self._bind_resident_buffers(stream)
         if n > 1 and units > self.topk and (self._call_scores is None or self._call_scores.shape[2] < units):
             cols = max(-(-units // 256) * 256, 2 * (self._call_scores.shape[2] if self._call_scores is not None else 0))
+            self._retire(self._call_scores)
             self._call_scores = torch.empty((-(-rc.max_tokens // self.exc_block_size), self.num_units, cols), dtype=torch.float32, device=self.device)
             rc.d_call_scores, rc.scores_cols = self._call_scores.data_ptr(), cols
         B, H, D = self.num_units, self.unit_size, self.head_width
@@ -953,6 +962,7 @@ class ContextManager:
         grown[:, :N] = self.reps[:, :N]
         scores = torch.empty((B, rows), dtype=torch.float32, device=self.device)
         scores[:, :N] = self.unit_scores[:, :N]          # scores prepared ahead for the next block
+        self._retire(self.reps, self.unit_scores)
         self.reps, self.unit_scores = grown, scores
         self._bind_resident_reps() if self._resident else self._bind_reps()
 
@@ -1054,6 +1064,7 @@ class ContextManager:
                         blocks, cols = -(-self._call_tokens // exc), self.num_global_block + (call_end - st) // self.block_size + 2
                         if self._call_scores is None or self._call_scores.shape[2] < cols or self._call_scores.shape[0] < blocks:
                             cols = max(-(-cols // 256) * 256, 2 * (self._call_scores.shape[2] if self._call_scores is not None else 0))
+                            self._retire(self._call_scores)
                             self._call_scores = torch.empty((blocks, self.num_units, cols), dtype=torch.float32, device=self.device)
                         fa.d_call_scores, fa.call_scores_cols = self._call_scores.data_ptr(), self._call_scores.shape[2]
                         check(self._lib.infllm_call_front(self._layer, self._fa_ref, self._main_raw), "infllm_call_front")

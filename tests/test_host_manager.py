@@ -139,3 +139,29 @@ def test_a_batch_takes_its_memory_in_smaller_steps():
     unit = 2 * 8 * 128 * 128 * 2                                    # one row's unit of the reference's geometry: 512 KiB
     steps = {b: ContextManager._units_per_chunk(b * unit) for b in (1, 2, 8, 64, 1024)}
     assert steps == {1: 64, 2: 64, 8: 16, 64: 4, 1024: 4}
+
+
+def test_replaced_buffers_wait_for_the_stream_that_uses_them(one_stream, monkeypatch):
+    """A manager that has moved to another stream: the allocator would hand a replaced buffer out again in the order of the
+    stream it was made on, while launches of the other one still read it."""
+    class Buffer:
+        is_cuda, device, streams = True, "cuda:0", None
+
+        def __init__(self, *shape):
+            self.t, self.shape = torch.zeros(shape, dtype=torch.bfloat16), torch.Size(shape)
+
+        def __getitem__(self, i):
+            return self.t[i]
+
+        def record_stream(self, stream):
+            self.streams = stream
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev=None: "the call's stream")
+    cm = resident_manager(Native())
+    monkeypatch.setattr(cm, "_add_chunks", lambda n: True)
+    cm.length, cm.reps, cm.unit_scores, cm._call_scores = 400, Buffer(1, 16, 128), Buffer(1, 16), Buffer(1, 1, 8)
+    old = cm.reps, cm.unit_scores, cm._call_scores
+    row = lambda h: torch.zeros((1, h, 2, 64), dtype=torch.bfloat16)
+    cm._append_resident(row(2), row(1), row(1), 2)
+    assert cm.reps.shape[1] >= 21 and [b.streams for b in old] == ["the call's stream"] * 3
+    cm._resident = None
