@@ -232,7 +232,6 @@ class ContextManager:
         self._policy = []
         self._layer = None
         self._resident = None         # native handle while the units are resident in HBM
-        self._base_stats = None
         self._timing_cap, self._timing_stride = 0, 1
         self._mass_units = None                # lru-s: selections of the block whose unit masses are still on the device
         global _SIDE_STREAM
@@ -461,9 +460,8 @@ class ContextManager:
     def _resident_books(self, wait):
         """The bookkeeping of the selections so far (wait: of all of them) into the counters."""
         check(self._lib.infllm_resident_state(self._resident, 1 if wait else 0, self._state), "infllm_resident_state")
-        st, base = self._state, self._base_stats
         for i, name in ((4, "blocks"), (5, "hits"), (6, "misses"), (7, "evictions")):
-            self._stats[name] = int(st[i]) + (base[name] if base else 0)
+            self._stats[name] = int(self._state[i])
 
     @property
     def stats(self):
