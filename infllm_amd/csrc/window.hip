@@ -163,8 +163,13 @@ int launch_stage_rows(StageJob &j, int dim, void *stream) {
 // 5 us; the smallest estimate wins.  Equal workgroups run in rounds; where the first queries see few keys (a prompt's first
 // call) the short workgroups fill up behind the long ones, which start first, so that the launch lasts as long as its longest
 // or as its sum, and a quarter of its longest more where the chip does not hold it at once (causal, one call of 32 heads:
-// 1,500 tokens 60 -> 51 us and 2,048 tokens 77.7 -> 71.7 with two splits, where rounds said one).  max_parts: splits that the partial rows have
-// room for.
+// 1,500 tokens 60 -> 51 us and 2,048 tokens 77.7 -> 71.7 with two splits, where rounds said one).
+// The constants are those of heads of 128.  Heads of 64 (a CU holds two of their workgroups) and the operator's stages take
+// them too: against the best of 1, 2, 3, 4, 6 and 8 splits forced, whole passes - causal prompts of 1,500 / 2,500 / 4,001 tokens,
+// 32 heads of 128: 71.3 / 110.3 / 179.2 us by the rule, 68.5 / 109.8 / 178.6 best; 36 heads of 64: 66.2 / 113.8 / 178.4, 64.2 /
+// 113.7 / 177.2 best; the operator's two stages of 300 / 512 / 900 queries: 53.3 / 57.6 / 80.7, 52.5 / 57.8 / 82.8 best, 36 heads of
+// 64 in rows of 128 120.5 / 124.9 / 178.8, 119.8 / 124.0 / 178.8 best; of 64 queries 58.9 by the rule (11 splits), 52.6 best (6).
+// max_parts: splits that the partial rows have room for.
 int infllm_attn_splits(int64_t wgs, int64_t tiles, int32_t max_parts, double mean_tiles) {
     const bool equal = mean_tiles > 0.9 * (double)tiles;
     int best = 1;
