@@ -12,7 +12,8 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HOT = ("attn_stage_kernel", "local_score_kernel", "retrieve_fused_kernel", "unit_scores_rows_kernel", "unit_scores_queries_kernel",
-       "call_rank_kernel", "ingest_kernel")
+       "call_rank_kernel", "ingest_kernel", "carve_score_kernel", "decode_attn_kernel", "stage_rows_kernel", "rank_kernel", "decode_finish_kernel",
+       "attn_merge")
 
 
 def _hipcc():
@@ -22,7 +23,7 @@ def _hipcc():
     pytest.skip("no hipcc")
 
 
-@pytest.mark.parametrize("source", ["attn.hip", "score.hip", "retrieve.hip", "ingest.hip"])
+@pytest.mark.parametrize("source", ["attn.hip", "score.hip", "retrieve.hip", "ingest.hip", "decode.hip", "window.hip", "resident.hip"])
 def test_hot_kernels_keep_their_registers(source, tmp_path):
     cmd = [_hipcc(), "--offload-arch=gfx950", "-O3", "-std=c++17", "-c", "--offload-device-only", "-Xclang", "-target-feature", "-Xclang",
            "-packed-fp32-ops", "-Rpass-analysis=kernel-resource-usage", os.path.join(ROOT, "infllm_amd", "csrc", source), "-o",
@@ -46,3 +47,5 @@ def test_hot_kernels_keep_their_registers(source, tmp_path):
         assert v.get("VGPRs Spill") == 0 and v.get("ScratchSize [bytes/lane]") == 0, (k, v)
     if source == "attn.hip":                   # 8 waves per workgroup, one workgroup per CU: two waves per SIMD need <= 256 registers
         assert all(v["Occupancy [waves/SIMD]"] >= 2 for k, v in hot.items()), hot
+    if source == "decode.hip":                 # two workgroups of four waves per CU and more in flight: three waves per SIMD
+        assert all(v["Occupancy [waves/SIMD]"] >= 3 for k, v in hot.items()), hot

@@ -49,6 +49,27 @@ def test_struct_layouts_match_header_sizes():
     assert ctypes.sizeof(_lib.BatchDesc) == 6 * 8 + 8 + 2 * 4
 
 
+def test_struct_layouts_match_the_header_field_by_field(tmp_path):
+    """Every argument block as the C compiler lays it out: sizes, and the place of every field by its name."""
+    import ctypes
+    import subprocess
+    from infllm_amd.attention import _sink_window
+    text = open(os.path.join(ROOT, "include", "infllm_hip.h")).read()
+    names = re.findall(r"\}\s*(infllm_[a-z_]+)\s*;", text)
+    bound = {"infllm_" + re.sub(r"(?<=[a-z])(?=[A-Z])", "_", n).lower(): t for n, t in vars(_lib).items()
+             if isinstance(t, type) and issubclass(t, ctypes.Structure) and t is not ctypes.Structure}
+    assert set(bound) == set(names), set(bound) ^ set(names)
+    lines = ["#include <stddef.h>", '#include "infllm_hip.h"']
+    for name, t in bound.items():
+        lines.append(f"_Static_assert(sizeof({name}) == {ctypes.sizeof(t)}, \"{name}\");")
+        lines += [f"_Static_assert(offsetof({name}, {f[0]}) == {getattr(t, f[0]).offset}, \"{name}.{f[0]}\");" for f in t._fields_]
+    source = tmp_path / "layout.c"
+    source.write_text("\n".join(lines))
+    p = subprocess.run(["gcc", "-std=c11", "-fsyntax-only", "-I", os.path.join(ROOT, "include"), str(source)], capture_output=True, text=True)
+    assert p.returncode == 0, p.stderr[:2000]
+    assert _sink_window._ARGS.size == ctypes.sizeof(_lib.WindowArgs)              # packed by format instead
+
+
 @pytest.mark.parametrize("strategy", ["lru", "fifo"])
 def test_cache_policy_equals_oracle_model(strategy):
     rng = random.Random(5)
