@@ -1,4 +1,4 @@
-"""Rows of heads narrower than the 128 dimensions the gfx950 kernels are built for.
+"""Rows of heads narrower than the 128 dimensions that every gfx950 kernel here takes.
 
 MiniCPM-2B has head_dim 64 (the reference ships config/minicpm-inf-llm.yaml for it, and its operators take any
 head_dim up to 128: torch_impl.py is shape-agnostic, triton_impl.py:412 lists 16 / 32 / 64 / 128).  Such rows run
@@ -7,8 +7,12 @@ representative's score or to an output row, so only the softmax scale 1/sqrt(D) 
 
 Where the kernel applies RoPE itself (the prologue, infllm_rope_rows) the two halves of a row go to dimensions
 [0, D/2) and [64, 64 + D/2): the rotation pairs dimension d with d + D/2 (rope.py:31-33), which are d and d + 64 in
-the wide row - the pairing the kernels use - and the frequencies of the unused slots are zero.  Twice the bytes and
-flops a kernel built for 64 would need: a way to run such models, not a fast path.
+the wide row - the pairing the kernels use - and the frequencies of the unused slots are zero.
+
+Heads of 64 travel in rows of their own where there are kernels for them: the sliding-window and causal types
+(_sink_window.py) and the streaming memory with its units in HBM (ContextManager, head_width 64).  Widened rows are for
+every other width, for the memory that the host drives, and (plainly padded, no rotation being involved) for the
+multi-stage operator, at twice the bytes and flops of a kernel built for 64.
 """
 import torch
 

@@ -255,7 +255,7 @@ def score_topk_queries(reps, n, qbars, k, scores, idx):
                                                qbars.shape[0], k, scores.data_ptr(), scores.stride(0), idx.data_ptr(), idx.stride(0),
                                                _stream())
     if rc == 1:
-        raise ValueError(f"score_topk_queries: rows of {reps.shape[1]} elements (supported: 512, 1024, 2048, 4096)")
+        raise ValueError(f"score_topk_queries: rows of {reps.shape[1]} elements (supported: multiples of 8 up to 4608)")
     check(rc, "infllm_score_topk_queries")
 
 

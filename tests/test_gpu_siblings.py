@@ -65,7 +65,7 @@ def test_sink_window_types_follow_oracle(kind, calls, n_local, n_init):
 
 @pytest.mark.parametrize("kind", ["stream-llm", "infinite-lm", "origin"])
 def test_sibling_types_with_heads_of_64(kind, monkeypatch):
-    """head_dim 64 through the same three types: rows are widened for the kernels and cut back (attention/_rows.py)."""
+    """head_dim 64 through the same three types, in rows of their own width."""
     import sys
     from infllm_amd.attention import ATTN_FORWRAD
     monkeypatch.setattr(sys.modules[__name__], "D", 64)
