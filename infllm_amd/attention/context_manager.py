@@ -982,13 +982,16 @@ class ContextManager:
                     and global_v.data_ptr() == local_v.data_ptr()):
                 raise ValueError("local and global q/k/v must be the same tensors (as inf_llm_forward passes them)")
         q, k, v = local_q, local_k, local_v
-        if q.dtype != torch.bfloat16:
-            raise TypeError(f"the HIP path computes in bfloat16; got {q.dtype}")
-        assert q.dim() == 4 and q.is_cuda
+        bf, dev = torch.bfloat16, q.device                      # (the native calls take addresses: nothing behind here checks them)
+        if q.dtype is not bf or k.dtype is not bf or v.dtype is not bf:
+            raise TypeError(f"the HIP path computes in bfloat16; got {q.dtype}, {k.dtype}, {v.dtype}")
+        if k.device != dev or v.device != dev:
+            raise ValueError(f"q, k and v must be on one device, got {dev}, {k.device}, {v.device}")
         batch_size, _, input_length, width = q.shape
-        for t in (k, v):
-            t0, _, t2, t3 = t.shape
-            assert t0 == batch_size and t2 == input_length and t3 == width
+        kv_shape = k.shape
+        t0, _, t2, t3 = kv_shape
+        assert t0 == batch_size and t2 == input_length and t3 == width and v.shape == kv_shape, "q, keys and values differ in shape"
+        assert q.is_cuda
         if self.perhead:                                        # context_manager.py:690-704
             heads, heads_kv = q.size(1), k.size(1)
             rep = lambda t: (t.reshape(batch_size, heads_kv, 1, input_length, -1)

@@ -165,3 +165,20 @@ def test_replaced_buffers_wait_for_the_stream_that_uses_them(one_stream, monkeyp
     cm._append_resident(row(2), row(1), row(1), 2)
     assert cm.reps.shape[1] >= 21 and [b.streams for b in old] == ["the call's stream"] * 3
     cm._resident = None
+
+
+@pytest.mark.parametrize("k,v,error", [
+    (((1, 2, 5, 128), torch.half, "cpu"), ((1, 2, 5, 128), torch.half, "cpu"), TypeError),
+    (((1, 2, 5, 128), torch.bfloat16, "cpu"), ((1, 2, 5, 128), torch.float8_e4m3fn, "cpu"), TypeError),
+    (((1, 2, 5, 128), torch.bfloat16, "meta"), ((1, 2, 5, 128), torch.bfloat16, "cpu"), ValueError),
+    (((1, 2, 5, 128), torch.bfloat16, "cpu"), ((1, 1, 5, 128), torch.bfloat16, "cpu"), AssertionError),
+])
+def test_keys_and_values_that_would_be_read_out_of_range_are_refused(k, v, error, monkeypatch):
+    """another type, device or head count than the queries and keys have (before anything is set up or launched)"""
+    cm = ContextManager.__new__(ContextManager)
+    cm.perhead, cm.initialized = False, False
+    monkeypatch.setattr(ContextManager, "_init", lambda *a: pytest.fail("accepted"))
+    q = torch.zeros((1, 4, 5, 128), dtype=torch.bfloat16)
+    k, v = (torch.zeros(shape, dtype=dtype, device=device) for shape, dtype, device in (k, v))
+    with pytest.raises(error, match=None if error is not AssertionError else "shape"):
+        cm.append(q, k, v, q, k, v)
