@@ -218,6 +218,17 @@ def test_constructor_contract():
     assert callable(fwd)
 
 
+@pytest.mark.parametrize("k,v", [((1, 2, 9, 128), (1, 2, 9, 128)), ((2, 2, 9, 128), (2, 2, 8, 128)), ((2, 2, 9, 128), (2, 1, 9, 128)),
+                                 ((2, 3, 9, 128), (2, 3, 9, 128)), ((2, 2, 9, 64), (2, 2, 9, 64)), ((2, 2, 9, 128), (2, 2, 9, 64))])
+def test_the_operator_refuses_keys_and_values_that_do_not_fit_its_queries(k, v):
+    """(batch, lengths, head counts, widths: the stage would read them out of range)"""
+    from infllm_amd.attention.dot_production_attention import get_multi_stage_dot_production_attention
+    q = torch.zeros((2, 4, 5, 128), dtype=torch.bfloat16)
+    attn = get_multi_stage_dot_production_attention(False)[0](q.shape, q.dtype, q.device)
+    with pytest.raises(ValueError, match="do not fit"):
+        attn.append(q, torch.zeros(k, dtype=torch.bfloat16), torch.zeros(v, dtype=torch.bfloat16), end=True)
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "absent.so"))
