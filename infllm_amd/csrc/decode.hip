@@ -236,7 +236,7 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
 #pragma unroll
         for (int w = 0; w < kDecWaves; ++w)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) den += sl[w][r][h] * (sm[w][r][h] == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((sm[w][r][h] - mx) * scale));
+            for (int r = 0; r < 4; ++r) den += sm[w][r][h] == -INFINITY ? sl[w][r][h] : sl[w][r][h] * __builtin_amdgcn_exp2f((sm[w][r][h] - mx) * scale);
 #pragma unroll
         for (int w = 0; w < kDecWaves; ++w)
 #pragma unroll
