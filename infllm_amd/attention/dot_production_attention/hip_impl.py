@@ -35,13 +35,13 @@ class HipMultiStageDotProductionAttention(MultiStageDotProductionAttention):
 
     def append(self, q, k, v, sliding_window=None, complement_sliding_window=False, end=False, get_score=False,
                *args, **kwargs):
-        assert tuple(q.shape) == self.q_shape
+        assert q.shape == self.q_shape
         assert not self.end, "append after end"
-        d = q.shape[-1]
-        if k.dim() != 4 or k.shape != v.shape or k.shape[0] != q.shape[0] or k.shape[3] != d or k.shape[1] == 0 or q.shape[1] % k.shape[1]:
-            raise ValueError(f"keys {tuple(k.shape)} and values {tuple(v.shape)} do not fit queries {tuple(q.shape)}")    # (read by address)
-        if k.device != q.device or v.device != q.device:
-            raise ValueError(f"q, k and v must be on one device, got {q.device}, {k.device}, {v.device}")
+        (batch, heads, _, d), shape, dev = self.q_shape, k.shape, q.device
+        if len(shape) != 4 or v.shape != shape or shape[0] != batch or shape[3] != d or shape[1] == 0 or heads % shape[1]:
+            raise ValueError(f"keys {tuple(shape)} and values {tuple(v.shape)} do not fit queries {self.q_shape}")      # (read by address)
+        if k.device != dev or v.device != dev:
+            raise ValueError(f"q, k and v must be on one device, got {dev}, {k.device}, {v.device}")
         if d < ops.HEAD_DIM:
             q, k, v = (F.pad(t, (0, ops.HEAD_DIM - d)) for t in (q, k, v))
         q, k, v = ops._bf16_4d(q, "q"), ops._bf16_4d(k, "k"), ops._bf16_4d(v, "v")
