@@ -125,6 +125,7 @@ def test_units_leave_memory_to_the_other_users_of_the_device(free, reserved, all
     cm._chunk_host, cm._chunk_dev = (ctypes.c_uint64 * 16)(), torch.zeros((16,), dtype=torch.int64)
     mem = cm._chunk_bytes
     monkeypatch.setattr(context_manager._Units, "used", {})
+    monkeypatch.setattr(context_manager._Units, "asked", {})
     monkeypatch.setattr(ContextManager, "_resident_limit", lambda self: 10 * mem)
     monkeypatch.setattr(torch.cuda, "mem_get_info", lambda dev: (free * mem, 100 * mem))
     monkeypatch.setattr(torch.cuda, "memory_reserved", lambda dev: reserved * mem)
@@ -133,6 +134,24 @@ def test_units_leave_memory_to_the_other_users_of_the_device(free, reserved, all
     assert len(cm._chunks) == (2 if fits else 0)
     assert context_manager._Units.used.get(0, 0) == len(cm._chunks) * mem
     cm._resident = None
+
+
+def test_the_driver_is_asked_again_when_what_it_granted_is_used_up(monkeypatch):
+    cm, asked = resident_manager(Native()), []
+    monkeypatch.setattr(context_manager._Units, "asked", {})
+    monkeypatch.setattr(context_manager, "_ASK_BYTES", 100)
+    left = [1000, 1000, 200, 120]
+
+    def info(dev):
+        asked.append(dev)
+        return left[len(asked) - 1], 800                            # an eighth: 100
+
+    monkeypatch.setattr(torch.cuda, "mem_get_info", info)
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda dev: 0)
+    monkeypatch.setattr(torch.cuda, "memory_allocated", lambda dev: 0)
+    cm.resident_bytes, cm._resident = None, None
+    assert [cm._leaves_room(40) for _ in range(9)] == [True] * 8 + [False]      # asked at the 1st, 4th, 7th (60 to spare) and 9th
+    assert len(asked) == 4
 
 
 def test_a_batch_takes_its_memory_in_smaller_steps():
