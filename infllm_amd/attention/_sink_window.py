@@ -26,7 +26,7 @@ import threading
 import torch
 
 from .. import _lib
-from ..ops import HEAD_DIM, _stream
+from ..ops import HEAD_DIM, _stream, rows16
 from ._rows import check_head_dim, narrow, wide_inv_freq, widen
 
 _KINDS = {"origin": 0, "stream-llm": 1, "infinite-lm": 2}
@@ -68,20 +68,11 @@ class _Room:
         return True
 
 
-def _rows16(t):
-    """rows the kernels can read: unit stride inside a row, 16-byte alignment"""
-    *outer, inner = t.stride()
-    odd = 0
-    for s in outer:
-        odd |= s
-    return t if inner == 1 and not odd & 7 and not t.data_ptr() & 15 else t.contiguous()
-
-
 def _cache_rows(t, dim):
     """(a cached tensor as the native call takes it: rows next to each other, its batch and head strides)"""
     sb, sh, sl, inner = t.stride()
     if inner != 1 or sl != dim or (sb | sh) & 7 or t.data_ptr() & 15:
-        t = t.contiguous()
+        t = t.clone(memory_format=torch.contiguous_format)
         sb, sh, _, _ = t.stride()
     return t, sb, sh
 
@@ -90,7 +81,7 @@ def _heads(x, batch, length, heads, dim):
     """(tensor that is kept alive, batch, head and row strides) of projected rows [batch, length, heads * dim]"""
     if x.shape != (batch, length, heads * dim):
         x = x.view(batch, length, heads * dim)
-    x = _rows16(x)
+    x = rows16(x)
     return x, x.stride(0), dim, x.stride(1)
 
 
@@ -158,7 +149,8 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
             cached_k, cached_v = widen(old_k, dim_head), widen(old_v, dim_head)
             raw_old = None if raw_old is None else widen(raw_old, dim_head)
         if raw_old is not None:
-            raw_old = raw_old.contiguous()
+            if not raw_old.is_contiguous() or raw_old.data_ptr() & 15:
+                raw_old = raw_old.clone(memory_format=torch.contiguous_format)
             raw_rows = raw_old.size(2)
     rows_all, len_k = rows_old + n_new, seen + n_new
     bf = dict(dtype=torch.bfloat16, device=dev)

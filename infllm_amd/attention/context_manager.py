@@ -45,7 +45,7 @@ import torch
 
 from .. import _lib
 from .._lib import BackArgs, FrontArgs, LayerDesc, ResidentCall, ResidentDesc, check
-from ..ops import HEAD_DIM, KEY_TILE, current_stream
+from ..ops import HEAD_DIM, KEY_TILE, current_stream, rows16
 
 from ._rows import check_head_dim, narrow as _narrow, wide_inv_freq, widen as _widen
 
@@ -1020,9 +1020,6 @@ class ContextManager:
             q, k, v = _widen(q, self.dim_head), _widen(k, self.dim_head), _widen(v, self.dim_head)
         assert q.shape[:2] == (self.num_units, self.unit_size) and k.shape[1] == self.unit_size_kv
 
-        def rows16(t):          # rows must be contiguous and 16-byte aligned for the vector loads
-            s0, s1, s2, s3 = t.stride()
-            return t if s3 == 1 and not (s0 | s1 | s2) & 7 and not t.data_ptr() & 15 else t.contiguous()
         q, k, v = rows16(q), rows16(k), rows16(v)
         if self._resident:
             out = self._append_resident(q, k, v, input_length, by_token)

@@ -52,13 +52,21 @@ def _need(cond, msg):
         raise ValueError(msg)
 
 
+def rows16(t):
+    """The tensor as kernels can read it with 16-byte loads: unit stride inside a row, every other stride and the address whole
+    multiples of 16 bytes.  Else a copy - a clone, not contiguous(), which hands a contiguous tensor back however it is aligned."""
+    *outer, inner = t.stride()
+    odd = 0
+    for s in outer:
+        odd |= s
+    return t if inner == 1 and not odd & 7 and not t.data_ptr() & 15 else t.clone(memory_format=torch.contiguous_format)
+
+
 def _bf16_4d(t, name, dims=(HEAD_DIM,)):
     _need(t.is_cuda, f"{name} must be a GPU tensor")
     _need(t.dtype == torch.bfloat16, f"{name} must be bfloat16 (the HIP path computes in bf16), got {t.dtype}")
     _need(t.dim() == 4 and t.shape[-1] in dims, f"{name} must be [B, heads, len, {dims[-1]}], got {tuple(t.shape)}")
-    if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:-1]):
-        t = t.contiguous()
-    return t
+    return rows16(t)
 
 
 def ingest(q, k, v, pos0, glb_pos, inv_freq, distance_scale, ring_k_raw, ring_k_rot, ring_v, ring_score, q_loc, q_glb,

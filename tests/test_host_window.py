@@ -135,3 +135,34 @@ def test_which_calls_write_behind_the_cache_they_are_given(native):
     assert where(beyond) != where(full) and beyond[0].shape[2] == 288
     _, same = layer("origin", (beyond[0].detach(), beyond[1].detach()), 1)            # another tensor of the same rows
     assert where(same) == where(beyond)
+
+
+def misaligned(*shape):
+    """contiguous, but two bytes off"""
+    n = 1
+    for d in shape:
+        n *= d
+    return torch.arange(n + 8).bfloat16()[1:1 + n].view(shape)
+
+
+def test_rows_are_handed_on_aligned():
+    """(contiguous() gives a contiguous tensor back however it is aligned, and whatever the strides of its single-element dims)"""
+    from infllm_amd.ops import rows16
+    single = torch.zeros((1, 2, 1, 128), dtype=torch.bfloat16).as_strided((1, 2, 1, 128), (3, 128, 5, 1))
+    odd = torch.zeros((2, 3, 5, 130), dtype=torch.bfloat16)[..., :128]
+    for t in (misaligned(2, 3, 5, 128), single, odd, torch.zeros((2, 3, 128, 5), dtype=torch.bfloat16).transpose(2, 3)):
+        r = rows16(t)
+        assert torch.equal(r, t) and r.data_ptr() % 16 == 0 and r.stride(3) == 1 and all(s % 8 == 0 for s in r.stride()[:3])
+    fine = torch.zeros((2, 5, 3, 128), dtype=torch.bfloat16).transpose(1, 2)
+    assert rows16(fine) is fine
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_misaligned_rows_and_caches_are_copied(kind, native):
+    _, past = layer(kind, None, 30)
+    cache = tuple(misaligned(*t.shape) if torch.is_tensor(t) else t for t in past)
+    layer(kind, cache, 1, q=misaligned(B, 1, H * D), k=misaligned(B, 1, HKV * D), v=misaligned(B, 1, HKV * D))
+    fields = [n for n, _ in _sink_window._lib.WindowArgs._fields_]
+    args = dict(zip(fields, native.calls[-1][0]))
+    addresses = {n: args[n] for n in fields if n.startswith("d_") and n != "d_inv_freq"}
+    assert addresses["d_old_k"] and all(a % 16 == 0 for a in addresses.values()), addresses
