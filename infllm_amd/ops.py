@@ -63,9 +63,12 @@ def rows16(t):
 
 
 def _bf16_4d(t, name, dims=(HEAD_DIM,)):
-    _need(t.is_cuda, f"{name} must be a GPU tensor")
-    _need(t.dtype == torch.bfloat16, f"{name} must be bfloat16 (the HIP path computes in bf16), got {t.dtype}")
-    _need(t.dim() == 4 and t.shape[-1] in dims, f"{name} must be [B, heads, len, {dims[-1]}], got {tuple(t.shape)}")
+    if not t.is_cuda:
+        raise ValueError(f"{name} must be a GPU tensor")
+    if t.dtype is not torch.bfloat16:
+        raise ValueError(f"{name} must be bfloat16 (the HIP path computes in bf16), got {t.dtype}")
+    if t.dim() != 4 or t.shape[3] not in dims:
+        raise ValueError(f"{name} must be [B, heads, len, {dims[-1]}], got {tuple(t.shape)}")
     return rows16(t)
 
 
