@@ -15,7 +15,7 @@
 // and P never leaves registers.  MFMA row r of a 32-key sub-tile is bound to key
 // pi(r) = 16*(r>>4) + 8*((r>>2)&1) + 4*((r>>3)&1) + (r&3); with that binding the 16
 // accumulator registers of a lane are two runs of 8 consecutive keys, which is exactly
-// the k-slice the second MFMA wants from the lane.  V is transposed on its way into LDS.
+// the k-slice the second MFMA wants from the lane.  V is transposed on its way out of LDS.
 #include <cstdlib>
 
 #include "common.h"
@@ -30,7 +30,7 @@
 namespace {
 
 constexpr int kWaves = 8;                  // 2 per SIMD inside ONE workgroup: a K/V tile in LDS feeds 256 query rows
-constexpr int kStages = 4;                 // K/V tiles resident in LDS: the pair being multiplied and the pair in flight
+constexpr int kStages = 4;                 // K/V tiles resident in LDS
 constexpr int kThreads = kWaves * kWave;
 constexpr int kQTile = 32;                 // queries per wave
 constexpr int kBig = 1 << 29;              // clamp for mask distances held in int32
@@ -109,21 +109,19 @@ __device__ __forceinline__ int swz(int row) {
 }
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ s16x4 lds_read_tr(const bf16_t *p) {
-    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p);
+__device__ __forceinline__ s16x4 lds_read_tr(uint32_t at) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(uintptr_t)at);
 }
 // Issued as inline assembly on purpose.  With the builtin, the compiler tracks the transfer as an LDS store that
 // may alias every later LDS read and puts `s_waitcnt vmcnt(0)` in front of the first operand read of the tile being
 // multiplied - which waits for the tiles just requested for LATER and serialises load and math completely.  The
 // kernel orders the transfers itself: vmcnt(0) and a barrier before a buffer is read, a barrier before it is refilled.
-__device__ __forceinline__ void load_to_lds16(const bf16_t *g, bf16_t *lds_wave_base) {
-    const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)lds_wave_base);
-    uint32_t saved_m0;                    // M0 is the compiler's to manage: put back what it held
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved_m0)
-                 : "s"(lds), "v"(g)
-                 : "memory");
+// The row address is a scalar base and a 32-bit byte offset of the lane.  M0 is overwritten: nothing else in these kernels
+// uses it (LDS instructions have not since gfx9).
+__device__ __forceinline__ void load_to_lds16(const bf16_t *base, uint32_t lane_off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(lane_off), "s"(base) : "memory");
 }
+__device__ __forceinline__ uint32_t lds_address(const char *p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p; }
 
 template <int D>
 constexpr int kTileBytes = kTile * D * 2;         // one K (or V) tile in LDS
@@ -168,8 +166,9 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
                                                                  std::conditional_t<INLINE, InlinePages, NoInlinePages>) {
     constexpr bool HAS_LIN = MODE != kPaged, HAS_PAG = MODE != kLinear, TWO = MODE == kBoth || MODE == kSinks;
     constexpr int kRow = D * 2, kTB = kTileBytes<D>;                     // bytes of a row, of a tile
+    constexpr bool PING = D == 128;
     const infllm_attn_args &ap = TWO ? a2 : a;                 // the paged stage's arguments
-    extern __shared__ __attribute__((aligned(16))) char lds_dyn[];      // kStages K tiles, then kStages V tiles
+    extern __shared__ __attribute__((aligned(1024))) char lds_dyn[];    // kStages K tiles, then kStages V tiles
     char *const Ks = lds_dyn, *const Vs = lds_dyn + kStages * kTB;
     __shared__ int wg_lo[kWaves], wg_hi[kWaves];
 
@@ -246,54 +245,57 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
 
     bf16x8 qreg[D / 16];                     // Q as the B operand: lane = (query col, k-group); loaded behind the first tiles
 
-    // ---- per-lane LDS byte offsets of the MFMA operands (inside one tile buffer)
-    uint32_t k_off[D / 16];                  // K operand kk of sub-tile 0 (sub-tile 1: + 32 rows)
-#pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) k_off[kk] = col * kRow + (((kk * 2 + grp) ^ swz<D>(col)) * 16);
-    uint32_t v_off[D / 32][2];               // V^T operand of d-tile dt, key half e, of 16-key step 0 (step gi: + 16*gi rows)
+    // ---- per-lane LDS byte offsets of the MFMA operands (inside one tile buffer).  One address makes the others: the chunk
+    //      bits of an address are the row's swizzle XOR the operand's number, so K operand kk of sub-tile 0 is at
+    //      k_off ^ kk * 32 (sub-tile 1: + 32 rows), and the V^T operand of d-tile dt, key half e, of 16-key step gi at
+    //      (v_off ^ (dt * 64 + e * 16)) + e * 4 rows + gi * 16 rows.  (Tile buffers begin at multiples of 256 bytes.)
+    const uint32_t k_off = lds_address(Ks) + col * kRow + ((grp ^ swz<D>(col)) * 16);
+    uint32_t v_off;
     {
         const int lam = lane & 15, g16 = lane >> 4;
         const int vr = 8 * (g16 >> 1) + (lam >> 2);              // lane 4*j + q addresses key j ...
         const int vc = 2 * (g16 & 1) + ((lam & 3) >> 1);         // ... at 4 consecutive d: 16-byte chunk
         const int vh = 8 * (lam & 1);                            //     and byte offset inside it
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-            for (int e = 0; e < 2; ++e) v_off[dt][e] = (vr + 4 * e) * kRow + (((dt * 4 + vc) ^ swz<D>(vr + 4 * e)) * 16) + vh;
+        v_off = lds_address(Vs) + vr * kRow + ((vc ^ swz<D>(vr)) * 16) + vh;
     }
 
     // ---- tile loads: an instruction fills 1024 bytes of LDS (4 rows of 128 elements or 8 of 64); wave w fills the 8 rows
     //      from 8*w on; lane -> (row, position).
-    //      The wave-uniform tile base advances with the loop; the per-lane offsets are loop invariant.
+    //      A wave issues an instruction every four to five cycles whatever its kind (a dependent scalar one every eight),
+    //      so the some 300 scalar ones that a tile's addresses and checks used to take cost more than its MFMAs: the tile's
+    //      base advances in scalar registers, and which tiles are whole, and which of them a wave sees without a mask, are
+    //      ranges that are known before the loop.
     constexpr int kRowsPerLd = 1024 / kRow, kLd = kTile / (kRowsPerLd * kWaves);  // load instructions per wave and tile, for K and for V
-    uint32_t gk_off[kLd], gv_off[kLd];        // element offsets inside a linear tile
-    uint32_t pk_off[kLd], pv_off[kLd];        // ... inside a page (rows of D elements)
-    int gk_row[kLd], gv_row[kLd];
-    {
-        const int ld_pos = lane & (D / 8 - 1), ld_sub = lane / (D / 8);
+    // byte offsets, inside a tile, of what this lane fetches for load i: rows of kd (vd) elements
+    auto tile_row = [&](int i) { return kRowsPerLd * (kLd * wave + i) + lane / (D / 8); };      // row of the LDS tile
+    auto k_offset = [&](int i, int64_t kd) {                                                     // (of a K tile: key k_lds_row of it)
+        const int R = tile_row(i);
+        return (uint32_t)(k_lds_row(R) * kd + ((lane & (D / 8 - 1)) ^ swz<D>(R)) * 8) * 2;
+    };
+    auto v_offset = [&](int i, int64_t vd) {
+        const int R = tile_row(i);
+        return (uint32_t)(R * vd + ((lane & (D / 8 - 1)) ^ swz<D>(R)) * 8) * 2;
+    };
+    uint32_t ld_k[kLd], ld_v[kLd];           // those of the linear source (of the pages, where there is nothing else)
 #pragma unroll
-        for (int i = 0; i < kLd; ++i) {
-            const int R = kRowsPerLd * (kLd * wave + i) + ld_sub, chunk = ld_pos ^ swz<D>(R);
-            gk_row[i] = k_lds_row(R);
-            gv_row[i] = R;
-            if (HAS_LIN) {
-                gk_off[i] = (uint32_t)(gk_row[i] * a.k_sl + chunk * 8);
-                gv_off[i] = (uint32_t)(R * a.v_sl + chunk * 8);
-            }
-            if (HAS_PAG) {
-                pk_off[i] = (uint32_t)(gk_row[i] * D + chunk * 8);
-                pv_off[i] = (uint32_t)(R * D + chunk * 8);
-            }
-        }
+    for (int i = 0; i < kLd; ++i) {
+        ld_k[i] = k_offset(i, HAS_LIN ? a.k_sl : D);
+        ld_v[i] = v_offset(i, HAS_LIN ? a.v_sl : D);
     }
-    const bf16_t *k_head = nullptr, *v_head = nullptr;          // linear source: row 0 of this kv head
-    int64_t ring_row = 0;                                        // ring row of the linear tile to load next
+    // the linear tile to load next (a tile never wraps: cap is a multiple of the tile), and tiles to the end of the ring
+    const bf16_t *k_next = nullptr, *v_next = nullptr;
+    const int64_t k_step = (int64_t)kTile * a.k_sl, v_step = (int64_t)kTile * a.v_sl;
+    const int64_t ring_k = (int64_t)((uint64_t)a.cap * (uint64_t)a.k_sl), ring_v = (int64_t)((uint64_t)a.cap * (uint64_t)a.v_sl);
+    int to_wrap = 0;
     if (HAS_LIN) {
-        k_head = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh;
-        v_head = (const bf16_t *)a.d_v + (int64_t)b * a.v_sb + (int64_t)g * a.v_sh;
         const int first = lin_t0 + min(g_t0, n_lin);
-        ring_row = (int64_t)(first - (int)(fdiv(first, geo.cap_tiles) * geo.cap_tiles.d)) * kTile;
+        const int slot = first - (int)(fdiv(first, geo.cap_tiles) * geo.cap_tiles.d);
+        k_next = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + (int64_t)slot * kTile * a.k_sl;
+        v_next = (const bf16_t *)a.d_v + (int64_t)b * a.v_sb + (int64_t)g * a.v_sh + (int64_t)slot * kTile * a.v_sl;
+        to_wrap = (int)min((int64_t)INT32_MAX, (int64_t)geo.cap_tiles.d - slot);
     }
+    // linear tiles whose 64 rows are all in the source: list indices [whole_lo, whole_hi)
+    const int whole_lo = HAS_LIN ? floordiv64(a.j_lo + kTile - 1) - lin_t0 : 0, whole_hi = HAS_LIN ? floordiv64(a.j_hi) - lin_t0 : 0;
     // The page table is read through the constant address space: the index is wave-uniform, so these become scalar
     // loads.  As vector loads they would share the vmcnt counter with the tile transfers, and waiting for a page
     // entry would wait for every tile in flight.  The table is written by an earlier kernel and is read-only here.
@@ -304,53 +306,82 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
                                                                              offsetof(KernargLayout, pages)) + (int64_t)b * n_pag;
     else
         page_table = (const __attribute__((address_space(4))) infllm_page *)(uintptr_t)ap.d_pages + (int64_t)b * n_pag;
-    auto load_tile = [&](int u, int buf) {     // list index; linear tiles are requested in ascending order
+    // the page to load next: its entry is read a tile ahead of its use
+    const bf16_t *page_k = nullptr, *page_v = nullptr;
+    int page_valid = 0;
+    auto next_page = [&](int u) {
+        const __attribute__((address_space(4))) infllm_page *entry = page_table + min(max(u - n_lin, 0), n_pag - 1);
+        const int64_t hs = entry->head_stride;
+        page_k = (const bf16_t *)entry->k + (int64_t)g * hs;
+        page_v = (const bf16_t *)entry->v + (int64_t)g * hs;
+        page_valid = entry->n_valid;
+    };
+    constexpr bool PAGES = MODE == kPaged || MODE == kBoth;
+    if (PAGES && n_pag > 0) next_page(g_t0);
+    const uint32_t lds_k = lds_address(Ks) + wave * (kLd * 1024), lds_v = lds_address(Vs) + wave * (kLd * 1024);
+    // requests tile u into the tile buffer `at` bytes in; tiles are requested in ascending order.  Returns the rows of a page.
+    bool whole = false;                      // the tile requested last was whole: 2 * kLd loads of this wave
+    auto load_tile = [&](int u, uint32_t at) {
         const bf16_t *kbase, *vbase;
-        int row_lo, row_hi;                   // valid rows of this tile: [row_lo, row_hi)
         const bool paged = MODE == kPaged || (TWO && u >= n_lin);
+        int valid = kTile;
         if (MODE == kSinks && paged) {
             const int64_t j0 = (int64_t)(u - n_lin) * kTile;
             kbase = (const bf16_t *)ap.d_k + (int64_t)b * ap.k_sb + (int64_t)g * ap.k_sh + j0 * D;
             vbase = (const bf16_t *)ap.d_v + (int64_t)b * ap.v_sb + (int64_t)g * ap.v_sh + j0 * D;
-            row_lo = 0;
-            row_hi = (int)min((int64_t)kTile, ap.j_hi - j0);
+            valid = (int)min((int64_t)kTile, ap.j_hi - j0);
+            whole = valid == kTile;
         } else if (paged) {
-            const __attribute__((address_space(4))) infllm_page *entry = page_table + (u - n_lin);
-            const int64_t hs = entry->head_stride;
-            kbase = (const bf16_t *)entry->k + (int64_t)g * hs;
-            vbase = (const bf16_t *)entry->v + (int64_t)g * hs;
-            row_lo = 0;
-            row_hi = entry->n_valid;
+            kbase = page_k, vbase = page_v, valid = page_valid;
+            whole = valid == kTile;
+            next_page(u + 1);
         } else {
-            const int64_t j0 = (int64_t)(lin_t0 + u) * kTile;
-            kbase = k_head + ring_row * a.k_sl;       // cap is a multiple of the tile, so a tile never wraps
-            vbase = v_head + ring_row * a.v_sl;
-            ring_row += kTile;
-            if (ring_row >= a.cap) ring_row -= a.cap;
-            row_lo = (int)max((int64_t)0, a.j_lo - j0);
-            row_hi = (int)min((int64_t)kTile, a.j_hi - j0);
+            kbase = k_next, vbase = v_next;
+            k_next += k_step, v_next += v_step;
+            if (--to_wrap == 0) {
+                asm volatile("" ::: "memory");         // (a branch, not selects on every tile)
+                k_next -= ring_k, v_next -= ring_v;
+                to_wrap = (int)geo.cap_tiles.d;
+            }
+            whole = u >= whole_lo && u < whole_hi;
         }
-        char *kdst = Ks + buf * kTB + wave * (kLd * 1024), *vdst = Vs + buf * kTB + wave * (kLd * 1024);
-        if (row_lo == 0 && row_hi == kTile) {          // the common case: no per-lane predicate
+        const uint32_t kdst = lds_k + at, vdst = lds_v + at;
+        uint32_t k_src[kLd], v_src[kLd];
+#pragma unroll
+        for (int i = 0; i < kLd; ++i) {
+            k_src[i] = TWO && paged ? k_offset(i, D) : ld_k[i];
+            v_src[i] = TWO && paged ? v_offset(i, D) : ld_v[i];
+        }
+        if (whole) {                                   // the common case: no per-lane predicate
 #pragma unroll
             for (int i = 0; i < kLd; ++i) {
-                load_to_lds16(kbase + (paged ? pk_off[i] : gk_off[i]), (bf16_t *)(kdst + i * 1024));
-                load_to_lds16(vbase + (paged ? pv_off[i] : gv_off[i]), (bf16_t *)(vdst + i * 1024));
+                load_to_lds16(kbase, k_src[i], kdst + i * 1024);
+                load_to_lds16(vbase, v_src[i], vdst + i * 1024);
             }
         } else {
+            int row_lo = 0, row_hi = valid;            // valid rows of this tile: [row_lo, row_hi)
+            if (!paged) {
+                const int64_t j0 = (int64_t)(lin_t0 + u) * kTile;
+                row_lo = (int)max((int64_t)0, a.j_lo - j0);
+                row_hi = (int)min((int64_t)kTile, a.j_hi - j0);
+            }
+            char *kz = Ks + at + wave * (kLd * 1024), *vz = Vs + at + wave * (kLd * 1024);
 #pragma unroll
             for (int i = 0; i < kLd; ++i) {
                 // rows outside the source are written as zeros: their keys are masked, but 0 * stale must stay 0
-                if (gk_row[i] >= row_lo && gk_row[i] < row_hi) load_to_lds16(kbase + (paged ? pk_off[i] : gk_off[i]), (bf16_t *)(kdst + i * 1024));
-                else *(u32x4 *)(kdst + i * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
-                if (gv_row[i] >= row_lo && gv_row[i] < row_hi) load_to_lds16(vbase + (paged ? pv_off[i] : gv_off[i]), (bf16_t *)(vdst + i * 1024));
-                else *(u32x4 *)(vdst + i * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+                const int rv = tile_row(i), rk = k_lds_row(rv);
+                if (rk >= row_lo && rk < row_hi) load_to_lds16(kbase, k_src[i], kdst + i * 1024);
+                else *(u32x4 *)(kz + i * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+                if (rv >= row_lo && rv < row_hi) load_to_lds16(vbase, v_src[i], vdst + i * 1024);
+                else *(u32x4 *)(vz + i * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
             }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
+        return valid;
     };
 
     // ---- running softmax state of this lane's query (max kept in raw logit units, allowed to lag)
-    float m_run = -INFINITY, l_run = 0.f, neg_ms = 0.f;
+    float m_run = -INFINITY, m_limit = -INFINITY, l_run = 0.f, neg_ms = 0.f;
     f32x16 oacc[D / 32];
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt)
@@ -359,71 +390,50 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
 
     const float scale = a.softmax_scale * 1.4426950408889634f;
     const float lazy = kLazyLog2 / scale;
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    // kb / vb: k_off / v_off in the tile's buffer
+    auto k_operand = [&](uint32_t kb, int kk, int ks) {
+        return *(const __attribute__((address_space(3))) u32x4 *)(uintptr_t)((kb ^ (kk * 32)) + ks * 32 * kRow);
+    };
+    auto v_operand = [&](uint32_t vb, int dt, int gi) {
+        s16x8 v;
+        v.lo = lds_read_tr((vb ^ (dt * 64)) + gi * 16 * kRow);
+        v.hi = lds_read_tr((vb ^ (dt * 64 + 16)) + (gi * 16 + 4) * kRow);
+        return __builtin_bit_cast(u32x4, v);
+    };
 
-    auto tile_math = [&](int buf, int t) {
-        const char *kb = Ks + buf * kTB, *vb = Vs + buf * kTB;
-        // Heads of 64: registers are what two workgroups on a CU are short of, so an operand's address is made from the first
-        // one's where it is read: kk flips chunk bits 1 and 2 of a K row.  (Said anew per tile, or the compiler keeps them all.)
-        uint32_t k_base = k_off[0];
-        if (D == 64) asm volatile("" : "+v"(k_base));
-        f32x16 s[2];
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[ks][r] = 0.f;
-        {
-            // 16 K operands in groups of 4 (kk pair x both sub-tiles): a group is requested from LDS while the
-            // MFMAs of the previous one run; scheduling fences keep the compiler from serialising read -> MFMA
-            constexpr int KG = D == 128 ? 4 : 2, NG = D / 8 / KG;      // (heads of 64: 8 operands, in groups of 2)
-            bf16x8 ka[NG][KG];
-            auto k_operand = [&](int i) {          // i = kk * 2 + ks
-                return *(const bf16x8 *)(kb + (i & 1) * 32 * kRow + (D == 128 ? k_off[i >> 1] : k_base ^ ((i >> 1) * 32)));
-            };
-#pragma unroll
-            for (int j = 0; j < KG; ++j) ka[0][j] = k_operand(j);
-#pragma unroll
-            for (int gi = 0; gi < NG; ++gi) {
-                __builtin_amdgcn_sched_barrier(0);
-                if (gi < NG - 1) {
-#pragma unroll
-                    for (int j = 0; j < KG; ++j) ka[gi + 1][j] = k_operand((gi + 1) * KG + j);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-#pragma unroll
-                for (int j = 0; j < KG; ++j) {
-                    const int i = gi * KG + j;
-                    s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[gi][j], qreg[i >> 1], s[i & 1], 0, 0, 0);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // ---- mask (only tiles that touch a boundary); distances are clamped into int32
-        bool need_mask;
-        int row_lo = 0, row_hi = kTile;
-        int d0 = 0;                            // dist of (this lane's query, key 0 of the tile)
+    // Tiles that this wave sees whole, without a mask: of the linear ones [clear_lo, clear_hi), of the sinks' those in front
+    // of clear_pag
+    int clear_lo = whole_lo, clear_hi = whole_hi, clear_pag = 0;
+    if (HAS_LIN) {
+        const int64_t q0 = (int64_t)i0 + a.offset, q1 = (int64_t)i1 + a.offset;
+        auto tile_of = [&](int64_t j) { return (int)min(max(j >> 6, (int64_t)-kBig), (int64_t)kBig); };
+        if (a.mask == INFLLM_MASK_WINDOW) {            // every key at a distance of 0 or more from the first query, below the window from the last
+            clear_lo = max(clear_lo, tile_of(q1 - a.window) + 1 - lin_t0);
+            clear_hi = min(clear_hi, tile_of(q0 - (kTile - 1)) + 1 - lin_t0);
+        } else if (a.mask == INFLLM_MASK_COMPLEMENT)
+            clear_hi = min(clear_hi, tile_of(q0 - (kTile - 1) - a.window) + 1 - lin_t0);
+        clear_hi = min(clear_hi, n_lin);
+        if (MODE == kSinks) clear_pag = n_lin + min(floordiv64(ap.j_hi), tile_of((int64_t)i0 + ap.offset - (kTile - 1) - ap.window) + 1);
+    }
+    // the mask of a tile's scores (valid: rows of a page)
+    auto mask = [&](f32x16 (&s)[2], int t, [[maybe_unused]] int valid) {
         const bool paged = MODE == kPaged || (TWO && t >= n_lin);
-        if (MODE == kSinks && paged) {
-            const int64_t j0 = (int64_t)(t - n_lin) * kTile, e0 = (int64_t)i0 + ap.offset - j0;
-            row_hi = (int)min((int64_t)kTile, ap.j_hi - j0);
-            need_mask = row_hi < kTile || e0 - (kTile - 1) < ap.window;
-            d0 = (int)min(max(e0, (int64_t)-kBig), (int64_t)kBig) + col;
-        } else if (paged) {
-            row_hi = page_table[t - n_lin].n_valid;
-            need_mask = row_hi < kTile;
-        } else {
-            const int64_t j0 = (int64_t)(lin_t0 + t) * kTile;
-            row_lo = (int)max((int64_t)0, a.j_lo - j0);
-            row_hi = (int)min((int64_t)kTile, a.j_hi - j0);
-            need_mask = row_lo > 0 || row_hi < kTile;
-            const int64_t e0 = (int64_t)i0 + a.offset - j0;       // dist(query i0, key j0)
-            if (a.mask == INFLLM_MASK_WINDOW) {
-                need_mask |= (e0 < kTile - 1) || (e0 + (i1 - i0) >= a.window);
-            } else if (a.mask == INFLLM_MASK_COMPLEMENT) {
-                need_mask |= (e0 - (kTile - 1) < a.window);
+        if (!(PAGES && paged ? valid == kTile : TWO && paged ? t < clear_pag : t >= clear_lo && t < clear_hi)) {
+            int row_lo = 0, row_hi = kTile;
+            int d0 = 0;                        // dist of (this lane's query, key 0 of the tile), clamped into int32
+            if (MODE == kSinks && paged) {
+                const int64_t j0 = (int64_t)(t - n_lin) * kTile, e0 = (int64_t)i0 + ap.offset - j0;
+                row_hi = (int)min((int64_t)kTile, ap.j_hi - j0);
+                d0 = (int)min(max(e0, (int64_t)-kBig), (int64_t)kBig) + col;
+            } else if (paged) {
+                row_hi = valid;
+            } else {
+                const int64_t j0 = (int64_t)(lin_t0 + t) * kTile, e0 = (int64_t)i0 + a.offset - j0;
+                row_lo = (int)max((int64_t)0, a.j_lo - j0);
+                row_hi = (int)min((int64_t)kTile, a.j_hi - j0);
+                d0 = (int)min(max(e0, (int64_t)-kBig), (int64_t)kBig) + col;
             }
-            d0 = (int)min(max(e0, (int64_t)-kBig), (int64_t)kBig) + col;
-        }
-        if (need_mask) {
             // Whatever the mask, a lane's query sees ONE run of the tile's keys: its bounds are found once, and a key costs a
             // subtraction and a compare (a mask's conditions key by key: 150 branches in the sinks' form of the kernel).
             // dist = dl - kc; kc is the compile-time part of register r's key, which is kc + 8 * grp
@@ -445,15 +455,19 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
                     s[ks][r] = vis ? s[ks][r] : -INFINITY;
                 }
         }
-        float tmax = -INFINITY;
+    };
+    // the running max that a tile's scores move, and with it the accumulators
+    auto max_and_rescale = [&](f32x16 (&s)[2]) {
+        // (four chains: a dependent instruction waits twice as long as another)
+        float tm[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
+        for (int r = 0; r < 8; r += 2)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[ks][r]);
-        tmax = fmaxf(tmax, wave_xor32(tmax));
+            for (int i = 0; i < 4; ++i) tm[i] = fmaxf(fmaxf(tm[i], s[i & 1][8 * (i >> 1) + r]), s[i & 1][8 * (i >> 1) + r + 1]);
+        const float tmax = wave_max32(fmaxf(fmaxf(fmaxf(tm[0], tm[1]), tm[2]), tm[3]));
         // lazy running max: it only moves when a score would exceed it by more than 2^kLazyLog2 after scaling,
         // so the rescale of the output accumulators is rare; probabilities stay below 2^kLazyLog2
-        const bool moved = tmax > m_run + lazy;
+        const bool moved = tmax > m_limit;
         if (__builtin_amdgcn_ballot_w64(moved) != 0) {
             const float m_new = moved ? tmax : m_run;
             const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale);      // exp2(-inf) = 0 on the first move
@@ -464,8 +478,40 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
 #pragma unroll
                 for (int r = 0; r < 16; ++r) oacc[dt][r] *= al;
             m_run = m_new;
+            m_limit = m_new + lazy;
             neg_ms = (m_run == -INFINITY) ? 0.f : -m_run * scale;
         }
+    };
+    // heads of 64: a tile's arithmetic by itself; the SIMD's other three waves fill its waits
+    auto tile_math = [&](int buf, int t) {
+        uint32_t kb = k_off + buf * kTB, vb = v_off + buf * kTB;
+        asm volatile("" : "+v"(kb), "+v"(vb));       // (an operand's address is made where it is read: registers are short)
+        f32x16 s[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[ks][r] = 0.f;
+        {
+            // 8 K operands in groups of 2: a group is requested from LDS while the MFMAs of the previous one run;
+            // scheduling fences keep the compiler from serialising read -> MFMA
+            u32x4 ka[D / 16][2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) ka[0][j] = k_operand(kb, 0, j);
+#pragma unroll
+            for (int gi = 0; gi < D / 16; ++gi) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (gi < D / 16 - 1) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) ka[gi + 1][j] = k_operand(kb, gi + 1, j);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int j = 0; j < 2; ++j) s[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ka[gi][j]), qreg[gi], s[j], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        mask(s, t, PAGES && (MODE == kPaged || t >= n_lin) ? page_table[t - n_lin].n_valid : kTile);
+        max_and_rescale(s);
         // The row sum is taken over the probabilities AS ROUNDED to bf16, the values the second MFMA multiplies: the
         // output is then an exact convex combination of value rows (a row on which one key carries nearly all the
         // weight comes out as that value row, whatever the rounding of its weight), and a pair costs one dot
@@ -483,27 +529,13 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         };
         exps(0, 0, 16);                        // the first 32 keys now; the other 32 beside the MFMAs that consume these
         {
-            // 4 steps of 16 keys, 4 MFMAs each; the V^T operands of a step are requested from LDS while the
-            // MFMAs of the previous step run
-            typedef short s16x8 __attribute__((ext_vector_type(8)));
-            constexpr bool AHEAD = D == 128;      // (heads of 64: the SIMD's other waves fill the wait, see kWgsPerCu)
-            s16x8 va[2][D / 32];
-            auto v_operands = [&](int gi, s16x8 *dst) {
-#pragma unroll
-                for (int dt = 0; dt < D / 32; ++dt) {
-                    dst[dt].lo = lds_read_tr((const bf16_t *)(vb + gi * 16 * kRow + v_off[dt][0]));
-                    dst[dt].hi = lds_read_tr((const bf16_t *)(vb + gi * 16 * kRow + v_off[dt][1]));
-                }
-            };
-            if (AHEAD) v_operands(0, va[0]);
+            // 4 steps of 16 keys
 #pragma unroll
             for (int gi = 0; gi < 4; ++gi) {
+                u32x4 va[D / 32];
                 __builtin_amdgcn_sched_barrier(0);
-                if (!AHEAD) v_operands(gi, va[gi & 1]);
-                if (AHEAD && gi < 3) {
-                    v_operands(gi + 1, va[(gi + 1) & 1]);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+#pragma unroll
+                for (int dt = 0; dt < D / 32; ++dt) va[dt] = v_operand(vb, dt, gi);
                 const int ks = gi >> 1, mm = gi & 1;
                 u32x4 praw{pw[ks][4 * mm], pw[ks][4 * mm + 1], pw[ks][4 * mm + 2], pw[ks][4 * mm + 3]};
                 bf16x8 pb = __builtin_bit_cast(bf16x8, praw);
@@ -513,7 +545,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
                 if (gi < 2) exps(1, 8 * gi, 8 * gi + 8);
 #pragma unroll
                 for (int dt = 0; dt < D / 32; ++dt)
-                    oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va[gi & 1][dt]), pb, oacc[dt], 0, 0, 0);
+                    oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va[dt]), pb, oacc[dt], 0, 0, 0);
                 if (gi < 2) {
 #pragma unroll
                     for (int dt = 0; dt < D / 32; ++dt) {
@@ -529,12 +561,6 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         l_run += psum[0] + psum[1];
     };
 
-    // Tiles are handled in pairs: one barrier per two tiles.  While the pair (t, t+1) is multiplied, the next
-    // pair is on its way into the other two buffers, which were last read before the previous barrier; the
-    // loads of a pair are the only ones outstanding, so landing = vmcnt(0).
-    static_assert(kStages == 4, "two buffer pairs");
-    for (int p = 0; p < 2; ++p)
-        if (g_t0 + p < g_t1) load_tile(g_t0 + p, p);
     auto load_q = [&](const infllm_attn_args &src) {
         const int qi = i0 + col;
         const bool ok = live && qi < src.Lq;
@@ -545,11 +571,24 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             qreg[kk] = __builtin_bit_cast(bf16x8, raw);
         }
     };
+    // does this wave see tile u at all?  (pages: every live wave; linear tiles: the wave's own visible range)
+    auto mine = [&](int u) {
+        if (MODE == kSinks && u >= n_lin) return live && (int64_t)i1 + ap.offset - ap.window >= (int64_t)(u - n_lin) * kTile;
+        return (HAS_PAG && u >= n_lin) ? live : (u >= wu0 && u < wu1);
+    };
     // the queries of the stage this split starts in; a split that crosses from the linear tiles into the pages swaps
     // them for the paged stage's queries at its first page (once per workgroup: that wait also covers the tiles in flight)
     bool q_paged = MODE == kPaged || (TWO && g_t0 >= n_lin);
     load_q(q_paged ? ap : a);
 
+    if constexpr (!PING) {
+    // Tiles are handled in pairs: one barrier per two tiles.  While the pair (t, t+1) is multiplied, the next
+    // pair is on its way into the other two buffers, which were last read before the previous barrier; the
+    // loads of a pair are the only ones outstanding, so landing = vmcnt(0).
+    static_assert(PING || kStages == 4, "two buffer pairs");
+    for (int p = 0; p < 2; ++p)
+        if (g_t0 + p < g_t1) load_tile(g_t0 + p, p * kTB);
+    load_q(q_paged ? ap : a);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // The compiler does not know that the wait above also covered the query rows; passing them through an empty
     // asm makes it place its own wait for them HERE rather than in front of their first use inside the loop,
@@ -557,15 +596,10 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(qreg[kk]));
     __syncthreads();
-    // does this wave see tile u at all?  (pages: every live wave; linear tiles: the wave's own visible range)
-    auto mine = [&](int u) {
-        if (MODE == kSinks && u >= n_lin) return live && (int64_t)i1 + ap.offset - ap.window >= (int64_t)(u - n_lin) * kTile;
-        return (HAS_PAG && u >= n_lin) ? live : (u >= wu0 && u < wu1);
-    };
     for (int t = g_t0; t < g_t1; t += 2) {
         const int buf = (t - g_t0) & 3;                          // 0 or 2
-        if (t + 2 < g_t1) load_tile(t + 2, buf ^ 2);
-        if (t + 3 < g_t1) load_tile(t + 3, (buf ^ 2) + 1);
+        if (t + 2 < g_t1) load_tile(t + 2, (buf ^ 2) * kTB);
+        if (t + 3 < g_t1) load_tile(t + 3, ((buf ^ 2) + 1) * kTB);
 #pragma unroll
         for (int e = 0; e < 2; ++e) {                            // wave-uniform conditions; barriers stay outside
             const int u = t + e;
@@ -579,12 +613,212 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     }
+    } else {
+    // Heads of 128.  A SIMD runs MFMAs of one wave beside vector instructions of another, but its two waves, at the same
+    // place of the same code, want the same of the two at any time.  So waves w and w + 4, which share a SIMD, take turns:
+    // while one multiplies - P.V of the tile before, then K.Q of this one, 36 MFMAs of 32 cycles -, the other forms its
+    // probabilities.  The second four are half a tile behind, by one more barrier in front of their loop, and a barrier ends
+    // each half.  A wave requests its rows of tile t + 2 while it multiplies with t and sees those of t + 1 through at the end
+    // of that half, a tile's time after their request; the values of t - 2, whose buffer t + 2 takes, were last read a tile
+    // earlier.  What the halves cost was found one instruction at a time (cycles of a tile and two waves; 4,200 with both
+    // waves in step): the turns with the instructions of the old loop 4,600, row sums without dot instructions (they run on
+    // the matrix pipe and wait until it is empty, also of the other wave's work) and MFMAs first (s_setprio) 4,450, addresses
+    // and checks out of the loop 3,290, operand reads between the MFMAs instead of in runs of 8 and row sums as MFMAs 3,010,
+    // the maximum in four chains and reads between the exponentials 2,800.  8,192 queries x 4,096 window keys, 32 heads:
+    // 587 -> 500 us of N(0, 1) data, 510 -> 372 of zeros, on which the card does not lower its clock.
+    f32x16 s[2];
+    uint32_t pw[2][8];
+    u32x4 ones{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+    asm volatile("" : "+v"(ones));
+    // A half's 32 operands, one per MFMA: 0-15 the V^T of the tile before (16-key step, then d-tile), 16-31 the K of this one.
+    // Each is requested 8 MFMAs ahead, into the registers of the one that has just been used, and between the MFMAs: a run
+    // of reads keeps the wave from issuing them.
+    u32x4 op[8];
+    uint32_t at = 0;                       // the buffer of the tile at hand
+    auto request = [&](int i, uint32_t vb, uint32_t kb) {
+        op[i & 7] = i < 16 ? v_operand(vb, (i & 3) % (D / 32), i >> 2) : k_operand(kb, ((i - 16) >> 1) % (D / 16), i & 1);
+    };
+    auto exps = [&](int ks, int r0, int r1) {
+#pragma unroll
+        for (int r = r0; r < r1; r += 2) {
+            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[ks][r], scale, neg_ms));
+            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[ks][r + 1], scale, neg_ms));
+            pw[ks][r >> 1] = pack_bf16x2(p0, p1);
+            asm volatile("" : "+v"(pw[ks][r >> 1]));                                // formed here, not where it is read
+        }
+    };
+    // O += P.V of the tile before; the first 8 operands are on their way when it begins.  The row sums - over the probabilities
+    // AS ROUNDED to bf16, see tile_math - are one more MFMA per step, against ones: 128 cycles of a matrix pipe that has them
+    // to spare, where 64 shifts and additions took 220 of the vector half.
+    auto pv_mul = [&](uint32_t vb, uint32_t kb, auto meanwhile) {
+        f32x16 sums;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sums[r] = 0.f;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            __builtin_amdgcn_sched_barrier(0);
+            meanwhile(g);
+            const u32x4 praw{pw[g >> 1][4 * (g & 1)], pw[g >> 1][4 * (g & 1) + 1], pw[g >> 1][4 * (g & 1) + 2], pw[g >> 1][4 * (g & 1) + 3]};
+            const bf16x8 pb = __builtin_bit_cast(bf16x8, praw);
+#pragma unroll
+            for (int dt = 0; dt < D / 32; ++dt) {
+                oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, op[(4 * g + dt) & 7]), pb, oacc[dt], 0, 0, 0);
+                request(4 * g + dt + 8, vb, kb);
+            }
+            sums = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ones), pb, sums, 0, 0, 0);
+#pragma unroll
+            for (int dt = 0; dt < D / 32; ++dt) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                  // one MFMA
+                __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);                  // an operand's address
+                if (g < 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);       // its reads
+                else __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        l_run += sums[0];
+    };
+    // S = K.Q of this tile; its first 8 operands are on their way
+    auto qk_mul = [&](uint32_t kb) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[ks][r] = 0.f;
+#pragma unroll
+        for (int g = 4; g < 8; ++g) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = 4 * g + j;
+                s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, op[i & 7]), qreg[((i - 16) >> 1) % (D / 16)], s[i & 1], 0, 0, 0);
+                if (i + 8 < 32) request(i + 8, 0, kb);
+            }
+            if (g < 6) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // the vector half: max and rescale, the probabilities, the first 8 operands of P.V
+    auto probabilities = [&]() {
+        max_and_rescale(s);
+        __builtin_amdgcn_sched_barrier(0);
+        exps(0, 0, 16);
+        exps(1, 0, 16);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) request(i, v_off + at, 0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);                      // two keys' multiply-adds
+            __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);                      // their exponentials
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                      // a read
+            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);                      // rounding, an address
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto half_end = [&]() { asm volatile("s_barrier" ::: "memory"); };
+    auto all_but_last = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * kLd) : "memory"); };      // but the rows of one whole tile
+    auto landed = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
+    const bool second = wave >= 4;
+    int t = g_t0;                          // the tile at hand, and rows of the pages t, t + 1, t + 2
+    int valid0 = kTile, valid1 = kTile, valid2 = kTile;
+    if (t < g_t1) valid0 = load_tile(t, 0);
+    load_q(q_paged ? ap : a);
+    landed();
+    // (as above: the query rows' wait belongs here)
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(qreg[kk]));
+    if (t + 1 < g_t1) valid1 = load_tile(t + 1, kTB);
+    half_end();
+    if (second) half_end();
+    bool have_p = false;                   // the tile before has probabilities that wait for their values
+    // A tile with nothing special about it - whole, seen without a mask, the tile before seen too and the one to request
+    // whole - takes the form without branches.  Of the pages that is known one at a time.
+    const int hot_lo = max(max(wu0 + 1, g_t0 + 1), clear_lo), hot_hi = min(min(min(wu1, clear_hi), min(whole_hi, g_t1) - 2), n_lin - 2);
+    auto is_hot = [&]() {
+        if (MODE == kPaged) return t + 2 < g_t1 && valid0 == kTile && page_valid == kTile;
+        return t < hot_hi;
+    };
+    const int64_t k_back = k_step - ring_k, v_back = v_step - ring_v;
+    auto hot = [&]() {
+        const uint32_t kb = k_off + at, vb = v_off + ((at - kTB) & (4 * kTB - 1));
+        const uint32_t to = (at + 2 * kTB) & (4 * kTB - 1), kdst = lds_k + to, vdst = lds_v + to;
+        const bf16_t *kbase = k_next, *vbase = v_next;
+        if (MODE == kPaged)
+            kbase = page_k, vbase = page_v;
+        else {
+            --to_wrap;
+            k_next += to_wrap == 0 ? k_back : k_step;
+            v_next += to_wrap == 0 ? v_back : v_step;
+            to_wrap = to_wrap == 0 ? (int)geo.cap_tiles.d : to_wrap;
+        }
+        __builtin_amdgcn_s_setprio(1);       // the MFMAs go first
+        pv_mul(vb, kb, [&](int g) {          // the tile after next: a request beside each of the four steps
+            static_assert(D != 128 || kLd == 2, "two loads of K and of V a wave");
+            if (g < kLd) load_to_lds16(kbase, ld_k[g % kLd], kdst + g * 1024);
+            else load_to_lds16(vbase, ld_v[g % kLd], vdst + (g - kLd) * 1024);
+        });
+        qk_mul(kb);
+        if (MODE == kPaged) next_page(t + 3);
+        all_but_last();
+        half_end();
+        __builtin_amdgcn_s_setprio(0);
+        probabilities();
+        half_end();
+        at = (at + kTB) & (4 * kTB - 1);
+        if (PAGES) valid0 = valid1, valid1 = kTile;
+        ++t;
+    };
+    auto special = [&]() {
+        whole = false;
+        if (t + 2 < g_t1) valid2 = load_tile(t + 2, (at + 2 * kTB) & (4 * kTB - 1));
+        if (TWO && t >= n_lin && !q_paged) {
+            load_q(ap);
+            q_paged = true;
+        }
+        const bool see = mine(t);
+        const uint32_t kb = k_off + at;
+        __builtin_amdgcn_s_setprio(1);
+        if (have_p) pv_mul(v_off + ((at - kTB) & (4 * kTB - 1)), kb, [](int) {});
+        else {
+#pragma unroll
+            for (int i = 16; i < 24; ++i) request(i, 0, kb);
+        }
+        if (see) qk_mul(kb);
+        if (whole) all_but_last();
+        else landed();
+        half_end();
+        __builtin_amdgcn_s_setprio(0);
+        if (see) {
+            mask(s, t, valid0);
+            probabilities();
+        }
+        have_p = see;
+        half_end();
+        at = (at + kTB) & (4 * kTB - 1);
+        if (PAGES) valid0 = valid1, valid1 = valid2;
+        ++t;
+    };
+    while (t < g_t1) {
+        if (have_p && (MODE == kPaged || t >= hot_lo) && is_hot())
+            do hot();
+            while (is_hot());
+        special();
+    }
+    if (have_p) pv_mul(v_off + ((at - kTB) & (4 * kTB - 1)), k_off, [](int) {});
+    if (!second) half_end();
+    half_end();                            // every tile has been read: the epilogue stages rows in the buffers
+    }
 
     // ---- epilogue: normalised partial + base-2 log-sum-exp.  The accumulators hold O^T (a lane owns a query and
     //      scattered 4-float pieces of its row); they go through this wave's 16 KB of the now idle tile buffers so
     //      that every store instruction writes two whole 512-byte rows.
     if (!live) return;
-    const float l_tot = l_run + wave_xor32(l_run);
+    const float l_tot = PING ? l_run : l_run + wave_xor32(l_run);
     const int qi = i0 + col;
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     int64_t row0 = (((int64_t)split * a.B + b) * a.H + h) * a.Lq + i0;            // row of this wave's first query
@@ -783,6 +1017,8 @@ int check_linear_stage(const infllm_attn_args *a) {
     INFLLM_REQUIRE(a->j_hi < (1ll << 36), "attn_stage: key range beyond 2^36 rows");
     INFLLM_REQUIRE((a->k_sl % 8 | a->k_sh % 8 | a->k_sb % 8 | a->v_sl % 8 | a->v_sh % 8 | a->v_sb % 8) == 0,
                    "attn_stage: k/v strides must be multiples of 8");
+    INFLLM_REQUIRE(a->k_sl >= 0 && a->v_sl >= 0 && a->k_sl < (1ll << 25) && a->v_sl < (1ll << 25), "attn_stage: k/v rows of %lld / %lld elements apart",
+                   (long long)a->k_sl, (long long)a->v_sl);          // (a lane's offset inside a tile is 32 bits of bytes)
     return 0;
 }
 

@@ -62,6 +62,12 @@ __device__ __forceinline__ float wave_xor32(float x) {
     return __shfl_xor(x, 32, 64);
 }
 
+// the larger of a lane's value and that of the lane 32 away, in both: vector instructions (a shuffle is a trip through LDS)
+__device__ __forceinline__ float wave_max32(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 __device__ __forceinline__ uint32_t order_key(float f) {
     uint32_t u = __float_as_uint(f);
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);       // larger float <=> larger key
