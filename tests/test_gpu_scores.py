@@ -1,0 +1,55 @@
+"""Local scores where a stage of queries is masked in part: the diagonal, the far end of the window, ranges of keys that begin
+and end inside a wave's, queries that end inside a stage, rings that wrap - for launches whose waves hold 32 keys and 64.
+
+Against 64 bits over the same bf16 inputs and the same log-sum-exps.  A probability is exp2 of a 32-bit sum of 128 products (an
+error of some 2^-20 of the logit's size, below 2^5 here) and a score a 32-bit sum of up to 600 of them: 1e-4 relative, 1e-5
+absolute."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+def _rand(shape, seed):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).bfloat16()
+
+
+def _visible(mask, Lq, lo, hi, offset, window):
+    dist = torch.arange(Lq)[:, None] - torch.arange(lo, hi)[None, :] + offset
+    return {0: torch.ones_like(dist, dtype=torch.bool), 1: (dist >= 0) & (dist < window), 2: dist >= window}[mask]
+
+
+@pytest.mark.parametrize("H,Hkv,keys", [(4, 2, 700), (64, 64, 2100)])           # 32 keys a wave; 64
+@pytest.mark.parametrize("Lq", [1, 33, 130, 512, 600])
+@pytest.mark.parametrize("mask", ["none", "window", "complement"])
+def test_scores_of_partly_masked_stages(H, Hkv, keys, Lq, mask):
+    from infllm_amd import ops
+    cap, lo = 2304, 77
+    hi = lo + keys
+    code = dict(none=ops.MASK_NONE, window=ops.MASK_WINDOW, complement=ops.MASK_COMPLEMENT)[mask]
+    offset, window = hi - Lq - 45, keys - 150                 # the last 45 keys behind every query, the first ones out of the window
+    q, k = _rand((1, H, Lq, D), 1), _rand((1, Hkv, keys, D), 2)
+    ring = torch.full((1, Hkv, cap, D), float("nan"), dtype=torch.bfloat16)
+    base = 2304 * 3 - 500                                      # positions base + j, j in [lo, hi): they wrap
+    rows = (torch.arange(lo, hi) + base) % cap
+    ring[:, :, rows] = k
+    kk = k.repeat_interleave(H // Hkv, dim=1).double()
+    s = torch.matmul(q.double(), kk.transpose(2, 3).contiguous()) / math.sqrt(D) * math.log2(math.e)
+    vis = _visible(code, Lq, lo, hi, offset, window)
+    s = s.masked_fill(~vis, float("-inf"))
+    lse = torch.logsumexp(s * math.log(2.0), -1) / math.log(2.0)
+    lse32 = lse.float()
+    want = torch.where(vis, torch.exp2(s - torch.where(torch.isfinite(lse), lse32.double(), math.inf)[..., None]), 0.0).sum(2)
+    start = torch.rand((1, H, cap), generator=torch.Generator().manual_seed(3))
+    score = start.cuda()
+    ops.local_score(q.cuda(), ring.cuda(), torch.where(torch.isfinite(lse32), lse32, math.inf).cuda(), score, cap=cap, j_lo=base + lo, j_hi=base + hi, mask=code,
+                    offset=offset + base, window=window, accumulate=True, score_cap=cap)
+    got = score.cpu()
+    other = torch.ones(cap, dtype=torch.bool)
+    other[rows] = False
+    assert torch.equal(got[:, :, other], start[:, :, other])
+    assert torch.allclose(got[:, :, rows].double(), want + start[:, :, rows].double(), rtol=1e-4, atol=1e-5), float(
+        (got[:, :, rows].double() - want - start[:, :, rows].double()).abs().max())
