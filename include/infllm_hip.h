@@ -696,6 +696,7 @@ typedef struct {
     float *d_call_scores;                             /* [blocks, B, scores_cols], scores_cols >= the units after the call */
     int64_t scores_cols;
     int32_t *d_base;                                  /* [blocks, B, topk] */
+    uint32_t *d_ticket;                               /* one word, zero when the workspaces are made; every call leaves it zero */
 } infllm_resident_call;
 int infllm_resident_append(void *handle, const infllm_resident_call *a, void *stream);
 int64_t infllm_resident_part_rows(const infllm_resident_desc *d);

@@ -116,7 +116,7 @@ class ResidentCall(C.Structure):
         ("d_unit_scores", c_vp), ("unit_scores_sb", c_i64), ("h_chunks", c_vp), ("d_chunks", c_vp),
         ("d_q_loc", c_vp), ("d_q_glb", c_vp), ("d_qpart", c_vp), ("d_qbar", c_vp), ("d_o_part", c_vp), ("d_lse_part", c_vp), ("part_rows", c_i64),
         ("d_o_part2", c_vp), ("d_lse_part2", c_vp), ("part_rows2", c_i64), ("d_lse", c_vp), ("d_logits", c_vp),
-        ("d_call_scores", c_vp), ("scores_cols", c_i64), ("d_base", c_vp),
+        ("d_call_scores", c_vp), ("scores_cols", c_i64), ("d_base", c_vp), ("d_ticket", c_vp),
     ]
 
 

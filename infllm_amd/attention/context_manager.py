@@ -559,7 +559,8 @@ class ContextManager:
                            o_part=torch.empty((part_rows * D,), **f16), lse_part=torch.empty((part_rows,), **f32),
                            o_part2=torch.empty((self._part_rows2 * D,), **f16), lse_part2=torch.empty((self._part_rows2,), **f32),
                            lse=torch.empty((B * H * max(T, exc),), **f32), logits=torch.empty((B * H * self.n_local,), **f32),
-                           base=torch.empty((blocks * B * self.topk,), dtype=torch.int32, device=self.device))
+                           base=torch.empty((blocks * B * self.topk,), dtype=torch.int32, device=self.device),
+                           ticket=torch.zeros((1,), dtype=torch.int32, device=self.device))
             _CALL_BUFFERS[key] = buf
         self._call_buf = buf
         rc = self._rc

@@ -10,7 +10,7 @@ struct CarveCopy {
     bf16_t *out_a, *out_b;
     int64_t out_sb, out_su, out_sh;
     int32_t ring_cap, slot0;                       // n <= ring_cap rows from ring row slot0 on
-    int32_t Hkv, B, n, unit_rows, x_extra;         // x_extra = extra workgroups along x (0: no copy)
+    int32_t Hkv, B, n, unit_rows, x_extra;         // x_extra = extra workgroups along x (repr_keys_kernel; 0: no copy)
 };
 
 // element e = (ring, batch row, kv head, row, 16-byte chunk)

@@ -53,9 +53,8 @@ __device__ __forceinline__ void write_page(const PageList &j, int u, int p, cons
     j.out[(int64_t)u * j.n_pages + p] = pg;
 }
 
-// After a block has carved n_new units: workgroup x scores them under the mean query of the call's block j0 + x; the one
-// of block j_sel ranks that block's list of the call's start against all units carved since, and turns the selection into
-// the block's page table.
+// After a block has carved n_new units: they are scored under the mean queries of the call's blocks from j0 on; block j_sel's
+// list of the call's start is ranked against all units carved since, and the selection becomes the block's page table.
 struct RankJob {
     const bf16_t *reps;
     int64_t rep_sb, rep_su;
@@ -75,61 +74,64 @@ struct RankLds {
     int32_t e_id[kRankEntries], sel[64];
 };
 
-// workgroup x of 256 threads (the sums are unit_scores_rows_kernel's, term by term: a unit's score does not depend on which
-// kernel computed it)
+// 256 threads: scores of the new units under the mean queries of blocks j0 + x0 .. j0 + x0 + nx - 1, and the ranking if the block
+// j_sel is one of them (the sums are unit_scores_rows_kernel's, term by term: a unit's score does not depend on which kernel
+// computed it).  A wave keeps a unit's row and takes the mean queries in turn, each piece of the next one requested as soon as
+// its place is free.
 template <int CPL>
-__device__ __forceinline__ void rank_block(const RankJob &jb, int x, RankLds &lds) {
+__device__ __forceinline__ void rank_blocks(const RankJob &jb, int x0, int nx, RankLds &lds) {
     float *fresh = lds.fresh;
     uint32_t *e_key = lds.e_key;
     int32_t *e_id = lds.e_id, *sel = lds.sel;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, C = jb.C;
-    const int j = jb.j0 + x;
-    const bool is_sel = j == jb.j_sel;
+    const bool is_sel = jb.j_sel >= jb.j0 + x0 && jb.j_sel < jb.j0 + x0 + nx;
     const int n = jb.n_list + jb.first_new + jb.n_new - jb.n_base;
     for (int u = 0; u < jb.B; ++u) {
-        const float *qbar = jb.qbars + ((int64_t)j * jb.B + u) * C;
-        float *scores = jb.scores + ((int64_t)j * jb.B + u) * jb.cols;
         // the ranking threads' entries, asked for ahead of the scoring
         int my_id[2] = {-1, -1};
         float my_score[2] = {0.f, 0.f};
         if (is_sel) {
+            const int64_t row = (int64_t)jb.j_sel * jb.B + u;
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int e = tid + 256 * i;
                 if (e >= n) continue;
-                my_id[i] = e < jb.n_list ? jb.base[((int64_t)j * jb.B + u) * jb.k + e] : jb.n_base + (e - jb.n_list);
-                if (my_id[i] < jb.first_new) my_score[i] = scores[my_id[i]];
+                my_id[i] = e < jb.n_list ? jb.base[row * jb.k + e] : jb.n_base + (e - jb.n_list);
+                if (my_id[i] < jb.first_new) my_score[i] = jb.scores[row * jb.cols + my_id[i]];
             }
         }
-        if (jb.n_new > 0) {
-            float q[CPL][8];
+        for (int r = wave; r < jb.n_new; r += 4) {
+            const bf16_t *row = jb.reps + (int64_t)u * jb.rep_sb + (int64_t)(jb.first_new + r) * jb.rep_su + lane * 8;
+            u32x4 w[CPL];
+            f32x4 q[CPL][2];
 #pragma unroll
-            for (int c = 0; c < CPL; ++c) {
+            for (int c = 0; c < CPL; ++c) w[c] = c * 512 + lane * 8 < C ? *(const u32x4 *)(row + c * 512) : u32x4{0, 0, 0, 0};
+            auto request = [&](int x, int c) {
+                const float *qbar = jb.qbars + ((int64_t)(jb.j0 + x) * jb.B + u) * C + lane * 8 + c * 512;
                 const bool in = c * 512 + lane * 8 < C;
-                const f32x4 lo = in ? *(const f32x4 *)(qbar + c * 512 + lane * 8) : f32x4{0.f, 0.f, 0.f, 0.f};
-                const f32x4 hi = in ? *(const f32x4 *)(qbar + c * 512 + lane * 8 + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int i = 0; i < 4; ++i) q[c][i] = lo[i], q[c][4 + i] = hi[i];
-            }
-            for (int r = wave; r < jb.n_new; r += 4) {
-                const bf16_t *row = jb.reps + (int64_t)u * jb.rep_sb + (int64_t)(jb.first_new + r) * jb.rep_su + lane * 8;
-                u32x4 w[CPL];
+                for (int i = 0; i < 2; ++i) q[c][i] = in ? *(const f32x4 *)(qbar + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+            };
 #pragma unroll
-                for (int c = 0; c < CPL; ++c) w[c] = c * 512 + lane * 8 < C ? *(const u32x4 *)(row + c * 512) : u32x4{0, 0, 0, 0};
+            for (int c = 0; c < CPL; ++c) request(x0, c);
+            for (int x = x0; x < x0 + nx; ++x) {
                 float acc0 = 0.f, acc1 = 0.f;
 #pragma unroll
-                for (int c = 0; c < CPL; ++c)
+                for (int c = 0; c < CPL; ++c) {
+                    asm volatile("" : "+v"(w[c]));               // (kept as it is: unpacked once for all x it would be twice the registers)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        acc0 += bf16_bits_to_f32(w[c][i] & 0xffffu) * q[c][2 * i];
-                        acc1 += bf16_bits_to_f32(w[c][i] >> 16) * q[c][2 * i + 1];
+                        acc0 += bf16_bits_to_f32(w[c][i] & 0xffffu) * q[c][i >> 1][2 * (i & 1)];
+                        acc1 += bf16_bits_to_f32(w[c][i] >> 16) * q[c][i >> 1][2 * (i & 1) + 1];
                     }
+                    if (x + 1 < x0 + nx) request(x + 1, c);
+                }
                 float acc = acc0 + acc1;
 #pragma unroll
                 for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
                 if (lane == 0) {
-                    scores[jb.first_new + r] = acc;
-                    fresh[r] = acc;
+                    jb.scores[((int64_t)(jb.j0 + x) * jb.B + u) * jb.cols + jb.first_new + r] = acc;
+                    if (jb.j0 + x == jb.j_sel) fresh[r] = acc;
                 }
             }
         }

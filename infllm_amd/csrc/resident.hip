@@ -35,10 +35,11 @@ int infllm_attn_merge_blocked(const uint16_t *d_o_part, const float *d_lse_part,
                               void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse, void *stream, int32_t dim);
 int infllm_local_score_dim(const infllm_score_args *a, int32_t dim, void *stream);
 int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream, int32_t dim);
-int infllm_local_score_merged_rank(const infllm_score_args *a, const MergeJob *job, const RankJob *rank, int32_t n_rank, void *stream, int32_t dim);
-int infllm_carve_score(const infllm_score_args *a, const MergeJob *job, const void *d_ring_k_raw, const void *d_ring_v, int64_t t0, int32_t bs, int32_t n_units,
-                       int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
-                       int64_t out_sh, void *stream, int32_t dim);
+bool infllm_block_end_takes(int32_t n, int32_t P, int32_t bs, bool units, bool ring_is_track);
+bool infllm_block_end_ranks(int32_t C, int32_t dim);
+int infllm_block_end(const infllm_score_args *a, const MergeJob *job, const void *d_ring_k_raw, const void *d_ring_v, int64_t t0, int32_t bs, int32_t n_units,
+                     int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
+                     int64_t out_sh, const RankJob *rank, int32_t n_rank, uint32_t *d_ticket, void *stream, int32_t dim);
 int infllm_repr_keys_carve(const float *d_ring_score, const void *d_ring_k_raw, int64_t ring_cap, int32_t B, int32_t H, int32_t Hkv,
                            int64_t t0, int32_t bs, int32_t n_units, int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su,
                            int32_t *d_idx_out, const void *d_ring_v, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
@@ -55,7 +56,7 @@ namespace {
 template <int CPL>
 __global__ __launch_bounds__(256) void rank_kernel(RankJob jb) {
     __shared__ RankLds lds;
-    rank_block<CPL>(jb, blockIdx.x, lds);
+    rank_blocks<CPL>(jb, blockIdx.x, 1, lds);
 }
 
 // the page table of a selection that is already in memory
@@ -341,42 +342,58 @@ infllm_ingest_args ingest_args(const Resident *R, const infllm_resident_call *a,
     return in;
 }
 
-// Init tokens and units that leave the window behind a block ending at b1.  With sc / job the block's scores of those units
-// have not been added yet: the launch that picks their representatives takes them along, and the merge of the block's
-// partials, where it can - units of 32, 64, 96 or 128 tokens (their keys are in LDS), blocks of up to 512 queries (a wave per 32 of
-// them), up to eight partials -; else nothing is done (1 is returned), and scores, representatives and ranking are launches of their own: prompts
-// of 16,001 / 131,072 tokens 3,212 -> 3,313 and 30,565 -> 31,790 us, 24,300 with 36 heads of 64 3,516 -> 3,595.
-int carve(Resident *R, const infllm_resident_call *a, const Carve &c, hipStream_t st, const infllm_score_args *sc = nullptr, MergeJob *job = nullptr) {
+// Init tokens that leave the window behind a block.
+int carve_init(Resident *R, const Carve &c, hipStream_t st) {
+    if (c.take <= 0) return 0;
     const infllm_resident_desc &d = R->d;
-    if (sc && c.count > 0 && (d.block_size % 32 != 0 || d.block_size > 128 || sc->Lq > 512 || job->P > 8)) return 1;
-    if (c.take > 0) {
-        INFLLM_REQUIRE(R->init_len + c.take <= d.init_cap, "resident: init overflow");
-        bf16_t *ik = (bf16_t *)d.d_init_kv + (int64_t)R->init_len * d.dim;
-        const int64_t sh = d.init_cap * d.dim, sb = 2 * (int64_t)d.Hkv * sh;
-        const int rc = infllm_gather_rows_pair(d.d_ring_k_raw, ik, d.d_ring_v, ik + (int64_t)d.Hkv * sh, d.ring_cap, d.B, d.Hkv, R->cursor, c.take, c.take,
-                                               sb, 0, sh, st, d.dim);
-        if (rc) return rc;
-        R->cursor += c.take;
-        R->init_len += c.take;
-    }
-    const int64_t unit_elems = (int64_t)d.Hkv * d.block_size * d.dim;
-    for (int done = 0; done < c.count;) {                     // units of one chunk at a time
-        const int unit = R->n_units, n = std::min(c.count - done, d.units_per_chunk - unit % d.units_per_chunk);
-        INFLLM_REQUIRE(unit + n <= a->n_chunks * d.units_per_chunk && unit + n <= a->rep_rows, "resident: no room for unit %d", unit + n - 1);
-        bf16_t *home = unit_home(R, a, unit);
-        const int rc = sc ? infllm_carve_score(sc, job, d.d_ring_k_raw, d.d_ring_v, R->cursor, d.block_size, n, d.repr_topk,
-                                               (bf16_t *)a->d_reps + unit * a->rep_su, a->rep_sb, a->rep_su, home, home + unit_elems, 2 * unit_elems,
-                                               (int64_t)d.B * 2 * unit_elems, (int64_t)d.block_size * d.dim, st, d.dim)
-                          : infllm_repr_keys_carve(d.d_ring_score, d.d_ring_k_raw, d.ring_cap, d.B, d.H, d.Hkv, R->cursor, d.block_size, n, d.repr_topk,
-                                              (bf16_t *)a->d_reps + unit * a->rep_su, a->rep_sb, a->rep_su, nullptr, d.d_ring_v, home, home + unit_elems,
-                                              2 * unit_elems, (int64_t)d.B * 2 * unit_elems, (int64_t)d.block_size * d.dim, st, d.dim);
-        if (rc) return rc < 0 ? rc : infllm_fail(-2, "resident: no carving kernel after the checks");
-        if (sc) job->out = nullptr;                               // merged along with the first of them
-        R->cursor += (int64_t)n * d.block_size;
-        R->n_units += n;
-        done += n;
-    }
+    INFLLM_REQUIRE(R->init_len + c.take <= d.init_cap, "resident: init overflow");
+    bf16_t *ik = (bf16_t *)d.d_init_kv + (int64_t)R->init_len * d.dim;
+    const int64_t sh = d.init_cap * d.dim, sb = 2 * (int64_t)d.Hkv * sh;
+    const int rc = infllm_gather_rows_pair(d.d_ring_k_raw, ik, d.d_ring_v, ik + (int64_t)d.Hkv * sh, d.ring_cap, d.B, d.Hkv, R->cursor, c.take, c.take, sb, 0,
+                                           sh, st, d.dim);
+    if (rc) return rc;
+    R->cursor += c.take;
+    R->init_len += c.take;
     return 0;
+}
+
+// Units that one launch carves: those from position t0 on, at most n and of one chunk.  The state moves on behind them.
+struct UnitRun {
+    int32_t n = 0;
+    int64_t t0 = 0;
+    bf16_t *rep = nullptr, *home_k = nullptr, *home_v = nullptr;
+};
+int next_run(Resident *R, const infllm_resident_call *a, int n, UnitRun *run) {
+    const infllm_resident_desc &d = R->d;
+    *run = UnitRun{};
+    if (n <= 0) return 0;
+    const int unit = R->n_units;
+    run->n = std::min(n, d.units_per_chunk - unit % d.units_per_chunk);
+    INFLLM_REQUIRE(unit + run->n <= a->n_chunks * d.units_per_chunk && unit + run->n <= a->rep_rows, "resident: no room for unit %d", unit + run->n - 1);
+    run->t0 = R->cursor;
+    run->rep = (bf16_t *)a->d_reps + unit * a->rep_su;
+    run->home_k = unit_home(R, a, unit);
+    run->home_v = run->home_k + (int64_t)d.Hkv * d.block_size * d.dim;
+    R->cursor += (int64_t)run->n * d.block_size;
+    R->n_units += run->n;
+    return 0;
+}
+
+// Init tokens and units that leave the window, with scores that are complete.
+int carve(Resident *R, const infllm_resident_call *a, const Carve &c, hipStream_t st) {
+    const infllm_resident_desc &d = R->d;
+    int rc = carve_init(R, c, st);
+    const int64_t unit_elems = (int64_t)d.Hkv * d.block_size * d.dim;
+    UnitRun run;
+    for (int done = 0; done < c.count && !rc; done += run.n) {
+        rc = next_run(R, a, c.count - done, &run);
+        if (rc) return rc;
+        rc = infllm_repr_keys_carve(d.d_ring_score, d.d_ring_k_raw, d.ring_cap, d.B, d.H, d.Hkv, run.t0, d.block_size, run.n, d.repr_topk, run.rep, a->rep_sb,
+                                    a->rep_su, nullptr, d.d_ring_v, run.home_k, run.home_v, 2 * unit_elems, (int64_t)d.B * 2 * unit_elems,
+                                    (int64_t)d.block_size * d.dim, st, d.dim);
+        if (rc > 0) return infllm_fail(-2, "resident: no carving kernel after the checks");
+    }
+    return rc;
 }
 
 // one query
@@ -650,29 +667,44 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             if (rc) return rc;
             parts += ns_g;
         }
-        // ---- merge and local score, in one launch where the key range is long enough
+        // ---- what ends the block
         bf16_t *out = (bf16_t *)a->d_out + (st0 + (int64_t)i * exc) * a->o_sl;
         MergeJob job;
         rc = infllm_merge_job(o_loc, lse_loc, nsplit, ns_g ? a->d_o_part2 : nullptr, ns_g ? a->d_lse_part2 : nullptr, ns_g, B, d.H, nb, out, a->o_sb, a->o_sh,
                               a->o_sl, a->d_lse, &job, D);
         if (rc) return rc;
         infllm_score_args sc = score_args((int64_t)i * exc, nb, lo, b1);
-        // What the next block waits for comes first where there is a kernel for it - the scores and representatives of the units
-        // that leave the window now, in one launch that merges the block's partials along the way -, then the rest of the scores,
-        // with the ranking riding along.
+        // Blocks with a kernel for it - long key ranges, up to eight partials, up to 512 queries and units of 32, 64, 96 or 128
+        // tokens where units leave - end in one launch (infllm_block_end): scores, merge, the units that leave and the next
+        // block's ranking.  The others' scores with the merge, carving and ranking are launches of their own.  (Prompts of 16,001 /
+        // 131,072 tokens, 24,300 with 36 heads of 64: two launches, carving in front of the scores, 3,035 / 29,430 / 3,468 us, one
+        // 2,882 / 28,140 / 3,400.)
         const Carve c = carve_after(d, R->cursor, R->init_len, b1);
-        const bool one = parts <= 8 && b1 - lo > 1024;               // (the form that carries them takes long key ranges)
-        rc = one ? carve(R, a, c, st, &sc, &job) : 1;
-        if (rc < 0) return rc;
-        const bool early = rc == 0;
-        if (!early) {
-            rc = one ? infllm_local_score_merged(&sc, &job, st, D) : 1;
+        const bool early = b1 - lo > 1024 && infllm_block_end_takes(nb, parts, d.block_size, c.count > 0, true);
+        UnitRun run;
+        auto end_block = [&](const infllm_score_args &s, const RankJob *rank, int n_rank) {
+            const int64_t unit_elems = (int64_t)d.Hkv * d.block_size * d.dim;
+            return infllm_block_end(&s, &job, d.d_ring_k_raw, d.d_ring_v, run.t0, d.block_size, run.n, d.repr_topk, run.rep, a->rep_sb, a->rep_su, run.home_k,
+                                    run.home_v, 2 * unit_elems, (int64_t)d.B * 2 * unit_elems, (int64_t)d.block_size * d.dim, rank, n_rank, a->d_ticket, st, D);
+        };
+        if (early) {
+            rc = carve_init(R, c, st);
+            if (!rc) rc = next_run(R, a, c.count, &run);
+            for (int done = run.n; !rc && done < c.count; done += run.n) {      // (units of several chunks: all but the last chunk's ahead)
+                infllm_score_args none = sc;
+                none.j_lo = none.j_hi;
+                rc = end_block(none, nullptr, 0);
+                job.out = nullptr;                                               // merged along with the first of them
+                if (!rc) rc = next_run(R, a, c.count - done, &run);
+            }
+            if (rc) return rc;
+        } else {
+            rc = parts <= 8 ? infllm_local_score_merged(&sc, &job, st, D) : 1;
             if (rc < 0) return rc;
             if (rc == 1) {
                 rc = infllm_attn_merge2(o_loc, lse_loc, nsplit, ns_g ? a->d_o_part2 : nullptr, ns_g ? a->d_lse_part2 : nullptr, ns_g, B, d.H, nb, out,
                                         a->o_sb, a->o_sh, a->o_sl, a->d_lse, st, D);
-                if (rc) return rc;
-                rc = infllm_local_score_dim(&sc, D, st);
+                if (!rc) rc = infllm_local_score_dim(&sc, D, st);
                 if (rc) return rc;
             }
             rc = carve(R, a, c, st);
@@ -705,17 +737,10 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
         bool ranked = !rank;
         if (early) {
             sc.j_lo = std::max(lo, R->cursor);
-            const bool carry = rank && C <= 9 * 512 && b1 - sc.j_lo > 1024;
-            rc = carry ? infllm_local_score_merged_rank(&sc, &job, &jb, n_rank, st, D) : infllm_local_score_merged(&sc, &job, st, D);
-            if (rc < 0) return rc;
+            const bool carry = rank && infllm_block_end_ranks(C, D);
+            rc = end_block(sc, carry ? &jb : nullptr, n_rank);
+            if (rc) return rc;
             ranked = ranked || carry;
-            if (rc == 1) {                                           // a short window once the units have left it
-                rc = job.out ? infllm_attn_merge2(o_loc, lse_loc, nsplit, ns_g ? a->d_o_part2 : nullptr, ns_g ? a->d_lse_part2 : nullptr, ns_g, B, d.H, nb,
-                                                  out, a->o_sb, a->o_sh, a->o_sl, a->d_lse, st, D) : 0;
-                if (rc) return rc;
-                rc = infllm_local_score_dim(&sc, D, st);
-                if (rc) return rc;
-            }
         }
         if (!ranked) {
             rc = launch_rank(R, jb, n_rank, st);
@@ -807,7 +832,7 @@ extern "C" int infllm_resident_append(void *handle, const infllm_resident_call *
             INFLLM_REQUIRE(a->d_logits, "resident_append: null logits");
             rc = decode_step(R, a, pos, st);
         } else {
-            INFLLM_REQUIRE(a->d_qpart && a->d_o_part2 && a->d_lse_part2 && a->d_lse && a->d_base, "resident_append: null pointer");
+            INFLLM_REQUIRE(a->d_qpart && a->d_o_part2 && a->d_lse_part2 && a->d_lse && a->d_base && a->d_ticket, "resident_append: null pointer");
             rc = prompt_call(R, a, pos, n, st);
         }
         if (rc) return rc;

@@ -26,50 +26,20 @@ constexpr int kQPad = D + 8;               // LDS row of Q (bf16 elements): 272 
 // launch is a chain of stages that each wait for one global load (there is next to no arithmetic to hide it behind),
 // so it takes stages of 128 queries and half as many of them.
 //
-// MERGE: the launch also carries the merge of the block's partial attention outputs: every scoring workgroup merges
-// two (row, 8 dims) pieces per thread (merge_issue / merge_finish of common.h) while it waits for its keys.  The two
-// kinds of work do not depend on each other - the scoring workgroups join the partial log-sum-exps themselves, by
-// the merge's own arithmetic - and the merge is a handful of loads per thread that are in flight during a wait the
-// workgroup has anyway: one launch instead of two on the chain from one block's selection to the next, and no
-// workgroups of its own that would queue for the scoring workgroups' places.  In this form the joined log-sum-exps of
-// ALL the launch's queries are put into LDS once, in the same wait, instead of stage by stage.
+// MERGE: the launch also carries the merge of the block's partial attention outputs, in workgroups behind the scoring ones.
+// The two kinds of work do not depend on each other - the scoring workgroups join the partial log-sum-exps themselves, by
+// the merge's own arithmetic, those of ALL the launch's queries at once in the wait for their keys.
 struct ScoreMerge {
     MergeJob job;
     int32_t score_tiles;               // blockIdx.y below this scores, from there on merges
 };
-// RANK: the launch also ranks the units for the next block (rank.h), in workgroups of their own that are dispatched first:
-// a chain of latencies that needs next to nothing of the chip, and that the scores do not depend on
-struct ScoreMergeRank : ScoreMerge {
-    RankJob rank;
-    int32_t rank_slots, n_rank;        // rows of the grid in front that rank; workgroups in them with something to do
-};
 struct NoScoreMerge {};
-constexpr int kScore = 0, kScoreMerge = 1, kScoreMergeRank = 2;
 
-template <int D, int KS, int QS, int WITH = kScore>
-__global__ __launch_bounds__(256, 2) void local_score_kernel(
-    infllm_score_args a, std::conditional_t<WITH == kScoreMergeRank, ScoreMergeRank, std::conditional_t<WITH == kScoreMerge, ScoreMerge, NoScoreMerge>> sm) {
-    constexpr bool MERGE = WITH != kScore;
+// One workgroup of 256 threads: tile `slot` (in the order they are dispatched) of n_tiles of the keys, query head bx.  MERGE:
+// the joined log-sum-exps of all the queries go into LDS once, from the partial ones at a.d_lse + lps.
+template <int D, int KS, int QS, bool MERGE>
+__device__ __forceinline__ void score_tile(const infllm_score_args &a, const PartSets lps, int bx, int slot, int n_tiles, char *score_lds) {
     constexpr int kWaveKeys = 32 * KS, kKeysPerWg = 4 * kWaveKeys, kQStage = QS;
-    int n_tiles = gridDim.y, slot = blockIdx.y;
-    PartSets lps{a.n_parts, 0, 0};
-    extern __shared__ __attribute__((aligned(16))) char score_lds[];
-    if constexpr (WITH == kScoreMergeRank) {
-        slot -= sm.rank_slots;
-        if (slot < 0) {
-            const int x = (int)blockIdx.y * gridDim.x + blockIdx.x;
-            if (x < sm.n_rank) rank_block<9>(sm.rank, x, *(RankLds *)score_lds);
-            return;
-        }
-    }
-    if constexpr (MERGE) {
-        n_tiles = sm.score_tiles;
-        if (slot >= n_tiles) {
-            merge_piece<D>(sm.job, ((int64_t)(slot - n_tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x);
-            return;
-        }
-        lps = sm.job.ps;
-    }
     bf16_t(*Qs)[kQStage][kQPad<D>] = (bf16_t(*)[kQStage][kQPad<D>])score_lds;                               // [2][QS][kQPad]
     float(*Ls)[kQStage] = (float(*)[kQStage])(score_lds + 2 * kQStage * kQPad<D> * sizeof(bf16_t));      // [2][QS]
     [[maybe_unused]] float *Lall = (float *)Ls;                                                        // MERGE: [Lq rounded up to QS]
@@ -77,10 +47,10 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int col = lane & 31, grp = lane >> 5;
     const int G = a.H / a.Hkv;
-    // blockIdx.x walks the kv heads first, then the query heads of a group: workgroups go to the 8 XCDs round-robin by
+    // bx walks the kv heads first, then the query heads of a group: workgroups go to the 8 XCDs round-robin by
     // linear id, so with 8 (16, ...) kv heads the query heads that share a K tile sit behind the same L2 and that tile
     // leaves HBM once instead of once per query head
-    const int b = blockIdx.x / a.H, hx = blockIdx.x % a.H, g = hx % a.Hkv, h = g * G + hx / a.Hkv;
+    const int b = bx / a.H, hx = bx % a.H, g = hx % a.Hkv, h = g * G + hx / a.Hkv;
     // Workgroups are dispatched x fastest: all heads of one key tile, then the next tile.  The two tiles at either end
     // of a masked key range see only part of the queries and finish early, so they go last: when the grid is a little
     // more than what the chip holds at once, the workgroups that start late are then the short ones.
@@ -220,7 +190,7 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(
         // A stage with pairs that are masked takes the same form with a select behind every exponential: it costs a third more
         // than an unmasked one, where sub-tiles looked at one by one (and left out where nothing was visible) cost twice as
         // much - and the workgroups on the diagonal end a launch.  Together with two queries' log-sum-exps per trip to memory: the
-        // operator over 512 queries x (4,608 + 2,624) keys 112.5 -> 106.8 us, a prompt of 131,072 tokens 29,680 -> 28,930.
+        // operator over 512 queries x (4,608 + 2,624) keys 112.5 -> 106.8 us, a prompt of 131,072 tokens 29,520 -> 28,935.
         auto stage = [&](auto masked) {
             constexpr int kSub = kQStage / 32;
             constexpr bool kMasked = decltype(masked)::value;
@@ -305,6 +275,238 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(
     }
 }
 
+template <int D, int KS, int QS, bool MERGE = false>
+__global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a, std::conditional_t<MERGE, ScoreMerge, NoScoreMerge> sm) {
+    extern __shared__ __attribute__((aligned(16))) char score_lds[];
+    if constexpr (MERGE) {
+        const int slot = blockIdx.y;
+        if (slot >= sm.score_tiles) {
+            merge_piece<D>(sm.job, ((int64_t)(slot - sm.score_tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x);
+            return;
+        }
+        score_tile<D, KS, QS, true>(a, sm.job.ps, blockIdx.x, slot, sm.score_tiles, score_lds);
+    } else
+        score_tile<D, KS, QS, false>(a, PartSets{a.n_parts, 0, 0}, blockIdx.x, blockIdx.y, gridDim.y, score_lds);
+}
+
+// What ends a block, in one launch: the scores of its keys, the merge of its partial outputs, the units that leave the window
+// with it (their rows to their home, their representatives) and the next block's selection and page table.
+//
+// The next block waits for a chain of latencies in it that needs little of the chip: the block's share of the scores of the
+// keys that leave -> the representatives of the units they make up (context_manager.py:268-277) -> the ranking.  The rest - the
+// scores of the keys that stay, the merge, the units' rows - depends on none of it and fills the chip meanwhile.  So the
+// carving workgroups (one per unit and head: 128 keys x 512 queries, half of them outside the window) come first in the grid;
+// the one that is done last ranks.  As two launches, carving with the merge and the rest of the scores with the ranking, which
+// can begin when the first has ended: 5 us a block of 512 queries x 4,096 keys x 32 heads more (17.2 + 28).
+//
+// A carving workgroup's steps are as short as they can be: everything it reads is requested at once; the unit's keys are in
+// LDS (every wave needs them all), four sub-tiles of 32 queries a wave take turns with each of them; a sub-tile's column sums
+// are added in the order of the queries, as score_tile adds them (the same bits); the picks by counting, all rows at once.
+constexpr int kCarveMaxLq = 512, kCarveMaxUnit = 128;
+struct BlockEnd {
+    infllm_score_args s;               // the keys that stay
+    MergeJob merge;                    // the block's partials (out NULL: merged before)
+    int32_t n_carve, n_score, n_copy, n_rank;      // workgroups of each kind, in this order, those that merge behind them; blocks to rank for (0: none)
+    // units that leave
+    const bf16_t *ring_k_raw;
+    int32_t slot0, cap, to_first;      // ring row of the first unit; dist of query 0 to the first unit's first key
+    int32_t win, bs, n_units, repr_topk;
+    bf16_t *rep_out;
+    int64_t rep_sb, rep_su;
+    CarveCopy cc;
+    RankJob rank;
+    uint32_t *ticket;                  // zero; the last of the carving workgroups to finish puts it back
+};
+
+template <int D>
+struct CarveLds {
+    bf16_t keys[kCarveMaxUnit * D];                // chunk c of row r at c ^ (r mod kChunks)
+    float lse[kCarveMaxLq];
+    float sums[kCarveMaxLq / 32][2][kCarveMaxUnit];
+    uint64_t rank_key[kCarveMaxUnit];
+    int32_t chosen[kCarveMaxUnit];
+};
+
+template <int D>
+__device__ __forceinline__ void carve_unit(const BlockEnd &j, int h, int u, int b, CarveLds<D> &lds) {
+    constexpr int kChunks = D / 8, kSubs = kCarveMaxLq / 32 / 4;                   // sub-tiles a wave
+    const infllm_score_args &a = j.s;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 31, grp = lane >> 5;
+    const int g = h / (a.H / a.Hkv), bs = j.bs;
+    const float scale = a.softmax_scale * 1.4426950408889634f;
+    auto slot_of = [&](int r) {                                   // ring row of row r of the unit
+        const int s = j.slot0 + u * bs + r;
+        return s < j.cap ? s : s - j.cap;
+    };
+    // queries that see any of the unit's keys: i < n_q (they all lie behind the keys); sub-tiles wave, wave + 4, .. are this wave's
+    const int d_first = j.to_first - u * bs;                      // distance of query 0 to the unit's first key
+    const int n_q = max(min(a.Lq, j.win + bs - 1 - d_first), 0), n_sub = (n_q + 31) / 32;
+    bf16x8 qa[kSubs][D / 16];
+#pragma unroll
+    for (int i = 0; i < kSubs; ++i)
+        if (wave + 4 * i < n_sub) {
+            const bf16_t *row = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh +
+                                (int64_t)min((wave + 4 * i) * 32 + col, a.Lq - 1) * a.q_sl + grp * 8;
+#pragma unroll
+            for (int kk = 0; kk < D / 16; ++kk) qa[i][kk] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(row + kk * 16));
+        }
+    constexpr int kLoads = kCarveMaxUnit * kChunks / 256;
+    u32x4 rows[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int r = (tid + i * 256) / kChunks, c = tid % kChunks;
+        if (r < bs) rows[i] = *(const u32x4 *)((const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + (int64_t)slot_of(r) * a.k_sl + c * 8);
+    }
+    float track = 0.f;
+    if (tid < bs) track = a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + slot_of(tid)];
+    {                                                            // joined log-sum-exps (score_tile's join), two queries a thread
+        const int64_t all = (int64_t)a.B * a.H * a.Lq;
+        const float *lse = a.d_lse + ((int64_t)b * a.H + h) * a.Lq;
+        float l8[2][8];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int p = 0; p < 8; ++p) l8[e][p] = tid + e * 256 < min(n_sub * 32, a.Lq) && p < a.n_parts ? lse[j.merge.ps.l(p, all) + tid + e * 256] : -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            float m8 = -INFINITY, den = 0.f;
+#pragma unroll
+            for (int p = 0; p < 8; ++p) m8 = fmaxf(m8, l8[e][p]);
+            if (m8 != -INFINITY) {
+#pragma unroll
+                for (int p = 0; p < 8; ++p) den += __builtin_amdgcn_exp2f(l8[e][p] - m8);
+            }
+            lds.lse[tid + e * 256] = den > 0.f ? m8 + log2f(den) : INFINITY;      // +inf => probability 0
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int r = (tid + i * 256) / kChunks, c = tid % kChunks;
+        if (r < bs) *(u32x4 *)&lds.keys[(r * kChunks + (c ^ (r % kChunks))) * 8] = rows[i];
+    }
+    __syncthreads();
+    for (int kg = 0; kg < bs / 32; ++kg) {
+        const bf16_t *krow = &lds.keys[(kg * 32 + col) * D];
+        f32x16 s[kSubs];
+#pragma unroll
+        for (int i = 0; i < kSubs; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[i][r] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) {
+            const bf16x8 key = *(const bf16x8 *)(krow + ((kk * 2 + grp) ^ (col % kChunks)) * 8);
+#pragma unroll
+            for (int i = 0; i < kSubs; ++i)
+                if (wave + 4 * i < n_sub) s[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[i][kk], key, s[i], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < kSubs; ++i) {
+            const int sub = wave + 4 * i;
+            if (sub >= n_sub) break;
+            f32x4 l4[4];
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) l4[q4] = *(const f32x4 *)&lds.lse[sub * 32 + 8 * q4 + 4 * grp];
+            const int e0 = d_first + sub * 32 - kg * 32;         // distance of the sub-tile's first query to the group's first key
+            float acc = 0.f;
+            if (e0 - 31 >= 0 && e0 + 31 < j.win) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc += __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][r], scale, -l4[r >> 2][r & 3]));
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int dist = e0 - col + 8 * (r >> 2) + 4 * grp + (r & 3);
+                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][r], scale, -l4[r >> 2][r & 3]));
+                    acc += dist >= 0 && dist < j.win ? p : 0.f;
+                }
+            }
+            lds.sums[sub][grp][kg * 32 + col] = acc;
+        }
+    }
+    __syncthreads();
+    // ---- the representatives: row r's place in the order is the number of rows in front of it
+    if (tid < kCarveMaxUnit) {
+        uint64_t key = 0;
+        if (tid < bs) {
+            float lo = 0.f, hi = 0.f;
+            if (n_sub == kCarveMaxLq / 32) {
+#pragma unroll
+                for (int st = 0; st < kCarveMaxLq / 32; ++st) lo += lds.sums[st][0][tid], hi += lds.sums[st][1][tid];
+            } else {
+#pragma unroll 4
+                for (int st = 0; st < n_sub; ++st) lo += lds.sums[st][0][tid], hi += lds.sums[st][1][tid];
+            }
+            key = pick_key(track + (lo + hi), tid);
+        }
+        lds.rank_key[tid] = key;
+    }
+    __syncthreads();
+    {
+        constexpr int kLanes = 256 / kCarveMaxUnit;              // lanes that count for a row
+        const int r = tid / kLanes, p = tid % kLanes;
+        const uint64_t own = lds.rank_key[r];
+        int before = 0;
+#pragma unroll 16
+        for (int i = 0; i < kCarveMaxUnit / kLanes; ++i) before += lds.rank_key[i * kLanes + p] > own;
+#pragma unroll
+        for (int o = 1; o < kLanes; o <<= 1) before += __shfl_xor(before, o, 64);
+        if (p == 0 && r < bs && before < j.repr_topk) lds.chosen[before] = r;
+    }
+    __syncthreads();
+    if (tid * 2 < D) {
+        const bf16_t *raw = j.ring_k_raw + ((int64_t)b * a.Hkv + g) * j.cap * D + tid * 2;
+        float a0 = 0.f, a1 = 0.f;
+#pragma unroll 4
+        for (int i = 0; i < j.repr_topk; ++i) {
+            const uint32_t w = *(const uint32_t *)(raw + (int64_t)slot_of(lds.chosen[i]) * D);
+            a0 += bf16_bits_to_f32(w & 0xffffu);
+            a1 += bf16_bits_to_f32(w >> 16);
+        }
+        const float inv = 1.f / (float)j.repr_topk;
+        // performed at the level of the memory hierarchy that all XCDs share: the workgroup that ranks reads it there
+        __hip_atomic_store((uint32_t *)(j.rep_out + (int64_t)b * j.rep_sb + (int64_t)u * j.rep_su + (int64_t)h * D + tid * 2), pack_bf16x2(a0 * inv, a1 * inv),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// Rows of representatives that the ranking takes, in 512s: 36 heads of 128, 40 of 64.  (Registers: heads of 64 with 32 keys a wave
+// are three workgroups to a CU, which leaves 168 of them.)
+template <int D>
+constexpr int kRankCpl = D == 64 ? 5 : 9;
+
+template <int D, int KS>
+__global__ __launch_bounds__(256, (D == 64 && KS == 1 ? 3 : 2)) void block_end_kernel(BlockEnd j) {
+    extern __shared__ __attribute__((aligned(16))) char score_lds[];
+    __shared__ int last;
+    int x = blockIdx.x;
+    if (x < j.n_carve) {
+        if (j.n_units > 0) {
+            const int rest = x / j.s.H;
+            carve_unit<D>(j, x - rest * j.s.H, rest % j.n_units, rest / j.n_units, *(CarveLds<D> *)score_lds);
+            if (j.n_rank == 0) return;
+            // The representatives are the only thing that crosses workgroups, and their stores have been performed where every
+            // XCD sees them before the ticket is drawn: no workgroup has to write its L2 back.
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (threadIdx.x == 0) last = __hip_atomic_fetch_add(j.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)j.n_carve - 1;
+            __syncthreads();
+            if (!last) return;
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            if (threadIdx.x == 0) __hip_atomic_store(j.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        rank_blocks<kRankCpl<D>>(j.rank, 0, j.n_rank, *(RankLds *)score_lds);
+        return;
+    }
+    x -= j.n_carve;
+    if (x < j.n_score) {
+        const int rows = j.s.B * j.s.H;
+        score_tile<D, KS, 128, true>(j.s, j.merge.ps, x % rows, x / rows, j.n_score / rows, score_lds);
+        return;
+    }
+    x -= j.n_score;
+    if (x < j.n_copy) carve_copy<D>(j.cc, (int64_t)x * 256 + threadIdx.x);
+    else merge_piece<D>(j.merge, (int64_t)(x - j.n_copy) * 256 + threadIdx.x);
+}
+
 }  // namespace
 
 namespace {
@@ -342,8 +544,8 @@ int score_lds_setup() {
         if (e == hipSuccess)
             e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)score_lds_bytes<D>(128));
-        for (const void *k : {(const void *)local_score_kernel<D, 2, 128, kScoreMerge>, (const void *)local_score_kernel<D, 2, 128, kScoreMergeRank>,
-                              (const void *)local_score_kernel<D, 1, 128, kScoreMerge>, (const void *)local_score_kernel<D, 1, 128, kScoreMergeRank>})
+        for (const void *k : {(const void *)local_score_kernel<D, 2, 128, true>, (const void *)local_score_kernel<D, 1, 128, true>,
+                              (const void *)block_end_kernel<D, 2>, (const void *)block_end_kernel<D, 1>})
             if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)score_lds_bytes_merged<D>(128, kMergedMaxLq));
         if (e != hipSuccess) return infllm_fail(-2, "local_score: %s", hipGetErrorString(e));
         lds_set.store(true, std::memory_order_release);
@@ -379,7 +581,7 @@ int score_launch(const infllm_score_args *a, void *stream) {
 }
 
 template <int D>
-int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *stream, const RankJob *rank = nullptr, int n_rank = 0) {
+int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *stream) {
     INFLLM_REQUIRE(a && job, "local_score_merged: null argument");
     INFLLM_REQUIRE(job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1 && job->P <= 8,
                    "local_score_merged: the merge does not belong to these queries");
@@ -397,230 +599,94 @@ int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *s
     const int score_tiles = (int)((tiles + 3) / 4);
     const int64_t merge_wgs = ((int64_t)job->B * job->H * job->Lq * (D / 8) + 255) / 256;
     const int gx = sc.B * sc.H;
-    const int merge_slots = job->out ? (int)((merge_wgs + gx - 1) / gx) : 0;      // (none: the job has been done by then)
-    if (rank) {
-        INFLLM_REQUIRE(rank->C <= 9 * 512 && rank->C % 8 == 0 && n_rank >= 1, "local_score_merged: no ranking for rows of %d elements", rank->C);
-        ScoreMergeRank sm;
-        sm.job = *job;
-        sm.score_tiles = score_tiles;
-        sm.rank = *rank;
-        sm.n_rank = n_rank;
-        sm.rank_slots = (n_rank + gx - 1) / gx;
-        const auto kern = wide ? local_score_kernel<D, 2, 128, kScoreMergeRank> : local_score_kernel<D, 1, 128, kScoreMergeRank>;
-        hipLaunchKernelGGL(kern, dim3(gx, (unsigned)(sm.rank_slots + score_tiles + merge_slots)), dim3(256), score_lds_bytes_merged<D>(128, sc.Lq),
-                           (hipStream_t)stream, sc, sm);
-        INFLLM_CHECK_LAUNCH("local_score_merged");
-        return 0;
-    }
-    const auto kern = wide ? local_score_kernel<D, 2, 128, kScoreMerge> : local_score_kernel<D, 1, 128, kScoreMerge>;
+    const int merge_slots = (int)((merge_wgs + gx - 1) / gx);
+    const auto kern = wide ? local_score_kernel<D, 2, 128, true> : local_score_kernel<D, 1, 128, true>;
     hipLaunchKernelGGL(kern, dim3(gx, (unsigned)(score_tiles + merge_slots)), dim3(256), score_lds_bytes_merged<D>(128, sc.Lq), (hipStream_t)stream, sc,
                        ScoreMerge{*job, score_tiles});
     INFLLM_CHECK_LAUNCH("local_score_merged");
     return 0;
 }
 
-// The keys that leave the window behind this block: the block's share of their scores, added to what the earlier blocks left
-// in the track, and at once the representatives of the units they make up (context_manager.py:268-277) - what the next
-// block's retrieval waits for, in one launch in front of the rest of the scores.  A chain of latencies with little work in
-// it (a workgroup per unit and head: 128 keys x 512 queries, half of them outside the window), so each step is as short as
-// it can be: a wave per sub-tile of 32 queries, whose rows are requested at once together with everything else the kernel
-// reads; the unit's keys in LDS (every wave needs them all); a sub-tile's column sums added in the order of the queries, as
-// local_score_kernel adds them (the same bits); the picks by counting, all rows at once.  The workgroups behind the heads'
-// copy the units' rows to their home and merge the block's partial outputs: independent work for a chip that is half idle.
-constexpr int kCarveMaxLq = 512, kCarveMaxUnit = 128;
-struct CarveScore {
-    infllm_score_args s;
-    MergeJob merge;
-    const bf16_t *ring_k_raw;
-    int32_t slot0, cap, to_first;      // ring row of the first unit; dist of query 0 to the first unit's first key
-    int32_t win, bs, n_units, repr_topk;
-    bf16_t *rep_out;
-    int64_t rep_sb, rep_su;
-    CarveCopy cc;
-};
-
-template <int D>
-__global__ __launch_bounds__(1024) void carve_score_kernel(CarveScore j) {
-    constexpr int kChunks = D / 8;
-    __shared__ __attribute__((aligned(16))) bf16_t keys[kCarveMaxUnit * D];        // chunk c of row r at c ^ (r mod kChunks)
-    __shared__ float lse_sh[kCarveMaxLq];
-    __shared__ float sums[kCarveMaxLq / 32][2][kCarveMaxUnit];
-    __shared__ uint64_t rank_key[kCarveMaxUnit];
-    __shared__ int32_t chosen[kCarveMaxUnit];
-    const infllm_score_args &a = j.s;
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 31, grp = lane >> 5;
-    if ((int)blockIdx.x >= a.H) {
-        const int x = (int)blockIdx.x - a.H;
-        const int64_t wg = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
-        if (x < j.cc.x_extra) carve_copy<D>(j.cc, (wg * j.cc.x_extra + x) * 1024 + tid);
-        else merge_piece<D>(j.merge, (wg * ((int)gridDim.x - a.H - j.cc.x_extra) + (x - j.cc.x_extra)) * 1024 + tid);
-        return;
-    }
-    const int h = blockIdx.x, u = blockIdx.y, b = blockIdx.z, g = h / (a.H / a.Hkv), bs = j.bs;
-    const float scale = a.softmax_scale * 1.4426950408889634f;
-    auto slot_of = [&](int r) {                                   // ring row of row r of the unit
-        const int s = j.slot0 + u * bs + r;
-        return s < j.cap ? s : s - j.cap;
-    };
-    // queries that see any of the unit's keys: i < n_q (they all lie behind the keys), one sub-tile of 32 a wave
-    const int d_first = j.to_first - u * bs;                      // distance of query 0 to the unit's first key
-    const int n_q = max(min(a.Lq, j.win + bs - 1 - d_first), 0), n_sub = (n_q + 31) / 32;
-    const bool works = wave < n_sub;
-    bf16x8 qa[D / 16];
-    if (works) {
-        const bf16_t *row = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)min(wave * 32 + col, a.Lq - 1) * a.q_sl + grp * 8;
-#pragma unroll
-        for (int kk = 0; kk < D / 16; ++kk) qa[kk] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(row + kk * 16));
-    }
-    constexpr int kLoads = kCarveMaxUnit * kChunks / 1024;
-    u32x4 k_in[kLoads], raw_in[kLoads];
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-        const int r = (tid + i * 1024) / kChunks, c = tid % kChunks;
-        if (r >= bs) continue;
-        const int64_t at = (int64_t)slot_of(r);
-        k_in[i] = *(const u32x4 *)((const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + at * a.k_sl + c * 8);
-        raw_in[i] = *(const u32x4 *)(j.ring_k_raw + (((int64_t)b * a.Hkv + g) * j.cap + at) * D + c * 8);
-    }
-    float track = 0.f;
-    if (tid < bs) track = a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + slot_of(tid)];
-    if (tid < n_sub * 32) {                                      // joined log-sum-exps (local_score_kernel's join)
-        const int64_t rows = (int64_t)a.B * a.H * a.Lq;
-        const float *lse = a.d_lse + ((int64_t)b * a.H + h) * a.Lq;
-        float l8[8], m8 = -INFINITY, den = 0.f;
-#pragma unroll
-        for (int p = 0; p < 8; ++p) l8[p] = tid < a.Lq && p < a.n_parts ? lse[j.merge.ps.l(p, rows) + tid] : -INFINITY;
-#pragma unroll
-        for (int p = 0; p < 8; ++p) m8 = fmaxf(m8, l8[p]);
-        if (m8 != -INFINITY) {
-#pragma unroll
-            for (int p = 0; p < 8; ++p) den += __builtin_amdgcn_exp2f(l8[p] - m8);
-        }
-        lse_sh[tid] = den > 0.f ? m8 + log2f(den) : INFINITY;    // +inf => probability 0
-    }
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-        const int r = (tid + i * 1024) / kChunks, c = tid % kChunks;
-        if (r < bs) *(u32x4 *)&keys[(r * kChunks + (c ^ (r % kChunks))) * 8] = k_in[i];
-    }
-    __syncthreads();
-    if (works) {
-        f32x4 l4[4];
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) l4[q4] = *(const f32x4 *)&lse_sh[wave * 32 + 8 * q4 + 4 * grp];
-        for (int kg = 0; kg < bs / 32; ++kg) {
-            const bf16_t *krow = &keys[(kg * 32 + col) * D];
-            f32x16 s;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = 0.f;
-#pragma unroll
-            for (int kk = 0; kk < D / 16; ++kk)
-                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[kk], *(const bf16x8 *)(krow + ((kk * 2 + grp) ^ (col % kChunks)) * 8), s, 0, 0, 0);
-            const int e0 = d_first + wave * 32 - kg * 32;        // distance of the sub-tile's first query to the group's first key
-            float acc = 0.f;
-            if (e0 - 31 >= 0 && e0 + 31 < j.win) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc += __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale, -l4[r >> 2][r & 3]));
-            } else {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int dist = e0 - col + 8 * (r >> 2) + 4 * grp + (r & 3);
-                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale, -l4[r >> 2][r & 3]));
-                    acc += dist >= 0 && dist < j.win ? p : 0.f;
-                }
-            }
-            sums[wave][grp][kg * 32 + col] = acc;
-        }
-    }
-    __syncthreads();
-    // ---- the representatives: row r's place in the order is the number of rows in front of it; the raw keys take the place
-    //      of the rotated ones meanwhile
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i)
-        if ((tid + i * 1024) / kChunks < bs) *(u32x4 *)&keys[(tid + i * 1024) * 8] = raw_in[i];
-    if (tid < kCarveMaxUnit) {
-        uint64_t key = 0;
-        if (tid < bs) {
-            float lo = 0.f, hi = 0.f;
-            if (n_sub == kCarveMaxLq / 32) {
-#pragma unroll
-                for (int st = 0; st < kCarveMaxLq / 32; ++st) lo += sums[st][0][tid], hi += sums[st][1][tid];
-            } else {
-#pragma unroll 4
-                for (int st = 0; st < n_sub; ++st) lo += sums[st][0][tid], hi += sums[st][1][tid];
-            }
-            key = pick_key(track + (lo + hi), tid);
-        }
-        rank_key[tid] = key;
-    }
-    __syncthreads();
-    {
-        const int r = tid >> 3, p = tid & 7;
-        const uint64_t own = rank_key[r];
-        int before = 0;
-#pragma unroll
-        for (int i = 0; i < kCarveMaxUnit / 8; ++i) before += rank_key[i * 8 + p] > own;
-#pragma unroll
-        for (int o = 1; o < 8; o <<= 1) before += __shfl_xor(before, o, 64);
-        if (p == 0 && r < bs && before < j.repr_topk) chosen[before] = r;
-    }
-    __syncthreads();
-    if (tid * 2 >= D) return;
-    float a0 = 0.f, a1 = 0.f;
-    for (int i = 0; i < j.repr_topk; ++i) {
-        const uint32_t w = *(const uint32_t *)&keys[chosen[i] * D + tid * 2];
-        a0 += bf16_bits_to_f32(w & 0xffffu);
-        a1 += bf16_bits_to_f32(w >> 16);
-    }
-    const float inv = 1.f / (float)j.repr_topk;
-    *(uint32_t *)(j.rep_out + (int64_t)b * j.rep_sb + (int64_t)u * j.rep_su + (int64_t)h * D + tid * 2) = pack_bf16x2(a0 * inv, a1 * inv);
-}
-
 }  // namespace
 
-// library-internal: scores and representatives of the n_units units of bs tokens from position t0 on, which leave the
-// window behind the block of `a` (whose d_lse / n_parts are set from the job's partials), their rows to their home (as
-// infllm_repr_keys_carve lays them out), and the job itself, the merge of the block's partials (job->out NULL: none).  Returns 1, with nothing
-// launched, for units or blocks the kernel does not take.
-int infllm_carve_score(const infllm_score_args *a, const MergeJob *job, const void *d_ring_k_raw, const void *d_ring_v, int64_t t0, int32_t bs, int32_t n_units,
-                       int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
-                       int64_t out_sh, void *stream, int32_t dim) {
-    INFLLM_REQUIRE(a && job && d_ring_k_raw && d_ring_v && d_rep_out && d_out_k && d_out_v, "carve_score: null pointer");
-    INFLLM_REQUIRE(dim == 128 || dim == 64, "carve_score: head_dim %d", dim);
-    if (n_units == 0) return 0;
-    if (bs % 32 != 0 || bs > kCarveMaxUnit || a->Lq > kCarveMaxLq || job->P > 8 || a->mask != INFLLM_MASK_WINDOW || a->cap != a->score_cap) return 1;
-    CarveScore j{};
+template <int D>
+static int block_end_launch(BlockEnd &j, bool scores, hipStream_t st) {
+    static_assert(sizeof(CarveLds<D>) <= 2 * 128 * kQPad<D> * sizeof(bf16_t) + 128 * sizeof(float) && sizeof(RankLds) <= sizeof(CarveLds<D>), "LDS of a workgroup");
+    const int rc = score_lds_setup<D>();
+    if (rc) return rc;
+    const infllm_score_args &a = j.s;
+    const bool wide = scores && wide_waves(a);
+    if (scores) {
+        const int wave_keys = wide ? 64 : 32;
+        const int64_t tiles = (a.j_hi - 1) / wave_keys - a.j_lo / wave_keys + 1;
+        j.n_score = (int32_t)((tiles + 3) / 4 * a.B * a.H);
+    }
+    const int64_t copies = (int64_t)2 * a.B * a.Hkv * j.n_units * j.bs * (D / 8), pieces = j.merge.out ? (int64_t)a.B * a.H * a.Lq * (D / 8) : 0;
+    INFLLM_REQUIRE(copies < (1ll << 32), "block_end: copy too large");
+    j.n_copy = (int32_t)((copies + 255) / 256);
+    const int64_t wgs = (int64_t)j.n_carve + j.n_score + j.n_copy + (pieces + 255) / 256;
+    INFLLM_REQUIRE(wgs < (1ll << 31), "block_end: grid too large");
+    if (wgs == 0) return 0;
+    const auto kern = wide ? block_end_kernel<D, 2> : block_end_kernel<D, 1>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(256), score_lds_bytes_merged<D>(128, a.Lq), st, j);
+    INFLLM_CHECK_LAUNCH("block_end");
+    return 0;
+}
+
+// library-internal: does infllm_block_end take blocks of n queries with P partials and units of bs tokens?
+bool infllm_block_end_takes(int32_t n, int32_t P, int32_t bs, bool units, bool ring_is_track) {
+    return P <= 8 && n <= kMergedMaxLq && (!units || (n <= kCarveMaxLq && bs % 32 == 0 && bs <= kCarveMaxUnit && ring_is_track));
+}
+
+// ... and does it rank units by rows of C elements?
+bool infllm_block_end_ranks(int32_t C, int32_t dim) { return C % 8 == 0 && C <= (dim == 64 ? kRankCpl<64> : kRankCpl<128>) * 512; }
+
+// library-internal: the scores of the block's queries (`a`, whose d_lse / n_parts are set from the job's partials) for keys
+// [a->j_lo, a->j_hi) unless that is empty, the merge of the job (out NULL: done before), scores and representatives of the n_units
+// units of bs tokens from position t0 on, which leave the window behind the block, and their rows to their home (as
+// infllm_repr_keys_carve lays them out); and, with rank, the scores of the units it names for n_rank blocks and the selection.
+int infllm_block_end(const infllm_score_args *a, const MergeJob *job, const void *d_ring_k_raw, const void *d_ring_v, int64_t t0, int32_t bs, int32_t n_units,
+                     int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
+                     int64_t out_sh, const RankJob *rank, int32_t n_rank, uint32_t *d_ticket, void *stream, int32_t dim) {
+    INFLLM_REQUIRE(a && job, "block_end: null pointer");
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "block_end: head_dim %d", dim);
+    INFLLM_REQUIRE(infllm_block_end_takes(a->Lq, job->P, bs, n_units > 0, a->cap == a->score_cap) && a->mask == INFLLM_MASK_WINDOW, "block_end: no kernel for this block");
+    BlockEnd j{};
     j.s = *a;
     j.s.d_lse = job->lse_part;
     j.s.n_parts = job->P;
     const int rc = check_score_args(&j.s);
     if (rc) return rc;
-    INFLLM_REQUIRE(repr_topk >= 1 && repr_topk <= bs && n_units > 0 && t0 >= 0 && (int64_t)n_units * bs <= a->cap && n_units <= 65535 && a->B <= 65535,
-                   "carve_score: bad sizes");
-    INFLLM_REQUIRE(t0 + (int64_t)n_units * bs <= a->offset + 1, "carve_score: the units reach into the block");
-    INFLLM_REQUIRE((rep_sb | rep_su) % 2 == 0 && (out_sb | out_su | out_sh) % 8 == 0, "carve_score: bad strides");
-    INFLLM_REQUIRE(job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1, "carve_score: the merge does not belong to these queries");
-    INFLLM_REQUIRE(a->cap < (1ll << 30), "carve_score: ring too large");
+    INFLLM_REQUIRE(job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1, "block_end: the merge does not belong to these queries");
     j.merge = *job;
-    j.ring_k_raw = (const bf16_t *)d_ring_k_raw;
-    j.slot0 = (int32_t)(t0 % a->cap); j.cap = (int32_t)a->cap; j.bs = bs; j.n_units = n_units; j.repr_topk = repr_topk;
-    j.to_first = (int32_t)std::min<int64_t>(a->offset - t0, 1 << 29);
-    j.win = (int32_t)std::min<int64_t>(a->window, 1 << 28);
-    j.rep_out = (bf16_t *)d_rep_out; j.rep_sb = rep_sb; j.rep_su = rep_su;
-    CarveCopy &cc = j.cc;
-    cc.ring_a = (const bf16_t *)d_ring_k_raw; cc.ring_b = (const bf16_t *)d_ring_v;
-    cc.out_a = (bf16_t *)d_out_k; cc.out_b = (bf16_t *)d_out_v;
-    cc.ring_cap = j.cap; cc.slot0 = j.slot0; cc.out_sb = out_sb; cc.out_su = out_su; cc.out_sh = out_sh;
-    cc.Hkv = a->Hkv; cc.B = a->B; cc.n = n_units * bs; cc.unit_rows = bs;
-    const int64_t per_x = (int64_t)n_units * a->B, elems = (int64_t)2 * a->B * a->Hkv * cc.n * (dim / 8), pieces = (int64_t)a->B * a->H * a->Lq * (dim / 8);
-    INFLLM_REQUIRE(elems < (1ll << 32), "carve_score: copy too large");
-    cc.x_extra = (int32_t)(((elems + 1023) / 1024 + per_x - 1) / per_x);
-    const int32_t x_merge = job->out ? (int32_t)(((pieces + 1023) / 1024 + per_x - 1) / per_x) : 0;
-    const dim3 grid(a->H + cc.x_extra + x_merge, n_units, a->B);
-    if (dim == 128) hipLaunchKernelGGL(carve_score_kernel<128>, grid, dim3(1024), 0, (hipStream_t)stream, j);
-    else hipLaunchKernelGGL(carve_score_kernel<64>, grid, dim3(1024), 0, (hipStream_t)stream, j);
-    INFLLM_CHECK_LAUNCH("carve_score");
-    return 0;
+    if (n_units > 0) {
+        INFLLM_REQUIRE(d_ring_k_raw && d_ring_v && d_rep_out && d_out_k && d_out_v, "block_end: null pointer");
+        INFLLM_REQUIRE(repr_topk >= 1 && repr_topk <= bs && t0 >= 0 && (int64_t)n_units * bs <= a->cap, "block_end: bad sizes");
+        INFLLM_REQUIRE(t0 + (int64_t)n_units * bs <= a->offset + 1, "block_end: the units reach into the block");
+        INFLLM_REQUIRE((rep_sb | rep_su) % 2 == 0 && (out_sb | out_su | out_sh) % 8 == 0, "block_end: bad strides");
+        INFLLM_REQUIRE(a->cap < (1ll << 30) && (int64_t)a->H * n_units * a->B < (1ll << 30), "block_end: ring or batch too large");
+        j.n_carve = a->H * n_units * a->B;
+        j.ring_k_raw = (const bf16_t *)d_ring_k_raw;
+        j.slot0 = (int32_t)(t0 % a->cap); j.cap = (int32_t)a->cap; j.bs = bs; j.n_units = n_units; j.repr_topk = repr_topk;
+        j.to_first = (int32_t)std::min<int64_t>(a->offset - t0, 1 << 29);
+        j.win = (int32_t)std::min<int64_t>(a->window, 1 << 28);
+        j.rep_out = (bf16_t *)d_rep_out; j.rep_sb = rep_sb; j.rep_su = rep_su;
+        CarveCopy &cc = j.cc;
+        cc.ring_a = (const bf16_t *)d_ring_k_raw; cc.ring_b = (const bf16_t *)d_ring_v;
+        cc.out_a = (bf16_t *)d_out_k; cc.out_b = (bf16_t *)d_out_v;
+        cc.ring_cap = j.cap; cc.slot0 = j.slot0; cc.out_sb = out_sb; cc.out_su = out_su; cc.out_sh = out_sh;
+        cc.Hkv = a->Hkv; cc.B = a->B; cc.n = n_units * bs; cc.unit_rows = bs;
+    }
+    if (rank) {
+        INFLLM_REQUIRE(infllm_block_end_ranks(rank->C, dim) && n_rank >= 1 && rank->n_new <= kRankNew && d_ticket, "block_end: no ranking for rows of %d elements", rank->C);
+        INFLLM_REQUIRE(rank->n_list + rank->first_new + rank->n_new - rank->n_base <= kRankEntries, "block_end: too many units to rank");
+        j.rank = *rank;
+        j.n_rank = n_rank;
+        j.ticket = d_ticket;
+        j.n_carve = std::max(j.n_carve, 1);                       // (nothing carved: a workgroup that only ranks)
+    }
+    const bool scores = a->j_hi > a->j_lo;
+    return dim == 128 ? block_end_launch<128>(j, scores, (hipStream_t)stream) : block_end_launch<64>(j, scores, (hipStream_t)stream);
 }
 
 extern "C" int infllm_local_score(const infllm_score_args *a, void *stream) { return score_launch<kD>(a, stream); }
@@ -637,9 +703,4 @@ int infllm_local_score_dim(const infllm_score_args *a, int32_t dim, void *stream
 int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream, int32_t dim) {
     INFLLM_REQUIRE(dim == 128 || dim == 64, "local_score: head_dim %d", dim);
     return dim == 128 ? score_launch_merged<128>(a, job, stream) : score_launch_merged<64>(a, job, stream);
-}
-// ... and with the next block's ranking in n_rank workgroups
-int infllm_local_score_merged_rank(const infllm_score_args *a, const MergeJob *job, const RankJob *rank, int32_t n_rank, void *stream, int32_t dim) {
-    INFLLM_REQUIRE(rank && (dim == 128 || dim == 64), "local_score: bad ranking");
-    return dim == 128 ? score_launch_merged<128>(a, job, stream, rank, n_rank) : score_launch_merged<64>(a, job, stream, rank, n_rank);
 }
