@@ -53,8 +53,8 @@ __device__ __forceinline__ void write_page(const PageList &j, int u, int p, cons
     j.out[(int64_t)u * j.n_pages + p] = pg;
 }
 
-// After a block has carved n_new units: they are scored under the mean queries of the call's blocks from j0 on; block j_sel's
-// list of the call's start is ranked against all units carved since, and the selection becomes the block's page table.
+// After a block has carved units: every unit is scored under the mean queries of the call's later blocks, and block j_sel's list
+// of the call's start is ranked against all units carved since; the selection becomes the block's page table.
 struct RankJob {
     const bf16_t *reps;
     int64_t rep_sb, rep_su;
@@ -62,97 +62,104 @@ struct RankJob {
     float *scores;                         // [blocks][B][cols]
     int64_t cols;
     const int32_t *base;                   // [blocks][B][k], n_list entries of a row are filled
-    int32_t B, C, k, n_list, n_base, first_new, n_new, j0, j_sel;
+    int32_t B, C, k, n_list, n_base, j0, j_sel;
+    int32_t first_new, n_new;              // the units that have no scores under block j0 and later ones yet, from first_new on,
+    int32_t n_before;                      // and how many of them were there before this launch
     int32_t *log;                          // pinned: [B][k] ids, then the sequence number
     int32_t seq;
     PageList pages;
 };
 
 struct RankLds {
-    float fresh[kRankNew];
-    uint32_t e_key[kRankEntries];
-    int32_t e_id[kRankEntries], sel[64];
+    float fresh[2 * kRankNew];
+    uint64_t e_key[kRankEntries];
+    int32_t sel[64];
 };
 
-// 256 threads: scores of the new units under the mean queries of blocks j0 + x0 .. j0 + x0 + nx - 1, and the ranking if the block
-// j_sel is one of them (the sums are unit_scores_rows_kernel's, term by term: a unit's score does not depend on which kernel
-// computed it).  A wave keeps a unit's row and takes the mean queries in turn, each piece of the next one requested as soon as
-// its place is free.
+// 256 threads: scores of n_new units from jb.first_new on under the mean query of block j0 + x, and the ranking if that is block
+// j_sel (the sums are unit_scores_rows_kernel's, term by term: a unit's score does not depend on which kernel computed it).  All
+// of it is a chain of trips to memory: what can be requested ahead of another answer is.
 template <int CPL>
-__device__ __forceinline__ void rank_blocks(const RankJob &jb, int x0, int nx, RankLds &lds) {
+__device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, RankLds &lds) {
     float *fresh = lds.fresh;
-    uint32_t *e_key = lds.e_key;
-    int32_t *e_id = lds.e_id, *sel = lds.sel;
+    uint64_t *e_key = lds.e_key;
+    int32_t *sel = lds.sel;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, C = jb.C;
-    const bool is_sel = jb.j_sel >= jb.j0 + x0 && jb.j_sel < jb.j0 + x0 + nx;
-    const int n = jb.n_list + jb.first_new + jb.n_new - jb.n_base;
+    const int j = jb.j0 + x;
+    const bool is_sel = j == jb.j_sel;
+    const int n = jb.n_list + jb.first_new + n_new - jb.n_base;
     for (int u = 0; u < jb.B; ++u) {
+        const float *qbar = jb.qbars + ((int64_t)j * jb.B + u) * C + lane * 8;
+        float *scores = jb.scores + ((int64_t)j * jb.B + u) * jb.cols;
         // the ranking threads' entries, asked for ahead of the scoring
         int my_id[2] = {-1, -1};
         float my_score[2] = {0.f, 0.f};
         if (is_sel) {
-            const int64_t row = (int64_t)jb.j_sel * jb.B + u;
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int e = tid + 256 * i;
                 if (e >= n) continue;
-                my_id[i] = e < jb.n_list ? jb.base[row * jb.k + e] : jb.n_base + (e - jb.n_list);
-                if (my_id[i] < jb.first_new) my_score[i] = jb.scores[row * jb.cols + my_id[i]];
+                my_id[i] = e < jb.n_list ? jb.base[((int64_t)j * jb.B + u) * jb.k + e] : jb.n_base + (e - jb.n_list);
+                if (my_id[i] < jb.first_new) my_score[i] = scores[my_id[i]];
             }
         }
-        for (int r = wave; r < jb.n_new; r += 4) {
-            const bf16_t *row = jb.reps + (int64_t)u * jb.rep_sb + (int64_t)(jb.first_new + r) * jb.rep_su + lane * 8;
-            u32x4 w[CPL];
+        if (wave < n_new) {
             f32x4 q[CPL][2];
+            u32x4 w[CPL], ahead[CPL];
+            auto request = [&](int r) {
+                const bf16_t *row = jb.reps + (int64_t)u * jb.rep_sb + (int64_t)(jb.first_new + r) * jb.rep_su + lane * 8;
 #pragma unroll
-            for (int c = 0; c < CPL; ++c) w[c] = c * 512 + lane * 8 < C ? *(const u32x4 *)(row + c * 512) : u32x4{0, 0, 0, 0};
-            auto request = [&](int x, int c) {
-                const float *qbar = jb.qbars + ((int64_t)(jb.j0 + x) * jb.B + u) * C + lane * 8 + c * 512;
-                const bool in = c * 512 + lane * 8 < C;
-#pragma unroll
-                for (int i = 0; i < 2; ++i) q[c][i] = in ? *(const f32x4 *)(qbar + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int c = 0; c < CPL; ++c) ahead[c] = c * 512 + lane * 8 < C ? *(const u32x4 *)(row + c * 512) : u32x4{0, 0, 0, 0};
             };
+            request(wave);
 #pragma unroll
-            for (int c = 0; c < CPL; ++c) request(x0, c);
-            for (int x = x0; x < x0 + nx; ++x) {
+            for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) q[c][i] = c * 512 + lane * 8 < C ? *(const f32x4 *)(qbar + c * 512 + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int r = wave; r < n_new; r += 4) {
+#pragma unroll
+                for (int c = 0; c < CPL; ++c) w[c] = ahead[c];
+                if (r + 4 < n_new) request(r + 4);
                 float acc0 = 0.f, acc1 = 0.f;
 #pragma unroll
-                for (int c = 0; c < CPL; ++c) {
-                    asm volatile("" : "+v"(w[c]));               // (kept as it is: unpacked once for all x it would be twice the registers)
+                for (int c = 0; c < CPL; ++c)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         acc0 += bf16_bits_to_f32(w[c][i] & 0xffffu) * q[c][i >> 1][2 * (i & 1)];
                         acc1 += bf16_bits_to_f32(w[c][i] >> 16) * q[c][i >> 1][2 * (i & 1) + 1];
                     }
-                    if (x + 1 < x0 + nx) request(x + 1, c);
-                }
                 float acc = acc0 + acc1;
 #pragma unroll
                 for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
                 if (lane == 0) {
-                    jb.scores[((int64_t)(jb.j0 + x) * jb.B + u) * jb.cols + jb.first_new + r] = acc;
-                    if (jb.j0 + x == jb.j_sel) fresh[r] = acc;
+                    scores[jb.first_new + r] = acc;
+                    fresh[r] = acc;
                 }
             }
         }
         if (!is_sel) continue;                                   // workgroup-uniform
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < 2; ++i) {                            // descending score, equal scores in ascending id: all distinct
             const int e = tid + 256 * i;
             if (e >= n) continue;
-            e_id[e] = my_id[i];
-            e_key[e] = order_key(my_id[i] >= jb.first_new ? fresh[my_id[i] - jb.first_new] : my_score[i]);
+            const float score = my_id[i] >= jb.first_new ? fresh[my_id[i] - jb.first_new] : my_score[i];
+            e_key[e] = ((uint64_t)order_key(score) << 32) | (uint32_t)~my_id[i];
         }
         __syncthreads();
-        for (int e = tid; e < n; e += 256) {
-            const uint32_t key = e_key[e];
-            const int id = e_id[e];
+        for (int e0 = 0; e0 < n; e0 += 64) {                     // an entry's place is the number of entries in front of it: four lanes count
+            const int e = e0 + (tid >> 2), p = tid & 3;
+            const uint64_t own = e_key[min(e, n - 1)];
             int rank = 0;
-            for (int o = 0; o < n; ++o) rank += (e_key[o] > key || (e_key[o] == key && e_id[o] < id)) ? 1 : 0;
-            if (rank < jb.k) {
+#pragma unroll 4
+            for (int o = p; o < n; o += 4) rank += e_key[o] > own ? 1 : 0;
+            rank += __shfl_xor(rank, 1, 64);
+            rank += __shfl_xor(rank, 2, 64);
+            if (p == 0 && e < n && rank < jb.k) {
+                const int id = (int)~(uint32_t)own;
                 sel[rank] = id;
-                jb.log[(int64_t)u * jb.k + rank] = id;
+                // (written through to the host's memory: a fence would write the whole L2 back)
+                __hip_atomic_store(jb.log + (int64_t)u * jb.k + rank, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             }
         }
         __syncthreads();
@@ -160,8 +167,8 @@ __device__ __forceinline__ void rank_blocks(const RankJob &jb, int x0, int nx, R
         __syncthreads();                                         // the lists are rewritten for the next row
     }
     if (is_sel) {
-        __threadfence_system();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // every wave's ids have arrived
         __syncthreads();
-        if (tid == 0) __hip_atomic_store(jb.log + (int64_t)jb.B * jb.k, jb.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (tid == 0) __hip_atomic_store(jb.log + (int64_t)jb.B * jb.k, jb.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }

@@ -56,7 +56,7 @@ namespace {
 template <int CPL>
 __global__ __launch_bounds__(256) void rank_kernel(RankJob jb) {
     __shared__ RankLds lds;
-    rank_blocks<CPL>(jb, blockIdx.x, 1, lds);
+    rank_block<CPL>(jb, blockIdx.x, jb.n_new, lds);
 }
 
 // the page table of a selection that is already in memory
@@ -311,7 +311,7 @@ PageList page_list(const Resident *R, const infllm_resident_call *a, int n_sel, 
 
 int launch_rank(Resident *R, const RankJob &jb, int n_wgs, hipStream_t st) {
     const int cpl = (jb.C + 511) / 512;
-    INFLLM_REQUIRE(jb.C % 8 == 0 && cpl <= 16 && jb.n_new <= kRankNew && jb.n_list + jb.first_new + jb.n_new - jb.n_base <= kRankEntries,
+    INFLLM_REQUIRE(jb.C % 8 == 0 && cpl <= 16 && jb.n_new <= 2 * kRankNew && jb.n_list + jb.first_new + jb.n_new - jb.n_base <= kRankEntries,
                    "resident: no ranking for rows of %d elements, %d new units", jb.C, jb.n_new);
 #define RANK(n) hipLaunchKernelGGL(rank_kernel<n>, dim3(n_wgs), dim3(256), 0, st, jb)
     if (cpl <= 1) RANK(1);
@@ -571,6 +571,7 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
     };
     int32_t j_done = -1;                          // the block whose page table is on the device
     int plain_end = 0;                            // blocks in front of this one are done
+    int32_t scored = n0;                          // units that have scores under the mean queries of all blocks to come
     for (int i = 0; i < n_blocks; ++i) {
         const int nb = std::min(exc, n - i * exc);
         const int64_t b0 = call_b0 + (int64_t)i * exc, b1 = b0 + nb, lo = std::max<int64_t>(0, b0 - d.n_local);
@@ -639,7 +640,7 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             RankJob jb{};
             jb.reps = (const bf16_t *)a->d_reps; jb.rep_sb = a->rep_sb; jb.rep_su = a->rep_su;
             jb.qbars = a->d_qbar; jb.scores = a->d_call_scores; jb.cols = a->scores_cols; jb.base = a->d_base;
-            jb.B = B; jb.C = C; jb.k = d.topk; jb.n_list = n_list; jb.n_base = n0; jb.first_new = N; jb.n_new = 0; jb.j0 = jb.j_sel = i;
+            jb.B = B; jb.C = C; jb.k = d.topk; jb.n_list = n_list; jb.n_base = n0; jb.first_new = scored; jb.n_new = N - scored; jb.j0 = jb.j_sel = i;
             jb.log = d.d_log + (int64_t)slot * (B * d.topk + 1); jb.seq = seq;
             jb.pages = pl;
             rc = launch_rank(R, jb, 1, st);
@@ -720,7 +721,7 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             const bool select = N1 > d.topk;
             jb.reps = (const bf16_t *)a->d_reps; jb.rep_sb = a->rep_sb; jb.rep_su = a->rep_su;
             jb.qbars = a->d_qbar; jb.scores = a->d_call_scores; jb.cols = a->scores_cols; jb.base = a->d_base;
-            jb.B = B; jb.C = C; jb.k = d.topk; jb.n_list = n_list; jb.n_base = n0; jb.first_new = N; jb.n_new = N1 - N;
+            jb.B = B; jb.C = C; jb.k = d.topk; jb.n_list = n_list; jb.n_base = n0; jb.first_new = scored; jb.n_new = N1 - scored; jb.n_before = N - scored;
             jb.j0 = i + 1; jb.j_sel = select ? i + 1 : -1;
             if (select) {
                 int32_t slot = 0, seq = 0;
@@ -740,11 +741,12 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             const bool carry = rank && infllm_block_end_ranks(C, D);
             rc = end_block(sc, carry ? &jb : nullptr, n_rank);
             if (rc) return rc;
-            ranked = ranked || carry;
+            if (carry) ranked = true, scored = N;
         }
         if (!ranked) {
             rc = launch_rank(R, jb, n_rank, st);
             if (rc) return rc;
+            scored = N1;
         }
     }
     return 0;

@@ -54,11 +54,13 @@ __device__ __forceinline__ void score_tile(const infllm_score_args &a, const Par
     // Workgroups are dispatched x fastest: all heads of one key tile, then the next tile.  The two tiles at either end
     // of a masked key range see only part of the queries and finish early, so they go last: when the grid is a little
     // more than what the chip holds at once, the workgroups that start late are then the short ones.
-    // Where the queries are (nearly) as many as the keys, a tile's work falls from the first to the last instead: a CU that
+    // (None at the low end when the first query sees it.)  Where the queries are (nearly) as many as the keys, a tile's work falls from the first to the last instead: a CU that
     // takes one of the first half and one of the second gets a long and a short one.
     int tile = slot;
     if (a.mask == INFLLM_MASK_WINDOW && a.Lq >= (a.j_hi - a.j_lo) - (a.j_hi - a.j_lo) / 4)
         tile = slot < (n_tiles + 1) / 2 ? slot : n_tiles - 1 - (slot - (n_tiles + 1) / 2);
+    else if (a.mask == INFLLM_MASK_WINDOW && a.j_lo >= a.offset + a.Lq - a.window)
+        tile = slot;
     else if (n_tiles >= 6 && a.mask != INFLLM_MASK_NONE)
         tile = slot < n_tiles - 4 ? slot + 2 : slot == n_tiles - 4 ? 1 : slot == n_tiles - 3 ? n_tiles - 2 : slot == n_tiles - 2 ? 0 : n_tiles - 1;
     const int64_t jg = (a.j_lo / kWaveKeys + (int64_t)tile * 4) * kWaveKeys;         // first key of the workgroup
@@ -297,7 +299,10 @@ __global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a
 // scores of the keys that stay, the merge, the units' rows - depends on none of it and fills the chip meanwhile.  So the
 // carving workgroups (one per unit and head: 128 keys x 512 queries, half of them outside the window) come first in the grid;
 // the one that is done last ranks.  As two launches, carving with the merge and the rest of the scores with the ranking, which
-// can begin when the first has ended: 5 us a block of 512 queries x 4,096 keys x 32 heads more (17.2 + 28).
+// can begin when the first has ended: 5 us a block of 512 queries x 4,096 keys x 32 heads more (17.2 + 28).  What the last one does
+// is what the launch waits for, beside a chip full of other loads: it scores under one mean query (four took 18.6 us, the scores'
+// last workgroup ends 3 to 10 us earlier), sees to nothing but its own stores, and counts with four lanes an entry: prompts of
+// 131,072 tokens 27,610 -> 26,830 us, of 24,300 with 36 heads of 64 3,350 -> 3,200.
 //
 // A carving workgroup's steps are as short as they can be: everything it reads is requested at once; the unit's keys are in
 // LDS (every wave needs them all), four sub-tiles of 32 queries a wave take turns with each of them; a sub-tile's column sums
@@ -306,7 +311,7 @@ constexpr int kCarveMaxLq = 512, kCarveMaxUnit = 128;
 struct BlockEnd {
     infllm_score_args s;               // the keys that stay
     MergeJob merge;                    // the block's partials (out NULL: merged before)
-    int32_t n_carve, n_score, n_copy, n_rank;      // workgroups of each kind, in this order, those that merge behind them; blocks to rank for (0: none)
+    int32_t n_carve, n_score, n_copy, n_early;     // workgroups of each kind, in this order, those that merge behind them
     // units that leave
     const bf16_t *ring_k_raw;
     int32_t slot0, cap, to_first;      // ring row of the first unit; dist of query 0 to the first unit's first key
@@ -315,6 +320,7 @@ struct BlockEnd {
     int64_t rep_sb, rep_su;
     CarveCopy cc;
     RankJob rank;
+    int32_t ranks;                     // does the launch rank?
     uint32_t *ticket;                  // zero; the last of the carving workgroups to finish puts it back
 };
 
@@ -482,7 +488,7 @@ __global__ __launch_bounds__(256, (D == 64 && KS == 1 ? 3 : 2)) void block_end_k
         if (j.n_units > 0) {
             const int rest = x / j.s.H;
             carve_unit<D>(j, x - rest * j.s.H, rest % j.n_units, rest / j.n_units, *(CarveLds<D> *)score_lds);
-            if (j.n_rank == 0) return;
+            if (!j.ranks) return;
             // The representatives are the only thing that crosses workgroups, and their stores have been performed where every
             // XCD sees them before the ticket is drawn: no workgroup has to write its L2 back.
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -493,7 +499,7 @@ __global__ __launch_bounds__(256, (D == 64 && KS == 1 ? 3 : 2)) void block_end_k
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             if (threadIdx.x == 0) __hip_atomic_store(j.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        rank_blocks<kRankCpl<D>>(j.rank, 0, j.n_rank, *(RankLds *)score_lds);
+        rank_block<kRankCpl<D>>(j.rank, 0, j.rank.n_new, *(RankLds *)score_lds);
         return;
     }
     x -= j.n_carve;
@@ -503,6 +509,11 @@ __global__ __launch_bounds__(256, (D == 64 && KS == 1 ? 3 : 2)) void block_end_k
         return;
     }
     x -= j.n_score;
+    if (x < j.n_early) {                                          // the units carved before, for the blocks behind the next
+        rank_block<kRankCpl<D>>(j.rank, x + 1, j.rank.n_before, *(RankLds *)score_lds);
+        return;
+    }
+    x -= j.n_early;
     if (x < j.n_copy) carve_copy<D>(j.cc, (int64_t)x * 256 + threadIdx.x);
     else merge_piece<D>(j.merge, (int64_t)(x - j.n_copy) * 256 + threadIdx.x);
 }
@@ -624,7 +635,7 @@ static int block_end_launch(BlockEnd &j, bool scores, hipStream_t st) {
     const int64_t copies = (int64_t)2 * a.B * a.Hkv * j.n_units * j.bs * (D / 8), pieces = j.merge.out ? (int64_t)a.B * a.H * a.Lq * (D / 8) : 0;
     INFLLM_REQUIRE(copies < (1ll << 32), "block_end: copy too large");
     j.n_copy = (int32_t)((copies + 255) / 256);
-    const int64_t wgs = (int64_t)j.n_carve + j.n_score + j.n_copy + (pieces + 255) / 256;
+    const int64_t wgs = (int64_t)j.n_carve + j.n_score + j.n_early + j.n_copy + (pieces + 255) / 256;
     INFLLM_REQUIRE(wgs < (1ll << 31), "block_end: grid too large");
     if (wgs == 0) return 0;
     const auto kern = wide ? block_end_kernel<D, 2> : block_end_kernel<D, 1>;
@@ -644,7 +655,9 @@ bool infllm_block_end_ranks(int32_t C, int32_t dim) { return C % 8 == 0 && C <= 
 // library-internal: the scores of the block's queries (`a`, whose d_lse / n_parts are set from the job's partials) for keys
 // [a->j_lo, a->j_hi) unless that is empty, the merge of the job (out NULL: done before), scores and representatives of the n_units
 // units of bs tokens from position t0 on, which leave the window behind the block, and their rows to their home (as
-// infllm_repr_keys_carve lays them out); and, with rank, the scores of the units it names for n_rank blocks and the selection.
+// infllm_repr_keys_carve lays them out); and, with rank, the selection of block rank->j0 and its scores of the rank->n_new units,
+// and the scores of the first n_before of them under the n_rank - 1 blocks behind it.  (The units carved now get those with the next
+// block: the workgroup that finishes last, which the launch waits for, scores for one block only.)
 int infllm_block_end(const infllm_score_args *a, const MergeJob *job, const void *d_ring_k_raw, const void *d_ring_v, int64_t t0, int32_t bs, int32_t n_units,
                      int32_t repr_topk, void *d_rep_out, int64_t rep_sb, int64_t rep_su, void *d_out_k, void *d_out_v, int64_t out_sb, int64_t out_su,
                      int64_t out_sh, const RankJob *rank, int32_t n_rank, uint32_t *d_ticket, void *stream, int32_t dim) {
@@ -678,10 +691,11 @@ int infllm_block_end(const infllm_score_args *a, const MergeJob *job, const void
         cc.Hkv = a->Hkv; cc.B = a->B; cc.n = n_units * bs; cc.unit_rows = bs;
     }
     if (rank) {
-        INFLLM_REQUIRE(infllm_block_end_ranks(rank->C, dim) && n_rank >= 1 && rank->n_new <= kRankNew && d_ticket, "block_end: no ranking for rows of %d elements", rank->C);
+        INFLLM_REQUIRE(infllm_block_end_ranks(rank->C, dim) && n_rank >= 1 && rank->n_new <= 2 * kRankNew && rank->n_before <= rank->n_new && d_ticket, "block_end: no ranking for rows of %d elements", rank->C);
         INFLLM_REQUIRE(rank->n_list + rank->first_new + rank->n_new - rank->n_base <= kRankEntries, "block_end: too many units to rank");
         j.rank = *rank;
-        j.n_rank = n_rank;
+        j.ranks = 1;
+        j.n_early = rank->n_before > 0 ? n_rank - 1 : 0;
         j.ticket = d_ticket;
         j.n_carve = std::max(j.n_carve, 1);                       // (nothing carved: a workgroup that only ranks)
     }
