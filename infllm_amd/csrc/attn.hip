@@ -100,29 +100,10 @@ struct StageGeom {
 //                          supplies the address of 4 consecutive d of key j, and lane i receives element
 //                          i of keys j = 0..3, i.e. 4 consecutive keys at one d.
 __device__ __forceinline__ int k_lds_row(int key) { return (key & ~12) | ((key & 4) << 1) | ((key & 8) >> 1); }
-// Heads of 64: a row is 128 bytes (8 chunks), two rows share a 256-byte line.  16 consecutive rows, one chunk each, hit 16
-// different places when the row pairs use 8 different positions; the four row pairs' bit that decides the upper or lower
-// four chunks is the pair's lowest, so that the transposing read's 4 rows x 4 chunks x 2 halves are 32 different slots.
-template <int D>
-__device__ __forceinline__ int swz(int row) {
-    return D == 128 ? ((row & 3) << 2) | ((row >> 2) & 3) : (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
-}
-
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ s16x4 lds_read_tr(uint32_t at) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(uintptr_t)at);
 }
-// Issued as inline assembly on purpose.  With the builtin, the compiler tracks the transfer as an LDS store that
-// may alias every later LDS read and puts `s_waitcnt vmcnt(0)` in front of the first operand read of the tile being
-// multiplied - which waits for the tiles just requested for LATER and serialises load and math completely.  The
-// kernel orders the transfers itself: vmcnt(0) and a barrier before a buffer is read, a barrier before it is refilled.
-// The row address is a scalar base and a 32-bit byte offset of the lane.  M0 is overwritten: nothing else in these kernels
-// uses it (LDS instructions have not since gfx9).
-__device__ __forceinline__ void load_to_lds16(const bf16_t *base, uint32_t lane_off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(lane_off), "s"(base) : "memory");
-}
-__device__ __forceinline__ uint32_t lds_address(const char *p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p; }
-
 template <int D>
 constexpr int kTileBytes = kTile * D * 2;         // one K (or V) tile in LDS
 constexpr float kLazyLog2 = 8.f;                  // the running max may lag the true max by 2^8

@@ -70,7 +70,9 @@ struct RankJob {
     PageList pages;
 };
 
+template <int CPL>
 struct RankLds {
+    float q[CPL * 512];                    // the mean query
     float fresh[2 * kRankNew];
     uint64_t e_key[kRankEntries];
     int32_t sel[64];
@@ -80,7 +82,7 @@ struct RankLds {
 // j_sel (the sums are unit_scores_rows_kernel's, term by term: a unit's score does not depend on which kernel computed it).  All
 // of it is a chain of trips to memory: what can be requested ahead of another answer is.
 template <int CPL>
-__device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, RankLds &lds) {
+__device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, RankLds<CPL> &lds) {
     float *fresh = lds.fresh;
     uint64_t *e_key = lds.e_key;
     int32_t *sel = lds.sel;
@@ -89,7 +91,7 @@ __device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, 
     const bool is_sel = j == jb.j_sel;
     const int n = jb.n_list + jb.first_new + n_new - jb.n_base;
     for (int u = 0; u < jb.B; ++u) {
-        const float *qbar = jb.qbars + ((int64_t)j * jb.B + u) * C + lane * 8;
+        const float *qbar = jb.qbars + ((int64_t)j * jb.B + u) * C;
         float *scores = jb.scores + ((int64_t)j * jb.B + u) * jb.cols;
         // the ranking threads' entries, asked for ahead of the scoring
         int my_id[2] = {-1, -1};
@@ -103,42 +105,38 @@ __device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, 
                 if (my_id[i] < jb.first_new) my_score[i] = scores[my_id[i]];
             }
         }
-        if (wave < n_new) {
-            f32x4 q[CPL][2];
-            u32x4 w[CPL], ahead[CPL];
-            auto request = [&](int r) {
-                const bf16_t *row = jb.reps + (int64_t)u * jb.rep_sb + (int64_t)(jb.first_new + r) * jb.rep_su + lane * 8;
+        u32x4 w[CPL];
+        auto request = [&](int r) {
+            const bf16_t *row = jb.reps + (int64_t)u * jb.rep_sb + (int64_t)(jb.first_new + r) * jb.rep_su + lane * 8;
 #pragma unroll
-                for (int c = 0; c < CPL; ++c) ahead[c] = c * 512 + lane * 8 < C ? *(const u32x4 *)(row + c * 512) : u32x4{0, 0, 0, 0};
-            };
-            request(wave);
+            for (int c = 0; c < CPL; ++c) w[c] = c * 512 + lane * 8 < C ? *(const u32x4 *)(row + c * 512) : u32x4{0, 0, 0, 0};
+        };
+        if (wave < n_new) request(wave);
+        for (int e = tid * 4; e < C; e += 1024) *(f32x4 *)(lds.q + e) = *(const f32x4 *)(qbar + e);
+        __syncthreads();
+        for (int r = wave; r < n_new; r += 4) {
+            float acc0 = 0.f, acc1 = 0.f;
 #pragma unroll
-            for (int c = 0; c < CPL; ++c)
+            for (int c = 0; c < CPL; ++c) {
+                if (c * 512 + lane * 8 >= C) continue;
+                const f32x4 q[2] = {*(const f32x4 *)(lds.q + c * 512 + lane * 8), *(const f32x4 *)(lds.q + c * 512 + lane * 8 + 4)};
 #pragma unroll
-                for (int i = 0; i < 2; ++i) q[c][i] = c * 512 + lane * 8 < C ? *(const f32x4 *)(qbar + c * 512 + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
-            for (int r = wave; r < n_new; r += 4) {
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) w[c] = ahead[c];
-                if (r + 4 < n_new) request(r + 4);
-                float acc0 = 0.f, acc1 = 0.f;
-#pragma unroll
-                for (int c = 0; c < CPL; ++c)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        acc0 += bf16_bits_to_f32(w[c][i] & 0xffffu) * q[c][i >> 1][2 * (i & 1)];
-                        acc1 += bf16_bits_to_f32(w[c][i] >> 16) * q[c][i >> 1][2 * (i & 1) + 1];
-                    }
-                float acc = acc0 + acc1;
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-                if (lane == 0) {
-                    scores[jb.first_new + r] = acc;
-                    fresh[r] = acc;
+                for (int i = 0; i < 4; ++i) {
+                    acc0 += bf16_bits_to_f32(w[c][i] & 0xffffu) * q[i >> 1][2 * (i & 1)];
+                    acc1 += bf16_bits_to_f32(w[c][i] >> 16) * q[i >> 1][2 * (i & 1) + 1];
                 }
             }
+            if (r + 4 < n_new) request(r + 4);
+            float acc = acc0 + acc1;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+            if (lane == 0) {
+                scores[jb.first_new + r] = acc;
+                fresh[r] = acc;
+            }
         }
-        if (!is_sel) continue;                                   // workgroup-uniform
         __syncthreads();
+        if (!is_sel) continue;                                   // workgroup-uniform
 #pragma unroll
         for (int i = 0; i < 2; ++i) {                            // descending score, equal scores in ascending id: all distinct
             const int e = tid + 256 * i;

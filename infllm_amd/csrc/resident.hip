@@ -55,7 +55,7 @@ namespace {
 
 template <int CPL>
 __global__ __launch_bounds__(256) void rank_kernel(RankJob jb) {
-    __shared__ RankLds lds;
+    __shared__ __attribute__((aligned(16))) RankLds<CPL> lds;
     rank_block<CPL>(jb, blockIdx.x, jb.n_new, lds);
 }
 

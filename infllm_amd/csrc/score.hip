@@ -312,10 +312,11 @@ struct BlockEnd {
     infllm_score_args s;               // the keys that stay
     MergeJob merge;                    // the block's partials (out NULL: merged before)
     int32_t n_carve, n_score, n_copy, n_early;     // workgroups of each kind, in this order, those that merge behind them
+    int32_t cap, slot0;                // rows of the ring; that of the first key of the first scoring workgroup
     // units that leave
     const bf16_t *ring_k_raw;
-    int32_t slot0, cap, to_first;      // ring row of the first unit; dist of query 0 to the first unit's first key
-    int32_t win, bs, n_units, repr_topk;
+    int64_t t0;                        // their first key, and its row
+    int32_t unit_slot0, bs, n_units, repr_topk;
     bf16_t *rep_out;
     int64_t rep_sb, rep_su;
     CarveCopy cc;
@@ -324,146 +325,207 @@ struct BlockEnd {
     uint32_t *ticket;                  // zero; the last of the carving workgroups to finish puts it back
 };
 
+// Column sums of the block's probabilities for 128 * KS consecutive keys of a query head, 32 * KS a wave and KS a lane (both
+// halves of the wave get them).  The keys are those from position jg on, in row `slot` of the ring, of which [lo, hi) count.
+//
+// A wave's exponentials and MFMAs overlap (half a sub-tile of 32 queries apart), so the loop runs at the rate of the vector unit
+// (768 cycles of a sub-tile of 32 queries x 64 keys); what is left is a launch of one or two rounds of workgroups whose first 7
+// of 20 us are the wait for their keys.  So registers and LDS are kept to a third of a CU: all carving and scoring workgroups of
+// 512 queries x 4,096 keys x 32 heads are in flight at once, one's wait beside another's loop.  The queries go from memory
+// straight into LDS (64 rows a stage, three stages in turn, no registers on the way), and a wave's two accumulators are the halves
+// of a sub-tile instead of two sub-tiles.  With half a CU each (score_tile, and carving workgroups with a loop of their own):
+// prompts of 131,072 / 16,001 tokens 27,000 -> 26,000 / 2,816 -> 2,726 us, of 24,300 with 36 heads of 64 3,185 -> 3,136.
+constexpr int kQRows = 64;                             // queries of a stage
 template <int D>
-struct CarveLds {
-    bf16_t keys[kCarveMaxUnit * D];                // chunk c of row r at c ^ (r mod kChunks)
-    float lse[kCarveMaxLq];
-    float sums[kCarveMaxLq / 32][2][kCarveMaxUnit];
-    uint64_t rank_key[kCarveMaxUnit];
-    int32_t chosen[kCarveMaxUnit];
-};
+constexpr size_t kQBytes = (size_t)3 * kQRows * D * sizeof(bf16_t);
 
-template <int D>
-__device__ __forceinline__ void carve_unit(const BlockEnd &j, int h, int u, int b, CarveLds<D> &lds) {
-    constexpr int kChunks = D / 8, kSubs = kCarveMaxLq / 32 / 4;                   // sub-tiles a wave
-    const infllm_score_args &a = j.s;
+template <int D, int KS>
+__device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartSets lps, int b, int h, int64_t jg, int slot, int cap, int lo, int hi, char *lds,
+                                         float (&sums)[KS]) {
+    constexpr int kWaveKeys = 32 * KS, kRow = D * 2, kStage = kQRows * kRow;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 31, grp = lane >> 5;
-    const int g = h / (a.H / a.Hkv), bs = j.bs;
+    b = __builtin_amdgcn_readfirstlane(b), h = __builtin_amdgcn_readfirstlane(h), slot = __builtin_amdgcn_readfirstlane(slot);
+    lo = __builtin_amdgcn_readfirstlane(lo), hi = __builtin_amdgcn_readfirstlane(hi);
+    const int g = __builtin_amdgcn_readfirstlane(h / (a.H / a.Hkv)), Lq = a.Lq;
     const float scale = a.softmax_scale * 1.4426950408889634f;
-    auto slot_of = [&](int r) {                                   // ring row of row r of the unit
-        const int s = j.slot0 + u * bs + r;
-        return s < j.cap ? s : s - j.cap;
+    float *Lall = (float *)(lds + kQBytes<D>);
+    // a key's distance to query q is q + d - its place among the keys
+    const int d = (int)(a.offset - jg), win = (int)min(a.window, (int64_t)1 << 30);
+    // queries that see any of the keys, in stages
+    const int q_lo = max(lo - d, 0), q_hi = min((int64_t)hi - d - 1 + win, (int64_t)Lq);
+    const int st_lo = q_lo / kQRows, st_hi = hi > lo && q_hi > q_lo ? (q_hi - 1) / kQRows + 1 : st_lo;
+
+    // ---- queries into LDS: an instruction fills 1024 bytes; a wave the rows from 16 * wave on
+    constexpr int kRowsPerLd = 1024 / kRow, kLd = kQRows / (4 * kRowsPerLd);
+    const bf16_t *qbase = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh;
+    const uint32_t q_lds = lds_address(lds) + wave * (kLd * 1024);
+    auto load_stage = [&](int s, int buf) {
+#pragma unroll
+        for (int i = 0; i < kLd; ++i) {
+            const int r = kRowsPerLd * (kLd * wave + i) + lane / (D / 8);                   // (rows behind the last query: the last one's, masked)
+            const int q = min(s * kQRows + r, Lq - 1);
+            load_to_lds16(qbase, (uint32_t)((int64_t)q * a.q_sl + ((lane & (D / 8 - 1)) ^ swz<D>(r)) * 8) * 2, q_lds + buf * kStage + i * 1024);
+        }
     };
-    // queries that see any of the unit's keys: i < n_q (they all lie behind the keys); sub-tiles wave, wave + 4, .. are this wave's
-    const int d_first = j.to_first - u * bs;                      // distance of query 0 to the unit's first key
-    const int n_q = max(min(a.Lq, j.win + bs - 1 - d_first), 0), n_sub = (n_q + 31) / 32;
-    bf16x8 qa[kSubs][D / 16];
+    if (st_lo < st_hi) load_stage(st_lo, 0);
+    if (st_lo + 1 < st_hi) load_stage(st_lo + 1, 1);
+
+    // ---- this wave's keys as the B operand (lane = key column)
+    bf16x8 kreg[KS][D / 16];
 #pragma unroll
-    for (int i = 0; i < kSubs; ++i)
-        if (wave + 4 * i < n_sub) {
-            const bf16_t *row = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh +
-                                (int64_t)min((wave + 4 * i) * 32 + col, a.Lq - 1) * a.q_sl + grp * 8;
-#pragma unroll
-            for (int kk = 0; kk < D / 16; ++kk) qa[i][kk] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(row + kk * 16));
-        }
-    constexpr int kLoads = kCarveMaxUnit * kChunks / 256;
-    u32x4 rows[kLoads];
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-        const int r = (tid + i * 256) / kChunks, c = tid % kChunks;
-        if (r < bs) rows[i] = *(const u32x4 *)((const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + (int64_t)slot_of(r) * a.k_sl + c * 8);
-    }
-    float track = 0.f;
-    if (tid < bs) track = a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + slot_of(tid)];
-    {                                                            // joined log-sum-exps (score_tile's join), two queries a thread
-        const int64_t all = (int64_t)a.B * a.H * a.Lq;
-        const float *lse = a.d_lse + ((int64_t)b * a.H + h) * a.Lq;
-        float l8[2][8];
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-#pragma unroll
-            for (int p = 0; p < 8; ++p) l8[e][p] = tid + e * 256 < min(n_sub * 32, a.Lq) && p < a.n_parts ? lse[j.merge.ps.l(p, all) + tid + e * 256] : -INFINITY;
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            float m8 = -INFINITY, den = 0.f;
-#pragma unroll
-            for (int p = 0; p < 8; ++p) m8 = fmaxf(m8, l8[e][p]);
-            if (m8 != -INFINITY) {
-#pragma unroll
-                for (int p = 0; p < 8; ++p) den += __builtin_amdgcn_exp2f(l8[e][p] - m8);
-            }
-            lds.lse[tid + e * 256] = den > 0.f ? m8 + log2f(den) : INFINITY;      // +inf => probability 0
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-        const int r = (tid + i * 256) / kChunks, c = tid % kChunks;
-        if (r < bs) *(u32x4 *)&lds.keys[(r * kChunks + (c ^ (r % kChunks))) * 8] = rows[i];
-    }
-    __syncthreads();
-    for (int kg = 0; kg < bs / 32; ++kg) {
-        const bf16_t *krow = &lds.keys[(kg * 32 + col) * D];
-        f32x16 s[kSubs];
-#pragma unroll
-        for (int i = 0; i < kSubs; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[i][r] = 0.f;
+    for (int ks = 0; ks < KS; ++ks) {
+        const int r = wave * kWaveKeys + ks * 32 + col;
+        int row = slot + r;
+        row = row < cap ? row : row - cap;
+        const bf16_t *krow = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + (int64_t)row * a.k_sl + grp * 8;
 #pragma unroll
         for (int kk = 0; kk < D / 16; ++kk) {
-            const bf16x8 key = *(const bf16x8 *)(krow + ((kk * 2 + grp) ^ (col % kChunks)) * 8);
-#pragma unroll
-            for (int i = 0; i < kSubs; ++i)
-                if (wave + 4 * i < n_sub) s[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[i][kk], key, s[i], 0, 0, 0);
+            const u32x4 raw = r >= lo && r < hi ? *(const u32x4 *)(krow + kk * 16) : u32x4{0, 0, 0, 0};
+            kreg[ks][kk] = __builtin_bit_cast(bf16x8, raw);
         }
+    }
+    // ---- joined log-sum-exps of all queries, two a thread: one trip to memory for 512
+    {
+        const int64_t all = (int64_t)a.B * a.H * Lq;
+        const float *lse = a.d_lse + ((int64_t)b * a.H + h) * Lq;
+        const int padded = (Lq + kQRows - 1) / kQRows * kQRows;
+        for (int i0 = tid; i0 < padded; i0 += 512) {
+            float l8[2][8];
 #pragma unroll
-        for (int i = 0; i < kSubs; ++i) {
-            const int sub = wave + 4 * i;
-            if (sub >= n_sub) break;
-            f32x4 l4[4];
+            for (int e = 0; e < 2; ++e)
 #pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) l4[q4] = *(const f32x4 *)&lds.lse[sub * 32 + 8 * q4 + 4 * grp];
-            const int e0 = d_first + sub * 32 - kg * 32;         // distance of the sub-tile's first query to the group's first key
-            float acc = 0.f;
-            if (e0 - 31 >= 0 && e0 + 31 < j.win) {
+                for (int p = 0; p < 8; ++p) l8[e][p] = i0 + e * 256 < Lq && p < a.n_parts ? lse[lps.l(p, all) + i0 + e * 256] : -INFINITY;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) acc += __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][r], scale, -l4[r >> 2][r & 3]));
-            } else {
+            for (int e = 0; e < 2; ++e) {
+                float m8 = -INFINITY, den = 0.f;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int dist = e0 - col + 8 * (r >> 2) + 4 * grp + (r & 3);
-                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][r], scale, -l4[r >> 2][r & 3]));
-                    acc += dist >= 0 && dist < j.win ? p : 0.f;
+                for (int p = 0; p < 8; ++p) m8 = fmaxf(m8, l8[e][p]);
+                if (m8 != -INFINITY) {
+#pragma unroll
+                    for (int p = 0; p < 8; ++p) den += __builtin_amdgcn_exp2f(l8[e][p] - m8);
                 }
+                if (i0 + e * 256 < padded) Lall[i0 + e * 256] = den > 0.f ? m8 + log2f(den) : INFINITY;      // +inf => probability 0
             }
-            lds.sums[sub][grp][kg * 32 + col] = acc;
         }
     }
     __syncthreads();
-    // ---- the representatives: row r's place in the order is the number of rows in front of it
-    if (tid < kCarveMaxUnit) {
-        uint64_t key = 0;
-        if (tid < bs) {
-            float lo = 0.f, hi = 0.f;
-            if (n_sub == kCarveMaxLq / 32) {
+
+    const int w_first = wave * kWaveKeys;
+    const int w_lo = max(lo, w_first), w_hi = min(hi, w_first + kWaveKeys);                   // the wave's keys that count
+    const bool whole = w_lo == w_first && w_hi == w_first + kWaveKeys;
+    float colsum[KS] = {};
+    int buf = 0;
+    for (int s = st_lo; s < st_hi; ++s) {
+        // this wave's rows of the stage have landed (those of the next may be on their way), then everyone's; the buffer that
+        // the stage after next takes was read a stage ago
+        if (s + 1 < st_hi) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kLd) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_barrier" ::: "memory");
+        if (s + 2 < st_hi) load_stage(s + 2, buf == 0 ? 2 : buf - 1);
+        const int i0 = s * kQRows;
+        auto stage = [&](auto masked) {
+            constexpr bool kMasked = decltype(masked)::value;
+            constexpr int kSteps = kQRows / 32 * KS;            // (sub-tile of 32 queries, 32 keys), keys first
+            int q_first[KS];                                    // the queries that see this lane's keys: q_first .. q_first + q_count - 1
+            uint32_t q_count[KS];
+            if constexpr (kMasked) {
 #pragma unroll
-                for (int st = 0; st < kCarveMaxLq / 32; ++st) lo += lds.sums[st][0][tid], hi += lds.sums[st][1][tid];
-            } else {
-#pragma unroll 4
-                for (int st = 0; st < n_sub; ++st) lo += lds.sums[st][0][tid], hi += lds.sums[st][1][tid];
+                for (int ks = 0; ks < KS; ++ks) {
+                    const int r = w_first + ks * 32 + col - d;
+                    q_first[ks] = min(max(r, 0), Lq);
+                    q_count[ks] = (uint32_t)max((int)min(max((int64_t)r + win, (int64_t)0), (int64_t)Lq) - q_first[ks], 0);
+                }
             }
-            key = pick_key(track + (lo + hi), tid);
-        }
-        lds.rank_key[tid] = key;
+            f32x16 acc[2];
+            bf16x8 qa[D / 16];                                  // A operand: lane = query row
+            const uint32_t q_at = lds_address(lds) + buf * kStage + col * kRow + ((grp ^ swz<D>(col)) * 16);
+            auto issue = [&](int t) {
+                const int qs = t / KS, ks = t % KS;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[t & 1][r] = 0.f;
+#pragma unroll
+                for (int kk = 0; kk < D / 16; ++kk) {
+                    if (ks == 0) qa[kk] = __builtin_bit_cast(bf16x8, *(const __attribute__((address_space(3))) u32x4 *)(uintptr_t)((q_at ^ (kk * 32)) + qs * 32 * kRow));
+                    acc[t & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[kk], kreg[ks][kk], acc[t & 1], 0, 0, 0);
+                }
+            };
+            issue(0);
+            __builtin_amdgcn_sched_barrier(0);                  // (the fences keep the steps apart: registers)
+#pragma unroll
+            for (int t = 0; t < kSteps; ++t) {
+                const int qs = t / KS, ks = t % KS;
+                if (t + 1 < kSteps) issue(t + 1);
+                f32x4 l4[4];
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) l4[q4] = *(const f32x4 *)&Lall[i0 + qs * 32 + 8 * q4 + 4 * grp];
+                const int from = kMasked ? i0 + qs * 32 + 4 * grp - q_first[ks] : 0;
+                float sum = 0.f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {                  // query 8 * (r >> 2) + 4 * grp + (r & 3) of the sub-tile
+                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[t & 1][r], scale, -l4[r >> 2][r & 3]));
+                    if (kMasked) sum += (uint32_t)(from + 8 * (r >> 2) + (r & 3)) < q_count[ks] ? p : 0.f;
+                    else sum += p;
+                }
+                colsum[ks] += sum;
+                if (t + 1 < kSteps) {
+#pragma unroll
+                    for (int i = 0; i < D / 16; ++i) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // MFMA
+                        __builtin_amdgcn_sched_group_barrier(0x002, (kMasked ? 2 : 1) * 512 / D, 0);      // VALU
+                        __builtin_amdgcn_sched_group_barrier(0x400, 256 / D, 0);      // transcendental
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        // every pair is visible / some are (wave-uniform)
+        if (whole && i0 + kQRows <= Lq && i0 + d - (w_first + kWaveKeys - 1) >= 0 && i0 + kQRows - 1 + d - w_first < win) stage(std::false_type{});
+        else if (w_hi > w_lo && i0 + kQRows - 1 + d - w_lo >= 0 && i0 + d - (w_hi - 1) < win) stage(std::true_type{});
+        buf = buf == 2 ? 0 : buf + 1;
     }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) sums[ks] = colsum[ks] + wave_xor32(colsum[ks]);
+}
+
+// The representatives of a unit for one head: the unit's scores complete, the picks by counting - a row's place in the order is
+// the number of rows in front of it -, all rows at once.
+template <int D>
+__device__ __forceinline__ void carve_unit(const BlockEnd &j, int h, int u, int b, char *lds) {
+    const infllm_score_args &a = j.s;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 31, bs = j.bs;
+    int slot = j.unit_slot0 + u * bs;
+    slot = slot < j.cap ? slot : slot - j.cap;
+    auto slot_of = [&](int r) {                                   // ring row of row r of the unit
+        const int s = slot + r;
+        return s < j.cap ? s : s - j.cap;
+    };
+    const int own_row = wave * 32 + col;
+    const float track = own_row < bs ? a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + slot_of(own_row)] : 0.f;
+    float sum[1];
+    key_sums<D, 1>(a, j.merge.ps, b, h, j.t0 + (int64_t)u * bs, slot, j.cap, 0, bs, lds, sum);
+    __syncthreads();                                             // (the queries' place is free)
+    uint64_t *rank_key = (uint64_t *)lds;
+    int32_t *chosen = (int32_t *)(rank_key + kCarveMaxUnit);
+    if (lane < 32) rank_key[own_row] = own_row < bs ? pick_key(track + sum[0], own_row) : 0;
     __syncthreads();
     {
         constexpr int kLanes = 256 / kCarveMaxUnit;              // lanes that count for a row
         const int r = tid / kLanes, p = tid % kLanes;
-        const uint64_t own = lds.rank_key[r];
+        const uint64_t own = rank_key[r];
         int before = 0;
 #pragma unroll 16
-        for (int i = 0; i < kCarveMaxUnit / kLanes; ++i) before += lds.rank_key[i * kLanes + p] > own;
+        for (int i = 0; i < kCarveMaxUnit / kLanes; ++i) before += rank_key[i * kLanes + p] > own;
 #pragma unroll
         for (int o = 1; o < kLanes; o <<= 1) before += __shfl_xor(before, o, 64);
-        if (p == 0 && r < bs && before < j.repr_topk) lds.chosen[before] = r;
+        if (p == 0 && r < bs && before < j.repr_topk) chosen[before] = r;
     }
     __syncthreads();
     if (tid * 2 < D) {
-        const bf16_t *raw = j.ring_k_raw + ((int64_t)b * a.Hkv + g) * j.cap * D + tid * 2;
+        const bf16_t *raw = j.ring_k_raw + ((int64_t)b * a.Hkv + h / (a.H / a.Hkv)) * j.cap * D + tid * 2;
         float a0 = 0.f, a1 = 0.f;
 #pragma unroll 4
         for (int i = 0; i < j.repr_topk; ++i) {
-            const uint32_t w = *(const uint32_t *)(raw + (int64_t)slot_of(lds.chosen[i]) * D);
+            const uint32_t w = *(const uint32_t *)(raw + (int64_t)slot_of(chosen[i]) * D);
             a0 += bf16_bits_to_f32(w & 0xffffu);
             a1 += bf16_bits_to_f32(w >> 16);
         }
@@ -480,37 +542,52 @@ template <int D>
 constexpr int kRankCpl = D == 64 ? 5 : 9;
 
 template <int D, int KS>
-__global__ __launch_bounds__(256, (D == 64 && KS == 1 ? 3 : 2)) void block_end_kernel(BlockEnd j) {
-    extern __shared__ __attribute__((aligned(16))) char score_lds[];
-    __shared__ int last;
+__global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(BlockEnd j) {
+    extern __shared__ __attribute__((aligned(1024))) char score_lds[];
     int x = blockIdx.x;
     if (x < j.n_carve) {
         if (j.n_units > 0) {
             const int rest = x / j.s.H;
-            carve_unit<D>(j, x - rest * j.s.H, rest % j.n_units, rest / j.n_units, *(CarveLds<D> *)score_lds);
+            carve_unit<D>(j, x - rest * j.s.H, rest % j.n_units, rest / j.n_units, score_lds);
             if (!j.ranks) return;
             // The representatives are the only thing that crosses workgroups, and their stores have been performed where every
             // XCD sees them before the ticket is drawn: no workgroup has to write its L2 back.
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
+            int &last = *(int *)(score_lds + kCarveMaxUnit * 16);
             if (threadIdx.x == 0) last = __hip_atomic_fetch_add(j.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)j.n_carve - 1;
             __syncthreads();
             if (!last) return;
+            __syncthreads();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             if (threadIdx.x == 0) __hip_atomic_store(j.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        rank_block<kRankCpl<D>>(j.rank, 0, j.rank.n_new, *(RankLds *)score_lds);
+        rank_block<kRankCpl<D>>(j.rank, 0, j.rank.n_new, *(RankLds<kRankCpl<D>> *)score_lds);
         return;
     }
     x -= j.n_carve;
     if (x < j.n_score) {
-        const int rows = j.s.B * j.s.H;
-        score_tile<D, KS, 128, true>(j.s, j.merge.ps, x % rows, x / rows, j.n_score / rows, score_lds);
+        // (heads of different kv heads next to each other: see score_tile)
+        const infllm_score_args &a = j.s;
+        const int rows = a.B * a.H, tile = x / rows, bx = x - tile * rows, b = bx / a.H, hx = bx - b * a.H, g = hx % a.Hkv, h = g * (a.H / a.Hkv) + hx / a.Hkv;
+        constexpr int kKeys = 128 * KS;
+        const int64_t jg = a.j_lo / (32 * KS) * (32 * KS) + (int64_t)tile * kKeys;
+        int slot = j.slot0 + tile * kKeys;
+        slot = slot < j.cap ? slot : slot - j.cap;
+        const int lo = (int)max(a.j_lo - jg, (int64_t)0), hi = (int)min(a.j_hi - jg, (int64_t)kKeys);
+        float sums[KS];
+        key_sums<D, KS>(a, j.merge.ps, b, h, jg, slot, j.cap, lo, hi, score_lds, sums);
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int r = (threadIdx.x >> 6) * (32 * KS) + ks * 32 + lane, row = slot + r < j.cap ? slot + r : slot + r - j.cap;
+            if (lane < 32 && r >= lo && r < hi) a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + row] += sums[ks];
+        }
         return;
     }
     x -= j.n_score;
     if (x < j.n_early) {                                          // the units carved before, for the blocks behind the next
-        rank_block<kRankCpl<D>>(j.rank, x + 1, j.rank.n_before, *(RankLds *)score_lds);
+        rank_block<kRankCpl<D>>(j.rank, x + 1, j.rank.n_before, *(RankLds<kRankCpl<D>> *)score_lds);
         return;
     }
     x -= j.n_early;
@@ -555,8 +632,7 @@ int score_lds_setup() {
         if (e == hipSuccess)
             e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)score_lds_bytes<D>(128));
-        for (const void *k : {(const void *)local_score_kernel<D, 2, 128, true>, (const void *)local_score_kernel<D, 1, 128, true>,
-                              (const void *)block_end_kernel<D, 2>, (const void *)block_end_kernel<D, 1>})
+        for (const void *k : {(const void *)local_score_kernel<D, 2, 128, true>, (const void *)local_score_kernel<D, 1, 128, true>})
             if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)score_lds_bytes_merged<D>(128, kMergedMaxLq));
         if (e != hipSuccess) return infllm_fail(-2, "local_score: %s", hipGetErrorString(e));
         lds_set.store(true, std::memory_order_release);
@@ -622,15 +698,14 @@ int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *s
 
 template <int D>
 static int block_end_launch(BlockEnd &j, bool scores, hipStream_t st) {
-    static_assert(sizeof(CarveLds<D>) <= 2 * 128 * kQPad<D> * sizeof(bf16_t) + 128 * sizeof(float) && sizeof(RankLds) <= sizeof(CarveLds<D>), "LDS of a workgroup");
-    const int rc = score_lds_setup<D>();
-    if (rc) return rc;
+    static_assert(sizeof(RankLds<kRankCpl<D>>) <= kQBytes<D> && kCarveMaxUnit * 16 + 4 <= kQBytes<D>, "LDS of a workgroup");
     const infllm_score_args &a = j.s;
     const bool wide = scores && wide_waves(a);
     if (scores) {
         const int wave_keys = wide ? 64 : 32;
         const int64_t tiles = (a.j_hi - 1) / wave_keys - a.j_lo / wave_keys + 1;
         j.n_score = (int32_t)((tiles + 3) / 4 * a.B * a.H);
+        j.slot0 = (int32_t)(a.j_lo / wave_keys * wave_keys % a.cap);
     }
     const int64_t copies = (int64_t)2 * a.B * a.Hkv * j.n_units * j.bs * (D / 8), pieces = j.merge.out ? (int64_t)a.B * a.H * a.Lq * (D / 8) : 0;
     INFLLM_REQUIRE(copies < (1ll << 32), "block_end: copy too large");
@@ -639,7 +714,7 @@ static int block_end_launch(BlockEnd &j, bool scores, hipStream_t st) {
     INFLLM_REQUIRE(wgs < (1ll << 31), "block_end: grid too large");
     if (wgs == 0) return 0;
     const auto kern = wide ? block_end_kernel<D, 2> : block_end_kernel<D, 1>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(256), score_lds_bytes_merged<D>(128, a.Lq), st, j);
+    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(256), kQBytes<D> + (size_t)(a.Lq + kQRows - 1) / kQRows * kQRows * sizeof(float), st, j);
     INFLLM_CHECK_LAUNCH("block_end");
     return 0;
 }
@@ -671,23 +746,24 @@ int infllm_block_end(const infllm_score_args *a, const MergeJob *job, const void
     const int rc = check_score_args(&j.s);
     if (rc) return rc;
     INFLLM_REQUIRE(job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1, "block_end: the merge does not belong to these queries");
+    INFLLM_REQUIRE(a->accumulate && a->cap < (1ll << 30) && (int64_t)a->Lq * a->q_sl < (1ll << 30) && a->j_hi <= a->offset + a->Lq &&
+                       a->j_lo >= a->offset - a->cap && a->cap >= 256 && a->j_hi - a->j_lo + 64 <= a->cap, "block_end: bad ring or strides");
     j.merge = *job;
+    j.cap = (int32_t)a->cap;
     if (n_units > 0) {
         INFLLM_REQUIRE(d_ring_k_raw && d_ring_v && d_rep_out && d_out_k && d_out_v, "block_end: null pointer");
         INFLLM_REQUIRE(repr_topk >= 1 && repr_topk <= bs && t0 >= 0 && (int64_t)n_units * bs <= a->cap, "block_end: bad sizes");
         INFLLM_REQUIRE(t0 + (int64_t)n_units * bs <= a->offset + 1, "block_end: the units reach into the block");
         INFLLM_REQUIRE((rep_sb | rep_su) % 2 == 0 && (out_sb | out_su | out_sh) % 8 == 0, "block_end: bad strides");
-        INFLLM_REQUIRE(a->cap < (1ll << 30) && (int64_t)a->H * n_units * a->B < (1ll << 30), "block_end: ring or batch too large");
+        INFLLM_REQUIRE((int64_t)a->H * n_units * a->B < (1ll << 30), "block_end: batch too large");
         j.n_carve = a->H * n_units * a->B;
         j.ring_k_raw = (const bf16_t *)d_ring_k_raw;
-        j.slot0 = (int32_t)(t0 % a->cap); j.cap = (int32_t)a->cap; j.bs = bs; j.n_units = n_units; j.repr_topk = repr_topk;
-        j.to_first = (int32_t)std::min<int64_t>(a->offset - t0, 1 << 29);
-        j.win = (int32_t)std::min<int64_t>(a->window, 1 << 28);
+        j.t0 = t0; j.unit_slot0 = (int32_t)(t0 % a->cap); j.bs = bs; j.n_units = n_units; j.repr_topk = repr_topk;
         j.rep_out = (bf16_t *)d_rep_out; j.rep_sb = rep_sb; j.rep_su = rep_su;
         CarveCopy &cc = j.cc;
         cc.ring_a = (const bf16_t *)d_ring_k_raw; cc.ring_b = (const bf16_t *)d_ring_v;
         cc.out_a = (bf16_t *)d_out_k; cc.out_b = (bf16_t *)d_out_v;
-        cc.ring_cap = j.cap; cc.slot0 = j.slot0; cc.out_sb = out_sb; cc.out_su = out_su; cc.out_sh = out_sh;
+        cc.ring_cap = j.cap; cc.slot0 = j.unit_slot0; cc.out_sb = out_sb; cc.out_su = out_su; cc.out_sh = out_sh;
         cc.Hkv = a->Hkv; cc.B = a->B; cc.n = n_units * bs; cc.unit_rows = bs;
     }
     if (rank) {
