@@ -74,6 +74,9 @@ __device__ __forceinline__ int swz(int row) {
 // kernel orders the transfers itself: vmcnt(0) and a barrier before a buffer is read, a barrier before it is refilled.
 // The row address is a scalar base and a 32-bit byte offset of the lane.  M0 is overwritten: nothing else in these kernels
 // uses it (LDS instructions have not since gfx9).
+__device__ __forceinline__ void load_to_lds4(const float *base, uint32_t lane_off, uint32_t lds) {      // 4 bytes a lane, at lds + 4 * lane
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(lds), "v"(lane_off), "s"(base) : "memory");
+}
 __device__ __forceinline__ void load_to_lds16(const bf16_t *base, uint32_t lane_off, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(lane_off), "s"(base) : "memory");
 }

@@ -35,6 +35,20 @@ struct ScoreMerge {
 };
 struct NoScoreMerge {};
 
+// Workgroups are dispatched x fastest: all heads of one key tile, then the next tile.  The two tiles at either end of a masked key
+// range see only part of the queries and finish early, so they go last: when the grid is a little more than what the chip holds
+// at once, the workgroups that start late are then the short ones.  (None at the low end when the first query sees it.)  Where the
+// queries are (nearly) as many as the keys, a tile's work falls from the first to the last instead: a CU that takes one of the
+// first half and one of the second gets a long and a short one.
+__device__ __forceinline__ int tile_of_slot(const infllm_score_args &a, int slot, int n_tiles) {
+    if (a.mask == INFLLM_MASK_WINDOW && a.Lq >= (a.j_hi - a.j_lo) - (a.j_hi - a.j_lo) / 4)
+        return slot < (n_tiles + 1) / 2 ? slot : n_tiles - 1 - (slot - (n_tiles + 1) / 2);
+    if (a.mask == INFLLM_MASK_WINDOW && a.j_lo >= a.offset + a.Lq - a.window) return slot;
+    if (n_tiles >= 6 && a.mask != INFLLM_MASK_NONE)
+        return slot < n_tiles - 4 ? slot + 2 : slot == n_tiles - 4 ? 1 : slot == n_tiles - 3 ? n_tiles - 2 : slot == n_tiles - 2 ? 0 : n_tiles - 1;
+    return slot;
+}
+
 // One workgroup of 256 threads: tile `slot` (in the order they are dispatched) of n_tiles of the keys, query head bx.  MERGE:
 // the joined log-sum-exps of all the queries go into LDS once, from the partial ones at a.d_lse + lps.
 template <int D, int KS, int QS, bool MERGE>
@@ -51,18 +65,7 @@ __device__ __forceinline__ void score_tile(const infllm_score_args &a, const Par
     // linear id, so with 8 (16, ...) kv heads the query heads that share a K tile sit behind the same L2 and that tile
     // leaves HBM once instead of once per query head
     const int b = bx / a.H, hx = bx % a.H, g = hx % a.Hkv, h = g * G + hx / a.Hkv;
-    // Workgroups are dispatched x fastest: all heads of one key tile, then the next tile.  The two tiles at either end
-    // of a masked key range see only part of the queries and finish early, so they go last: when the grid is a little
-    // more than what the chip holds at once, the workgroups that start late are then the short ones.
-    // (None at the low end when the first query sees it.)  Where the queries are (nearly) as many as the keys, a tile's work falls from the first to the last instead: a CU that
-    // takes one of the first half and one of the second gets a long and a short one.
-    int tile = slot;
-    if (a.mask == INFLLM_MASK_WINDOW && a.Lq >= (a.j_hi - a.j_lo) - (a.j_hi - a.j_lo) / 4)
-        tile = slot < (n_tiles + 1) / 2 ? slot : n_tiles - 1 - (slot - (n_tiles + 1) / 2);
-    else if (a.mask == INFLLM_MASK_WINDOW && a.j_lo >= a.offset + a.Lq - a.window)
-        tile = slot;
-    else if (n_tiles >= 6 && a.mask != INFLLM_MASK_NONE)
-        tile = slot < n_tiles - 4 ? slot + 2 : slot == n_tiles - 4 ? 1 : slot == n_tiles - 3 ? n_tiles - 2 : slot == n_tiles - 2 ? 0 : n_tiles - 1;
+    const int tile = tile_of_slot(a, slot, n_tiles);
     const int64_t jg = (a.j_lo / kWaveKeys + (int64_t)tile * 4) * kWaveKeys;         // first key of the workgroup
     const int64_t j0 = jg + (int64_t)wave * kWaveKeys;                               // first key of this wave
     const float scale = a.softmax_scale * 1.4426950408889634f;
@@ -312,7 +315,7 @@ struct BlockEnd {
     infllm_score_args s;               // the keys that stay
     MergeJob merge;                    // the block's partials (out NULL: merged before)
     int32_t n_carve, n_score, n_copy, n_early;     // workgroups of each kind, in this order, those that merge behind them
-    int32_t cap, slot0;                // rows of the ring; that of the first key of the first scoring workgroup
+    int32_t cap, slot0, win;           // rows of the ring; that of the first key of the first scoring workgroup; the window
     // units that leave
     const bf16_t *ring_k_raw;
     int64_t t0;                        // their first key, and its row
@@ -325,8 +328,11 @@ struct BlockEnd {
     uint32_t *ticket;                  // zero; the last of the carving workgroups to finish puts it back
 };
 
-// Column sums of the block's probabilities for 128 * KS consecutive keys of a query head, 32 * KS a wave and KS a lane (both
-// halves of the wave get them).  The keys are those from position jg on, in row `slot` of the ring, of which [lo, hi) count.
+// Column sums of the probabilities for 128 * KS consecutive keys of a query head, 32 * KS a wave and KS a lane (both halves of
+// the wave get them).  The keys are those from position jg on, of which [lo, hi) count; key r of them lies in row slot + r of the
+// ring, or a ring's length before.  A key is visible at distances [first, beyond) of a query.  JOIN: the log-sum-exps are
+// joined from partial ones (at a.d_lse + lps), of all queries before the first stage; else they are finished (a.d_lse) and
+// come with a stage's queries.
 //
 // A wave's exponentials and MFMAs overlap (half a sub-tile of 32 queries apart), so the loop runs at the rate of the vector unit
 // (768 cycles of a sub-tile of 32 queries x 64 keys); what is left is a launch of one or two rounds of workgroups whose first 7
@@ -339,25 +345,26 @@ constexpr int kQRows = 64;                             // queries of a stage
 template <int D>
 constexpr size_t kQBytes = (size_t)3 * kQRows * D * sizeof(bf16_t);
 
-template <int D, int KS>
-__device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartSets lps, int b, int h, int64_t jg, int slot, int cap, int lo, int hi, char *lds,
-                                         float (&sums)[KS]) {
+template <int D, int KS, bool JOIN>
+__device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartSets lps, int b, int h, int64_t jg, int slot, int cap, int lo, int hi, int first,
+                                         int beyond, char *lds, float (&sums)[KS]) {
     constexpr int kWaveKeys = 32 * KS, kRow = D * 2, kStage = kQRows * kRow;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 31, grp = lane >> 5;
     b = __builtin_amdgcn_readfirstlane(b), h = __builtin_amdgcn_readfirstlane(h), slot = __builtin_amdgcn_readfirstlane(slot);
     lo = __builtin_amdgcn_readfirstlane(lo), hi = __builtin_amdgcn_readfirstlane(hi);
     const int g = __builtin_amdgcn_readfirstlane(h / (a.H / a.Hkv)), Lq = a.Lq;
     const float scale = a.softmax_scale * 1.4426950408889634f;
-    float *Lall = (float *)(lds + kQBytes<D>);
+    float *Ls = (float *)(lds + kQBytes<D>);                       // JOIN: [Lq rounded up to a stage]; else [3][kQRows]
     // a key's distance to query q is q + d - its place among the keys
-    const int d = (int)(a.offset - jg), win = (int)min(a.window, (int64_t)1 << 30);
+    const int d = (int)min(max(a.offset - jg, (int64_t)-(1 << 29)), (int64_t)(1 << 29));
     // queries that see any of the keys, in stages
-    const int q_lo = max(lo - d, 0), q_hi = min((int64_t)hi - d - 1 + win, (int64_t)Lq);
+    const int q_lo = max(lo - d + first, 0), q_hi = (int)min((int64_t)hi - d - 1 + beyond, (int64_t)Lq);
     const int st_lo = q_lo / kQRows, st_hi = hi > lo && q_hi > q_lo ? (q_hi - 1) / kQRows + 1 : st_lo;
 
     // ---- queries into LDS: an instruction fills 1024 bytes; a wave the rows from 16 * wave on
     constexpr int kRowsPerLd = 1024 / kRow, kLd = kQRows / (4 * kRowsPerLd);
     const bf16_t *qbase = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh;
+    const float *lse = a.d_lse + ((int64_t)b * a.H + h) * Lq;
     const uint32_t q_lds = lds_address(lds) + wave * (kLd * 1024);
     auto load_stage = [&](int s, int buf) {
 #pragma unroll
@@ -366,6 +373,8 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
             const int q = min(s * kQRows + r, Lq - 1);
             load_to_lds16(qbase, (uint32_t)((int64_t)q * a.q_sl + ((lane & (D / 8 - 1)) ^ swz<D>(r)) * 8) * 2, q_lds + buf * kStage + i * 1024);
         }
+        if (!JOIN && lane < kQRows / 4)
+            load_to_lds4(lse, (uint32_t)min(s * kQRows + wave * (kQRows / 4) + lane, Lq - 1) * 4, lds_address((char *)(Ls + buf * kQRows + wave * (kQRows / 4))));
     };
     if (st_lo < st_hi) load_stage(st_lo, 0);
     if (st_lo + 1 < st_hi) load_stage(st_lo + 1, 1);
@@ -385,9 +394,8 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
         }
     }
     // ---- joined log-sum-exps of all queries, two a thread: one trip to memory for 512
-    {
+    if constexpr (JOIN) {
         const int64_t all = (int64_t)a.B * a.H * Lq;
-        const float *lse = a.d_lse + ((int64_t)b * a.H + h) * Lq;
         const int padded = (Lq + kQRows - 1) / kQRows * kQRows;
         for (int i0 = tid; i0 < padded; i0 += 512) {
             float l8[2][8];
@@ -404,12 +412,17 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
 #pragma unroll
                     for (int p = 0; p < 8; ++p) den += __builtin_amdgcn_exp2f(l8[e][p] - m8);
                 }
-                if (i0 + e * 256 < padded) Lall[i0 + e * 256] = den > 0.f ? m8 + log2f(den) : INFINITY;      // +inf => probability 0
+                if (i0 + e * 256 < padded) Ls[i0 + e * 256] = den > 0.f ? m8 + log2f(den) : INFINITY;      // +inf => probability 0
             }
         }
+        __syncthreads();
     }
-    __syncthreads();
 
+    // (the keys' wait belongs here: in front of their first use, inside the loop, it would be one for the stages on their way)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(kreg[ks][kk]));
     const int w_first = wave * kWaveKeys;
     const int w_lo = max(lo, w_first), w_hi = min(hi, w_first + kWaveKeys);                   // the wave's keys that count
     const bool whole = w_lo == w_first && w_hi == w_first + kWaveKeys;
@@ -418,7 +431,7 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
     for (int s = st_lo; s < st_hi; ++s) {
         // this wave's rows of the stage have landed (those of the next may be on their way), then everyone's; the buffer that
         // the stage after next takes was read a stage ago
-        if (s + 1 < st_hi) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kLd) : "memory");
+        if (s + 1 < st_hi) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(JOIN ? kLd : kLd + 1) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         asm volatile("s_barrier" ::: "memory");
         if (s + 2 < st_hi) load_stage(s + 2, buf == 0 ? 2 : buf - 1);
@@ -432,8 +445,8 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
                     const int r = w_first + ks * 32 + col - d;
-                    q_first[ks] = min(max(r, 0), Lq);
-                    q_count[ks] = (uint32_t)max((int)min(max((int64_t)r + win, (int64_t)0), (int64_t)Lq) - q_first[ks], 0);
+                    q_first[ks] = min(max(r + first, 0), Lq);
+                    q_count[ks] = (uint32_t)max((int)min(max((int64_t)r + beyond, (int64_t)0), (int64_t)Lq) - q_first[ks], 0);
                 }
             }
             f32x16 acc[2];
@@ -457,7 +470,7 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
                 if (t + 1 < kSteps) issue(t + 1);
                 f32x4 l4[4];
 #pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) l4[q4] = *(const f32x4 *)&Lall[i0 + qs * 32 + 8 * q4 + 4 * grp];
+                for (int q4 = 0; q4 < 4; ++q4) l4[q4] = *(const f32x4 *)&Ls[(JOIN ? i0 : buf * kQRows) + qs * 32 + 8 * q4 + 4 * grp];
                 const int from = kMasked ? i0 + qs * 32 + 4 * grp - q_first[ks] : 0;
                 float sum = 0.f;
 #pragma unroll
@@ -479,12 +492,43 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
             }
         };
         // every pair is visible / some are (wave-uniform)
-        if (whole && i0 + kQRows <= Lq && i0 + d - (w_first + kWaveKeys - 1) >= 0 && i0 + kQRows - 1 + d - w_first < win) stage(std::false_type{});
-        else if (w_hi > w_lo && i0 + kQRows - 1 + d - w_lo >= 0 && i0 + d - (w_hi - 1) < win) stage(std::true_type{});
+        if (whole && i0 + kQRows <= Lq && i0 + d - (w_first + kWaveKeys - 1) >= first && i0 + kQRows - 1 + d - w_first < beyond) stage(std::false_type{});
+        else if (w_hi > w_lo && i0 + kQRows - 1 + d - w_lo >= first && i0 + d - (w_hi - 1) < beyond) stage(std::true_type{});
         buf = buf == 2 ? 0 : buf + 1;
     }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) sums[ks] = colsum[ks] + wave_xor32(colsum[ks]);
+}
+
+// Heads of different kv heads next to each other, see score_tile.
+__device__ __forceinline__ void head_of(const infllm_score_args &a, int bx, int &b, int &h) {
+    b = bx / a.H;
+    const int hx = bx - b * a.H, rest = hx / a.Hkv;
+    h = (hx - rest * a.Hkv) * (a.H / a.Hkv) + rest;
+}
+
+// The scores of a launch whose log-sum-exps are finished: the form of the kernel that keeps three workgroups on a CU
+// (operator over 512 queries x (4,608 + 2,624) keys 108.4 -> 102.9 us a pass, prompt of 16,001 tokens 2,745 -> 2,723).
+template <int D, int KS>
+__global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void scores_kernel(infllm_score_args a, int slot0, int cap, int first, int beyond) {
+    extern __shared__ __attribute__((aligned(1024))) char score_lds[];
+    constexpr int kKeys = 128 * KS;
+    int b, h;
+    head_of(a, blockIdx.x, b, h);
+    const int tile = tile_of_slot(a, blockIdx.y, gridDim.y);
+    const int64_t jg = a.j_lo / (32 * KS) * (32 * KS) + (int64_t)tile * kKeys;
+    const int lo = (int)max(a.j_lo - jg, (int64_t)0), hi = (int)min(a.j_hi - jg, (int64_t)kKeys);
+    float sums[KS];
+    key_sums<D, KS, false>(a, PartSets{}, b, h, jg, slot0 + tile * kKeys, cap, lo, hi, first, beyond, score_lds, sums);
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        const int r = (threadIdx.x >> 6) * (32 * KS) + ks * 32 + lane;
+        if (lane < 32 && r >= lo && r < hi) {
+            float *dst = a.d_score + (int64_t)b * a.score_sb + (int64_t)h * a.score_sh + (jg + r) % a.score_cap;
+            *dst = a.accumulate ? *dst + sums[ks] : sums[ks];
+        }
+    }
 }
 
 // The representatives of a unit for one head: the unit's scores complete, the picks by counting - a row's place in the order is
@@ -493,8 +537,7 @@ template <int D>
 __device__ __forceinline__ void carve_unit(const BlockEnd &j, int h, int u, int b, char *lds) {
     const infllm_score_args &a = j.s;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 31, bs = j.bs;
-    int slot = j.unit_slot0 + u * bs;
-    slot = slot < j.cap ? slot : slot - j.cap;
+    const int slot = j.unit_slot0 + u * bs;
     auto slot_of = [&](int r) {                                   // ring row of row r of the unit
         const int s = slot + r;
         return s < j.cap ? s : s - j.cap;
@@ -502,7 +545,7 @@ __device__ __forceinline__ void carve_unit(const BlockEnd &j, int h, int u, int 
     const int own_row = wave * 32 + col;
     const float track = own_row < bs ? a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + slot_of(own_row)] : 0.f;
     float sum[1];
-    key_sums<D, 1>(a, j.merge.ps, b, h, j.t0 + (int64_t)u * bs, slot, j.cap, 0, bs, lds, sum);
+    key_sums<D, 1, true>(a, j.merge.ps, b, h, j.t0 + (int64_t)u * bs, slot, j.cap, 0, bs, 0, j.win, lds, sum);
     __syncthreads();                                             // (the queries' place is free)
     uint64_t *rank_key = (uint64_t *)lds;
     int32_t *chosen = (int32_t *)(rank_key + kCarveMaxUnit);
@@ -567,16 +610,16 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(Block
     }
     x -= j.n_carve;
     if (x < j.n_score) {
-        // (heads of different kv heads next to each other: see score_tile)
         const infllm_score_args &a = j.s;
-        const int rows = a.B * a.H, tile = x / rows, bx = x - tile * rows, b = bx / a.H, hx = bx - b * a.H, g = hx % a.Hkv, h = g * (a.H / a.Hkv) + hx / a.Hkv;
+        const int rows = a.B * a.H, tile = x / rows;
+        int b, h;
+        head_of(a, x - tile * rows, b, h);
         constexpr int kKeys = 128 * KS;
         const int64_t jg = a.j_lo / (32 * KS) * (32 * KS) + (int64_t)tile * kKeys;
-        int slot = j.slot0 + tile * kKeys;
-        slot = slot < j.cap ? slot : slot - j.cap;
+        const int slot = j.slot0 + tile * kKeys;
         const int lo = (int)max(a.j_lo - jg, (int64_t)0), hi = (int)min(a.j_hi - jg, (int64_t)kKeys);
         float sums[KS];
-        key_sums<D, KS>(a, j.merge.ps, b, h, jg, slot, j.cap, lo, hi, score_lds, sums);
+        key_sums<D, KS, true>(a, j.merge.ps, b, h, jg, slot, j.cap, lo, hi, 0, j.win, score_lds, sums);
         const int lane = threadIdx.x & 63;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
@@ -652,6 +695,20 @@ int score_launch(const infllm_score_args *a, void *stream) {
     int rc = check_score_args(a);
     if (rc) return rc;
     if (a->j_hi <= a->j_lo) return 0;
+    constexpr int64_t kMax = 1 << 30;
+    if (a->n_parts <= 0 && (a->cap < kMax || a->j_hi < kMax) && (int64_t)a->Lq * a->q_sl < kMax) {
+        const bool wide = wide_waves(*a);
+        const int wave_keys = wide ? 64 : 32;
+        const int64_t tiles = (a->j_hi - 1) / wave_keys - a->j_lo / wave_keys + 1, window = std::min(std::max(a->window, -kMax), kMax);
+        const int cap = (int)std::min(a->cap, kMax), slot0 = (int)(a->j_lo % a->cap - a->j_lo % wave_keys);      // (below 0: rows that do not count)
+        const int first = (int)(a->mask == INFLLM_MASK_WINDOW ? 0 : a->mask == INFLLM_MASK_COMPLEMENT ? window : -kMax);
+        const int beyond = (int)(a->mask == INFLLM_MASK_WINDOW ? std::max<int64_t>(window, 0) : kMax);
+        const auto kern = wide ? scores_kernel<D, 2> : scores_kernel<D, 1>;
+        hipLaunchKernelGGL(kern, dim3(a->B * a->H, (unsigned)((tiles + 3) / 4)), dim3(256), kQBytes<D> + 3 * kQRows * sizeof(float), (hipStream_t)stream, *a, slot0,
+                           cap, first, beyond);
+        INFLLM_CHECK_LAUNCH("local_score");
+        return 0;
+    }
     rc = score_lds_setup<D>();
     if (rc) return rc;
     if (wide_waves(*a)) {
@@ -705,7 +762,7 @@ static int block_end_launch(BlockEnd &j, bool scores, hipStream_t st) {
         const int wave_keys = wide ? 64 : 32;
         const int64_t tiles = (a.j_hi - 1) / wave_keys - a.j_lo / wave_keys + 1;
         j.n_score = (int32_t)((tiles + 3) / 4 * a.B * a.H);
-        j.slot0 = (int32_t)(a.j_lo / wave_keys * wave_keys % a.cap);
+        j.slot0 = (int32_t)(a.j_lo % a.cap - a.j_lo % wave_keys);       // (below 0: rows that do not count)
     }
     const int64_t copies = (int64_t)2 * a.B * a.Hkv * j.n_units * j.bs * (D / 8), pieces = j.merge.out ? (int64_t)a.B * a.H * a.Lq * (D / 8) : 0;
     INFLLM_REQUIRE(copies < (1ll << 32), "block_end: copy too large");
@@ -747,9 +804,10 @@ int infllm_block_end(const infllm_score_args *a, const MergeJob *job, const void
     if (rc) return rc;
     INFLLM_REQUIRE(job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1, "block_end: the merge does not belong to these queries");
     INFLLM_REQUIRE(a->accumulate && a->cap < (1ll << 30) && (int64_t)a->Lq * a->q_sl < (1ll << 30) && a->j_hi <= a->offset + a->Lq &&
-                       a->j_lo >= a->offset - a->cap && a->cap >= 256 && a->j_hi - a->j_lo + 64 <= a->cap, "block_end: bad ring or strides");
+                       a->j_lo >= a->offset - a->cap, "block_end: bad ring or strides");
     j.merge = *job;
     j.cap = (int32_t)a->cap;
+    j.win = (int32_t)std::min<int64_t>(a->window, 1 << 30);
     if (n_units > 0) {
         INFLLM_REQUIRE(d_ring_k_raw && d_ring_v && d_rep_out && d_out_k && d_out_v, "block_end: null pointer");
         INFLLM_REQUIRE(repr_topk >= 1 && repr_topk <= bs && t0 >= 0 && (int64_t)n_units * bs <= a->cap, "block_end: bad sizes");
