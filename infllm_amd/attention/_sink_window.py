@@ -183,7 +183,7 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
     rows_q = batch * num_heads * len_q
     q_bytes = (2 if kind else 1) * rows_q * dim * 2
     part_rows = 64 * rows_q if rows_q <= 2048 else _SPLIT_ROWS if 2 * rows_q <= _SPLIT_ROWS else 0
-    work_bytes = q_bytes + part_rows * (2 * dim + 4)
+    work_bytes = q_bytes + part_rows * (2 * dim + 4) + (4 * rows_q if len_q == 1 else 0)
     work = torch.empty((work_bytes,), dtype=torch.uint8, device=dev)
     out = torch.empty((batch, len_q, num_heads * dim), **bf)
     okp = ovp = 0

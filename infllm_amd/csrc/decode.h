@@ -32,6 +32,10 @@ struct DecodeJob {
     int64_t unit_elems, row_elems, unit_v_off, unit_sh;
     float *logits;                         // optional [B, H, logit_stride]: scaled logits in base 2 (see DecodeSeg)
     int64_t logit_stride;
+    // Optional, without logits: the launch joins its splits itself, the finished row of head h goes to out + b * out_sb + h * out_sh.
+    bf16_t *out;
+    int64_t out_sb, out_sh;
+    uint32_t *ticket;                      // [B * H] zeros, zeros again behind the launch
 };
 
 int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int64_t blocks, int32_t max_splits);

@@ -38,13 +38,16 @@ __device__ __forceinline__ void each_head(F &&f) {
 
 // D: head dimension (128 or 64); NG: query heads handled together (columns of the MFMA; heads beyond the group's last are
 // zero queries whose results are not written)
-template <int D, int NG, bool LOGITS>
+template <int D, int NG, bool LOGITS, bool JOIN>
 __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(DecodeJob j) {
     constexpr int KK = D / 32;                     // k-steps of the first MFMA
     constexpr int LPR = D / 8;                     // lanes that hold a value row, 16 bytes each
     constexpr int VL = kDecodeBlock * LPR / 64;    // value loads per block: 4 (D = 128) or 2 (D = 64)
     constexpr int GRP = 64 / LPR;                  // value rows of one load: one (D = 128) or two (D = 64) per row group
-    __shared__ float red[kDecWaves][GRP][NG][D];
+    constexpr int kJoin = 10;                      // words of a lane in the join of the splits
+    constexpr int kRed = kDecWaves * GRP * NG * D;
+    __shared__ __attribute__((aligned(16))) float red_room[!JOIN || kRed > kDecWaves * kWave * kJoin ? kRed : kDecWaves * kWave * kJoin];
+    float(*red)[GRP][NG][D] = (float(*)[GRP][NG][D])red_room;
     __shared__ float sm[kDecWaves][4][NG], sl[kDecWaves][4][NG];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int col = lane & 15, rg = lane >> 4;
@@ -226,9 +229,11 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         *(f32x4 *)(dst + 4) = f32x4{acc[h][4] * f, acc[h][5] * f, acc[h][6] * f, acc[h][7] * f};
     });
     __syncthreads();
-    for (int e = threadIdx.x; e < nh * D; e += kDecWaves * kWave) {
+    const int64_t row0 = ((int64_t)split * j.B + b) * j.H + h0;
+    for (int e = threadIdx.x * 2; e < nh * D; e += kDecWaves * kWave * 2) {
         const int h = e / D, d = e % D;
-        float mx = -INFINITY, den = 0.f, o = 0.f;
+        float mx = -INFINITY, den = 0.f;
+        float2 o{0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < kDecWaves; ++w)
 #pragma unroll
@@ -240,21 +245,100 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
 #pragma unroll
         for (int w = 0; w < kDecWaves; ++w)
 #pragma unroll
-            for (int r = 0; r < GRP; ++r) o += red[w][r][h][d];
-        const int64_t row = ((int64_t)split * j.B + b) * j.H + h0 + h;
-        ((_Float16 *)j.o_part)[row * D + d] = (_Float16)(den == 0.f ? 0.f : o / den);
-        if (d == 0) j.lse_part[row] = den > 0.f ? mx * scale + log2f(den) : -INFINITY;
+            for (int r = 0; r < GRP; ++r) o.x += red[w][r][h][d], o.y += red[w][r][h][d + 1];
+        const f16x2 part{(_Float16)(den == 0.f ? 0.f : o.x / den), (_Float16)(den == 0.f ? 0.f : o.y / den)};
+        const float lse = den > 0.f ? mx * scale + log2f(den) : -INFINITY;
+        uint32_t *dst = (uint32_t *)(j.o_part + (row0 + h) * D + d);
+        if (!JOIN) {
+            *dst = __builtin_bit_cast(uint32_t, part);
+            if (d == 0) j.lse_part[row0 + h] = lse;
+        } else {                                   // (performed where every XCD sees it: the split that ends last reads it)
+            __hip_atomic_store(dst, __builtin_bit_cast(uint32_t, part), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (d == 0) __hip_atomic_store(j.lse_part + row0 + h, lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    if constexpr (JOIN) {
+        // ---- The split that ends last joins them: a launch of its own is 4.8 us, of which next to nothing is work.  Every split's
+        //      stores have been performed before its ticket is drawn, and nothing else crosses workgroups, so that none has to
+        //      write its L2 back.  Wave w takes every fourth split, a lane one head's 8 elements (merge_piece's arithmetic).
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        int &last = *(int *)&sm[0][0][0];
+        uint32_t *ticket = j.ticket + (int64_t)b * gridDim.y + blockIdx.y;
+        if (threadIdx.x == 0) last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        __syncthreads();
+        if (!last) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();                           // (the word is sm's)
+        const int h = lane / LPR, at = (lane & (LPR - 1)) * 8;                 // (heads of 64: four of them are 32 lanes)
+        const bool on = h < nh;
+        const int64_t step = (int64_t)j.B * j.H, row = (int64_t)b * j.H + h0 + (on ? h : 0);
+        float mx = -INFINITY, den = 0.f, o[8] = {};
+        constexpr int kBatch = 8;                  // splits whose rows are requested together
+        for (int s0 = wave; s0 < (int)gridDim.x; s0 += kBatch * kDecWaves) {
+            float l8[kBatch];
+            f16x8 o8[kBatch];
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {
+                const int s = s0 + i * kDecWaves;
+                const bool in = on && s < (int)gridDim.x;
+                l8[i] = in ? j.lse_part[s * step + row] : -INFINITY;
+                o8[i] = in ? *(const f16x8 *)((const _Float16 *)j.o_part + (s * step + row) * D + at) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            }
+            float mn = mx;
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) mn = fmaxf(mn, l8[i]);
+            const float al = mx == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mx - mn), base = mn == -INFINITY ? 0.f : mn;
+            if (mx != -INFINITY) {
+                den *= al;
+#pragma unroll
+                for (int d = 0; d < 8; ++d) o[d] *= al;
+            }
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {     // exp2(-inf) = 0: empty splits hold zeros, those with a logit that was no number NaN
+                const float w = __builtin_amdgcn_exp2f(l8[i] - base);
+#pragma unroll
+                for (int d = 0; d < 8; ++d) o[d] += (float)o8[i][d] * w;
+                den += w;
+            }
+            mx = mn;
+        }
+        float *mine = red_room + (wave * 64 + lane) * kJoin;                   // 8 sums, the maximum, the weight
+#pragma unroll
+        for (int d = 0; d < 8; ++d) mine[d] = o[d];
+        mine[8] = mx, mine[9] = den;
+        __syncthreads();
+        if (wave != 0 || !on) return;
+        mx = -INFINITY, den = 0.f;
+#pragma unroll
+        for (int d = 0; d < 8; ++d) o[d] = 0.f;
+#pragma unroll
+        for (int w = 0; w < kDecWaves; ++w) mx = fmaxf(mx, red_room[(w * 64 + lane) * kJoin + 8]);
+        const float base = mx == -INFINITY ? 0.f : mx;
+#pragma unroll
+        for (int w = 0; w < kDecWaves; ++w) {
+            const float *part = red_room + (w * 64 + lane) * kJoin;
+            const float f = __builtin_amdgcn_exp2f(part[8] - base);
+            // (a wave whose splits are all empty or no numbers: its sums are zeros or NaN, taken with weight 0)
+#pragma unroll
+            for (int d = 0; d < 8; ++d) o[d] += part[d] * f;
+            den += part[9] * f;
+        }
+        const float inv = den > 0.f ? 1.f / den : 0.f;
+        *(u32x4 *)(j.out + (int64_t)b * j.out_sb + (int64_t)(h0 + h) * j.out_sh + at) =
+            u32x4{pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv), pack_bf16x2(o[4] * inv, o[5] * inv), pack_bf16x2(o[6] * inv, o[7] * inv)};
     }
 }
 
-template <int D, bool LOGITS>
+template <int D, bool LOGITS, bool JOIN>
 int launch(const DecodeJob *job, void *stream) {
     const int G = job->H / job->Hkv;
     const int NG = G >= 3 ? 4 : G;
     const dim3 grid(job->nsplit, job->Hkv * ((G + NG - 1) / NG), job->B);
-    if (NG == 1) hipLaunchKernelGGL((decode_attn_kernel<D, 1, LOGITS>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
-    else if (NG == 2) hipLaunchKernelGGL((decode_attn_kernel<D, 2, LOGITS>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
-    else hipLaunchKernelGGL((decode_attn_kernel<D, 4, LOGITS>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
+    if (NG == 1) hipLaunchKernelGGL((decode_attn_kernel<D, 1, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
+    else if (NG == 2) hipLaunchKernelGGL((decode_attn_kernel<D, 2, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
+    else hipLaunchKernelGGL((decode_attn_kernel<D, 4, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
     INFLLM_CHECK_LAUNCH("decode_attn");
     return 0;
 }
@@ -285,6 +369,8 @@ int infllm_decode_attn(const DecodeJob *job, int32_t dim, void *stream) {
         else INFLLM_REQUIRE(sg.rows == 0 || (sg.k && sg.v), "decode_attn: null range");
     }
     INFLLM_REQUIRE(dim == 128 || dim == 64, "decode_attn: head_dim %d", dim);
-    if (job->logits) return dim == 128 ? launch<128, true>(job, stream) : launch<64, true>(job, stream);
-    return dim == 128 ? launch<128, false>(job, stream) : launch<64, false>(job, stream);
+    INFLLM_REQUIRE(!job->out || (!job->logits && job->ticket && ((job->out_sb | job->out_sh) & 7) == 0), "decode_attn: bad output");
+    if (job->logits) return dim == 128 ? launch<128, true, false>(job, stream) : launch<64, true, false>(job, stream);
+    if (job->out) return dim == 128 ? launch<128, false, true>(job, stream) : launch<64, false, true>(job, stream);
+    return dim == 128 ? launch<128, false, false>(job, stream) : launch<64, false, false>(job, stream);
 }

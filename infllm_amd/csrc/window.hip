@@ -1,6 +1,6 @@
 // One call of an attention type with a plain cache - attention sinks + sliding window (inf_llm/attention/stream_llm.py:6-111,
 // infinite_lm.py:6-100) or causal attention (origin.py:4-79) - in two or three launches: the new tokens' rows (rotary
-// embedding, cache), the attention, and the merge of its key splits where it has any.
+// embedding, cache), the attention, and the merge of its key splits where several queries have any.
 #include <algorithm>
 
 #include "decode.h"
@@ -8,10 +8,6 @@
 
 int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, int32_t dim, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
                        void *stream);
-int infllm_attn_merge2(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2, const float *d_lse_part2,
-                       int32_t P2, int32_t B, int32_t H, int32_t Lq, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse,
-                       void *stream, int32_t dim);
-
 namespace {
 
 // rows [0, n) of a source to a destination, for every (batch row, kv head); rows are D elements apart on both sides
@@ -39,6 +35,8 @@ struct StageJob {
     int64_t raw_sb, raw_sh;
     int32_t n_raw;
     int32_t tiles;                             // workgroups along x that stage rows; the rest copy
+    uint32_t *clear;                           // n_clear words to set to zero (the decode kernel's tickets)
+    int32_t n_clear;
     RowCopy copy[kCopies];
 };
 
@@ -76,6 +74,8 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
         }
         return;
     }
+    if (blockIdx.x == 0 && b == 0 && g == 0)
+        for (int i = tid; i < j.n_clear; i += 256) j.clear[i] = 0;
     const int G = j.H / j.Hkv;
     const int p0 = blockIdx.x * kPosPerBlock, np = min(kPosPerBlock, j.n - p0);
     // ---- requests first: up to four query heads, the key head, the value head
@@ -211,6 +211,12 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     const int n_sink = sink_stage ? (int)std::min<int64_t>(a->n_init, rows_all) : 0;
     INFLLM_REQUIRE(!sink_stage || a->kind != 2 || (a->d_raw && a->raw_new >= n_sink), "window_forward: un-rotated sinks missing");
     const int64_t q_bytes = (causal ? 1 : 2) * q_elems * 2;
+    const int64_t rows_q = (int64_t)a->B * a->H * a->n_q;
+    // partial rows: what is left behind the queries (and a ticket per head, for a step)
+    const int64_t part_rows = std::max<int64_t>(0, a->work_bytes - q_bytes - (a->n_q == 1 ? 4 * rows_q : 0)) / (2 * D + 4);
+    const int max_parts = (int)std::min<int64_t>(part_rows / rows_q, 64);
+    const bool step = a->n_q == 1 && max_parts >= 1;
+    uint32_t *ticket = (uint32_t *)((char *)a->d_work + q_bytes + part_rows * (2 * D + 4));
     INFLLM_REQUIRE(a->work_bytes >= q_bytes, "window_forward: scratch of %lld bytes for %lld", (long long)a->work_bytes, (long long)q_bytes);
     bf16_t *q_loc = (bf16_t *)a->d_work, *q_sink = causal ? nullptr : q_loc + q_elems;
 
@@ -239,6 +245,7 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         j.raw_sh = raw_sh; j.raw_sb = raw_sh * a->Hkv;
         j.n_raw = a->raw_new - a->raw_old;
     }
+    if (step) j.clear = ticket, j.n_clear = (int32_t)rows_q;
     int nc = 0;
     auto copy = [&](const void *src, int64_t ss_b, int64_t ss_h, int64_t s_row, void *dst, int64_t ds_b, int64_t ds_h, int64_t d_row, int64_t n) {
         if (n > 0) j.copy[nc++] = RowCopy{(const bf16_t *)src + s_row * D, (bf16_t *)dst + d_row * D, ss_b, ss_h, ds_b, ds_h, (int32_t)n};
@@ -291,13 +298,10 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     }
 
     // ---- attention
-    const int64_t rows_q = (int64_t)a->B * a->H * a->n_q;
-    const int64_t part_rows = (a->work_bytes - q_bytes) / (2 * D + 4);
-    int max_parts = (int)std::min<int64_t>(part_rows / rows_q, 64);
     const bf16_t *sk = a->kind == 2 ? (const bf16_t *)a->d_raw : bk;
     const int64_t sk_sh = a->kind == 2 ? raw_sh : bk_sh, sk_sb = a->kind == 2 ? raw_sh * a->Hkv : bk_sb;
     const float scale = a->softmax_scale;
-    if (a->n_q == 1 && max_parts >= 1) {
+    if (step) {
         DecodeJob d{};
         d.q[0] = q_loc; d.q[1] = sink_stage ? q_sink : q_loc;
         d.q_sb = (int64_t)a->H * D; d.q_sh = D;
@@ -313,9 +317,9 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, blocks, max_parts);
         d.o_part = (uint16_t *)((char *)a->d_work + q_bytes);
         d.lse_part = (float *)((char *)a->d_work + q_bytes + part_rows * 2 * D);
-        rc = infllm_decode_attn(&d, D, stream);
-        if (rc) return rc;
-        return infllm_attn_merge2(d.o_part, d.lse_part, d.nsplit, nullptr, nullptr, 0, a->B, a->H, 1, a->d_out, a->o_sb, a->o_sh, a->o_sl, nullptr, stream, D);
+        d.out = (bf16_t *)a->d_out; d.out_sb = a->o_sb; d.out_sh = a->o_sh;
+        d.ticket = ticket;
+        return infllm_decode_attn(&d, D, stream);
     }
     infllm_attn_args l{}, s{};
     l.d_q = q_loc;
