@@ -47,8 +47,8 @@ int infllm_repr_keys_carve(const float *d_ring_score, const void *d_ring_k_raw, 
 int infllm_gather_rows_pair(const void *d_ring_a, void *d_out_a, const void *d_ring_b, void *d_out_b, int64_t ring_cap, int32_t B,
                             int32_t Hkv, int64_t t0, int32_t n, int32_t unit_rows, int64_t out_sb, int64_t out_su, int64_t out_sh,
                             void *stream, int32_t dim);
-int infllm_retrieve_fused(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar, int32_t k, float *d_scores,
-                          int32_t *d_idx, int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, void *stream);
+int infllm_retrieve_step(const void *d_reps, int64_t rep_stride, int32_t N, const infllm_ingest_args *in, int32_t dim, int32_t b, bool prologue, int32_t k,
+                         float *d_scores, int32_t *d_idx, void *stream);
 int infllm_key_splits(const infllm_layer_desc *d, int32_t n_queries, int32_t n_tiles);
 
 namespace {
@@ -403,11 +403,10 @@ int decode_step(Resident *R, const infllm_resident_call *a, int64_t st0, hipStre
     const int64_t b0 = R->length, b1 = b0 + 1;
     infllm_ingest_args in = ingest_args(R, a, st0, 1);
     const bool retrieve = N > d.topk;
-    int rc = infllm_ingest_dim(&in, d.dim, retrieve ? a->d_qbar : nullptr, st);
-    if (rc) return rc;
     const int n_sel = std::min(N, d.topk);
     const int32_t *ids = d.d_iota;
     FinishJob f{};
+    int rc = 1;
     if (retrieve) {
         int32_t slot = 0;
         rc = take_slot(R, &slot, &f.seq);
@@ -415,18 +414,24 @@ int decode_step(Resident *R, const infllm_resident_call *a, int64_t st0, hipStre
         f.log = d.d_log + (int64_t)slot * (B * d.topk + 1);
         f.ids = d.d_ids; f.n_ids = B * d.topk;
         ids = d.d_ids;
-        for (int u = 0; u < B; ++u) {
+        for (int u = 0; u < B; ++u) {                            // the prologue rides with the first row's retrieval
+            rc = infllm_retrieve_step((const bf16_t *)a->d_reps + (int64_t)u * a->rep_sb, a->rep_su, N, &in, d.dim, u, u == 0, d.topk,
+                                      a->d_unit_scores + (int64_t)u * a->unit_scores_sb, d.d_ids + (int64_t)u * d.topk, st);
+            if (rc < 0) return rc;
+            if (rc == 1) break;                                  // (of all rows or of none: it depends on their length and number)
+        }
+    }
+    if (rc == 1) {
+        rc = infllm_ingest_dim(&in, d.dim, retrieve ? a->d_qbar : nullptr, st);
+        for (int u = 0; u < B && retrieve && !rc; ++u) {
             const bf16_t *reps = (const bf16_t *)a->d_reps + (int64_t)u * a->rep_sb;
             float *scores = a->d_unit_scores + (int64_t)u * a->unit_scores_sb;
-            const float *qbar = a->d_qbar + (int64_t)u * C;
-            rc = infllm_retrieve_fused(reps, a->rep_su, N, C, qbar, d.topk, scores, d.d_ids + (int64_t)u * d.topk, nullptr, nullptr, 0, st);
-            if (rc == 1) {
-                rc = infllm_unit_scores(reps, a->rep_su, 0, N, C, qbar, scores, st);
-                if (!rc) rc = infllm_topk(scores, N, d.topk, d.d_ids + (int64_t)u * d.topk, st);
-            }
-            if (rc) return rc;
+            rc = infllm_unit_scores(reps, a->rep_su, 0, N, C, a->d_qbar + (int64_t)u * C, scores, st);
+            if (!rc) rc = infllm_topk(scores, N, d.topk, d.d_ids + (int64_t)u * d.topk, st);
         }
-    } else
+        if (rc) return rc;
+    }
+    if (!retrieve)
         R->queue.push_back(Resident::Entry{n_sel, 0, 0});
     DecodeJob j{};
     j.q[0] = (const bf16_t *)a->d_q_loc; j.q[1] = (const bf16_t *)a->d_q_glb;

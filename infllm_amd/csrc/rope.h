@@ -61,3 +61,48 @@ __device__ __forceinline__ void rope_angles(int64_t pos0, int np, int64_t glb_po
         cs_glb[f] = make_float2((float)c, (float)s);
     }
 }
+
+// One new position (a decode step) of one kv head: its query heads rotated to their position and to the one angle of the units,
+// its key and value into the rings, its scores at zero - what ingest_kernel does for a tile of one.  256 threads; cs: D float2.
+template <int D>
+__device__ __forceinline__ void ingest_one(const infllm_ingest_args &a, int b, int g, float2 *cs) {
+    constexpr int HALF = D / 2, C2 = D / 16;
+    const int tid = threadIdx.x, G = a.H / a.Hkv;
+    const bf16_t *q = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)g * G * a.q_sh;
+    u32x4 lo{}, hi{}, k_lo{}, k_hi{}, v_row{};
+    if (tid < G * C2) {                                      // (more than 32 (64) heads: the rest below)
+        lo = *(const u32x4 *)(q + (int64_t)(tid / C2) * a.q_sh + tid % C2 * 8);
+        hi = *(const u32x4 *)(q + (int64_t)(tid / C2) * a.q_sh + HALF + tid % C2 * 8);
+    }
+    if (tid < C2) {
+        const bf16_t *src = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + tid * 8;
+        k_lo = *(const u32x4 *)src, k_hi = *(const u32x4 *)(src + HALF);
+    }
+    if (tid < 2 * C2) v_row = *(const u32x4 *)((const bf16_t *)a.d_v + (int64_t)b * a.v_sb + (int64_t)g * a.v_sh + tid * 8);
+    rope_angles<HALF>(a.pos0, 1, a.glb_pos, a.distance_scale, a.d_inv_freq, (float2(*)[HALF])cs, cs + HALF);
+    __syncthreads();
+    for (int e = tid; e < G * C2; e += 256) {
+        const int c = e % C2, h = e / C2;
+        if (e >= 256) {
+            lo = *(const u32x4 *)(q + (int64_t)h * a.q_sh + c * 8);
+            hi = *(const u32x4 *)(q + (int64_t)h * a.q_sh + HALF + c * 8);
+        }
+        const int64_t o = ((int64_t)b * a.H + g * G + h) * D + c * 8;
+        Rot8 r = rotate8(lo, hi, cs + c * 8);
+        *(u32x4 *)((bf16_t *)a.d_q_loc + o) = r.lo;
+        *(u32x4 *)((bf16_t *)a.d_q_loc + o + HALF) = r.hi;
+        r = rotate8(lo, hi, cs + HALF + c * 8);
+        *(u32x4 *)((bf16_t *)a.d_q_glb + o) = r.lo;
+        *(u32x4 *)((bf16_t *)a.d_q_glb + o + HALF) = r.hi;
+    }
+    const int64_t slot = a.pos0 % a.ring_cap, at = (((int64_t)b * a.Hkv + g) * a.ring_cap + slot) * D;
+    if (tid < C2) {
+        *(u32x4 *)((bf16_t *)a.d_ring_k_raw + at + tid * 8) = k_lo;
+        *(u32x4 *)((bf16_t *)a.d_ring_k_raw + at + HALF + tid * 8) = k_hi;
+        const Rot8 r = rotate8(k_lo, k_hi, cs + tid * 8);
+        *(u32x4 *)((bf16_t *)a.d_ring_k_rot + at + tid * 8) = r.lo;
+        *(u32x4 *)((bf16_t *)a.d_ring_k_rot + at + HALF + tid * 8) = r.hi;
+    }
+    if (tid < 2 * C2) *(u32x4 *)((bf16_t *)a.d_ring_v + at + tid * 8) = v_row;
+    for (int h = tid; h < G; h += 256) a.d_ring_score[((int64_t)b * a.H + g * G + h) * a.ring_cap + slot] = 0.f;
+}
