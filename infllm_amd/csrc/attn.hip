@@ -437,6 +437,18 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
                 }
         }
     };
+    // Row sums are taken over the probabilities AS ROUNDED to bf16, the values that P.V multiplies: the output is then an exact
+    // convex combination of value rows (a row on which one key carries nearly all the weight comes out as that value row,
+    // whatever the rounding of its weight).  In a product of 4 x 4 x 4 blocks every lane is a column of its own block, so
+    // against ones it receives the sum of its own four values: 8 cycles of the matrix pipe for 4 keys.  (As one more 32 x
+    // 32 x 16 product per step, 128 cycles a tile instead of 64, prompts of 131,072 tokens 26,020 -> 25,495 us, the operator over
+    // 512 x (4,608 + 2,624) 102.7 -> 101.3; as 64 shifts and additions 220 cycles of the vector half.)
+    s16x4 ones{0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    asm volatile("" : "+v"(ones));
+    auto add_row_sums = [&](u32x4 p, f32x4 sums) {
+        sums = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(s16x4, u32x2{p[0], p[1]}), sums, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(s16x4, u32x2{p[2], p[3]}), sums, 0, 0, 0);
+    };
     // the running max that a tile's scores move, and with it the accumulators
     auto max_and_rescale = [&](f32x16 (&s)[2]) {
         // (four chains: a dependent instruction waits twice as long as another)
@@ -493,11 +505,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         }
         mask(s, t, PAGES && (MODE == kPaged || t >= n_lin) ? page_table[t - n_lin].n_valid : kTile);
         max_and_rescale(s);
-        // The row sum is taken over the probabilities AS ROUNDED to bf16, the values the second MFMA multiplies: the
-        // output is then an exact convex combination of value rows (a row on which one key carries nearly all the
-        // weight comes out as that value row, whatever the rounding of its weight), and a pair costs one dot
-        // instruction instead of two additions.
-        float psum[2] = {0.f, 0.f};
+        f32x4 sums{0.f, 0.f, 0.f, 0.f};
         uint32_t pw[2][8];
         auto exps = [&](int ks, int r0, int r1) {
 #pragma unroll
@@ -505,7 +513,6 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
                 float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[ks][r], scale, neg_ms));
                 float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[ks][r + 1], scale, neg_ms));
                 pw[ks][r >> 1] = pack_bf16x2(p0, p1);
-                psum[ks] = sum_bf16x2(pw[ks][r >> 1], psum[ks]);
             }
         };
         exps(0, 0, 16);                        // the first 32 keys now; the other 32 beside the MFMAs that consume these
@@ -527,6 +534,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
 #pragma unroll
                 for (int dt = 0; dt < D / 32; ++dt)
                     oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va[dt]), pb, oacc[dt], 0, 0, 0);
+                sums = add_row_sums(praw, sums);
                 if (gi < 2) {
 #pragma unroll
                     for (int dt = 0; dt < D / 32; ++dt) {
@@ -539,7 +547,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        l_run += psum[0] + psum[1];
+        l_run += sums[0];
     };
 
     auto load_q = [&](const infllm_attn_args &src) {
@@ -609,8 +617,6 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     // 587 -> 500 us of N(0, 1) data, 510 -> 372 of zeros, on which the card does not lower its clock.
     f32x16 s[2];
     uint32_t pw[2][8];
-    u32x4 ones{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
-    asm volatile("" : "+v"(ones));
     // A half's 32 operands, one per MFMA: 0-15 the V^T of the tile before (16-key step, then d-tile), 16-31 the K of this one.
     // Each is requested 8 MFMAs ahead, into the registers of the one that has just been used, and between the MFMAs: a run
     // of reads keeps the wave from issuing them.
@@ -628,13 +634,9 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             asm volatile("" : "+v"(pw[ks][r >> 1]));                                // formed here, not where it is read
         }
     };
-    // O += P.V of the tile before; the first 8 operands are on their way when it begins.  The row sums - over the probabilities
-    // AS ROUNDED to bf16, see tile_math - are one more MFMA per step, against ones: 128 cycles of a matrix pipe that has them
-    // to spare, where 64 shifts and additions took 220 of the vector half.
+    // O += P.V of the tile before; the first 8 operands are on their way when it begins.
     auto pv_mul = [&](uint32_t vb, uint32_t kb, auto meanwhile) {
-        f32x16 sums;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sums[r] = 0.f;
+        f32x4 sums{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             __builtin_amdgcn_sched_barrier(0);
@@ -646,7 +648,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
                 oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, op[(4 * g + dt) & 7]), pb, oacc[dt], 0, 0, 0);
                 request(4 * g + dt + 8, vb, kb);
             }
-            sums = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ones), pb, sums, 0, 0, 0);
+            sums = add_row_sums(praw, sums);
 #pragma unroll
             for (int dt = 0; dt < D / 32; ++dt) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                  // one MFMA
@@ -799,7 +801,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     //      scattered 4-float pieces of its row); they go through this wave's 16 KB of the now idle tile buffers so
     //      that every store instruction writes two whole 512-byte rows.
     if (!live) return;
-    const float l_tot = PING ? l_run : l_run + wave_xor32(l_run);
+    const float l_tot = l_run + wave_xor32(l_run);
     const int qi = i0 + col;
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     int64_t row0 = (((int64_t)split * a.B + b) * a.H + h) * a.Lq + i0;            // row of this wave's first query
