@@ -568,7 +568,6 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     // the queries of the stage this split starts in; a split that crosses from the linear tiles into the pages swaps
     // them for the paged stage's queries at its first page (once per workgroup: that wait also covers the tiles in flight)
     bool q_paged = MODE == kPaged || (TWO && g_t0 >= n_lin);
-    load_q(q_paged ? ap : a);
 
     if constexpr (!PING) {
     // Tiles are handled in pairs: one barrier per two tiles.  While the pair (t, t+1) is multiplied, the next
@@ -709,13 +708,40 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     const bool second = wave >= 4;
     int t = g_t0;                          // the tile at hand, and rows of the pages t, t + 1, t + 2
     int valid0 = kTile, valid1 = kTile, valid2 = kTile;
-    if (t < g_t1) valid0 = load_tile(t, 0);
-    load_q(q_paged ? ap : a);
-    landed();
-    // (as above: the query rows' wait belongs here)
+    // The wave's queries, the first tile and the second are requested at once, and only the second may still be on its way when
+    // the loop begins.  The queries come by way of LDS - the two buffers that the third and fourth tile take -, because a load
+    // into registers is waited for by the compiler, which knows of no other: with everything in flight.  (With the second tile
+    // behind the first one's arrival and queries into registers: operator over 512 x (4,608 + 2,624) keys 101.0 -> 102.2 us,
+    // causal prompt of 8,001 tokens 536 -> 540.  Pages, whose second tile's address is an entry of its own to wait for, gain
+    // nothing by it: prompt of 131,072 25,690 us with, 25,350 without.)
+    const infllm_attn_args &first = q_paged ? ap : a;
+    if (MODE != kPaged && first.q_sl < (int64_t)1 << 26) {
+        const uint32_t at_q = (wave < 4 ? lds_address(Ks) : lds_address(Vs)) + 2 * kTB + (wave & 3) * (kQTile * kRow);
+        const bf16_t *rows = (const bf16_t *)first.d_q + (int64_t)b * first.q_sb + (int64_t)h * first.q_sh + (int64_t)i0 * first.q_sl;
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(qreg[kk]));
-    if (t + 1 < g_t1) valid1 = load_tile(t + 1, kTB);
+        for (int i = 0; i < kQTile * kRow / 1024; ++i) {
+            const int r = kRowsPerLd * i + lane / (D / 8);                              // (rows behind the last: it again, never stored)
+            load_to_lds16(rows, (uint32_t)(min(r, first.Lq - 1 - i0) * (int)first.q_sl + ((lane & (D / 8 - 1)) ^ swz<D>(r)) * 8) * 2, at_q + i * 1024);
+        }
+        if (t < g_t1) valid0 = load_tile(t, 0);
+        whole = false;
+        if (t + 1 < g_t1) valid1 = load_tile(t + 1, kTB);
+        if (whole) all_but_last();
+        else landed();
+        const uint32_t own = at_q + col * kRow + ((grp ^ swz<D>(col)) * 16);
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) {
+            qreg[kk] = __builtin_bit_cast(bf16x8, *(const __attribute__((address_space(3))) u32x4 *)(uintptr_t)(own ^ (kk * 32)));
+            asm volatile("" : "+v"(qreg[kk]));                                          // (read before the barrier)
+        }
+    } else {                               // pages, and rows further apart than a 32-bit offset reaches
+        if (t < g_t1) valid0 = load_tile(t, 0);
+        load_q(first);
+        landed();
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(qreg[kk]));
+        if (t + 1 < g_t1) valid1 = load_tile(t + 1, kTB);
+    }
     half_end();
     if (second) half_end();
     bool have_p = false;                   // the tile before has probabilities that wait for their values
