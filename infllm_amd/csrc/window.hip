@@ -17,7 +17,7 @@ struct RowCopy {
     int64_t s_sb, s_sh, d_sb, d_sh;
     int32_t n;
 };
-constexpr int kCopies = 6;
+constexpr int kCopies = 7;
 constexpr int kCopyRows = 64;                  // rows a copying workgroup moves
 
 struct StageJob {
@@ -31,6 +31,11 @@ struct StageJob {
     bf16_t *q_loc, *q_glb;                     // [B, H, n, D]; q_glb NULL: no sinks
     bf16_t *dk, *dv;                           // where row 0 of head 0 goes, rotated / as it is
     int64_t dk_sb, dk_sh, dv_sb, dv_sh;
+    // A second place for some of the rows (NULL: none): row p is row r = c_first + p of all that the call sees; those with
+    // r < c_head go to row r, those with r >= c_tail to row c_head + r - c_tail.
+    bf16_t *ck, *cv;
+    int64_t ck_sb, ck_sh, cv_sb, cv_sh;
+    int32_t c_first, c_head, c_tail;
     bf16_t *raw;                               // where un-rotated row 0 goes, rows [0, n_raw)
     int64_t raw_sb, raw_sh;
     int32_t n_raw;
@@ -129,18 +134,33 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
         }
     }
     if (j.do_kv) {
+        auto second = [&](int p) {
+            if (!j.ck) return -1;
+            const int r = j.c_first + p;
+            return r < j.c_head ? r : r >= j.c_tail ? j.c_head + r - j.c_tail : -1;
+        };
         if (kp < np) {
             bf16_t *dst = j.dk + (int64_t)b * j.dk_sb + (int64_t)g * j.dk_sh + (int64_t)(p0 + kp) * D;
             const Rot8 r = rotate8(k_lo, k_hi, &cs_pos[kp][kc * 8]);
             *(u32x4 *)(dst + kc * 8) = r.lo;
             *(u32x4 *)(dst + HALF + kc * 8) = r.hi;
+            const int at = second(p0 + kp);
+            if (at >= 0) {
+                dst = j.ck + (int64_t)b * j.ck_sb + (int64_t)g * j.ck_sh + (int64_t)at * D;
+                *(u32x4 *)(dst + kc * 8) = r.lo;
+                *(u32x4 *)(dst + HALF + kc * 8) = r.hi;
+            }
             if (p0 + kp < j.n_raw) {
                 bf16_t *raw = j.raw + (int64_t)b * j.raw_sb + (int64_t)g * j.raw_sh + (int64_t)(p0 + kp) * D;
                 *(u32x4 *)(raw + kc * 8) = k_lo;
                 *(u32x4 *)(raw + HALF + kc * 8) = k_hi;
             }
         }
-        if (vp < np) *(u32x4 *)(j.dv + (int64_t)b * j.dv_sb + (int64_t)g * j.dv_sh + (int64_t)(p0 + vp) * D + vc * 8) = v_row;
+        if (vp < np) {
+            *(u32x4 *)(j.dv + (int64_t)b * j.dv_sb + (int64_t)g * j.dv_sh + (int64_t)(p0 + vp) * D + vc * 8) = v_row;
+            const int at = second(p0 + vp);
+            if (at >= 0) *(u32x4 *)(j.cv + (int64_t)b * j.cv_sb + (int64_t)g * j.cv_sh + (int64_t)at * D + vc * 8) = v_row;
+        }
     }
 }
 
@@ -262,6 +282,19 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         copy(a->d_old_k, a->ok_sb, a->ok_sh, from, bk, bk_sb, bk_sh, a->n_init, tail);
         copy(a->d_old_v, a->ov_sb, a->ov_sh, from, bv, bv_sb, bv_sh, a->n_init, tail);
     }
+    if (all) {
+        // The new cache - all rows, or the sinks and the tail - besides everything: old rows are copied to both places, new ones
+        // written to both.  (Copied out of everything by a launch behind this
+        // one: sinks + window over 16,001 tokens 1,077 us, so 1,063.)
+        const int64_t head = cut ? a->n_init : a->rows_new, tail0 = rows_all - (a->rows_new - head), old_head = std::min<int64_t>(head, a->rows_old);
+        copy(a->d_old_k, a->ok_sb, a->ok_sh, 0, a->d_cache_k, a->ck_sb, a->ck_sh, 0, old_head);
+        copy(a->d_old_v, a->ov_sb, a->ov_sh, 0, a->d_cache_v, a->cv_sb, a->cv_sh, 0, old_head);
+        copy(a->d_old_k, a->ok_sb, a->ok_sh, tail0, a->d_cache_k, a->ck_sb, a->ck_sh, head, a->rows_old - tail0);
+        copy(a->d_old_v, a->ov_sb, a->ov_sh, tail0, a->d_cache_v, a->cv_sb, a->cv_sh, head, a->rows_old - tail0);
+        j.ck = (bf16_t *)a->d_cache_k; j.cv = (bf16_t *)a->d_cache_v;
+        j.ck_sb = a->ck_sb; j.ck_sh = a->ck_sh; j.cv_sb = a->cv_sb; j.cv_sh = a->cv_sh;
+        j.c_first = a->rows_old; j.c_head = (int32_t)head; j.c_tail = (int32_t)tail0;
+    }
     if (j.n_raw > 0 && a->raw_old > 0)
         copy(a->d_raw_old, (int64_t)a->raw_old * D * a->Hkv, (int64_t)a->raw_old * D, 0, a->d_raw, raw_sh * a->Hkv, raw_sh, 0, a->raw_old);
     int rc;
@@ -285,18 +318,6 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         rc = launch_stage_rows(j, D, stream);
         if (rc) return rc;
     }
-    if (all) {                                  // the new cache out of everything: all of it, or the sinks and the tail
-        StageJob c{};
-        c.B = a->B; c.H = a->H; c.Hkv = a->Hkv;
-        const int64_t head = cut ? a->n_init : a->rows_new, tail = a->rows_new - head;
-        c.copy[0] = RowCopy{bk, (bf16_t *)a->d_cache_k, bk_sb, bk_sh, a->ck_sb, a->ck_sh, (int32_t)head};
-        c.copy[1] = RowCopy{bv, (bf16_t *)a->d_cache_v, bv_sb, bv_sh, a->cv_sb, a->cv_sh, (int32_t)head};
-        c.copy[2] = RowCopy{bk + (rows_all - tail) * D, (bf16_t *)a->d_cache_k + head * D, bk_sb, bk_sh, a->ck_sb, a->ck_sh, (int32_t)tail};
-        c.copy[3] = RowCopy{bv + (rows_all - tail) * D, (bf16_t *)a->d_cache_v + head * D, bv_sb, bv_sh, a->cv_sb, a->cv_sh, (int32_t)tail};
-        rc = launch_stage_rows(c, D, stream);
-        if (rc) return rc;
-    }
-
     // ---- attention
     const bf16_t *sk = a->kind == 2 ? (const bf16_t *)a->d_raw : bk;
     const int64_t sk_sh = a->kind == 2 ? raw_sh : bk_sh, sk_sb = a->kind == 2 ? raw_sh * a->Hkv : bk_sb;
