@@ -265,6 +265,12 @@ typedef struct {
     int64_t score_sb, score_sh, score_cap;
 } infllm_score_args;
 int infllm_local_score(const infllm_score_args *a, void *stream);
+/* infllm_attn_merge_pair and the scores of one stage against the joint log-sum-exps in one launch (a->d_lse and n_parts are set
+ * from the partials; heads of 128).  Returns 1, with nothing launched, where that form does not apply: more than 8 partials or
+ * 2048 queries, at most 1024 keys, positions beyond 2^30. */
+int infllm_local_score_merge_pair(const infllm_score_args *a, const uint16_t *d_o_part, const float *d_lse_part, int32_t P1,
+                                  const uint16_t *d_o_part2, const float *d_lse_part2, int32_t P2, void *d_out, int64_t o_sb,
+                                  int64_t o_sh, int64_t o_sl, float *d_lse, void *stream);
 
 /* ---------------------------------------------------------------------------
  * Retrieval: unit scores + top-k.

@@ -189,6 +189,7 @@ SYMBOLS = {
     "infllm_attn_fwd_noalloc": (c_i32, [C.POINTER(AttnArgs), C.POINTER(AttnArgs), c_vp, c_i64, c_i64, c_i64, c_vp, c_vp]),
     "infllm_window_forward": (c_i32, [c_vp, c_vp]),      # infllm_window_args: WindowArgs by reference, or its bytes
     "infllm_local_score": (c_i32, [C.POINTER(ScoreArgs), c_vp]),
+    "infllm_local_score_merge_pair": (c_i32, [C.POINTER(ScoreArgs), c_vp, c_vp, c_i32, c_vp, c_vp, c_i32, c_vp, c_i64, c_i64, c_i64, c_vp, c_vp]),
     "infllm_unit_scores": (c_i32, [c_vp, c_i64, c_i32, c_i32, c_i32, c_vp, c_vp, c_vp]),
     "infllm_topk": (c_i32, [c_vp, c_i32, c_i32, c_vp, c_vp]),
     "infllm_score_topk": (c_i32, [c_vp, c_i64, c_i32, c_i32, c_vp, c_i32, c_vp, c_vp, c_vp]),

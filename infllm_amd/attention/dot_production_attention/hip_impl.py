@@ -72,16 +72,22 @@ class HipMultiStageDotProductionAttention(MultiStageDotProductionAttention):
             self._lse_parts = [self._lse_parts[0], torch.cat(self._lse_parts[1:], dim=0)]
         self.ret = torch.empty((B, H, Lq, D), dtype=torch.bfloat16, device=dev)
         self.lse = torch.empty((B, H, Lq), dtype=torch.float32, device=dev)
-        ops.attn_merge_sets(self._o_parts, self._lse_parts, self.ret, self.lse)
+        scores = [torch.empty((B, H, stage[1].shape[2]), dtype=torch.float32, device=dev) if stage[5] else None for stage in self._stages]   # every cell is written
+        wanted = [i for i, score in enumerate(scores) if score is not None and score.shape[2] > 0]
+        first = wanted[0] if wanted else None                 # the scores that the merge's launch can take along
+        if first is not None:
+            q, k, mask, offset, window, _, scale = self._stages[first]
+            if not ops.merge_sets_and_score(self._o_parts, self._lse_parts, self.ret, self.lse, q, k, scores[first], mask=mask, offset=offset,
+                                            window=window, softmax_scale=scale):
+                first = None
+        if first is None:
+            ops.attn_merge_sets(self._o_parts, self._lse_parts, self.ret, self.lse)
         if d < D:
             self.ret = self.ret[..., :d].contiguous()
-        for q, k, mask, offset, window, want, scale in self._stages:
-            if not want:
-                self.score_list.append(None)
-                continue
-            score = torch.empty((B, H, k.shape[2]), dtype=torch.float32, device=dev)       # every cell is written
-            if k.shape[2] > 0:
-                ops.local_score(q, k, self.lse, score, j_lo=0, j_hi=k.shape[2], mask=mask, offset=offset,
-                                window=window, accumulate=False, softmax_scale=scale)
-            self.score_list.append(score)
+        for i in wanted:
+            if i != first:
+                q, k, mask, offset, window, _, scale = self._stages[i]
+                ops.local_score(q, k, self.lse, scores[i], j_lo=0, j_hi=k.shape[2], mask=mask, offset=offset, window=window, accumulate=False,
+                                softmax_scale=scale)
+        self.score_list.extend(scores)
         self._o_parts, self._lse_parts = [], []

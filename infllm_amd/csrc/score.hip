@@ -25,10 +25,6 @@ constexpr int kQPad = D + 8;               // LDS row of Q (bf16 elements): 272 
 // bounds the short launches that sit on the critical path between two blocks.  QS = queries per LDS stage: a short
 // launch is a chain of stages that each wait for one global load (there is next to no arithmetic to hide it behind),
 // so it takes stages of 128 queries and half as many of them.
-//
-// MERGE: the launch also carries the merge of the block's partial attention outputs, in workgroups behind the scoring ones.
-// The two kinds of work do not depend on each other - the scoring workgroups join the partial log-sum-exps themselves, by
-// the merge's own arithmetic, those of ALL the launch's queries at once in the wait for their keys.
 struct ScoreMerge {
     MergeJob job;
     int32_t score_tiles;               // blockIdx.y below this scores, from there on merges
@@ -49,14 +45,14 @@ __device__ __forceinline__ int tile_of_slot(const infllm_score_args &a, int slot
     return slot;
 }
 
-// One workgroup of 256 threads: tile `slot` (in the order they are dispatched) of n_tiles of the keys, query head bx.  MERGE:
-// the joined log-sum-exps of all the queries go into LDS once, from the partial ones at a.d_lse + lps.
-template <int D, int KS, int QS, bool MERGE>
+// The general form, for partial log-sum-exps in any number and rings or rows that 32 bits do not address (the others:
+// scores_kernel).  One workgroup of 256 threads: tile `slot` (in the order they are dispatched) of n_tiles of the keys, query
+// head bx.
+template <int D, int KS, int QS>
 __device__ __forceinline__ void score_tile(const infllm_score_args &a, const PartSets lps, int bx, int slot, int n_tiles, char *score_lds) {
     constexpr int kWaveKeys = 32 * KS, kKeysPerWg = 4 * kWaveKeys, kQStage = QS;
     bf16_t(*Qs)[kQStage][kQPad<D>] = (bf16_t(*)[kQStage][kQPad<D>])score_lds;                               // [2][QS][kQPad]
     float(*Ls)[kQStage] = (float(*)[kQStage])(score_lds + 2 * kQStage * kQPad<D> * sizeof(bf16_t));      // [2][QS]
-    [[maybe_unused]] float *Lall = (float *)Ls;                                                        // MERGE: [Lq rounded up to QS]
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int col = lane & 31, grp = lane >> 5;
@@ -120,7 +116,7 @@ __device__ __forceinline__ void score_tile(const infllm_score_args &a, const Par
             const int qi = i0 + ld_row + kLdRows * i;
             qbuf[i] = qi < a.Lq ? *(const u32x4 *)(qbase + (int64_t)qi * a.q_sl + ld_chunk * 8) : u32x4{0, 0, 0, 0};
         }
-        if (!MERGE && tid < kQStage) {
+        if (tid < kQStage) {
             if (i0 + tid >= a.Lq) {
                 lbuf = INFINITY;                                                  // +inf => probability 0
             } else if (a.n_parts <= 0) {
@@ -148,34 +144,11 @@ __device__ __forceinline__ void score_tile(const infllm_score_args &a, const Par
     auto store_stage = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < kQStage / kLdRows; ++i) *(u32x4 *)&Qs[buf][ld_row + kLdRows * i][ld_chunk * 8] = qbuf[i];
-        if (!MERGE && tid < kQStage) Ls[buf][tid] = lbuf;
+        if (tid < kQStage) Ls[buf][tid] = lbuf;
     };
 
     float colsum[KS] = {};
     if (st_hi > st_lo) load_stage(st_lo);
-    if constexpr (MERGE) {
-        // joined log-sum-exps of every query of the launch (the per-stage join above for one group of 8 partials)
-        const int64_t rows = (int64_t)a.B * a.H * a.Lq;
-        const int lq_pad = (a.Lq + kQStage - 1) / kQStage * kQStage;
-        for (int i0 = tid; i0 < lq_pad; i0 += 512) {                       // two queries a thread: one trip to memory for 512
-            float l8[2][8];
-#pragma unroll
-            for (int e = 0; e < 2; ++e)
-#pragma unroll
-                for (int p = 0; p < 8; ++p) l8[e][p] = i0 + e * 256 < a.Lq && p < a.n_parts ? lse[lps.l(p, rows) + i0 + e * 256] : -INFINITY;
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                float m8 = -INFINITY, den = 0.f;
-#pragma unroll
-                for (int p = 0; p < 8; ++p) m8 = fmaxf(m8, l8[e][p]);
-                if (m8 != -INFINITY) {
-#pragma unroll
-                    for (int p = 0; p < 8; ++p) den += __builtin_amdgcn_exp2f(l8[e][p] - m8);
-                }
-                if (i0 + e * 256 < lq_pad) Lall[i0 + e * 256] = den > 0.f ? m8 + log2f(den) : INFINITY;              // +inf => probability 0
-            }
-        }
-    }
     if (st_hi > st_lo) {
         store_stage(0);
         if (st_lo + 1 < st_hi) load_stage(st_lo + 1);
@@ -220,7 +193,7 @@ __device__ __forceinline__ void score_tile(const infllm_score_args &a, const Par
 #pragma unroll
                 for (int kk = 0; kk < D / 16; ++kk) qa[kk] = *(const bf16x8 *)(qrow + kk * 16);
 #pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) l4[pb][q4] = *(const f32x4 *)(MERGE ? &Lall[i0 + qs * 32 + 8 * q4 + 4 * grp] : &Ls[cur][qs * 32 + 8 * q4 + 4 * grp]);
+                for (int q4 = 0; q4 < 4; ++q4) l4[pb][q4] = *(const f32x4 *)&Ls[cur][qs * 32 + 8 * q4 + 4 * grp];
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
@@ -280,18 +253,10 @@ __device__ __forceinline__ void score_tile(const infllm_score_args &a, const Par
     }
 }
 
-template <int D, int KS, int QS, bool MERGE = false>
-__global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a, std::conditional_t<MERGE, ScoreMerge, NoScoreMerge> sm) {
+template <int D, int KS, int QS>
+__global__ __launch_bounds__(256, 2) void local_score_kernel(infllm_score_args a) {
     extern __shared__ __attribute__((aligned(16))) char score_lds[];
-    if constexpr (MERGE) {
-        const int slot = blockIdx.y;
-        if (slot >= sm.score_tiles) {
-            merge_piece<D>(sm.job, ((int64_t)(slot - sm.score_tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x);
-            return;
-        }
-        score_tile<D, KS, QS, true>(a, sm.job.ps, blockIdx.x, slot, sm.score_tiles, score_lds);
-    } else
-        score_tile<D, KS, QS, false>(a, PartSets{a.n_parts, 0, 0}, blockIdx.x, blockIdx.y, gridDim.y, score_lds);
+    score_tile<D, KS, QS>(a, PartSets{a.n_parts, 0, 0}, blockIdx.x, blockIdx.y, gridDim.y, score_lds);
 }
 
 // What ends a block, in one launch: the scores of its keys, the merge of its partial outputs, the units that leave the window
@@ -509,17 +474,32 @@ __device__ __forceinline__ void head_of(const infllm_score_args &a, int bx, int 
 
 // The scores of a launch whose log-sum-exps are finished: the form of the kernel that keeps three workgroups on a CU
 // (operator over 512 queries x (4,608 + 2,624) keys 108.4 -> 102.9 us a pass, prompt of 16,001 tokens 2,745 -> 2,723).
-template <int D, int KS>
-__global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void scores_kernel(infllm_score_args a, int slot0, int cap, int first, int beyond) {
+//
+// MERGE: the launch also carries the merge of the partial attention outputs, in workgroups behind the scoring ones, which join the
+// partial log-sum-exps themselves, by the merge's own arithmetic (the operator, whose merge was a launch in front of this one:
+// 101.0 -> 96.8 us).
+template <int D, int KS, bool MERGE>
+__global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void scores_kernel(infllm_score_args a, int slot0, int cap, int first, int beyond,
+                                                                        std::conditional_t<MERGE, ScoreMerge, NoScoreMerge> sm) {
     extern __shared__ __attribute__((aligned(1024))) char score_lds[];
     constexpr int kKeys = 128 * KS;
+    int n_tiles = gridDim.y;
+    PartSets lps{};
+    if constexpr (MERGE) {
+        n_tiles = sm.score_tiles;
+        if ((int)blockIdx.y >= n_tiles) {
+            merge_piece<D>(sm.job, ((int64_t)((int)blockIdx.y - n_tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x);
+            return;
+        }
+        lps = sm.job.ps;
+    }
     int b, h;
     head_of(a, blockIdx.x, b, h);
-    const int tile = tile_of_slot(a, blockIdx.y, gridDim.y);
+    const int tile = tile_of_slot(a, blockIdx.y, n_tiles);
     const int64_t jg = a.j_lo / (32 * KS) * (32 * KS) + (int64_t)tile * kKeys;
     const int lo = (int)max(a.j_lo - jg, (int64_t)0), hi = (int)min(a.j_hi - jg, (int64_t)kKeys);
     float sums[KS];
-    key_sums<D, KS, false>(a, PartSets{}, b, h, jg, slot0 + tile * kKeys, cap, lo, hi, first, beyond, score_lds, sums);
+    key_sums<D, KS, MERGE>(a, lps, b, h, jg, slot0 + tile * kKeys, cap, lo, hi, first, beyond, score_lds, sums);
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -662,10 +642,7 @@ int check_score_args(const infllm_score_args *a) {
 template <int D>
 size_t score_lds_bytes(int qs) { return (size_t)(2 * qs * kQPad<D> * sizeof(bf16_t) + 2 * qs * sizeof(float)); }
 constexpr int kScoreCus = 256;
-constexpr int kMergedMaxLq = 2048;                     // MERGE: 4 bytes of LDS per query of the launch
-template <int D>
-size_t score_lds_bytes_merged(int qs, int lq) { return (size_t)(2 * qs * kQPad<D> * sizeof(bf16_t) + (size_t)((lq + qs - 1) / qs * qs) * sizeof(float)); }
-
+constexpr int kMergedMaxLq = 2048;                     // 4 bytes of LDS per query whose log-sum-exps are joined in the launch
 template <int D>
 int score_lds_setup() {
     static std::atomic<bool> lds_set{false};           // dynamic LDS above 64 KiB must be enabled once per kernel
@@ -675,8 +652,6 @@ int score_lds_setup() {
         if (e == hipSuccess)
             e = hipFuncSetAttribute((const void *)local_score_kernel<D, 2, 128>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)score_lds_bytes<D>(128));
-        for (const void *k : {(const void *)local_score_kernel<D, 2, 128, true>, (const void *)local_score_kernel<D, 1, 128, true>})
-            if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)score_lds_bytes_merged<D>(128, kMergedMaxLq));
         if (e != hipSuccess) return infllm_fail(-2, "local_score: %s", hipGetErrorString(e));
         lds_set.store(true, std::memory_order_release);
     }
@@ -690,36 +665,45 @@ inline bool wide_waves(const infllm_score_args &a) {
     return a.j_hi - a.j_lo > 1024 && (int64_t)a.B * a.H * (((a.j_hi - 1) / 64 - a.j_lo / 64 + 4) / 4) >= 2 * kScoreCus;
 }
 
+// what the forms of score.hip that keep positions in 32 bits take
+constexpr int64_t kMaxRows = 1 << 30;
+inline bool in_reach(const infllm_score_args &a) { return (a.cap < kMaxRows || a.j_hi < kMaxRows) && (int64_t)a.Lq * a.q_sl < kMaxRows; }
+
+// job: the log-sum-exps are to be joined (a.n_parts of them), and its merge goes along
+template <int D, bool MERGE>
+int scores_launch(const infllm_score_args &a, const MergeJob *job, void *stream) {
+    const bool wide = wide_waves(a);
+    const int wave_keys = wide ? 64 : 32, gx = a.B * a.H;
+    const int64_t tiles = (a.j_hi - 1) / wave_keys - a.j_lo / wave_keys + 1, window = std::min(std::max(a.window, -kMaxRows), kMaxRows);
+    const int cap = (int)std::min(a.cap, kMaxRows), slot0 = (int)(a.j_lo % a.cap - a.j_lo % wave_keys);      // (below 0: rows that do not count)
+    const int first = (int)(a.mask == INFLLM_MASK_WINDOW ? 0 : a.mask == INFLLM_MASK_COMPLEMENT ? window : -kMaxRows);
+    const int beyond = (int)(a.mask == INFLLM_MASK_WINDOW ? std::max<int64_t>(window, 0) : kMaxRows);
+    int rows = (int)((tiles + 3) / 4);
+    const auto kern = wide ? scores_kernel<D, 2, MERGE> : scores_kernel<D, 1, MERGE>;
+    if constexpr (MERGE) {
+        const ScoreMerge sm{*job, rows};
+        rows += (int)((((int64_t)job->B * job->H * job->Lq * (D / 8) + 255) / 256 + gx - 1) / gx);
+        INFLLM_REQUIRE(rows <= 65535, "local_score: %d rows of workgroups", rows);
+        hipLaunchKernelGGL(kern, dim3(gx, rows), dim3(256), kQBytes<D> + (size_t)(a.Lq + kQRows - 1) / kQRows * kQRows * sizeof(float), (hipStream_t)stream, a, slot0,
+                           cap, first, beyond, sm);
+    } else
+        hipLaunchKernelGGL(kern, dim3(gx, rows), dim3(256), kQBytes<D> + 3 * kQRows * sizeof(float), (hipStream_t)stream, a, slot0, cap, first, beyond, NoScoreMerge{});
+    INFLLM_CHECK_LAUNCH("local_score");
+    return 0;
+}
+
 template <int D>
 int score_launch(const infllm_score_args *a, void *stream) {
     int rc = check_score_args(a);
     if (rc) return rc;
     if (a->j_hi <= a->j_lo) return 0;
-    constexpr int64_t kMax = 1 << 30;
-    if (a->n_parts <= 0 && (a->cap < kMax || a->j_hi < kMax) && (int64_t)a->Lq * a->q_sl < kMax) {
-        const bool wide = wide_waves(*a);
-        const int wave_keys = wide ? 64 : 32;
-        const int64_t tiles = (a->j_hi - 1) / wave_keys - a->j_lo / wave_keys + 1, window = std::min(std::max(a->window, -kMax), kMax);
-        const int cap = (int)std::min(a->cap, kMax), slot0 = (int)(a->j_lo % a->cap - a->j_lo % wave_keys);      // (below 0: rows that do not count)
-        const int first = (int)(a->mask == INFLLM_MASK_WINDOW ? 0 : a->mask == INFLLM_MASK_COMPLEMENT ? window : -kMax);
-        const int beyond = (int)(a->mask == INFLLM_MASK_WINDOW ? std::max<int64_t>(window, 0) : kMax);
-        const auto kern = wide ? scores_kernel<D, 2> : scores_kernel<D, 1>;
-        hipLaunchKernelGGL(kern, dim3(a->B * a->H, (unsigned)((tiles + 3) / 4)), dim3(256), kQBytes<D> + 3 * kQRows * sizeof(float), (hipStream_t)stream, *a, slot0,
-                           cap, first, beyond);
-        INFLLM_CHECK_LAUNCH("local_score");
-        return 0;
-    }
+    if (a->n_parts <= 0 && in_reach(*a)) return scores_launch<D, false>(*a, nullptr, stream);
     rc = score_lds_setup<D>();
     if (rc) return rc;
-    if (wide_waves(*a)) {
-        const int64_t tiles = (a->j_hi - 1) / 64 - a->j_lo / 64 + 1;
-        hipLaunchKernelGGL((local_score_kernel<D, 2, 128>), dim3(a->B * a->H, (unsigned)((tiles + 3) / 4)), dim3(256), score_lds_bytes<D>(128),
-                           (hipStream_t)stream, *a, NoScoreMerge{});
-    } else {
-        const int64_t tiles = (a->j_hi - 1) / 32 - a->j_lo / 32 + 1;
-        hipLaunchKernelGGL((local_score_kernel<D, 1, 128>), dim3(a->B * a->H, (unsigned)((tiles + 3) / 4)), dim3(256), score_lds_bytes<D>(128),
-                           (hipStream_t)stream, *a, NoScoreMerge{});
-    }
+    const bool wide = wide_waves(*a);
+    const int64_t tiles = wide ? (a->j_hi - 1) / 64 - a->j_lo / 64 + 1 : (a->j_hi - 1) / 32 - a->j_lo / 32 + 1;
+    const auto kern = wide ? local_score_kernel<D, 2, 128> : local_score_kernel<D, 1, 128>;
+    hipLaunchKernelGGL(kern, dim3(a->B * a->H, (unsigned)((tiles + 3) / 4)), dim3(256), score_lds_bytes<D>(128), (hipStream_t)stream, *a);
     INFLLM_CHECK_LAUNCH("local_score");
     return 0;
 }
@@ -732,23 +716,10 @@ int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *s
     infllm_score_args sc = *a;
     sc.d_lse = job->lse_part;
     sc.n_parts = job->P;
-    int rc = check_score_args(&sc);
+    const int rc = check_score_args(&sc);
     if (rc) return rc;
-    if (sc.j_hi - sc.j_lo <= 1024 || sc.Lq > kMergedMaxLq) return 1;
-    rc = score_lds_setup<D>();
-    if (rc) return rc;
-    const bool wide = wide_waves(sc);
-    const int wave_keys = wide ? 64 : 32;
-    const int64_t tiles = (sc.j_hi - 1) / wave_keys - sc.j_lo / wave_keys + 1;
-    const int score_tiles = (int)((tiles + 3) / 4);
-    const int64_t merge_wgs = ((int64_t)job->B * job->H * job->Lq * (D / 8) + 255) / 256;
-    const int gx = sc.B * sc.H;
-    const int merge_slots = (int)((merge_wgs + gx - 1) / gx);
-    const auto kern = wide ? local_score_kernel<D, 2, 128, true> : local_score_kernel<D, 1, 128, true>;
-    hipLaunchKernelGGL(kern, dim3(gx, (unsigned)(score_tiles + merge_slots)), dim3(256), score_lds_bytes_merged<D>(128, sc.Lq), (hipStream_t)stream, sc,
-                       ScoreMerge{*job, score_tiles});
-    INFLLM_CHECK_LAUNCH("local_score_merged");
-    return 0;
+    if (sc.j_hi - sc.j_lo <= 1024 || sc.Lq > kMergedMaxLq || !in_reach(sc)) return 1;
+    return scores_launch<D, true>(sc, job, stream);
 }
 
 }  // namespace
@@ -851,4 +822,16 @@ int infllm_local_score_dim(const infllm_score_args *a, int32_t dim, void *stream
 int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream, int32_t dim) {
     INFLLM_REQUIRE(dim == 128 || dim == 64, "local_score: head_dim %d", dim);
     return dim == 128 ? score_launch_merged<128>(a, job, stream) : score_launch_merged<64>(a, job, stream);
+}
+
+// ... for the operator: scores and the merge over two sets of partials (P1 + P2 <= 8), heads of 128
+int infllm_merge_job(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2, const float *d_lse_part2, int32_t P2, int32_t B,
+                     int32_t H, int32_t Lq, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse, MergeJob *job, int32_t dim);
+extern "C" int infllm_local_score_merge_pair(const infllm_score_args *a, const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2,
+                                             const float *d_lse_part2, int32_t P2, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl, float *d_lse, void *stream) {
+    INFLLM_REQUIRE(a && d_out, "local_score_merge_pair: null pointer");
+    if (P1 + P2 > 8 || a->j_hi <= a->j_lo) return 1;
+    MergeJob job;
+    const int rc = infllm_merge_job(d_o_part, d_lse_part, P1, d_o_part2, d_lse_part2, P2, a->B, a->H, a->Lq, d_out, o_sb, o_sh, o_sl, d_lse, &job, kD);
+    return rc ? rc : score_launch_merged<kD>(a, &job, stream);
 }

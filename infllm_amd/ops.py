@@ -228,9 +228,7 @@ def attn_merge_sets(o_parts, lse_parts, out, lse):
           "infllm_attn_merge_pair")
 
 
-def local_score(q, k, lse, score, *, cap=None, j_lo=0, j_hi=None, mask=MASK_NONE, offset=0, window=0,
-                accumulate=True, score_cap=None, softmax_scale=None):
-    """score[b,h,j % score_cap] (+)= column sums of the stage's final probabilities."""
+def _score_args(q, k, score, cap, j_lo, j_hi, mask, offset, window, accumulate, score_cap, softmax_scale):
     B, H, Lq, D = q.shape
     a = ScoreArgs()
     a.d_q, a.q_sb, a.q_sh, a.q_sl = q.data_ptr(), q.stride(0), q.stride(1), q.stride(2)
@@ -239,11 +237,34 @@ def local_score(q, k, lse, score, *, cap=None, j_lo=0, j_hi=None, mask=MASK_NONE
     a.cap = cap if cap is not None else NO_WRAP
     a.j_lo, a.j_hi = j_lo, (j_hi if j_hi is not None else k.shape[2])
     a.mask, a.accumulate, a.offset, a.window = mask, int(accumulate), offset, window
-    a.d_lse = lse.data_ptr()
     a.softmax_scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(D)
     a.d_score, a.score_sb, a.score_sh = score.data_ptr(), score.stride(0), score.stride(1)
     a.score_cap = score_cap if score_cap is not None else NO_WRAP
+    return a
+
+
+def local_score(q, k, lse, score, *, cap=None, j_lo=0, j_hi=None, mask=MASK_NONE, offset=0, window=0,
+                accumulate=True, score_cap=None, softmax_scale=None):
+    """score[b,h,j % score_cap] (+)= column sums of the stage's final probabilities."""
+    a = _score_args(q, k, score, cap, j_lo, j_hi, mask, offset, window, accumulate, score_cap, softmax_scale)
+    a.d_lse = lse.data_ptr()
     check(_lib.load().infllm_local_score(a, _stream()), "infllm_local_score")
+
+
+def merge_sets_and_score(o_parts, lse_parts, out, lse, q, k, score, *, mask=MASK_NONE, offset=0, window=0, softmax_scale=None):
+    """attn_merge_sets and the (first) scores of one stage against the joint log-sum-exps, in one launch; False, with nothing
+    done, where there is no such launch."""
+    _need(out.stride(-1) == 1 and out.dtype == torch.bfloat16 and 1 <= len(o_parts) <= 2, "bad merge arguments")
+    two = len(o_parts) == 2
+    a = _score_args(q, k, score, None, 0, None, mask, offset, window, False, None, softmax_scale)
+    a.d_lse = lse_parts[0].data_ptr()
+    status = _lib.load().infllm_local_score_merge_pair(a, o_parts[0].data_ptr(), lse_parts[0].data_ptr(), o_parts[0].shape[0],
+                                                       o_parts[1].data_ptr() if two else None, lse_parts[1].data_ptr() if two else None,
+                                                       o_parts[1].shape[0] if two else 0, out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
+                                                       lse.data_ptr(), _stream())
+    if status != 1:
+        check(status, "infllm_local_score_merge_pair")
+    return status == 0
 
 
 def score_topk(reps, n, qbar, k, scores, idx):

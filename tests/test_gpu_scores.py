@@ -53,3 +53,30 @@ def test_scores_of_partly_masked_stages(H, Hkv, keys, Lq, mask):
     assert torch.equal(got[:, :, other], start[:, :, other])
     assert torch.allclose(got[:, :, rows].double(), want + start[:, :, rows].double(), rtol=1e-4, atol=1e-5), float(
         (got[:, :, rows].double() - want - start[:, :, rows].double()).abs().max())
+
+
+@pytest.mark.parametrize("H,Hkv,keys", [(4, 2, 1025), (64, 64, 2100)])
+@pytest.mark.parametrize("Lq,parts", [(1, (1, 0)), (33, (2, 1)), (512, (4, 4)), (2048, (1, 2))])
+@pytest.mark.parametrize("mask", ["none", "window", "complement"])
+def test_scores_with_the_merge_of_the_partials(H, Hkv, keys, Lq, parts, mask):
+    """One launch against the two: rows and log-sum-exps bit for bit, scores up to the order of nothing (the same sums)."""
+    from infllm_amd import ops
+    if H * Lq > 64 * 512:
+        H, Hkv = 4, 2
+    code = dict(none=ops.MASK_NONE, window=ops.MASK_WINDOW, complement=ops.MASK_COMPLEMENT)[mask]
+    where = dict(mask=code, offset=keys - Lq, window=keys - 100)
+    g = torch.Generator().manual_seed(5)
+    q, k = _rand((2, H, Lq, D), 1).cuda(), _rand((2, Hkv, keys, D), 2).cuda()
+    sets = [p for p in parts if p]
+    o_parts = [torch.randn((p, 2, H, Lq, D), generator=g).half().cuda() for p in sets]
+    lse_parts = [(4 + torch.randn((p, 2, H, Lq), generator=g)).cuda() for p in sets]
+    out, lse, score = (torch.empty((2, H, Lq, D), dtype=torch.bfloat16, device="cuda"), torch.empty((2, H, Lq), device="cuda"),
+                       torch.empty((2, H, keys), device="cuda"))
+    assert ops.merge_sets_and_score(o_parts, lse_parts, out, lse, q, k, score, **where)
+    want_out, want_lse, want = torch.empty_like(out), torch.empty_like(lse), torch.empty_like(score)
+    ops.attn_merge_sets(o_parts, lse_parts, want_out, want_lse)
+    ops.local_score(q, k, want_lse, want, accumulate=False, **where)
+    assert torch.equal(out, want_out) and torch.equal(lse, want_lse)
+    assert torch.allclose(score, want, rtol=1e-6, atol=0)
+    small = torch.empty((2, H, 1024), device="cuda")
+    assert not ops.merge_sets_and_score(o_parts, lse_parts, out, lse, q, k[:, :, :1024], small, **where)       # (too few keys)
