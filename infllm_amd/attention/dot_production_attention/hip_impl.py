@@ -72,22 +72,31 @@ class HipMultiStageDotProductionAttention(MultiStageDotProductionAttention):
             self._lse_parts = [self._lse_parts[0], torch.cat(self._lse_parts[1:], dim=0)]
         self.ret = torch.empty((B, H, Lq, D), dtype=torch.bfloat16, device=dev)
         self.lse = torch.empty((B, H, Lq), dtype=torch.float32, device=dev)
-        scores = [torch.empty((B, H, stage[1].shape[2]), dtype=torch.float32, device=dev) if stage[5] else None for stage in self._stages]   # every cell is written
-        wanted = [i for i, score in enumerate(scores) if score is not None and score.shape[2] > 0]
-        first = wanted[0] if wanted else None                 # the scores that the merge's launch can take along
-        if first is not None:
-            q, k, mask, offset, window, _, scale = self._stages[first]
-            if not ops.merge_sets_and_score(self._o_parts, self._lse_parts, self.ret, self.lse, q, k, scores[first], mask=mask, offset=offset,
-                                            window=window, softmax_scale=scale):
-                first = None
-        if first is None:
+        # The merge's launch takes the scores of a stage along where there are enough keys to fill it: what it refuses is not offered
+        # to it (a small pass is bound by this host code).
+        merged, late = None, []
+        if Lq <= 2048 and sum(len(part) for part in self._lse_parts) <= 8:
+            merged = next((i for i, stage in enumerate(self._stages) if stage[5] and stage[1].shape[2] > 1024), None)
+        if merged is None:
             ops.attn_merge_sets(self._o_parts, self._lse_parts, self.ret, self.lse)
+        for i, (q, k, mask, offset, window, want, scale) in enumerate(self._stages):
+            if not want:
+                self.score_list.append(None)
+                continue
+            score = torch.empty((B, H, k.shape[2]), dtype=torch.float32, device=dev)       # every cell is written
+            if i == merged:
+                if ops.merge_sets_and_score(self._o_parts, self._lse_parts, self.ret, self.lse, q, k, score, mask=mask, offset=offset, window=window,
+                                            softmax_scale=scale):
+                    self.score_list.append(score)
+                    continue
+                ops.attn_merge_sets(self._o_parts, self._lse_parts, self.ret, self.lse)
+            self.score_list.append(score)
+            late.append((i, score))
+        for i, score in late:                     # (behind the merge, wherever it was)
+            q, k, mask, offset, window, _, scale = self._stages[i]
+            if k.shape[2] > 0:
+                ops.local_score(q, k, self.lse, score, j_lo=0, j_hi=k.shape[2], mask=mask, offset=offset,
+                                window=window, accumulate=False, softmax_scale=scale)
         if d < D:
             self.ret = self.ret[..., :d].contiguous()
-        for i in wanted:
-            if i != first:
-                q, k, mask, offset, window, _, scale = self._stages[i]
-                ops.local_score(q, k, self.lse, scores[i], j_lo=0, j_hi=k.shape[2], mask=mask, offset=offset, window=window, accumulate=False,
-                                softmax_scale=scale)
-        self.score_list.extend(scores)
         self._o_parts, self._lse_parts = [], []

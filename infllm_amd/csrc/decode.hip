@@ -10,7 +10,8 @@
 //   the softmax runs per lane over those (its own running maximum and sum, no exchange between lanes);
 //   O[head, d] += p[key] * v[key, d] on the vector units in fp32: a row group reads its own four keys' value rows
 //   (16 lanes x 16 bytes), and a head's probability reaches the row's lanes by a DPP row broadcast.
-// The states of all row groups and waves are joined through LDS at the end, the splits by the merge kernels.
+// The states of all row groups and waves are joined through LDS at the end, the splits by the one that ends last, or by a merge
+// or finishing kernel.
 // A logit that is NaN or +infinity makes its query's row NaN, as the softmax has it: a lane that saw nothing but NaN still has
 // its maximum at -infinity, so its sum is taken as it is, and a split whose sum is no number writes NaN rather than zeros.
 // 32,768 keys x 8 kv heads (134 MB): 648 us with the tile kernel of attn.hip at one split, 33 us here.

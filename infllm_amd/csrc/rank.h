@@ -1,5 +1,5 @@
-// A selection and what becomes of it on the device, for units resident in HBM (resident.hip; the local-score launch of
-// score.hip carries it along).
+// A selection and what becomes of it on the device, for units resident in HBM (resident.hip; the launch that ends a block,
+// score.hip, carries it along).
 #pragma once
 #include "common.h"
 

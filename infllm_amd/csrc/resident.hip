@@ -9,9 +9,9 @@
 // in a pinned log.
 //
 // A call of several queries: prologue of all its tokens, mean queries, the k best of the units that exist for every
-// block's mean query (one pass), the local stage of all blocks; then per block the global stage, merge + local score, the
-// units it carves (representatives, rows into their home) and the ranking for the next block.  A single query (a decode
-// step): prologue, retrieval, one streaming attention launch over window, units, sinks and remainder, and one that joins
+// block's mean query (one pass), the local stage of all blocks; then per block the global stage, and one launch for merge, local
+// score, the units it carves (representatives, rows into their home) and the ranking for the next block.  A single query (a decode
+// step): prologue with the retrieval, one streaming attention launch over window, units, sinks and remainder, and one that joins
 // its splits and adds the probabilities to the window's score track - no second read of the window's keys.
 #include <algorithm>
 #include <atomic>
