@@ -234,6 +234,8 @@ typedef struct {
     int64_t work_bytes;
     void *d_out;                            /* bf16 rows [b, h, i] at b*o_sb + h*o_sh + i*o_sl */
     int64_t o_sb, o_sh, o_sl;
+    void *d_ticket;                         /* B * H words that are zero, and zero again when the stream has done the call: with them
+                                             * a step is one launch; NULL: it stages its rows in a launch of their own */
     float softmax_scale;                    /* 1/sqrt(dim) of the model (dim itself may be a wider row) */
     int32_t reserved;
 } infllm_window_args;

@@ -30,8 +30,22 @@ from ..ops import HEAD_DIM, _stream, rows16
 from ._rows import check_head_dim, narrow, wide_inv_freq, widen
 
 _KINDS = {"origin": 0, "stream-llm": 1, "infinite-lm": 2}
-_ARGS = struct.Struct("@3P9q8i2qPd2P4q2P4q2i4P2iPqP3qf4x")        # infllm_window_args
+_ARGS = struct.Struct("@3P9q8i2qPd2P4q2P4q2i4P2iPqP3qPf4x")        # infllm_window_args
 _SPLIT_ROWS = 131072                # partial rows that key splits of a call of several queries may take
+
+_tickets = {}                        # (device index, stream) -> words that every launch on the stream leaves zero
+
+
+def _ticket(dev, stream, n):
+    """The address of n zeros for a step's launch; 0 (the step takes two launches) where they would have to be made inside a
+    capture, whose zeroing runs only when it is replayed."""
+    key = (dev.index, stream)
+    t = _tickets.get(key)
+    if t is None or t.numel() < n:
+        if dev.type == "cuda" and torch.cuda.is_current_stream_capturing():
+            return 0
+        t = _tickets[key] = torch.zeros((max(n, 1024),), dtype=torch.int32, device=dev)
+    return t.data_ptr()
 
 
 class _Room:
@@ -198,7 +212,8 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
                       ov_sh, new_k.data_ptr(), new_v.data_ptr(), nk_sb, nk_sh, nv_sb, nv_sh, rows_old, rows_new,
                       all_kv[0].data_ptr() if all_kv is not None else 0, all_kv[1].data_ptr() if all_kv is not None else 0,
                       raw_old.data_ptr() if raw_old is not None else 0, raw.data_ptr() if raw is not None else 0, raw_rows, raw_new, work.data_ptr(),
-                      work_bytes, out.data_ptr(), len_q * num_heads * dim, dim, num_heads * dim, 1.0 / math.sqrt(dim_head))
+                      work_bytes, out.data_ptr(), len_q * num_heads * dim, dim, num_heads * dim, _ticket(dev, stream, rows_q) if len_q == 1 else 0,
+                      1.0 / math.sqrt(dim_head))
     _lib.check(_lib.load().infllm_window_forward(args, stream), "infllm_window_forward")
     if not native:
         out = narrow(out.view(batch, len_q, num_heads, dim), dim_head).reshape(batch, len_q, num_heads * dim_head)

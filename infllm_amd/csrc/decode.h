@@ -38,5 +38,56 @@ struct DecodeJob {
     uint32_t *ticket;                      // [B * H] zeros, zeros again behind the launch
 };
 
+// rows [0, n) of a source to a destination, for every (batch row, kv head); rows are D elements apart on both sides
+struct RowCopy {
+    const bf16_t *src;
+    bf16_t *dst;
+    int64_t s_sb, s_sh, d_sb, d_sh;
+    int32_t n;
+};
+constexpr int kCopies = 7;
+constexpr int kCopyRows = 64;                  // rows a copying workgroup of 256 threads moves
+
+template <int D>
+__device__ __forceinline__ void copy_rows(const RowCopy (&copies)[kCopies], int piece, int b, int g) {
+    const int tid = threadIdx.x;
+    for (int c = 0; c < kCopies; ++c) {
+        const RowCopy &rc = copies[c];
+        const int n = (rc.n + kCopyRows - 1) / kCopyRows;
+        if (piece >= n) {
+            piece -= n;
+            continue;
+        }
+        const int r0 = piece * kCopyRows, m = min(kCopyRows, rc.n - r0) * (D / 8);
+        const u32x4 *src = (const u32x4 *)(rc.src + (int64_t)b * rc.s_sb + (int64_t)g * rc.s_sh + (int64_t)r0 * D);
+        u32x4 *dst = (u32x4 *)(rc.dst + (int64_t)b * rc.d_sb + (int64_t)g * rc.d_sh + (int64_t)r0 * D);
+        constexpr int U = kCopyRows * (D / 8) / 256;
+        u32x4 x[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+            if (tid + 256 * i < m) x[i] = src[tid + 256 * i];
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+            if (tid + 256 * i < m) dst[tid + 256 * i] = x[i];
+        return;
+    }
+}
+
+// The rows of the step itself, as they come (DecodeJob's ranges are the rows that were there before, its q is not used): the
+// launch rotates the query to its position and to the angle of the sinks, attends the new key, and leaves the key and the value
+// where the cache has them, with the copies of old rows that the cache needs.
+struct StepRows {
+    const bf16_t *q, *k, *v;               // [B, H, D], [B, Hkv, D]
+    int64_t q_sb, q_sh, k_sb, k_sh, v_sb, v_sh;
+    int64_t pos, glb_pos;
+    const float *inv_freq;
+    double distance_scale;
+    bf16_t *dk, *dv, *raw;                 // rotated key, value, key as it is (NULL: nowhere)
+    int64_t dk_sb, dk_sh, dv_sb, dv_sh, raw_sb, raw_sh;
+    RowCopy copy[kCopies];
+    int32_t pieces;                        // copying workgroups per (batch row, kv head)
+};
+
+int infllm_decode_step(const DecodeJob *job, const StepRows *rows, int32_t dim, void *stream);
 int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int64_t blocks, int32_t max_splits);
 int infllm_decode_attn(const DecodeJob *job, int32_t dim, void *stream);

@@ -16,6 +16,7 @@
 // its maximum at -infinity, so its sum is taken as it is, and a split whose sum is no number writes NaN rather than zeros.
 // 32,768 keys x 8 kv heads (134 MB): 648 us with the tile kernel of attn.hip at one split, 33 us here.
 #include "decode.h"
+#include "rope.h"
 
 #include <type_traits>
 
@@ -39,8 +40,39 @@ __device__ __forceinline__ void each_head(F &&f) {
 
 // D: head dimension (128 or 64); NG: query heads handled together (columns of the MFMA; heads beyond the group's last are
 // zero queries whose results are not written)
-template <int D, int NG, bool LOGITS, bool JOIN>
-__global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(DecodeJob j) {
+//
+// FRONT: the step's rows come as they are (StepRows).  Rotating them in a launch in front cost 5 us on a chain of two, and its
+// cache writes, copies included, were waited for by an attention that can read the old cache: here every workgroup rotates its
+// heads' queries while its first rows are on their way, the last split attends the new key, and workgroups behind the splits
+// write the cache (stream-llm, one token over 9,000: 25.4 -> 22.7 us; causal, over 8,192: 26.7 -> 24.0).
+struct NoFront {};
+template <int D>
+__device__ __forceinline__ void leave_rows(const StepRows &f, int b, int g, float2 *cs) {      // 256 threads
+    constexpr int HALF = D / 2, C2 = D / 16;
+    const int tid = threadIdx.x;
+    u32x4 lo{}, hi{}, v{};
+    if (tid < C2) {
+        const bf16_t *src = f.k + (int64_t)b * f.k_sb + (int64_t)g * f.k_sh + tid * 8;
+        lo = *(const u32x4 *)src, hi = *(const u32x4 *)(src + HALF);
+    }
+    if (tid < 2 * C2) v = *(const u32x4 *)(f.v + (int64_t)b * f.v_sb + (int64_t)g * f.v_sh + tid * 8);
+    rope_angles<HALF>(f.pos, 1, f.glb_pos, f.distance_scale, f.inv_freq, (float2(*)[HALF])cs, cs + HALF);
+    __syncthreads();
+    if (tid < C2) {
+        const Rot8 r = rotate8(lo, hi, cs + tid * 8);
+        bf16_t *dst = f.dk + (int64_t)b * f.dk_sb + (int64_t)g * f.dk_sh + tid * 8;
+        *(u32x4 *)dst = r.lo, *(u32x4 *)(dst + HALF) = r.hi;
+        if (f.raw) {
+            dst = f.raw + (int64_t)b * f.raw_sb + (int64_t)g * f.raw_sh + tid * 8;
+            *(u32x4 *)dst = lo, *(u32x4 *)(dst + HALF) = hi;
+        }
+    }
+    if (tid < 2 * C2) *(u32x4 *)(f.dv + (int64_t)b * f.dv_sb + (int64_t)g * f.dv_sh + tid * 8) = v;
+}
+
+template <int D, int NG, bool LOGITS, bool JOIN, bool FRONT = false>
+__global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(DecodeJob j, std::conditional_t<FRONT, StepRows, NoFront> f) {
+    static_assert(!FRONT || JOIN, "a step with its rows joins its splits");
     constexpr int KK = D / 32;                     // k-steps of the first MFMA
     constexpr int LPR = D / 8;                     // lanes that hold a value row, 16 bytes each
     constexpr int VL = kDecodeBlock * LPR / 64;    // value loads per block: 4 (D = 128) or 2 (D = 64)
@@ -53,7 +85,15 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int col = lane & 15, rg = lane >> 4;
     const int G = j.H / j.Hkv, chunks = (G + NG - 1) / NG;
-    const int split = blockIdx.x, g = blockIdx.y / chunks, c = blockIdx.y % chunks, b = blockIdx.z;
+    const int split = blockIdx.x, g = blockIdx.y / chunks, c = blockIdx.y % chunks, b = blockIdx.z, n_split = FRONT ? j.nsplit : (int)gridDim.x;
+    if constexpr (FRONT) {
+        if (split >= n_split) {
+            if (c != 0) return;
+            if (split == n_split) leave_rows<D>(f, b, g, (float2 *)red_room);
+            else copy_rows<D>(f.copy, split - n_split - 1, b, g);
+            return;
+        }
+    }
     const int h0 = g * G + c * NG, nh = min(NG, G - c * NG);
     const float scale = j.scale * 1.4426950408889634f;
     const float lazy = kLazyDec / scale;
@@ -61,7 +101,7 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     // ---- the list of blocks: every range rounded up to whole blocks (units: every unit by itself)
     int n_blocks = 0;
     for (int s = 0; s < j.n_seg; ++s) n_blocks += (j.seg[s].rows + kDecodeBlock - 1) / kDecodeBlock * (j.seg[s].ids ? j.seg[s].n_ids : 1);
-    const int b_lo = (int)((int64_t)n_blocks * split / gridDim.x), b_hi = (int)((int64_t)n_blocks * (split + 1) / gridDim.x);
+    const int b_lo = (int)((int64_t)n_blocks * split / n_split), b_hi = (int)((int64_t)n_blocks * (split + 1) / n_split);
 
     struct Block {
         const bf16_t *k, *v;
@@ -110,8 +150,17 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         }
     };
 
+    __shared__ __attribute__((aligned(16))) bf16_t new_rows[FRONT ? 2 * NG + 1 : 1][FRONT ? D : 8];      // the queries at both angles, the new key
     bf16x8 qreg[KK];
     auto load_q = [&](int which) {
+        if constexpr (FRONT) {
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) {
+                const u32x4 raw = *(const u32x4 *)&new_rows[which * NG + min(col, nh - 1)][rg * 8 + kk * 32];
+                qreg[kk] = __builtin_bit_cast(bf16x8, col < nh ? raw : u32x4{0, 0, 0, 0});
+            }
+            return;
+        }
         const bf16_t *q = j.q[which] + (int64_t)b * j.q_sb + (int64_t)(h0 + min(col, nh - 1)) * j.q_sh + rg * 8;
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
@@ -185,9 +234,36 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     };
 
     int q_now = -1, blk = b_lo + wave;
+    Block cur{};
     if (blk < b_hi) {
-        Block cur = find(blk);
+        cur = find(blk);
         load(cur, 0);
+    }
+    if constexpr (FRONT) {
+        constexpr int HALF = D / 2, C2 = D / 16;
+        float2 *cs = (float2 *)red_room;
+        const int r = threadIdx.x / C2, at = threadIdx.x % C2 * 8;
+        const bool is_q = r < nh, is_k = r == NG;
+        u32x4 lo{}, hi{};
+        if (is_q || is_k) {
+            const bf16_t *src = (is_q ? f.q + (int64_t)b * f.q_sb + (int64_t)(h0 + r) * f.q_sh : f.k + (int64_t)b * f.k_sb + (int64_t)g * f.k_sh) + at;
+            lo = *(const u32x4 *)src, hi = *(const u32x4 *)(src + HALF);
+        }
+        rope_angles<HALF>(f.pos, 1, f.glb_pos, f.distance_scale, f.inv_freq, (float2(*)[HALF])cs, cs + HALF);
+        __syncthreads();
+        if (is_q || is_k) {
+            Rot8 x = rotate8(lo, hi, cs + at);
+            bf16_t *dst = new_rows[is_q ? r : 2 * NG] + at;
+            *(u32x4 *)dst = x.lo, *(u32x4 *)(dst + HALF) = x.hi;
+            if (is_q) {
+                x = rotate8(lo, hi, cs + HALF + at);
+                dst = new_rows[NG + r] + at;
+                *(u32x4 *)dst = x.lo, *(u32x4 *)(dst + HALF) = x.hi;
+            }
+        }
+        __syncthreads();
+    }
+    if (blk < b_hi) {
         load_q(cur.q);
         q_now = cur.q;
         for (int buf = 0; blk < b_hi; blk += 2 * kDecWaves) {        // two blocks per turn, so that the buffers are fixed registers
@@ -206,6 +282,17 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
             }
             if (nxt.q != q_now) load_q(q_now = nxt.q);
             step(nxt, 1);
+        }
+    }
+    if constexpr (FRONT) {
+        if (split == n_split - 1 && wave == kDecWaves - 1) {                   // the new key: a block of one
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) kbuf[0][kk] = *(const u32x4 *)&new_rows[2 * NG][rg * 8 + kk * 32];
+            const bf16_t *row = f.v + (int64_t)b * f.v_sb + (int64_t)g * f.v_sh + (lane & (LPR - 1)) * 8;
+#pragma unroll
+            for (int i = 0; i < VL; ++i) vbuf[0][i] = *(const u32x4 *)row;
+            if (q_now != 0) load_q(0);
+            step(Block{nullptr, nullptr, 1, 0, -1}, 0);
         }
     }
 
@@ -266,7 +353,7 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         __syncthreads();
         int &last = *(int *)&sm[0][0][0];
         uint32_t *ticket = j.ticket + (int64_t)b * gridDim.y + blockIdx.y;
-        if (threadIdx.x == 0) last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        if (threadIdx.x == 0) last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)n_split - 1;
         __syncthreads();
         if (!last) return;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -277,13 +364,13 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         const int64_t step = (int64_t)j.B * j.H, row = (int64_t)b * j.H + h0 + (on ? h : 0);
         float mx = -INFINITY, den = 0.f, o[8] = {};
         constexpr int kBatch = 8;                  // splits whose rows are requested together
-        for (int s0 = wave; s0 < (int)gridDim.x; s0 += kBatch * kDecWaves) {
+        for (int s0 = wave; s0 < n_split; s0 += kBatch * kDecWaves) {
             float l8[kBatch];
             f16x8 o8[kBatch];
 #pragma unroll
             for (int i = 0; i < kBatch; ++i) {
                 const int s = s0 + i * kDecWaves;
-                const bool in = on && s < (int)gridDim.x;
+                const bool in = on && s < n_split;
                 l8[i] = in ? j.lse_part[s * step + row] : -INFINITY;
                 o8[i] = in ? *(const f16x8 *)((const _Float16 *)j.o_part + (s * step + row) * D + at) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
             }
@@ -337,10 +424,21 @@ int launch(const DecodeJob *job, void *stream) {
     const int G = job->H / job->Hkv;
     const int NG = G >= 3 ? 4 : G;
     const dim3 grid(job->nsplit, job->Hkv * ((G + NG - 1) / NG), job->B);
-    if (NG == 1) hipLaunchKernelGGL((decode_attn_kernel<D, 1, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
-    else if (NG == 2) hipLaunchKernelGGL((decode_attn_kernel<D, 2, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
-    else hipLaunchKernelGGL((decode_attn_kernel<D, 4, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job);
+    if (NG == 1) hipLaunchKernelGGL((decode_attn_kernel<D, 1, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, NoFront{});
+    else if (NG == 2) hipLaunchKernelGGL((decode_attn_kernel<D, 2, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, NoFront{});
+    else hipLaunchKernelGGL((decode_attn_kernel<D, 4, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, NoFront{});
     INFLLM_CHECK_LAUNCH("decode_attn");
+    return 0;
+}
+
+template <int D>
+int launch_step(const DecodeJob *job, const StepRows *rows, void *stream) {
+    const int G = job->H / job->Hkv, NG = G >= 3 ? 4 : G;
+    const dim3 grid(job->nsplit + 1 + rows->pieces, job->Hkv * ((G + NG - 1) / NG), job->B);
+    const auto kern = NG == 1 ? decode_attn_kernel<D, 1, false, true, true> : NG == 2 ? decode_attn_kernel<D, 2, false, true, true>
+                                                                                  : decode_attn_kernel<D, 4, false, true, true>;
+    hipLaunchKernelGGL(kern, grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, *rows);
+    INFLLM_CHECK_LAUNCH("decode_step");
     return 0;
 }
 
@@ -357,11 +455,11 @@ int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int64_t blocks, int3
     return s < 1 ? 1 : (int)s;
 }
 
-int infllm_decode_attn(const DecodeJob *job, int32_t dim, void *stream) {
-    INFLLM_REQUIRE(job && job->q[0] && job->q[1] && job->o_part && job->lse_part, "decode_attn: null pointer");
+static int check_job(const DecodeJob *job, int32_t dim) {
+    INFLLM_REQUIRE(job && job->o_part && job->lse_part, "decode_attn: null pointer");
     INFLLM_REQUIRE(job->B > 0 && job->H > 0 && job->Hkv > 0 && job->H % job->Hkv == 0 && job->B <= 65535, "decode_attn: bad geometry B=%d H=%d Hkv=%d", job->B,
                    job->H, job->Hkv);
-    INFLLM_REQUIRE(job->n_seg >= 1 && job->n_seg <= kDecodeSegs && job->nsplit >= 1 && job->nsplit <= 128, "decode_attn: %d ranges, %d splits", job->n_seg,
+    INFLLM_REQUIRE(job->n_seg >= 0 && job->n_seg <= kDecodeSegs && job->nsplit >= 1 && job->nsplit <= 128, "decode_attn: %d ranges, %d splits", job->n_seg,
                    job->nsplit);
     for (int s = 0; s < job->n_seg; ++s) {
         const DecodeSeg &sg = job->seg[s];
@@ -370,6 +468,22 @@ int infllm_decode_attn(const DecodeJob *job, int32_t dim, void *stream) {
         else INFLLM_REQUIRE(sg.rows == 0 || (sg.k && sg.v), "decode_attn: null range");
     }
     INFLLM_REQUIRE(dim == 128 || dim == 64, "decode_attn: head_dim %d", dim);
+    return 0;
+}
+
+// rows: the step's own (their strides multiples of 8 elements); job->out and job->ticket are set, the ranges are plain ones
+int infllm_decode_step(const DecodeJob *job, const StepRows *rows, int32_t dim, void *stream) {
+    const int rc = check_job(job, dim);
+    if (rc) return rc;
+    INFLLM_REQUIRE(rows && rows->q && rows->k && rows->v && rows->inv_freq && rows->dk && rows->dv && rows->pieces >= 0, "decode_step: null pointer");
+    INFLLM_REQUIRE(job->out && job->ticket && !job->logits && ((job->out_sb | job->out_sh) & 7) == 0, "decode_step: bad output");
+    return dim == 128 ? launch_step<128>(job, rows, stream) : launch_step<64>(job, rows, stream);
+}
+
+int infllm_decode_attn(const DecodeJob *job, int32_t dim, void *stream) {
+    const int rc = check_job(job, dim);
+    if (rc) return rc;
+    INFLLM_REQUIRE(job->q[0] && job->q[1] && job->n_seg >= 1, "decode_attn: no query or range");
     INFLLM_REQUIRE(!job->out || (!job->logits && job->ticket && ((job->out_sb | job->out_sh) & 7) == 0), "decode_attn: bad output");
     if (job->logits) return dim == 128 ? launch<128, true, false>(job, stream) : launch<64, true, false>(job, stream);
     if (job->out) return dim == 128 ? launch<128, false, true>(job, stream) : launch<64, false, true>(job, stream);

@@ -1,6 +1,6 @@
 // One call of an attention type with a plain cache - attention sinks + sliding window (inf_llm/attention/stream_llm.py:6-111,
 // infinite_lm.py:6-100) or causal attention (origin.py:4-79) - in two or three launches: the new tokens' rows (rotary
-// embedding, cache), the attention, and the merge of its key splits where several queries have any.
+// embedding, cache), the attention, and the merge of its key splits where several queries have any.  A step is one launch.
 #include <algorithm>
 
 #include "decode.h"
@@ -9,16 +9,6 @@
 int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, int32_t dim, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
                        void *stream);
 namespace {
-
-// rows [0, n) of a source to a destination, for every (batch row, kv head); rows are D elements apart on both sides
-struct RowCopy {
-    const bf16_t *src;
-    bf16_t *dst;
-    int64_t s_sb, s_sh, d_sb, d_sh;
-    int32_t n;
-};
-constexpr int kCopies = 7;
-constexpr int kCopyRows = 64;                  // rows a copying workgroup moves
 
 struct StageJob {
     const bf16_t *q, *k, *v;                   // new rows
@@ -56,27 +46,7 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
     __shared__ float2 cs_glb[HALF];
     const int tid = threadIdx.x, b = blockIdx.y, g = blockIdx.z;
     if ((int)blockIdx.x >= j.tiles) {
-        int piece = (int)blockIdx.x - j.tiles;
-        for (int c = 0; c < kCopies; ++c) {
-            const RowCopy &rc = j.copy[c];
-            const int n = (rc.n + kCopyRows - 1) / kCopyRows;
-            if (piece >= n) {
-                piece -= n;
-                continue;
-            }
-            const int r0 = piece * kCopyRows, m = min(kCopyRows, rc.n - r0) * (D / 8);
-            const u32x4 *src = (const u32x4 *)(rc.src + (int64_t)b * rc.s_sb + (int64_t)g * rc.s_sh + (int64_t)r0 * D);
-            u32x4 *dst = (u32x4 *)(rc.dst + (int64_t)b * rc.d_sb + (int64_t)g * rc.d_sh + (int64_t)r0 * D);
-            constexpr int U = kCopyRows * (D / 8) / 256;
-            u32x4 x[U];
-#pragma unroll
-            for (int i = 0; i < U; ++i)
-                if (tid + 256 * i < m) x[i] = src[tid + 256 * i];
-#pragma unroll
-            for (int i = 0; i < U; ++i)
-                if (tid + 256 * i < m) dst[tid + 256 * i] = x[i];
-            return;
-        }
+        copy_rows<D>(j.copy, (int)blockIdx.x - j.tiles, b, g);
         return;
     }
     if (blockIdx.x == 0 && b == 0 && g == 0)
@@ -297,6 +267,44 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     }
     if (j.n_raw > 0 && a->raw_old > 0)
         copy(a->d_raw_old, (int64_t)a->raw_old * D * a->Hkv, (int64_t)a->raw_old * D, 0, a->d_raw, raw_sh * a->Hkv, raw_sh, 0, a->raw_old);
+    // ---- A step whose old rows hold all it sees but its own key is one launch.  Not where nothing is copied and the rows are so many
+    //      that their stream is what the step costs: every workgroup's rotation holds its stream up for 2 us then, which a launch in
+    //      front spends on one.  Causal steps of 8 key heads of 128 over 500 / 8,192 / 16,384 / 24,000 / 32,768 tokens: one launch
+    //      24.2 / 24.0 / 24.6 / 30.3 / 38.0 us, two 27.3 / 26.7 / 26.3 / 30.2 / 36.0.
+    const int64_t near_rows = causal ? rows_base : std::min<int64_t>(rows_base, a->n_local);       // of the new cache, the last of them the new one
+    const int64_t far_rows = std::max<int64_t>(0, std::min<int64_t>(n_sink, len_k - a->n_local));  // sink j is seen from a distance of at least n_local
+    const void *raw_from = a->raw_new > a->raw_old ? a->d_raw_old : a->d_raw;
+    const int64_t raw_from_sh = (int64_t)(a->raw_new > a->raw_old ? a->raw_old : a->raw_new) * D;
+    const bool streams = nc == 0 && (int64_t)a->B * a->Hkv * (near_rows + far_rows) * D * 4 > (int64_t)96 << 20;
+    if (step && !streams && a->n_new == 1 && !all && a->d_ticket && near_rows >= 1 && near_rows - 1 <= a->rows_old && far_rows <= a->rows_old &&
+        (far_rows == 0 || a->kind != 2 || (raw_from && far_rows * D <= raw_from_sh))) {
+        DecodeJob d{};
+        d.B = a->B; d.H = a->H; d.Hkv = a->Hkv;
+        d.scale = a->softmax_scale;
+        const bf16_t *ok = (const bf16_t *)a->d_old_k, *ov = (const bf16_t *)a->d_old_v;
+        const int64_t near_old = near_rows - 1, from = a->rows_old - near_old;
+        if (near_old > 0) d.seg[d.n_seg++] = DecodeSeg{ok + from * D, ov + from * D, a->ok_sb, a->ok_sh, a->ov_sb, a->ov_sh, (int32_t)near_old, 0, 0, nullptr, -1};
+        if (far_rows > 0)
+            d.seg[d.n_seg++] = a->kind == 2 ? DecodeSeg{(const bf16_t *)raw_from, ov, raw_from_sh * a->Hkv, raw_from_sh, a->ov_sb, a->ov_sh, (int32_t)far_rows, 1, 0, nullptr, -1}
+                                            : DecodeSeg{ok, ov, a->ok_sb, a->ok_sh, a->ov_sb, a->ov_sh, (int32_t)far_rows, 1, 0, nullptr, -1};
+        d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, (near_old + kDecodeBlock - 1) / kDecodeBlock + (far_rows + kDecodeBlock - 1) / kDecodeBlock, max_parts);
+        d.o_part = (uint16_t *)((char *)a->d_work + q_bytes);
+        d.lse_part = (float *)((char *)a->d_work + q_bytes + part_rows * 2 * D);
+        d.out = (bf16_t *)a->d_out; d.out_sb = a->o_sb; d.out_sh = a->o_sh;
+        d.ticket = (uint32_t *)a->d_ticket;
+        StepRows f{};
+        f.q = j.q; f.k = j.k; f.v = j.v;
+        f.q_sb = a->q_sb; f.q_sh = a->q_sh; f.k_sb = a->k_sb; f.k_sh = a->k_sh; f.v_sb = a->v_sb; f.v_sh = a->v_sh;
+        f.pos = a->seen; f.glb_pos = j.glb_pos;
+        f.inv_freq = a->d_inv_freq; f.distance_scale = a->distance_scale;
+        f.dk = j.dk; f.dv = j.dv; f.dk_sb = j.dk_sb; f.dk_sh = j.dk_sh; f.dv_sb = j.dv_sb; f.dv_sh = j.dv_sh;
+        if (j.n_raw > 0) f.raw = j.raw, f.raw_sb = j.raw_sb, f.raw_sh = j.raw_sh;
+        for (int i = 0; i < kCopies; ++i) {
+            f.copy[i] = j.copy[i];
+            f.pieces += (j.copy[i].n + kCopyRows - 1) / kCopyRows;
+        }
+        return infllm_decode_step(&d, &f, D, stream);
+    }
     int rc;
     if (a->n_q == a->n_new) {
         j.do_q = j.do_kv = 1;
@@ -328,11 +336,10 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         d.q_sb = (int64_t)a->H * D; d.q_sh = D;
         d.B = a->B; d.H = a->H; d.Hkv = a->Hkv;
         d.scale = scale;
-        const int64_t near = causal ? rows_base : std::min<int64_t>(rows_base, a->n_local);       // the last rows
+        const int64_t near = near_rows;                                                              // the last rows
         d.seg[0] = DecodeSeg{bk + (rows_base - near) * D, bv + (rows_base - near) * D, bk_sb, bk_sh, bv_sb, bv_sh, (int32_t)near, 0, 0, nullptr, -1};
         d.n_seg = 1;
-        // sink j is seen from a distance of at least n_local: j <= position - n_local
-        const int64_t far = std::min<int64_t>(n_sink, len_k - a->n_local);
+        const int64_t far = far_rows;
         if (far > 0) d.seg[d.n_seg++] = DecodeSeg{sk, bv, sk_sb, sk_sh, bv_sb, bv_sh, (int32_t)far, 1, 0, nullptr, -1};
         const int64_t blocks = (near + kDecodeBlock - 1) / kDecodeBlock + (far > 0 ? (far + kDecodeBlock - 1) / kDecodeBlock : 0);
         d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, blocks, max_parts);
