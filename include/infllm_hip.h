@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define INFLLM_ABI_VERSION 1
+#define INFLLM_ABI_VERSION 2
 #define INFLLM_HEAD_DIM 128
 #define INFLLM_KEY_TILE 64
 
