@@ -235,7 +235,8 @@ typedef struct {
     void *d_out;                            /* bf16 rows [b, h, i] at b*o_sb + h*o_sh + i*o_sl */
     int64_t o_sb, o_sh, o_sl;
     void *d_ticket;                         /* B * H words that are zero, and zero again when the stream has done the call: with them
-                                             * a step is one launch; NULL: it stages its rows in a launch of their own */
+                                             * a step is one launch; NULL: it stages its rows in a launch of their own.  No other launch
+                                             * may use them meanwhile: a step that a graph captures gets words of that graph, or none */
     float softmax_scale;                    /* 1/sqrt(dim) of the model (dim itself may be a wider row) */
     int32_t reserved;
 } infllm_window_args;

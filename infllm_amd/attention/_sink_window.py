@@ -36,14 +36,18 @@ _SPLIT_ROWS = 131072                # partial rows that key splits of a call of 
 _tickets = {}                        # (device index, stream) -> words that every launch on the stream leaves zero
 
 
+def _capturing(dev):
+    return dev.type == "cuda" and torch.cuda.is_current_stream_capturing()
+
+
 def _ticket(dev, stream, n):
-    """The address of n zeros for a step's launch; 0 (the step takes two launches) where they would have to be made inside a
-    capture, whose zeroing runs only when it is replayed."""
+    """The address of n zeros for a step's launch; 0 inside a capture, whose launches run when and where the graph is replayed,
+    beside whatever else counts in the words then: the step takes two launches, the first of which clears words of its own."""
+    if _capturing(dev):
+        return 0
     key = (dev.index, stream)
     t = _tickets.get(key)
     if t is None or t.numel() < n:
-        if dev.type == "cuda" and torch.cuda.is_current_stream_capturing():
-            return 0
         t = _tickets[key] = torch.zeros((max(n, 1024),), dtype=torch.int32, device=dev)
     return t.data_ptr()
 

@@ -137,6 +137,25 @@ def test_which_calls_write_behind_the_cache_they_are_given(native):
     assert where(same) == where(beyond)
 
 
+def tickets(native):
+    names = [n for n, _ in _sink_window._lib.WindowArgs._fields_]
+    return [args[names.index("d_ticket")] for args, _ in native.calls]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_captured_step_keeps_no_address_of_shared_words(kind, native, monkeypatch):
+    """A graph may be replayed beside another that was captured on the same stream, beside eager steps, and long after: its steps
+    count in words of their own scratch, also where a warm-up has made words already."""
+    _, past = layer(kind, None, 30)
+    _, past = layer(kind, past, 1)
+    assert tickets(native)[-1] != 0
+    monkeypatch.setattr(_sink_window, "_capturing", lambda dev: True, raising=False)
+    _, past = layer(kind, past, 1)
+    assert tickets(native)[-1] == 0
+    layer(kind, past, 1)
+    assert tickets(native)[-1] == 0
+
+
 def misaligned(*shape):
     """contiguous, but two bytes off"""
     n = 1
