@@ -238,7 +238,7 @@ typedef struct {
                                              * a step is one launch; NULL: it stages its rows in a launch of their own.  No other launch
                                              * may use them meanwhile: a step that a graph captures gets words of that graph, or none */
     float softmax_scale;                    /* 1/sqrt(dim) of the model (dim itself may be a wider row) */
-    int32_t reserved;
+    int32_t ticket_fresh;                   /* 1: d_ticket's words hold anything; the call sets them to zero (a step in its two launches) */
 } infllm_window_args;
 int infllm_window_forward(const infllm_window_args *a, void *stream);
 

@@ -74,7 +74,7 @@ class WindowArgs(C.Structure):
         ("rows_old", c_i32), ("rows_new", c_i32),
         ("d_all_k", c_vp), ("d_all_v", c_vp), ("d_raw_old", c_vp), ("d_raw", c_vp), ("raw_old", c_i32), ("raw_new", c_i32),
         ("d_work", c_vp), ("work_bytes", c_i64), ("d_out", c_vp), ("o_sb", c_i64), ("o_sh", c_i64), ("o_sl", c_i64),
-        ("d_ticket", c_vp), ("softmax_scale", c_f32), ("reserved", c_i32),
+        ("d_ticket", c_vp), ("softmax_scale", c_f32), ("ticket_fresh", c_i32),
     ]
 
 

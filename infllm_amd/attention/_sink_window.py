@@ -30,26 +30,34 @@ from ..ops import HEAD_DIM, _stream, rows16
 from ._rows import check_head_dim, narrow, wide_inv_freq, widen
 
 _KINDS = {"origin": 0, "stream-llm": 1, "infinite-lm": 2}
-_ARGS = struct.Struct("@3P9q8i2qPd2P4q2P4q2i4P2iPqP3qPf4x")        # infllm_window_args
+_ARGS = struct.Struct("@3P9q8i2qPd2P4q2P4q2i4P2iPqP3qPfi")        # infllm_window_args
 _SPLIT_ROWS = 131072                # partial rows that key splits of a call of several queries may take
-
-_tickets = {}                        # (device index, stream) -> words that every launch on the stream leaves zero
-
 
 def _capturing(dev):
     return dev.type == "cuda" and torch.cuda.is_current_stream_capturing()
 
 
-def _ticket(dev, stream, n):
-    """The address of n zeros for a step's launch; 0 inside a capture, whose launches run when and where the graph is replayed,
-    beside whatever else counts in the words then: the step takes two launches, the first of which clears words of its own."""
-    if _capturing(dev):
-        return 0
-    key = (dev.index, stream)
-    t = _tickets.get(key)
-    if t is None or t.numel() < n:
-        t = _tickets[key] = torch.zeros((max(n, 1024),), dtype=torch.int32, device=dev)
-    return t.data_ptr()
+def _take_words(past_k, n, dev, stream):
+    """(n words or more in which a step counts its finished key splits, their address, their number, the stream they belong to) and
+    whether the call has to clear them, or None: it counts in words of its own scratch.
+
+    The words are zero between the launches that use them, and only one call has them at a time: it takes them off the storage of
+    the cache it continues (one operation, whichever threads go on from that cache) and leaves them with the cache it returns.
+    Their launches are then in the order of their stream, which is also the one that the allocator gives them out again in.
+    Inside a capture there are none: its launches run when and where the graph is replayed, beside whatever else counts by then
+    (and the default stream, 0, cannot be captured)."""
+    if stream and _capturing(dev):
+        return None, 0
+    if past_k is not None:
+        held = past_k.untyped_storage().__dict__.pop("_infllm_words", None)
+        if held is not None and held[3] == stream and held[2] >= n:
+            return held, 0
+    t = torch.empty((n,), dtype=torch.int32, device=dev)
+    return (t, t.data_ptr(), n, stream), 1
+
+
+def _ticket(words):
+    return words[1] if words is not None else 0
 
 
 class _Room:
@@ -198,6 +206,7 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
             _Room(both, rows_all, stream)
             new_k, new_v = both.narrow(3, 0, rows_all).unbind(0)
 
+    words, fresh = _take_words(old_k, batch * num_heads, dev, stream)
     rows_q = batch * num_heads * len_q
     q_bytes = (2 if kind else 1) * rows_q * dim * 2
     part_rows = 64 * rows_q if rows_q <= 2048 else _SPLIT_ROWS if 2 * rows_q <= _SPLIT_ROWS else 0
@@ -210,19 +219,21 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
         cached_k, ok_sb, ok_sh = _cache_rows(cached_k, dim)
         cached_v, ov_sb, ov_sh = _cache_rows(cached_v, dim)
         okp, ovp = cached_k.data_ptr(), cached_v.data_ptr()
-    (nk_sb, nk_sh, _, _), (nv_sb, nv_sh, _, _) = new_k.stride(), new_v.stride()
+    n_sb, n_sh, _, _ = new_k.stride()                          # (and new_v's: halves of one buffer)
     args = _ARGS.pack(q.data_ptr(), k.data_ptr(), v.data_ptr(), q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl, batch, num_heads, num_heads_kv, dim,
                       len_q, n_new, kind, n_init, n_local, seen, inv_freq.data_ptr(), float(position_bias.distance_scale), okp, ovp, ok_sb, ok_sh, ov_sb,
-                      ov_sh, new_k.data_ptr(), new_v.data_ptr(), nk_sb, nk_sh, nv_sb, nv_sh, rows_old, rows_new,
+                      ov_sh, new_k.data_ptr(), new_v.data_ptr(), n_sb, n_sh, n_sb, n_sh, rows_old, rows_new,
                       all_kv[0].data_ptr() if all_kv is not None else 0, all_kv[1].data_ptr() if all_kv is not None else 0,
                       raw_old.data_ptr() if raw_old is not None else 0, raw.data_ptr() if raw is not None else 0, raw_rows, raw_new, work.data_ptr(),
-                      work_bytes, out.data_ptr(), len_q * num_heads * dim, dim, num_heads * dim, _ticket(dev, stream, rows_q) if len_q == 1 else 0,
-                      1.0 / math.sqrt(dim_head))
+                      work_bytes, out.data_ptr(), len_q * num_heads * dim, dim, num_heads * dim, _ticket(words),
+                      1.0 / math.sqrt(dim_head), fresh)
     _lib.check(_lib.load().infllm_window_forward(args, stream), "infllm_window_forward")
     if not native:
         out = narrow(out.view(batch, len_q, num_heads, dim), dim_head).reshape(batch, len_q, num_heads * dim_head)
         new_k, new_v = narrow(new_k, dim_head), narrow(new_v, dim_head)
         raw = None if raw is None else narrow(raw, dim_head)
+    if words is not None:
+        new_k.untyped_storage()._infllm_words = words
     return out, (new_k, new_v, len_k, raw)
 
 

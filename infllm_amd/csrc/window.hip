@@ -30,7 +30,7 @@ struct StageJob {
     int64_t raw_sb, raw_sh;
     int32_t n_raw;
     int32_t tiles;                             // workgroups along x that stage rows; the rest copy
-    uint32_t *clear;                           // n_clear words to set to zero (the decode kernel's tickets)
+    uint32_t *clear;                           // n_clear words to set to zero (tickets: of the decode kernel, or of steps to come)
     int32_t n_clear;
     RowCopy copy[kCopies];
 };
@@ -206,7 +206,8 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     const int64_t part_rows = std::max<int64_t>(0, a->work_bytes - q_bytes - (a->n_q == 1 ? 4 * rows_q : 0)) / (2 * D + 4);
     const int max_parts = (int)std::min<int64_t>(part_rows / rows_q, 64);
     const bool step = a->n_q == 1 && max_parts >= 1;
-    uint32_t *ticket = (uint32_t *)((char *)a->d_work + q_bytes + part_rows * (2 * D + 4));
+    const bool fresh = a->d_ticket && a->ticket_fresh != 0;
+    uint32_t *ticket = fresh ? (uint32_t *)a->d_ticket : (uint32_t *)((char *)a->d_work + q_bytes + part_rows * (2 * D + 4));
     INFLLM_REQUIRE(a->work_bytes >= q_bytes, "window_forward: scratch of %lld bytes for %lld", (long long)a->work_bytes, (long long)q_bytes);
     bf16_t *q_loc = (bf16_t *)a->d_work, *q_sink = causal ? nullptr : q_loc + q_elems;
 
@@ -235,7 +236,7 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         j.raw_sh = raw_sh; j.raw_sb = raw_sh * a->Hkv;
         j.n_raw = a->raw_new - a->raw_old;
     }
-    if (step) j.clear = ticket, j.n_clear = (int32_t)rows_q;
+    if (step || fresh) j.clear = ticket, j.n_clear = a->B * a->H;
     int nc = 0;
     auto copy = [&](const void *src, int64_t ss_b, int64_t ss_h, int64_t s_row, void *dst, int64_t ds_b, int64_t ds_h, int64_t d_row, int64_t n) {
         if (n > 0) j.copy[nc++] = RowCopy{(const bf16_t *)src + s_row * D, (bf16_t *)dst + d_row * D, ss_b, ss_h, ds_b, ds_h, (int32_t)n};
@@ -276,7 +277,7 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     const void *raw_from = a->raw_new > a->raw_old ? a->d_raw_old : a->d_raw;
     const int64_t raw_from_sh = (int64_t)(a->raw_new > a->raw_old ? a->raw_old : a->raw_new) * D;
     const bool streams = nc == 0 && (int64_t)a->B * a->Hkv * (near_rows + far_rows) * D * 4 > (int64_t)96 << 20;
-    if (step && !streams && a->n_new == 1 && !all && a->d_ticket && near_rows >= 1 && near_rows - 1 <= a->rows_old && far_rows <= a->rows_old &&
+    if (step && !streams && a->n_new == 1 && !all && a->d_ticket && !fresh && near_rows >= 1 && near_rows - 1 <= a->rows_old && far_rows <= a->rows_old &&
         (far_rows == 0 || a->kind != 2 || (raw_from && far_rows * D <= raw_from_sh))) {
         DecodeJob d{};
         d.B = a->B; d.H = a->H; d.Hkv = a->Hkv;

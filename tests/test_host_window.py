@@ -1,5 +1,8 @@
 """CPU-only checks of the sliding-window and causal attention types' host side: what reaches the native call, with a stand-in
 for the library that records it."""
+import threading
+import weakref
+
 import pytest
 import torch
 
@@ -154,6 +157,80 @@ def test_a_captured_step_keeps_no_address_of_shared_words(kind, native, monkeypa
     assert tickets(native)[-1] == 0
     layer(kind, past, 1)
     assert tickets(native)[-1] == 0
+
+
+class Words:
+    """remembers which tensors of 32-bit words torch.zeros and torch.empty have made, and whether they are still there"""
+
+    def __init__(self, monkeypatch, before=lambda: None):
+        self.made = []
+
+        def remembering(make):
+            def call(shape, **kw):
+                if kw.get("dtype") is not torch.int32:
+                    return make(shape, **kw)
+                before()
+                t = make(shape, **kw)
+                self.made.append((t.data_ptr(), t.numel() * 4, weakref.ref(t)))
+                return t
+            return call
+        for name in ("zeros", "empty"):
+            monkeypatch.setattr(torch, name, remembering(getattr(torch, name)))
+
+    def owner(self, address, words):
+        """the tensor that is alive and holds the words at that address"""
+        return [r for at, size, r in self.made if r() is not None and at <= address and address + 4 * words <= at + size]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_two_threads_steps_count_in_words_that_stay(kind, native, monkeypatch):
+    """Both make words at once, for one stream: whichever are kept, the kernels got addresses of memory that is not given away."""
+    meet = threading.Barrier(2)
+    words = Words(monkeypatch, lambda: meet.wait(timeout=20))
+    caches = [None, None]
+
+    def step(i):
+        caches[i] = layer(kind, None, 1)[1]
+    threads = [threading.Thread(target=step, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(native.calls) == 2 and all(caches)
+    for address in tickets(native):
+        assert words.owner(address, B * H)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_words_of_a_cache_are_used_by_one_call_at_a_time(kind, native, monkeypatch):
+    """A second continuation of a prompt, which another thread or another stream may make, has words of its own; so has a larger
+    batch; and none are replaced while a launch may count in them.  Words that hold anything yet are said to."""
+    words = Words(monkeypatch)
+    _, prompt = layer(kind, None, 70)
+    inside = {}
+    launch = native.infllm_window_forward
+
+    def meanwhile(args, stream):                              # a step within the step: as two threads do it
+        status = launch(args, stream)
+        if not inside:
+            inside["cache"] = None
+            inside["cache"] = layer(kind, prompt, 1)[1]
+        return status
+    monkeypatch.setattr(native, "infllm_window_forward", meanwhile)
+    _, one = layer(kind, prompt, 1)
+    first, second = tickets(native)[-2:]
+    assert first and second and first != second
+    assert words.owner(first, B * H) and words.owner(second, B * H)
+    _, one = layer(kind, one, 1)
+    assert tickets(native)[-1] in (first, second)             # (a cache's steps go on with its words)
+    _, large = layer(kind, None, 1, batch=400)
+    assert words.owner(tickets(native)[-1], 400 * H) and tickets(native)[-1] not in (first, second)
+    assert words.owner(first, B * H) or words.owner(second, B * H)
+    monkeypatch.setattr(_sink_window, "_stream", lambda: 8)
+    _, other = layer(kind, one, 1)
+    assert tickets(native)[-1] not in (0, first, second)      # (two streams' launches have no order)
+    layer(kind, other, 1)
+    assert [args[-1] for args, _ in native.calls] == [1, 0, 1, 0, 1, 1, 0]
 
 
 def misaligned(*shape):
