@@ -128,7 +128,7 @@ typedef struct {
     int32_t B, H, Hkv, Lq;
     /* linear source (d_pages == NULL) */
     const void *d_k, *d_v;
-    int64_t k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;
+    int64_t k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;      /* k_sl, v_sl below 2^27 (two rows: below 2^31; one: any) */
     int64_t cap;                   /* rows of the ring; >= j_hi for a plain tensor */
     int64_t j_lo, j_hi;            /* key index range held by the source */
     int32_t mask;                  /* INFLLM_MASK_* */

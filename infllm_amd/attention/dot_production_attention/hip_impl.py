@@ -48,6 +48,8 @@ class HipMultiStageDotProductionAttention(MultiStageDotProductionAttention):
         B, H, Lq, D = q.shape
         scale = 1.0 / math.sqrt(d)
         len_k = k.shape[2]
+        if len_k > 1 and (k.stride(2) | v.stride(2)) >= 1 << 27:          # rows further apart than the kernel's offsets reach
+            k, v = (t.clone(memory_format=torch.contiguous_format) for t in (k, v))
         if sliding_window is None:
             mask, offset, window = ops.MASK_NONE, 0, 0
         else:

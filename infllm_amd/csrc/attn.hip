@@ -247,21 +247,24 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     //      base advances in scalar registers, and which tiles are whole, and which of them a wave sees without a mask, are
     //      ranges that are known before the loop.
     constexpr int kRowsPerLd = 1024 / kRow, kLd = kTile / (kRowsPerLd * kWaves);  // load instructions per wave and tile, for K and for V
-    // byte offsets, inside a tile, of what this lane fetches for load i: rows of kd (vd) elements
+    // byte offsets, from row `first` of a tile, of what this lane fetches for load i: rows of kd (vd) elements
     auto tile_row = [&](int i) { return kRowsPerLd * (kLd * wave + i) + lane / (D / 8); };      // row of the LDS tile
-    auto k_offset = [&](int i, int64_t kd) {                                                     // (of a K tile: key k_lds_row of it)
+    auto k_offset = [&](int i, int64_t kd, int first) {                                          // (of a K tile: key k_lds_row of it)
         const int R = tile_row(i);
-        return (uint32_t)(k_lds_row(R) * kd + ((lane & (D / 8 - 1)) ^ swz<D>(R)) * 8) * 2;
+        return (uint32_t)((k_lds_row(R) - first) * kd + ((lane & (D / 8 - 1)) ^ swz<D>(R)) * 8) * 2;
     };
-    auto v_offset = [&](int i, int64_t vd) {
+    auto v_offset = [&](int i, int64_t vd, int first) {
         const int R = tile_row(i);
-        return (uint32_t)(R * vd + ((lane & (D / 8 - 1)) ^ swz<D>(R)) * 8) * 2;
+        return (uint32_t)((R - first) * vd + ((lane & (D / 8 - 1)) ^ swz<D>(R)) * 8) * 2;
     };
-    uint32_t ld_k[kLd], ld_v[kLd];           // those of the linear source (of the pages, where there is nothing else)
+    // Those of the linear source (of the pages, where there is nothing else).  Its rows may lie far apart: the base is that of the
+    // first row the wave fetches, so that 32 bits have to reach over a wave's eight rows and not over the tile's 64.
+    const int wave_rk = k_lds_row(kRowsPerLd * kLd * wave), wave_rv = kRowsPerLd * kLd * wave;
+    uint32_t ld_k[kLd], ld_v[kLd];
 #pragma unroll
     for (int i = 0; i < kLd; ++i) {
-        ld_k[i] = k_offset(i, HAS_LIN ? a.k_sl : D);
-        ld_v[i] = v_offset(i, HAS_LIN ? a.v_sl : D);
+        ld_k[i] = k_offset(i, HAS_LIN ? a.k_sl : D, HAS_LIN ? wave_rk : 0);
+        ld_v[i] = v_offset(i, HAS_LIN ? a.v_sl : D, HAS_LIN ? wave_rv : 0);
     }
     // the linear tile to load next (a tile never wraps: cap is a multiple of the tile), and tiles to the end of the ring
     const bf16_t *k_next = nullptr, *v_next = nullptr;
@@ -271,8 +274,8 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     if (HAS_LIN) {
         const int first = lin_t0 + min(g_t0, n_lin);
         const int slot = first - (int)(fdiv(first, geo.cap_tiles) * geo.cap_tiles.d);
-        k_next = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + (int64_t)slot * kTile * a.k_sl;
-        v_next = (const bf16_t *)a.d_v + (int64_t)b * a.v_sb + (int64_t)g * a.v_sh + (int64_t)slot * kTile * a.v_sl;
+        k_next = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + ((int64_t)slot * kTile + wave_rk) * a.k_sl;
+        v_next = (const bf16_t *)a.d_v + (int64_t)b * a.v_sb + (int64_t)g * a.v_sh + ((int64_t)slot * kTile + wave_rv) * a.v_sl;
         to_wrap = (int)min((int64_t)INT32_MAX, (int64_t)geo.cap_tiles.d - slot);
     }
     // linear tiles whose 64 rows are all in the source: list indices [whole_lo, whole_hi)
@@ -330,8 +333,8 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         uint32_t k_src[kLd], v_src[kLd];
 #pragma unroll
         for (int i = 0; i < kLd; ++i) {
-            k_src[i] = TWO && paged ? k_offset(i, D) : ld_k[i];
-            v_src[i] = TWO && paged ? v_offset(i, D) : ld_v[i];
+            k_src[i] = TWO && paged ? k_offset(i, D, 0) : ld_k[i];
+            v_src[i] = TWO && paged ? v_offset(i, D, 0) : ld_v[i];
         }
         if (whole) {                                   // the common case: no per-lane predicate
 #pragma unroll
@@ -1026,8 +1029,11 @@ int check_linear_stage(const infllm_attn_args *a) {
     INFLLM_REQUIRE(a->j_hi < (1ll << 36), "attn_stage: key range beyond 2^36 rows");
     INFLLM_REQUIRE((a->k_sl % 8 | a->k_sh % 8 | a->k_sb % 8 | a->v_sl % 8 | a->v_sh % 8 | a->v_sb % 8) == 0,
                    "attn_stage: k/v strides must be multiples of 8");
-    INFLLM_REQUIRE(a->k_sl >= 0 && a->v_sl >= 0 && a->k_sl < (1ll << 25) && a->v_sl < (1ll << 25), "attn_stage: k/v rows of %lld / %lld elements apart",
-                   (long long)a->k_sl, (long long)a->v_sl);          // (a lane's offset inside a tile is 32 bits of bytes)
+    // A lane's offset is 32 bits of bytes, from the first row that its wave fetches of a tile: up to 11 keys (k_lds_row), as many as there are.
+    const int64_t rows = a->j_hi - a->j_lo, far = rows <= 0 ? 0 : std::min<int64_t>(11, a->j_lo % kTile + rows - 1);
+    const int64_t most = far == 0 ? INT64_MAX : ((1ll << 31) - 128) / far;
+    INFLLM_REQUIRE(far == 0 || (a->k_sl >= 0 && a->v_sl >= 0 && a->k_sl <= most && a->v_sl <= most), "attn_stage: k/v rows of %lld / %lld elements apart",
+                   (long long)a->k_sl, (long long)a->v_sl);
     return 0;
 }
 
