@@ -718,7 +718,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     // causal prompt of 8,001 tokens 536 -> 540.  Pages, whose second tile's address is an entry of its own to wait for, gain
     // nothing by it: prompt of 131,072 25,690 us with, 25,350 without.)
     const infllm_attn_args &first = q_paged ? ap : a;
-    if (MODE != kPaged && first.q_sl < (int64_t)1 << 26) {
+    if (MODE != kPaged && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
         const uint32_t at_q = (wave < 4 ? lds_address(Ks) : lds_address(Vs)) + 2 * kTB + (wave & 3) * (kQTile * kRow);
         const bf16_t *rows = (const bf16_t *)first.d_q + (int64_t)b * first.q_sb + (int64_t)h * first.q_sh + (int64_t)i0 * first.q_sl;
 #pragma unroll
@@ -737,7 +737,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             qreg[kk] = __builtin_bit_cast(bf16x8, *(const __attribute__((address_space(3))) u32x4 *)(uintptr_t)(own ^ (kk * 32)));
             asm volatile("" : "+v"(qreg[kk]));                                          // (read before the barrier)
         }
-    } else {                               // pages, and rows further apart than a 32-bit offset reaches
+    } else {                               // pages, and rows that a 32-bit offset does not reach: far apart, or backwards
         if (t < g_t1) valid0 = load_tile(t, 0);
         load_q(first);
         landed();

@@ -667,7 +667,9 @@ inline bool wide_waves(const infllm_score_args &a) {
 
 // what the forms of score.hip that keep positions in 32 bits take
 constexpr int64_t kMaxRows = 1 << 30;
-inline bool in_reach(const infllm_score_args &a) { return (a.cap < kMaxRows || a.j_hi < kMaxRows) && (int64_t)a.Lq * a.q_sl < kMaxRows; }
+inline bool in_reach(const infllm_score_args &a) {
+    return (a.cap < kMaxRows || a.j_hi < kMaxRows) && a.Lq < kMaxRows && a.q_sl >= 0 && a.q_sl < kMaxRows && a.Lq * a.q_sl < kMaxRows;
+}
 
 // job: the log-sum-exps are to be joined (a.n_parts of them), and its merge goes along
 template <int D, bool MERGE>
