@@ -665,10 +665,13 @@ inline bool wide_waves(const infllm_score_args &a) {
     return a.j_hi - a.j_lo > 1024 && (int64_t)a.B * a.H * (((a.j_hi - 1) / 64 - a.j_lo / 64 + 4) / 4) >= 2 * kScoreCus;
 }
 
-// what the forms of score.hip that keep positions in 32 bits take
+// What the forms of score.hip that keep positions in 32 bits take.  A query's distance to a key stays below 2^30 then (2^28 between the
+// first ones, up to 2^28 queries, a range of keys below 2^24), so that a window of that or more may be cut to it.
 constexpr int64_t kMaxRows = 1 << 30;
 inline bool in_reach(const infllm_score_args &a) {
-    return (a.cap < kMaxRows || a.j_hi < kMaxRows) && a.Lq < kMaxRows && a.q_sl >= 0 && a.q_sl < kMaxRows && a.Lq * a.q_sl < kMaxRows;
+    const int64_t apart = a.mask == INFLLM_MASK_NONE ? 0 : a.offset - a.j_lo;
+    return (a.cap < kMaxRows || a.j_hi < kMaxRows) && a.Lq < kMaxRows / 4 && a.q_sl >= 0 && a.q_sl < kMaxRows && a.Lq * a.q_sl < kMaxRows &&
+           apart > -kMaxRows / 4 && apart < kMaxRows / 4;
 }
 
 // job: the log-sum-exps are to be joined (a.n_parts of them), and its merge goes along

@@ -55,6 +55,23 @@ def test_scores_of_partly_masked_stages(H, Hkv, keys, Lq, mask):
         (got[:, :, rows].double() - want - start[:, :, rows].double()).abs().max())
 
 
+@pytest.mark.parametrize("mask", ["window", "complement"])
+@pytest.mark.parametrize("apart,window", [(2 * 10 ** 9, 15 * 10 ** 8), (2 * 10 ** 9, 2 * 10 ** 9 - 50), (6 * 10 ** 8, 6 * 10 ** 8 - 50), (2 ** 28 + 9, 2 ** 28), (2 ** 28 - 9, 2 ** 28),
+                                          (2 ** 40, 2 ** 41), (-2 ** 31, 2 ** 33), (5, 2 ** 31 - 1), (-9, -5)])
+def test_scores_of_keys_far_from_their_queries(apart, window, mask):
+    """(positions that a caller gives: 32 bits hold neither such distances nor such windows)"""
+    from infllm_amd import ops
+    H, Lq, keys = 4, 70, 1100
+    code = dict(window=ops.MASK_WINDOW, complement=ops.MASK_COMPLEMENT)[mask]
+    q, k = _rand((1, H, Lq, D), 1), _rand((1, H, keys, D), 2)
+    s = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) / math.sqrt(D) * math.log2(math.e)
+    lse = torch.logsumexp(s * math.log(2.0), -1).float() / math.log(2.0)
+    want = (torch.exp2(s - lse.double()[..., None]) * _visible(code, Lq, 0, keys, apart, window)).sum(2)
+    score = torch.empty((1, H, keys), device="cuda")
+    ops.local_score(q.cuda(), k.cuda(), lse.cuda(), score, mask=code, offset=apart, window=window, accumulate=False)
+    assert torch.allclose(score.cpu().double(), want, rtol=1e-4, atol=1e-5)
+
+
 @pytest.mark.parametrize("H,Hkv,keys", [(4, 2, 1025), (64, 64, 2100)])
 @pytest.mark.parametrize("Lq,parts", [(1, (1, 0)), (33, (2, 1)), (512, (4, 4)), (2048, (1, 2))])
 @pytest.mark.parametrize("mask", ["none", "window", "complement"])
