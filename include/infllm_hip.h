@@ -285,6 +285,8 @@ int infllm_local_score_merge_pair(const infllm_score_args *a, const uint16_t *d_
  *                order, context_manager.py:495-515); equal scores go to the lower index
  *                first, at the boundary and in the order.
  * reps [N,C] bf16 row stride rep_stride; C = H*128.  k <= 1024.
+ * One launch up to N = 16384, k = 64 and rows of 4608 elements; two where that does not reach, in a call that a graph captures (its
+ * replays run beside anything) and, in a process of many streams, on those beyond the 256th.
  */
 int infllm_score_topk(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C,
                       const float *d_qbar, int32_t k,
@@ -706,7 +708,7 @@ typedef struct {
     float *d_call_scores;                             /* [blocks, B, scores_cols], scores_cols >= the units after the call */
     int64_t scores_cols;
     int32_t *d_base;                                  /* [blocks, B, topk] */
-    uint32_t *d_ticket;                               /* one word, zero when the workspaces are made; every call leaves it zero */
+    uint32_t *d_ticket;                               /* one word, zero when the workspaces are made; every call leaves it zero (a call of one token may have NULL) */
 } infllm_resident_call;
 int infllm_resident_append(void *handle, const infllm_resident_call *a, void *stream);
 int64_t infllm_resident_part_rows(const infllm_resident_desc *d);

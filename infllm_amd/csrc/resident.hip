@@ -48,7 +48,7 @@ int infllm_gather_rows_pair(const void *d_ring_a, void *d_out_a, const void *d_r
                             int32_t Hkv, int64_t t0, int32_t n, int32_t unit_rows, int64_t out_sb, int64_t out_su, int64_t out_sh,
                             void *stream, int32_t dim);
 int infllm_retrieve_step(const void *d_reps, int64_t rep_stride, int32_t N, const infllm_ingest_args *in, int32_t dim, int32_t b, bool prologue, int32_t k,
-                         float *d_scores, int32_t *d_idx, void *stream);
+                         float *d_scores, int32_t *d_idx, uint32_t *d_ticket, void *stream);
 int infllm_key_splits(const infllm_layer_desc *d, int32_t n_queries, int32_t n_tiles);
 
 namespace {
@@ -416,7 +416,7 @@ int decode_step(Resident *R, const infllm_resident_call *a, int64_t st0, hipStre
         ids = d.d_ids;
         for (int u = 0; u < B; ++u) {                            // the prologue rides with the first row's retrieval
             rc = infllm_retrieve_step((const bf16_t *)a->d_reps + (int64_t)u * a->rep_sb, a->rep_su, N, &in, d.dim, u, u == 0, d.topk,
-                                      a->d_unit_scores + (int64_t)u * a->unit_scores_sb, d.d_ids + (int64_t)u * d.topk, st);
+                                      a->d_unit_scores + (int64_t)u * a->unit_scores_sb, d.d_ids + (int64_t)u * d.topk, a->d_ticket, st);
             if (rc < 0) return rc;
             if (rc == 1) break;                                  // (of all rows or of none: it depends on their length and number)
         }

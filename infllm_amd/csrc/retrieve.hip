@@ -432,8 +432,35 @@ __global__ __launch_bounds__(256) void score_new_rank_kernel(const bf16_t *reps,
 // number, say) the exact k-th largest composite is built bit by bit instead - slower, never wrong.
 constexpr int kRetrThreads = 512;
 constexpr int kSurvivorCap = 1024;
-constexpr int kTicketSlots = 64;
-static __device__ unsigned int retrieval_tickets[kTicketSlots];       // zero at load; the last workgroup puts its slot back to zero
+//
+// The ticket is a word that is zero before and behind every launch, and that no two launches may count in at a time.  A manager
+// has one among its workspaces; a retrieval by itself takes the library's word for its stream, whose launches follow each other.
+constexpr int kTicketSlots = 256;
+static __device__ unsigned int retrieval_tickets[kTicketSlots];       // zero at load
+
+// The place of the stream's word, -1: it has none, as every place is another stream's (they are never given back), the handle
+// means another stream in every thread, or the launch is captured: a graph is replayed on any stream, beside anything.
+int ticket_slot(hipStream_t st) {
+    static std::atomic<uint64_t> owner[kTicketSlots];                 // 1 + the stream's handle, 0: free
+    if (st == hipStreamPerThread) return -1;
+    if (st) {                                                         // (the default stream cannot be captured)
+        hipStreamCaptureStatus status;
+        if (hipStreamIsCapturing(st, &status) != hipSuccess || status != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return -1;
+        }
+    }
+    const uint64_t key = (uint64_t)(uintptr_t)st + 1;
+    const int first = (int)((key * 0x9e3779b97f4a7c15ull) >> 56);
+    static_assert(kTicketSlots == 256, "8 bits of the product");
+    for (int i = 0; i < kTicketSlots; ++i) {
+        std::atomic<uint64_t> &place = owner[(first + i) % kTicketSlots];
+        uint64_t seen = place.load(std::memory_order_relaxed);
+        if (seen == 0 && place.compare_exchange_strong(seen, key, std::memory_order_relaxed)) return (first + i) % kTicketSlots;
+        if (seen == key) return (first + i) % kTicketSlots;
+    }
+    return -1;
+}
 
 // the selection by one workgroup of kRetrThreads threads over N <= NB * 16 * kRetrThreads scores; a thread keeps its
 // keys (units tid, tid + kRetrThreads, ...) in registers
@@ -552,7 +579,7 @@ struct NoFront {};
 template <int CPL, int ROWS, bool TAIL, bool FRONT = false>
 __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16_t *reps, int64_t rep_stride, int N, int C_, const float *qbar,
                                                                       float *scores, int k, int32_t *idx_out, int32_t *idx_out2,
-                                                                      int32_t *flag, int32_t flag_value, int ticket_slot,
+                                                                      int32_t *flag, int32_t flag_value, uint32_t *own_ticket, int ticket_slot,
                                                                       std::conditional_t<FRONT, StepFront, NoFront> front) {
     extern __shared__ float qs[];                                // the mean query
     __shared__ int is_last;
@@ -643,14 +670,15 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
     // every wave's score stores have been performed before the workgroup takes its ticket
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    unsigned int *const ticket = own_ticket ? own_ticket : &retrieval_tickets[ticket_slot];
     if (threadIdx.x == 0) {
-        const unsigned int drawn = __hip_atomic_fetch_add(&retrieval_tickets[ticket_slot], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned int drawn = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         is_last = drawn == (unsigned int)n_wgs - 1;
     }
     __syncthreads();
     if (!is_last) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    if (threadIdx.x == 0) __hip_atomic_store(&retrieval_tickets[ticket_slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (N <= 16 * kRetrThreads) select_topk_block<1>(scores, N, k, idx_out, idx_out2);
     else select_topk_block<2>(scores, N, k, idx_out, idx_out2);
     publish(flag, flag_value);
@@ -1087,14 +1115,13 @@ extern "C" int infllm_score_topk_queries(const void *d_reps, int64_t rep_stride,
 // library-internal: unit scores of all N units and the k best of them in ONE launch (retrieve_fused_kernel), the ids
 // leaving as infllm_topk_publish_pair leaves them.  Returns 1, with nothing launched, where that kernel does not apply
 // (rows of more than 4608 elements or not of whole 16-byte chunks, more than 16384 units, k > 64): the caller then launches the two steps.
+// ticket: the caller's word, or NULL and slot >= 0: the library's word there; neither: returns 1.
 static int retrieve_launch(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar, int32_t k, float *d_scores, int32_t *d_idx,
-                           int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, const StepFront *front, bool whole_front, void *stream) {
+                           int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, const StepFront *front, bool whole_front, uint32_t *ticket, int slot, void *stream) {
     INFLLM_REQUIRE(d_reps && (d_qbar || front) && d_scores && d_idx, "retrieve: null pointer");
     INFLLM_REQUIRE(N > 0 && k > 0 && k <= N, "retrieve: k=%d with N=%d", k, N);
     INFLLM_REQUIRE(rep_stride >= C && rep_stride % 8 == 0, "retrieve: row stride %lld", (long long)rep_stride);
-    if (N > 16384 || k > 64 || C % 8 != 0 || C > 9 * 512) return 1;
-    static std::atomic<unsigned int> next_slot{0};
-    const int slot = (int)(next_slot.fetch_add(1, std::memory_order_relaxed) % kTicketSlots);
+    if (N > 16384 || k > 64 || C % 8 != 0 || C > 9 * 512 || (!ticket && slot < 0)) return 1;
     constexpr int waves_per_wg = kRetrThreads / 64;
     const bool deep = N >= 4096;
     const int per_wg = waves_per_wg * (deep ? 2 : 1);
@@ -1113,11 +1140,11 @@ static int retrieve_launch(const void *d_reps, int64_t rep_stride, int32_t N, in
     if (front) {                                                                                                                     \
         auto kern = deep ? retrieve_fused_kernel<c, 2, tail, true> : retrieve_fused_kernel<c, 1, tail, true>;                        \
         hipLaunchKernelGGL(kern, dim3(wgs + extra), dim3(kRetrThreads), (size_t)c * 512 * sizeof(float), st, reps, rep_stride, N, C,  \
-                           d_qbar, d_scores, k, d_idx, d_idx2, d_flag, flag_value, slot, f);                                         \
+                           d_qbar, d_scores, k, d_idx, d_idx2, d_flag, flag_value, ticket, slot, f);                                 \
     } else {                                                                                                                         \
         auto kern = deep ? retrieve_fused_kernel<c, 2, tail> : retrieve_fused_kernel<c, 1, tail>;                                    \
         hipLaunchKernelGGL(kern, dim3(wgs), dim3(kRetrThreads), (size_t)c * 512 * sizeof(float), st, reps, rep_stride, N, C, d_qbar,  \
-                           d_scores, k, d_idx, d_idx2, d_flag, flag_value, slot, NoFront{});                                         \
+                           d_scores, k, d_idx, d_idx2, d_flag, flag_value, ticket, slot, NoFront{});                         \
     }
     if (C == 512) { FUSED_CASE(1, false) }
     else if (C == 1024) { FUSED_CASE(2, false) }
@@ -1132,14 +1159,14 @@ static int retrieve_launch(const void *d_reps, int64_t rep_stride, int32_t N, in
 }
 
 int infllm_retrieve_fused(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar, int32_t k, float *d_scores,
-                          int32_t *d_idx, int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, void *stream) {
-    return retrieve_launch(d_reps, rep_stride, N, C, d_qbar, k, d_scores, d_idx, d_idx2, d_flag, flag_value, nullptr, false, stream);
+                          int32_t *d_idx, int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, uint32_t *d_ticket, void *stream) {
+    return retrieve_launch(d_reps, rep_stride, N, C, d_qbar, k, d_scores, d_idx, d_idx2, d_flag, flag_value, nullptr, false, d_ticket, -1, stream);
 }
 
 // library-internal: the same for the one query of a decode step, batch row b of `in` (whose d_qpart is not used); with `prologue`
 // the launch also does what infllm_ingest_dim does for the step, for all batch rows
 int infllm_retrieve_step(const void *d_reps, int64_t rep_stride, int32_t N, const infllm_ingest_args *in, int32_t dim, int32_t b, bool prologue, int32_t k,
-                         float *d_scores, int32_t *d_idx, void *stream) {
+                         float *d_scores, int32_t *d_idx, uint32_t *d_ticket, void *stream) {
     INFLLM_REQUIRE(in && in->n == 1 && in->d_q && in->d_k && in->d_v && in->d_inv_freq && in->d_ring_k_raw && in->d_ring_k_rot && in->d_ring_v &&
                        in->d_ring_score && in->d_q_loc && in->d_q_glb, "retrieve_step: null pointer");
     INFLLM_REQUIRE(in->B > 0 && in->H > 0 && in->Hkv > 0 && in->H % in->Hkv == 0 && in->pos0 >= 0 && in->ring_cap > 0 && b >= 0 && b < in->B,
@@ -1151,7 +1178,7 @@ int infllm_retrieve_step(const void *d_reps, int64_t rep_stride, int32_t N, cons
     f.in = *in;
     f.dim = dim;
     f.b = b;
-    return retrieve_launch(d_reps, rep_stride, N, in->H * dim, nullptr, k, d_scores, d_idx, nullptr, nullptr, 0, &f, prologue, stream);
+    return retrieve_launch(d_reps, rep_stride, N, in->H * dim, nullptr, k, d_scores, d_idx, nullptr, nullptr, 0, &f, prologue, d_ticket, -1, stream);
 }
 
 extern "C" int infllm_score_topk(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar,
@@ -1159,7 +1186,8 @@ extern "C" int infllm_score_topk(const void *d_reps, int64_t rep_stride, int32_t
     INFLLM_REQUIRE(N > 0 && k >= 0 && k <= N, "score_topk: k=%d with N=%d", k, N);
     if (k > 0) {
         INFLLM_REQUIRE(d_idx, "score_topk: null index pointer");
-        const int frc = infllm_retrieve_fused(d_reps, rep_stride, N, C, d_qbar, k, d_scores, d_idx, nullptr, nullptr, 0, stream);
+        const int frc = retrieve_launch(d_reps, rep_stride, N, C, d_qbar, k, d_scores, d_idx, nullptr, nullptr, 0, nullptr, false, nullptr,
+                                        ticket_slot((hipStream_t)stream), stream);
         if (frc != 1) return frc;
     }
     int rc = infllm_unit_scores(d_reps, rep_stride, 0, N, C, d_qbar, d_scores, stream);

@@ -117,6 +117,7 @@ struct Layer {
     bool mass_pending = false;
     int32_t topk_seq = 0;
     hipStream_t topk_stream = nullptr;    // stream of the last selection (to fall back on when the poll gives up)
+    uint32_t *d_ticket = nullptr;         // the retrievals' word (their launches follow each other): zero between them
     // the top-k of the units that existed when the next block was prepared, chosen ahead of the chain: [B,topk]
     // device ids (this handle's own allocation) and the unit count they were chosen from (-1: none)
     int32_t *d_cand = nullptr;
@@ -203,7 +204,7 @@ int infllm_call_rank(const CallRankJob *job, int32_t C, int32_t n_wgs, void *str
 int infllm_call_rank_room();
 constexpr int kMaxCallBlocks = 16;
 int infllm_retrieve_fused(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar, int32_t k, float *d_scores,
-                          int32_t *d_idx, int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, void *stream);
+                          int32_t *d_idx, int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, uint32_t *d_ticket, void *stream);
 int infllm_inline_page_limit();
 int infllm_copy_units(const void *const *d_src, void *const *d_dst, int32_t n, int64_t nbytes, void *stream);
 int infllm_merge_job(const uint16_t *d_o_part, const float *d_lse_part, int32_t P1, const uint16_t *d_o_part2, const float *d_lse_part2,
@@ -866,6 +867,12 @@ extern "C" void *infllm_layer_create(const infllm_layer_desc *desc) {
         L->d_cand = nullptr;                        // not fatal: selections then run over all units every time
         (void)hipGetLastError();
     }
+    const uint32_t zero = 0;
+    if (hipMalloc((void **)&L->d_ticket, sizeof(zero)) != hipSuccess || hipMemcpy(L->d_ticket, &zero, sizeof(zero), hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipGetLastError();
+        if (L->d_ticket) (void)hipFree(L->d_ticket);
+        L->d_ticket = nullptr;                      // not fatal: a retrieval is two launches then
+    }
     L->dma_busy.assign(d.carve_slots, 0);
     L->dma_first.assign(d.carve_slots, 0);
     L->dma_count.assign(d.carve_slots, 0);
@@ -935,6 +942,7 @@ extern "C" int infllm_layer_destroy(void *layer) {
         for (hipEvent_t e : t.ev)
             if (e) (void)hipEventDestroy(e);
     if (L->d_cand) (void)hipFree(L->d_cand);
+    if (L->d_ticket) (void)hipFree(L->d_ticket);
     if (L->d_base) (void)hipFree(L->d_base);
     if (L->h_cand) (void)hipHostFree(L->h_cand);
     for (void *c : L->ahead.shadow)
@@ -1091,7 +1099,7 @@ int run_retrieval(Layer *L, const void *reps, int64_t rep_sb, int64_t rep_su, fl
         const bf16_t *reps_u = (const bf16_t *)reps + (int64_t)u * rep_sb;
         float *scores_u = scores + (int64_t)u * scores_sb;
         int rc = infllm_retrieve_fused(reps_u, rep_su, n_units, C, qbar + (int64_t)u * C, d.topk, scores_u, d.d_topk_idx + (int64_t)u * d.topk,
-                                       nullptr, last ? d.d_topk_flag : nullptr, L->topk_seq, stream);
+                                       nullptr, last ? d.d_topk_flag : nullptr, L->topk_seq, L->d_ticket, stream);
         if (rc < 0) return rc;
         if (rc == 1) {
             rc = infllm_unit_scores(reps_u, rep_su, 0, n_units, C, qbar + (int64_t)u * C, scores_u, stream);
@@ -1445,7 +1453,7 @@ extern "C" int infllm_block_front(void *layer, const infllm_front_args *a, void 
                 int32_t *cand_host = buf >= 0 ? cand_buffer(L, buf) + (int64_t)u * d.topk : nullptr;
                 int32_t *cand_flag = buf >= 0 && u == d.B - 1 ? cand_buffer(L, buf) + (int64_t)d.B * d.topk : nullptr;
                 rc = want_cand ? infllm_retrieve_fused(reps_u, a->rep_su, a->n_units, C, qbar_u, d.topk, scores_u, L->d_cand + (int64_t)u * d.topk,
-                                                       cand_host, cand_flag, L->cand_seq, stream)
+                                                       cand_host, cand_flag, L->cand_seq, L->d_ticket, stream)
                                : 1;
                 if (rc < 0) return rc;
                 if (rc == 1) {
