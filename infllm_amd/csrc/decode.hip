@@ -43,7 +43,7 @@ __device__ __forceinline__ void each_head(F &&f) {
 //
 // FRONT: the step's rows come as they are (StepRows).  Rotating them in a launch in front cost 5 us on a chain of two, and its
 // cache writes, copies included, were waited for by an attention that can read the old cache: here every workgroup rotates its
-// heads' queries while its first rows are on their way, the last split attends the new key, and workgroups behind the splits
+// heads' queries while its first rows are on their way, the last split attends the new key, and workgroups behind all splits
 // write the cache (stream-llm, one token over 9,000: 25.4 -> 22.7 us; causal, over 8,192: 26.7 -> 24.0).
 struct NoFront {};
 template <int D>
@@ -85,12 +85,13 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int col = lane & 15, rg = lane >> 4;
     const int G = j.H / j.Hkv, chunks = (G + NG - 1) / NG;
-    const int split = blockIdx.x, g = blockIdx.y / chunks, c = blockIdx.y % chunks, b = blockIdx.z, n_split = FRONT ? j.nsplit : (int)gridDim.x;
+    const int split = blockIdx.x, g = blockIdx.y / chunks, c = blockIdx.y % chunks, b = blockIdx.z, n_split = gridDim.x;
     if constexpr (FRONT) {
-        if (split >= n_split) {
-            if (c != 0) return;
-            if (split == n_split) leave_rows<D>(f, b, g, (float2 *)red_room);
-            else copy_rows<D>(f.copy, split - n_split - 1, b, g);
+        if (b >= j.B) {
+            const int x = split + n_split * ((int)blockIdx.y + (int)gridDim.y * (b - j.B)), per = 1 + f.pieces, bg = x / per, piece = x - bg * per;
+            if (bg >= j.B * j.Hkv) return;
+            if (piece == 0) leave_rows<D>(f, bg / j.Hkv, bg % j.Hkv, (float2 *)red_room);
+            else copy_rows<D>(f.copy, piece - 1, bg / j.Hkv, bg % j.Hkv);
             return;
         }
     }
@@ -434,7 +435,16 @@ int launch(const DecodeJob *job, void *stream) {
 template <int D>
 int launch_step(const DecodeJob *job, const StepRows *rows, void *stream) {
     const int G = job->H / job->Hkv, NG = G >= 3 ? 4 : G;
-    const dim3 grid(job->nsplit + 1 + rows->pieces, job->Hkv * ((G + NG - 1) / NG), job->B);
+    const int y = job->Hkv * ((G + NG - 1) / NG);
+    // The workgroups that write the cache come behind all splits, in batch rows of their own.  In the grid's first dimension, behind
+    // the splits of every head, they took places among the 512 that the chip has at two workgroups a CU and left again, so that some
+    // CUs got three splits and some one, and a row of 65 spread the heads of a group, which read the same keys, over the XCDs: causal
+    // steps of 8 key heads over 24,000 / 32,768 / 49,152 tokens 31.8 / 39.3 / 52.1 us so, 29.3 / 33.2 / 42.4 now, 32.5 / 36.5 / 45.7 as two
+    // launches; of 2 key heads with 16 query heads each over 65,536 / 98,304 60.9 / 88.2, 38.1 / 54.1 and 47.2 / 63.1; of 36 heads of 64
+    // over 10,000 26.7, 26.7 and 32.2.
+    const int64_t extra = (int64_t)(1 + rows->pieces) * job->Hkv * job->B, planes = (extra + (int64_t)job->nsplit * y - 1) / ((int64_t)job->nsplit * y);
+    if (job->B + planes > 65535 || extra >= (1ll << 30)) return 1;
+    const dim3 grid(job->nsplit, y, (unsigned)(job->B + planes));
     const auto kern = NG == 1 ? decode_attn_kernel<D, 1, false, true, true> : NG == 2 ? decode_attn_kernel<D, 2, false, true, true>
                                                                                   : decode_attn_kernel<D, 4, false, true, true>;
     hipLaunchKernelGGL(kern, grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, *rows);
@@ -471,7 +481,8 @@ static int check_job(const DecodeJob *job, int32_t dim) {
     return 0;
 }
 
-// rows: the step's own (their strides multiples of 8 elements); job->out and job->ticket are set, the ranges are plain ones
+// rows: the step's own (their strides multiples of 8 elements); job->out and job->ticket are set, the ranges are plain ones.  Returns
+// 1, with nothing launched, where the grid does not hold the batch.
 int infllm_decode_step(const DecodeJob *job, const StepRows *rows, int32_t dim, void *stream) {
     const int rc = check_job(job, dim);
     if (rc) return rc;

@@ -268,16 +268,13 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     }
     if (j.n_raw > 0 && a->raw_old > 0)
         copy(a->d_raw_old, (int64_t)a->raw_old * D * a->Hkv, (int64_t)a->raw_old * D, 0, a->d_raw, raw_sh * a->Hkv, raw_sh, 0, a->raw_old);
-    // ---- A step whose old rows hold all it sees but its own key is one launch.  Not where nothing is copied and the rows are so many
-    //      that their stream is what the step costs: every workgroup's rotation holds its stream up for 2 us then, which a launch in
-    //      front spends on one.  Causal steps of 8 key heads of 128 over 500 / 8,192 / 16,384 / 24,000 / 32,768 tokens: one launch
-    //      24.2 / 24.0 / 24.6 / 30.3 / 38.0 us, two 27.3 / 26.7 / 26.3 / 30.2 / 36.0.
+    // ---- A step whose old rows hold all it sees but its own key is one launch.
+    int rc;
     const int64_t near_rows = causal ? rows_base : std::min<int64_t>(rows_base, a->n_local);       // of the new cache, the last of them the new one
     const int64_t far_rows = std::max<int64_t>(0, std::min<int64_t>(n_sink, len_k - a->n_local));  // sink j is seen from a distance of at least n_local
     const void *raw_from = a->raw_new > a->raw_old ? a->d_raw_old : a->d_raw;
     const int64_t raw_from_sh = (int64_t)(a->raw_new > a->raw_old ? a->raw_old : a->raw_new) * D;
-    const bool streams = nc == 0 && (int64_t)a->B * a->Hkv * (near_rows + far_rows) * D * 4 > (int64_t)96 << 20;
-    if (step && !streams && a->n_new == 1 && !all && a->d_ticket && !fresh && near_rows >= 1 && near_rows - 1 <= a->rows_old && far_rows <= a->rows_old &&
+    if (step && a->n_new == 1 && !all && a->d_ticket && !fresh && near_rows >= 1 && near_rows - 1 <= a->rows_old && far_rows <= a->rows_old &&
         (far_rows == 0 || a->kind != 2 || (raw_from && far_rows * D <= raw_from_sh))) {
         DecodeJob d{};
         d.B = a->B; d.H = a->H; d.Hkv = a->Hkv;
@@ -304,9 +301,9 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
             f.copy[i] = j.copy[i];
             f.pieces += (j.copy[i].n + kCopyRows - 1) / kCopyRows;
         }
-        return infllm_decode_step(&d, &f, D, stream);
+        rc = infllm_decode_step(&d, &f, D, stream);
+        if (rc != 1) return rc;
     }
-    int rc;
     if (a->n_q == a->n_new) {
         j.do_q = j.do_kv = 1;
         j.n = a->n_q;
