@@ -160,8 +160,8 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
     inv_freq = position_bias.inv_freq
     if inv_freq.device != dev or inv_freq.dtype != torch.float32 or inv_freq.numel() != dim // 2 or not inv_freq.is_contiguous():
         inv_freq = inv_freq.to(device=dev, dtype=torch.float32).contiguous() if native else wide_inv_freq(inv_freq, dev)
-    if inv_freq.numel() != dim // 2:
-        raise ValueError(f"the rotary embedding is built for head_dim {2 * position_bias.inv_freq.numel()}, the heads have {dim_head}")
+        if inv_freq.numel() != dim // 2:
+            raise ValueError(f"the rotary embedding is built for head_dim {2 * position_bias.inv_freq.numel()}, the heads have {dim_head}")
 
     old_k = old_v = raw_old = None
     seen = rows_old = raw_rows = 0
@@ -179,19 +179,19 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
                 raw_old = raw_old.clone(memory_format=torch.contiguous_format)
             raw_rows = raw_old.size(2)
     rows_all, len_k = rows_old + n_new, seen + n_new
-    bf = dict(dtype=torch.bfloat16, device=dev)
+    bf = torch.bfloat16
     cut = kind and len_k > n_local + n_init and rows_all > n_local + n_init
     raw, raw_new = raw_old, raw_rows
     if kind == 2 and raw_rows < n_init and seen == raw_rows:   # un-rotated copies of the first n_init keys
         raw_new = min(n_init, len_k)
-        raw = torch.empty((batch, num_heads_kv, raw_new, dim), **bf)
+        raw = torch.empty((batch, num_heads_kv, raw_new, dim), dtype=bf, device=dev)
     all_kv = None
     if cut:
         rows_new = n_init + n_local
-        cache = torch.empty((2, batch, num_heads_kv, rows_new, dim), **bf)
+        cache = torch.empty((2, batch, num_heads_kv, rows_new, dim), dtype=bf, device=dev)
         new_k, new_v = cache.unbind(0)
         if len_q > 1 or n_new > 1:
-            all_kv = torch.empty((2, batch, num_heads_kv, rows_all, dim), **bf)
+            all_kv = torch.empty((2, batch, num_heads_kv, rows_all, dim), dtype=bf, device=dev)
     else:
         rows_new = rows_all
         shape = (batch, num_heads_kv, rows_all, dim)
@@ -202,7 +202,7 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
             cap = rows_all + max(256, rows_all // 4)
             if kind:
                 cap = max(rows_all, min(cap, n_local + n_init))
-            both = torch.empty((2, batch, num_heads_kv, cap, dim), **bf)
+            both = torch.empty((2, batch, num_heads_kv, cap, dim), dtype=bf, device=dev)
             _Room(both, rows_all, stream)
             new_k, new_v = both.narrow(3, 0, rows_all).unbind(0)
 
@@ -212,7 +212,7 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
     part_rows = 64 * rows_q if rows_q <= 2048 else _SPLIT_ROWS if 2 * rows_q <= _SPLIT_ROWS else 0
     work_bytes = q_bytes + part_rows * (2 * dim + 4) + (4 * rows_q if len_q == 1 else 0)
     work = torch.empty((work_bytes,), dtype=torch.uint8, device=dev)
-    out = torch.empty((batch, len_q, num_heads * dim), **bf)
+    out = torch.empty((batch, len_q, num_heads * dim), dtype=bf, device=dev)
     okp = ovp = 0
     ok_sb = ok_sh = ov_sb = ov_sh = 0
     if rows_old:

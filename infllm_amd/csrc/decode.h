@@ -46,31 +46,34 @@ struct RowCopy {
     int32_t n;
 };
 constexpr int kCopies = 7;
-constexpr int kCopyRows = 64;                  // rows a copying workgroup of 256 threads moves
-
+// Rows that a copying workgroup of 256 threads moves, and beside the splits of a step, which waits for the last of them: splits of
+// heads of 128 leave it a third of the chip, so few and long ones; those of heads of 64 leave it most.  (infinite-lm, one token over
+// 9,000, window of 4,096, 8 key heads of 128: 64 rows 22.9 us, 256 rows 21.0; stream-llm over 6,000, 36 heads of 64: 24.4, 27.4.)
+constexpr int kCopyRows = 64;
 template <int D>
+constexpr int kStepCopyRows = D == 128 ? 256 : 64;
+
+template <int D, int kRows>
 __device__ __forceinline__ void copy_rows(const RowCopy (&copies)[kCopies], int piece, int b, int g) {
     const int tid = threadIdx.x;
-    for (int c = 0; c < kCopies; ++c) {
-        const RowCopy &rc = copies[c];
-        const int n = (rc.n + kCopyRows - 1) / kCopyRows;
-        if (piece >= n) {
-            piece -= n;
-            continue;
-        }
-        const int r0 = piece * kCopyRows, m = min(kCopyRows, rc.n - r0) * (D / 8);
-        const u32x4 *src = (const u32x4 *)(rc.src + (int64_t)b * rc.s_sb + (int64_t)g * rc.s_sh + (int64_t)r0 * D);
-        u32x4 *dst = (u32x4 *)(rc.dst + (int64_t)b * rc.d_sb + (int64_t)g * rc.d_sh + (int64_t)r0 * D);
-        constexpr int U = kCopyRows * (D / 8) / 256;
-        u32x4 x[U];
-#pragma unroll
-        for (int i = 0; i < U; ++i)
-            if (tid + 256 * i < m) x[i] = src[tid + 256 * i];
-#pragma unroll
-        for (int i = 0; i < U; ++i)
-            if (tid + 256 * i < m) dst[tid + 256 * i] = x[i];
-        return;
+    int c = 0;
+    for (; c < kCopies; ++c) {
+        const int n = (copies[c].n + kRows - 1) / kRows;
+        if (piece < n) break;
+        piece -= n;
     }
+    if (c == kCopies) return;
+    const RowCopy &rc = copies[c];
+    const int r0 = piece * kRows, m = min(kRows, rc.n - r0) * (D / 8);
+    const u32x4 *src = (const u32x4 *)(rc.src + (int64_t)b * rc.s_sb + (int64_t)g * rc.s_sh + (int64_t)r0 * D);
+    u32x4 *dst = (u32x4 *)(rc.dst + (int64_t)b * rc.d_sb + (int64_t)g * rc.d_sh + (int64_t)r0 * D);
+    constexpr int U = kRows * (D / 8) / 256;
+    u32x4 x[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) x[i] = src[min(tid + 256 * i, m - 1)];              // (every one loaded: conditions here made the compiler spill)
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+        if (tid + 256 * i < m) dst[tid + 256 * i] = x[i];
 }
 
 // The rows of the step itself, as they come (DecodeJob's ranges are the rows that were there before, its q is not used): the

@@ -88,10 +88,9 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     const int split = blockIdx.x, g = blockIdx.y / chunks, c = blockIdx.y % chunks, b = blockIdx.z, n_split = gridDim.x;
     if constexpr (FRONT) {
         if (b >= j.B) {
-            const int x = split + n_split * ((int)blockIdx.y + (int)gridDim.y * (b - j.B)), per = 1 + f.pieces, bg = x / per, piece = x - bg * per;
-            if (bg >= j.B * j.Hkv) return;
-            if (piece == 0) leave_rows<D>(f, bg / j.Hkv, bg % j.Hkv, (float2 *)red_room);
-            else copy_rows<D>(f.copy, piece - 1, bg / j.Hkv, bg % j.Hkv);
+            const int x = split + n_split * ((int)blockIdx.y + (int)gridDim.y * (b - j.B)), n_rows = j.B * j.Hkv, at = x - n_rows, bg = at / max(f.pieces, 1);
+            if (at < 0) leave_rows<D>(f, x / j.Hkv, x % j.Hkv, (float2 *)red_room);
+            else if (at < n_rows * f.pieces) copy_rows<D, kStepCopyRows<D>>(f.copy, at - bg * f.pieces, bg / j.Hkv, bg % j.Hkv);
             return;
         }
     }

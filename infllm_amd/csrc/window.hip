@@ -46,7 +46,7 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
     __shared__ float2 cs_glb[HALF];
     const int tid = threadIdx.x, b = blockIdx.y, g = blockIdx.z;
     if ((int)blockIdx.x >= j.tiles) {
-        copy_rows<D>(j.copy, (int)blockIdx.x - j.tiles, b, g);
+        copy_rows<D, kCopyRows>(j.copy, (int)blockIdx.x - j.tiles, b, g);
         return;
     }
     if (blockIdx.x == 0 && b == 0 && g == 0)
@@ -297,9 +297,10 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         f.inv_freq = a->d_inv_freq; f.distance_scale = a->distance_scale;
         f.dk = j.dk; f.dv = j.dv; f.dk_sb = j.dk_sb; f.dk_sh = j.dk_sh; f.dv_sb = j.dv_sb; f.dv_sh = j.dv_sh;
         if (j.n_raw > 0) f.raw = j.raw, f.raw_sb = j.raw_sb, f.raw_sh = j.raw_sh;
+        const int piece_rows = D == 128 ? kStepCopyRows<128> : kStepCopyRows<64>;
         for (int i = 0; i < kCopies; ++i) {
             f.copy[i] = j.copy[i];
-            f.pieces += (j.copy[i].n + kCopyRows - 1) / kCopyRows;
+            f.pieces += (j.copy[i].n + piece_rows - 1) / piece_rows;
         }
         rc = infllm_decode_step(&d, &f, D, stream);
         if (rc != 1) return rc;
