@@ -1,5 +1,6 @@
 """Local scores where a stage of queries is masked in part: the diagonal, the far end of the window, ranges of keys that begin
-and end inside a wave's, queries that end inside a stage, rings that wrap - for launches whose waves hold 32 keys and 64.
+and end inside a wave's, queries that end inside a stage, rings that wrap - for launches whose waves hold 32 keys and 64, of
+the kernel for finished log-sum-exps and of the general one.
 
 Against 64 bits over the same bf16 inputs and the same log-sum-exps.  A probability is exp2 of a 32-bit sum of 128 products (an
 error of some 2^-20 of the logit's size, below 2^5 here) and a score a 32-bit sum of up to 600 of them: 1e-4 relative, 1e-5
@@ -26,7 +27,19 @@ def _visible(mask, Lq, lo, hi, offset, window):
 @pytest.mark.parametrize("Lq", [1, 33, 130, 512, 600])
 @pytest.mark.parametrize("mask", ["none", "window", "complement"])
 def test_scores_of_partly_masked_stages(H, Hkv, keys, Lq, mask):
-    from infllm_amd import ops
+    _partly_masked(H, Hkv, keys, Lq, mask)
+
+
+# The general kernel, for log-sum-exps in parts: one part, fewer than eight, eight, more than a turn of eight
+@pytest.mark.parametrize("H,Hkv,keys", [(4, 2, 700), (64, 64, 2100)])
+@pytest.mark.parametrize("Lq,parts", [(1, 1), (33, 3), (130, 8), (512, 2), (600, 11)])
+@pytest.mark.parametrize("mask", ["none", "window", "complement"])
+def test_scores_of_the_general_kernel(H, Hkv, keys, Lq, parts, mask):
+    _partly_masked(H, Hkv, keys, Lq, mask, parts)
+
+
+def _partly_masked(H, Hkv, keys, Lq, mask, parts=0):
+    from infllm_amd import _lib, ops
     cap, lo = 2304, 77
     hi = lo + keys
     code = dict(none=ops.MASK_NONE, window=ops.MASK_WINDOW, complement=ops.MASK_COMPLEMENT)[mask]
@@ -45,8 +58,18 @@ def test_scores_of_partly_masked_stages(H, Hkv, keys, Lq, mask):
     want = torch.where(vis, torch.exp2(s - torch.where(torch.isfinite(lse), lse32.double(), math.inf)[..., None]), 0.0).sum(2)
     start = torch.rand((1, H, cap), generator=torch.Generator().manual_seed(3))
     score = start.cuda()
-    ops.local_score(q.cuda(), ring.cuda(), torch.where(torch.isfinite(lse32), lse32, math.inf).cuda(), score, cap=cap, j_lo=base + lo, j_hi=base + hi, mask=code,
-                    offset=offset + base, window=window, accumulate=True, score_cap=cap)
+    where = dict(cap=cap, j_lo=base + lo, j_hi=base + hi, mask=code, offset=offset + base, window=window, accumulate=True, score_cap=cap)
+    if parts:                                                  # shares of the sum; a share of nothing in the first of several
+        share = torch.softmax(torch.randn((parts, 1, H, Lq), generator=torch.Generator().manual_seed(4)).double(), 0)
+        if parts > 1:
+            share[1] += share[0]
+            share[0] = 0
+        lses, q_dev, k_dev = (lse32 + torch.log2(share)).float().cuda(), q.cuda(), ring.cuda()      # (-inf where nothing is visible)
+        a = ops._score_args(q_dev, k_dev, score, softmax_scale=None, **where)
+        a.d_lse, a.n_parts = lses.data_ptr(), parts
+        _lib.check(_lib.load().infllm_local_score(a, ops._stream()), "infllm_local_score")
+    else:
+        ops.local_score(q.cuda(), ring.cuda(), torch.where(torch.isfinite(lse32), lse32, math.inf).cuda(), score, **where)
     got = score.cpu()
     other = torch.ones(cap, dtype=torch.bool)
     other[rows] = False
