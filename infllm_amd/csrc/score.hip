@@ -3,13 +3,16 @@
 // that InfLLM accumulates per token to choose representative keys
 // (inf_llm/attention/context_manager.py:623-625).
 //
-// It needs the final log-sum-exp of every query, so it runs after the merge and
-// recomputes Q.K^T.  Orientation: S[query, key] with keys in the MFMA column, so a lane
-// owns one key and the column sum is a running per-lane scalar.  A workgroup owns 256
-// consecutive keys of one query head: each of its 4 waves keeps 64 keys in registers
-// (B operand) for the whole kernel, while tiles of 64 or 128 queries stream through LDS
-// (A operand, shared by the 4 waves, double buffered).  Exactly one lane writes each
-// (head, key) cell, so results are deterministic.
+// It needs the final log-sum-exp of every query, so it runs after the merge, or joins the partial ones itself, and
+// recomputes Q.K^T.  Orientation: S[query, key] with keys in the MFMA column, so a lane owns one key (or two) and the
+// column sum is a running per-lane scalar.  A workgroup of four waves owns 128 or 256 consecutive keys of one query
+// head, 32 or 64 of them in a wave's registers (B operand) for the whole kernel, while the queries stream through
+// LDS (A operand, shared by the waves).  Exactly one lane writes each (head, key) cell, so results are deterministic.
+//
+// key_sums is that loop: three workgroups a CU, queries from memory straight into LDS, positions in 32 bits.  It is in
+// scores_kernel (a launch of scores, with or without the merge) and in block_end_kernel (what ends a block).  score_tile is
+// the general form behind it (local_score_kernel): two workgroups a CU, queries by way of registers, any number of partial
+// log-sum-exps, positions in 64 bits.
 #include "carve.h"
 #include "rank.h"
 #include <algorithm>
@@ -21,10 +24,6 @@ namespace {
 template <int D>
 constexpr int kQPad = D + 8;               // LDS row of Q (bf16 elements): 272 (144) bytes rotates the banks
 
-// KS = 32-key halves per wave: 2 for long key ranges; 1 halves the work of a wave per query stage, which is what
-// bounds the short launches that sit on the critical path between two blocks.  QS = queries per LDS stage: a short
-// launch is a chain of stages that each wait for one global load (there is next to no arithmetic to hide it behind),
-// so it takes stages of 128 queries and half as many of them.
 struct ScoreMerge {
     MergeJob job;
     int32_t score_tiles;               // blockIdx.y below this scores, from there on merges
@@ -47,7 +46,10 @@ __device__ __forceinline__ int tile_of_slot(const infllm_score_args &a, int slot
 
 // The general form, for partial log-sum-exps in any number and rings or rows that 32 bits do not address (the others:
 // scores_kernel).  One workgroup of 256 threads: tile `slot` (in the order they are dispatched) of n_tiles of the keys, query
-// head bx.
+// head bx.  KS = 32-key halves per wave: 2 for long key ranges; 1 halves the work of a wave per query stage, which is what
+// bounds the short launches that sit on the critical path between two blocks.  QS = queries per LDS stage: a short
+// launch is a chain of stages that each wait for one global load (there is next to no arithmetic to hide it behind),
+// so it takes stages of 128 queries and half as many of them.
 template <int D, int KS, int QS>
 __device__ __forceinline__ void score_tile(const infllm_score_args &a, const PartSets lps, int bx, int slot, int n_tiles, char *score_lds) {
     constexpr int kWaveKeys = 32 * KS, kKeysPerWg = 4 * kWaveKeys, kQStage = QS;
