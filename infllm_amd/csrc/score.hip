@@ -27,6 +27,7 @@ constexpr int kQPad = D + 8;               // LDS row of Q (bf16 elements): 272 
 struct ScoreMerge {
     MergeJob job;
     int32_t score_tiles;               // blockIdx.y below this scores, from there on merges
+    float empty;                       // see key_sums
 };
 struct NoScoreMerge {};
 
@@ -299,7 +300,9 @@ struct BlockEnd {
 // the wave get them).  The keys are those from position jg on, of which [lo, hi) count; key r of them lies in row slot + r of the
 // ring, or a ring's length before.  A key is visible at distances [first, beyond) of a query.  JOIN: the log-sum-exps are
 // joined from partial ones (at a.d_lse + lps), of all queries before the first stage; else they are finished (a.d_lse) and
-// come with a stage's queries.
+// come with a stage's queries.  `empty` stands for the sum of a query whose partial ones are all empty: one that sees nothing, or
+// whose logits are no numbers.  +infinity leaves those out; -infinity, what a finished sum holds then, makes the scores of all keys
+// that such a query sees infinite or NaN.
 //
 // A wave's exponentials and MFMAs overlap (half a sub-tile of 32 queries apart), so the loop runs at the rate of the vector unit
 // (768 cycles of a sub-tile of 32 queries x 64 keys); what is left is a launch of one or two rounds of workgroups whose first 7
@@ -314,7 +317,7 @@ constexpr size_t kQBytes = (size_t)3 * kQRows * D * sizeof(bf16_t);
 
 template <int D, int KS, bool JOIN>
 __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartSets lps, int b, int h, int64_t jg, int slot, int cap, int lo, int hi, int first,
-                                         int beyond, char *lds, float (&sums)[KS]) {
+                                         int beyond, float empty, char *lds, float (&sums)[KS]) {
     constexpr int kWaveKeys = 32 * KS, kRow = D * 2, kStage = kQRows * kRow;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 31, grp = lane >> 5;
     b = __builtin_amdgcn_readfirstlane(b), h = __builtin_amdgcn_readfirstlane(h), slot = __builtin_amdgcn_readfirstlane(slot);
@@ -379,7 +382,7 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
 #pragma unroll
                     for (int p = 0; p < 8; ++p) den += __builtin_amdgcn_exp2f(l8[e][p] - m8);
                 }
-                if (i0 + e * 256 < padded) Ls[i0 + e * 256] = den > 0.f ? m8 + log2f(den) : INFINITY;      // +inf => probability 0
+                if (i0 + e * 256 < padded) Ls[i0 + e * 256] = den > 0.f ? m8 + log2f(den) : empty;
             }
         }
         __syncthreads();
@@ -487,6 +490,7 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void scores_kernel(infllm_s
     constexpr int kKeys = 128 * KS;
     int n_tiles = gridDim.y;
     PartSets lps{};
+    float empty = 0.f;
     if constexpr (MERGE) {
         n_tiles = sm.score_tiles;
         if ((int)blockIdx.y >= n_tiles) {
@@ -494,6 +498,7 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void scores_kernel(infllm_s
             return;
         }
         lps = sm.job.ps;
+        empty = sm.empty;
     }
     int b, h;
     head_of(a, blockIdx.x, b, h);
@@ -501,7 +506,7 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void scores_kernel(infllm_s
     const int64_t jg = a.j_lo / (32 * KS) * (32 * KS) + (int64_t)tile * kKeys;
     const int lo = (int)max(a.j_lo - jg, (int64_t)0), hi = (int)min(a.j_hi - jg, (int64_t)kKeys);
     float sums[KS];
-    key_sums<D, KS, MERGE>(a, lps, b, h, jg, slot0 + tile * kKeys, cap, lo, hi, first, beyond, score_lds, sums);
+    key_sums<D, KS, MERGE>(a, lps, b, h, jg, slot0 + tile * kKeys, cap, lo, hi, first, beyond, empty, score_lds, sums);
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -527,7 +532,7 @@ __device__ __forceinline__ void carve_unit(const BlockEnd &j, int h, int u, int 
     const int own_row = wave * 32 + col;
     const float track = own_row < bs ? a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + slot_of(own_row)] : 0.f;
     float sum[1];
-    key_sums<D, 1, true>(a, j.merge.ps, b, h, j.t0 + (int64_t)u * bs, slot, j.cap, 0, bs, 0, j.win, lds, sum);
+    key_sums<D, 1, true>(a, j.merge.ps, b, h, j.t0 + (int64_t)u * bs, slot, j.cap, 0, bs, 0, j.win, INFINITY, lds, sum);
     __syncthreads();                                             // (the queries' place is free)
     uint64_t *rank_key = (uint64_t *)lds;
     int32_t *chosen = (int32_t *)(rank_key + kCarveMaxUnit);
@@ -601,7 +606,7 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(Block
         const int slot = j.slot0 + tile * kKeys;
         const int lo = (int)max(a.j_lo - jg, (int64_t)0), hi = (int)min(a.j_hi - jg, (int64_t)kKeys);
         float sums[KS];
-        key_sums<D, KS, true>(a, j.merge.ps, b, h, jg, slot, j.cap, lo, hi, 0, j.win, score_lds, sums);
+        key_sums<D, KS, true>(a, j.merge.ps, b, h, jg, slot, j.cap, lo, hi, 0, j.win, INFINITY, score_lds, sums);
         const int lane = threadIdx.x & 63;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
@@ -678,7 +683,7 @@ inline bool in_reach(const infllm_score_args &a) {
 
 // job: the log-sum-exps are to be joined (a.n_parts of them), and its merge goes along
 template <int D, bool MERGE>
-int scores_launch(const infllm_score_args &a, const MergeJob *job, void *stream) {
+int scores_launch(const infllm_score_args &a, const MergeJob *job, float empty, void *stream) {
     const bool wide = wide_waves(a);
     const int wave_keys = wide ? 64 : 32, gx = a.B * a.H;
     const int64_t tiles = (a.j_hi - 1) / wave_keys - a.j_lo / wave_keys + 1, window = std::min(std::max(a.window, -kMaxRows), kMaxRows);
@@ -688,7 +693,7 @@ int scores_launch(const infllm_score_args &a, const MergeJob *job, void *stream)
     int rows = (int)((tiles + 3) / 4);
     const auto kern = wide ? scores_kernel<D, 2, MERGE> : scores_kernel<D, 1, MERGE>;
     if constexpr (MERGE) {
-        const ScoreMerge sm{*job, rows};
+        const ScoreMerge sm{*job, rows, empty};
         rows += (int)((((int64_t)job->B * job->H * job->Lq * (D / 8) + 255) / 256 + gx - 1) / gx);
         INFLLM_REQUIRE(rows <= 65535, "local_score: %d rows of workgroups", rows);
         hipLaunchKernelGGL(kern, dim3(gx, rows), dim3(256), kQBytes<D> + (size_t)(a.Lq + kQRows - 1) / kQRows * kQRows * sizeof(float), (hipStream_t)stream, a, slot0,
@@ -704,7 +709,7 @@ int score_launch(const infllm_score_args *a, void *stream) {
     int rc = check_score_args(a);
     if (rc) return rc;
     if (a->j_hi <= a->j_lo) return 0;
-    if (a->n_parts <= 0 && in_reach(*a)) return scores_launch<D, false>(*a, nullptr, stream);
+    if (a->n_parts <= 0 && in_reach(*a)) return scores_launch<D, false>(*a, nullptr, 0.f, stream);
     rc = score_lds_setup<D>();
     if (rc) return rc;
     const bool wide = wide_waves(*a);
@@ -716,7 +721,7 @@ int score_launch(const infllm_score_args *a, void *stream) {
 }
 
 template <int D>
-int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *stream) {
+int score_launch_merged(const infllm_score_args *a, const MergeJob *job, float empty, void *stream) {
     INFLLM_REQUIRE(a && job, "local_score_merged: null argument");
     INFLLM_REQUIRE(job->B == a->B && job->H == a->H && job->Lq == a->Lq && job->P >= 1 && job->P <= 8,
                    "local_score_merged: the merge does not belong to these queries");
@@ -726,7 +731,7 @@ int score_launch_merged(const infllm_score_args *a, const MergeJob *job, void *s
     const int rc = check_score_args(&sc);
     if (rc) return rc;
     if (sc.j_hi - sc.j_lo <= 1024 || sc.Lq > kMergedMaxLq || !in_reach(sc)) return 1;
-    return scores_launch<D, true>(sc, job, stream);
+    return scores_launch<D, true>(sc, job, empty, stream);
 }
 
 }  // namespace
@@ -828,7 +833,7 @@ int infllm_local_score_dim(const infllm_score_args *a, int32_t dim, void *stream
 // returns 1, with nothing launched, where the one-launch form does not apply (short key ranges).
 int infllm_local_score_merged(const infllm_score_args *a, const MergeJob *job, void *stream, int32_t dim) {
     INFLLM_REQUIRE(dim == 128 || dim == 64, "local_score: head_dim %d", dim);
-    return dim == 128 ? score_launch_merged<128>(a, job, stream) : score_launch_merged<64>(a, job, stream);
+    return dim == 128 ? score_launch_merged<128>(a, job, INFINITY, stream) : score_launch_merged<64>(a, job, INFINITY, stream);
 }
 
 // ... for the operator: scores and the merge over two sets of partials (P1 + P2 <= 8), heads of 128
@@ -840,5 +845,5 @@ extern "C" int infllm_local_score_merge_pair(const infllm_score_args *a, const u
     if (P1 + P2 > 8 || a->j_hi <= a->j_lo) return 1;
     MergeJob job;
     const int rc = infllm_merge_job(d_o_part, d_lse_part, P1, d_o_part2, d_lse_part2, P2, a->B, a->H, a->Lq, d_out, o_sb, o_sh, o_sl, d_lse, &job, kD);
-    return rc ? rc : score_launch_merged<kD>(a, &job, stream);
+    return rc ? rc : score_launch_merged<kD>(a, &job, -INFINITY, stream);
 }

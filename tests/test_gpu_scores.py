@@ -118,5 +118,12 @@ def test_scores_with_the_merge_of_the_partials(H, Hkv, keys, Lq, parts, mask):
     ops.local_score(q, k, want_lse, want, accumulate=False, **where)
     assert torch.equal(out, want_out) and torch.equal(lse, want_lse)
     assert torch.allclose(score, want, rtol=1e-6, atol=0)
+    for lse_part, o_part in zip(lse_parts, o_parts):             # a query whose logits are no numbers: empty sums, rows of NaN
+        lse_part[:, :, :, Lq // 2], o_part[:, :, :, Lq // 2] = -math.inf, math.nan
+    assert ops.merge_sets_and_score(o_parts, lse_parts, out, lse, q, k, score, **where)
+    ops.attn_merge_sets(o_parts, lse_parts, want_out, want_lse)
+    ops.local_score(q, k, want_lse, want, accumulate=False, **where)
+    assert out[:, :, Lq // 2].isnan().all() and torch.allclose(out.float(), want_out.float(), rtol=0, atol=0, equal_nan=True) and torch.equal(lse, want_lse)
+    assert torch.allclose(score, want, rtol=1e-6, atol=0, equal_nan=True) and (mask == "complement" or not score.isfinite().all())
     small = torch.empty((2, H, 1024), device="cuda")
     assert not ops.merge_sets_and_score(o_parts, lse_parts, out, lse, q, k[:, :, :1024], small, **where)       # (too few keys)
