@@ -32,6 +32,14 @@ struct DecodeJob {
     int64_t unit_elems, row_elems, unit_v_off, unit_sh;
     float *logits;                         // optional [B, H, logit_stride]: scaled logits in base 2 (see DecodeSeg)
     int64_t logit_stride;
+    int32_t new_logit;                     // of a step with its rows: where the new key's logit goes (-1: not kept)
+    // Optional: the launch selects the units itself (the one range that has ids, of n_ids units; `ids` is not read): the best of the
+    // n_scores units with scores at unit_scores + b * unit_scores_sb, into ids_out [B, n_ids] too.  The first lead_segs ranges, with the
+    // units among them, belong to the first lead_splits splits, the others to the rest.
+    const float *unit_scores;
+    int64_t unit_scores_sb;
+    int32_t n_scores, lead_segs, lead_splits;
+    int32_t *ids_out;
     // Optional, without logits: the launch joins its splits itself, the finished row of head h goes to out + b * out_sb + h * out_sh.
     bf16_t *out;
     int64_t out_sb, out_sh;
@@ -77,14 +85,17 @@ __device__ __forceinline__ void copy_rows(const RowCopy (&copies)[kCopies], int 
 }
 
 // The rows of the step itself, as they come (DecodeJob's ranges are the rows that were there before, its q is not used): the
-// launch rotates the query to its position and to the angle of the sinks, attends the new key, and leaves the key and the value
-// where the cache has them, with the copies of old rows that the cache needs.
-struct StepRows {
+// launch rotates the query to its position and to the angle of the sinks or units, and attends the new key.
+struct StepQkv {
     const bf16_t *q, *k, *v;               // [B, H, D], [B, Hkv, D]
     int64_t q_sb, q_sh, k_sb, k_sh, v_sb, v_sh;
     int64_t pos, glb_pos;
     const float *inv_freq;
     double distance_scale;
+};
+// ... of the sliding-window and causal types: it also leaves the key and the value where the cache has them, with the copies of
+// old rows that the cache needs.
+struct StepRows : StepQkv {
     bf16_t *dk, *dv, *raw;                 // rotated key, value, key as it is (NULL: nowhere)
     int64_t dk_sb, dk_sh, dv_sb, dv_sh, raw_sb, raw_sh;
     RowCopy copy[kCopies];
@@ -93,4 +104,6 @@ struct StepRows {
 
 int infllm_decode_step(const DecodeJob *job, const StepRows *rows, int32_t dim, void *stream);
 int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int64_t blocks, int32_t max_splits);
+int infllm_decode_memory_step(const DecodeJob *job, const infllm_ingest_args *in, int32_t dim, void *stream);
 int infllm_decode_attn(const DecodeJob *job, int32_t dim, void *stream);
+int infllm_decode_lead_splits(int32_t nsplit, int64_t lead_blocks, int64_t blocks);

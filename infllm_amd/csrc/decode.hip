@@ -17,7 +17,9 @@
 // 32,768 keys x 8 kv heads (134 MB): 648 us with the tile kernel of attn.hip at one split, 33 us here.
 #include "decode.h"
 #include "rope.h"
+#include "select.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -41,11 +43,15 @@ __device__ __forceinline__ void each_head(F &&f) {
 // D: head dimension (128 or 64); NG: query heads handled together (columns of the MFMA; heads beyond the group's last are
 // zero queries whose results are not written)
 //
-// FRONT: the step's rows come as they are (StepRows).  Rotating them in a launch in front cost 5 us on a chain of two, and its
+// Front: the step's rows come as they are (StepQkv).  Rotating them in a launch in front cost 5 us on a chain of two, and its
 // cache writes, copies included, were waited for by an attention that can read the old cache: here every workgroup rotates its
 // heads' queries while its first rows are on their way, the last split attends the new key, and workgroups behind all splits
-// write the cache (stream-llm, one token over 9,000: 25.4 -> 22.7 us; causal, over 8,192: 26.7 -> 24.0).
+// write the cache (stream-llm, one token over 9,000: 25.4 -> 22.7 us; causal, over 8,192: 26.7 -> 24.0).  A step of the streaming memory
+// that selects nothing has the rest of its prologue there (MemoryRows).
 struct NoFront {};
+struct MemoryRows : StepQkv {
+    infllm_ingest_args in;
+};
 template <int D>
 __device__ __forceinline__ void leave_rows(const StepRows &f, int b, int g, float2 *cs) {      // 256 threads
     constexpr int HALF = D / 2, C2 = D / 16;
@@ -70,9 +76,14 @@ __device__ __forceinline__ void leave_rows(const StepRows &f, int b, int g, floa
     if (tid < 2 * C2) *(u32x4 *)(f.dv + (int64_t)b * f.dv_sb + (int64_t)g * f.dv_sh + tid * 8) = v;
 }
 
-template <int D, int NG, bool LOGITS, bool JOIN, bool FRONT = false>
-__global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(DecodeJob j, std::conditional_t<FRONT, StepRows, NoFront> f) {
-    static_assert(!FRONT || JOIN, "a step with its rows joins its splits");
+// SELECT: the units of the job are selected here (DecodeJob), by every workgroup that reads any of them, each for itself.  A launch that
+// selects for all has to hand over inside: scores stored where every XCD sees them, a ticket, and one workgroup's trips to memory
+// while the chip waits.  Here the others attend the window meanwhile, two thirds of the keys, which need no selection.  (Kernels of a
+// step, 32 heads of 128: behind 64K tokens scores with selection 12.5 + attention 13.4 us, so 8.4 + 12.8; behind 512K 17.1 + 12.8,
+// 11.8 + 14.6.  The window attended in the launch of the scores instead, beside the selection there: 18.5 + 9.8 and 25.7 + 9.6.)
+template <int D, int NG, bool LOGITS, bool JOIN, typename Front = NoFront, bool SELECT = false>
+__global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(DecodeJob j, Front f) {
+    constexpr bool FRONT = !std::is_same_v<Front, NoFront>;
     constexpr int KK = D / 32;                     // k-steps of the first MFMA
     constexpr int LPR = D / 8;                     // lanes that hold a value row, 16 bytes each
     constexpr int VL = kDecodeBlock * LPR / 64;    // value loads per block: 4 (D = 128) or 2 (D = 64)
@@ -86,11 +97,20 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     const int col = lane & 15, rg = lane >> 4;
     const int G = j.H / j.Hkv, chunks = (G + NG - 1) / NG;
     const int split = blockIdx.x, g = blockIdx.y / chunks, c = blockIdx.y % chunks, b = blockIdx.z, n_split = gridDim.x;
+    // the ranges that this workgroup's split is one of, and which one of how many
+    const bool lead = SELECT && split < j.lead_splits;
+    const int seg_lo = SELECT && !lead ? j.lead_segs : 0, seg_hi = lead ? j.lead_segs : j.n_seg;
+    const int part = SELECT && !lead ? split - j.lead_splits : split, n_part = !SELECT ? n_split : lead ? j.lead_splits : n_split - j.lead_splits;
     if constexpr (FRONT) {
         if (b >= j.B) {
-            const int x = split + n_split * ((int)blockIdx.y + (int)gridDim.y * (b - j.B)), n_rows = j.B * j.Hkv, at = x - n_rows, bg = at / max(f.pieces, 1);
-            if (at < 0) leave_rows<D>(f, x / j.Hkv, x % j.Hkv, (float2 *)red_room);
-            else if (at < n_rows * f.pieces) copy_rows<D, kStepCopyRows<D>>(f.copy, at - bg * f.pieces, bg / j.Hkv, bg % j.Hkv);
+            const int x = split + n_split * ((int)blockIdx.y + (int)gridDim.y * (b - j.B)), n_rows = j.B * j.Hkv;
+            if constexpr (std::is_same_v<Front, MemoryRows>) {
+                if (x < n_rows) ingest_one<D>(f.in, x / j.Hkv, x % j.Hkv, (float2 *)red_room);
+            } else {
+                const int at = x - n_rows, bg = at / max(f.pieces, 1);
+                if (at < 0) leave_rows<D>(f, x / j.Hkv, x % j.Hkv, (float2 *)red_room);
+                else if (at < n_rows * f.pieces) copy_rows<D, kStepCopyRows<D>>(f.copy, at - bg * f.pieces, bg / j.Hkv, bg % j.Hkv);
+            }
             return;
         }
     }
@@ -100,8 +120,17 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
 
     // ---- the list of blocks: every range rounded up to whole blocks (units: every unit by itself)
     int n_blocks = 0;
-    for (int s = 0; s < j.n_seg; ++s) n_blocks += (j.seg[s].rows + kDecodeBlock - 1) / kDecodeBlock * (j.seg[s].ids ? j.seg[s].n_ids : 1);
-    const int b_lo = (int)((int64_t)n_blocks * split / n_split), b_hi = (int)((int64_t)n_blocks * (split + 1) / n_split);
+    for (int s = seg_lo; s < seg_hi; ++s) n_blocks += (j.seg[s].rows + kDecodeBlock - 1) / kDecodeBlock * (j.seg[s].n_ids > 0 ? j.seg[s].n_ids : 1);
+    const int b_lo = (int)((int64_t)n_blocks * part / n_part), b_hi = (int)((int64_t)n_blocks * (part + 1) / n_part);
+    __shared__ int32_t chosen[SELECT ? kSelectMost : 1];
+    if constexpr (SELECT) {
+        static_assert(sizeof(SelectLds<kDecWaves * kWave>) <= sizeof(red_room));
+        if (lead) {
+            select_units<kDecWaves * kWave>(j.unit_scores + (int64_t)b * j.unit_scores_sb, j.n_scores, j.seg[0].n_ids, chosen, *(SelectLds<kDecWaves * kWave> *)red_room);
+            if (split == 0 && blockIdx.y == 0)
+                for (int i = threadIdx.x; i < j.seg[0].n_ids; i += kDecWaves * kWave) j.ids_out[(int64_t)b * j.seg[0].n_ids + i] = chosen[i];
+        }
+    }
 
     struct Block {
         const bf16_t *k, *v;
@@ -109,17 +138,17 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     };
     auto find = [&](int blk) {                     // wave-uniform
         Block r{nullptr, nullptr, 0, 0, -1};
-        for (int s = 0; s < j.n_seg; ++s) {
+        for (int s = seg_lo; s < seg_hi; ++s) {
             const DecodeSeg &sg = j.seg[s];
-            const int per = (sg.rows + kDecodeBlock - 1) / kDecodeBlock, n = sg.ids ? per * sg.n_ids : per;
+            const int per = (sg.rows + kDecodeBlock - 1) / kDecodeBlock, n = sg.n_ids > 0 ? per * sg.n_ids : per;
             if (blk >= n) {
                 blk -= n;
                 continue;
             }
             r.q = sg.q;
-            if (sg.ids) {
+            if (sg.n_ids > 0) {
                 const int i = blk / per, r0 = (blk - i * per) * kDecodeBlock;
-                const int u = __builtin_amdgcn_readfirstlane(sg.ids[(int64_t)b * sg.n_ids + i]);
+                const int u = __builtin_amdgcn_readfirstlane(SELECT ? chosen[i] : sg.ids[(int64_t)b * sg.n_ids + i]);
                 const int ch = u / j.per_chunk;
                 const bf16_t *base = (const bf16_t *)(uintptr_t)j.chunk[ch] + (int64_t)(u - ch * j.per_chunk) * j.unit_elems + (int64_t)b * j.row_elems +
                                      (int64_t)g * j.unit_sh + (int64_t)r0 * D;
@@ -292,7 +321,7 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
 #pragma unroll
             for (int i = 0; i < VL; ++i) vbuf[0][i] = *(const u32x4 *)row;
             if (q_now != 0) load_q(0);
-            step(Block{nullptr, nullptr, 1, 0, -1}, 0);
+            step(Block{nullptr, nullptr, 1, 0, LOGITS ? j.new_logit : -1}, 0);
         }
     }
 
@@ -419,14 +448,14 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     }
 }
 
-template <int D, bool LOGITS, bool JOIN>
+template <int D, bool LOGITS, bool JOIN, bool SELECT = false>
 int launch(const DecodeJob *job, void *stream) {
     const int G = job->H / job->Hkv;
     const int NG = G >= 3 ? 4 : G;
     const dim3 grid(job->nsplit, job->Hkv * ((G + NG - 1) / NG), job->B);
-    if (NG == 1) hipLaunchKernelGGL((decode_attn_kernel<D, 1, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, NoFront{});
-    else if (NG == 2) hipLaunchKernelGGL((decode_attn_kernel<D, 2, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, NoFront{});
-    else hipLaunchKernelGGL((decode_attn_kernel<D, 4, LOGITS, JOIN>), grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, NoFront{});
+    const auto kern = NG == 1 ? decode_attn_kernel<D, 1, LOGITS, JOIN, NoFront, SELECT> : NG == 2 ? decode_attn_kernel<D, 2, LOGITS, JOIN, NoFront, SELECT>
+                                                                                                  : decode_attn_kernel<D, 4, LOGITS, JOIN, NoFront, SELECT>;
+    hipLaunchKernelGGL(kern, grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, NoFront{});
     INFLLM_CHECK_LAUNCH("decode_attn");
     return 0;
 }
@@ -444,10 +473,28 @@ int launch_step(const DecodeJob *job, const StepRows *rows, void *stream) {
     const int64_t extra = (int64_t)(1 + rows->pieces) * job->Hkv * job->B, planes = (extra + (int64_t)job->nsplit * y - 1) / ((int64_t)job->nsplit * y);
     if (job->B + planes > 65535 || extra >= (1ll << 30)) return 1;
     const dim3 grid(job->nsplit, y, (unsigned)(job->B + planes));
-    const auto kern = NG == 1 ? decode_attn_kernel<D, 1, false, true, true> : NG == 2 ? decode_attn_kernel<D, 2, false, true, true>
-                                                                                  : decode_attn_kernel<D, 4, false, true, true>;
+    const auto kern = NG == 1 ? decode_attn_kernel<D, 1, false, true, StepRows> : NG == 2 ? decode_attn_kernel<D, 2, false, true, StepRows>
+                                                                                  : decode_attn_kernel<D, 4, false, true, StepRows>;
     hipLaunchKernelGGL(kern, grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, *rows);
     INFLLM_CHECK_LAUNCH("decode_step");
+    return 0;
+}
+
+// A step of the streaming memory that selects nothing: all its ranges are known, so its prologue can ride along.
+template <int D>
+int launch_memory_step(const DecodeJob *job, const infllm_ingest_args *in, void *stream) {
+    const int G = job->H / job->Hkv, NG = G >= 3 ? 4 : G;
+    const int y = job->Hkv * ((G + NG - 1) / NG);
+    const int64_t planes = ((int64_t)job->B * job->Hkv + (int64_t)job->nsplit * y - 1) / ((int64_t)job->nsplit * y);
+    INFLLM_REQUIRE(job->B + planes <= 65535, "decode_memory_step: a batch of %d", job->B);
+    MemoryRows rows{};
+    (StepQkv &)rows = StepQkv{(const bf16_t *)in->d_q, (const bf16_t *)in->d_k, (const bf16_t *)in->d_v, in->q_sb, in->q_sh, in->k_sb, in->k_sh, in->v_sb,
+                              in->v_sh, in->pos0, in->glb_pos, in->d_inv_freq, in->distance_scale};
+    rows.in = *in;
+    const auto kern = NG == 1 ? decode_attn_kernel<D, 1, true, false, MemoryRows> : NG == 2 ? decode_attn_kernel<D, 2, true, false, MemoryRows>
+                                                                                            : decode_attn_kernel<D, 4, true, false, MemoryRows>;
+    hipLaunchKernelGGL(kern, dim3(job->nsplit, y, (unsigned)(job->B + planes)), dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, rows);
+    INFLLM_CHECK_LAUNCH("decode_memory_step");
     return 0;
 }
 
@@ -473,7 +520,7 @@ static int check_job(const DecodeJob *job, int32_t dim) {
     for (int s = 0; s < job->n_seg; ++s) {
         const DecodeSeg &sg = job->seg[s];
         INFLLM_REQUIRE(sg.rows >= 0 && (sg.q == 0 || sg.q == 1), "decode_attn: bad range");
-        if (sg.ids) INFLLM_REQUIRE(job->chunk && job->per_chunk > 0 && sg.n_ids >= 0, "decode_attn: units without an arena");
+        if (sg.n_ids > 0) INFLLM_REQUIRE(job->chunk && job->per_chunk > 0 && (sg.ids || job->unit_scores), "decode_attn: units without an arena");
         else INFLLM_REQUIRE(sg.rows == 0 || (sg.k && sg.v), "decode_attn: null range");
     }
     INFLLM_REQUIRE(dim == 128 || dim == 64, "decode_attn: head_dim %d", dim);
@@ -490,11 +537,45 @@ int infllm_decode_step(const DecodeJob *job, const StepRows *rows, int32_t dim, 
     return dim == 128 ? launch_step<128>(job, rows, stream) : launch_step<64>(job, rows, stream);
 }
 
+// in: the prologue of the step, as infllm_ingest_dim takes it; the job's ranges leave out its key, job->new_logit is that key's place.
+// (A batch of up to 32,767.)
+int infllm_decode_memory_step(const DecodeJob *job, const infllm_ingest_args *in, int32_t dim, void *stream) {
+    const int rc = check_job(job, dim);
+    if (rc) return rc;
+    INFLLM_REQUIRE(in && in->n == 1 && in->d_q && in->d_k && in->d_v && in->d_inv_freq && in->d_ring_k_raw && in->d_ring_k_rot && in->d_ring_v &&
+                       in->d_ring_score && in->d_q_loc && in->d_q_glb && job->logits, "decode_memory_step: null pointer");
+    INFLLM_REQUIRE(in->B == job->B && in->H == job->H && in->Hkv == job->Hkv && in->pos0 >= 0 && in->ring_cap > 0, "decode_memory_step: bad geometry");
+    INFLLM_REQUIRE((in->q_sl % 8 | in->q_sh % 8 | in->q_sb % 8 | in->k_sl % 8 | in->k_sh % 8 | in->k_sb % 8 | in->v_sl % 8 | in->v_sh % 8 | in->v_sb % 8) == 0,
+                   "decode_memory_step: strides must be multiples of 8 elements (16-byte rows)");
+    return dim == 128 ? launch_memory_step<128>(job, in, stream) : launch_memory_step<64>(job, in, stream);
+}
+
+// How many of a launch's splits the ranges get that wait for a selection (lead_blocks of 16 keys) so that they end with the others:
+// the selection takes about as long as three blocks of a wave (479 units: taken for 1 / 2 / 3 / 6 blocks 15.5 / 13.2 / 12.8 / 13.0 us;
+// 4,096: 17.2 / 14.5 / 14.6 / 14.7).
+int infllm_decode_lead_splits(int32_t nsplit, int64_t lead_blocks, int64_t blocks) {
+    int best = 1;
+    int64_t best_time = INT64_MAX;
+    for (int s = 1; s < nsplit; ++s) {
+        const int64_t lead = kDecWaves * s, rest = kDecWaves * (nsplit - s), time = std::max((lead_blocks + lead - 1) / lead + 3, (blocks + rest - 1) / rest);
+        if (time < best_time) best = s, best_time = time;
+    }
+    return best;
+}
+
 int infllm_decode_attn(const DecodeJob *job, int32_t dim, void *stream) {
     const int rc = check_job(job, dim);
     if (rc) return rc;
     INFLLM_REQUIRE(job->q[0] && job->q[1] && job->n_seg >= 1, "decode_attn: no query or range");
     INFLLM_REQUIRE(!job->out || (!job->logits && job->ticket && ((job->out_sb | job->out_sh) & 7) == 0), "decode_attn: bad output");
+    if (job->unit_scores) {
+        INFLLM_REQUIRE(job->logits && job->ids_out && job->lead_segs >= 1 && job->lead_segs < job->n_seg && job->lead_splits >= 1 && job->lead_splits < job->nsplit,
+                       "decode_attn: bad selection");
+        for (int s = 0; s < job->n_seg; ++s)
+            INFLLM_REQUIRE(s == 0 ? job->seg[s].n_ids >= 1 && job->seg[s].n_ids <= kSelectMost && job->seg[s].n_ids <= job->n_scores : job->seg[s].n_ids == 0,
+                           "decode_attn: the first range, and no other, is that of the units");
+        return dim == 128 ? launch<128, true, false, true>(job, stream) : launch<64, true, false, true>(job, stream);
+    }
     if (job->logits) return dim == 128 ? launch<128, true, false>(job, stream) : launch<64, true, false>(job, stream);
     if (job->out) return dim == 128 ? launch<128, false, true>(job, stream) : launch<64, false, true>(job, stream);
     return dim == 128 ? launch<128, false, false>(job, stream) : launch<64, false, false>(job, stream);

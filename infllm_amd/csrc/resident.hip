@@ -11,7 +11,7 @@
 // A call of several queries: prologue of all its tokens, mean queries, the k best of the units that exist for every
 // block's mean query (one pass), the local stage of all blocks; then per block the global stage, and one launch for merge, local
 // score, the units it carves (representatives, rows into their home) and the ranking for the next block.  A single query (a decode
-// step): prologue with the retrieval, one streaming attention launch over window, units, sinks and remainder, and one that joins
+// step): prologue with the units' scores, one streaming attention launch over window, units, sinks and remainder, and one that joins
 // its splits and adds the probabilities to the window's score track - no second read of the window's keys.
 #include <algorithm>
 #include <atomic>
@@ -47,8 +47,8 @@ int infllm_repr_keys_carve(const float *d_ring_score, const void *d_ring_k_raw, 
 int infllm_gather_rows_pair(const void *d_ring_a, void *d_out_a, const void *d_ring_b, void *d_out_b, int64_t ring_cap, int32_t B,
                             int32_t Hkv, int64_t t0, int32_t n, int32_t unit_rows, int64_t out_sb, int64_t out_su, int64_t out_sh,
                             void *stream, int32_t dim);
-int infllm_retrieve_step(const void *d_reps, int64_t rep_stride, int32_t N, const infllm_ingest_args *in, int32_t dim, int32_t b, bool prologue, int32_t k,
-                         float *d_scores, int32_t *d_idx, uint32_t *d_ticket, void *stream);
+int infllm_step_scores(const void *d_reps, int64_t rep_stride, int32_t N, const infllm_ingest_args *in, int32_t dim, int32_t b, bool prologue, float *d_scores,
+                       void *stream);
 int infllm_key_splits(const infllm_layer_desc *d, int32_t n_queries, int32_t n_tiles);
 
 namespace {
@@ -396,80 +396,97 @@ int carve(Resident *R, const infllm_resident_call *a, const Carve &c, hipStream_
     return rc;
 }
 
-// one query
+// One query.  A step that selects takes the scores of all units, with the prologue, then the attention, which selects, then the end
+// of the step; a step that attends all units has the prologue with the attention (two launches for three: 4 us of a prompt of 1,999
+// tokens, whose last token is one).
 int decode_step(Resident *R, const infllm_resident_call *a, int64_t st0, hipStream_t st) {
     const infllm_resident_desc &d = R->d;
     const int C = d.H * d.dim, N = R->n_units, B = d.B;
     const int64_t b0 = R->length, b1 = b0 + 1;
-    infllm_ingest_args in = ingest_args(R, a, st0, 1);
+    const infllm_ingest_args in = ingest_args(R, a, st0, 1);
     const bool retrieve = N > d.topk;
     const int n_sel = std::min(N, d.topk);
-    const int32_t *ids = d.d_iota;
+    DecodeJob j{};
+    j.q[0] = (const bf16_t *)a->d_q_loc; j.q[1] = (const bf16_t *)a->d_q_glb;
+    j.q_sb = C; j.q_sh = d.dim;
+    j.B = B; j.H = d.H; j.Hkv = d.Hkv;
+    j.scale = d.softmax_scale;
+    j.nsplit = (int32_t)std::min<int64_t>(64, a->part_rows / ((int64_t)B * d.H));
     FinishJob f{};
-    int rc = 1;
+    int rc = 0;
+    bool selects = false;                                        // the attention does, from scores
     if (retrieve) {
         int32_t slot = 0;
         rc = take_slot(R, &slot, &f.seq);
         if (rc) return rc;
         f.log = d.d_log + (int64_t)slot * (B * d.topk + 1);
         f.ids = d.d_ids; f.n_ids = B * d.topk;
-        ids = d.d_ids;
-        for (int u = 0; u < B; ++u) {                            // the prologue rides with the first row's retrieval
-            rc = infllm_retrieve_step((const bf16_t *)a->d_reps + (int64_t)u * a->rep_sb, a->rep_su, N, &in, d.dim, u, u == 0, d.topk,
-                                      a->d_unit_scores + (int64_t)u * a->unit_scores_sb, d.d_ids + (int64_t)u * d.topk, a->d_ticket, st);
+        selects = j.nsplit >= 2;
+        for (int u = 0; u < B && selects; ++u) {                  // the prologue rides with the first row's scores
+            rc = infllm_step_scores((const bf16_t *)a->d_reps + (int64_t)u * a->rep_sb, a->rep_su, N, &in, d.dim, u, u == 0,
+                                    a->d_unit_scores + (int64_t)u * a->unit_scores_sb, st);
             if (rc < 0) return rc;
-            if (rc == 1) break;                                  // (of all rows or of none: it depends on their length and number)
+            if (rc == 1) selects = false;                         // (of all rows or of none: it depends on their length and number)
         }
-    }
-    if (rc == 1) {
-        rc = infllm_ingest_dim(&in, d.dim, retrieve ? a->d_qbar : nullptr, st);
-        for (int u = 0; u < B && retrieve && !rc; ++u) {
-            const bf16_t *reps = (const bf16_t *)a->d_reps + (int64_t)u * a->rep_sb;
-            float *scores = a->d_unit_scores + (int64_t)u * a->unit_scores_sb;
-            rc = infllm_unit_scores(reps, a->rep_su, 0, N, C, a->d_qbar + (int64_t)u * C, scores, st);
-            if (!rc) rc = infllm_topk(scores, N, d.topk, d.d_ids + (int64_t)u * d.topk, st);
+        if (!selects) {
+            rc = infllm_ingest_dim(&in, d.dim, a->d_qbar, st);
+            for (int u = 0; u < B && !rc; ++u) {
+                const bf16_t *reps = (const bf16_t *)a->d_reps + (int64_t)u * a->rep_sb;
+                float *scores = a->d_unit_scores + (int64_t)u * a->unit_scores_sb;
+                rc = infllm_unit_scores(reps, a->rep_su, 0, N, C, a->d_qbar + (int64_t)u * C, scores, st);
+                if (!rc) rc = infllm_topk(scores, N, d.topk, d.d_ids + (int64_t)u * d.topk, st);
+            }
+            if (rc) return rc;
         }
+    } else
+        R->queue.push_back(Resident::Entry{n_sel, 0, 0});
+    const bool rides = !retrieve && B <= 32767;                  // the prologue with the attention (whose grid holds 65,535 batch rows)
+    if (!retrieve && !rides) {
+        rc = infllm_ingest_dim(&in, d.dim, nullptr, st);
         if (rc) return rc;
     }
-    if (!retrieve)
-        R->queue.push_back(Resident::Entry{n_sel, 0, 0});
-    DecodeJob j{};
-    j.q[0] = (const bf16_t *)a->d_q_loc; j.q[1] = (const bf16_t *)a->d_q_glb;
-    j.q_sb = C; j.q_sh = d.dim;
-    j.B = B; j.H = d.H; j.Hkv = d.Hkv;
-    j.scale = d.softmax_scale;
     int64_t blocks = 0;
-    auto seg = [&](const void *k, const void *v, int64_t sb, int64_t sh, int64_t vsb, int64_t vsh, int64_t rows, int q, int logit0) {
-        j.seg[j.n_seg++] = DecodeSeg{(const bf16_t *)k, (const bf16_t *)v, sb, sh, vsb, vsh, (int32_t)rows, q, 0, nullptr, logit0};
+    auto seg = [&](const void *k, const void *v, int64_t sb, int64_t sh, int64_t rows, int q, int logit0) {
+        j.seg[j.n_seg++] = DecodeSeg{(const bf16_t *)k, (const bf16_t *)v, sb, sh, sb, sh, (int32_t)rows, q, 0, nullptr, logit0};
         blocks += (rows + kDecodeBlock - 1) / kDecodeBlock;
     };
     const int64_t ring_sh = d.ring_cap * d.dim, ring_sb = d.Hkv * ring_sh;
     auto ring = [&](const void *k, int64_t lo, int64_t hi, int q, bool logits) {
         for (int64_t pos = lo; pos < hi;) {
             const int64_t row = pos % d.ring_cap, n = std::min(hi - pos, d.ring_cap - row);
-            seg((const bf16_t *)k + row * d.dim, (const bf16_t *)d.d_ring_v + row * d.dim, ring_sb, ring_sh, ring_sb, ring_sh, n, q, logits ? (int)(pos - lo) : -1);
+            seg((const bf16_t *)k + row * d.dim, (const bf16_t *)d.d_ring_v + row * d.dim, ring_sb, ring_sh, n, q, logits ? (int)(pos - lo) : -1);
             pos += n;
         }
     };
-    const int64_t j_lo = std::max<int64_t>(0, b1 - d.n_local);
-    ring(d.d_ring_k_rot, j_lo, b1, 0, true);
     if (n_sel > 0) {
         DecodeSeg &sg = j.seg[j.n_seg++];
         sg = DecodeSeg{};
-        sg.rows = d.block_size; sg.q = 1; sg.n_ids = n_sel; sg.ids = ids; sg.logit0 = -1;
+        sg.rows = d.block_size; sg.q = 1; sg.n_ids = n_sel; sg.ids = retrieve ? d.d_ids : d.d_iota; sg.logit0 = -1;
         blocks += (int64_t)n_sel * ((d.block_size + kDecodeBlock - 1) / kDecodeBlock);
         j.chunk = a->d_chunks; j.per_chunk = d.units_per_chunk;
         j.unit_sh = (int64_t)d.block_size * d.dim; j.unit_v_off = d.Hkv * j.unit_sh; j.row_elems = 2 * j.unit_v_off; j.unit_elems = B * j.row_elems;
     }
     if (R->init_len > 0) {
         const int64_t sh = d.init_cap * d.dim, sb = 2 * d.Hkv * sh;
-        seg(d.d_init_kv, (const bf16_t *)d.d_init_kv + d.Hkv * sh, sb, sh, sb, sh, R->init_len, 1, -1);
+        seg(d.d_init_kv, (const bf16_t *)d.d_init_kv + d.Hkv * sh, sb, sh, R->init_len, 1, -1);
     }
     ring(d.d_ring_k_raw, R->cursor, std::max(b1 - d.n_local, R->cursor), 1, false);
-    j.nsplit = infllm_decode_splits(B, d.H, d.Hkv, blocks, (int32_t)std::min<int64_t>(64, a->part_rows / ((int64_t)B * d.H)));
+    const int64_t far_blocks = blocks, j_lo = std::max<int64_t>(0, b1 - d.n_local);
+    const int far_segs = j.n_seg;
+    j.new_logit = (int32_t)(b0 - j_lo);
+    ring(d.d_ring_k_rot, j_lo, rides ? b0 : b1, 0, true);
+    j.nsplit = infllm_decode_splits(B, d.H, d.Hkv, blocks, j.nsplit);
     j.o_part = a->d_o_part; j.lse_part = a->d_lse_part;
     j.logits = a->d_logits; j.logit_stride = d.n_local;
-    rc = infllm_decode_attn(&j, d.dim, st);
+    if (selects) {
+        j.nsplit = std::max(j.nsplit, 2);
+        j.unit_scores = a->d_unit_scores; j.unit_scores_sb = a->unit_scores_sb;
+        j.n_scores = N;
+        j.lead_segs = far_segs;
+        j.lead_splits = infllm_decode_lead_splits(j.nsplit, far_blocks, blocks - far_blocks);
+        j.ids_out = d.d_ids;
+    }
+    rc = rides ? infllm_decode_memory_step(&j, &in, d.dim, st) : infllm_decode_attn(&j, d.dim, st);
     if (rc) return rc;
     f.o_part = (const _Float16 *)a->d_o_part; f.lse_part = a->d_lse_part;
     f.P = j.nsplit; f.B = B; f.H = d.H;

@@ -565,13 +565,14 @@ __device__ __forceinline__ void select_topk_block(const float *scores, int N, in
     }
 }
 
-// A decode step's retrieval takes the step's prologue along (FRONT).  The mean of one query is the query itself, rotated to the
-// angle that all units are seen under: every retrieving workgroup rotates it anew, while its rows of representatives are on their
+// A decode step's scores take the step's prologue along (FRONT).  The mean of one query is the query itself, rotated to the
+// angle that all units are seen under: every scoring workgroup rotates it anew, while its rows of representatives are on their
 // way, and workgroups of their own behind them do the rest of the prologue, which only the attention needs.  A launch less on a
-// chain of four (one token behind 64K tokens 33.3 -> 30.2 us, behind 512K 39.3 -> 34.4).
+// chain of four (one token behind 64K tokens 33.3 -> 30.2 us, behind 512K 39.3 -> 34.4).  The selection is the attention's
+// (decode.hip): the launch ends with its scores.
 struct StepFront {
     infllm_ingest_args in;             // one new position
-    int32_t dim, b, n_retrieve;        // whose query (batch row) the retrieval is for; workgroups that retrieve
+    int32_t dim, b, n_retrieve;        // whose query (batch row) the scores are for; workgroups that score
 };
 struct NoFront {};
 
@@ -663,10 +664,14 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
                 for (int j = 0; j < CPL; ++j) w[r][j] = in_row(j) ? __builtin_nontemporal_load((const u32x4 *)(row + j * 512)) : u32x4{0, 0, 0, 0};
             }
             const float acc = wave_sum(acc0 + acc1);
-            if (lane == 0) __hip_atomic_store(scores + cur, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (lane == 0) {
+                if constexpr (FRONT) scores[cur] = acc;
+                else __hip_atomic_store(scores + cur, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
         }
         n += ROWS * n_waves;
     }
+    if constexpr (FRONT) return;
     // every wave's score stores have been performed before the workgroup takes its ticket
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -1118,10 +1123,10 @@ extern "C" int infllm_score_topk_queries(const void *d_reps, int64_t rep_stride,
 // ticket: the caller's word, or NULL and slot >= 0: the library's word there; neither: returns 1.
 static int retrieve_launch(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar, int32_t k, float *d_scores, int32_t *d_idx,
                            int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, const StepFront *front, bool whole_front, uint32_t *ticket, int slot, void *stream) {
-    INFLLM_REQUIRE(d_reps && (d_qbar || front) && d_scores && d_idx, "retrieve: null pointer");
+    INFLLM_REQUIRE(d_reps && (d_qbar || front) && d_scores && (d_idx || front), "retrieve: null pointer");
     INFLLM_REQUIRE(N > 0 && k > 0 && k <= N, "retrieve: k=%d with N=%d", k, N);
     INFLLM_REQUIRE(rep_stride >= C && rep_stride % 8 == 0, "retrieve: row stride %lld", (long long)rep_stride);
-    if (N > 16384 || k > 64 || C % 8 != 0 || C > 9 * 512 || (!ticket && slot < 0)) return 1;
+    if (N > 16384 || k > 64 || C % 8 != 0 || C > 9 * 512 || (!front && !ticket && slot < 0)) return 1;
     constexpr int waves_per_wg = kRetrThreads / 64;
     const bool deep = N >= 4096;
     const int per_wg = waves_per_wg * (deep ? 2 : 1);
@@ -1163,22 +1168,22 @@ int infllm_retrieve_fused(const void *d_reps, int64_t rep_stride, int32_t N, int
     return retrieve_launch(d_reps, rep_stride, N, C, d_qbar, k, d_scores, d_idx, d_idx2, d_flag, flag_value, nullptr, false, d_ticket, -1, stream);
 }
 
-// library-internal: the same for the one query of a decode step, batch row b of `in` (whose d_qpart is not used); with `prologue`
-// the launch also does what infllm_ingest_dim does for the step, for all batch rows
-int infllm_retrieve_step(const void *d_reps, int64_t rep_stride, int32_t N, const infllm_ingest_args *in, int32_t dim, int32_t b, bool prologue, int32_t k,
-                         float *d_scores, int32_t *d_idx, uint32_t *d_ticket, void *stream) {
+// library-internal: the scores alone, under the one query of a decode step, batch row b of `in` (whose d_qpart is not used); with
+// `prologue` the launch also does what infllm_ingest_dim does for the step, for all batch rows
+int infllm_step_scores(const void *d_reps, int64_t rep_stride, int32_t N, const infllm_ingest_args *in, int32_t dim, int32_t b, bool prologue, float *d_scores,
+                       void *stream) {
     INFLLM_REQUIRE(in && in->n == 1 && in->d_q && in->d_k && in->d_v && in->d_inv_freq && in->d_ring_k_raw && in->d_ring_k_rot && in->d_ring_v &&
-                       in->d_ring_score && in->d_q_loc && in->d_q_glb, "retrieve_step: null pointer");
+                       in->d_ring_score && in->d_q_loc && in->d_q_glb, "step_scores: null pointer");
     INFLLM_REQUIRE(in->B > 0 && in->H > 0 && in->Hkv > 0 && in->H % in->Hkv == 0 && in->pos0 >= 0 && in->ring_cap > 0 && b >= 0 && b < in->B,
-                   "retrieve_step: bad geometry B=%d H=%d Hkv=%d", in->B, in->H, in->Hkv);
+                   "step_scores: bad geometry B=%d H=%d Hkv=%d", in->B, in->H, in->Hkv);
     INFLLM_REQUIRE((in->q_sl % 8 | in->q_sh % 8 | in->q_sb % 8 | in->k_sl % 8 | in->k_sh % 8 | in->k_sb % 8 | in->v_sl % 8 | in->v_sh % 8 | in->v_sb % 8) == 0,
-                   "retrieve_step: strides must be multiples of 8 elements (16-byte rows)");
-    INFLLM_REQUIRE(dim == 128 || dim == 64, "retrieve_step: head_dim %d", dim);
+                   "step_scores: strides must be multiples of 8 elements (16-byte rows)");
+    INFLLM_REQUIRE(dim == 128 || dim == 64, "step_scores: head_dim %d", dim);
     StepFront f{};
     f.in = *in;
     f.dim = dim;
     f.b = b;
-    return retrieve_launch(d_reps, rep_stride, N, in->H * dim, nullptr, k, d_scores, d_idx, nullptr, nullptr, 0, &f, prologue, d_ticket, -1, stream);
+    return retrieve_launch(d_reps, rep_stride, N, in->H * dim, nullptr, 1, d_scores, nullptr, nullptr, nullptr, 0, &f, prologue, nullptr, -1, stream);
 }
 
 extern "C" int infllm_score_topk(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar,
