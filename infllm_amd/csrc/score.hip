@@ -311,43 +311,48 @@ struct BlockEnd {
 // straight into LDS (64 rows a stage, three stages in turn, no registers on the way), and a wave's two accumulators are the halves
 // of a sub-tile instead of two sub-tiles.  With half a CU each (score_tile, and carving workgroups with a loop of their own):
 // prompts of 131,072 / 16,001 tokens 27,000 -> 26,000 / 2,816 -> 2,726 us, of 24,300 with 36 heads of 64 3,185 -> 3,136.
+//
+// QR queries a stage, NB stages in LDS; QG groups of four waves hold the same keys and share a stage's queries (see paired_waves).
 constexpr int kQRows = 64;                             // queries of a stage
 template <int D>
 constexpr size_t kQBytes = (size_t)3 * kQRows * D * sizeof(bf16_t);
 
-template <int D, int KS, bool JOIN>
+template <int D, int KS, bool JOIN, int QR = kQRows, int NB = 3, int QG = 1>
 __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartSets lps, int b, int h, int64_t jg, int slot, int cap, int lo, int hi, int first,
                                          int beyond, float empty, char *lds, float (&sums)[KS]) {
-    constexpr int kWaveKeys = 32 * KS, kRow = D * 2, kStage = kQRows * kRow;
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 31, grp = lane >> 5;
+    constexpr int kWaveKeys = 32 * KS, kRow = D * 2, kStage = QR * kRow;
+    constexpr int kThreads = 256 * QG, kOwn = QR / QG;             // of a stage's queries those that are a group's
+    const int tid = threadIdx.x, any_wave = __builtin_amdgcn_readfirstlane(tid >> 6), wave = any_wave & 3, group = any_wave >> 2;
+    const int lane = tid & 63, col = lane & 31, grp = lane >> 5;
     b = __builtin_amdgcn_readfirstlane(b), h = __builtin_amdgcn_readfirstlane(h), slot = __builtin_amdgcn_readfirstlane(slot);
     lo = __builtin_amdgcn_readfirstlane(lo), hi = __builtin_amdgcn_readfirstlane(hi);
     const int g = __builtin_amdgcn_readfirstlane(h / (a.H / a.Hkv)), Lq = a.Lq;
     const float scale = a.softmax_scale * 1.4426950408889634f;
-    float *Ls = (float *)(lds + kQBytes<D>);                       // JOIN: [Lq rounded up to a stage]; else [3][kQRows]
+    float *Ls = (float *)(lds + NB * kStage);                       // JOIN: [Lq rounded up to a stage]; else [NB][QR]
     // a key's distance to query q is q + d - its place among the keys
     const int d = (int)min(max(a.offset - jg, (int64_t)-(1 << 29)), (int64_t)(1 << 29));
     // queries that see any of the keys, in stages
     const int q_lo = max(lo - d + first, 0), q_hi = (int)min((int64_t)hi - d - 1 + beyond, (int64_t)Lq);
-    const int st_lo = q_lo / kQRows, st_hi = hi > lo && q_hi > q_lo ? (q_hi - 1) / kQRows + 1 : st_lo;
+    const int st_lo = q_lo / QR, st_hi = hi > lo && q_hi > q_lo ? (q_hi - 1) / QR + 1 : st_lo;
 
     // ---- queries into LDS: an instruction fills 1024 bytes; a wave the rows from 16 * wave on
-    constexpr int kRowsPerLd = 1024 / kRow, kLd = kQRows / (4 * kRowsPerLd);
+    constexpr int kRowsPerLd = 1024 / kRow, kLd = QR / (4 * QG * kRowsPerLd);
     const bf16_t *qbase = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh;
     const float *lse = a.d_lse + ((int64_t)b * a.H + h) * Lq;
-    const uint32_t q_lds = lds_address(lds) + wave * (kLd * 1024);
+    const uint32_t q_lds = lds_address(lds) + any_wave * (kLd * 1024);
     auto load_stage = [&](int s, int buf) {
 #pragma unroll
         for (int i = 0; i < kLd; ++i) {
-            const int r = kRowsPerLd * (kLd * wave + i) + lane / (D / 8);                   // (rows behind the last query: the last one's, masked)
-            const int q = min(s * kQRows + r, Lq - 1);
+            const int r = kRowsPerLd * (kLd * any_wave + i) + lane / (D / 8);                   // (rows behind the last query: the last one's, masked)
+            const int q = min(s * QR + r, Lq - 1);
             load_to_lds16(qbase, (uint32_t)((int64_t)q * a.q_sl + ((lane & (D / 8 - 1)) ^ swz<D>(r)) * 8) * 2, q_lds + buf * kStage + i * 1024);
         }
-        if (!JOIN && lane < kQRows / 4)
-            load_to_lds4(lse, (uint32_t)min(s * kQRows + wave * (kQRows / 4) + lane, Lq - 1) * 4, lds_address((char *)(Ls + buf * kQRows + wave * (kQRows / 4))));
+        constexpr int kLse = QR / (4 * QG);
+        if (!JOIN && lane < kLse)
+            load_to_lds4(lse, (uint32_t)min(s * QR + any_wave * kLse + lane, Lq - 1) * 4, lds_address((char *)(Ls + buf * QR + any_wave * kLse)));
     };
     if (st_lo < st_hi) load_stage(st_lo, 0);
-    if (st_lo + 1 < st_hi) load_stage(st_lo + 1, 1);
+    if (NB > 2 && st_lo + 1 < st_hi) load_stage(st_lo + 1, 1);
 
     // ---- this wave's keys as the B operand (lane = key column)
     bf16x8 kreg[KS][D / 16];
@@ -366,13 +371,13 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
     // ---- joined log-sum-exps of all queries, two a thread: one trip to memory for 512
     if constexpr (JOIN) {
         const int64_t all = (int64_t)a.B * a.H * Lq;
-        const int padded = (Lq + kQRows - 1) / kQRows * kQRows;
-        for (int i0 = tid; i0 < padded; i0 += 512) {
+        const int padded = (Lq + QR - 1) / QR * QR;
+        for (int i0 = tid; i0 < padded; i0 += 2 * kThreads) {
             float l8[2][8];
 #pragma unroll
             for (int e = 0; e < 2; ++e)
 #pragma unroll
-                for (int p = 0; p < 8; ++p) l8[e][p] = i0 + e * 256 < Lq && p < a.n_parts ? lse[lps.l(p, all) + i0 + e * 256] : -INFINITY;
+                for (int p = 0; p < 8; ++p) l8[e][p] = i0 + e * kThreads < Lq && p < a.n_parts ? lse[lps.l(p, all) + i0 + e * kThreads] : -INFINITY;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 float m8 = -INFINITY, den = 0.f;
@@ -382,7 +387,7 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
 #pragma unroll
                     for (int p = 0; p < 8; ++p) den += __builtin_amdgcn_exp2f(l8[e][p] - m8);
                 }
-                if (i0 + e * 256 < padded) Ls[i0 + e * 256] = den > 0.f ? m8 + log2f(den) : empty;
+                if (i0 + e * kThreads < padded) Ls[i0 + e * kThreads] = den > 0.f ? m8 + log2f(den) : empty;
             }
         }
         __syncthreads();
@@ -399,16 +404,16 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
     float colsum[KS] = {};
     int buf = 0;
     for (int s = st_lo; s < st_hi; ++s) {
-        // this wave's rows of the stage have landed (those of the next may be on their way), then everyone's; the buffer that
-        // the stage after next takes was read a stage ago
-        if (s + 1 < st_hi) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(JOIN ? kLd : kLd + 1) : "memory");
+        // this wave's rows of the stage have landed (of three buffers, those of the next may be on their way), then everyone's; the
+        // buffer that is requested next was read a stage ago
+        if (NB > 2 && s + 1 < st_hi) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(JOIN ? kLd : kLd + 1) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         asm volatile("s_barrier" ::: "memory");
-        if (s + 2 < st_hi) load_stage(s + 2, buf == 0 ? 2 : buf - 1);
-        const int i0 = s * kQRows;
+        if (s + NB - 1 < st_hi) load_stage(s + NB - 1, buf == 0 ? NB - 1 : buf - 1);
+        const int i0 = s * QR + group * kOwn;                   // this wave's first query of the stage
         auto stage = [&](auto masked) {
             constexpr bool kMasked = decltype(masked)::value;
-            constexpr int kSteps = kQRows / 32 * KS;            // (sub-tile of 32 queries, 32 keys), keys first
+            constexpr int kSteps = kOwn / 32 * KS;          // (sub-tile of 32 queries, 32 keys), keys first
             int q_first[KS];                                    // the queries that see this lane's keys: q_first .. q_first + q_count - 1
             uint32_t q_count[KS];
             if constexpr (kMasked) {
@@ -421,7 +426,7 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
             }
             f32x16 acc[2];
             bf16x8 qa[D / 16];                                  // A operand: lane = query row
-            const uint32_t q_at = lds_address(lds) + buf * kStage + col * kRow + ((grp ^ swz<D>(col)) * 16);
+            const uint32_t q_at = lds_address(lds) + buf * kStage + (group * kOwn + col) * kRow + ((grp ^ swz<D>(col)) * 16);
             auto issue = [&](int t) {
                 const int qs = t / KS, ks = t % KS;
 #pragma unroll
@@ -440,7 +445,7 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
                 if (t + 1 < kSteps) issue(t + 1);
                 f32x4 l4[4];
 #pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) l4[q4] = *(const f32x4 *)&Ls[(JOIN ? i0 : buf * kQRows) + qs * 32 + 8 * q4 + 4 * grp];
+                for (int q4 = 0; q4 < 4; ++q4) l4[q4] = *(const f32x4 *)&Ls[(JOIN ? i0 : buf * QR + group * kOwn) + qs * 32 + 8 * q4 + 4 * grp];
                 const int from = kMasked ? i0 + qs * 32 + 4 * grp - q_first[ks] : 0;
                 float sum = 0.f;
 #pragma unroll
@@ -462,12 +467,24 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
             }
         };
         // every pair is visible / some are (wave-uniform)
-        if (whole && i0 + kQRows <= Lq && i0 + d - (w_first + kWaveKeys - 1) >= first && i0 + kQRows - 1 + d - w_first < beyond) stage(std::false_type{});
-        else if (w_hi > w_lo && i0 + kQRows - 1 + d - w_lo >= first && i0 + d - (w_hi - 1) < beyond) stage(std::true_type{});
-        buf = buf == 2 ? 0 : buf + 1;
+        if (whole && i0 + kOwn <= Lq && i0 + d - (w_first + kWaveKeys - 1) >= first && i0 + kOwn - 1 + d - w_first < beyond) stage(std::false_type{});
+        else if (w_hi > w_lo && i0 + kOwn - 1 + d - w_lo >= first && i0 + d - (w_hi - 1) < beyond) stage(std::true_type{});
+        buf = buf == NB - 1 ? 0 : buf + 1;
     }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) sums[ks] = colsum[ks] + wave_xor32(colsum[ks]);
+    if constexpr (QG > 1) {                                     // the first group gets the sums of all, in the order of the queries
+        float(*part)[4][KS][64] = (float(*)[4][KS][64])lds;
+        __syncthreads();
+        if (group > 0)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) part[group - 1][wave][ks][lane] = sums[ks];
+        __syncthreads();
+#pragma unroll
+        for (int o = 0; o < QG - 1; ++o)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) sums[ks] += part[o][wave][ks][lane];
+    }
 }
 
 // Heads of different kv heads next to each other, see score_tile.
@@ -483,18 +500,24 @@ __device__ __forceinline__ void head_of(const infllm_score_args &a, int bx, int 
 // MERGE: the launch also carries the merge of the partial attention outputs, in workgroups behind the scoring ones, which join the
 // partial log-sum-exps themselves, by the merge's own arithmetic (the operator, whose merge was a launch in front of this one:
 // 101.0 -> 96.8 us).
-template <int D, int KS, bool MERGE>
-__global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void scores_kernel(infllm_score_args a, int slot0, int cap, int first, int beyond,
+struct ScoreForm {
+    int ks, rows, bufs, groups;            // 32-key halves of a wave; queries of a stage, stages in LDS, groups of waves that share one
+};
+enum { kWide = 0, kNarrow = 1, kPaired = 2 };
+constexpr ScoreForm kScoreForms[3] = {{2, 64, 3, 1}, {1, 64, 3, 1}, {1, 128, 2, 2}};
+template <int D, int FORM, bool MERGE>
+__global__ __launch_bounds__(256 * kScoreForms[FORM].groups, (D == 64 || FORM == kPaired ? 4 : 3)) void scores_kernel(infllm_score_args a, int slot0, int cap, int first, int beyond,
                                                                         std::conditional_t<MERGE, ScoreMerge, NoScoreMerge> sm) {
     extern __shared__ __attribute__((aligned(1024))) char score_lds[];
-    constexpr int kKeys = 128 * KS;
+    constexpr ScoreForm F = kScoreForms[FORM];
+    constexpr int KS = F.ks, kKeys = 128 * KS;
     int n_tiles = gridDim.y;
     PartSets lps{};
     float empty = 0.f;
     if constexpr (MERGE) {
         n_tiles = sm.score_tiles;
         if ((int)blockIdx.y >= n_tiles) {
-            merge_piece<D>(sm.job, ((int64_t)((int)blockIdx.y - n_tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x);
+            merge_piece<D>(sm.job, ((int64_t)((int)blockIdx.y - n_tiles) * gridDim.x + blockIdx.x) * (256 * F.groups) + threadIdx.x);
             return;
         }
         lps = sm.job.ps;
@@ -506,12 +529,12 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void scores_kernel(infllm_s
     const int64_t jg = a.j_lo / (32 * KS) * (32 * KS) + (int64_t)tile * kKeys;
     const int lo = (int)max(a.j_lo - jg, (int64_t)0), hi = (int)min(a.j_hi - jg, (int64_t)kKeys);
     float sums[KS];
-    key_sums<D, KS, MERGE>(a, lps, b, h, jg, slot0 + tile * kKeys, cap, lo, hi, first, beyond, empty, score_lds, sums);
+    key_sums<D, KS, MERGE, F.rows, F.bufs, F.groups>(a, lps, b, h, jg, slot0 + tile * kKeys, cap, lo, hi, first, beyond, empty, score_lds, sums);
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
         const int r = (threadIdx.x >> 6) * (32 * KS) + ks * 32 + lane;
-        if (lane < 32 && r >= lo && r < hi) {
+        if (lane < 32 && r >= lo && r < hi && threadIdx.x < 256) {
             float *dst = a.d_score + (int64_t)b * a.score_sb + (int64_t)h * a.score_sh + (jg + r) % a.score_cap;
             *dst = a.accumulate ? *dst + sums[ks] : sums[ks];
         }
@@ -682,26 +705,55 @@ inline bool in_reach(const infllm_score_args &a) {
 }
 
 // job: the log-sum-exps are to be joined (a.n_parts of them), and its merge goes along
-template <int D, bool MERGE>
+template <int D, int FORM, bool MERGE>
 int scores_launch(const infllm_score_args &a, const MergeJob *job, float empty, void *stream) {
-    const bool wide = wide_waves(a);
-    const int wave_keys = wide ? 64 : 32, gx = a.B * a.H;
+    constexpr ScoreForm F = kScoreForms[FORM];
+    constexpr int wave_keys = 32 * F.ks, threads = 256 * F.groups;
+    constexpr size_t q_bytes = (size_t)F.bufs * F.rows * D * sizeof(bf16_t);
+    const int gx = a.B * a.H;
     const int64_t tiles = (a.j_hi - 1) / wave_keys - a.j_lo / wave_keys + 1, window = std::min(std::max(a.window, -kMaxRows), kMaxRows);
     const int cap = (int)std::min(a.cap, kMaxRows), slot0 = (int)(a.j_lo % a.cap - a.j_lo % wave_keys);      // (below 0: rows that do not count)
     const int first = (int)(a.mask == INFLLM_MASK_WINDOW ? 0 : a.mask == INFLLM_MASK_COMPLEMENT ? window : -kMaxRows);
     const int beyond = (int)(a.mask == INFLLM_MASK_WINDOW ? std::max<int64_t>(window, 0) : kMaxRows);
     int rows = (int)((tiles + 3) / 4);
-    const auto kern = wide ? scores_kernel<D, 2, MERGE> : scores_kernel<D, 1, MERGE>;
+    const auto kern = scores_kernel<D, FORM, MERGE>;
+    constexpr size_t most = q_bytes + (MERGE ? kMergedMaxLq : F.bufs * F.rows) * sizeof(float);
+    if constexpr (most > 65536) {                       // dynamic LDS above 64 KiB must be enabled once per kernel
+        static std::atomic<bool> lds_set{false};
+        if (!lds_set.load(std::memory_order_acquire)) {
+            const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
+            if (e != hipSuccess) return infllm_fail(-2, "local_score: %s", hipGetErrorString(e));
+            lds_set.store(true, std::memory_order_release);
+        }
+    }
     if constexpr (MERGE) {
         const ScoreMerge sm{*job, rows, empty};
-        rows += (int)((((int64_t)job->B * job->H * job->Lq * (D / 8) + 255) / 256 + gx - 1) / gx);
+        rows += (int)((((int64_t)job->B * job->H * job->Lq * (D / 8) + threads - 1) / threads + gx - 1) / gx);
         INFLLM_REQUIRE(rows <= 65535, "local_score: %d rows of workgroups", rows);
-        hipLaunchKernelGGL(kern, dim3(gx, rows), dim3(256), kQBytes<D> + (size_t)(a.Lq + kQRows - 1) / kQRows * kQRows * sizeof(float), (hipStream_t)stream, a, slot0,
+        hipLaunchKernelGGL(kern, dim3(gx, rows), dim3(threads), q_bytes + (size_t)(a.Lq + F.rows - 1) / F.rows * F.rows * sizeof(float), (hipStream_t)stream, a, slot0,
                            cap, first, beyond, sm);
     } else
-        hipLaunchKernelGGL(kern, dim3(gx, rows), dim3(256), kQBytes<D> + 3 * kQRows * sizeof(float), (hipStream_t)stream, a, slot0, cap, first, beyond, NoScoreMerge{});
+        hipLaunchKernelGGL(kern, dim3(gx, rows), dim3(threads), q_bytes + F.bufs * F.rows * sizeof(float), (hipStream_t)stream, a, slot0, cap, first, beyond,
+                           NoScoreMerge{});
     INFLLM_CHECK_LAUNCH("local_score");
     return 0;
+}
+
+// A narrow launch that the chip holds at once at two workgroups a CU (heads of 64: three) lasts as long as its longest workgroup, a
+// chain of stages whose waits and pipeline ends weigh as much as their work: it takes twice the waves a workgroup and twice the
+// queries a stage.  Beyond that the smaller workgroups fill up better, and few queries are no chain.  (Causal, 32 heads of 128: 500 /
+// 1,000 / 1,998 queries 12.1 / 19.5 / 35.0 us, so 10.2 / 15.5 / 28.3; 2,700: 47.6 and 51.4; 200 queries x 2,000 keys 10.6 and 11.1; 36 heads of
+// 64: 1,024 / 2,700 / 3,100 16.8 / 39.0 / 44.7 and 12.9 / 34.8 / 50.1; 8 heads of 128: 3,100 47.8 and 34.9.)
+template <int D>
+inline bool paired_waves(const infllm_score_args &a) {
+    return a.Lq >= 256 && (int64_t)a.B * a.H * (((a.j_hi - 1) / 32 - a.j_lo / 32 + 4) / 4) <= (D == 64 ? 3 : 2) * kScoreCus;
+}
+
+template <int D, bool MERGE>
+int scores_launch(const infllm_score_args &a, const MergeJob *job, float empty, void *stream) {
+    if (wide_waves(a)) return scores_launch<D, kWide, MERGE>(a, job, empty, stream);
+    if (paired_waves<D>(a)) return scores_launch<D, kPaired, MERGE>(a, job, empty, stream);
+    return scores_launch<D, kNarrow, MERGE>(a, job, empty, stream);
 }
 
 template <int D>

@@ -30,6 +30,13 @@ def test_scores_of_partly_masked_stages(H, Hkv, keys, Lq, mask):
     _partly_masked(H, Hkv, keys, Lq, mask)
 
 
+# Two groups of waves that share a stage of 128 queries: launches of few workgroups and 256 queries or more
+@pytest.mark.parametrize("Lq", [255, 256, 257, 319, 384, 385])
+@pytest.mark.parametrize("mask", ["none", "window", "complement"])
+def test_scores_of_paired_waves(Lq, mask):
+    _partly_masked(4, 2, 900, Lq, mask)
+
+
 # The general kernel, for log-sum-exps in parts: one part, fewer than eight, eight, more than a turn of eight
 @pytest.mark.parametrize("H,Hkv,keys", [(4, 2, 700), (64, 64, 2100)])
 @pytest.mark.parametrize("Lq,parts", [(1, 1), (33, 3), (130, 8), (512, 2), (600, 11)])
