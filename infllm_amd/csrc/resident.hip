@@ -613,10 +613,6 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             at.nsplit = nsplit;
             at.softmax_scale = d.softmax_scale;
             at.d_o_part = a->d_o_part; at.d_lse_part = a->d_lse_part;
-            const int ti = timer_begin(R, 0, gn, (int)(b0 + gn - lo), st);
-            rc = infllm_attn_stage_blocked(&at, exc, block_rows, st, D);
-            timer_end(R, 0, ti, st);
-            if (rc) return rc;
             // Blocks that read nothing but the window and from which nothing leaves (a stream's first n_local tokens) have no
             // chain from one to the next: their partials are merged and their scores taken in one launch each for all of them
             // (eight blocks: 16 launches of some 20 us; 4,096 queries at once keep the chip full).
@@ -626,14 +622,30 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
                 const Carve c = carve_after(d, R->cursor, R->init_len, e1);
                 if (c.take || c.count || page_list(R, a, std::min(N, d.topk), e1).n_pages) break;
             }
+            const int q0 = i * exc, nq = std::min(m * exc, n - q0);
+            // ... or both in one launch, where all blocks of this one are such and few enough for it: their partials are those of one
+            // long block then (1,998 queries: the merge's 10 us)
+            const bool whole = m >= 2 && nq == gn && gn <= 2048;
+            const int ti = timer_begin(R, 0, gn, (int)(b0 + gn - lo), st);
+            rc = infllm_attn_stage_blocked(&at, whole ? (gn + 31) / 32 * 32 : exc, whole ? (int64_t)nsplit * B * d.H * gn : block_rows, st, D);
+            timer_end(R, 0, ti, st);
+            if (rc) return rc;
             if (m >= 2) {
-                const int q0 = i * exc, nq = std::min(m * exc, n - q0);
-                rc = infllm_attn_merge_blocked(a->d_o_part, a->d_lse_part, nsplit, B, d.H, nq, exc, block_rows, (bf16_t *)a->d_out + (st0 + q0) * a->o_sl, a->o_sb,
-                                               a->o_sh, a->o_sl, a->d_lse, st, D);
-                if (rc) return rc;
+                bf16_t *out = (bf16_t *)a->d_out + (st0 + q0) * a->o_sl;
                 const infllm_score_args sc = score_args(q0, nq, lo, b0 + nq);
-                rc = infllm_local_score_dim(&sc, D, st);
-                if (rc) return rc;
+                rc = 1;
+                if (whole) {
+                    MergeJob job;
+                    rc = infllm_merge_job(a->d_o_part, a->d_lse_part, nsplit, nullptr, nullptr, 0, B, d.H, gn, out, a->o_sb, a->o_sh, a->o_sl, a->d_lse, &job, D);
+                    if (!rc) rc = infllm_local_score_merged(&sc, &job, st, D);
+                    if (rc < 0) return rc;
+                }
+                if (rc == 1) {
+                    rc = infllm_attn_merge_blocked(a->d_o_part, a->d_lse_part, nsplit, B, d.H, nq, whole ? gn : exc, block_rows, out, a->o_sb, a->o_sh, a->o_sl,
+                                                   a->d_lse, st, D);
+                    if (!rc) rc = infllm_local_score_dim(&sc, D, st);
+                    if (rc) return rc;
+                }
                 plain_end = i + m;
             }
         }
