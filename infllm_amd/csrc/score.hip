@@ -595,10 +595,20 @@ template <int D>
 constexpr int kRankCpl = D == 64 ? 5 : 9;
 
 template <int D, int KS>
-__global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(BlockEnd j) {
+__global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(BlockEnd) {
     extern __shared__ __attribute__((aligned(1024))) char score_lds[];
+    // The arguments where they lie, for each kind of workgroup anew.  (As the parameter they are loads that all kinds share, made in
+    // front of the first branch and kept: 215 scalar registers were written to vector lanes and back on every workgroup's way.  Prompts of
+    // 16,001 / 131,072 tokens 2,692 -> 2,624 / 25,698 -> 24,969 us, of 24,300 with 36 heads of 64 unchanged.)
+    auto arguments = []() -> const BlockEnd & {
+        auto *p = (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p));
+        return *(const BlockEnd *)p;
+    };
     int x = blockIdx.x;
-    if (x < j.n_carve) {
+    const int n_carve = arguments().n_carve;
+    if (x < n_carve) {
+        const BlockEnd &j = arguments();
         if (j.n_units > 0) {
             const int rest = x / j.s.H;
             carve_unit<D>(j, x - rest * j.s.H, rest % j.n_units, rest / j.n_units, score_lds);
@@ -618,8 +628,10 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(Block
         rank_block<kRankCpl<D>>(j.rank, 0, j.rank.n_new, *(RankLds<kRankCpl<D>> *)score_lds);
         return;
     }
-    x -= j.n_carve;
-    if (x < j.n_score) {
+    x -= n_carve;
+    const int n_score = arguments().n_score;
+    if (x < n_score) {
+        const BlockEnd &j = arguments();
         const infllm_score_args &a = j.s;
         const int rows = a.B * a.H, tile = x / rows;
         int b, h;
@@ -638,7 +650,8 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(Block
         }
         return;
     }
-    x -= j.n_score;
+    x -= n_score;
+    const BlockEnd &j = arguments();
     if (x < j.n_early) {                                          // the units carved before, for the blocks behind the next
         rank_block<kRankCpl<D>>(j.rank, x + 1, j.rank.n_before, *(RankLds<kRankCpl<D>> *)score_lds);
         return;
