@@ -3,8 +3,11 @@
 #pragma once
 #include "common.h"
 
+#include <type_traits>
+
 constexpr int kRankEntries = 320;          // the k <= 64 best of the call's start + 256 units carved since
 constexpr int kRankNew = 64;               // units carved by one block
+constexpr int kRankChunks = 256;           // addresses of chunks of units that a ranking workgroup keeps
 
 // The page table of a block: selected units, init tokens, overflow remainder of the ring (the order of the host-built
 // tables of stream.hip).
@@ -15,17 +18,18 @@ struct PageList {
     int64_t cursor, overflow_end, ring_cap, init_cap;
     const bf16_t *init_kv, *ring_k, *ring_v;
     const uint64_t *chunk;                 // device: chunks of units, [per_chunk, B, 2, Hkv, bs, dim] each
-    int32_t per_chunk, B;
+    int32_t per_chunk, B, n_chunks;
 };
 
-__device__ __forceinline__ void write_page(const PageList &j, int u, int p, const int32_t *ids) {
+// chunk: the table, where it has been read already
+__device__ __forceinline__ void write_page(const PageList &j, int u, int p, const int32_t *ids, const uint64_t *chunk) {
     const int64_t unit_elems = (int64_t)j.Hkv * j.bs * j.dim;
     infllm_page pg;
     pg.reserved = 0;
     if (p < j.n_unit_pages) {
         const int s = p / j.tiles_per_unit, t0 = (p - s * j.tiles_per_unit) * kTile;
         const int unit = ids[s], ch = unit / j.per_chunk;
-        const bf16_t *kb = (const bf16_t *)(uintptr_t)j.chunk[ch] + (((int64_t)(unit - ch * j.per_chunk) * j.B + u) * 2) * unit_elems + (int64_t)t0 * j.dim;
+        const bf16_t *kb = (const bf16_t *)(uintptr_t)chunk[ch] + (((int64_t)(unit - ch * j.per_chunk) * j.B + u) * 2) * unit_elems + (int64_t)t0 * j.dim;
         pg.k = kb;
         pg.v = kb + unit_elems;
         pg.head_stride = (int64_t)j.bs * j.dim;
@@ -76,13 +80,16 @@ struct RankLds {
     float fresh[2 * kRankNew];
     uint64_t e_key[kRankEntries];
     int32_t sel[64];
+    uint64_t chunk[kRankChunks];
 };
 
 // 256 threads: scores of n_new units from jb.first_new on under the mean query of block j0 + x, and the ranking if that is block
 // j_sel (the sums are unit_scores_rows_kernel's, term by term: a unit's score does not depend on which kernel computed it).  All
-// of it is a chain of trips to memory: what can be requested ahead of another answer is.
+// of it is a chain of trips to memory on the way to the next block, beside workgroups that keep the chip busy: everything whose
+// address is known is requested at once, what depends on it next, and nothing is read behind the ranking.  all_pages: the pages
+// behind the units' too (else another workgroup writes those, which depend on no selection).
 template <int CPL>
-__device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, RankLds<CPL> &lds) {
+__device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, bool all_pages, RankLds<CPL> &lds) {
     float *fresh = lds.fresh;
     uint64_t *e_key = lds.e_key;
     int32_t *sel = lds.sel;
@@ -90,6 +97,7 @@ __device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, 
     const int j = jb.j0 + x;
     const bool is_sel = j == jb.j_sel;
     const int n = jb.n_list + jb.first_new + n_new - jb.n_base;
+    const bool kept = is_sel && jb.pages.n_chunks <= kRankChunks;
     for (int u = 0; u < jb.B; ++u) {
         const float *qbar = jb.qbars + ((int64_t)j * jb.B + u) * C;
         float *scores = jb.scores + ((int64_t)j * jb.B + u) * jb.cols;
@@ -100,9 +108,7 @@ __device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, 
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int e = tid + 256 * i;
-                if (e >= n) continue;
-                my_id[i] = e < jb.n_list ? jb.base[((int64_t)j * jb.B + u) * jb.k + e] : jb.n_base + (e - jb.n_list);
-                if (my_id[i] < jb.first_new) my_score[i] = scores[my_id[i]];
+                if (e < n) my_id[i] = e < jb.n_list ? jb.base[((int64_t)j * jb.B + u) * jb.k + e] : jb.n_base + (e - jb.n_list);
             }
         }
         u32x4 w[CPL];
@@ -112,7 +118,21 @@ __device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, 
             for (int c = 0; c < CPL; ++c) w[c] = c * 512 + lane * 8 < C ? *(const u32x4 *)(row + c * 512) : u32x4{0, 0, 0, 0};
         };
         if (wave < n_new) request(wave);
-        for (int e = tid * 4; e < C; e += 1024) *(f32x4 *)(lds.q + e) = *(const f32x4 *)(qbar + e);
+        constexpr int kQ = (CPL * 512 + 1023) / 1024;
+        f32x4 q_in[kQ];
+#pragma unroll
+        for (int i = 0; i < kQ; ++i) q_in[i] = *(const f32x4 *)(qbar + min(i * 1024 + tid * 4, C - 4));
+        uint64_t chunk_in = 0;
+        if (kept && u == 0 && tid < jb.pages.n_chunks) chunk_in = jb.pages.chunk[tid];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (is_sel && tid + 256 * i < n && my_id[i] < jb.first_new) my_score[i] = scores[my_id[i]];
+#pragma unroll
+        for (int i = 0; i < kQ; ++i) {
+            const int e = i * 1024 + tid * 4;
+            if (e < C) *(f32x4 *)(lds.q + e) = q_in[i];
+        }
+        if (kept && u == 0) lds.chunk[tid] = chunk_in;
         __syncthreads();
         for (int r = wave; r < n_new; r += 4) {
             float acc0 = 0.f, acc1 = 0.f;
@@ -145,23 +165,29 @@ __device__ __forceinline__ void rank_block(const RankJob &jb, int x, int n_new, 
             e_key[e] = ((uint64_t)order_key(score) << 32) | (uint32_t)~my_id[i];
         }
         __syncthreads();
-        for (int e0 = 0; e0 < n; e0 += 64) {                     // an entry's place is the number of entries in front of it: four lanes count
-            const int e = e0 + (tid >> 2), p = tid & 3;
-            const uint64_t own = e_key[min(e, n - 1)];
-            int rank = 0;
-#pragma unroll 4
-            for (int o = p; o < n; o += 4) rank += e_key[o] > own ? 1 : 0;
-            rank += __shfl_xor(rank, 1, 64);
-            rank += __shfl_xor(rank, 2, 64);
-            if (p == 0 && e < n && rank < jb.k) {
-                const int id = (int)~(uint32_t)own;
-                sel[rank] = id;
-                // (written through to the host's memory: a fence would write the whole L2 back)
-                __hip_atomic_store(jb.log + (int64_t)u * jb.k + rank, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        auto count = [&](auto lanes) {                           // an entry's place is the number of entries in front of it: some lanes count
+            constexpr int L = decltype(lanes)::value;
+            for (int e0 = 0; e0 < n; e0 += 256 / L) {
+                const int e = e0 + tid / L, p = tid % L;
+                const uint64_t own = e_key[min(e, n - 1)];
+                int rank = 0;
+#pragma unroll 16
+                for (int o = p; o < n; o += L) rank += e_key[o] > own ? 1 : 0;
+#pragma unroll
+                for (int o = 1; o < L; o <<= 1) rank += __shfl_xor(rank, o, 64);
+                if (p == 0 && e < n && rank < jb.k) {
+                    const int id = (int)~(uint32_t)own;
+                    sel[rank] = id;
+                    // (written through to the host's memory: a fence would write the whole L2 back)
+                    __hip_atomic_store(jb.log + (int64_t)u * jb.k + rank, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                }
             }
-        }
+        };
+        if (n <= 64) count(std::integral_constant<int, 4>{});
+        else count(std::integral_constant<int, 2>{});
         __syncthreads();
-        for (int p = tid; p < jb.pages.n_pages; p += 256) write_page(jb.pages, u, p, sel);
+        const int n_write = all_pages ? jb.pages.n_pages : jb.pages.n_unit_pages;
+        for (int p = tid; p < n_write; p += 256) write_page(jb.pages, u, p, sel, kept ? lds.chunk : jb.pages.chunk);
         __syncthreads();                                         // the lists are rewritten for the next row
     }
     if (is_sel) {

@@ -56,13 +56,13 @@ namespace {
 template <int CPL>
 __global__ __launch_bounds__(256) void rank_kernel(RankJob jb) {
     __shared__ __attribute__((aligned(16))) RankLds<CPL> lds;
-    rank_block<CPL>(jb, blockIdx.x, jb.n_new, lds);
+    rank_block<CPL>(jb, blockIdx.x, jb.n_new, true, lds);
 }
 
 // the page table of a selection that is already in memory
 __global__ __launch_bounds__(256) void pages_kernel(PageList j, const int32_t *ids, int n_ids) {
     const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p < j.n_pages) write_page(j, blockIdx.y, p, ids + (int64_t)blockIdx.y * n_ids);
+    if (p < j.n_pages) write_page(j, blockIdx.y, p, ids + (int64_t)blockIdx.y * n_ids, j.chunk);
 }
 
 // The end of a decode step: output rows = the joined splits; the window's score track += the probabilities, from the
@@ -305,7 +305,7 @@ PageList page_list(const Resident *R, const infllm_resident_call *a, int n_sel, 
     j.Hkv = d.Hkv; j.bs = d.block_size; j.init_len = R->init_len; j.dim = d.dim;
     j.ring_cap = d.ring_cap; j.init_cap = d.init_cap;
     j.init_kv = (const bf16_t *)d.d_init_kv; j.ring_k = (const bf16_t *)d.d_ring_k_raw; j.ring_v = (const bf16_t *)d.d_ring_v;
-    j.chunk = a->d_chunks; j.per_chunk = d.units_per_chunk; j.B = d.B;
+    j.chunk = a->d_chunks; j.per_chunk = d.units_per_chunk; j.B = d.B; j.n_chunks = a->n_chunks;
     return j;
 }
 

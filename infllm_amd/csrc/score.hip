@@ -282,7 +282,7 @@ constexpr int kCarveMaxLq = 512, kCarveMaxUnit = 128;
 struct BlockEnd {
     infllm_score_args s;               // the keys that stay
     MergeJob merge;                    // the block's partials (out NULL: merged before)
-    int32_t n_carve, n_score, n_copy, n_early;     // workgroups of each kind, in this order, those that merge behind them
+    int32_t n_carve, n_score, n_copy, n_early;     // workgroups of each kind (carve, score, early, copy), those that merge behind them
     int32_t cap, slot0, win;           // rows of the ring; that of the first key of the first scoring workgroup; the window
     // units that leave
     const bf16_t *ring_k_raw;
@@ -625,7 +625,8 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(Block
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             if (threadIdx.x == 0) __hip_atomic_store(j.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        rank_block<kRankCpl<D>>(j.rank, 0, j.rank.n_new, *(RankLds<kRankCpl<D>> *)score_lds);
+        __builtin_amdgcn_s_setprio(3);                            // (the launch waits for it)
+        rank_block<kRankCpl<D>>(j.rank, 0, j.rank.n_new, false, *(RankLds<kRankCpl<D>> *)score_lds);
         return;
     }
     x -= n_carve;
@@ -652,8 +653,12 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(Block
     }
     x -= n_score;
     const BlockEnd &j = arguments();
-    if (x < j.n_early) {                                          // the units carved before, for the blocks behind the next
-        rank_block<kRankCpl<D>>(j.rank, x + 1, j.rank.n_before, *(RankLds<kRankCpl<D>> *)score_lds);
+    if (x < j.n_early) {                                          // the first: pages that depend on no selection; the others: the units
+        const PageList &pages = j.rank.pages;                     // carved before, for the blocks behind the next
+        if (x > 0) rank_block<kRankCpl<D>>(j.rank, x, j.rank.n_before, false, *(RankLds<kRankCpl<D>> *)score_lds);
+        else
+            for (int e = threadIdx.x, n = pages.n_pages - pages.n_unit_pages; e < n * pages.B; e += 256)
+                write_page(pages, e / n, pages.n_unit_pages + e % n, nullptr, nullptr);
         return;
     }
     x -= j.n_early;
@@ -877,7 +882,7 @@ int infllm_block_end(const infllm_score_args *a, const MergeJob *job, const void
         INFLLM_REQUIRE(rank->n_list + rank->first_new + rank->n_new - rank->n_base <= kRankEntries, "block_end: too many units to rank");
         j.rank = *rank;
         j.ranks = 1;
-        j.n_early = rank->n_before > 0 ? n_rank - 1 : 0;
+        j.n_early = 1 + (rank->n_before > 0 ? n_rank - 1 : 0);
         j.ticket = d_ticket;
         j.n_carve = std::max(j.n_carve, 1);                       // (nothing carved: a workgroup that only ranks)
     }
