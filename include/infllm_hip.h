@@ -654,7 +654,7 @@ int64_t infllm_layer_fetched_units(void *layer);
  *   units       chunks of units_per_chunk units [.., B, 2, Hkv, block_size, dim]; h_chunks / d_chunks: their addresses, as
  *               the host and as the device reads them
  *   d_log       log_slots x (B * topk + 1) ints of pinned memory, device and host view
- *   d_ids       [B, topk]; d_iota: 0, 1, .. topk - 1; d_pages: [B, max_pages]
+ *   d_ids       [B, topk]; d_pages: [B, max_pages]; d_iota: not read (a selection of every unit needs no list)
  *   h_caches    [B] policy objects (infllm_cache_create, lru or fifo) */
 typedef struct {
     int32_t B, H, Hkv, dim;

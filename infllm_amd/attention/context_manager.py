@@ -381,14 +381,13 @@ class ContextManager:
         self._chunk_host = (ctypes.c_uint64 * 16)()
         self._chunk_dev = torch.empty((16,), dtype=torch.int64, device=dev)
         self._ids = torch.empty((B, topk), **i32)
-        self._iota = torch.arange(topk, **i32)
         self._pages = torch.empty((B * self.max_pages * ctypes.sizeof(_lib.Page),), dtype=torch.uint8, device=dev)
         self._log, seq = _Units.take_log(self._dev_index, B * topk + 1)
         self._caches = (ctypes.c_void_p * B)(*[pol.handle for pol in self._policy])
         d = self._resident_desc(self.head_width)
         d.d_ring_k_raw, d.d_ring_k_rot = self.ring_k_raw.data_ptr(), self.ring_k_rot.data_ptr()
         d.d_ring_v, d.d_ring_score, d.d_init_kv = self.ring_v.data_ptr(), self.ring_score.data_ptr(), self.init_kv.data_ptr()
-        d.d_pages, d.d_ids, d.d_iota = self._pages.data_ptr(), self._ids.data_ptr(), self._iota.data_ptr()
+        d.d_pages, d.d_ids = self._pages.data_ptr(), self._ids.data_ptr()
         d.d_log, d.h_log = self._lib.infllm_host_device_pointer(self._log.data_ptr()), self._log.data_ptr()
         d.h_caches, d.d_inv_freq = ctypes.addressof(self._caches), self.inv_freq.data_ptr()
         d.distance_scale, d.softmax_scale = float(self.position_embedding.distance_scale), 1.0 / (self.dim_head ** 0.5)

@@ -124,7 +124,6 @@ enum { kLinear = 0, kPaged = 1, kBoth = 2, kSinks = 3 };
 // kernel reads them where they lie in its argument segment - scalar loads through the constant address space, like the
 // table in device memory, but no kernel has to run beforehand to put it there.  The parameter is never touched as a
 // C++ object (that would copy it to scratch memory for the dynamic index).
-constexpr int kInlinePages = 64;
 struct InlinePages {
     infllm_page p[kInlinePages];
 };

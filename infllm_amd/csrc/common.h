@@ -20,6 +20,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kD = INFLLM_HEAD_DIM;       // head_dim
 constexpr int kTile = INFLLM_KEY_TILE;    // keys per tile
+constexpr int kInlinePages = 64;          // page table entries that a launch of the paged stage can carry
 constexpr int kWave = 64;
 
 // thread-local error text, returned by infllm_last_error()

@@ -5,15 +5,15 @@
 constexpr int kDecodeSegs = 6;
 constexpr int kDecodeBlock = 16;           // keys a wave takes at a time
 
-// `rows` consecutive rows of D elements, row stride D, of every (batch row, kv head).  With `ids` the rows are those of
-// `n_ids` units of `rows` rows each, unit u of batch row b at chunk[u / per_chunk] + (u % per_chunk) * unit_elems + b *
+// `rows` consecutive rows of D elements, row stride D, of every (batch row, kv head).  With `n_ids` > 0 the rows are
+// those of `n_ids` units of `rows` rows each, unit u of batch row b at chunk[u / per_chunk] + (u % per_chunk) * unit_elems + b *
 // row_elems, where its keys are followed by its values (v_off elements on), heads k_sh apart.
 struct DecodeSeg {
     const bf16_t *k, *v;
     int64_t k_sb, k_sh, v_sb, v_sh;
     int32_t rows, q;                       // q: which of the job's two rotations of the query this range is attended with
     int32_t n_ids;
-    const int32_t *ids;                    // [B, n_ids] on the device, NULL: a plain range
+    const int32_t *ids;                    // [B, n_ids] on the device, NULL: units 0, 1, .. (n_ids > 0) or a plain range
     int32_t logit0;                        // row r's scaled logit goes to logits[.., logit0 + r]; -1: not kept
 };
 
@@ -33,7 +33,7 @@ struct DecodeJob {
     float *logits;                         // optional [B, H, logit_stride]: scaled logits in base 2 (see DecodeSeg)
     int64_t logit_stride;
     int32_t new_logit;                     // of a step with its rows: where the new key's logit goes (-1: not kept)
-    // Optional: the launch selects the units itself (the one range that has ids, of n_ids units; `ids` is not read): the best of the
+    // Optional: the launch selects the units itself (the one range of units, n_ids of them; `ids` is not read): the best of the
     // n_scores units with scores at unit_scores + b * unit_scores_sb, into ids_out [B, n_ids] too.  The first lead_segs ranges, with the
     // units among them, belong to the first lead_splits splits, the others to the rest.
     const float *unit_scores;

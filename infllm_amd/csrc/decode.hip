@@ -148,7 +148,7 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
             r.q = sg.q;
             if (sg.n_ids > 0) {
                 const int i = blk / per, r0 = (blk - i * per) * kDecodeBlock;
-                const int u = __builtin_amdgcn_readfirstlane(SELECT ? chosen[i] : sg.ids[(int64_t)b * sg.n_ids + i]);
+                const int u = __builtin_amdgcn_readfirstlane(SELECT ? chosen[i] : sg.ids ? sg.ids[(int64_t)b * sg.n_ids + i] : i);
                 const int ch = u / j.per_chunk;
                 const bf16_t *base = (const bf16_t *)(uintptr_t)j.chunk[ch] + (int64_t)(u - ch * j.per_chunk) * j.unit_elems + (int64_t)b * j.row_elems +
                                      (int64_t)g * j.unit_sh + (int64_t)r0 * D;
@@ -520,7 +520,7 @@ static int check_job(const DecodeJob *job, int32_t dim) {
     for (int s = 0; s < job->n_seg; ++s) {
         const DecodeSeg &sg = job->seg[s];
         INFLLM_REQUIRE(sg.rows >= 0 && (sg.q == 0 || sg.q == 1), "decode_attn: bad range");
-        if (sg.n_ids > 0) INFLLM_REQUIRE(job->chunk && job->per_chunk > 0 && (sg.ids || job->unit_scores), "decode_attn: units without an arena");
+        if (sg.n_ids > 0) INFLLM_REQUIRE(job->chunk && job->per_chunk > 0, "decode_attn: units without an arena");
         else INFLLM_REQUIRE(sg.rows == 0 || (sg.k && sg.v), "decode_attn: null range");
     }
     INFLLM_REQUIRE(dim == 128 || dim == 64, "decode_attn: head_dim %d", dim);

@@ -21,32 +21,34 @@ struct PageList {
     int32_t per_chunk, B, n_chunks;
 };
 
-// chunk: the table, where it has been read already
-__device__ __forceinline__ void write_page(const PageList &j, int u, int p, const int32_t *ids, const uint64_t *chunk) {
+// Page p of batch row u.  ids: the selection, NULL: every unit in order; chunk: the table of addresses, where it has been read already.
+__host__ __device__ __forceinline__ infllm_page page_of(const PageList &j, int u, int p, const int32_t *ids, const uint64_t *chunk) {
     const int64_t unit_elems = (int64_t)j.Hkv * j.bs * j.dim;
     infllm_page pg;
     pg.reserved = 0;
     if (p < j.n_unit_pages) {
         const int s = p / j.tiles_per_unit, t0 = (p - s * j.tiles_per_unit) * kTile;
-        const int unit = ids[s], ch = unit / j.per_chunk;
+        const int unit = ids ? ids[s] : s, ch = unit / j.per_chunk;
         const bf16_t *kb = (const bf16_t *)(uintptr_t)chunk[ch] + (((int64_t)(unit - ch * j.per_chunk) * j.B + u) * 2) * unit_elems + (int64_t)t0 * j.dim;
         pg.k = kb;
         pg.v = kb + unit_elems;
         pg.head_stride = (int64_t)j.bs * j.dim;
-        pg.n_valid = min(j.bs - t0, kTile);
+        pg.n_valid = j.bs - t0 < kTile ? j.bs - t0 : kTile;
     } else if (p < j.n_unit_pages + j.n_init_pages) {
         const int t0 = (p - j.n_unit_pages) * kTile;
         const bf16_t *ik = j.init_kv + (int64_t)u * 2 * j.Hkv * j.init_cap * j.dim + (int64_t)t0 * j.dim;
         pg.k = ik;
         pg.v = ik + (int64_t)j.Hkv * j.init_cap * j.dim;
         pg.head_stride = j.init_cap * j.dim;
-        pg.n_valid = min(j.init_len - t0, kTile);
+        pg.n_valid = j.init_len - t0 < kTile ? j.init_len - t0 : kTile;
     } else {
         const int want = p - j.n_unit_pages - j.n_init_pages;
         int64_t pos = j.cursor, len = 0;
         for (int i = 0; i <= want; ++i) {          // runs of <= 64 rows that do not cross the end of the ring
             pos += len;
-            len = min(min(j.overflow_end - pos, (int64_t)kTile), j.ring_cap - pos % j.ring_cap);
+            const int64_t left = j.overflow_end - pos, lap = j.ring_cap - pos % j.ring_cap;
+            len = left < kTile ? left : kTile;
+            len = lap < len ? lap : len;
         }
         const int64_t row = pos % j.ring_cap;
         pg.k = j.ring_k + ((int64_t)u * j.Hkv * j.ring_cap + row) * j.dim;
@@ -54,7 +56,11 @@ __device__ __forceinline__ void write_page(const PageList &j, int u, int p, cons
         pg.head_stride = j.ring_cap * j.dim;
         pg.n_valid = (int)len;
     }
-    j.out[(int64_t)u * j.n_pages + p] = pg;
+    return pg;
+}
+
+__device__ __forceinline__ void write_page(const PageList &j, int u, int p, const int32_t *ids, const uint64_t *chunk) {
+    j.out[(int64_t)u * j.n_pages + p] = page_of(j, u, p, ids, chunk);
 }
 
 // After a block has carved units: every unit is scored under the mean queries of the call's later blocks, and block j_sel's list

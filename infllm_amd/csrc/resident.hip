@@ -59,10 +59,10 @@ __global__ __launch_bounds__(256) void rank_kernel(RankJob jb) {
     rank_block<CPL>(jb, blockIdx.x, jb.n_new, true, lds);
 }
 
-// the page table of a selection that is already in memory
-__global__ __launch_bounds__(256) void pages_kernel(PageList j, const int32_t *ids, int n_ids) {
+// the page table of a block that attends every unit, where the attention's launch does not hold it
+__global__ __launch_bounds__(256) void pages_kernel(PageList j) {
     const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p < j.n_pages) write_page(j, blockIdx.y, p, ids + (int64_t)blockIdx.y * n_ids, j.chunk);
+    if (p < j.n_pages) write_page(j, blockIdx.y, p, nullptr, j.chunk);
 }
 
 // The end of a decode step: output rows = the joined splits; the window's score track += the probabilities, from the
@@ -461,7 +461,7 @@ int decode_step(Resident *R, const infllm_resident_call *a, int64_t st0, hipStre
     if (n_sel > 0) {
         DecodeSeg &sg = j.seg[j.n_seg++];
         sg = DecodeSeg{};
-        sg.rows = d.block_size; sg.q = 1; sg.n_ids = n_sel; sg.ids = retrieve ? d.d_ids : d.d_iota; sg.logit0 = -1;
+        sg.rows = d.block_size; sg.q = 1; sg.n_ids = n_sel; sg.ids = retrieve ? d.d_ids : nullptr; sg.logit0 = -1;
         blocks += (int64_t)n_sel * ((d.block_size + kDecodeBlock - 1) / kDecodeBlock);
         j.chunk = a->d_chunks; j.per_chunk = d.units_per_chunk;
         j.unit_sh = (int64_t)d.block_size * d.dim; j.unit_v_off = d.Hkv * j.unit_sh; j.row_elems = 2 * j.unit_v_off; j.unit_elems = B * j.row_elems;
@@ -664,8 +664,15 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
         INFLLM_REQUIRE(pl.n_pages <= d.max_pages, "resident: %d pages exceed the table (%d)", pl.n_pages, d.max_pages);
         const bool all_units = N <= d.topk;
         if (all_units) R->queue.push_back(Resident::Entry{N, 0, 0});
-        if (all_units && pl.n_pages > 0) {
-            hipLaunchKernelGGL(pages_kernel, dim3((pl.n_pages + 255) / 256, B), dim3(256), 0, st, pl, d.d_iota, 0);
+        // A block that attends every unit has its table from here, and the launch of the global stage takes one of up to 64 pages along
+        // (a launch of its own for the table: 4.7 us; five of them in a prompt of 16,001 tokens: 2,729 us with, 2,708 without).
+        infllm_page carried[kInlinePages];
+        const bool carries = all_units && pl.n_pages > 0 && (int64_t)B * pl.n_pages <= kInlinePages;
+        if (carries) {
+            for (int u = 0; u < B; ++u)
+                for (int p = 0; p < pl.n_pages; ++p) carried[u * pl.n_pages + p] = page_of(pl, u, p, nullptr, a->h_chunks);
+        } else if (all_units && pl.n_pages > 0) {
+            hipLaunchKernelGGL(pages_kernel, dim3((pl.n_pages + 255) / 256, B), dim3(256), 0, st, pl);
             INFLLM_CHECK_LAUNCH("pages");
         } else if (!all_units && j_done != i) {                   // the call's first block (the others' tables came with the previous block)
             int32_t slot = 0, seq = 0;
@@ -697,7 +704,7 @@ int prompt_call(Resident *R, const infllm_resident_call *a, int64_t st0, int n, 
             const int tw = timer_begin(R, 2, nb, 0, st);          // (where the stream of the host-driven path waits for missed units)
             timer_end(R, 2, tw, st);
             const int ti = timer_begin(R, 1, nb, pl.n_pages * kTile, st);
-            rc = infllm_attn_paged(&at, nullptr, st, D);
+            rc = infllm_attn_paged(&at, carries ? carried : nullptr, st, D);
             timer_end(R, 1, ti, st);
             if (rc) return rc;
             parts += ns_g;
@@ -817,7 +824,7 @@ extern "C" void *infllm_resident_create(const infllm_resident_desc *desc) {
     if (d.exc <= 0 || d.exc > d.n_local || d.block_size <= 0 || d.topk > d.max_cached || d.n_init < 0) return bad("bad knobs");
     if (infllm_resident_fits(desc) != 1) return bad("geometry without this path");
     if (d.ring_cap % kTile || d.ring_cap < (int64_t)d.n_local + 2 * d.exc + d.block_size) return bad("ring too small or unaligned");
-    if (!d.d_ring_k_raw || !d.d_ring_k_rot || !d.d_ring_v || !d.d_ring_score || !d.d_init_kv || !d.d_ids || !d.d_iota || !d.d_pages || !d.d_log || !d.h_log ||
+    if (!d.d_ring_k_raw || !d.d_ring_k_rot || !d.d_ring_v || !d.d_ring_score || !d.d_init_kv || !d.d_ids || !d.d_pages || !d.d_log || !d.h_log ||
         !d.h_caches || !d.d_inv_freq)
         return bad("null buffer");
     if (d.log_slots < 2 || d.units_per_chunk < 1 || d.init_cap < 1 || d.max_pages < 1 || d.max_splits < 1 || d.num_cus < 1 || d.group_blocks < 1) return bad("bad capacities");
