@@ -37,23 +37,38 @@ def _capturing(dev):
     return dev.type == "cuda" and torch.cuda.is_current_stream_capturing()
 
 
-def _take_words(past_k, n, dev, stream):
-    """(n words or more in which a step counts its finished key splits, their address, their number, the stream they belong to) and
-    whether the call has to clear them, or None: it counts in words of its own scratch.
+_STEP_BYTES = 4 << 20               # scratch of a call of one token that is kept for the next one, at most
 
-    The words are zero between the launches that use them, and only one call has them at a time: it takes them off the storage of
-    the cache it continues (one operation, whichever threads go on from that cache) and leaves them with the cache it returns.
-    Their launches are then in the order of their stream, which is also the one that the allocator gives them out again in.
+
+def _step_bytes(kind, batch, heads, dim):
+    """scratch of a call of one token: its rotated queries, up to 64 key splits of its rows, their sums"""
+    rows = batch * heads
+    splits = 64 * rows if rows <= 2048 else _SPLIT_ROWS if 2 * rows <= _SPLIT_ROWS else 0
+    return (2 if kind else 1) * rows * dim * 2 + splits * (2 * dim + 4) + 4 * rows
+
+
+def _take_words(past_k, n, step_bytes, dev, stream):
+    """((tensor, address of n words or more in which a step counts its finished key splits, their number, the stream they belong to,
+    address and size of a step's scratch behind them, size 0 where it would be more than _STEP_BYTES) and whether the call has to clear
+    the words, or None: it counts in words of its own scratch.
+
+    The words are zero between the launches that use them, and only one call has them and the scratch at a time: it takes them off the
+    storage of the cache it continues (one operation, whichever threads go on from that cache) and leaves them with the cache it
+    returns.  Their launches are then in the order of their stream, which is also the one that the allocator gives them out again in.
     Inside a capture there are none: its launches run when and where the graph is replayed, beside whatever else counts by then
     (and the default stream, 0, cannot be captured)."""
     if stream and _capturing(dev):
         return None, 0
+    if step_bytes > _STEP_BYTES:
+        step_bytes = 0
     if past_k is not None:
         held = past_k.untyped_storage().__dict__.pop("_infllm_words", None)
-        if held is not None and held[3] == stream and held[2] >= n:
+        if held is not None and held[3] == stream and held[2] >= n and held[5] >= step_bytes:
             return held, 0
-    t = torch.empty((n,), dtype=torch.int32, device=dev)
-    return (t, t.data_ptr(), n, stream), 1
+    head = -(-4 * n // 256) * 256
+    t = torch.empty((head + step_bytes,), dtype=torch.uint8, device=dev)
+    ptr = t.data_ptr()
+    return (t, ptr, n, stream, ptr + head, step_bytes), 1
 
 
 def _ticket(words):
@@ -95,25 +110,28 @@ class _Room:
 
 
 def _cache_rows(t, dim):
-    """(a cached tensor as the native call takes it: rows next to each other, its batch and head strides)"""
+    """(a cached tensor as the native call takes it: rows next to each other, its address, batch and head strides)"""
     sb, sh, sl, inner = t.stride()
-    if inner != 1 or sl != dim or (sb | sh) & 7 or t.data_ptr() & 15:
+    ptr = t.data_ptr()
+    if inner != 1 or sl != dim or (sb | sh) & 7 or ptr & 15:
         t = t.clone(memory_format=torch.contiguous_format)
         sb, sh, _, _ = t.stride()
-    return t, sb, sh
+        ptr = t.data_ptr()
+    return t, ptr, sb, sh
 
 
 def _heads(x, batch, length, heads, dim):
-    """(tensor that is kept alive, batch, head and row strides) of projected rows [batch, length, heads * dim]"""
+    """(tensor that is kept alive, address, batch, head and row strides) of projected rows [batch, length, heads * dim]"""
     if x.shape != (batch, length, heads * dim):
         x = x.view(batch, length, heads * dim)
     x = rows16(x)
-    return x, x.stride(0), dim, x.stride(1)
+    sb, sl, _ = x.stride()
+    return x, x.data_ptr(), sb, dim, sl
 
 
 def _wide_heads(x, batch, length, heads, dim):
     x = widen(x.view(batch, length, heads, dim), dim)
-    return x, x.stride(0), x.stride(2), x.stride(1)
+    return x, x.data_ptr(), x.stride(0), x.stride(2), x.stride(1)
 
 
 def _on_gpu(x):
@@ -154,9 +172,9 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
     native = dim_head in (64, HEAD_DIM)                        # other widths travel in rows of 128
     dim = dim_head if native else HEAD_DIM
     split = _heads if native else _wide_heads
-    q, q_sb, q_sh, q_sl = split(xq, batch, len_q, num_heads, dim_head)
-    k, k_sb, k_sh, k_sl = split(xk, batch, n_new, num_heads_kv, dim_head)
-    v, v_sb, v_sh, v_sl = split(xv, batch, n_new, num_heads_kv, dim_head)
+    q, q_ptr, q_sb, q_sh, q_sl = split(xq, batch, len_q, num_heads, dim_head)
+    k, k_ptr, k_sb, k_sh, k_sl = split(xk, batch, n_new, num_heads_kv, dim_head)
+    v, v_ptr, v_sb, v_sh, v_sl = split(xv, batch, n_new, num_heads_kv, dim_head)
     inv_freq = position_bias.inv_freq
     if inv_freq.device != dev or inv_freq.dtype != torch.float32 or inv_freq.numel() != dim // 2 or not inv_freq.is_contiguous():
         inv_freq = inv_freq.to(device=dev, dtype=torch.float32).contiguous() if native else wide_inv_freq(inv_freq, dev)
@@ -197,7 +215,8 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
         shape = (batch, num_heads_kv, rows_all, dim)
         room = _Room.of(old_k) if past is not None and native else None
         if room is not None and room.claim(old_k, old_v, n_new, stream):
-            new_k, new_v = (t.as_strided(shape, t.stride(), t.storage_offset()) for t in (old_k, old_v))
+            strides = old_k.stride()                           # (and old_v's)
+            new_k, new_v = old_k.as_strided(shape, strides, old_k.storage_offset()), old_v.as_strided(shape, strides, old_v.storage_offset())
         else:
             cap = rows_all + max(256, rows_all // 4)
             if kind:
@@ -206,25 +225,31 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
             _Room(both, rows_all, stream)
             new_k, new_v = both.narrow(3, 0, rows_all).unbind(0)
 
-    words, fresh = _take_words(old_k, batch * num_heads, dev, stream)
-    rows_q = batch * num_heads * len_q
-    q_bytes = (2 if kind else 1) * rows_q * dim * 2
-    part_rows = 64 * rows_q if rows_q <= 2048 else _SPLIT_ROWS if 2 * rows_q <= _SPLIT_ROWS else 0
-    work_bytes = q_bytes + part_rows * (2 * dim + 4) + (4 * rows_q if len_q == 1 else 0)
-    work = torch.empty((work_bytes,), dtype=torch.uint8, device=dev)
+    step_bytes = _step_bytes(kind, batch, num_heads, dim)
+    words, fresh = _take_words(old_k, batch * num_heads, step_bytes, dev, stream)
+    work_bytes = step_bytes
+    if len_q > 1:
+        rows_q = batch * num_heads * len_q
+        part_rows = 64 * rows_q if rows_q <= 2048 else _SPLIT_ROWS if 2 * rows_q <= _SPLIT_ROWS else 0
+        work_bytes = (2 if kind else 1) * rows_q * dim * 2 + part_rows * (2 * dim + 4)
+    # (a step's scratch comes with its words: one allocation of the three that its output, its cache and it take)
+    if len_q == 1 and words is not None and words[5]:
+        work_ptr = words[4]
+    else:
+        work = torch.empty((work_bytes,), dtype=torch.uint8, device=dev)
+        work_ptr = work.data_ptr()
     out = torch.empty((batch, len_q, num_heads * dim), dtype=bf, device=dev)
     okp = ovp = 0
     ok_sb = ok_sh = ov_sb = ov_sh = 0
     if rows_old:
-        cached_k, ok_sb, ok_sh = _cache_rows(cached_k, dim)
-        cached_v, ov_sb, ov_sh = _cache_rows(cached_v, dim)
-        okp, ovp = cached_k.data_ptr(), cached_v.data_ptr()
+        cached_k, okp, ok_sb, ok_sh = _cache_rows(cached_k, dim)
+        cached_v, ovp, ov_sb, ov_sh = _cache_rows(cached_v, dim)
     n_sb, n_sh, _, _ = new_k.stride()                          # (and new_v's: halves of one buffer)
-    args = _ARGS.pack(q.data_ptr(), k.data_ptr(), v.data_ptr(), q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl, batch, num_heads, num_heads_kv, dim,
+    args = _ARGS.pack(q_ptr, k_ptr, v_ptr, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl, batch, num_heads, num_heads_kv, dim,
                       len_q, n_new, kind, n_init, n_local, seen, inv_freq.data_ptr(), float(position_bias.distance_scale), okp, ovp, ok_sb, ok_sh, ov_sb,
                       ov_sh, new_k.data_ptr(), new_v.data_ptr(), n_sb, n_sh, n_sb, n_sh, rows_old, rows_new,
                       all_kv[0].data_ptr() if all_kv is not None else 0, all_kv[1].data_ptr() if all_kv is not None else 0,
-                      raw_old.data_ptr() if raw_old is not None else 0, raw.data_ptr() if raw is not None else 0, raw_rows, raw_new, work.data_ptr(),
+                      raw_old.data_ptr() if raw_old is not None else 0, raw.data_ptr() if raw is not None else 0, raw_rows, raw_new, work_ptr,
                       work_bytes, out.data_ptr(), len_q * num_heads * dim, dim, num_heads * dim, _ticket(words),
                       1.0 / math.sqrt(dim_head), fresh)
     _lib.check(_lib.load().infllm_window_forward(args, stream), "infllm_window_forward")

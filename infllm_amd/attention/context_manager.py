@@ -37,7 +37,9 @@ fetch) and infllm_block_back, plus infllm_block_prefetch for the next block.
 """
 import contextlib
 import ctypes
+import functools
 import os
+import struct
 import threading
 import weakref
 
@@ -63,6 +65,23 @@ _NUM_CUS = 256               # MI355X
 _PAGE_SLOTS = 4
 _CARVE_SLOTS = 4             # staging slots of the carve, used in turn (more of them serve more misses on the device - 16: 18 %,
                              # 64: 57 % of the benchmark stream's - but the stream is no faster for it, measured)
+
+
+_CALL_ROWS = struct.Struct("@3P9qP4q")      # the first fields of an infllm_resident_call, d_q to n
+
+
+@functools.lru_cache(None)
+def _device_bytes(index):
+    return torch.cuda.get_device_properties(index).total_memory
+
+
+def _addressed(t):
+    """rows16(t), with its address and strides"""
+    strides, ptr = t.stride(), t.data_ptr()
+    if strides[3] != 1 or (strides[0] | strides[1] | strides[2]) & 7 or ptr & 15:
+        t = t.clone(memory_format=torch.contiguous_format)
+        strides, ptr = t.stride(), t.data_ptr()
+    return t, ptr, strides
 
 
 class _Buffers(dict):
@@ -104,7 +123,7 @@ class _Units:
         with cls.lock:
             pool = cls.logs.setdefault((dev, n), [])
             for i, (log, seq) in enumerate(pool):
-                if seq == 0 or int(log[(seq % _LOG_SLOTS) * stride + stride - 1]) == seq:
+                if seq == 0 or ctypes.c_int32.from_address(log.data_ptr() + 4 * ((seq % _LOG_SLOTS) * stride + stride - 1)).value == seq:
                     del pool[i]
                     return log, seq
         return torch.zeros((n,), dtype=torch.int32, pin_memory=True), 0
@@ -255,7 +274,7 @@ class ContextManager:
         return not (self.record_trace or self.select_in_steps or not self.fetch_ahead)
 
     def _init(self, q, k, resident=None):
-        """q, k: rows of the heads' own width.  resident: None to choose."""
+        """q, k: rows of the heads' own width.  resident: False to have the host drive, None to choose."""
         B, H = q.shape[0], q.shape[1]
         Hkv = k.shape[1]
         dev = q.device
@@ -292,8 +311,8 @@ class ContextManager:
         if self.record_trace:
             for pol in self._policy:
                 pol.evicted_log = []
-        if resident is None:
-            resident = self._can_be_resident()
+        desc = None if resident is False else self._can_be_resident()
+        resident = desc is not None
         # Blocks per launch of the local stage.  With the host between the blocks two: a launch covers the wait for a fetch.
         # Without it as many as a call has (131,072 tokens: 33.0 -> 32.4 ms, 24,300 of the smaller geometry: 5.2 -> 4.7), unless
         # launches are timed one by one: a sample is a launch of two blocks.
@@ -307,11 +326,15 @@ class ContextManager:
         self.init_kv = torch.empty((B, 2, Hkv, max(self.n_init, 1), D), **bf)
         self.reps = torch.empty((B, 16, H * D), **bf)
         self.unit_scores = torch.empty((B, 16), **f32)
-        self.inv_freq = (self.position_embedding.inv_freq.to(device=dev, dtype=torch.float32).contiguous() if D == self.dim_head
-                         else wide_inv_freq(self.position_embedding.inv_freq, dev))
+        inv_freq = self.position_embedding.inv_freq
+        if D != self.dim_head:
+            inv_freq = wide_inv_freq(inv_freq, dev)
+        elif inv_freq.device != dev or inv_freq.dtype != torch.float32 or not inv_freq.is_contiguous():
+            inv_freq = inv_freq.to(device=dev, dtype=torch.float32).contiguous()
+        self.inv_freq = inv_freq
         self.slot_bytes = 2 * Hkv * bs * D * 2              # one unit of one batch row
         self.unit_bytes = B * self.slot_bytes               # one unit, all batch rows
-        self._init_resident() if resident else self._init_host()
+        self._init_resident(desc) if resident else self._init_host()
         self._call_stream = None               # stream the call buffers were taken for (they are bound at the first append)
         self.initialized = True
 
@@ -321,7 +344,7 @@ class ContextManager:
             return 0
         if self.resident_bytes is not None:
             return self.resident_bytes
-        return torch.cuda.get_device_properties(self._dev_index).total_memory // 4
+        return _device_bytes(self._dev_index) // 4
 
     def _leaves_room(self, n):
         """Whether the device still has memory for its other users once the units take n bytes more: units that found a home in
@@ -350,44 +373,47 @@ class ContextManager:
         return n
 
     def _resident_desc(self, D):
+        """The descriptor of a resident memory with rows of D elements; its buffers are not in it yet."""
         d = ResidentDesc()
         d.B, d.H, d.Hkv, d.dim = self.num_units, self.unit_size, self.unit_size_kv, D
         d.n_local, d.n_init, d.block_size, d.exc = self.n_local, self.n_init, self.block_size, self.exc_block_size
         d.topk, d.repr_topk, d.max_cached = self.topk, self.repr_topk, self.max_cached_block
-        d.max_splits, d.num_cus, d.call_tokens, d.group_blocks = _MAX_SPLITS, _NUM_CUS, self._call_tokens, getattr(self, "_local_group", 1)
+        d.max_splits, d.num_cus, d.call_tokens, d.group_blocks = _MAX_SPLITS, _NUM_CUS, self._call_tokens, 1
         unit_bytes = 2 * self.num_units * self.unit_size_kv * self.block_size * D * 2
         d.max_pages, d.units_per_chunk, d.log_slots = self.max_pages, self._units_per_chunk(unit_bytes), _LOG_SLOTS
         d.ring_cap, d.init_cap = self.ring_cap, max(self.n_init, 1)
         return d
 
     def _can_be_resident(self):
+        """The descriptor of the resident memory, or None: the host drives."""
         if not self._wants_resident() or self.cache_strategy == "lru-s" or self.chunk_topk_calc is not None or self.topk < 1:
-            return False
+            return None
         # the switches that choose between ways of the host-driven path ask for that path
         if any(name in os.environ for name in ("INFLLM_FETCH_AHEAD_ALWAYS", "INFLLM_NO_DMA_FETCH", "INFLLM_NO_DMA_ENGINE", "INFLLM_NO_STAGING_COPY",
                                                "INFLLM_NO_CALL_LISTS", "INFLLM_CALL_LISTS_ROOM", "INFLLM_PAGE_TABLE_KERNEL", "INFLLM_SCORE_MERGE_APART")):
-            return False
+            return None
         limit = self._resident_limit()
         if not limit or _Units.used.get(self._dev_index, 0) >= limit:
-            return False
-        return self._lib.infllm_resident_fits(ctypes.byref(self._resident_desc(64 if self.dim_head == 64 else HEAD_DIM))) == 1
+            return None
+        d = self._resident_desc(64 if self.dim_head == 64 else HEAD_DIM)
+        return d if self._lib.infllm_resident_fits(ctypes.byref(d)) == 1 else None
 
-    def _init_resident(self):
+    def _init_resident(self, d):
         dev, B, topk = self.device, self.num_units, self.topk
-        i32 = dict(dtype=torch.int32, device=dev)
         self._chunks = []                       # homes of the units: [_chunk_units, B, 2, Hkv, bs, D] each
-        self._chunk_units = self._units_per_chunk(self.unit_bytes)
+        self._chunk_units = d.units_per_chunk
         self._chunk_bytes = self._chunk_units * self.unit_bytes
         self._chunk_host = (ctypes.c_uint64 * 16)()
-        self._chunk_dev = torch.empty((16,), dtype=torch.int64, device=dev)
-        self._ids = torch.empty((B, topk), **i32)
-        self._pages = torch.empty((B * self.max_pages * ctypes.sizeof(_lib.Page),), dtype=torch.uint8, device=dev)
+        # addresses of the units' homes, and behind the 16 of them a page table and a selection
+        page_words = B * self.max_pages * ctypes.sizeof(_lib.Page) // 8
+        self._chunk_dev = self._tables = torch.empty((16 + page_words + (B * topk + 1) // 2,), dtype=torch.int64, device=dev)
         self._log, seq = _Units.take_log(self._dev_index, B * topk + 1)
         self._caches = (ctypes.c_void_p * B)(*[pol.handle for pol in self._policy])
-        d = self._resident_desc(self.head_width)
+        d.group_blocks = self._local_group
         d.d_ring_k_raw, d.d_ring_k_rot = self.ring_k_raw.data_ptr(), self.ring_k_rot.data_ptr()
         d.d_ring_v, d.d_ring_score, d.d_init_kv = self.ring_v.data_ptr(), self.ring_score.data_ptr(), self.init_kv.data_ptr()
-        d.d_pages, d.d_ids = self._pages.data_ptr(), self._ids.data_ptr()
+        d.d_pages = self._tables.data_ptr() + 8 * 16
+        d.d_ids = d.d_pages + 8 * page_words
         d.d_log, d.h_log = self._lib.infllm_host_device_pointer(self._log.data_ptr()), self._log.data_ptr()
         d.h_caches, d.d_inv_freq = ctypes.addressof(self._caches), self.inv_freq.data_ptr()
         d.distance_scale, d.softmax_scale = float(self.position_embedding.distance_scale), 1.0 / (self.dim_head ** 0.5)
@@ -399,7 +425,7 @@ class ContextManager:
         if self._timing_cap:
             check(self._lib.infllm_resident_timing(self._resident, self._timing_cap, self._timing_stride), "infllm_resident_timing")
         self._state = (ctypes.c_int64 * 10)()
-        self._streams = {torch.cuda.current_stream(dev).cuda_stream}
+        self._streams = {torch._C._cuda_getCurrentRawStream(self._dev_index)}
         self._rc = ResidentCall()
         self._rc_ref = ctypes.byref(self._rc)
         self._rc.h_chunks, self._rc.d_chunks = ctypes.addressof(self._chunk_host), self._chunk_dev.data_ptr()
@@ -429,7 +455,7 @@ class ContextManager:
                 grown = (ctypes.c_uint64 * (2 * n))()
                 grown[:n] = self._chunk_host[:]
                 table = torch.empty((2 * n,), dtype=torch.int64, device=self.device)
-                table[:n] = self._chunk_dev
+                table[:n] = self._chunk_dev[:n]
                 self._retire(self._chunk_dev)
                 self._chunk_host, self._chunk_dev = grown, table
                 self._rc.h_chunks, self._rc.d_chunks = ctypes.addressof(grown), table.data_ptr()
@@ -523,12 +549,11 @@ class ContextManager:
             self._call_scores = torch.empty((-(-rc.max_tokens // self.exc_block_size), self.num_units, cols), dtype=torch.float32, device=self.device)
             rc.d_call_scores, rc.scores_cols = self._call_scores.data_ptr(), cols
         B, H, D = self.num_units, self.unit_size, self.head_width
+        by_token = by_token and n > 1                            # (one token's rows lie the same either way)
         out = torch.empty((B, n, H, D) if by_token else (B, H, n, D), dtype=torch.bfloat16, device=q.device)
-        rc.d_q, rc.d_k, rc.d_v, rc.d_out, rc.n = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), n
-        rc.q_sb, rc.q_sh, rc.q_sl, _ = q.stride()
-        rc.k_sb, rc.k_sh, rc.k_sl, _ = k.stride()
-        rc.v_sb, rc.v_sh, rc.v_sl, _ = v.stride()
-        rc.o_sb, rc.o_sl, rc.o_sh = (n * H * D, H * D, D) if by_token else (n * H * D, D, n * D)
+        (q, q_ptr, q_st), (k, k_ptr, k_st), (v, v_ptr, v_st) = _addressed(q), _addressed(k), _addressed(v)
+        o_sh, o_sl = (D, H * D) if by_token else (n * D, D)
+        _CALL_ROWS.pack_into(rc, 0, q_ptr, k_ptr, v_ptr, *q_st[:3], *k_st[:3], *v_st[:3], out.data_ptr(), n * H * D, o_sh, o_sl, n)
         with self._call_buf.lock:
             status = self._lib.infllm_resident_append(self._resident, self._rc_ref, stream)
         if status:
@@ -539,7 +564,7 @@ class ContextManager:
         self.cursor = self.init_len + units * self.block_size
         if self.cache_strategy == "lru":
             self.load_count += -(-n // self.exc_block_size)
-        return out.permute(0, 2, 1, 3) if by_token else out
+        return out.transpose(1, 2) if by_token else out
 
     def _bind_resident_buffers(self, stream):
         """Workspaces of a call: dead between append() calls, so the managers that work on one stream share one set; the set's
@@ -560,11 +585,12 @@ class ContextManager:
                            lse=torch.empty((B * H * max(T, exc),), **f32), logits=torch.empty((B * H * self.n_local,), **f32),
                            base=torch.empty((blocks * B * self.topk,), dtype=torch.int32, device=self.device),
                            ticket=torch.zeros((1,), dtype=torch.int32, device=self.device))
+            buf.addresses = [("d_" + name, t.data_ptr()) for name, t in buf.items()]
             _CALL_BUFFERS[key] = buf
         self._call_buf = buf
         rc = self._rc
-        for name, t in buf.items():
-            setattr(rc, "d_" + name, t.data_ptr())
+        for name, address in buf.addresses:
+            setattr(rc, name, address)
         rc.part_rows, rc.part_rows2 = part_rows, self._part_rows2
         self._call_stream = stream
         self._streams.add(stream)
@@ -996,39 +1022,40 @@ class ContextManager:
             raise TypeError(f"the HIP path computes in bfloat16; got {q.dtype}, {k.dtype}, {v.dtype}")
         if k.device != dev or v.device != dev:
             raise ValueError(f"q, k and v must be on one device, got {dev}, {k.device}, {v.device}")
-        batch_size, _, input_length, width = q.shape
+        batch_size, heads, input_length, width = q.shape
         kv_shape = k.shape
-        t0, _, t2, t3 = kv_shape
+        t0, heads_kv, t2, t3 = kv_shape
         assert t0 == batch_size and t2 == input_length and t3 == width and v.shape == kv_shape, "q, keys and values differ in shape"
         assert q.is_cuda
+        units, unit_heads, unit_heads_kv = batch_size, heads, heads_kv
         if self.perhead:                                        # context_manager.py:690-704
-            heads, heads_kv = q.size(1), k.size(1)
             rep = lambda t: (t.reshape(batch_size, heads_kv, 1, input_length, -1)
                               .expand(batch_size, heads_kv, heads // heads_kv, input_length, -1)
                               .reshape(batch_size * heads, 1, input_length, -1))
             q, k, v = q.reshape(batch_size * heads, 1, input_length, -1), rep(k), rep(v)
+            units, unit_heads, unit_heads_kv = batch_size * heads, 1, 1
         if not self.initialized:
-            self.dim_head = q.size(3)
-            check_head_dim(self.dim_head)
-        if q.size(3) != self.dim_head:
-            raise ValueError(f"head_dim changed from {self.dim_head} to {q.size(3)}")
-        if not self.initialized:
+            self.dim_head = width
+            check_head_dim(width)
             self._init(q, k)
+        elif width != self.dim_head:
+            raise ValueError(f"head_dim changed from {self.dim_head} to {width}")
         if self._resident and not self._wants_resident():
             self._leave_resident()
-        if self.head_width != self.dim_head:
-            q, k, v = _widen(q, self.dim_head), _widen(k, self.dim_head), _widen(v, self.dim_head)
-        assert q.shape[:2] == (self.num_units, self.unit_size) and k.shape[1] == self.unit_size_kv
+        if self.head_width != width:
+            q, k, v = _widen(q, width), _widen(k, width), _widen(v, width)
+        assert units == self.num_units and unit_heads == self.unit_size and unit_heads_kv == self.unit_size_kv
 
-        q, k, v = rows16(q), rows16(k), rows16(v)
         if self._resident:
             out = self._append_resident(q, k, v, input_length, by_token)
             if out is not None:
-                out = self._own_width(out)
+                if self.head_width != width:
+                    out = self._own_width(out)
                 return out.reshape(batch_size, heads, input_length, -1) if self.perhead else out
             self._leave_resident()
             if self.head_width != q.shape[-1]:
                 q, k, v = (_widen(t, self.dim_head) for t in (q, k, v))
+        q, k, v = rows16(q), rows16(k), rows16(v)
         out = torch.empty((self.num_units, self.unit_size, input_length, self.head_width), dtype=torch.bfloat16, device=q.device)
         fa, ba = self._fa, self._ba
         fa.q_sb, fa.q_sh, fa.q_sl = q.stride(0), q.stride(1), q.stride(2)
