@@ -66,7 +66,7 @@ def _take_words(past_k, n, step_bytes, dev, stream):
         if held is not None and held[3] == stream and held[2] >= n and held[5] >= step_bytes:
             return held, 0
     head = -(-4 * n // 256) * 256
-    t = torch.empty((head + step_bytes,), dtype=torch.uint8, device=dev)
+    t = torch.empty(((head + step_bytes + 3) // 4,), dtype=torch.int32, device=dev)
     ptr = t.data_ptr()
     return (t, ptr, n, stream, ptr + head, step_bytes), 1
 
