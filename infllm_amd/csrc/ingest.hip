@@ -5,121 +5,134 @@
 
 namespace {
 
-// grid = (position tiles of 16, batch rows, kv heads): a workgroup rotates the query heads of one
-// kv-head group plus that group's key head, copies its value head, and leaves the sum of its
-// rotated-to-one-position queries over its positions in d_qpart (for the block's mean query; summed
-// before the rounding to bf16, so the mean query carries no rounding of its own).
+// grid = (position tiles of 16, batch rows, groups of KG kv heads): a workgroup rotates the query heads of its kv heads plus
+// their key heads, copies their value heads, and leaves the sum of its rotated-to-one-position queries over its positions in
+// d_qpart (for the block's mean query; summed before the rounding to bf16, so the mean query carries no rounding of its own).
 //
 // Angles (rope_angles): the rows the workgroup will rotate are requested from memory BEFORE that arithmetic, so the
 // two overlap.
 //
+// Bound by HBM, as long as the angles hide behind the rows (heads_together) and enough rows are on their way: the sums take their
+// 16 KB of LDS for a round of heads at a time, so that six workgroups are on a CU (for all four heads at once 41 KB and three: 8,192
+// tokens of 32 / 8 heads of 128 61.9 -> 53.3 us = 5.3 TB/s, 1,998 tokens 17.8 -> 14.6).
+//
 // D: head dimension (128 or 64).  qbar (optional): where the mean of the queries goes when the launch has a single
 // position tile (a decode step), whose partial sum is the whole sum.
-template <int D>
+template <int D, int KG>
 __global__ __launch_bounds__(256) void ingest_kernel(infllm_ingest_args a, float *qbar) {
     constexpr int kHalf = D / 2, C2 = D / 16;          // rotation pairs of a head; pairs of 16-byte chunks of a row
+    constexpr int kRound = 256 / (kPosPerBlock * C2);  // query heads that 256 threads rotate at once: 2 (4)
     __shared__ float2 cs_pos[kPosPerBlock][kHalf];
     __shared__ float2 cs_glb[kHalf];
-    __shared__ float red[4][kPosPerBlock][D];        // q_glb of 4 heads x 16 positions, for the partial sums
+    __shared__ float red[kRound][kPosPerBlock][D];   // their q_glb, for the partial sums
     const int tid = threadIdx.x;
-    const int b = blockIdx.y, g = blockIdx.z;
-    const int G = a.H / a.Hkv;
+    const int b = blockIdx.y, g0 = blockIdx.z * KG, ng = KG == 1 ? 1 : min(KG, a.Hkv - g0);
+    const int h0 = g0 * (a.H / a.Hkv), n_heads = ng * (a.H / a.Hkv);
     const int p0 = blockIdx.x * kPosPerBlock;
     const int np = min(kPosPerBlock, a.n - p0);
 
-    const bf16_t *q = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb;
-    const bf16_t *k = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh;
-    const bf16_t *v = (const bf16_t *)a.d_v + (int64_t)b * a.v_sb + (int64_t)g * a.v_sh;
-    bf16_t *q_loc = (bf16_t *)a.d_q_loc + (int64_t)b * a.H * a.n * D;
-    bf16_t *q_glb = (bf16_t *)a.d_q_glb + (int64_t)b * a.H * a.n * D;
-    const int64_t ring_g = ((int64_t)b * a.Hkv + g) * a.ring_cap * D;
-    bf16_t *rk_raw = (bf16_t *)a.d_ring_k_raw + ring_g;
-    bf16_t *rk_rot = (bf16_t *)a.d_ring_k_rot + ring_g;
-    bf16_t *rv = (bf16_t *)a.d_ring_v + ring_g;
+    const bf16_t *q = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h0 * a.q_sh;
+    const bf16_t *k = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g0 * a.k_sh;
+    const bf16_t *v = (const bf16_t *)a.d_v + (int64_t)b * a.v_sb + (int64_t)g0 * a.v_sh;
+    bf16_t *q_loc = (bf16_t *)a.d_q_loc + ((int64_t)b * a.H + h0) * a.n * D;
+    bf16_t *q_glb = (bf16_t *)a.d_q_glb + ((int64_t)b * a.H + h0) * a.n * D;
+    const int64_t ring_g = ((int64_t)b * a.Hkv + g0) * a.ring_cap * D;
     const int n_tiles = (a.n + kPosPerBlock - 1) / kPosPerBlock;
 
-    // ---- requests first: the first group of (up to) 4 query heads, the key head, the value head
-    constexpr int kQItems = 4 * kPosPerBlock * C2 / 256;   // 4 heads x 16 positions x 8 (4) chunk pairs over 256 threads
-    u32x4 q_lo[kQItems], q_hi[kQItems], k_lo, k_hi, v_row;
-    const int nh0 = min(4, G);
+    // ---- requests first: the first (up to) 4 query heads, the key heads, the value heads
+    constexpr int kQItems = 4 / kRound, kKItems = (KG * kPosPerBlock * C2 + 255) / 256, kVItems = (KG * kPosPerBlock * 2 * C2 + 255) / 256;
+    u32x4 q_lo[kQItems], q_hi[kQItems], k_lo[kKItems], k_hi[kKItems], v_row[kVItems];
+    const int qc = tid % C2, qp = tid / C2 % kPosPerBlock, qh = tid / (C2 * kPosPerBlock);      // of a round of heads
 #pragma unroll
     for (int i = 0; i < kQItems; ++i) {
-        const int e = tid + i * 256;
-        if (e < nh0 * np * C2) {
-            const int c = e % C2, p = e / C2 % np, hl = e / C2 / np;
-            const bf16_t *src = q + (int64_t)(g * G + hl) * a.q_sh + (int64_t)(p0 + p) * a.q_sl;
-            q_lo[i] = *(const u32x4 *)(src + c * 8);
-            q_hi[i] = *(const u32x4 *)(src + kHalf + c * 8);
+        if (qp < np && i * kRound + qh < n_heads) {
+            const bf16_t *src = q + (int64_t)(i * kRound + qh) * a.q_sh + (int64_t)(p0 + qp) * a.q_sl;
+            q_lo[i] = *(const u32x4 *)(src + qc * 8);
+            q_hi[i] = *(const u32x4 *)(src + kHalf + qc * 8);
         }
     }
-    if (tid < np * C2) {
-        const bf16_t *src = k + (int64_t)(p0 + tid / C2) * a.k_sl;
-        k_lo = *(const u32x4 *)(src + tid % C2 * 8);
-        k_hi = *(const u32x4 *)(src + kHalf + tid % C2 * 8);
+#pragma unroll
+    for (int i = 0; i < kKItems; ++i) {
+        const int e = tid + i * 256, c = e % C2, p = e / C2 % kPosPerBlock, kg = e / (C2 * kPosPerBlock);
+        if (p < np && kg < ng) {
+            const bf16_t *src = k + (int64_t)kg * a.k_sh + (int64_t)(p0 + p) * a.k_sl;
+            k_lo[i] = *(const u32x4 *)(src + c * 8);
+            k_hi[i] = *(const u32x4 *)(src + kHalf + c * 8);
+        }
     }
-    if (tid < np * 2 * C2) v_row = *(const u32x4 *)(v + (int64_t)(p0 + tid / (2 * C2)) * a.v_sl + tid % (2 * C2) * 8);
+#pragma unroll
+    for (int i = 0; i < kVItems; ++i) {
+        const int e = tid + i * 256, c = e % (2 * C2), p = e / (2 * C2) % kPosPerBlock, kg = e / (2 * C2 * kPosPerBlock);
+        if (p < np && kg < ng) v_row[i] = *(const u32x4 *)(v + (int64_t)kg * a.v_sh + (int64_t)(p0 + p) * a.v_sl + c * 8);
+    }
 
     // ---- angles
     rope_angles<kHalf>(a.pos0 + p0, np, a.glb_pos, a.distance_scale, a.d_inv_freq, cs_pos, cs_glb);
     __syncthreads();
 
-    // query heads of the group, 4 at a time: 8 threads per (head, position) row
-    for (int hg0 = 0; hg0 < G; hg0 += 4) {
-        const int nh = min(4, G - hg0);
+    // query heads, 4 at a time: C2 threads per (head, position) row
+    for (int hg0 = 0; hg0 < n_heads; hg0 += 4) {
 #pragma unroll
         for (int i = 0; i < kQItems; ++i) {
-            const int e = tid + i * 256;
-            if (e >= nh * np * C2) continue;
-            const int c = e % C2, p = e / C2 % np, hl = e / C2 / np;
-            const int h = g * G + hg0 + hl;
-            u32x4 lo = q_lo[i], hi = q_hi[i];
-            if (hg0 > 0) {
-                const bf16_t *src = q + (int64_t)h * a.q_sh + (int64_t)(p0 + p) * a.q_sl;
-                lo = *(const u32x4 *)(src + c * 8), hi = *(const u32x4 *)(src + kHalf + c * 8);
+            const int h = hg0 + i * kRound + qh;
+            if (qp < np && h < n_heads) {
+                u32x4 lo = q_lo[i], hi = q_hi[i];
+                if (hg0 > 0) {
+                    const bf16_t *src = q + (int64_t)h * a.q_sh + (int64_t)(p0 + qp) * a.q_sl;
+                    lo = *(const u32x4 *)(src + qc * 8), hi = *(const u32x4 *)(src + kHalf + qc * 8);
+                }
+                const int64_t o = ((int64_t)h * a.n + p0 + qp) * D;
+                Rot8 r = rotate8(lo, hi, &cs_pos[qp][qc * 8]);
+                *(u32x4 *)(q_loc + o + qc * 8) = r.lo;
+                *(u32x4 *)(q_loc + o + kHalf + qc * 8) = r.hi;
+                float raw[16];
+                r = rotate8(lo, hi, &cs_glb[qc * 8], raw);
+                *(u32x4 *)(q_glb + o + qc * 8) = r.lo;
+                *(u32x4 *)(q_glb + o + kHalf + qc * 8) = r.hi;
+                if (a.d_qpart || qbar) {
+                    *(f32x4 *)&red[qh][qp][qc * 8] = f32x4{raw[0], raw[1], raw[2], raw[3]};
+                    *(f32x4 *)&red[qh][qp][qc * 8 + 4] = f32x4{raw[4], raw[5], raw[6], raw[7]};
+                    *(f32x4 *)&red[qh][qp][kHalf + qc * 8] = f32x4{raw[8], raw[9], raw[10], raw[11]};
+                    *(f32x4 *)&red[qh][qp][kHalf + qc * 8 + 4] = f32x4{raw[12], raw[13], raw[14], raw[15]};
+                }
             }
-            int64_t o = ((int64_t)h * a.n + p0 + p) * D;
-            Rot8 r = rotate8(lo, hi, &cs_pos[p][c * 8]);
-            *(u32x4 *)(q_loc + o + c * 8) = r.lo;
-            *(u32x4 *)(q_loc + o + kHalf + c * 8) = r.hi;
-            float raw[16];
-            r = rotate8(lo, hi, &cs_glb[c * 8], raw);
-            *(u32x4 *)(q_glb + o + c * 8) = r.lo;
-            *(u32x4 *)(q_glb + o + kHalf + c * 8) = r.hi;
             if (a.d_qpart || qbar) {
-                *(f32x4 *)&red[hl][p][c * 8] = f32x4{raw[0], raw[1], raw[2], raw[3]};
-                *(f32x4 *)&red[hl][p][c * 8 + 4] = f32x4{raw[4], raw[5], raw[6], raw[7]};
-                *(f32x4 *)&red[hl][p][kHalf + c * 8] = f32x4{raw[8], raw[9], raw[10], raw[11]};
-                *(f32x4 *)&red[hl][p][kHalf + c * 8 + 4] = f32x4{raw[12], raw[13], raw[14], raw[15]};
+                __syncthreads();
+                const int d = tid % D, rh = tid / D, hs = hg0 + i * kRound + rh;
+                static_assert(kRound * D == 256);
+                if (hs < n_heads) {
+                    float s = 0.f;
+                    for (int p = 0; p < np; ++p) s += red[rh][p][d];          // fixed order
+                    if (qbar) qbar[((int64_t)b * a.H + h0 + hs) * D + d] = s * (1.f / (float)a.n);
+                    else a.d_qpart[(((int64_t)b * n_tiles + blockIdx.x) * a.H + h0 + hs) * D + d] = s;
+                }
+                __syncthreads();
             }
         }
-        if (a.d_qpart || qbar) {
-            __syncthreads();
-            for (int e = tid; e < nh * D; e += 256) {
-                const int d = e % D, hl = e / D;
-                float s = 0.f;
-                for (int p = 0; p < np; ++p) s += red[hl][p][d];          // fixed order
-                if (qbar) qbar[((int64_t)b * a.H + g * G + hg0 + hl) * D + d] = s * (1.f / (float)a.n);
-                else a.d_qpart[(((int64_t)b * n_tiles + blockIdx.x) * a.H + g * G + hg0 + hl) * D + d] = s;
-            }
-            __syncthreads();
-        }
     }
-    // key head: raw copy + rotated copy into the rings
-    if (tid < np * C2) {
-        const int c = tid % C2, p = tid / C2;
-        const int64_t o = ((a.pos0 + p0 + p) % a.ring_cap) * D;
-        *(u32x4 *)(rk_raw + o + c * 8) = k_lo;
-        *(u32x4 *)(rk_raw + o + kHalf + c * 8) = k_hi;
-        Rot8 r = rotate8(k_lo, k_hi, &cs_pos[p][c * 8]);
-        *(u32x4 *)(rk_rot + o + c * 8) = r.lo;
-        *(u32x4 *)(rk_rot + o + kHalf + c * 8) = r.hi;
+    // key heads: raw copy + rotated copy into the rings
+#pragma unroll
+    for (int i = 0; i < kKItems; ++i) {
+        const int e = tid + i * 256, c = e % C2, p = e / C2 % kPosPerBlock, kg = e / (C2 * kPosPerBlock);
+        if (p >= np || kg >= ng) continue;
+        const int64_t o = ring_g + (kg * a.ring_cap + (a.pos0 + p0 + p) % a.ring_cap) * D;
+        bf16_t *rk_raw = (bf16_t *)a.d_ring_k_raw + o, *rk_rot = (bf16_t *)a.d_ring_k_rot + o;
+        *(u32x4 *)(rk_raw + c * 8) = k_lo[i];
+        *(u32x4 *)(rk_raw + kHalf + c * 8) = k_hi[i];
+        Rot8 r = rotate8(k_lo[i], k_hi[i], &cs_pos[p][c * 8]);
+        *(u32x4 *)(rk_rot + c * 8) = r.lo;
+        *(u32x4 *)(rk_rot + kHalf + c * 8) = r.hi;
     }
-    // value head: plain copy
-    if (tid < np * 2 * C2) *(u32x4 *)(rv + ((a.pos0 + p0 + tid / (2 * C2)) % a.ring_cap) * D + tid % (2 * C2) * 8) = v_row;
+    // value heads: plain copy
+#pragma unroll
+    for (int i = 0; i < kVItems; ++i) {
+        const int e = tid + i * 256, c = e % (2 * C2), p = e / (2 * C2) % kPosPerBlock, kg = e / (2 * C2 * kPosPerBlock);
+        if (p < np && kg < ng) *(u32x4 *)((bf16_t *)a.d_ring_v + ring_g + (kg * a.ring_cap + (a.pos0 + p0 + p) % a.ring_cap) * D + c * 8) = v_row[i];
+    }
     // the score track of a new token starts at zero (context_manager.py:733-741)
-    for (int e = tid; e < G * np; e += 256) {
-        const int p = e % np, h = g * G + e / np;
-        a.d_ring_score[((int64_t)b * a.H + h) * a.ring_cap + (a.pos0 + p0 + p) % a.ring_cap] = 0.f;
+    for (int e = tid; e < n_heads * kPosPerBlock; e += 256) {
+        const int p = e % kPosPerBlock, h = h0 + e / kPosPerBlock;
+        if (p < np) a.d_ring_score[((int64_t)b * a.H + h) * a.ring_cap + (a.pos0 + p0 + p) % a.ring_cap] = 0.f;
     }
 }
 
@@ -290,9 +303,11 @@ extern "C" int infllm_ingest_dim(const infllm_ingest_args *a, int32_t dim, float
     INFLLM_REQUIRE(dim == 128 || dim == 64, "ingest: head_dim %d", dim);
     INFLLM_REQUIRE(!d_qbar || a->n <= kPosPerBlock, "ingest: the mean of %d queries takes more than one tile", a->n);
     if (a->n == 0) return 0;
-    dim3 grid((a->n + kPosPerBlock - 1) / kPosPerBlock, a->B, a->Hkv);
-    if (dim == 128) hipLaunchKernelGGL(ingest_kernel<128>, grid, dim3(256), 0, (hipStream_t)stream, *a, d_qbar);
-    else hipLaunchKernelGGL(ingest_kernel<64>, grid, dim3(256), 0, (hipStream_t)stream, *a, d_qbar);
+    const int kg = heads_together(a->n, a->B, a->H, a->Hkv);
+    const dim3 grid((a->n + kPosPerBlock - 1) / kPosPerBlock, a->B, (a->Hkv + kg - 1) / kg);
+    const auto kern = dim == 128 ? (kg == 4 ? ingest_kernel<128, 4> : kg == 2 ? ingest_kernel<128, 2> : ingest_kernel<128, 1>)
+                                 : (kg == 4 ? ingest_kernel<64, 4> : kg == 2 ? ingest_kernel<64, 2> : ingest_kernel<64, 1>);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, (hipStream_t)stream, *a, d_qbar);
     INFLLM_CHECK_LAUNCH("ingest");
     return 0;
 }

@@ -62,6 +62,16 @@ __device__ __forceinline__ void rope_angles(int64_t pos0, int np, int64_t glb_po
     }
 }
 
+// kv heads that a workgroup of a prompt's rows takes together: as many as make up to four query heads, where the workgroups of one
+// kv head each are more than the chip holds at once.  The angles are the chain of one wave, and the first waves of a CU's workgroups
+// share a SIMD: 36 key heads of 64 formed the angles of every 16 positions 36 times and waited for that SIMD and not for memory (ingest
+// of 4,096 tokens 45.2 -> 33.9 us, of 1,500 17.2 -> 13.2; causal staging of 4,096 24.0 -> 20.9).  Below the line neither form is the
+// faster one (300 - 450 tokens: 8 - 14 us either way), and copies of cached rows, in the same grid, want a workgroup for each head.
+inline int heads_together(int64_t n, int32_t B, int32_t H, int32_t Hkv) {
+    const int G = H / Hkv;
+    return G >= 3 || (n + kPosPerBlock - 1) / kPosPerBlock * B * Hkv <= 1024 ? 1 : G == 2 ? 2 : 4;
+}
+
 // One new position (a decode step) of one kv head: its query heads rotated to their position and to the one angle of the units,
 // its key and value into the rings, its scores at zero - what ingest_kernel does for a tile of one.  256 threads; cs: D float2.
 template <int D>

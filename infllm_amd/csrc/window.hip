@@ -36,69 +36,75 @@ struct StageJob {
 };
 
 // Bound by HBM for a prompt (a row read, one to three written), by the latency of the fp64 angles for a step.  grid =
-// (position tiles of 16, then pieces of the row copies; batch rows; kv heads): a workgroup rotates the query heads of a
-// kv head's group and its key head at 16 positions.  (One wave per row with its own sincos, a launch for every tensor and
+// (position tiles of 16, then pieces of the row copies; batch rows; groups of KG kv heads): a workgroup rotates the query heads of its
+// kv heads and their key heads at 16 positions.  (One wave per row with its own sincos, a launch for every tensor and
 // angle, and torch.cat for the cache: 13 launches and 2.1 x the bytes per call.)
-template <int D>
+template <int D, int KG>
 __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
     constexpr int HALF = D / 2, C2 = D / 16;           // chunk pairs of a row
     __shared__ float2 cs_pos[kPosPerBlock][HALF];
     __shared__ float2 cs_glb[HALF];
-    const int tid = threadIdx.x, b = blockIdx.y, g = blockIdx.z;
+    const int tid = threadIdx.x, b = blockIdx.y, g0 = blockIdx.z * KG, ng = KG == 1 ? 1 : min(KG, j.Hkv - g0);
     if ((int)blockIdx.x >= j.tiles) {
-        copy_rows<D, kCopyRows>(j.copy, (int)blockIdx.x - j.tiles, b, g);
+        for (int kg = 0; kg < ng; ++kg) copy_rows<D, kCopyRows>(j.copy, (int)blockIdx.x - j.tiles, b, g0 + kg);
         return;
     }
-    if (blockIdx.x == 0 && b == 0 && g == 0)
+    if (blockIdx.x == 0 && b == 0 && g0 == 0)
         for (int i = tid; i < j.n_clear; i += 256) j.clear[i] = 0;
-    const int G = j.H / j.Hkv;
+    const int h0 = g0 * (j.H / j.Hkv), n_heads = ng * (j.H / j.Hkv);
     const int p0 = blockIdx.x * kPosPerBlock, np = min(kPosPerBlock, j.n - p0);
-    // ---- requests first: up to four query heads, the key head, the value head
-    constexpr int kItems = 4 * kPosPerBlock * C2 / 256;                  // 2 (D = 128) or 1 (D = 64)
-    u32x4 q_lo[kItems], q_hi[kItems], k_lo, k_hi, v_row;
-    const bf16_t *q = j.q + (int64_t)b * j.q_sb;
+    // ---- requests first: up to four query heads, the key heads, the value heads
+    constexpr int kRound = 256 / (kPosPerBlock * C2), kItems = 4 / kRound;          // 2 (D = 128) or 1 (D = 64)
+    constexpr int kKItems = (KG * kPosPerBlock * C2 + 255) / 256, kVItems = (KG * kPosPerBlock * 2 * C2 + 255) / 256;
+    u32x4 q_lo[kItems], q_hi[kItems], k_lo[kKItems], k_hi[kKItems], v_row[kVItems];
+    const bf16_t *q = j.q + (int64_t)b * j.q_sb + (int64_t)h0 * j.q_sh;
+    const int qc = tid % C2, qp = tid / C2 % kPosPerBlock, qh = tid / (C2 * kPosPerBlock);
     if (j.do_q) {
 #pragma unroll
-        for (int i = 0; i < kItems; ++i) {
-            const int e = tid + i * 256, c = e % C2, p = e / C2 % kPosPerBlock, hl = e / C2 / kPosPerBlock;
-            if (hl < min(4, G) && p < np) {
-                const bf16_t *src = q + (int64_t)(g * G + hl) * j.q_sh + (int64_t)(p0 + p) * j.q_sl;
-                q_lo[i] = *(const u32x4 *)(src + c * 8);
-                q_hi[i] = *(const u32x4 *)(src + HALF + c * 8);
+        for (int i = 0; i < kItems; ++i)
+            if (i * kRound + qh < n_heads && qp < np) {
+                const bf16_t *src = q + (int64_t)(i * kRound + qh) * j.q_sh + (int64_t)(p0 + qp) * j.q_sl;
+                q_lo[i] = *(const u32x4 *)(src + qc * 8);
+                q_hi[i] = *(const u32x4 *)(src + HALF + qc * 8);
+            }
+    }
+    if (j.do_kv) {
+#pragma unroll
+        for (int i = 0; i < kKItems; ++i) {
+            const int e = tid + i * 256, c = e % C2, p = e / C2 % kPosPerBlock, kg = e / (C2 * kPosPerBlock);
+            if (p < np && kg < ng) {
+                const bf16_t *src = j.k + (int64_t)b * j.k_sb + (int64_t)(g0 + kg) * j.k_sh + (int64_t)(p0 + p) * j.k_sl;
+                k_lo[i] = *(const u32x4 *)(src + c * 8);
+                k_hi[i] = *(const u32x4 *)(src + HALF + c * 8);
             }
         }
-    }
-    const int kc = tid % C2, kp = tid / C2, vc = tid % (D / 8), vp = tid / (D / 8);
-    if (j.do_kv) {
-        if (kp < np) {
-            const bf16_t *src = j.k + (int64_t)b * j.k_sb + (int64_t)g * j.k_sh + (int64_t)(p0 + kp) * j.k_sl;
-            k_lo = *(const u32x4 *)(src + kc * 8);
-            k_hi = *(const u32x4 *)(src + HALF + kc * 8);
+#pragma unroll
+        for (int i = 0; i < kVItems; ++i) {
+            const int e = tid + i * 256, c = e % (2 * C2), p = e / (2 * C2) % kPosPerBlock, kg = e / (2 * C2 * kPosPerBlock);
+            if (p < np && kg < ng) v_row[i] = *(const u32x4 *)(j.v + (int64_t)b * j.v_sb + (int64_t)(g0 + kg) * j.v_sh + (int64_t)(p0 + p) * j.v_sl + c * 8);
         }
-        if (vp < np) v_row = *(const u32x4 *)(j.v + (int64_t)b * j.v_sb + (int64_t)g * j.v_sh + (int64_t)(p0 + vp) * j.v_sl + vc * 8);
     }
     rope_angles<HALF>(j.pos0 + p0, np, j.glb_pos, j.distance_scale, j.inv_freq, cs_pos, cs_glb);
     __syncthreads();
     if (j.do_q) {
-        for (int hg0 = 0; hg0 < G; hg0 += 4) {
+        for (int hg0 = 0; hg0 < n_heads; hg0 += 4) {
 #pragma unroll
             for (int i = 0; i < kItems; ++i) {
-                const int e = tid + i * 256, c = e % C2, p = e / C2 % kPosPerBlock, hl = e / C2 / kPosPerBlock;
-                if (hl >= min(4, G - hg0) || p >= np) continue;
-                const int h = g * G + hg0 + hl;
+                const int hl = hg0 + i * kRound + qh;
+                if (hl >= n_heads || qp >= np) continue;
                 u32x4 lo = q_lo[i], hi = q_hi[i];
                 if (hg0 > 0) {
-                    const bf16_t *src = q + (int64_t)h * j.q_sh + (int64_t)(p0 + p) * j.q_sl;
-                    lo = *(const u32x4 *)(src + c * 8), hi = *(const u32x4 *)(src + HALF + c * 8);
+                    const bf16_t *src = q + (int64_t)hl * j.q_sh + (int64_t)(p0 + qp) * j.q_sl;
+                    lo = *(const u32x4 *)(src + qc * 8), hi = *(const u32x4 *)(src + HALF + qc * 8);
                 }
-                const int64_t o = (((int64_t)b * j.H + h) * j.n + p0 + p) * D;
-                Rot8 r = rotate8(lo, hi, &cs_pos[p][c * 8]);
-                *(u32x4 *)(j.q_loc + o + c * 8) = r.lo;
-                *(u32x4 *)(j.q_loc + o + HALF + c * 8) = r.hi;
+                const int64_t o = (((int64_t)b * j.H + h0 + hl) * j.n + p0 + qp) * D;
+                Rot8 r = rotate8(lo, hi, &cs_pos[qp][qc * 8]);
+                *(u32x4 *)(j.q_loc + o + qc * 8) = r.lo;
+                *(u32x4 *)(j.q_loc + o + HALF + qc * 8) = r.hi;
                 if (j.q_glb) {
-                    r = rotate8(lo, hi, &cs_glb[c * 8]);
-                    *(u32x4 *)(j.q_glb + o + c * 8) = r.lo;
-                    *(u32x4 *)(j.q_glb + o + HALF + c * 8) = r.hi;
+                    r = rotate8(lo, hi, &cs_glb[qc * 8]);
+                    *(u32x4 *)(j.q_glb + o + qc * 8) = r.lo;
+                    *(u32x4 *)(j.q_glb + o + HALF + qc * 8) = r.hi;
                 }
             }
         }
@@ -109,27 +115,33 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
             const int r = j.c_first + p;
             return r < j.c_head ? r : r >= j.c_tail ? j.c_head + r - j.c_tail : -1;
         };
-        if (kp < np) {
-            bf16_t *dst = j.dk + (int64_t)b * j.dk_sb + (int64_t)g * j.dk_sh + (int64_t)(p0 + kp) * D;
-            const Rot8 r = rotate8(k_lo, k_hi, &cs_pos[kp][kc * 8]);
-            *(u32x4 *)(dst + kc * 8) = r.lo;
-            *(u32x4 *)(dst + HALF + kc * 8) = r.hi;
-            const int at = second(p0 + kp);
+#pragma unroll
+        for (int i = 0; i < kKItems; ++i) {
+            const int e = tid + i * 256, c = e % C2, p = e / C2 % kPosPerBlock, kg = e / (C2 * kPosPerBlock);
+            if (p >= np || kg >= ng) continue;
+            bf16_t *dst = j.dk + (int64_t)b * j.dk_sb + (int64_t)(g0 + kg) * j.dk_sh + (int64_t)(p0 + p) * D;
+            const Rot8 r = rotate8(k_lo[i], k_hi[i], &cs_pos[p][c * 8]);
+            *(u32x4 *)(dst + c * 8) = r.lo;
+            *(u32x4 *)(dst + HALF + c * 8) = r.hi;
+            const int at = second(p0 + p);
             if (at >= 0) {
-                dst = j.ck + (int64_t)b * j.ck_sb + (int64_t)g * j.ck_sh + (int64_t)at * D;
-                *(u32x4 *)(dst + kc * 8) = r.lo;
-                *(u32x4 *)(dst + HALF + kc * 8) = r.hi;
+                dst = j.ck + (int64_t)b * j.ck_sb + (int64_t)(g0 + kg) * j.ck_sh + (int64_t)at * D;
+                *(u32x4 *)(dst + c * 8) = r.lo;
+                *(u32x4 *)(dst + HALF + c * 8) = r.hi;
             }
-            if (p0 + kp < j.n_raw) {
-                bf16_t *raw = j.raw + (int64_t)b * j.raw_sb + (int64_t)g * j.raw_sh + (int64_t)(p0 + kp) * D;
-                *(u32x4 *)(raw + kc * 8) = k_lo;
-                *(u32x4 *)(raw + HALF + kc * 8) = k_hi;
+            if (p0 + p < j.n_raw) {
+                bf16_t *raw = j.raw + (int64_t)b * j.raw_sb + (int64_t)(g0 + kg) * j.raw_sh + (int64_t)(p0 + p) * D;
+                *(u32x4 *)(raw + c * 8) = k_lo[i];
+                *(u32x4 *)(raw + HALF + c * 8) = k_hi[i];
             }
         }
-        if (vp < np) {
-            *(u32x4 *)(j.dv + (int64_t)b * j.dv_sb + (int64_t)g * j.dv_sh + (int64_t)(p0 + vp) * D + vc * 8) = v_row;
-            const int at = second(p0 + vp);
-            if (at >= 0) *(u32x4 *)(j.cv + (int64_t)b * j.cv_sb + (int64_t)g * j.cv_sh + (int64_t)at * D + vc * 8) = v_row;
+#pragma unroll
+        for (int i = 0; i < kVItems; ++i) {
+            const int e = tid + i * 256, c = e % (2 * C2), p = e / (2 * C2) % kPosPerBlock, kg = e / (2 * C2 * kPosPerBlock);
+            if (p >= np || kg >= ng) continue;
+            *(u32x4 *)(j.dv + (int64_t)b * j.dv_sb + (int64_t)(g0 + kg) * j.dv_sh + (int64_t)(p0 + p) * D + c * 8) = v_row[i];
+            const int at = second(p0 + p);
+            if (at >= 0) *(u32x4 *)(j.cv + (int64_t)b * j.cv_sb + (int64_t)(g0 + kg) * j.cv_sh + (int64_t)at * D + c * 8) = v_row[i];
         }
     }
 }
@@ -139,9 +151,11 @@ int launch_stage_rows(StageJob &j, int dim, void *stream) {
     for (const RowCopy &c : j.copy) pieces += (c.n + kCopyRows - 1) / kCopyRows;
     j.tiles = j.do_q || j.do_kv ? (j.n + kPosPerBlock - 1) / kPosPerBlock : 0;
     if (j.tiles + pieces == 0) return 0;
-    const dim3 grid(j.tiles + pieces, j.B, j.Hkv);
-    if (dim == 128) hipLaunchKernelGGL(stage_rows_kernel<128>, grid, dim3(256), 0, (hipStream_t)stream, j);
-    else hipLaunchKernelGGL(stage_rows_kernel<64>, grid, dim3(256), 0, (hipStream_t)stream, j);
+    const int kg = heads_together(j.n, j.B, j.H, j.Hkv);
+    const dim3 grid(j.tiles + pieces, j.B, (j.Hkv + kg - 1) / kg);
+    const auto kern = dim == 128 ? (kg == 4 ? stage_rows_kernel<128, 4> : kg == 2 ? stage_rows_kernel<128, 2> : stage_rows_kernel<128, 1>)
+                                 : (kg == 4 ? stage_rows_kernel<64, 4> : kg == 2 ? stage_rows_kernel<64, 2> : stage_rows_kernel<64, 1>);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, (hipStream_t)stream, j);
     INFLLM_CHECK_LAUNCH("stage_rows");
     return 0;
 }
