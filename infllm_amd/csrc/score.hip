@@ -284,6 +284,11 @@ struct BlockEnd {
     MergeJob merge;                    // the block's partials (out NULL: merged before)
     int32_t n_carve, n_score, n_copy, n_early;     // workgroups of each kind (carve, score, early, copy), those that merge behind them
     int32_t cap, slot0, win;           // rows of the ring; that of the first key of the first scoring workgroup; the window
+    // The keys that are scored first, then the others in ascending order: those of the block's own first queries, masked for some of them and
+    // seen by all, are the longest.  They were the last but one, on the CUs that carve and score already, and the launch waited for
+    // them (32.5 us behind the first workgroup's start, most others 25 to 29).  Prompts of 16,001 / 131,072 tokens, 32 heads of 128:
+    // 2,613 -> 2,575 / 25,035 -> 24,602 us; 24,300 with 36 heads of 64, whose launch waits for the ranking: unchanged.
+    int32_t first_tile;
     // units that leave
     const bf16_t *ring_k_raw;
     int64_t t0;                        // their first key, and its row
@@ -634,10 +639,10 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(Block
     if (x < n_score) {
         const BlockEnd &j = arguments();
         const infllm_score_args &a = j.s;
-        const int rows = a.B * a.H, tile = x / rows;
-        int b, h;
-        head_of(a, x - tile * rows, b, h);
         constexpr int kKeys = 128 * KS;
+        const int rows = a.B * a.H, nth = x / rows, tile = nth == 0 ? j.first_tile : nth - (nth <= j.first_tile);
+        int b, h;
+        head_of(a, x - nth * rows, b, h);
         const int64_t jg = a.j_lo / (32 * KS) * (32 * KS) + (int64_t)tile * kKeys;
         const int slot = j.slot0 + tile * kKeys;
         const int lo = (int)max(a.j_lo - jg, (int64_t)0), hi = (int)min(a.j_hi - jg, (int64_t)kKeys);
@@ -816,6 +821,7 @@ static int block_end_launch(BlockEnd &j, bool scores, hipStream_t st) {
         const int64_t tiles = (a.j_hi - 1) / wave_keys - a.j_lo / wave_keys + 1;
         j.n_score = (int32_t)((tiles + 3) / 4 * a.B * a.H);
         j.slot0 = (int32_t)(a.j_lo % a.cap - a.j_lo % wave_keys);       // (below 0: rows that do not count)
+        j.first_tile = (int32_t)std::max<int64_t>(0, std::min((a.offset - a.j_lo / wave_keys * wave_keys) / (4 * wave_keys), (tiles + 3) / 4 - 1));
     }
     const int64_t copies = (int64_t)2 * a.B * a.Hkv * j.n_units * j.bs * (D / 8), pieces = j.merge.out ? (int64_t)a.B * a.H * a.Lq * (D / 8) : 0;
     INFLLM_REQUIRE(copies < (1ll << 32), "block_end: copy too large");
