@@ -321,6 +321,15 @@ struct BlockEnd {
 constexpr int kQRows = 64;                             // queries of a stage
 template <int D>
 constexpr size_t kQBytes = (size_t)3 * kQRows * D * sizeof(bf16_t);
+// A carving workgroup's stages: heads of 64 have room for 128 queries, of 32 keys a wave four steps instead of two, and the next block
+// waits for them (prompt of 24,300 tokens, 36 heads: 3,105 -> 3,089 us; the scores' own stages, four steps as they are, 0.5 % slower
+// with 128).  Heads of 128 have room for two stages of 96: 0.2 % slower, the scores' 2.8 %.
+template <int D>
+constexpr int kCarveRows = D == 64 ? 128 : 64;
+template <int D>
+constexpr int kCarveBufs = D == 64 ? 2 : 3;
+template <int D>
+constexpr size_t kCarveBytes = (size_t)kCarveBufs<D> * kCarveRows<D> * D * sizeof(bf16_t);
 
 template <int D, int KS, bool JOIN, int QR = kQRows, int NB = 3, int QG = 1>
 __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartSets lps, int b, int h, int64_t jg, int slot, int cap, int lo, int hi, int first,
@@ -560,7 +569,7 @@ __device__ __forceinline__ void carve_unit(const BlockEnd &j, int h, int u, int 
     const int own_row = wave * 32 + col;
     const float track = own_row < bs ? a.d_score[(int64_t)b * a.score_sb + (int64_t)h * a.score_sh + slot_of(own_row)] : 0.f;
     float sum[1];
-    key_sums<D, 1, true>(a, j.merge.ps, b, h, j.t0 + (int64_t)u * bs, slot, j.cap, 0, bs, 0, j.win, INFINITY, lds, sum);
+    key_sums<D, 1, true, kCarveRows<D>, kCarveBufs<D>>(a, j.merge.ps, b, h, j.t0 + (int64_t)u * bs, slot, j.cap, 0, bs, 0, j.win, INFINITY, lds, sum);
     __syncthreads();                                             // (the queries' place is free)
     uint64_t *rank_key = (uint64_t *)lds;
     int32_t *chosen = (int32_t *)(rank_key + kCarveMaxUnit);
@@ -813,7 +822,7 @@ int score_launch_merged(const infllm_score_args *a, const MergeJob *job, float e
 
 template <int D>
 static int block_end_launch(BlockEnd &j, bool scores, hipStream_t st) {
-    static_assert(sizeof(RankLds<kRankCpl<D>>) <= kQBytes<D> && kCarveMaxUnit * 16 + 4 <= kQBytes<D>, "LDS of a workgroup");
+    static_assert(kCarveBytes<D> >= kQBytes<D> && kCarveRows<D> >= kQRows && sizeof(RankLds<kRankCpl<D>>) <= kCarveBytes<D> && kCarveMaxUnit * 16 + 4 <= kCarveBytes<D>, "LDS of a workgroup");
     const infllm_score_args &a = j.s;
     const bool wide = scores && wide_waves(a);
     if (scores) {
@@ -830,7 +839,7 @@ static int block_end_launch(BlockEnd &j, bool scores, hipStream_t st) {
     INFLLM_REQUIRE(wgs < (1ll << 31), "block_end: grid too large");
     if (wgs == 0) return 0;
     const auto kern = wide ? block_end_kernel<D, 2> : block_end_kernel<D, 1>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(256), kQBytes<D> + (size_t)(a.Lq + kQRows - 1) / kQRows * kQRows * sizeof(float), st, j);
+    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(256), kCarveBytes<D> + (size_t)(a.Lq + kCarveRows<D> - 1) / kCarveRows<D> * kCarveRows<D> * sizeof(float), st, j);
     INFLLM_CHECK_LAUNCH("block_end");
     return 0;
 }
