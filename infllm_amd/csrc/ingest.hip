@@ -39,6 +39,7 @@ __global__ __launch_bounds__(256) void ingest_kernel(infllm_ingest_args a, float
     const int64_t ring_g = ((int64_t)b * a.Hkv + g0) * a.ring_cap * D;
     const int n_tiles = (a.n + kPosPerBlock - 1) / kPosPerBlock;
 
+    const float freq = rope_freq<kHalf>(a.d_inv_freq);
     // ---- requests first: the first (up to) 4 query heads, the key heads, the value heads
     constexpr int kQItems = 4 / kRound, kKItems = (KG * kPosPerBlock * C2 + 255) / 256, kVItems = (KG * kPosPerBlock * 2 * C2 + 255) / 256;
     u32x4 q_lo[kQItems], q_hi[kQItems], k_lo[kKItems], k_hi[kKItems], v_row[kVItems];
@@ -67,7 +68,7 @@ __global__ __launch_bounds__(256) void ingest_kernel(infllm_ingest_args a, float
     }
 
     // ---- angles
-    rope_angles<kHalf>(a.pos0 + p0, np, a.glb_pos, a.distance_scale, a.d_inv_freq, cs_pos, cs_glb);
+    rope_angles<kHalf>(a.pos0 + p0, np, a.glb_pos, a.distance_scale, freq, cs_pos, cs_glb);
     __syncthreads();
 
     // query heads, 4 at a time: C2 threads per (head, position) row

@@ -601,6 +601,18 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
     const int n_waves = n_wgs * waves_per_wg;
     int n = blockIdx.x * waves_per_wg + (threadIdx.x >> 6);     // rows n, n + n_waves, ... belong to this wave
     auto in_row = [&](int j) { return !TAIL || j * 512 + lane * 8 < C; };
+    float freq = 0.f;
+    u32x4 q_lo{}, q_hi{};                                        // (C <= 16 * kRetrThreads: eight pairs a thread)
+    if constexpr (FRONT) {                                       // the query ahead of the rows: it is waited for first
+        const infllm_ingest_args &in = front.in;
+        const int c2 = front.dim / 16, h = (int)threadIdx.x / c2;
+        freq = in.d_inv_freq[(int)threadIdx.x & (front.dim / 2 - 1)];
+        if (h < in.H) {
+            const bf16_t *src = (const bf16_t *)in.d_q + (int64_t)front.b * in.q_sb + (int64_t)h * in.q_sh + ((int)threadIdx.x - h * c2) * 8;
+            q_lo = *(const u32x4 *)src, q_hi = *(const u32x4 *)(src + front.dim / 2);
+        }
+        asm volatile("" ::: "memory");
+    }
     u32x4 w[ROWS][CPL];
 #pragma unroll
     for (int r = 0; r < ROWS; ++r)
@@ -613,14 +625,9 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
         __shared__ float2 cs[kD / 2];
         const infllm_ingest_args &in = front.in;
         const int half = front.dim / 2, c2 = front.dim / 16, tid = threadIdx.x, h = tid / c2, c = (tid - h * c2) * 8;
-        u32x4 lo{}, hi{};                                        // (C <= 16 * kRetrThreads: eight pairs a thread)
-        if (h < in.H) {
-            const bf16_t *src = (const bf16_t *)in.d_q + (int64_t)front.b * in.q_sb + (int64_t)h * in.q_sh + c;
-            lo = *(const u32x4 *)src, hi = *(const u32x4 *)(src + half);
-        }
         if (tid < half) {
             double sn, cn;
-            sincos((double)in.glb_pos * in.distance_scale * (double)in.d_inv_freq[tid], &sn, &cn);
+            sincos((double)in.glb_pos * in.distance_scale * (double)freq, &sn, &cn);
             cs[tid] = make_float2((float)cn, (float)sn);
         }
         if (TAIL)
@@ -628,7 +635,7 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
         __syncthreads();
         if (h < in.H) {
             float raw[16];
-            rotate8(lo, hi, cs + c, raw);
+            rotate8(q_lo, q_hi, cs + c, raw);
             float *dst = qs + h * front.dim + c;
 #pragma unroll
             for (int i = 0; i < 4; ++i) *(f32x4 *)(dst + (i >> 1) * half + (i & 1) * 4) = f32x4{raw[4 * i], raw[4 * i + 1], raw[4 * i + 2], raw[4 * i + 3]};

@@ -30,17 +30,26 @@ __device__ __forceinline__ Rot8 rotate8(u32x4 xlo, u32x4 xhi, const float2 *cs, 
     return r;
 }
 
+// This thread's frequency for rope_angles, to be asked for in front of the rows: what a wave requests comes back in that order, and the
+// angles' chain is to run while the rows are on their way.  (A step's chain began when the last of the rows in front of it had come.)
+template <int HALF>
+__device__ __forceinline__ float rope_freq(const float *inv_freq) {
+    const float f = inv_freq[threadIdx.x % HALF];
+    asm volatile("" ::: "memory");                               // (no later load goes ahead of it)
+    return f;
+}
+
 // cos / sin of (position x frequency) for the np <= 16 positions from pos0 on and for the one angle of position glb_pos,
 // by a workgroup of at least HALF * 2 threads (HALF = head_dim / 2 frequencies).  Only the FIRST position and the step of
 // one position are evaluated (fp64 sincos, one call per thread); the other positions follow by the angle-addition
 // recurrence in fp64, whose error after 15 steps is a few 1e-16 - far below the fp32 value the rotation consumes.  The
 // caller's barrier follows.
 template <int HALF>
-__device__ __forceinline__ void rope_angles(int64_t pos0, int np, int64_t glb_pos, double distance_scale, const float *inv_freq,
+__device__ __forceinline__ void rope_angles(int64_t pos0, int np, int64_t glb_pos, double distance_scale, float freq,
                                             float2 (*cs_pos)[HALF], float2 *cs_glb) {
     const int tid = threadIdx.x;
     if (tid < HALF) {
-        const double w = distance_scale * (double)inv_freq[tid];
+        const double w = distance_scale * (double)freq;
         double s, c;
         sincos((double)pos0 * w, &s, &c);
         cs_pos[0][tid] = make_float2((float)c, (float)s);
@@ -57,7 +66,7 @@ __device__ __forceinline__ void rope_angles(int64_t pos0, int np, int64_t glb_po
     } else if (tid < 2 * HALF) {
         const int f = tid - HALF;
         double s, c;
-        sincos((double)glb_pos * distance_scale * (double)inv_freq[f], &s, &c);
+        sincos((double)glb_pos * distance_scale * (double)freq, &s, &c);
         cs_glb[f] = make_float2((float)c, (float)s);
     }
 }
@@ -79,6 +88,7 @@ __device__ __forceinline__ void ingest_one(const infllm_ingest_args &a, int b, i
     constexpr int HALF = D / 2, C2 = D / 16;
     const int tid = threadIdx.x, G = a.H / a.Hkv;
     const bf16_t *q = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)g * G * a.q_sh;
+    const float freq = rope_freq<HALF>(a.d_inv_freq);
     u32x4 lo{}, hi{}, k_lo{}, k_hi{}, v_row{};
     if (tid < G * C2) {                                      // (more than 32 (64) heads: the rest below)
         lo = *(const u32x4 *)(q + (int64_t)(tid / C2) * a.q_sh + tid % C2 * 8);
@@ -89,7 +99,7 @@ __device__ __forceinline__ void ingest_one(const infllm_ingest_args &a, int b, i
         k_lo = *(const u32x4 *)src, k_hi = *(const u32x4 *)(src + HALF);
     }
     if (tid < 2 * C2) v_row = *(const u32x4 *)((const bf16_t *)a.d_v + (int64_t)b * a.v_sb + (int64_t)g * a.v_sh + tid * 8);
-    rope_angles<HALF>(a.pos0, 1, a.glb_pos, a.distance_scale, a.d_inv_freq, (float2(*)[HALF])cs, cs + HALF);
+    rope_angles<HALF>(a.pos0, 1, a.glb_pos, a.distance_scale, freq, (float2(*)[HALF])cs, cs + HALF);
     __syncthreads();
     for (int e = tid; e < G * C2; e += 256) {
         const int c = e % C2, h = e / C2;

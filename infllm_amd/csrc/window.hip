@@ -53,6 +53,7 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
         for (int i = tid; i < j.n_clear; i += 256) j.clear[i] = 0;
     const int h0 = g0 * (j.H / j.Hkv), n_heads = ng * (j.H / j.Hkv);
     const int p0 = blockIdx.x * kPosPerBlock, np = min(kPosPerBlock, j.n - p0);
+    const float freq = rope_freq<HALF>(j.inv_freq);
     // ---- requests first: up to four query heads, the key heads, the value heads
     constexpr int kRound = 256 / (kPosPerBlock * C2), kItems = 4 / kRound;          // 2 (D = 128) or 1 (D = 64)
     constexpr int kKItems = (KG * kPosPerBlock * C2 + 255) / 256, kVItems = (KG * kPosPerBlock * 2 * C2 + 255) / 256;
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
             if (p < np && kg < ng) v_row[i] = *(const u32x4 *)(j.v + (int64_t)b * j.v_sb + (int64_t)(g0 + kg) * j.v_sh + (int64_t)(p0 + p) * j.v_sl + c * 8);
         }
     }
-    rope_angles<HALF>(j.pos0 + p0, np, j.glb_pos, j.distance_scale, j.inv_freq, cs_pos, cs_glb);
+    rope_angles<HALF>(j.pos0 + p0, np, j.glb_pos, j.distance_scale, freq, cs_pos, cs_glb);
     __syncthreads();
     if (j.do_q) {
         for (int hg0 = 0; hg0 < n_heads; hg0 += 4) {
