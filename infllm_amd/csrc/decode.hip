@@ -82,8 +82,18 @@ __device__ __forceinline__ void leave_rows(const StepRows &f, int b, int g, floa
 // while the chip waits.  Here the others attend the window meanwhile, two thirds of the keys, which need no selection.  (Kernels of a
 // step, 32 heads of 128: behind 64K tokens scores with selection 12.5 + attention 13.4 us, so 8.4 + 12.8; behind 512K 17.1 + 12.8,
 // 11.8 + 14.6.  The window attended in the launch of the scores instead, beside the selection there: 18.5 + 9.8 and 25.7 + 9.6.)
+//
+// A split is a few microseconds of rows between a start and an end that are as long, so both are kept short.  What the host can divide it
+// divides (DecodePlan), and a workgroup finds its block in two trips to the arguments, not in some for every range.  At the end a wave
+// joins its four row groups by itself, and the waves' sums, each scaled to its wave's maximum, are read behind one barrier.  (The ranges walked
+// by every wave, the maxima of all 16 row groups read by all of them behind a barrier of their own: one token behind 64K / 512K
+// tokens 25.0 / 31.3 us a pass, 24.3 / 29.4 now, causal over 32,768 31.5 and 30.8.)
+struct DecodePlan {
+    int32_t G, chunks;                     // query heads of a kv head; workgroups that share them
+    int32_t end[kDecodeSegs];              // blocks of the ranges up to this one's last; behind the last range: INT32_MAX
+};
 template <int D, int NG, bool LOGITS, bool JOIN, typename Front = NoFront, bool SELECT = false>
-__global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(DecodeJob j, Front f) {
+__global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(DecodeJob j, DecodePlan plan, Front f) {
     constexpr bool FRONT = !std::is_same_v<Front, NoFront>;
     constexpr int KK = D / 32;                     // k-steps of the first MFMA
     constexpr int LPR = D / 8;                     // lanes that hold a value row, 16 bytes each
@@ -93,11 +103,12 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     constexpr int kRed = kDecWaves * GRP * NG * D;
     __shared__ __attribute__((aligned(16))) float red_room[!JOIN || kRed > kDecWaves * kWave * kJoin ? kRed : kDecWaves * kWave * kJoin];
     float(*red)[GRP][NG][D] = (float(*)[GRP][NG][D])red_room;
-    __shared__ float sm[kDecWaves][4][NG], sl[kDecWaves][4][NG];
+    __shared__ float sm[kDecWaves][NG], sl[kDecWaves][NG];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int col = lane & 15, rg = lane >> 4;
-    const int G = j.H / j.Hkv, chunks = (G + NG - 1) / NG;
-    const int split = blockIdx.x, g = blockIdx.y / chunks, c = blockIdx.y % chunks, b = blockIdx.z, n_split = gridDim.x;
+    const int G = plan.G, split = blockIdx.x, b = blockIdx.z, n_split = gridDim.x;
+    int g = blockIdx.y, c = 0;
+    if (plan.chunks > 1) g = (int)blockIdx.y / plan.chunks, c = (int)blockIdx.y - g * plan.chunks;
     // the ranges that this workgroup's split is one of, and which one of how many
     const bool lead = SELECT && split < j.lead_splits;
     const int seg_lo = SELECT && !lead ? j.lead_segs : 0, seg_hi = lead ? j.lead_segs : j.n_seg;
@@ -120,9 +131,9 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     const float lazy = kLazyDec / scale;
 
     // ---- the list of blocks: every range rounded up to whole blocks (units: every unit by itself)
-    int n_blocks = 0;
-    for (int s = seg_lo; s < seg_hi; ++s) n_blocks += (j.seg[s].rows + kDecodeBlock - 1) / kDecodeBlock * (j.seg[s].n_ids > 0 ? j.seg[s].n_ids : 1);
-    const int b_lo = (int)((int64_t)n_blocks * part / n_part), b_hi = (int)((int64_t)n_blocks * (part + 1) / n_part);
+    const int seg_first = seg_lo > 0 ? plan.end[seg_lo - 1] : 0, n_blocks = (seg_hi > 0 ? plan.end[seg_hi - 1] : 0) - seg_first;
+    const int each = n_blocks / n_part, over = n_blocks - each * n_part;                   // (of n_blocks * part / n_part, below)
+    const int b_lo = seg_first + each * part + over * part / n_part, b_hi = seg_first + each * (part + 1) + over * (part + 1) / n_part;
     __shared__ int32_t chosen[SELECT ? kSelectMost : 1];
     if constexpr (SELECT) {
         static_assert(sizeof(SelectLds<kDecWaves * kWave>) <= sizeof(red_room));
@@ -138,32 +149,28 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         int valid, q, row;                         // rows of the block, which query, where its logits go (-1: nowhere)
     };
     auto find = [&](int blk) {                     // wave-uniform
-        Block r{nullptr, nullptr, 0, 0, -1};
-        for (int s = seg_lo; s < seg_hi; ++s) {
-            const DecodeSeg &sg = j.seg[s];
-            const int per = (sg.rows + kDecodeBlock - 1) / kDecodeBlock, n = sg.n_ids > 0 ? per * sg.n_ids : per;
-            if (blk >= n) {
-                blk -= n;
-                continue;
-            }
-            r.q = sg.q;
-            if (sg.n_ids > 0) {
-                const int i = blk / per, r0 = (blk - i * per) * kDecodeBlock;
-                const int u = __builtin_amdgcn_readfirstlane(SELECT ? chosen[i] : sg.ids ? sg.ids[(int64_t)b * sg.n_ids + i] : i);
-                const int ch = u / j.per_chunk;
-                const bf16_t *base = (const bf16_t *)(uintptr_t)j.chunk[ch] + (int64_t)(u - ch * j.per_chunk) * j.unit_elems + (int64_t)b * j.row_elems +
-                                     (int64_t)g * j.unit_sh + (int64_t)r0 * D;
-                r.k = base;
-                r.v = base + j.unit_v_off;
-                r.valid = min(kDecodeBlock, sg.rows - r0);
-            } else {
-                const int r0 = blk * kDecodeBlock;
-                r.k = sg.k + (int64_t)b * sg.k_sb + (int64_t)g * sg.k_sh + (int64_t)r0 * D;
-                r.v = sg.v + (int64_t)b * sg.v_sb + (int64_t)g * sg.v_sh + (int64_t)r0 * D;
-                r.valid = min(kDecodeBlock, sg.rows - r0);
-                if (LOGITS && sg.logit0 >= 0) r.row = sg.logit0 + r0;
-            }
-            return r;
+        int s = 0, first = 0;
+#pragma unroll
+        for (int i = 0; i < kDecodeSegs - 1; ++i)
+            if (blk >= plan.end[i]) s = i + 1, first = plan.end[i];
+        blk -= first;
+        const DecodeSeg sg = j.seg[s];
+        Block r{nullptr, nullptr, 0, sg.q, -1};
+        if (sg.n_ids > 0) {
+            const int per = (sg.rows + kDecodeBlock - 1) / kDecodeBlock, i = blk / per, r0 = (blk - i * per) * kDecodeBlock;
+            const int u = __builtin_amdgcn_readfirstlane(SELECT ? chosen[i] : sg.ids ? sg.ids[(int64_t)b * sg.n_ids + i] : i);
+            const int ch = u / j.per_chunk;
+            const bf16_t *base = (const bf16_t *)(uintptr_t)j.chunk[ch] + (int64_t)(u - ch * j.per_chunk) * j.unit_elems + (int64_t)b * j.row_elems +
+                                 (int64_t)g * j.unit_sh + (int64_t)r0 * D;
+            r.k = base;
+            r.v = base + j.unit_v_off;
+            r.valid = min(kDecodeBlock, sg.rows - r0);
+        } else {
+            const int r0 = blk * kDecodeBlock;
+            r.k = sg.k + (int64_t)b * sg.k_sb + (int64_t)g * sg.k_sh + (int64_t)r0 * D;
+            r.v = sg.v + (int64_t)b * sg.v_sb + (int64_t)g * sg.v_sh + (int64_t)r0 * D;
+            r.valid = min(kDecodeBlock, sg.rows - r0);
+            if (LOGITS && sg.logit0 >= 0) r.row = sg.logit0 + r0;
         }
         return r;
     };
@@ -336,22 +343,22 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         }
     }
 
-    // ---- join the row groups and waves
-    if (col < NG) {
-        sm[wave][rg][col] = m;
-        sl[wave][rg][col] = l;
+    // ---- join the row groups of the wave, then the waves (m == -infinity: nothing seen yet, or logits that are no numbers, whose
+    //      sums have to stay NaN)
+    float mw = fmaxf(m, __shfl_xor(m, 16, 64));
+    mw = fmaxf(mw, __shfl_xor(mw, 32, 64));
+    const float to_mw = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mw) * scale);
+    float lw = m == -INFINITY ? l : l * to_mw;
+    lw += __shfl_xor(lw, 16, 64);
+    lw += __shfl_xor(lw, 32, 64);
+    if (lane < NG) {
+        sm[wave][lane] = mw;
+        sl[wave][lane] = lw;
     }
-    __syncthreads();
     const int vg = lane / LPR;                     // this lane's group of value rows: its own row group, or half of it
     each_head<NG>([&](auto hc) {
         constexpr int h = decltype(hc)::value;
-        float mx = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < kDecWaves; ++w)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sm[w][r][h]);
-        const float own = sm[wave][rg][h];
-        const float f = own == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((own - mx) * scale);
+        const float f = row_bcast<h>(to_mw);
         float *dst = &red[wave][vg][h][(lane & (LPR - 1)) * 8];
         *(f32x4 *)dst = f32x4{acc[h][0] * f, acc[h][1] * f, acc[h][2] * f, acc[h][3] * f};
         *(f32x4 *)(dst + 4) = f32x4{acc[h][4] * f, acc[h][5] * f, acc[h][6] * f, acc[h][7] * f};
@@ -363,17 +370,16 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         float mx = -INFINITY, den = 0.f;
         float2 o{0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < kDecWaves; ++w)
+        for (int w = 0; w < kDecWaves; ++w) mx = fmaxf(mx, sm[w][h]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sm[w][r][h]);
+        for (int w = 0; w < kDecWaves; ++w) {
+            const float f = sm[w][h] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((sm[w][h] - mx) * scale);
+            den += sm[w][h] == -INFINITY ? sl[w][h] : sl[w][h] * f;
+            float2 ow{0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < kDecWaves; ++w)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) den += sm[w][r][h] == -INFINITY ? sl[w][r][h] : sl[w][r][h] * __builtin_amdgcn_exp2f((sm[w][r][h] - mx) * scale);
-#pragma unroll
-        for (int w = 0; w < kDecWaves; ++w)
-#pragma unroll
-            for (int r = 0; r < GRP; ++r) o.x += red[w][r][h][d], o.y += red[w][r][h][d + 1];
+            for (int r = 0; r < GRP; ++r) ow.x += red[w][r][h][d], ow.y += red[w][r][h][d + 1];
+            o.x += ow.x * f, o.y += ow.y * f;
+        }
         const f16x2 part{(_Float16)(den == 0.f ? 0.f : o.x / den), (_Float16)(den == 0.f ? 0.f : o.y / den)};
         const float lse = den > 0.f ? mx * scale + log2f(den) : -INFINITY;
         uint32_t *dst = (uint32_t *)(j.o_part + (row0 + h) * D + d);
@@ -391,7 +397,7 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         //      write its L2 back.  Wave w takes every fourth split, a lane one head's 8 elements (merge_piece's arithmetic).
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        int &last = *(int *)&sm[0][0][0];
+        int &last = *(int *)&sm[0][0];
         uint32_t *ticket = j.ticket + (int64_t)b * gridDim.y + blockIdx.y;
         if (threadIdx.x == 0) last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)n_split - 1;
         __syncthreads();
@@ -459,6 +465,18 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     }
 }
 
+DecodePlan plan_of(const DecodeJob *job, int NG) {
+    DecodePlan p{};
+    p.G = job->H / job->Hkv;
+    p.chunks = (p.G + NG - 1) / NG;
+    int32_t n = 0;
+    for (int s = 0; s < kDecodeSegs; ++s) {
+        if (s < job->n_seg) n += (job->seg[s].rows + kDecodeBlock - 1) / kDecodeBlock * (job->seg[s].n_ids > 0 ? job->seg[s].n_ids : 1);
+        p.end[s] = s < job->n_seg ? n : INT32_MAX;
+    }
+    return p;
+}
+
 template <int D, bool LOGITS, bool JOIN, bool SELECT = false>
 int launch(const DecodeJob *job, void *stream) {
     const int G = job->H / job->Hkv;
@@ -466,7 +484,7 @@ int launch(const DecodeJob *job, void *stream) {
     const dim3 grid(job->nsplit, job->Hkv * ((G + NG - 1) / NG), job->B);
     const auto kern = NG == 1 ? decode_attn_kernel<D, 1, LOGITS, JOIN, NoFront, SELECT> : NG == 2 ? decode_attn_kernel<D, 2, LOGITS, JOIN, NoFront, SELECT>
                                                                                                   : decode_attn_kernel<D, 4, LOGITS, JOIN, NoFront, SELECT>;
-    hipLaunchKernelGGL(kern, grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, NoFront{});
+    hipLaunchKernelGGL(kern, grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, plan_of(job, NG), NoFront{});
     INFLLM_CHECK_LAUNCH("decode_attn");
     return 0;
 }
@@ -486,7 +504,7 @@ int launch_step(const DecodeJob *job, const StepRows *rows, void *stream) {
     const dim3 grid(job->nsplit, y, (unsigned)(job->B + planes));
     const auto kern = NG == 1 ? decode_attn_kernel<D, 1, false, true, StepRows> : NG == 2 ? decode_attn_kernel<D, 2, false, true, StepRows>
                                                                                   : decode_attn_kernel<D, 4, false, true, StepRows>;
-    hipLaunchKernelGGL(kern, grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, *rows);
+    hipLaunchKernelGGL(kern, grid, dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, plan_of(job, NG), *rows);
     INFLLM_CHECK_LAUNCH("decode_step");
     return 0;
 }
@@ -504,7 +522,7 @@ int launch_memory_step(const DecodeJob *job, const infllm_ingest_args *in, void 
     rows.in = *in;
     const auto kern = NG == 1 ? decode_attn_kernel<D, 1, true, false, MemoryRows> : NG == 2 ? decode_attn_kernel<D, 2, true, false, MemoryRows>
                                                                                             : decode_attn_kernel<D, 4, true, false, MemoryRows>;
-    hipLaunchKernelGGL(kern, dim3(job->nsplit, y, (unsigned)(job->B + planes)), dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, rows);
+    hipLaunchKernelGGL(kern, dim3(job->nsplit, y, (unsigned)(job->B + planes)), dim3(kDecWaves * kWave), 0, (hipStream_t)stream, *job, plan_of(job, NG), rows);
     INFLLM_CHECK_LAUNCH("decode_memory_step");
     return 0;
 }
