@@ -39,7 +39,7 @@ struct DecodeJob {
     const float *unit_scores;
     int64_t unit_scores_sb;
     int32_t n_scores, lead_segs, lead_splits;
-    int32_t *ids_out;
+    int32_t *ids_out, *log;                // log (optional, the host's memory): [B, n_ids] too
     // Optional, without logits: the launch joins its splits itself, the finished row of head h goes to out + b * out_sb + h * out_sh.
     bf16_t *out;
     int64_t out_sb, out_sh;

@@ -140,7 +140,10 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         if (lead) {
             select_units<kDecWaves * kWave>(j.unit_scores + (int64_t)b * j.unit_scores_sb, j.n_scores, j.seg[0].n_ids, chosen, *(SelectLds<kDecWaves * kWave> *)red_room);
             if (split == 0 && blockIdx.y == 0)
-                for (int i = threadIdx.x; i < j.seg[0].n_ids; i += kDecWaves * kWave) j.ids_out[(int64_t)b * j.seg[0].n_ids + i] = chosen[i];
+                for (int i = threadIdx.x; i < j.seg[0].n_ids; i += kDecWaves * kWave) {
+                    j.ids_out[(int64_t)b * j.seg[0].n_ids + i] = chosen[i];
+                    if (j.log) __hip_atomic_store(j.log + (int64_t)b * j.seg[0].n_ids + i, chosen[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                }
         }
     }
 
