@@ -365,6 +365,21 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
         if (!JOIN && lane < kLse)
             load_to_lds4(lse, (uint32_t)min(s * QR + any_wave * kLse + lane, Lq - 1) * 4, lds_address((char *)(Ls + buf * QR + any_wave * kLse)));
     };
+    // ---- partial log-sum-exps of the first queries, two a thread.  What a wave requests comes back in order: they are joined while the keys
+    //      are on their way (prompts of 24,300 tokens, 36 heads of 64, 2,859 -> 2,838 us, of 131,072 with 32 of 128 23,831 -> 23,705; waves in pairs, with up to 2,048 queries to join, are 0.8 % slower so).
+    const int64_t all = (int64_t)a.B * a.H * Lq;
+    float l8[2][8];
+    auto ask_sums = [&](int i0) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int p = 0; p < 8; ++p) l8[e][p] = i0 + e * kThreads < Lq && p < a.n_parts ? lse[lps.l(p, all) + i0 + e * kThreads] : -INFINITY;
+    };
+    constexpr bool kSumsFirst = JOIN && QG == 1;
+    if constexpr (kSumsFirst) {
+        ask_sums(tid);
+        asm volatile("" ::: "memory");
+    }
     if (st_lo < st_hi) load_stage(st_lo, 0);
     if (NB > 2 && st_lo + 1 < st_hi) load_stage(st_lo + 1, 1);
 
@@ -382,16 +397,11 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
             kreg[ks][kk] = __builtin_bit_cast(bf16x8, raw);
         }
     }
-    // ---- joined log-sum-exps of all queries, two a thread: one trip to memory for 512
+    // ---- joined log-sum-exps of all queries
     if constexpr (JOIN) {
-        const int64_t all = (int64_t)a.B * a.H * Lq;
         const int padded = (Lq + QR - 1) / QR * QR;
         for (int i0 = tid; i0 < padded; i0 += 2 * kThreads) {
-            float l8[2][8];
-#pragma unroll
-            for (int e = 0; e < 2; ++e)
-#pragma unroll
-                for (int p = 0; p < 8; ++p) l8[e][p] = i0 + e * kThreads < Lq && p < a.n_parts ? lse[lps.l(p, all) + i0 + e * kThreads] : -INFINITY;
+            if (!kSumsFirst || i0 >= 2 * kThreads) ask_sums(i0);
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 float m8 = -INFINITY, den = 0.f;
