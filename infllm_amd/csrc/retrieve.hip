@@ -1147,6 +1147,10 @@ static int retrieve_launch(const void *d_reps, int64_t rep_stride, int32_t N, in
         f = *front;
         f.n_retrieve = wgs;
         extra = whole_front ? f.in.B * f.in.Hkv : 0;
+        // A CU has room for one scoring workgroup: with 256 of them those of the prologue came behind the first to end, and the launch ended
+        // with them (8.7 to 11.2 us behind 4,096 units, the scores at 9.1).  A few scoring ones less, whose rows the others take: steps
+        // of 32 / 8 heads of 128 behind 2,048 / 4,096 / 8,192 units 24.5 -> 24.2 / 28.1 -> 27.0 / 34.4 -> 33.9 us (36 of 64: 27.6, 27.9).
+        if (extra <= 32 && wgs > 256 - extra) f.n_retrieve = wgs = 256 - extra;
     }
 #define FUSED_CASE(c, tail)                                                                                                          \
     if (front) {                                                                                                                     \
