@@ -20,6 +20,7 @@
 
 #include "common.h"
 #include "decode.h"
+#include "rope.h"
 
 #include <algorithm>
 #include <atomic>
@@ -151,6 +152,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     extern __shared__ __attribute__((aligned(1024))) char lds_dyn[];    // kStages K tiles, then kStages V tiles
     char *const Ks = lds_dyn, *const Vs = lds_dyn + kStages * kTB;
     __shared__ int wg_lo[kWaves], wg_hi[kWaves];
+    __shared__ __attribute__((aligned(16))) float2 sink_cs[MODE == kSinks ? D / 2 : 2];
 
     // the wave index is the same in every lane: said so, what derives from it (the wave's queries, tile range, mask
     // distances) stays in scalar registers
@@ -186,6 +188,8 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     const int h = g * G + hg;
     const int i0 = qt * kQTile, i1 = min(i0 + kQTile, a.Lq) - 1;
 
+    if (MODE == kSinks && wave < D / 64)                         // 256 bytes a wave, there with the first tile
+        load_to_lds4((const float *)ap.d_pages, wave * 256 + lane * 4, lds_address((char *)sink_cs) + wave * 256);
     int w_t0 = 0, w_t1 = 0;              // this wave's range of LINEAR tiles (absolute tile numbers)
     if (HAS_LIN && live) {
         StageRange r = visible_range(a, i0, i1);
@@ -552,10 +556,28 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         l_run += sums[0];
     };
 
-    auto load_q = [&](const infllm_attn_args &src) {
+    // The sinks' queries are the step's own rows, rotated here to the one angle of the sinks (d_pages of their arguments: cosine and sine of
+    // every frequency): staged beside the others they were a third of
+    // what the staging launch wrote (sinks + window of 4,096 over 16,001 tokens, 32 / 8 heads of 128: 1,063 -> 1,041 us; window of 2,048 over two rows
+    // of 8,001: 633 -> 612; 36 heads of 64, whose sinks' queries are a seventh: 371 -> 370).
+    auto load_q = [&](const infllm_attn_args &src, [[maybe_unused]] bool sinks) {
         const int qi = i0 + col;
         const bool ok = live && qi < src.Lq;
         const bf16_t *qrow = (const bf16_t *)src.d_q + (int64_t)b * src.q_sb + (int64_t)h * src.q_sh + (int64_t)qi * src.q_sl;
+        if (MODE == kSinks && sinks) {                           // (a query behind the last: it again, never stored)
+            qrow -= ok ? 0 : (int64_t)(qi - (src.Lq - 1)) * src.q_sl;
+#pragma unroll
+            for (int kk = 0; kk < D / 16; ++kk) qreg[kk] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(qrow + kk * 16 + grp * 8));
+#pragma unroll
+            for (int kk = 0; kk < D / 32; ++kk) {                // in place, a pair at a time: registers are short
+                __builtin_amdgcn_sched_barrier(0);
+                const Rot8 r = rotate8(__builtin_bit_cast(u32x4, qreg[kk]), __builtin_bit_cast(u32x4, qreg[kk + D / 32]), sink_cs + kk * 16 + grp * 8);
+                qreg[kk] = __builtin_bit_cast(bf16x8, r.lo);
+                qreg[kk + D / 32] = __builtin_bit_cast(bf16x8, r.hi);
+                asm volatile("" : "+v"(qreg[kk]), "+v"(qreg[kk + D / 32]));
+            }
+            return;
+        }
 #pragma unroll
         for (int kk = 0; kk < D / 16; ++kk) {
             u32x4 raw = ok ? *(const u32x4 *)(qrow + kk * 16 + grp * 8) : u32x4{0, 0, 0, 0};
@@ -578,7 +600,11 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     static_assert(PING || kStages == 4, "two buffer pairs");
     for (int p = 0; p < 2; ++p)
         if (g_t0 + p < g_t1) load_tile(g_t0 + p, p * kTB);
-    load_q(q_paged ? ap : a);
+    if (MODE == kSinks && q_paged) {                             // (a split that begins with the sinks: the angle first)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+    load_q(q_paged ? ap : a, q_paged);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // The compiler does not know that the wait above also covered the query rows; passing them through an empty
     // asm makes it place its own wait for them HERE rather than in front of their first use inside the loop,
@@ -595,7 +621,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             const int u = t + e;
             if (u >= g_t1) break;
             if (TWO && u >= n_lin && !q_paged) {
-                load_q(ap);
+                load_q(ap, true);
                 q_paged = true;
             }
             if (mine(u)) tile_math(buf + e, u);
@@ -717,7 +743,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     // causal prompt of 8,001 tokens 536 -> 540.  Pages, whose second tile's address is an entry of its own to wait for, gain
     // nothing by it: prompt of 131,072 25,690 us with, 25,350 without.)
     const infllm_attn_args &first = q_paged ? ap : a;
-    if (MODE != kPaged && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
+    if (MODE != kPaged && !(MODE == kSinks && q_paged) && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
         const uint32_t at_q = (wave < 4 ? lds_address(Ks) : lds_address(Vs)) + 2 * kTB + (wave & 3) * (kQTile * kRow);
         const bf16_t *rows = (const bf16_t *)first.d_q + (int64_t)b * first.q_sb + (int64_t)h * first.q_sh + (int64_t)i0 * first.q_sl;
 #pragma unroll
@@ -738,7 +764,11 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         }
     } else {                               // pages, and rows that a 32-bit offset does not reach: far apart, or backwards
         if (t < g_t1) valid0 = load_tile(t, 0);
-        load_q(first);
+        if (MODE == kSinks && q_paged) {                         // (a split that begins with the sinks: the angle first)
+            landed();
+            half_end();
+        }
+        load_q(first, q_paged);
         landed();
 #pragma unroll
         for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(qreg[kk]));
@@ -788,7 +818,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         whole = false;
         if (t + 2 < g_t1) valid2 = load_tile(t + 2, (at + 2 * kTB) & (4 * kTB - 1));
         if (TWO && t >= n_lin && !q_paged) {
-            load_q(ap);
+            load_q(ap, true);
             q_paged = true;
         }
         const bool see = mine(t);
@@ -1393,9 +1423,9 @@ int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *si
     rc = check_linear_stage(local);
     if (rc) return rc;
     if (sinks) {
-        INFLLM_REQUIRE(sinks->d_q && sinks->d_k && sinks->d_v && sinks->j_lo == 0 && sinks->j_hi >= 0 && sinks->k_sl == dim && sinks->v_sl == dim,
+        INFLLM_REQUIRE(sinks->d_q && sinks->d_pages && sinks->d_k && sinks->d_v && sinks->j_lo == 0 && sinks->j_hi >= 0 && sinks->k_sl == dim && sinks->v_sl == dim,
                        "attn_window: bad sink rows");
-        INFLLM_REQUIRE(sinks->q_sl == local->q_sl && sinks->q_sh == local->q_sh && sinks->q_sb == local->q_sb && sinks->Lq == local->Lq,
+        INFLLM_REQUIRE(sinks->Lq == local->Lq && sinks->B == local->B && sinks->H == local->H && ((sinks->q_sl | sinks->q_sh | sinks->q_sb) & 7) == 0,
                        "attn_window: the two stages disagree");
     }
     StageOut so;

@@ -18,7 +18,8 @@ struct StageJob {
     int64_t pos0, glb_pos;                     // position of row 0; the one angle of the sinks' queries
     const float *inv_freq;
     double distance_scale;
-    bf16_t *q_loc, *q_glb;                     // [B, H, n, D]; q_glb NULL: no sinks
+    bf16_t *q_loc, *q_glb;                     // [B, H, n, D]; q_glb NULL: not wanted
+    float2 *glb_cs;                            // cosine and sine of every frequency at the sinks' angle (NULL: not wanted)
     bf16_t *dk, *dv;                           // where row 0 of head 0 goes, rotated / as it is
     int64_t dk_sb, dk_sh, dv_sb, dv_sh;
     // A second place for some of the rows (NULL: none): row p is row r = c_first + p of all that the call sees; those with
@@ -87,6 +88,7 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
     }
     rope_angles<HALF>(j.pos0 + p0, np, j.glb_pos, j.distance_scale, freq, cs_pos, cs_glb);
     __syncthreads();
+    if (j.glb_cs && blockIdx.x == 0 && b == 0 && g0 == 0 && tid < HALF) j.glb_cs[tid] = cs_glb[tid];
     if (j.do_q) {
         for (int hg0 = 0; hg0 < n_heads; hg0 += 4) {
 #pragma unroll
@@ -241,7 +243,9 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     j.v_sb = a->v_sb; j.v_sh = a->v_sh; j.v_sl = a->v_sl;
     j.glb_pos = a->kind == 2 ? a->n_local - 1 : a->n_local + a->n_init - 1;
     j.inv_freq = a->d_inv_freq; j.distance_scale = a->distance_scale;
-    j.q_loc = q_loc; j.q_glb = sink_stage ? q_sink : nullptr;
+    j.q_loc = q_loc;
+    if (sink_stage && step) j.q_glb = q_sink;                    // (several queries are rotated to the sinks' angle where they are attended)
+    else if (sink_stage) j.glb_cs = (float2 *)q_sink;
     j.dk = bk + (rows_base - a->n_new) * D; j.dv = bv + (rows_base - a->n_new) * D;
     j.dk_sb = bk_sb; j.dk_sh = bk_sh; j.dv_sb = bv_sb; j.dv_sh = bv_sh;
     const int64_t raw_sh = (int64_t)a->raw_new * D;
@@ -379,7 +383,9 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     l.softmax_scale = scale;
     if (sink_stage) {
         s = l;
-        s.d_q = q_sink;
+        s.d_q = a->d_q;
+        s.q_sl = a->q_sl; s.q_sh = a->q_sh; s.q_sb = a->q_sb;
+        s.d_pages = (const infllm_page *)q_sink;
         s.d_k = sk; s.k_sh = sk_sh; s.k_sb = sk_sb;
         s.j_lo = 0; s.j_hi = n_sink;
         s.mask = INFLLM_MASK_COMPLEMENT;
