@@ -147,7 +147,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
                                                                  std::conditional_t<INLINE, InlinePages, NoInlinePages>) {
     constexpr bool HAS_LIN = MODE != kPaged, HAS_PAG = MODE != kLinear, TWO = MODE == kBoth || MODE == kSinks;
     constexpr int kRow = D * 2, kTB = kTileBytes<D>;                     // bytes of a row, of a tile
-    constexpr bool PING = D == 128;
+    constexpr bool PING = D == 128, kTurns = D == 128 && (MODE == kLinear || MODE == kSinks);
     const infllm_attn_args &ap = TWO ? a2 : a;                 // the paged stage's arguments
     extern __shared__ __attribute__((aligned(1024))) char lds_dyn[];    // kStages K tiles, then kStages V tiles
     char *const Ks = lds_dyn, *const Vs = lds_dyn + kStages * kTB;
@@ -583,6 +583,15 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             u32x4 raw = ok ? *(const u32x4 *)(qrow + kk * 16 + grp * 8) : u32x4{0, 0, 0, 0};
             qreg[kk] = __builtin_bit_cast(bf16x8, raw);
         }
+        if (kTurns && src.d_pages) {                             // rows as they come, to be rotated to their positions
+            const float2 *cs = (const float2 *)src.d_pages + (int64_t)min(qi, src.Lq - 1) * (D / 2) + grp * 8;
+#pragma unroll
+            for (int kk = 0; kk < D / 32; ++kk) {
+                const Rot8 r = rotate8(__builtin_bit_cast(u32x4, qreg[kk]), __builtin_bit_cast(u32x4, qreg[kk + D / 32]), cs + kk * 16);
+                qreg[kk] = __builtin_bit_cast(bf16x8, r.lo);
+                qreg[kk + D / 32] = __builtin_bit_cast(bf16x8, r.hi);
+            }
+        }
     };
     // does this wave see tile u at all?  (pages: every live wave; linear tiles: the wave's own visible range)
     auto mine = [&](int u) {
@@ -743,7 +752,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     // causal prompt of 8,001 tokens 536 -> 540.  Pages, whose second tile's address is an entry of its own to wait for, gain
     // nothing by it: prompt of 131,072 25,690 us with, 25,350 without.)
     const infllm_attn_args &first = q_paged ? ap : a;
-    if (MODE != kPaged && !(MODE == kSinks && q_paged) && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
+    if (MODE != kPaged && !(MODE == kSinks && q_paged) && !(kTurns && a.d_pages) && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
         const uint32_t at_q = (wave < 4 ? lds_address(Ks) : lds_address(Vs)) + 2 * kTB + (wave & 3) * (kQTile * kRow);
         const bf16_t *rows = (const bf16_t *)first.d_q + (int64_t)b * first.q_sb + (int64_t)h * first.q_sh + (int64_t)i0 * first.q_sl;
 #pragma unroll

@@ -19,6 +19,7 @@ struct StageJob {
     const float *inv_freq;
     double distance_scale;
     bf16_t *q_loc, *q_glb;                     // [B, H, n, D]; q_glb NULL: not wanted
+    float2 *pos_cs;                            // [n, D / 2] cosine and sine of every position and frequency (NULL: not wanted)
     float2 *glb_cs;                            // cosine and sine of every frequency at the sinks' angle (NULL: not wanted)
     bf16_t *dk, *dv;                           // where row 0 of head 0 goes, rotated / as it is
     int64_t dk_sb, dk_sh, dv_sb, dv_sh;
@@ -88,6 +89,8 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
     }
     rope_angles<HALF>(j.pos0 + p0, np, j.glb_pos, j.distance_scale, freq, cs_pos, cs_glb);
     __syncthreads();
+    if (j.pos_cs && b == 0 && g0 == 0)
+        for (int i = tid; i < np * HALF; i += 256) j.pos_cs[(int64_t)p0 * HALF + i] = cs_pos[0][i];
     if (j.glb_cs && blockIdx.x == 0 && b == 0 && g0 == 0 && tid < HALF) j.glb_cs[tid] = cs_glb[tid];
     if (j.do_q) {
         for (int hg0 = 0; hg0 < n_heads; hg0 += 4) {
@@ -154,7 +157,7 @@ int launch_stage_rows(StageJob &j, int dim, void *stream) {
     for (const RowCopy &c : j.copy) pieces += (c.n + kCopyRows - 1) / kCopyRows;
     j.tiles = j.do_q || j.do_kv ? (j.n + kPosPerBlock - 1) / kPosPerBlock : 0;
     if (j.tiles + pieces == 0) return 0;
-    const int kg = heads_together(j.n, j.B, j.H, j.Hkv);
+    const int kg = heads_together(j.n, j.B, j.do_q ? j.H : j.Hkv, j.Hkv);
     const dim3 grid(j.tiles + pieces, j.B, (j.Hkv + kg - 1) / kg);
     const auto kern = dim == 128 ? (kg == 4 ? stage_rows_kernel<128, 4> : kg == 2 ? stage_rows_kernel<128, 2> : stage_rows_kernel<128, 1>)
                                  : (kg == 4 ? stage_rows_kernel<64, 4> : kg == 2 ? stage_rows_kernel<64, 2> : stage_rows_kernel<64, 1>);
@@ -191,6 +194,12 @@ int infllm_attn_splits(int64_t wgs, int64_t tiles, int32_t max_parts, double mea
     return best;
 }
 
+// Queries of a call from which on the attention rotates them itself, by a table of cosines and sines, instead of the staging launch in front of
+// it: that one reads and writes 67 MB less of 4,096 tokens x 32 heads of 128, but a workgroup's second tile waits for its queries and
+// the table, which a launch of one or two rounds of workgroups feels.  Causal prompts of 2,049 / 3,073 / 4,097 / 6,145 tokens in one call, 32 heads
+// of 128: staged 79.7 / 111.1 / 169.2 / 338.1 us, so 81.3 / 108.1 / 163.1 / 329.8; sinks + window of 1,024 64.4 / 100.3 / 119.8 / 173.0 and 66.4 /
+// 103.9 / 116.4 / 168.4.  (36 heads of 64: no difference.)
+constexpr int64_t kTurnRows = 1 << 17;
 extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) {
     INFLLM_REQUIRE(a != nullptr, "window_forward: null argument block");
     INFLLM_REQUIRE(a->dim == 128 || a->dim == 64, "window_forward: head_dim %d is not 64 or 128", a->dim);
@@ -324,8 +333,12 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         rc = infllm_decode_step(&d, &f, D, stream);
         if (rc != 1) return rc;
     }
+    // The attention rotates the queries itself, by a table of cosines and sines in their place (which hold it from two heads on).
+    const bool turns = !step && a->n_q == a->n_new && (int64_t)a->B * a->H >= 2 && D == 128 && rows_q >= kTurnRows;
     if (a->n_q == a->n_new) {
-        j.do_q = j.do_kv = 1;
+        j.do_q = !turns;
+        j.do_kv = 1;
+        if (turns) j.pos_cs = (float2 *)q_loc;
         j.n = a->n_q;
         j.pos0 = a->seen;
         rc = launch_stage_rows(j, D, stream);
@@ -368,8 +381,14 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         return infllm_decode_attn(&d, D, stream);
     }
     infllm_attn_args l{}, s{};
-    l.d_q = q_loc;
-    l.q_sl = D; l.q_sh = (int64_t)a->n_q * D; l.q_sb = (int64_t)a->H * a->n_q * D;
+    if (turns) {
+        l.d_q = a->d_q;
+        l.q_sl = a->q_sl; l.q_sh = a->q_sh; l.q_sb = a->q_sb;
+        l.d_pages = (const infllm_page *)j.pos_cs;
+    } else {
+        l.d_q = q_loc;
+        l.q_sl = D; l.q_sh = (int64_t)a->n_q * D; l.q_sb = (int64_t)a->H * a->n_q * D;
+    }
     l.B = a->B; l.H = a->H; l.Hkv = a->Hkv; l.Lq = a->n_q;
     l.d_k = bk; l.d_v = bv;
     l.k_sl = l.v_sl = D;

@@ -38,3 +38,31 @@ def test_prompts_with_sinks(kind, D, H, Hkv, B, calls, n_local, n_init):
         pos += n
     err = (heads(got.cpu(), H) - torch.cat(want, dim=2)).abs()
     assert float(err.max()) <= 2e-2 and float(err.mean()) <= 2e-3, (float(err.max()), float(err.mean()))
+
+
+@pytest.mark.parametrize("kind", ["origin", "stream-llm", "infinite-lm"])
+@pytest.mark.parametrize("B,H,Hkv,n", [(1, 32, 8, 4099), (2, 33, 3, 2000)])
+def test_queries_rotated_where_they_are_attended(kind, B, H, Hkv, n):
+    """Calls of 2^17 query rows of 128 and more, whose attention rotates them, against the same heads in calls of a kv head each, whose
+    queries are staged: a last tile that is not full, a second call behind a cache, rows apart from each other."""
+    from infllm_amd.attention import ATTN_FORWRAD, RotaryEmbeddingESM
+    D, G, g = 128, H // Hkv, torch.Generator(device="cuda").manual_seed(n)
+    assert B * H * n >= 1 << 17 > B * G * n
+    q, k, v = torch.randn((B, 2 * n, (H + 2 * Hkv) * D), generator=g, device="cuda").bfloat16().split([H * D, Hkv * D, Hkv * D], dim=-1)
+    forward = ATTN_FORWRAD[kind](False) if kind == "origin" else ATTN_FORWRAD[kind](n // 2, 70, fattn=False)
+    rope, same = RotaryEmbeddingESM(D, base=1e4, device="cuda"), lambda t: t
+
+    def run(q, k, v, heads, kv_heads):
+        past, outs = None, []
+        for sl in (slice(0, n), slice(n, 2 * n)):
+            rows = [t[:, sl] for t in (q, k, v)]
+            o, past = forward(None, rows[0], rows[1], rope, True, past, same, same, lambda _: rows[2], same, D, heads, kv_heads)
+            outs.append(o)
+        return torch.cat(outs, dim=1)
+    got = run(q, k, v, H, Hkv).view(B, 2 * n, H, D)
+    for i in range(Hkv):
+        part = [t.reshape(B, 2 * n, -1, D)[:, :, i * m:(i + 1) * m].flatten(2) for t, m in ((q, G), (k, 1), (v, 1))]
+        want = run(*part, G, 1).view(B, 2 * n, G, D).float()
+        # results rounded to bf16, 2^-8 of an element each at most and a third of that in the mean square; the rest of 2^-7 for
+        # probabilities, partial rows and single rotated elements that are rounded another way
+        assert float((got[:, :, i * G:(i + 1) * G].float() - want).norm()) <= 2.0 ** -7 * float(want.norm()), i
