@@ -198,8 +198,9 @@ int infllm_attn_splits(int64_t wgs, int64_t tiles, int32_t max_parts, double mea
 // it: that one reads and writes 67 MB less of 4,096 tokens x 32 heads of 128, but a workgroup's second tile waits for its queries and
 // the table, which a launch of one or two rounds of workgroups feels.  Causal prompts of 2,049 / 3,073 / 4,097 / 6,145 tokens in one call, 32 heads
 // of 128: staged 79.7 / 111.1 / 169.2 / 338.1 us, so 81.3 / 108.1 / 163.1 / 329.8; sinks + window of 1,024 64.4 / 100.3 / 119.8 / 173.0 and 66.4 /
-// 103.9 / 116.4 / 168.4.  (36 heads of 64: no difference.)
-constexpr int64_t kTurnRows = 1 << 17;
+// 103.9 / 116.4 / 168.4; calls of 3,200 and windows of 2,048 / 4,096 121.5 / 118.4 and 123.1 / 115.2, of 3,500 behind one of 4,096 and windows of
+// 512 to 4,096 1 to 1.6 % faster so.  (36 heads of 64: no difference.)
+constexpr int64_t kTurnRows = 13 << 13;
 extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) {
     INFLLM_REQUIRE(a != nullptr, "window_forward: null argument block");
     INFLLM_REQUIRE(a->dim == 128 || a->dim == 64, "window_forward: head_dim %d is not 64 or 128", a->dim);
