@@ -752,7 +752,44 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     // causal prompt of 8,001 tokens 536 -> 540.  Pages, whose second tile's address is an entry of its own to wait for, gain
     // nothing by it: prompt of 131,072 25,690 us with, 25,350 without.)
     const infllm_attn_args &first = q_paged ? ap : a;
-    if (MODE != kPaged && !(MODE == kSinks && q_paged) && !(kTurns && a.d_pages) && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
+    // Rows to be rotated come that way too, and their angles (512 bytes a query) into the second tile's buffer, which is requested when
+    // they have been read.  (By lanes that each fetch their own query's pieces, 32 lines an instruction: sinks + window of 4,096 over 16,001
+    // tokens 1,060 -> 1,041 us, of 512 over 7,596 174.7 -> 167.2, causal prompt of 8,001 542 -> 535.)
+    // (Two tiles of queries a workgroup at most: four query heads a kv head, or eight and more.)
+    const bool turn_lds = kTurns && a.d_pages && !q_paged && (G == 4 || G >= 8) && (uint64_t)a.q_sl < (uint64_t)1 << 26 && a.Lq < 1 << 22;
+    if (turn_lds) {
+        const int qt0 = (int)fdiv(bx * kWaves, geo.group), half = wave >> 2;
+        const uint32_t at_q = (wave < 4 ? lds_address(Ks) : lds_address(Vs)) + 2 * kTB + (wave & 3) * (kQTile * kRow);
+        const bf16_t *rows = (const bf16_t *)a.d_q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)i0 * a.q_sl;
+#pragma unroll
+        for (int i = 0; i < kQTile * kRow / 1024; ++i) {
+            const int r = kRowsPerLd * i + lane / (D / 8);                              // (rows behind the last: it again, never stored)
+            load_to_lds16(rows, (uint32_t)(min(r, a.Lq - 1 - i0) * (int)a.q_sl + ((lane & (D / 8 - 1)) ^ swz<D>(r)) * 8) * 2, at_q + i * 1024);
+        }
+        const uint32_t angles = lds_address(half == 0 ? Ks : Vs) + kTB;                 // waves 0 - 3: of the first query tile, 4 - 7: of the second
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = ((wave & 3) * 4 + i) * 2 + (lane >> 5), q = min((qt0 + half) * kQTile + r, a.Lq - 1);
+            load_to_lds16((const bf16_t *)a.d_pages, (uint32_t)q * (D * 4) + ((lane & 31) ^ r) * 16, angles + ((wave & 3) * 4 + i) * 1024);
+        }
+        if (t < g_t1) valid0 = load_tile(t, 0);
+        landed();
+        half_end();
+        const uint32_t own = at_q + col * kRow + ((grp ^ swz<D>(col)) * 16);
+        const uint32_t own_angles = lds_address(qt == qt0 ? Ks : Vs) + kTB + col * (D * 4);
+#pragma unroll
+        for (int kk = 0; kk < D / 32; ++kk) {
+            const u32x4 lo = *(const __attribute__((address_space(3))) u32x4 *)(uintptr_t)(own ^ (kk * 32));
+            const u32x4 hi = *(const __attribute__((address_space(3))) u32x4 *)(uintptr_t)(own ^ ((kk + D / 32) * 32));
+            f32x4 cs[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) cs[i] = *(const __attribute__((address_space(3))) f32x4 *)(uintptr_t)(own_angles + (((kk * 8 + grp * 4 + i) ^ col) * 16));
+            const Rot8 r = rotate8(lo, hi, (const float2 *)cs);
+            qreg[kk] = __builtin_bit_cast(bf16x8, r.lo);
+            qreg[kk + D / 32] = __builtin_bit_cast(bf16x8, r.hi);
+            asm volatile("" : "+v"(qreg[kk]), "+v"(qreg[kk + D / 32]));                 // (read before the barrier)
+        }
+    } else if (MODE != kPaged && !(MODE == kSinks && q_paged) && !(kTurns && a.d_pages) && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
         const uint32_t at_q = (wave < 4 ? lds_address(Ks) : lds_address(Vs)) + 2 * kTB + (wave & 3) * (kQTile * kRow);
         const bf16_t *rows = (const bf16_t *)first.d_q + (int64_t)b * first.q_sb + (int64_t)h * first.q_sh + (int64_t)i0 * first.q_sl;
 #pragma unroll
@@ -784,6 +821,10 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         if (t + 1 < g_t1) valid1 = load_tile(t + 1, kTB);
     }
     half_end();
+    if (turn_lds) {
+        whole = false;
+        if (t + 1 < g_t1) valid1 = load_tile(t + 1, kTB);
+    }
     if (second) half_end();
     bool have_p = false;                   // the tile before has probabilities that wait for their values
     // A tile with nothing special about it - whole, seen without a mask, the tile before seen too and the one to request
