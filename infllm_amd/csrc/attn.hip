@@ -583,15 +583,6 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             u32x4 raw = ok ? *(const u32x4 *)(qrow + kk * 16 + grp * 8) : u32x4{0, 0, 0, 0};
             qreg[kk] = __builtin_bit_cast(bf16x8, raw);
         }
-        if (kTurns && src.d_pages) {                             // rows as they come, to be rotated to their positions
-            const float2 *cs = (const float2 *)src.d_pages + (int64_t)min(qi, src.Lq - 1) * (D / 2) + grp * 8;
-#pragma unroll
-            for (int kk = 0; kk < D / 32; ++kk) {
-                const Rot8 r = rotate8(__builtin_bit_cast(u32x4, qreg[kk]), __builtin_bit_cast(u32x4, qreg[kk + D / 32]), cs + kk * 16);
-                qreg[kk] = __builtin_bit_cast(bf16x8, r.lo);
-                qreg[kk + D / 32] = __builtin_bit_cast(bf16x8, r.hi);
-            }
-        }
     };
     // does this wave see tile u at all?  (pages: every live wave; linear tiles: the wave's own visible range)
     auto mine = [&](int u) {
@@ -755,8 +746,8 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     // Rows to be rotated come that way too, and their angles (512 bytes a query) into the second tile's buffer, which is requested when
     // they have been read.  (By lanes that each fetch their own query's pieces, 32 lines an instruction: sinks + window of 4,096 over 16,001
     // tokens 1,060 -> 1,041 us, of 512 over 7,596 174.7 -> 167.2, causal prompt of 8,001 542 -> 535.)
-    // (Two tiles of queries a workgroup at most: four query heads a kv head, or eight and more.)
-    const bool turn_lds = kTurns && a.d_pages && !q_paged && (G == 4 || G >= 8) && (uint64_t)a.q_sl < (uint64_t)1 << 26 && a.Lq < 1 << 22;
+    // (Two tiles of queries a workgroup at most: infllm_attn_turns.)
+    const bool turn_lds = kTurns && a.d_pages && !q_paged;
     if (turn_lds) {
         const int qt0 = (int)fdiv(bx * kWaves, geo.group), half = wave >> 2;
         const uint32_t at_q = (wave < 4 ? lds_address(Ks) : lds_address(Vs)) + 2 * kTB + (wave & 3) * (kQTile * kRow);
@@ -789,7 +780,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             qreg[kk + D / 32] = __builtin_bit_cast(bf16x8, r.hi);
             asm volatile("" : "+v"(qreg[kk]), "+v"(qreg[kk + D / 32]));                 // (read before the barrier)
         }
-    } else if (MODE != kPaged && !(MODE == kSinks && q_paged) && !(kTurns && a.d_pages) && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
+    } else if (MODE != kPaged && !(MODE == kSinks && q_paged) && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
         const uint32_t at_q = (wave < 4 ? lds_address(Ks) : lds_address(Vs)) + 2 * kTB + (wave & 3) * (kQTile * kRow);
         const bf16_t *rows = (const bf16_t *)first.d_q + (int64_t)b * first.q_sb + (int64_t)h * first.q_sh + (int64_t)i0 * first.q_sl;
 #pragma unroll
@@ -1465,6 +1456,12 @@ extern "C" int infllm_attn_merge_pair(const uint16_t *d_o_part, const float *d_l
 // library-internal: a linear stage and (sinks != NULL) the rows of a second source under the complement mask, under one
 // softmax, as rows of `dim` elements (128 or 64) in the caller's layout; local->nsplit key splits of the joint tile list,
 // with partial rows at local->d_o_part / d_lse_part when there is more than one
+// d_pages of `local`: NULL, or cosine and sine of every query's angles [Lq, 64], by which the launch rotates the rows as they come
+// (infllm_attn_turns); of `sinks`: of the one angle of theirs.
+bool infllm_attn_turns(int32_t H, int32_t Hkv, int32_t n_q, int64_t q_sl, int32_t dim) {
+    const int G = H / Hkv;
+    return dim == 128 && (G == 4 || G >= 8) && q_sl >= 0 && q_sl < 1 << 26 && n_q < 1 << 22;
+}
 int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, int32_t dim, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
                        void *stream) {
     INFLLM_REQUIRE(local && d_out && (dim == 128 || dim == 64), "attn_window: bad arguments");
@@ -1478,6 +1475,7 @@ int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *si
         INFLLM_REQUIRE(sinks->Lq == local->Lq && sinks->B == local->B && sinks->H == local->H && ((sinks->q_sl | sinks->q_sh | sinks->q_sb) & 7) == 0,
                        "attn_window: the two stages disagree");
     }
+    INFLLM_REQUIRE(!local->d_pages || infllm_attn_turns(local->H, local->Hkv, local->Lq, local->q_sl, dim), "attn_window: queries that are not rotated");
     StageOut so;
     if (local->nsplit == 1) {
         so.out = (bf16_t *)d_out;

@@ -8,6 +8,7 @@
 
 int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, int32_t dim, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
                        void *stream);
+bool infllm_attn_turns(int32_t H, int32_t Hkv, int32_t n_q, int64_t q_sl, int32_t dim);
 namespace {
 
 struct StageJob {
@@ -194,13 +195,6 @@ int infllm_attn_splits(int64_t wgs, int64_t tiles, int32_t max_parts, double mea
     return best;
 }
 
-// Queries of a call from which on the attention rotates them itself, by a table of cosines and sines, instead of the staging launch in front of
-// it: that one reads and writes 67 MB less of 4,096 tokens x 32 heads of 128, but a workgroup's second tile waits for its queries and
-// the table, which a launch of one or two rounds of workgroups feels.  Causal prompts of 2,049 / 3,073 / 4,097 / 6,145 tokens in one call, 32 heads
-// of 128: staged 79.7 / 111.1 / 169.2 / 338.1 us, so 81.3 / 108.1 / 163.1 / 329.8; sinks + window of 1,024 64.4 / 100.3 / 119.8 / 173.0 and 66.4 /
-// 103.9 / 116.4 / 168.4; calls of 3,200 and windows of 2,048 / 4,096 121.5 / 118.4 and 123.1 / 115.2, of 3,500 behind one of 4,096 and windows of
-// 512 to 4,096 1 to 1.6 % faster so.  (36 heads of 64: no difference.)
-constexpr int64_t kTurnRows = 13 << 13;
 extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) {
     INFLLM_REQUIRE(a != nullptr, "window_forward: null argument block");
     INFLLM_REQUIRE(a->dim == 128 || a->dim == 64, "window_forward: head_dim %d is not 64 or 128", a->dim);
@@ -334,8 +328,11 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         rc = infllm_decode_step(&d, &f, D, stream);
         if (rc != 1) return rc;
     }
-    // The attention rotates the queries itself, by a table of cosines and sines in their place (which hold it from two heads on).
-    const bool turns = !step && a->n_q == a->n_new && (int64_t)a->B * a->H >= 2 && D == 128 && rows_q >= kTurnRows;
+    // The attention rotates the queries itself, where it can, by a table of cosines and sines in their place (which hold it from two heads
+    // on): the staging reads and writes 67 MB less of 4,096 tokens x 32 heads of 128.  Staged / so, 32 / 8 heads of 128, causal prompts of
+    // 1,537 / 2,049 / 3,073 / 8,001 tokens 60.9 / 80.5 / 114.9 / 549.7 and 59.6 / 78.0 / 111.3 / 535.4 us; sinks + window of 1,024 over 1,537 /
+    // 3,073 67.5 / 101.8 and 67.2 / 101.3; below, the host bounds them.
+    const bool turns = !step && a->n_q == a->n_new && (int64_t)a->B * a->H >= 2 && infllm_attn_turns(a->H, a->Hkv, a->n_q, a->q_sl, D);
     if (a->n_q == a->n_new) {
         j.do_q = !turns;
         j.do_kv = 1;
