@@ -209,9 +209,9 @@ int infllm_attn_fwd_noalloc(const infllm_attn_args *local, const infllm_attn_arg
  * hold every key the call sees (n_q > 1 and the cache is cut); else NULL, and the attention reads the new cache.
  * d_raw: the un-rotated sinks (kind 2): raw_old of them in d_raw_old [B, Hkv, raw_old, dim], raw_new in d_raw (the same
  * pointer and counts when nothing is added).
- * d_work: scratch, work_bytes long: 2 * B * H * n_q * dim bf16 for the rotated queries (once for kind 0), the rest, if any, for
- * partial rows (more of it allows more key splits, up to 64 * B * H * n_q rows of 2 * dim + 4 bytes; a step, n_q == 1, takes
- * 4 * B * H bytes of it for tickets). */
+ * d_work: scratch, work_bytes long: 2 * B * H * n_q * dim bf16 (once for kind 0) for the rotated queries, or the angles that the
+ * attention rotates them by; the rest, if any, for partial rows (more of it allows more key splits, up to 64 * B * H * n_q rows of
+ * 2 * dim + 4 bytes; a step, n_q == 1, takes 4 * B * H bytes of it for tickets). */
 typedef struct {
     const void *d_q, *d_k, *d_v;            /* [B,H,n_q,dim], [B,Hkv,n_new,dim] */
     int64_t q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;

@@ -118,8 +118,11 @@ struct IntC {
 // source of `a`, then the page table of `a2` with `a2`'s queries - both stages of the operator in one launch, as ONE
 // list of tiles that the key splits divide between them (one set of partials, one fixed cost instead of two).  kSinks:
 // the linear source of `a`, then the first j_hi rows of the linear source of `a2` (rows of D elements, no ring) under the
-// complement mask with `a2`'s queries - the sliding window and the attention sinks of the sink + window types.
-enum { kLinear = 0, kPaged = 1, kBoth = 2, kSinks = 3 };
+// complement mask with `a2`'s queries - the sliding window and the attention sinks of the sink + window types - which the launch
+// rotates to the sinks' angle by the table of it that comes with them.  kSinksStaged: the same of queries that have been rotated, for
+// the one call whose scratch does not hold the table (a mode of its own: asking at run time cost the others 0.5 to 1.3 %, sinks +
+// window of 4,096 over 16,001 tokens 999 -> 1,013 us).
+enum { kLinear = 0, kPaged = 1, kBoth = 2, kSinks = 3, kSinksStaged = 4 };
 
 // The page table can ride in the launch itself (INLINE): the host passes up to kInlinePages entries by value, and the
 // kernel reads them where they lie in its argument segment - scalar loads through the constant address space, like the
@@ -145,7 +148,7 @@ constexpr int kWgsPerCu = D == 64 && (MODE == kLinear || MODE == kPaged) ? 2 : 1
 template <int D, int MODE, bool INLINE = false>
 __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage_kernel(infllm_attn_args a, infllm_attn_args a2, StageGeom geo,
                                                                  std::conditional_t<INLINE, InlinePages, NoInlinePages>) {
-    constexpr bool HAS_LIN = MODE != kPaged, HAS_PAG = MODE != kLinear, TWO = MODE == kBoth || MODE == kSinks;
+    constexpr bool HAS_LIN = MODE != kPaged, HAS_PAG = MODE != kLinear, SINKS = MODE == kSinks || MODE == kSinksStaged, TWO = MODE == kBoth || SINKS;
     constexpr int kRow = D * 2, kTB = kTileBytes<D>;                     // bytes of a row, of a tile
     constexpr bool PING = D == 128, kTurns = D == 128 && (MODE == kLinear || MODE == kSinks);
     const infllm_attn_args &ap = TWO ? a2 : a;                 // the paged stage's arguments
@@ -212,7 +215,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     }
     if (lin_t1 <= lin_t0) lin_t0 = lin_t1 = 0;
     // The unified tile list: u in [0, n_lin) is linear tile lin_t0 + u, u in [n_lin, n_lin + n_pag) is page u - n_lin.
-    const int n_lin = lin_t1 - lin_t0, n_pag = MODE == kSinks ? ((int)ap.j_hi + kTile - 1) >> 6 : HAS_PAG ? ap.n_pages : 0;
+    const int n_lin = lin_t1 - lin_t0, n_pag = SINKS ? ((int)ap.j_hi + kTile - 1) >> 6 : HAS_PAG ? ap.n_pages : 0;
     int g_t0, g_t1;                      // this split's share of the list
     {
         // n / nsplit tiles each; the n % nsplit left over go one each to a run of splits in the middle: the first and
@@ -312,7 +315,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         const bf16_t *kbase, *vbase;
         const bool paged = MODE == kPaged || (TWO && u >= n_lin);
         int valid = kTile;
-        if (MODE == kSinks && paged) {
+        if (SINKS && paged) {
             const int64_t j0 = (int64_t)(u - n_lin) * kTile;
             kbase = (const bf16_t *)ap.d_k + (int64_t)b * ap.k_sb + (int64_t)g * ap.k_sh + j0 * D;
             vbase = (const bf16_t *)ap.d_v + (int64_t)b * ap.v_sb + (int64_t)g * ap.v_sh + j0 * D;
@@ -401,7 +404,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         } else if (a.mask == INFLLM_MASK_COMPLEMENT)
             clear_hi = min(clear_hi, tile_of(q0 - (kTile - 1) - a.window) + 1 - lin_t0);
         clear_hi = min(clear_hi, n_lin);
-        if (MODE == kSinks) clear_pag = n_lin + min(floordiv64(ap.j_hi), tile_of((int64_t)i0 + ap.offset - (kTile - 1) - ap.window) + 1);
+        if (SINKS) clear_pag = n_lin + min(floordiv64(ap.j_hi), tile_of((int64_t)i0 + ap.offset - (kTile - 1) - ap.window) + 1);
     }
     // the mask of a tile's scores (valid: rows of a page)
     auto mask = [&](f32x16 (&s)[2], int t, [[maybe_unused]] int valid) {
@@ -409,7 +412,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         if (!(PAGES && paged ? valid == kTile : TWO && paged ? t < clear_pag : t >= clear_lo && t < clear_hi)) {
             int row_lo = 0, row_hi = kTile;
             int d0 = 0;                        // dist of (this lane's query, key 0 of the tile), clamped into int32
-            if (MODE == kSinks && paged) {
+            if (SINKS && paged) {
                 const int64_t j0 = (int64_t)(t - n_lin) * kTile, e0 = (int64_t)i0 + ap.offset - j0;
                 row_hi = (int)min((int64_t)kTile, ap.j_hi - j0);
                 d0 = (int)min(max(e0, (int64_t)-kBig), (int64_t)kBig) + col;
@@ -424,9 +427,9 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             // Whatever the mask, a lane's query sees ONE run of the tile's keys: its bounds are found once, and a key costs a
             // subtraction and a compare (a mask's conditions key by key: 150 branches in the sinks' form of the kernel).
             // dist = dl - kc; kc is the compile-time part of register r's key, which is kc + 8 * grp
-            const int win = (int)min(MODE == kSinks && paged ? ap.window : a.window, (int64_t)2 * kBig), dl = d0 - 8 * grp;
+            const int win = (int)min(SINKS && paged ? ap.window : a.window, (int64_t)2 * kBig), dl = d0 - 8 * grp;
             int lo_l = row_lo - 8 * grp, hi_l = row_hi - 8 * grp;
-            if (MODE == kSinks && paged) {
+            if (SINKS && paged) {
                 hi_l = min(hi_l, dl - win + 1);
             } else if (!paged) {
                 if (a.mask == INFLLM_MASK_WINDOW) lo_l = max(lo_l, dl - win + 1), hi_l = min(hi_l, dl + 1);
@@ -586,7 +589,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     };
     // does this wave see tile u at all?  (pages: every live wave; linear tiles: the wave's own visible range)
     auto mine = [&](int u) {
-        if (MODE == kSinks && u >= n_lin) return live && (int64_t)i1 + ap.offset - ap.window >= (int64_t)(u - n_lin) * kTile;
+        if (SINKS && u >= n_lin) return live && (int64_t)i1 + ap.offset - ap.window >= (int64_t)(u - n_lin) * kTile;
         return (HAS_PAG && u >= n_lin) ? live : (u >= wu0 && u < wu1);
     };
     // the queries of the stage this split starts in; a split that crosses from the linear tiles into the pages swaps
@@ -780,7 +783,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
             qreg[kk + D / 32] = __builtin_bit_cast(bf16x8, r.hi);
             asm volatile("" : "+v"(qreg[kk]), "+v"(qreg[kk + D / 32]));                 // (read before the barrier)
         }
-    } else if (MODE != kPaged && !(MODE == kSinks && q_paged) && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
+    } else if (MODE != kPaged && !(SINKS && q_paged) && (uint64_t)first.q_sl < (uint64_t)1 << 26) {
         const uint32_t at_q = (wave < 4 ? lds_address(Ks) : lds_address(Vs)) + 2 * kTB + (wave & 3) * (kQTile * kRow);
         const bf16_t *rows = (const bf16_t *)first.d_q + (int64_t)b * first.q_sb + (int64_t)h * first.q_sh + (int64_t)i0 * first.q_sl;
 #pragma unroll
@@ -1138,7 +1141,7 @@ int launch_mode(dim3 grid, const infllm_attn_args &a, const infllm_attn_args &a2
     return 0;
 }
 
-// mode: kLinear (a), kPaged (a), kBoth / kSinks (a = linear stage, a2 = the other stage); h_pages: NULL, or the paged
+// mode: kLinear (a), kPaged (a), kBoth / kSinks / kSinksStaged (a = linear stage, a2 = the other stage); h_pages: NULL, or the paged
 // stage's table [B, n_pages] in HOST memory, B * n_pages <= kInlinePages, which then travels in the launch (d_pages is
 // not read)
 template <int D = kD>
@@ -1167,7 +1170,8 @@ int launch_stage(int mode, const infllm_attn_args *a, const infllm_attn_args *a2
         case kLinear: return launch_mode<D, kLinear, false>(grid, *a, second, geo, NoInlinePages{}, stream);
         case kPaged: return launch_mode<D, kPaged, false>(grid, *a, second, geo, NoInlinePages{}, stream);
         case kBoth: return launch_mode<D, kBoth, false>(grid, *a, second, geo, NoInlinePages{}, stream);
-        default: return launch_mode<D, kSinks, false>(grid, *a, second, geo, NoInlinePages{}, stream);
+        case kSinks: return launch_mode<D, kSinks, false>(grid, *a, second, geo, NoInlinePages{}, stream);
+        default: return launch_mode<D, kSinksStaged, false>(grid, *a, second, geo, NoInlinePages{}, stream);
     }
 }
 
@@ -1457,7 +1461,7 @@ extern "C" int infllm_attn_merge_pair(const uint16_t *d_o_part, const float *d_l
 // softmax, as rows of `dim` elements (128 or 64) in the caller's layout; local->nsplit key splits of the joint tile list,
 // with partial rows at local->d_o_part / d_lse_part when there is more than one
 // d_pages of `local`: NULL, or cosine and sine of every query's angles [Lq, 64], by which the launch rotates the rows as they come
-// (infllm_attn_turns); of `sinks`: of the one angle of theirs.
+// (infllm_attn_turns); of `sinks`: of the one angle of theirs [dim / 2], by which it rotates the rows of their d_q, or NULL.
 bool infllm_attn_turns(int32_t H, int32_t Hkv, int32_t n_q, int64_t q_sl, int32_t dim) {
     const int G = H / Hkv;
     return dim == 128 && (G == 4 || G >= 8) && q_sl >= 0 && q_sl < 1 << 26 && n_q < 1 << 22;
@@ -1470,7 +1474,7 @@ int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *si
     rc = check_linear_stage(local);
     if (rc) return rc;
     if (sinks) {
-        INFLLM_REQUIRE(sinks->d_q && sinks->d_pages && sinks->d_k && sinks->d_v && sinks->j_lo == 0 && sinks->j_hi >= 0 && sinks->k_sl == dim && sinks->v_sl == dim,
+        INFLLM_REQUIRE(sinks->d_q && sinks->d_k && sinks->d_v && sinks->j_lo == 0 && sinks->j_hi >= 0 && sinks->k_sl == dim && sinks->v_sl == dim,
                        "attn_window: bad sink rows");
         INFLLM_REQUIRE(sinks->Lq == local->Lq && sinks->B == local->B && sinks->H == local->H && ((sinks->q_sl | sinks->q_sh | sinks->q_sb) & 7) == 0,
                        "attn_window: the two stages disagree");
@@ -1482,7 +1486,7 @@ int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *si
         so.o_sb = o_sb; so.o_sh = o_sh; so.o_sl = o_sl;
     } else
         INFLLM_REQUIRE(local->d_o_part && local->d_lse_part, "attn_window: splits without partial rows");
-    const int mode = sinks ? kSinks : kLinear;
+    const int mode = !sinks ? kLinear : sinks->d_pages ? kSinks : kSinksStaged;
     rc = dim == 128 ? launch_stage<128>(mode, local, sinks, stream, nullptr, so) : launch_stage<64>(mode, local, sinks, stream, nullptr, so);
     if (rc || local->nsplit == 1) return rc;
     return infllm_attn_merge2(local->d_o_part, local->d_lse_part, local->nsplit, nullptr, nullptr, 0, local->B, local->H, local->Lq, d_out, o_sb, o_sh, o_sl,

@@ -248,8 +248,11 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     j.glb_pos = a->kind == 2 ? a->n_local - 1 : a->n_local + a->n_init - 1;
     j.inv_freq = a->d_inv_freq; j.distance_scale = a->distance_scale;
     j.q_loc = q_loc;
-    if (sink_stage && step) j.q_glb = q_sink;                    // (several queries are rotated to the sinks' angle where they are attended)
-    else if (sink_stage) j.glb_cs = (float2 *)q_sink;
+    // Queries are rotated to the sinks' angle where they are attended, by a table of it in their place, which two rows fill and one
+    // row does not hold.
+    const bool sink_turns = sink_stage && !step && rows_q >= 2;
+    if (sink_turns) j.glb_cs = (float2 *)q_sink;
+    else if (sink_stage) j.q_glb = q_sink;
     j.dk = bk + (rows_base - a->n_new) * D; j.dv = bv + (rows_base - a->n_new) * D;
     j.dk_sb = bk_sb; j.dk_sh = bk_sh; j.dv_sb = bv_sb; j.dv_sh = bv_sh;
     const int64_t raw_sh = (int64_t)a->raw_new * D;
@@ -400,9 +403,12 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     l.softmax_scale = scale;
     if (sink_stage) {
         s = l;
-        s.d_q = a->d_q;
-        s.q_sl = a->q_sl; s.q_sh = a->q_sh; s.q_sb = a->q_sb;
-        s.d_pages = (const infllm_page *)q_sink;
+        if (sink_turns) {
+            s.d_q = a->d_q;
+            s.q_sl = a->q_sl; s.q_sh = a->q_sh; s.q_sb = a->q_sb;
+            s.d_pages = (const infllm_page *)q_sink;
+        } else
+            s.d_q = q_sink;
         s.d_k = sk; s.k_sh = sk_sh; s.k_sb = sk_sb;
         s.j_lo = 0; s.j_hi = n_sink;
         s.mask = INFLLM_MASK_COMPLEMENT;
