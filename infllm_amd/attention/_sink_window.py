@@ -49,8 +49,8 @@ def _step_bytes(kind, batch, heads, dim):
 
 def _take_words(past_k, n, step_bytes, dev, stream):
     """((tensor, address of n words or more in which a step counts its finished key splits, their number, the stream they belong to,
-    address and size of a step's scratch behind them, size 0 where it would be more than _STEP_BYTES) and whether the call has to clear
-    the words, or None: it counts in words of its own scratch.
+    address and size of a scratch behind them: of step_bytes or more, or, where that is more than _STEP_BYTES, of any size) and whether
+    the call has to clear the words, or None: it counts in words of its own scratch.
 
     The words are zero between the launches that use them, and only one call has them and the scratch at a time: it takes them off the
     storage of the cache it continues (one operation, whichever threads go on from that cache) and leaves them with the cache it
@@ -232,8 +232,9 @@ def _call(kind, n_local, n_init, query, key_value, position_bias, past, project_
         rows_q = batch * num_heads * len_q
         part_rows = 64 * rows_q if rows_q <= 2048 else _SPLIT_ROWS if 2 * rows_q <= _SPLIT_ROWS else 0
         work_bytes = (2 if kind else 1) * rows_q * dim * 2 + part_rows * (2 * dim + 4)
-    # (a step's scratch comes with its words: one allocation of the three that its output, its cache and it take)
-    if len_q == 1 and words is not None and words[5]:
+    # (a step's scratch comes with its words: one allocation of the three that its output, its cache and it take; words of a call that
+    # needed less come with less)
+    if len_q == 1 and words is not None and words[5] >= work_bytes:
         work_ptr = words[4]
     else:
         work = torch.empty((work_bytes,), dtype=torch.uint8, device=dev)

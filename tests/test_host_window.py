@@ -233,6 +233,34 @@ def test_words_of_a_cache_are_used_by_one_call_at_a_time(kind, native, monkeypat
     assert [args[-1] for args, _ in native.calls] == [1, 0, 1, 0, 1, 1, 0]
 
 
+def test_a_step_takes_no_more_scratch_than_its_cache_brings(native, monkeypatch):
+    """A causal cache of 248 query rows of 128 keeps a step's scratch of just under 4 MiB; a step of the sink + window types over the same
+    cache has the queries twice and takes more than is kept."""
+    made = []
+
+    def remembering(make):
+        def call(*args, **kw):
+            t = make(*args, **kw)
+            made.append((t.data_ptr(), t.numel() * t.element_size(), weakref.ref(t)))
+            return t
+        return call
+    monkeypatch.setattr(torch, "empty", remembering(torch.empty))
+    fields = [n for n, _ in _sink_window._lib.WindowArgs._fields_]
+    inside = []
+
+    def launch(args, stream):                                 # (while the call holds what it made)
+        a = dict(zip(fields, _sink_window._ARGS.unpack(args)))
+        inside.append(any(r() is not None and at <= a["d_work"] and a["d_work"] + a["work_bytes"] <= at + size for at, size, r in made))
+        return 0
+    monkeypatch.setattr(native, "infllm_window_forward", launch)
+    _, past = layer("origin", None, 30, batch=62)
+    _, past = layer("origin", past, 1, batch=62)
+    for kind in ("stream-llm", "origin"):
+        _, more = layer(kind, past if kind == "origin" else (past[0], past[1], 31, None), 1, batch=62)
+    layer("stream-llm", (more[0], more[1], 32, None), 1, batch=62)
+    assert inside == [True] * 5
+
+
 def misaligned(*shape):
     """contiguous, but two bytes off"""
     n = 1
