@@ -71,6 +71,9 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv &f) { return 
 
 // launch constants the kernel would otherwise derive with divisions
 struct StageGeom {
+    // Cosines and sines by which the launch rotates queries that come as they are: of every query's position [Lq, 64] (kLinear and kSinks,
+    // heads of 128; NULL: the linear stage's queries are rotated), of the sinks' one angle [D / 2] (kSinks).
+    const float2 *q_angles, *sink_angle;
     FastDiv gx, gy, hkv, group, nsplit, cap_tiles;
     int32_t n_tasks;
     // Partial rows by execution block (out_exc > 0): the queries are those of several consecutive execution blocks of
@@ -192,7 +195,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     const int i0 = qt * kQTile, i1 = min(i0 + kQTile, a.Lq) - 1;
 
     if (MODE == kSinks && wave < D / 64)                         // 256 bytes a wave, there with the first tile
-        load_to_lds4((const float *)ap.d_pages, wave * 256 + lane * 4, lds_address((char *)sink_cs) + wave * 256);
+        load_to_lds4((const float *)geo.sink_angle, wave * 256 + lane * 4, lds_address((char *)sink_cs) + wave * 256);
     int w_t0 = 0, w_t1 = 0;              // this wave's range of LINEAR tiles (absolute tile numbers)
     if (HAS_LIN && live) {
         StageRange r = visible_range(a, i0, i1);
@@ -559,10 +562,9 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         l_run += sums[0];
     };
 
-    // The sinks' queries are the step's own rows, rotated here to the one angle of the sinks (d_pages of their arguments: cosine and sine of
-    // every frequency): staged beside the others they were a third of
-    // what the staging launch wrote (sinks + window of 4,096 over 16,001 tokens, 32 / 8 heads of 128: 1,063 -> 1,041 us; window of 2,048 over two rows
-    // of 8,001: 633 -> 612; 36 heads of 64, whose sinks' queries are a seventh: 371 -> 370).
+    // The sinks' queries are the step's own rows, rotated here to the one angle of the sinks: staged beside the others they were a third
+    // of what the staging launch wrote (sinks + window of 4,096 over 16,001 tokens, 32 / 8 heads of 128: 1,063 -> 1,041 us; window of
+    // 2,048 over two rows of 8,001: 633 -> 612; 36 heads of 64, whose sinks' queries are a seventh: 371 -> 370).
     auto load_q = [&](const infllm_attn_args &src, [[maybe_unused]] bool sinks) {
         const int qi = i0 + col;
         const bool ok = live && qi < src.Lq;
@@ -750,7 +752,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     // they have been read.  (By lanes that each fetch their own query's pieces, 32 lines an instruction: sinks + window of 4,096 over 16,001
     // tokens 1,060 -> 1,041 us, of 512 over 7,596 174.7 -> 167.2, causal prompt of 8,001 542 -> 535.)
     // (Two tiles of queries a workgroup at most: infllm_attn_turns.)
-    const bool turn_lds = kTurns && a.d_pages && !q_paged;
+    const bool turn_lds = kTurns && geo.q_angles && !q_paged;
     if (turn_lds) {
         const int qt0 = (int)fdiv(bx * kWaves, geo.group), half = wave >> 2;
         const uint32_t at_q = (wave < 4 ? lds_address(Ks) : lds_address(Vs)) + 2 * kTB + (wave & 3) * (kQTile * kRow);
@@ -764,7 +766,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int r = ((wave & 3) * 4 + i) * 2 + (lane >> 5), q = min((qt0 + half) * kQTile + r, a.Lq - 1);
-            load_to_lds16((const bf16_t *)a.d_pages, (uint32_t)q * (D * 4) + ((lane & 31) ^ r) * 16, angles + ((wave & 3) * 4 + i) * 1024);
+            load_to_lds16((const bf16_t *)geo.q_angles, (uint32_t)q * (D * 4) + ((lane & 31) ^ r) * 16, angles + ((wave & 3) * 4 + i) * 1024);
         }
         if (t < g_t1) valid0 = load_tile(t, 0);
         landed();
@@ -1119,12 +1121,13 @@ int check_common(const infllm_attn_args *a) {
     return 0;
 }
 
-// Where a launch's rows go besides the argument block's partial buffers: see StageGeom
+// Where a launch's rows go besides the argument block's partial buffers, and what it rotates its queries by: see StageGeom
 struct StageOut {
     int out_exc = 0;
     int64_t out_block_rows = 0;
     bf16_t *out = nullptr;
     int64_t o_sb = 0, o_sh = 0, o_sl = 0;
+    const float2 *q_angles = nullptr, *sink_angle = nullptr;
 };
 
 template <int D, int MODE, bool INLINE, typename Pages>
@@ -1151,7 +1154,7 @@ int launch_stage(int mode, const infllm_attn_args *a, const infllm_attn_args *a2
     const int n_tasks = ((a->Lq + kQTile - 1) / kQTile) * G;
     dim3 grid((n_tasks + kWaves - 1) / kWaves, a->B * a->Hkv, a->nsplit);
     INFLLM_REQUIRE((int64_t)grid.x * grid.y * grid.z < (1ll << 31), "attn_stage: grid too large");
-    StageGeom geo{fast_div(grid.x), fast_div(grid.y), fast_div((uint32_t)a->Hkv), fast_div((uint32_t)G),
+    StageGeom geo{so.q_angles, so.sink_angle, fast_div(grid.x), fast_div(grid.y), fast_div((uint32_t)a->Hkv), fast_div((uint32_t)G),
                   fast_div((uint32_t)a->nsplit), fast_div(1), n_tasks, so.out_exc, so.out_block_rows,
                   fast_div((uint32_t)(so.out_exc > 0 ? so.out_exc : 1)), so.out, so.o_sb, so.o_sh, so.o_sl};
     // tile indices stay below 2^30, so any ring of 2^31 tiles or more never wraps: one divisor stands for all of them
@@ -1460,14 +1463,14 @@ extern "C" int infllm_attn_merge_pair(const uint16_t *d_o_part, const float *d_l
 // library-internal: a linear stage and (sinks != NULL) the rows of a second source under the complement mask, under one
 // softmax, as rows of `dim` elements (128 or 64) in the caller's layout; local->nsplit key splits of the joint tile list,
 // with partial rows at local->d_o_part / d_lse_part when there is more than one
-// d_pages of `local`: NULL, or cosine and sine of every query's angles [Lq, 64], by which the launch rotates the rows as they come
-// (infllm_attn_turns); of `sinks`: of the one angle of theirs [dim / 2], by which it rotates the rows of their d_q, or NULL.
+// q_angles: NULL, or cosine and sine of every query's angles [Lq, 64], by which the launch rotates local's rows (infllm_attn_turns);
+// sink_angle: NULL, or of the one angle of the sinks' queries [dim / 2], by which it rotates theirs
 bool infllm_attn_turns(int32_t H, int32_t Hkv, int32_t n_q, int64_t q_sl, int32_t dim) {
     const int G = H / Hkv;
     return dim == 128 && (G == 4 || G >= 8) && q_sl >= 0 && q_sl < 1 << 26 && n_q < 1 << 22;
 }
-int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, int32_t dim, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
-                       void *stream) {
+int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, const void *q_angles, const void *sink_angle, int32_t dim, void *d_out,
+                       int64_t o_sb, int64_t o_sh, int64_t o_sl, void *stream) {
     INFLLM_REQUIRE(local && d_out && (dim == 128 || dim == 64), "attn_window: bad arguments");
     int rc = check_common(local);
     if (rc) return rc;
@@ -1479,14 +1482,16 @@ int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *si
         INFLLM_REQUIRE(sinks->Lq == local->Lq && sinks->B == local->B && sinks->H == local->H && ((sinks->q_sl | sinks->q_sh | sinks->q_sb) & 7) == 0,
                        "attn_window: the two stages disagree");
     }
-    INFLLM_REQUIRE(!local->d_pages || infllm_attn_turns(local->H, local->Hkv, local->Lq, local->q_sl, dim), "attn_window: queries that are not rotated");
+    INFLLM_REQUIRE(!q_angles || infllm_attn_turns(local->H, local->Hkv, local->Lq, local->q_sl, dim), "attn_window: queries that are not rotated");
     StageOut so;
+    so.q_angles = (const float2 *)q_angles;
+    so.sink_angle = (const float2 *)sink_angle;
     if (local->nsplit == 1) {
         so.out = (bf16_t *)d_out;
         so.o_sb = o_sb; so.o_sh = o_sh; so.o_sl = o_sl;
     } else
         INFLLM_REQUIRE(local->d_o_part && local->d_lse_part, "attn_window: splits without partial rows");
-    const int mode = !sinks ? kLinear : sinks->d_pages ? kSinks : kSinksStaged;
+    const int mode = !sinks ? kLinear : sink_angle ? kSinks : kSinksStaged;
     rc = dim == 128 ? launch_stage<128>(mode, local, sinks, stream, nullptr, so) : launch_stage<64>(mode, local, sinks, stream, nullptr, so);
     if (rc || local->nsplit == 1) return rc;
     return infllm_attn_merge2(local->d_o_part, local->d_lse_part, local->nsplit, nullptr, nullptr, 0, local->B, local->H, local->Lq, d_out, o_sb, o_sh, o_sl,

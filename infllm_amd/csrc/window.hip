@@ -6,8 +6,8 @@
 #include "decode.h"
 #include "rope.h"
 
-int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, int32_t dim, void *d_out, int64_t o_sb, int64_t o_sh, int64_t o_sl,
-                       void *stream);
+int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, const void *q_angles, const void *sink_angle, int32_t dim, void *d_out,
+                       int64_t o_sb, int64_t o_sh, int64_t o_sl, void *stream);
 bool infllm_attn_turns(int32_t H, int32_t Hkv, int32_t n_q, int64_t q_sl, int32_t dim);
 namespace {
 
@@ -385,7 +385,6 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     if (turns) {
         l.d_q = a->d_q;
         l.q_sl = a->q_sl; l.q_sh = a->q_sh; l.q_sb = a->q_sb;
-        l.d_pages = (const infllm_page *)j.pos_cs;
     } else {
         l.d_q = q_loc;
         l.q_sl = D; l.q_sh = (int64_t)a->n_q * D; l.q_sb = (int64_t)a->H * a->n_q * D;
@@ -406,7 +405,6 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         if (sink_turns) {
             s.d_q = a->d_q;
             s.q_sl = a->q_sl; s.q_sh = a->q_sh; s.q_sb = a->q_sb;
-            s.d_pages = (const infllm_page *)q_sink;
         } else
             s.d_q = q_sink;
         s.d_k = sk; s.k_sh = sk_sh; s.k_sb = sk_sb;
@@ -422,5 +420,5 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     l.nsplit = infllm_attn_splits(wgs, tiles, max_parts, std::min((double)tiles, (near + n_sink) / kTile + 1.0));
     l.d_o_part = (uint16_t *)((char *)a->d_work + q_bytes);
     l.d_lse_part = (float *)((char *)a->d_work + q_bytes + part_rows * 2 * D);
-    return infllm_attn_window(&l, sink_stage ? &s : nullptr, D, a->d_out, a->o_sb, a->o_sh, a->o_sl, stream);
+    return infllm_attn_window(&l, sink_stage ? &s : nullptr, j.pos_cs, j.glb_cs, D, a->d_out, a->o_sb, a->o_sh, a->o_sl, stream);
 }
