@@ -335,7 +335,9 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     // on): the staging reads and writes 67 MB less of 4,096 tokens x 32 heads of 128.  Staged / so, 32 / 8 heads of 128, causal prompts of
     // 1,537 / 2,049 / 3,073 / 8,001 tokens 60.9 / 80.5 / 114.9 / 549.7 and 59.6 / 78.0 / 111.3 / 535.4 us; sinks + window of 1,024 over 1,537 /
     // 3,073 67.5 / 101.8 and 67.2 / 101.3; below, the host bounds them.
-    const bool turns = !step && a->n_q == a->n_new && (int64_t)a->B * a->H >= 2 && infllm_attn_turns(a->H, a->Hkv, a->n_q, a->q_sl, D);
+    // (Straight into LDS, 16 bytes a lane: rows that begin between two such pieces are staged, by loads into registers.)
+    const bool turns = !step && a->n_q == a->n_new && (int64_t)a->B * a->H >= 2 && infllm_attn_turns(a->H, a->Hkv, a->n_q, a->q_sl, D) &&
+                       ((uintptr_t)a->d_q & 15) == 0;
     if (a->n_q == a->n_new) {
         j.do_q = !turns;
         j.do_kv = 1;

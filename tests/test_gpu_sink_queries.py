@@ -65,3 +65,43 @@ def test_queries_rotated_where_they_are_attended(kind, B, H, Hkv, n):
         # results rounded to bf16, 2^-8 of an element each at most and a third of that in the mean square; the rest of 2^-7 for
         # probabilities, partial rows and single rotated elements that are rounded another way
         assert float((got[:, :, i].float() - want).norm()) <= 2.0 ** -7 * float(want.norm()), i
+
+
+@pytest.mark.parametrize("kind", ["origin", "stream-llm", "infinite-lm"])
+@pytest.mark.parametrize("off", [1, 2, 4, 8])
+def test_queries_at_any_address(kind, off, monkeypatch):
+    """Query rows that begin `off` elements behind a multiple of 16 bytes (a caller of the C function may have such): those of the calls
+    whose attention would take them straight into LDS are staged, and the results differ as the two ways do."""
+    from infllm_amd import _lib
+    from infllm_amd.attention import ATTN_FORWRAD, RotaryEmbeddingESM, _sink_window
+    B, H, Hkv, D, g = 1, 8, 2, 128, torch.Generator(device="cuda").manual_seed(off)
+    calls, fields, lib = [333, 70], [n for n, _ in _lib.WindowArgs._fields_], _lib.load()
+    x = [torch.randn((B, sum(calls), h * D), generator=g, device="cuda").bfloat16() for h in (H, Hkv, Hkv)]
+    forward = ATTN_FORWRAD[kind](False) if kind == "origin" else ATTN_FORWRAD[kind](100, 30, fattn=False)
+    rope, same, rooms = RotaryEmbeddingESM(D, base=1e4, device="cuda"), lambda t: t, []
+
+    class Moved:
+        def infllm_window_forward(self, args, stream):
+            a = dict(zip(fields, _sink_window._ARGS.unpack(args)))
+            n = B * a["n_q"] * H * D
+            rooms.append(torch.empty((n + 16,), dtype=torch.bfloat16, device="cuda"))
+            rooms[-1][off:off + n] = now[0].flatten()
+            assert a["d_q"] % 16 == 0 and a["q_sl"] == H * D and rooms[-1].data_ptr() % 16 == 0
+            a["d_q"] = rooms[-1].data_ptr() + 2 * off
+            return lib.infllm_window_forward(_sink_window._ARGS.pack(*(a[f] for f in fields)), stream)
+    now = [None]
+
+    def run():
+        past, outs, at = None, [], 0
+        for n in calls:
+            now[0], k, v = (t[:, at:at + n].contiguous() for t in x)
+            o, past = forward(None, now[0], k, rope, True, past, same, same, lambda _: v, same, D, H, Hkv)
+            outs.append(o)
+            at += n
+        return torch.cat(outs, dim=1).float()
+    want = run()
+    monkeypatch.setattr(_sink_window._lib, "load", lambda: Moved())
+    got = run()
+    assert len(rooms) == len(calls)
+    # (as above: roundings of rotated elements, probabilities and results to bf16)
+    assert torch.equal(got, want) if off == 8 else float((got - want).norm()) <= 2.0 ** -7 * float(want.norm())
