@@ -47,3 +47,23 @@ def test_blocks_end_as_they_do_launch_by_launch(name, calls, H, Hkv, B, kw, monk
     a, b = cm.export_state(), ref.export_state()
     assert torch.equal(a["units"], b["units"].cpu()) and torch.equal(a["reps"].cpu(), b["reps"].cpu())
     assert torch.allclose(a["tail_score"], b["tail_score"], rtol=2e-3, atol=1e-5)
+
+
+@pytest.mark.parametrize("H,Hkv,D,B", [(8, 2, 128, 1), (6, 3, 64, 2), (40, 8, 128, 1)])
+def test_blocks_behind_more_chunks_of_units_than_a_ranking_keeps_addresses_of(H, Hkv, D, B, monkeypatch):
+    """A chunk for every unit, and more units than the 256 whose addresses a ranking workgroup reads ahead (rows of 40 x 128: a launch of
+    its own ranks): the same bits as with a few large chunks."""
+    import infllm_amd.attention.context_manager as manager_module
+    calls, kw = [5120, 5120, 1, 1100], dict(KW, block_size=32, dim=D, exc_block_size=256)
+    q, k, v = (t.cuda() for t in make_stream(sum(calls), H, Hkv, 11, B=B, D=D))
+
+    def run(unit_chunk):
+        monkeypatch.setattr(manager_module, "_UNIT_CHUNK", unit_chunk)
+        cm = new_manager(1e4, **kw)
+        return cm, feed(cm, q, k, v, calls)
+    cm, got = run(1)
+    ref, want = run(64)
+    assert cm._resident and ref._resident and len(cm._chunks) == cm.num_global_block > 300 and len(ref._chunks) < 10
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert cm.stats == ref.stats and all(a.cached == b.cached for a, b in zip(cm.policy, ref.policy))
+    assert torch.equal(cm.export_state()["units"], ref.export_state()["units"])

@@ -34,5 +34,39 @@ def test_a_step_selects_the_best_units(units, topk, B, how):
         assert torch.isfinite(cm.append(q, k, v, q, k, v)).all()
         scores = cm.unit_scores[:, :units]
         want = torch.sort(scores, dim=1, descending=True, stable=True).indices[:, :topk]
-        ids = cm._tables.view(torch.int32)[-2 * ((B * topk + 1) // 2):][:B * topk].view(B, topk)      # the selection ends the manager's tables
-        assert torch.equal(ids.long(), want), step
+        torch.cuda.synchronize()
+        log = cm._log.view(-1, B * topk + 1)                  # (infllm_resident_desc: log_slots x (the selection, its sequence number))
+        ids = log[log[:, -1].argmax(), :-1].view(B, topk)
+        assert torch.equal(ids.long(), want.cpu()), step
+
+
+@pytest.mark.parametrize("units,H,Hkv,D,B", [(2500, 4, 1, 128, 34), (2100, 36, 36, 64, 1), (4500, 8, 8, 64, 5), (2049, 33, 33, 128, 1), (2300, 32, 32, 128, 1)])
+def test_prologues_of_many_heads_beside_the_scores(units, H, Hkv, D, B, monkeypatch):
+    """More (batch row, kv head) pairs than the scores leave places for (32 of 256), behind units that fill them; and 32, which they do:
+    scores of every batch row, the books, the rows and the score track, against the host-driven path."""
+    from infllm_amd.attention import ContextManager
+    bs, n_init, n_local, topk = 8, 8, 64, 16
+    g = torch.Generator(device="cuda").manual_seed(units + B)
+    bf = lambda *s: torch.randn(s, generator=g, device="cuda").bfloat16()
+    state = dict(length=n_init + units * bs + n_local, tail_k=bf(B, Hkv, n_local, D), tail_v=bf(B, Hkv, n_local, D), tail_score=None, init_k=bf(B, Hkv, n_init, D),
+                 init_v=bf(B, Hkv, n_init, D), units=bf(units, B, 2, Hkv, bs, D), reps=bf(B, units, H * D))
+    steps = [(bf(B, H, 1, D), bf(B, Hkv, 1, D), bf(B, Hkv, 1, D)) for _ in range(3)]
+
+    def manager():
+        cm = new_manager(1e4, n_init=n_init, n_local=n_local, block_size=bs, max_cached_block=64, topk=topk, exc_block_size=32, repr_topk=1, dim=D)
+        return cm.load_state(state), [cm.append(*step, *step) for step in steps]
+    cm, got = manager()
+    monkeypatch.setattr(ContextManager, "resident_bytes", 0)
+    ref, want = manager()
+    assert cm._resident and not ref._resident
+    for a, b in zip(got, want):
+        err = (a.float() - b.float()).abs()
+        assert float(err.max()) <= 2e-2 and float(err.mean()) <= 2e-3, float(err.max())
+    # 32-bit sums of H * D products of N(0, 1) and a rotated N(0, 1), in another order: partial sums of the order of (H * D) ** 0.5, in
+    # chains of some 64
+    assert float((cm.unit_scores[:, :units] - ref.unit_scores[:, :units]).abs().max()) <= (H * D) ** 0.5 * 64 * 2.0 ** -23
+    assert cm.stats == ref.stats and all(a.cached == b.cached for a, b in zip(cm.policy, ref.policy))
+    a, b = cm.export_state(), ref.export_state()
+    for name in ("tail_k", "tail_v", "init_k", "init_v"):
+        assert torch.equal(a[name], b[name]), name
+    assert torch.allclose(a["tail_score"], b["tail_score"], rtol=2e-3, atol=1e-5)
