@@ -1460,15 +1460,21 @@ extern "C" int infllm_attn_merge_pair(const uint16_t *d_o_part, const float *d_l
     return infllm_attn_merge2(d_o_part, d_lse_part, P1, d_o_part2, d_lse_part2, P2, B, H, Lq, d_out, o_sb, o_sh, o_sl, d_lse, stream, kD);
 }
 
+// library-internal: whether a launch rotates its linear queries itself.  A workgroup has room for the angles of two tiles of queries:
+// its eight waves take eight consecutive (tile, query head of the group) pairs from a multiple of eight on, and those lie in two tiles
+// at most of groups of four heads and of six and more.  Six and seven are still staged; rotated here they would be the faster too (48 / 8
+// and 28 / 4 heads, causal prompts of 1,537 / 3,073 / 8,001 tokens 67.3 / 157.8 / 745.5 us and 63.2 / 126.6 / 459.3 staged, 63.7 / 150.4 /
+// 719.5 and 61.7 / 123.1 / 446.1 so).  Heads of 64 take their queries another way.  32-bit offsets have to reach rows and angles.
+bool infllm_attn_turns(int32_t H, int32_t Hkv, int32_t n_q, int64_t q_sl, int32_t dim) {
+    const int G = H / Hkv;
+    return dim == 128 && (G == 4 || G >= 8) && q_sl >= 0 && q_sl < 1 << 26 && n_q < 1 << 22;
+}
+
 // library-internal: a linear stage and (sinks != NULL) the rows of a second source under the complement mask, under one
 // softmax, as rows of `dim` elements (128 or 64) in the caller's layout; local->nsplit key splits of the joint tile list,
 // with partial rows at local->d_o_part / d_lse_part when there is more than one
 // q_angles: NULL, or cosine and sine of every query's angles [Lq, 64], by which the launch rotates local's rows (infllm_attn_turns);
 // sink_angle: NULL, or of the one angle of the sinks' queries [dim / 2], by which it rotates theirs
-bool infllm_attn_turns(int32_t H, int32_t Hkv, int32_t n_q, int64_t q_sl, int32_t dim) {
-    const int G = H / Hkv;
-    return dim == 128 && (G == 4 || G >= 8) && q_sl >= 0 && q_sl < 1 << 26 && n_q < 1 << 22;
-}
 int infllm_attn_window(const infllm_attn_args *local, const infllm_attn_args *sinks, const void *q_angles, const void *sink_angle, int32_t dim, void *d_out,
                        int64_t o_sb, int64_t o_sh, int64_t o_sl, void *stream) {
     INFLLM_REQUIRE(local && d_out && (dim == 128 || dim == 64), "attn_window: bad arguments");

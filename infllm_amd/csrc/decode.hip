@@ -582,9 +582,12 @@ int infllm_decode_memory_step(const DecodeJob *job, const infllm_ingest_args *in
     return dim == 128 ? launch_memory_step<128>(job, in, stream) : launch_memory_step<64>(job, in, stream);
 }
 
-// How many of a launch's splits the ranges get that wait for a selection (lead_blocks of 16 keys) so that they end with the others:
-// the selection takes about as long as three blocks of a wave (479 units: taken for 1 / 2 / 3 / 6 blocks 15.5 / 13.2 / 12.8 / 13.0 us;
-// 4,096: 17.2 / 14.5 / 14.6 / 14.7).
+// How many of a launch's splits the ranges get that wait for a selection (lead_blocks of 16 keys) so that they end with the others: the
+// selection is taken for as long as three blocks of a wave.  It reads all scores twice and lasts the longer the more there are, but the
+// launch depends little on where between two and six the line lies.  (The kernel alone, 32 / 8 heads of 128, 16 of 20 / 479 / 4,096 /
+// 16,384 units, taken for 1, 2, 3, 6 and 9 blocks: 13.2 11.9 12.1 12.2 11.9 / 14.3 12.4 12.3 12.4 12.1 / 15.8 13.2 13.6 13.5 13.4 /
+// 23.2 20.7 20.7 20.6 20.6 us; 64 of 16,384: 36.9 36.1 36.5 36.8 36.1; 36 heads of 64, 15 splits each, 16 of
+// 512: 17.6 16.2 16.4 15.9 21.8.)
 int infllm_decode_lead_splits(int32_t nsplit, int64_t lead_blocks, int64_t blocks) {
     int best = 1;
     int64_t best_time = INT64_MAX;

@@ -66,8 +66,9 @@ __global__ __launch_bounds__(256) void pages_kernel(PageList j) {
 }
 
 // The end of a decode step: output rows = the joined splits; the window's score track += the probabilities, from the
-// logits that the attention launch left behind; and the step's selection on its way to the host's log, whose write across
-// the bus then runs beside the rest instead of behind the retrieval (which ended 3 us earlier without it).
+// logits that the attention launch left behind; and the number of the step in the host's log, where the attention that selected the
+// units has left their ids.  Of a selection that launches of its own made (more units or longer rows than a step's scores take, one split) the
+// ids are copied there too.
 // grid (B * H, 1 + ceil(window / 1024)): y == 0 joins, the others score.  A handful of loads per thread and nothing else, so
 // all of them are requested before the first is waited for (32 heads, 64 splits: 11.4 -> 6 us with the splits' rows as
 // 16-byte pieces, one batch instead of a chain of four).

@@ -21,7 +21,9 @@ struct SelectLds {
 template <int THREADS>
 __device__ __forceinline__ void select_units(const float *scores, int N, int k, int32_t *ids, SelectLds<THREADS> &lds) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int kBatch = 8;              // loads in flight (16: 479 scores 0.5 us more, 4,096 0.3 less)
+    // Loads in flight.  (16: the kernel of a step that takes 16 of 100 / 479 / 2,048 units 0.3 / 0.5 / 0.1 us longer, 64 of them 1.0 / 1.2 /
+    // 0.3; 16 of 4,096 / 8,192 / 16,384 0.2 / 0.9 / 1.4 shorter, 64 of them 0.6 / 1.4 / 1.9: a step seldom has more than 4,096.)
+    constexpr int kBatch = 8;
     auto each = [&](auto &&f) {            // f(score's key, unit) of this thread's units
         for (int n0 = tid; n0 < N; n0 += kBatch * THREADS) {
             float sc[kBatch];
