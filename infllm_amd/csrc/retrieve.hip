@@ -574,27 +574,32 @@ struct StepFront {
     infllm_ingest_args in;             // one new position
     int32_t dim, b, n_retrieve;        // whose query (batch row) the scores are for; workgroups that score
 };
-struct NoFront {};
+// ... of a retrieval by itself: the k best of the scores, by the workgroup that ends last (infllm_retrieve_fused)
+struct Selection {
+    const float *qbar;                 // the mean query
+    int32_t k;
+    int32_t *idx, *idx2, *flag;
+    int32_t flag_value;
+    uint32_t *ticket;                  // the caller's word, or NULL: the library's at `slot`
+    int32_t slot;
+};
 
 // CPL: 512-element pieces of a row; TAIL: the row is shorter than that (C elements; the lanes beyond it hold zeros)
-template <int CPL, int ROWS, bool TAIL, bool FRONT = false>
-__global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16_t *reps, int64_t rep_stride, int N, int C_, const float *qbar,
-                                                                      float *scores, int k, int32_t *idx_out, int32_t *idx_out2,
-                                                                      int32_t *flag, int32_t flag_value, uint32_t *own_ticket, int ticket_slot,
-                                                                      std::conditional_t<FRONT, StepFront, NoFront> front) {
+template <int CPL, int ROWS, bool TAIL, typename Job>
+__device__ __forceinline__ void score_rows(const bf16_t *reps, int64_t rep_stride, int N, int C_, float *scores, const Job &job) {
+    constexpr bool FRONT = std::is_same_v<Job, StepFront>;
     extern __shared__ float qs[];                                // the mean query
-    __shared__ int is_last;
     const int C = TAIL ? C_ : CPL * 512;
     const int lane = threadIdx.x & 63;
     const int waves_per_wg = kRetrThreads / 64;
     int n_wgs = gridDim.x;
     if constexpr (FRONT) {
-        n_wgs = front.n_retrieve;
+        n_wgs = job.n_retrieve;
         if ((int)blockIdx.x >= n_wgs) {
-            const int x = (int)blockIdx.x - n_wgs, b = x / front.in.Hkv, g = x - b * front.in.Hkv;
+            const int x = (int)blockIdx.x - n_wgs, b = x / job.in.Hkv, g = x - b * job.in.Hkv;
             if (threadIdx.x >= 256) return;                      // (whole waves; the others' barriers do not wait for them)
-            if (front.dim == 128) ingest_one<128>(front.in, b, g, (float2 *)qs);
-            else ingest_one<64>(front.in, b, g, (float2 *)qs);
+            if (job.dim == 128) ingest_one<128>(job.in, b, g, (float2 *)qs);
+            else ingest_one<64>(job.in, b, g, (float2 *)qs);
             return;
         }
     }
@@ -604,12 +609,12 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
     float freq = 0.f;
     u32x4 q_lo{}, q_hi{};                                        // (C <= 16 * kRetrThreads: eight pairs a thread)
     if constexpr (FRONT) {                                       // the query ahead of the rows: it is waited for first
-        const infllm_ingest_args &in = front.in;
-        const int c2 = front.dim / 16, h = (int)threadIdx.x / c2;
-        freq = in.d_inv_freq[(int)threadIdx.x & (front.dim / 2 - 1)];
+        const infllm_ingest_args &in = job.in;
+        const int c2 = job.dim / 16, h = (int)threadIdx.x / c2;
+        freq = in.d_inv_freq[(int)threadIdx.x & (job.dim / 2 - 1)];
         if (h < in.H) {
-            const bf16_t *src = (const bf16_t *)in.d_q + (int64_t)front.b * in.q_sb + (int64_t)h * in.q_sh + ((int)threadIdx.x - h * c2) * 8;
-            q_lo = *(const u32x4 *)src, q_hi = *(const u32x4 *)(src + front.dim / 2);
+            const bf16_t *src = (const bf16_t *)in.d_q + (int64_t)job.b * in.q_sb + (int64_t)h * in.q_sh + ((int)threadIdx.x - h * c2) * 8;
+            q_lo = *(const u32x4 *)src, q_hi = *(const u32x4 *)(src + job.dim / 2);
         }
         asm volatile("" ::: "memory");
     }
@@ -623,8 +628,8 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
         }
     if constexpr (FRONT) {
         __shared__ float2 cs[kD / 2];
-        const infllm_ingest_args &in = front.in;
-        const int half = front.dim / 2, c2 = front.dim / 16, tid = threadIdx.x, h = tid / c2, c = (tid - h * c2) * 8;
+        const infllm_ingest_args &in = job.in;
+        const int half = job.dim / 2, c2 = job.dim / 16, tid = threadIdx.x, h = tid / c2, c = (tid - h * c2) * 8;
         if (tid < half) {
             double sn, cn;
             sincos((double)in.glb_pos * in.distance_scale * (double)freq, &sn, &cn);
@@ -636,12 +641,12 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
         if (h < in.H) {
             float raw[16];
             rotate8(q_lo, q_hi, cs + c, raw);
-            float *dst = qs + h * front.dim + c;
+            float *dst = qs + h * job.dim + c;
 #pragma unroll
             for (int i = 0; i < 4; ++i) *(f32x4 *)(dst + (i >> 1) * half + (i & 1) * 4) = f32x4{raw[4 * i], raw[4 * i + 1], raw[4 * i + 2], raw[4 * i + 3]};
         }
     } else
-        for (int e = threadIdx.x * 4; e < CPL * 512; e += kRetrThreads * 4) *(f32x4 *)(qs + e) = e < C ? *(const f32x4 *)(qbar + e) : f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int e = threadIdx.x * 4; e < CPL * 512; e += kRetrThreads * 4) *(f32x4 *)(qs + e) = e < C ? *(const f32x4 *)(job.qbar + e) : f32x4{0.f, 0.f, 0.f, 0.f};
     __syncthreads();
     float q[CPL][8];
 #pragma unroll
@@ -678,22 +683,37 @@ __global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16
         }
         n += ROWS * n_waves;
     }
-    if constexpr (FRONT) return;
-    // every wave's score stores have been performed before the workgroup takes its ticket
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    unsigned int *const ticket = own_ticket ? own_ticket : &retrieval_tickets[ticket_slot];
-    if (threadIdx.x == 0) {
-        const unsigned int drawn = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        is_last = drawn == (unsigned int)n_wgs - 1;
+    if constexpr (!FRONT) {
+        __shared__ int is_last;
+        // every wave's score stores have been performed before the workgroup takes its ticket
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        unsigned int *const ticket = job.ticket ? job.ticket : &retrieval_tickets[job.slot];
+        if (threadIdx.x == 0) {
+            const unsigned int drawn = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+            is_last = drawn == (unsigned int)n_wgs - 1;
+        }
+        __syncthreads();
+        if (!is_last) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (N <= 16 * kRetrThreads) select_topk_block<1>(scores, N, job.k, job.idx, job.idx2);
+        else select_topk_block<2>(scores, N, job.k, job.idx, job.idx2);
+        publish(job.flag, job.flag_value);
     }
-    __syncthreads();
-    if (!is_last) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (N <= 16 * kRetrThreads) select_topk_block<1>(scores, N, k, idx_out, idx_out2);
-    else select_topk_block<2>(scores, N, k, idx_out, idx_out2);
-    publish(flag, flag_value);
+}
+
+// (The selection's arguments one by one: as a structure they are read where they are used, behind the scores, and the launch is 0.1 us
+// longer.)
+template <int CPL, int ROWS, bool TAIL>
+__global__ __launch_bounds__(kRetrThreads) void retrieve_fused_kernel(const bf16_t *reps, int64_t rep_stride, int N, int C, const float *qbar, float *scores,
+                                                                      int k, int32_t *idx, int32_t *idx2, int32_t *flag, int32_t flag_value,
+                                                                      uint32_t *ticket, int slot) {
+    score_rows<CPL, ROWS, TAIL>(reps, rep_stride, N, C, scores, Selection{qbar, k, idx, idx2, flag, flag_value, ticket, slot});
+}
+template <int CPL, int ROWS, bool TAIL>
+__global__ __launch_bounds__(kRetrThreads) void step_scores_kernel(const bf16_t *reps, int64_t rep_stride, int N, int C, float *scores, StepFront front) {
+    score_rows<CPL, ROWS, TAIL>(reps, rep_stride, N, C, scores, front);
 }
 
 // ---------------------------------------------------------------- representative keys
@@ -1127,13 +1147,14 @@ extern "C" int infllm_score_topk_queries(const void *d_reps, int64_t rep_stride,
 // library-internal: unit scores of all N units and the k best of them in ONE launch (retrieve_fused_kernel), the ids
 // leaving as infllm_topk_publish_pair leaves them.  Returns 1, with nothing launched, where that kernel does not apply
 // (rows of more than 4608 elements or not of whole 16-byte chunks, more than 16384 units, k > 64): the caller then launches the two steps.
-// ticket: the caller's word, or NULL and slot >= 0: the library's word there; neither: returns 1.
-static int retrieve_launch(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar, int32_t k, float *d_scores, int32_t *d_idx,
-                           int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, const StepFront *front, bool whole_front, uint32_t *ticket, int slot, void *stream) {
-    INFLLM_REQUIRE(d_reps && (d_qbar || front) && d_scores && (d_idx || front), "retrieve: null pointer");
-    INFLLM_REQUIRE(N > 0 && k > 0 && k <= N, "retrieve: k=%d with N=%d", k, N);
+// select (a word to count in of the caller, or slot >= 0: the library's there; neither: returns 1), or front: the scores of a step,
+// with its prologue if whole_front.
+static int retrieve_launch(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, float *d_scores, const Selection *select, const StepFront *front,
+                           bool whole_front, void *stream) {
+    INFLLM_REQUIRE(d_reps && d_scores && N > 0, "retrieve: null pointer or %d units", N);
+    INFLLM_REQUIRE(!select || (select->qbar && select->idx && select->k > 0 && select->k <= N), "retrieve: null pointer or k=%d with N=%d", select ? select->k : 0, N);
     INFLLM_REQUIRE(rep_stride >= C && rep_stride % 8 == 0, "retrieve: row stride %lld", (long long)rep_stride);
-    if (N > 16384 || k > 64 || C % 8 != 0 || C > 9 * 512 || (!front && !ticket && slot < 0)) return 1;
+    if (N > 16384 || C % 8 != 0 || C > 9 * 512 || (select && (select->k > 64 || (!select->ticket && select->slot < 0)))) return 1;
     constexpr int waves_per_wg = kRetrThreads / 64;
     const bool deep = N >= 4096;
     const int per_wg = waves_per_wg * (deep ? 2 : 1);
@@ -1154,13 +1175,14 @@ static int retrieve_launch(const void *d_reps, int64_t rep_stride, int32_t N, in
     }
 #define FUSED_CASE(c, tail)                                                                                                          \
     if (front) {                                                                                                                     \
-        auto kern = deep ? retrieve_fused_kernel<c, 2, tail, true> : retrieve_fused_kernel<c, 1, tail, true>;                        \
+        auto kern = deep ? step_scores_kernel<c, 2, tail> : step_scores_kernel<c, 1, tail>;                                          \
         hipLaunchKernelGGL(kern, dim3(wgs + extra), dim3(kRetrThreads), (size_t)c * 512 * sizeof(float), st, reps, rep_stride, N, C,  \
-                           d_qbar, d_scores, k, d_idx, d_idx2, d_flag, flag_value, ticket, slot, f);                                 \
+                           d_scores, f);                                                                                             \
     } else {                                                                                                                         \
         auto kern = deep ? retrieve_fused_kernel<c, 2, tail> : retrieve_fused_kernel<c, 1, tail>;                                    \
-        hipLaunchKernelGGL(kern, dim3(wgs), dim3(kRetrThreads), (size_t)c * 512 * sizeof(float), st, reps, rep_stride, N, C, d_qbar,  \
-                           d_scores, k, d_idx, d_idx2, d_flag, flag_value, ticket, slot, NoFront{});                         \
+        hipLaunchKernelGGL(kern, dim3(wgs), dim3(kRetrThreads), (size_t)c * 512 * sizeof(float), st, reps, rep_stride, N, C,          \
+                           select->qbar, d_scores, select->k, select->idx, select->idx2, select->flag, select->flag_value,           \
+                           select->ticket, select->slot);                                                                            \
     }
     if (C == 512) { FUSED_CASE(1, false) }
     else if (C == 1024) { FUSED_CASE(2, false) }
@@ -1176,7 +1198,8 @@ static int retrieve_launch(const void *d_reps, int64_t rep_stride, int32_t N, in
 
 int infllm_retrieve_fused(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar, int32_t k, float *d_scores,
                           int32_t *d_idx, int32_t *d_idx2, int32_t *d_flag, int32_t flag_value, uint32_t *d_ticket, void *stream) {
-    return retrieve_launch(d_reps, rep_stride, N, C, d_qbar, k, d_scores, d_idx, d_idx2, d_flag, flag_value, nullptr, false, d_ticket, -1, stream);
+    const Selection select{d_qbar, k, d_idx, d_idx2, d_flag, flag_value, d_ticket, -1};
+    return retrieve_launch(d_reps, rep_stride, N, C, d_scores, &select, nullptr, false, stream);
 }
 
 // library-internal: the scores alone, under the one query of a decode step, batch row b of `in` (whose d_qpart is not used); with
@@ -1194,7 +1217,7 @@ int infllm_step_scores(const void *d_reps, int64_t rep_stride, int32_t N, const 
     f.in = *in;
     f.dim = dim;
     f.b = b;
-    return retrieve_launch(d_reps, rep_stride, N, in->H * dim, nullptr, 1, d_scores, nullptr, nullptr, nullptr, 0, &f, prologue, nullptr, -1, stream);
+    return retrieve_launch(d_reps, rep_stride, N, in->H * dim, d_scores, nullptr, &f, prologue, stream);
 }
 
 extern "C" int infllm_score_topk(const void *d_reps, int64_t rep_stride, int32_t N, int32_t C, const float *d_qbar,
@@ -1202,8 +1225,8 @@ extern "C" int infllm_score_topk(const void *d_reps, int64_t rep_stride, int32_t
     INFLLM_REQUIRE(N > 0 && k >= 0 && k <= N, "score_topk: k=%d with N=%d", k, N);
     if (k > 0) {
         INFLLM_REQUIRE(d_idx, "score_topk: null index pointer");
-        const int frc = retrieve_launch(d_reps, rep_stride, N, C, d_qbar, k, d_scores, d_idx, nullptr, nullptr, 0, nullptr, false, nullptr,
-                                        ticket_slot((hipStream_t)stream), stream);
+        const Selection select{d_qbar, k, d_idx, nullptr, nullptr, 0, nullptr, ticket_slot((hipStream_t)stream)};
+        const int frc = retrieve_launch(d_reps, rep_stride, N, C, d_scores, &select, nullptr, false, stream);
         if (frc != 1) return frc;
     }
     int rc = infllm_unit_scores(d_reps, rep_stride, 0, N, C, d_qbar, d_scores, stream);

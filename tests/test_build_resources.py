@@ -11,7 +11,7 @@ import subprocess
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-HOT = ("attn_stage_kernel", "local_score_kernel", "retrieve_fused_kernel", "unit_scores_rows_kernel", "unit_scores_queries_kernel",
+HOT = ("attn_stage_kernel", "local_score_kernel", "retrieve_fused_kernel", "step_scores_kernel", "unit_scores_rows_kernel", "unit_scores_queries_kernel",
        "call_rank_kernel", "ingest_kernel", "block_end_kernel", "scores_kernel", "decode_attn_kernel", "stage_rows_kernel", "rank_kernel", "decode_finish_kernel",
        "attn_merge")
 
