@@ -227,7 +227,7 @@ def kernels_hbm_leg(dev):
         ops.attn_fwd(la, ga, o, lse)
     us = _event_time_us(decode_attn, 200, 2 * sets)
     nbytes = (n_local + 1 + n_glob) * HKV * D * 2 * 2
-    out.append(_hbm_entry("attn_stage_kernel<0> + <1> + attn_merge_wide_kernel", f"decode-shaped attention: 1 query x {H} heads over {n_local + 1} window keys "
+    out.append(_hbm_entry("decode_attn_kernel + attn_stage_kernel<128, 1, false> + attn_merge_wide_kernel", f"decode-shaped attention: 1 query x {H} heads over {n_local + 1} window keys "
                           f"({ns_l} key splits) and {n_glob} retrieved keys ({ns_g} splits), K and V read once, three launches; "
                           f"{sets} K/V sets in rotation", nbytes, us, 200,
                           traffic=counted_traffic("retrieval__decode8192.hbm_bytes.txt", "decode_attention_traffic_bytes")))
@@ -312,7 +312,7 @@ def decode_workload(args, dev):
                                f"max_cached {KNOBS['max_cached_block']}"},
         "roofline": {"bound": "hbm", "achieved": gbs, "peak": 8000.0, "unit": "GB/s", "frac": gbs / 8000.0,
                      "traffic": counted_traffic("retrieval__decode8192.hbm_bytes.txt", "unit_scores_traffic_bytes"),
-                     "kernel": f"unit_scores_kernel ({N} x {H * D} bf16 representatives, {N * H * D * 2 / 2 ** 20:.1f} MiB per retrieval)",
+                     "kernel": f"unit_scores_rows_kernel ({N} x {H * D} bf16 representatives, {N * H * D * 2 / 2 ** 20:.1f} MiB per retrieval)",
                      "avg_launch_ms": ms},
         "cache": cm.stats}))
 
@@ -572,7 +572,7 @@ def main():
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / MFMA_BF16_PEAK_TFLOPS,
                      "traffic": counted_traffic("attn_stage__stream32k.hbm_bytes.txt", "local_stage_traffic_bytes"),
-                     "kernel": f"attn_stage_kernel<0, false> (local stage, {q_launch} q x {n_local} visible keys x {H} heads per launch)",
+                     "kernel": f"attn_stage_kernel<128, 0, false> (local stage, {q_launch} q x {n_local} visible keys x {H} heads per launch)",
                      "avg_launch_ms": avg_ms, "launches_timed": len(steady),
                      "global_stage_avg_ms": sum(glob) / max(len(glob), 1)},
         "cache": cm_stats,
