@@ -1,4 +1,4 @@
-"""A decode step whose prologue rides with its retrieval: rows of representatives of every length class the retrieval has, heads of 64
+"""A decode step whose prologue rides with its scores: rows of representatives of every length class these have, heads of 64
 and 128, one to twelve heads a group, several batch rows, and rows too long for it - rings, books and state bit for bit those of
 the host-driven path, whose prologue is a launch of its own; outputs within the difference of the key splits."""
 import pytest
