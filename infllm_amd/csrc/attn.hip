@@ -36,6 +36,11 @@ constexpr int kThreads = kWaves * kWave;
 constexpr int kQTile = 32;                 // queries per wave
 constexpr int kBig = 1 << 29;              // clamp for mask distances held in int32
 
+// a wave-uniform distance clamped to int32, in scalar instructions (there is no scalar 64-bit comparison but for equality)
+__device__ __forceinline__ int clamp_big(int64_t x) {
+    return (uint64_t)(x + kBig) >> 30 == 0 ? (int)x : (int)(x >> 32) < 0 ? -kBig : kBig;
+}
+
 struct StageRange {
     int64_t lo, hi;   // key index range [lo, hi) visible to a span of queries
 };
@@ -86,6 +91,7 @@ struct StageGeom {
     // row [b, h, i] at b * o_sb + h * o_sh + i * o_sl; no partial rows, no merge.
     bf16_t *out;
     int64_t o_sb, o_sh, o_sl;
+    float scale;                            // what makes a logit of a product of rows, to base 2
 };
 
 // LDS layouts.  Tiles go from global memory straight into LDS (global_load_lds_dwordx4: lane l of a
@@ -148,11 +154,18 @@ struct KernargLayout {                     // the arguments as the launch lays t
 template <int D, int MODE>
 constexpr int kWgsPerCu = D == 64 && (MODE == kLinear || MODE == kPaged) ? 2 : 1;
 
-template <int D, int MODE, bool INLINE = false>
+// BASE2: the queries come with the softmax scale and log2(e) in them (types with a window, heads of 128), multiplied in where they are
+// rotated, ahead of their one rounding to bf16: their products with keys are logits to base 2.  The linear form starts the products
+// from less the running max (kFromMax), and a probability is an exponential and nothing else: the multiply-add that every score took
+// went into the power of the card, which lowers its clock under this loop.  The sinks' form has no registers for the 16 that hold the
+// max and adds it.  Causal prompt of 8,001 tokens, 32 / 8 heads: 533 -> 521.5 us, sinks + window of 4,096 over 16,001 1,037.5 -> 1,026.5.
+// (The streaming memory's queries stay as they are: 128K tokens 1.5 % faster so, 24,300 of 36 heads of 64 0.5 %.)
+template <int D, int MODE, bool INLINE = false, bool BASE2 = false>
 __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage_kernel(infllm_attn_args a, infllm_attn_args a2, StageGeom geo,
                                                                  std::conditional_t<INLINE, InlinePages, NoInlinePages>) {
     constexpr bool HAS_LIN = MODE != kPaged, HAS_PAG = MODE != kLinear, SINKS = MODE == kSinks || MODE == kSinksStaged, TWO = MODE == kBoth || SINKS;
     constexpr int kRow = D * 2, kTB = kTileBytes<D>;                     // bytes of a row, of a tile
+    constexpr bool kFromMax = BASE2 && D == 128 && !TWO;
     constexpr bool PING = D == 128, kTurns = D == 128 && (MODE == kLinear || MODE == kSinks);
     const infllm_attn_args &ap = TWO ? a2 : a;                 // the paged stage's arguments
     extern __shared__ __attribute__((aligned(1024))) char lds_dyn[];    // kStages K tiles, then kStages V tiles
@@ -285,7 +298,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         const int slot = first - (int)(fdiv(first, geo.cap_tiles) * geo.cap_tiles.d);
         k_next = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + ((int64_t)slot * kTile + wave_rk) * a.k_sl;
         v_next = (const bf16_t *)a.d_v + (int64_t)b * a.v_sb + (int64_t)g * a.v_sh + ((int64_t)slot * kTile + wave_rv) * a.v_sl;
-        to_wrap = (int)min((int64_t)INT32_MAX, (int64_t)geo.cap_tiles.d - slot);
+        to_wrap = (int)min((uint32_t)INT32_MAX, geo.cap_tiles.d - (uint32_t)slot);
     }
     // linear tiles whose 64 rows are all in the source: list indices [whole_lo, whole_hi)
     const int whole_lo = HAS_LIN ? floordiv64(a.j_lo + kTile - 1) - lin_t0 : 0, whole_hi = HAS_LIN ? floordiv64(a.j_hi) - lin_t0 : 0;
@@ -358,15 +371,18 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
                 row_lo = (int)max((int64_t)0, a.j_lo - j0);
                 row_hi = (int)min((int64_t)kTile, a.j_hi - j0);
             }
+            int ln = lane;
+            uint32_t nil = 0;
+            asm volatile("" : "+v"(ln), "+v"(nil));    // (places made here and not ahead of all tiles: registers are short)
             char *kz = Ks + at + wave * (kLd * 1024), *vz = Vs + at + wave * (kLd * 1024);
 #pragma unroll
             for (int i = 0; i < kLd; ++i) {
                 // rows outside the source are written as zeros: their keys are masked, but 0 * stale must stay 0
-                const int rv = tile_row(i), rk = k_lds_row(rv);
+                const int rv = kRowsPerLd * (kLd * wave + i) + ln / (D / 8), rk = k_lds_row(rv);
                 if (rk >= row_lo && rk < row_hi) load_to_lds16(kbase, k_src[i], kdst + i * 1024);
-                else *(u32x4 *)(kz + i * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+                else *(u32x4 *)(kz + i * 1024 + ln * 16) = u32x4{nil, nil, nil, nil};
                 if (rv >= row_lo && rv < row_hi) load_to_lds16(vbase, v_src[i], vdst + i * 1024);
-                else *(u32x4 *)(vz + i * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+                else *(u32x4 *)(vz + i * 1024 + ln * 16) = u32x4{nil, nil, nil, nil};
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
@@ -375,14 +391,16 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
 
     // ---- running softmax state of this lane's query (max kept in raw logit units, allowed to lag)
     float m_run = -INFINITY, m_limit = -INFINITY, l_run = 0.f, neg_ms = 0.f;
+    [[maybe_unused]] f32x16 from_max;         // kFromMax: what scores are taken from, 16 times less the max; 0 as long as there is none
+#pragma unroll
+    for (int r = 0; r < 16; ++r) from_max[r] = 0.f;
     f32x16 oacc[D / 32];
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
 
-    const float scale = a.softmax_scale * 1.4426950408889634f;
-    const float lazy = kLazyLog2 / scale;
+    const float scale = BASE2 ? 1.f : geo.scale, lazy = kLazyLog2 / scale;
     typedef short s16x8 __attribute__((ext_vector_type(8)));
     // kb / vb: k_off / v_off in the tile's buffer
     auto k_operand = [&](uint32_t kb, int kk, int ks) {
@@ -400,7 +418,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     int clear_lo = whole_lo, clear_hi = whole_hi, clear_pag = 0;
     if (HAS_LIN) {
         const int64_t q0 = (int64_t)i0 + a.offset, q1 = (int64_t)i1 + a.offset;
-        auto tile_of = [&](int64_t j) { return (int)min(max(j >> 6, (int64_t)-kBig), (int64_t)kBig); };
+        auto tile_of = [&](int64_t j) { return clamp_big(j >> 6); };
         if (a.mask == INFLLM_MASK_WINDOW) {            // every key at a distance of 0 or more from the first query, below the window from the last
             clear_lo = max(clear_lo, tile_of(q1 - a.window) + 1 - lin_t0);
             clear_hi = min(clear_hi, tile_of(q0 - (kTile - 1)) + 1 - lin_t0);
@@ -413,24 +431,28 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     auto mask = [&](f32x16 (&s)[2], int t, [[maybe_unused]] int valid) {
         const bool paged = MODE == kPaged || (TWO && t >= n_lin);
         if (!(PAGES && paged ? valid == kTile : TWO && paged ? t < clear_pag : t >= clear_lo && t < clear_hi)) {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));
+            const int col = ln & 31, grp = ln >> 5;
             int row_lo = 0, row_hi = kTile;
             int d0 = 0;                        // dist of (this lane's query, key 0 of the tile), clamped into int32
             if (SINKS && paged) {
                 const int64_t j0 = (int64_t)(t - n_lin) * kTile, e0 = (int64_t)i0 + ap.offset - j0;
                 row_hi = (int)min((int64_t)kTile, ap.j_hi - j0);
-                d0 = (int)min(max(e0, (int64_t)-kBig), (int64_t)kBig) + col;
+                d0 = clamp_big(e0) + col;
             } else if (paged) {
                 row_hi = valid;
             } else {
                 const int64_t j0 = (int64_t)(lin_t0 + t) * kTile, e0 = (int64_t)i0 + a.offset - j0;
                 row_lo = (int)max((int64_t)0, a.j_lo - j0);
                 row_hi = (int)min((int64_t)kTile, a.j_hi - j0);
-                d0 = (int)min(max(e0, (int64_t)-kBig), (int64_t)kBig) + col;
+                d0 = clamp_big(e0) + col;
             }
             // Whatever the mask, a lane's query sees ONE run of the tile's keys: its bounds are found once, and a key costs a
             // subtraction and a compare (a mask's conditions key by key: 150 branches in the sinks' form of the kernel).
             // dist = dl - kc; kc is the compile-time part of register r's key, which is kc + 8 * grp
-            const int win = (int)min(SINKS && paged ? ap.window : a.window, (int64_t)2 * kBig), dl = d0 - 8 * grp;
+            const int64_t win64 = SINKS && paged ? ap.window : a.window;
+            const int win = (int)(win64 >> 32) >= 0 && (uint64_t)win64 >> 30 != 0 ? 2 * kBig : (int)win64, dl = d0 - 8 * grp;
             int lo_l = row_lo - 8 * grp, hi_l = row_hi - 8 * grp;
             if (SINKS && paged) {
                 hi_l = min(hi_l, dl - win + 1);
@@ -455,8 +477,9 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     // against ones it receives the sum of its own four values: 8 cycles of the matrix pipe for 4 keys.  (As one more 32 x
     // 32 x 16 product per step, 128 cycles a tile instead of 64, prompts of 131,072 tokens 26,020 -> 25,495 us, the operator over
     // 512 x (4,608 + 2,624) 102.7 -> 101.3; as 64 shifts and additions 220 cycles of the vector half.)
-    s16x4 ones{0x3f80, 0x3f80, 0x3f80, 0x3f80};
-    asm volatile("" : "+v"(ones));
+    uint32_t one_one;
+    asm volatile("v_mov_b32 %0, 0x3f803f80" : "=v"(one_one));
+    const s16x4 ones = __builtin_bit_cast(s16x4, u32x2{one_one, one_one});
     auto add_row_sums = [&](u32x4 p, f32x4 sums) {
         sums = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(s16x4, u32x2{p[0], p[1]}), sums, 0, 0, 0);
         return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(s16x4, u32x2{p[2], p[3]}), sums, 0, 0, 0);
@@ -473,7 +496,20 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         // lazy running max: it only moves when a score would exceed it by more than 2^kLazyLog2 after scaling,
         // so the rescale of the output accumulators is rare; probabilities stay below 2^kLazyLog2
         const bool moved = tmax > m_limit;
-        if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+        if constexpr (kFromMax) {                // (scores are less the max already)
+            if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+                const float by = moved ? tmax : 0.f;
+                const float al = !moved ? 1.f : m_limit == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(-by);
+                m_limit = moved ? kLazyLog2 : m_limit;
+                l_run *= al;
+#pragma unroll
+                for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) oacc[dt][r] *= al;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) from_max[r] -= by, s[0][r] -= by, s[1][r] -= by;
+            }
+        } else if (__builtin_amdgcn_ballot_w64(moved) != 0) {
             const float m_new = moved ? tmax : m_run;
             const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale);      // exp2(-inf) = 0 on the first move
             const float al = moved ? alpha : 1.f;
@@ -660,8 +696,8 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     auto exps = [&](int ks, int r0, int r1) {
 #pragma unroll
         for (int r = r0; r < r1; r += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[ks][r], scale, neg_ms));
-            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[ks][r + 1], scale, neg_ms));
+            const float p0 = __builtin_amdgcn_exp2f(kFromMax ? s[ks][r] : __builtin_fmaf(s[ks][r], scale, neg_ms));
+            const float p1 = __builtin_amdgcn_exp2f(kFromMax ? s[ks][r + 1] : __builtin_fmaf(s[ks][r + 1], scale, neg_ms));
             pw[ks][r >> 1] = pack_bf16x2(p0, p1);
             asm volatile("" : "+v"(pw[ks][r >> 1]));                                // formed here, not where it is read
         }
@@ -694,17 +730,19 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
     };
     // S = K.Q of this tile; its first 8 operands are on their way
     auto qk_mul = [&](uint32_t kb) {
+        if constexpr (!kFromMax)
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
+            for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[ks][r] = 0.f;
+                for (int r = 0; r < 16; ++r) s[ks][r] = 0.f;
 #pragma unroll
         for (int g = 4; g < 8; ++g) {
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int i = 4 * g + j;
-                s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, op[i & 7]), qreg[((i - 16) >> 1) % (D / 16)], s[i & 1], 0, 0, 0);
+                s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, op[i & 7]), qreg[((i - 16) >> 1) % (D / 16)],
+                                                                   kFromMax && i < 18 ? from_max : s[i & 1], 0, 0, 0);
                 if (i + 8 < 32) request(i + 8, 0, kb);
             }
             if (g < 6) {
@@ -963,7 +1001,7 @@ __global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage
         }
     }
     if (qi >= a.Lq) return;
-    if (grp == 0) a.d_lse_part[row] = l_tot > 0.f ? m_run * scale + log2f(l_tot) : -INFINITY;
+    if (grp == 0) a.d_lse_part[row] = l_tot > 0.f ? (kFromMax ? -from_max[0] : m_run * scale) + log2f(l_tot) : -INFINITY;
 }
 
 // one thread per (row, 8 dims): P fp16 partials -> bf16 output row + final lse (merge_piece, common.h)
@@ -1130,16 +1168,16 @@ struct StageOut {
     const float2 *q_angles = nullptr, *sink_angle = nullptr;
 };
 
-template <int D, int MODE, bool INLINE, typename Pages>
+template <int D, int MODE, bool INLINE, bool BASE2, typename Pages>
 int launch_mode(dim3 grid, const infllm_attn_args &a, const infllm_attn_args &a2, const StageGeom &geo, const Pages &pages, void *stream) {
     constexpr size_t lds_bytes = 2 * kStages * kTileBytes<D>;
     static std::atomic<bool> lds_set{false};                  // dynamic LDS above 64 KiB must be enabled once per kernel
     if (!lds_set.load(std::memory_order_acquire)) {
-        const hipError_t e = hipFuncSetAttribute((const void *)attn_stage_kernel<D, MODE, INLINE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+        const hipError_t e = hipFuncSetAttribute((const void *)attn_stage_kernel<D, MODE, INLINE, BASE2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
         if (e != hipSuccess) return infllm_fail(-2, "attn_stage: %s", hipGetErrorString(e));
         lds_set.store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL((attn_stage_kernel<D, MODE, INLINE>), grid, dim3(kThreads), lds_bytes, (hipStream_t)stream, a, a2, geo, pages);
+    hipLaunchKernelGGL((attn_stage_kernel<D, MODE, INLINE, BASE2>), grid, dim3(kThreads), lds_bytes, (hipStream_t)stream, a, a2, geo, pages);
     INFLLM_CHECK_LAUNCH("attn_stage");
     return 0;
 }
@@ -1156,25 +1194,30 @@ int launch_stage(int mode, const infllm_attn_args *a, const infllm_attn_args *a2
     INFLLM_REQUIRE((int64_t)grid.x * grid.y * grid.z < (1ll << 31), "attn_stage: grid too large");
     StageGeom geo{so.q_angles, so.sink_angle, fast_div(grid.x), fast_div(grid.y), fast_div((uint32_t)a->Hkv), fast_div((uint32_t)G),
                   fast_div((uint32_t)a->nsplit), fast_div(1), n_tasks, so.out_exc, so.out_block_rows,
-                  fast_div((uint32_t)(so.out_exc > 0 ? so.out_exc : 1)), so.out, so.o_sb, so.o_sh, so.o_sl};
+                  fast_div((uint32_t)(so.out_exc > 0 ? so.out_exc : 1)), so.out, so.o_sb, so.o_sh, so.o_sl, a->softmax_scale * kLog2e};
     // tile indices stay below 2^30, so any ring of 2^31 tiles or more never wraps: one divisor stands for all of them
     if (mode != kPaged) geo.cap_tiles = fast_div((uint32_t)std::min<int64_t>(a->cap / kTile, 1ll << 31));
     const infllm_attn_args &second = a2 ? *a2 : *a;
+    const bool base2 = geo.scale == 1.f;
     if (h_pages) {
         const infllm_attn_args &pg = mode == kBoth ? second : *a;
         INFLLM_REQUIRE((mode == kPaged || mode == kBoth) && pg.n_pages >= 0 && (int64_t)pg.B * pg.n_pages <= kInlinePages,
                        "attn_stage: %d x %d pages do not fit a launch", pg.B, pg.n_pages);
         InlinePages table;
         memcpy(table.p, h_pages, sizeof(infllm_page) * pg.B * pg.n_pages);
-        return mode == kPaged ? launch_mode<D, kPaged, true>(grid, *a, second, geo, table, stream)
-                              : launch_mode<D, kBoth, true>(grid, *a, second, geo, table, stream);
+        if (mode == kBoth) return launch_mode<D, kBoth, true, false>(grid, *a, second, geo, table, stream);
+        return launch_mode<D, kPaged, true, false>(grid, *a, second, geo, table, stream);
     }
+    constexpr NoInlinePages none{};
+    constexpr bool kForms = D == 128;                // (of heads of 64 the types with a window scale their scores too)
+    INFLLM_REQUIRE(!kForms || base2 || (mode != kSinks && mode != kSinksStaged), "attn_stage: sinks of queries without the softmax scale");
     switch (mode) {
-        case kLinear: return launch_mode<D, kLinear, false>(grid, *a, second, geo, NoInlinePages{}, stream);
-        case kPaged: return launch_mode<D, kPaged, false>(grid, *a, second, geo, NoInlinePages{}, stream);
-        case kBoth: return launch_mode<D, kBoth, false>(grid, *a, second, geo, NoInlinePages{}, stream);
-        case kSinks: return launch_mode<D, kSinks, false>(grid, *a, second, geo, NoInlinePages{}, stream);
-        default: return launch_mode<D, kSinksStaged, false>(grid, *a, second, geo, NoInlinePages{}, stream);
+        case kLinear: return kForms && base2 ? launch_mode<D, kLinear, false, kForms>(grid, *a, second, geo, none, stream)
+                                             : launch_mode<D, kLinear, false, false>(grid, *a, second, geo, none, stream);
+        case kPaged: return launch_mode<D, kPaged, false, false>(grid, *a, second, geo, none, stream);
+        case kBoth: return launch_mode<D, kBoth, false, false>(grid, *a, second, geo, none, stream);
+        case kSinks: return launch_mode<D, kSinks, false, kForms>(grid, *a, second, geo, none, stream);
+        default: return launch_mode<D, kSinksStaged, false, kForms>(grid, *a, second, geo, none, stream);
     }
 }
 
