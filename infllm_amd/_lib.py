@@ -243,10 +243,24 @@ SYMBOLS = {
 }
 
 _lib = None
+_host = None
 
 
 class InfLLMHipError(RuntimeError):
     pass
+
+
+def host():
+    """The extension module of csrc/host.cpp: the host side of a step of the attention types with a plain cache."""
+    global _host
+    if _host is None:
+        import torch  # noqa: F401  (whose libraries the module is linked against)
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise InfLLMHipError(f"infllm_amd/_host.so cannot be loaded ({e}): build it with `python -m infllm_amd.build`") from e
+        _host = module
+    return _host
 
 
 def load():
@@ -270,6 +284,7 @@ def load():
         fn.restype, fn.argtypes = restype, argtypes
     if lib.infllm_version() != ABI_VERSION:
         raise InfLLMHipError(f"ABI version {lib.infllm_version()} != expected {ABI_VERSION}; rebuild the library")
+    host().bind(lib.infllm_window_forward, C.cast(lib.infllm_window_forward, c_vp).value)
     _lib = lib
     return lib
 

@@ -1,18 +1,20 @@
-"""Build libinfllm_hip.so (gfx950) in-tree with hipcc.
+"""Build libinfllm_hip.so (gfx950) with hipcc and the extension module _host.so with the host compiler, in-tree.
 
     python -m infllm_amd.build
 
-The library is cross-compiled (no GPU needed) and placed next to this file so
-that it travels with the source tree.
+The library is cross-compiled (no GPU needed).  Both are placed next to this file so
+that they travel with the source tree.
 """
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libinfllm_hip.so")
+HOST_PATH = os.path.join(HERE, "_host.so")
 SOURCES = ["abi.hip", "ingest.hip", "attn.hip", "score.hip", "retrieve.hip", "decode.hip", "window.hip", "cache.hip", "stream.hip", "resident.hip"]
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -28,10 +30,7 @@ def hipcc_path():
     raise RuntimeError("hipcc not found (set HIPCC or install ROCm)")
 
 
-def build(verbose=True, extra_flags=()):
-    # ROCr (libhsa-runtime64) is linked for the DMA-engine copy of carved units; in a process it is the copy the HIP
-    # runtime already loaded
-    cmd = [hipcc_path(), *HIPCC_FLAGS, *extra_flags, *[os.path.join(CSRC, s) for s in SOURCES], "-o", LIB_PATH, "-lhsa-runtime64"]
+def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     proc = subprocess.run(cmd, capture_output=True, text=True)
@@ -39,9 +38,31 @@ def build(verbose=True, extra_flags=()):
     noise = "is not a recognized feature for this target"
     err = "\n".join(l for l in proc.stderr.splitlines() if noise not in l)
     if proc.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + err)
+        raise RuntimeError(f"{os.path.basename(cmd[0])} failed:\n" + err)
     if verbose and err.strip():
         print(err, file=sys.stderr)
+
+
+def build_host(verbose=True):
+    """csrc/host.cpp against the installed torch.  (Its libraries are in the process when the module is imported: no path to them.)"""
+    import torch
+    from torch.utils import cpp_extension
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("no C++ compiler found (set CXX)")
+    include = [sysconfig.get_paths()["include"], *cpp_extension.include_paths()]
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-I{p}" for p in include],
+          os.path.join(CSRC, "host.cpp"), "-o", HOST_PATH, *[f"-L{p}" for p in cpp_extension.library_paths()], "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"],
+         verbose)
+    return HOST_PATH
+
+
+def build(verbose=True, extra_flags=()):
+    # ROCr (libhsa-runtime64) is linked for the DMA-engine copy of carved units; in a process it is the copy the HIP
+    # runtime already loaded
+    cmd = [hipcc_path(), *HIPCC_FLAGS, *extra_flags, *[os.path.join(CSRC, s) for s in SOURCES], "-o", LIB_PATH, "-lhsa-runtime64"]
+    _run(cmd, verbose)
+    build_host(verbose)
     return LIB_PATH
 
 
