@@ -54,14 +54,13 @@ struct RowCopy {
     int32_t n;
 };
 constexpr int kCopies = 7;
-// Rows that a copying workgroup of 256 threads moves, and beside the splits of a step, which waits for the last of them: splits of
-// heads of 128 leave it a third of the chip, so few and long ones; those of heads of 64 leave it most.  (infinite-lm, one token over
-// 9,000, window of 4,096, 8 key heads of 128: 64 rows 22.9 us, 256 rows 21.0; stream-llm over 6,000, 36 heads of 64: 24.4, 27.4.)
+// Rows that a copying workgroup moves: of a staging launch (256 threads), and beside the splits of a step (512), which waits for the last of
+// them, where few and long ones find room.  (One token over a full window, 64 / 128 / 256 rows: 72 heads of 64, window of 2,048, 28.6 / 23.1 /
+// 21.7 us; heads of 128 with workgroups of 256, window of 4,096: 64 rows 22.9, 256 rows 21.0.)
 constexpr int kCopyRows = 64;
-template <int D>
-constexpr int kStepCopyRows = D == 128 ? 256 : 64;
+constexpr int kStepCopyRows = 256;
 
-template <int D, int kRows>
+template <int D, int kRows, int THREADS = 256>
 __device__ __forceinline__ void copy_rows(const RowCopy (&copies)[kCopies], int piece, int b, int g) {
     const int tid = threadIdx.x;
     int c = 0;
@@ -75,13 +74,13 @@ __device__ __forceinline__ void copy_rows(const RowCopy (&copies)[kCopies], int 
     const int r0 = piece * kRows, m = min(kRows, rc.n - r0) * (D / 8);
     const u32x4 *src = (const u32x4 *)(rc.src + (int64_t)b * rc.s_sb + (int64_t)g * rc.s_sh + (int64_t)r0 * D);
     u32x4 *dst = (u32x4 *)(rc.dst + (int64_t)b * rc.d_sb + (int64_t)g * rc.d_sh + (int64_t)r0 * D);
-    constexpr int U = kRows * (D / 8) / 256;
+    constexpr int U = kRows * (D / 8) / THREADS;
     u32x4 x[U];
 #pragma unroll
-    for (int i = 0; i < U; ++i) x[i] = src[min(tid + 256 * i, m - 1)];              // (every one loaded: conditions here made the compiler spill)
+    for (int i = 0; i < U; ++i) x[i] = src[min(tid + THREADS * i, m - 1)];              // (every one loaded: conditions here made the compiler spill)
 #pragma unroll
     for (int i = 0; i < U; ++i)
-        if (tid + 256 * i < m) dst[tid + 256 * i] = x[i];
+        if (tid + THREADS * i < m) dst[tid + THREADS * i] = x[i];
 }
 
 // The rows of the step itself, as they come (DecodeJob's ranges are the rows that were there before, its q is not used): the
@@ -103,7 +102,7 @@ struct StepRows : StepQkv {
 };
 
 int infllm_decode_step(const DecodeJob *job, const StepRows *rows, int32_t dim, void *stream);
-int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int64_t blocks, int32_t max_splits);
+int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int32_t dim, int64_t blocks, int32_t max_splits, int64_t others = 0);
 int infllm_decode_memory_step(const DecodeJob *job, const infllm_ingest_args *in, int32_t dim, void *stream);
 int infllm_decode_attn(const DecodeJob *job, int32_t dim, void *stream);
 int infllm_decode_lead_splits(int32_t nsplit, int64_t lead_blocks, int64_t blocks);

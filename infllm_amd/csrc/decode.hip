@@ -24,7 +24,7 @@
 
 namespace {
 
-constexpr int kDecWaves = 4;
+constexpr int kDecWaves = 8;                       // (see decode_attn_kernel)
 constexpr float kLazyDec = 8.f;                    // the running maximum may lag the true one by 2^8
 
 template <int N>
@@ -84,44 +84,69 @@ __device__ __forceinline__ void leave_rows(const StepRows &f, int b, int g, floa
 // 11.8 + 14.6.  The window attended in the launch of the scores instead, beside the selection there: 18.5 + 9.8 and 25.7 + 9.6.)
 //
 // A split is a few microseconds of rows between a start and an end that are as long, so both are kept short.  What the host can divide it
-// divides (DecodePlan), and a workgroup finds its block in two trips to the arguments, not in some for every range.  At the end a wave
-// joins its four row groups by itself, and the waves' sums, each scaled to its wave's maximum, are read behind one barrier.  (The ranges walked
-// by every wave, the maxima of all 16 row groups read by all of them behind a barrier of their own: one token behind 64K / 512K
-// tokens 25.0 / 31.3 us a pass, 24.3 / 29.4 now, causal over 32,768 31.5 and 30.8.)
+// divides (DecodePlan), and a workgroup finds its block in two trips to the arguments (at_once).  At the end a wave adds up its four row
+// groups by itself, and the waves' sums, each scaled to its wave's maximum, are read behind one barrier.
+// Eight waves a workgroup, and a workgroup a CU: as many rows in flight as with two of four waves, for half the rotations and half the
+// partial rows.  The split that ends last reads those of its heads, which is the work of one CU: 64 KB with 64 splits, and with two trips for
+// them and a round of its L2's lines given up first (a fence; now what is read is asked for past that cache) 6 us of a step behind
+// 9,000 tokens, of which 3 are left: 1.3 until the rows are asked for, 0.4 until they are there.  The step's own key is a block of the list
+// like the others (as one more of the last wave it came behind a whole block's microsecond of every other wave).  One pass, 32 / 8 heads of
+// 128, four waves and this: causal behind 9,000 tokens 17.8 and 13.8 us, behind 32,768 30.0 and 28.1, stream-llm with its window of 4,096
+// 18.1 and 12.8, 4 batch rows and a window of 2,048 23.7 and 20.1; 36 heads of 64 behind 2,000 / 16,000 tokens 14.5 / 38.1, now 12.0 / 29.2, 4 batch
+// rows of 8,000 68.5 and 52.9; the streaming memory behind 512K tokens 26.4 and 24.8 (behind less the host bounds it).
 struct DecodePlan {
     int32_t G, chunks;                     // query heads of a kv head; workgroups that share them
+    int32_t blocks;                        // of all ranges
     int32_t end[kDecodeSegs];              // blocks of the ranges up to this one's last; behind the last range: INT32_MAX
 };
+// The arguments that lead to a workgroup's first loads, in ONE trip to them: the compiler fetched each where it was first used, which were
+// nine trips behind one another.  A word of every line that holds the ranges comes along, so that the range found is a trip to the cache.
+__device__ __forceinline__ void at_once(const DecodeJob &j, int &G, int &chunks, int &B, int &n_split, int (&ends)[kDecodeSegs - 1], StepQkv &r) {
+    static_assert(kDecodeSegs == 6 && sizeof(DecodeSeg) == 80);
+    const int near[7] = {(int)j.seg[0].k_sb, j.seg[0].n_ids, j.seg[1].n_ids, j.seg[2].n_ids, j.seg[3].n_ids, j.seg[4].n_ids, j.seg[5].n_ids};
+    asm volatile("" : "+s"(G), "+s"(chunks), "+s"(B), "+s"(n_split), "+s"(ends[0]), "+s"(ends[1]), "+s"(ends[2]), "+s"(ends[3]), "+s"(ends[4]),
+                      "+s"(r.q), "+s"(r.k), "+s"(r.v), "+s"(r.q_sb)
+                    : "s"(r.inv_freq), "s"(r.q_sh), "s"(r.k_sb), "s"(r.k_sh), "s"(r.v_sb), "s"(r.v_sh), "s"(near[0]), "s"(near[1]), "s"(near[2]), "s"(near[3]),
+                      "s"(near[4]), "s"(near[5]), "s"(near[6]));
+}
 template <int D, int NG, bool LOGITS, bool JOIN, typename Front = NoFront, bool SELECT = false>
-__global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(DecodeJob j, DecodePlan plan, Front f) {
+__global__ __launch_bounds__(kDecWaves * kWave, 2) void decode_attn_kernel(DecodeJob j, DecodePlan plan, Front f) {
     constexpr bool FRONT = !std::is_same_v<Front, NoFront>;
+    constexpr bool UNITS = !std::is_same_v<Front, StepRows>;
+    constexpr int NEW = FRONT;                     // the step's own key: a block behind the last
     constexpr int KK = D / 32;                     // k-steps of the first MFMA
     constexpr int LPR = D / 8;                     // lanes that hold a value row, 16 bytes each
     constexpr int VL = kDecodeBlock * LPR / 64;    // value loads per block: 4 (D = 128) or 2 (D = 64)
-    constexpr int GRP = 64 / LPR;                  // value rows of one load: one (D = 128) or two (D = 64) per row group
-    constexpr int kJoin = 10;                      // words of a lane in the join of the splits
-    constexpr int kRed = kDecWaves * GRP * NG * D;
-    __shared__ __attribute__((aligned(16))) float red_room[!JOIN || kRed > kDecWaves * kWave * kJoin ? kRed : kDecWaves * kWave * kJoin];
-    float(*red)[GRP][NG][D] = (float(*)[GRP][NG][D])red_room;
+    constexpr int kRed = kDecWaves * NG * D, kSel = SELECT ? (int)sizeof(SelectLds<kDecWaves * kWave>) / 4 : 0;
+    __shared__ __attribute__((aligned(16))) float red_room[kRed > kSel ? kRed : kSel];
+    float(*red)[NG][D] = (float(*)[NG][D])red_room;
     __shared__ float sm[kDecWaves][NG], sl[kDecWaves][NG];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int col = lane & 15, rg = lane >> 4;
-    const int G = plan.G, split = blockIdx.x, b = blockIdx.z, n_split = gridDim.x;
+    const int split = blockIdx.x, b = blockIdx.z;
+    int G = plan.G, chunks = plan.chunks, B = j.B, n_split = j.nsplit, ends[kDecodeSegs - 1];
+#pragma unroll
+    for (int i = 0; i < kDecodeSegs - 1; ++i) ends[i] = plan.end[i];
+    StepQkv own_rows{};
+    if constexpr (FRONT) own_rows = f;
+    at_once(j, G, chunks, B, n_split, ends, own_rows);
     int g = blockIdx.y, c = 0;
-    if (plan.chunks > 1) g = (int)blockIdx.y / plan.chunks, c = (int)blockIdx.y - g * plan.chunks;
+    if (chunks > 1) g = (int)blockIdx.y / chunks, c = (int)blockIdx.y - g * chunks;
     // the ranges that this workgroup's split is one of, and which one of how many
     const bool lead = SELECT && split < j.lead_splits;
     const int seg_lo = SELECT && !lead ? j.lead_segs : 0, seg_hi = lead ? j.lead_segs : j.n_seg;
     const int part = SELECT && !lead ? split - j.lead_splits : split, n_part = !SELECT ? n_split : lead ? j.lead_splits : n_split - j.lead_splits;
     if constexpr (FRONT) {
-        if (b >= j.B) {
-            const int x = split + n_split * ((int)blockIdx.y + (int)gridDim.y * (b - j.B)), n_rows = j.B * j.Hkv;
+        if (b >= B) {
+            const int x = split + n_split * ((int)blockIdx.y + j.Hkv * chunks * (b - B)), n_rows = B * j.Hkv;
             if constexpr (std::is_same_v<Front, MemoryRows>) {
+                if (threadIdx.x >= 256) return;
                 if (x < n_rows) ingest_one<D>(f.in, x / j.Hkv, x % j.Hkv, (float2 *)red_room);
             } else {
                 const int at = x - n_rows, bg = at / max(f.pieces, 1);
-                if (at < 0) leave_rows<D>(f, x / j.Hkv, x % j.Hkv, (float2 *)red_room);
-                else if (at < n_rows * f.pieces) copy_rows<D, kStepCopyRows<D>>(f.copy, at - bg * f.pieces, bg / j.Hkv, bg % j.Hkv);
+                if (at < 0) {
+                    if (threadIdx.x < 256) leave_rows<D>(f, x / j.Hkv, x % j.Hkv, (float2 *)red_room);
+                } else if (at < n_rows * f.pieces) copy_rows<D, kStepCopyRows, kDecWaves * kWave>(f.copy, at - bg * f.pieces, bg / j.Hkv, bg % j.Hkv);
             }
             return;
         }
@@ -131,12 +156,11 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     const float lazy = kLazyDec / scale;
 
     // ---- the list of blocks: every range rounded up to whole blocks (units: every unit by itself)
-    const int seg_first = seg_lo > 0 ? plan.end[seg_lo - 1] : 0, n_blocks = (seg_hi > 0 ? plan.end[seg_hi - 1] : 0) - seg_first;
+    const int seg_first = seg_lo > 0 ? plan.end[seg_lo - 1] : 0, n_blocks = (SELECT ? plan.end[seg_hi - 1] : plan.blocks) - seg_first + NEW;
     const int each = n_blocks / n_part, over = n_blocks - each * n_part;                   // (of n_blocks * part / n_part, below)
-    const int b_lo = seg_first + each * part + over * part / n_part, b_hi = seg_first + each * (part + 1) + over * (part + 1) / n_part;
+    const int b_lo = seg_first + each * part + over * part / n_part, b_hi = seg_first + each * (part + 1) + over * (part + 1) / n_part - (NEW && split == n_split - 1);
     __shared__ int32_t chosen[SELECT ? kSelectMost : 1];
     if constexpr (SELECT) {
-        static_assert(sizeof(SelectLds<kDecWaves * kWave>) <= sizeof(red_room));
         if (lead) {
             select_units<kDecWaves * kWave>(j.unit_scores + (int64_t)b * j.unit_scores_sb, j.n_scores, j.seg[0].n_ids, chosen, *(SelectLds<kDecWaves * kWave> *)red_room);
             if (split == 0 && blockIdx.y == 0)
@@ -155,11 +179,11 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         int s = 0, first = 0;
 #pragma unroll
         for (int i = 0; i < kDecodeSegs - 1; ++i)
-            if (blk >= plan.end[i]) s = i + 1, first = plan.end[i];
+            if (blk >= ends[i]) s = i + 1, first = ends[i];
         blk -= first;
         const DecodeSeg sg = j.seg[s];
         Block r{nullptr, nullptr, 0, sg.q, -1};
-        if (sg.n_ids > 0) {
+        if (UNITS && sg.n_ids > 0) {
             const int per = (sg.rows + kDecodeBlock - 1) / kDecodeBlock, i = blk / per, r0 = (blk - i * per) * kDecodeBlock;
             const int u = __builtin_amdgcn_readfirstlane(SELECT ? chosen[i] : sg.ids ? sg.ids[(int64_t)b * sg.n_ids + i] : i);
             const int ch = u / j.per_chunk;
@@ -277,18 +301,19 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
     // begins; two microseconds of the first block's six (workgroups begin their products at 4.4 instead of 6.6 us of a step that slides;
     // causal, one token over 32,768, 8 key heads of 128: 32.9 -> 31.5 us a pass).
     const int own = threadIdx.x / (D / 16), own_at = threadIdx.x % (D / 16) * 8;
-    const bool is_q = own < nh, is_k = own == NG, has_new = FRONT && split == n_split - 1 && wave == kDecWaves - 1;
+    const bool is_q = own < nh, is_k = own == NG, has_new = FRONT && split == n_split - 1 && wave == (b_hi - b_lo) % kDecWaves;
     u32x4 own_lo{}, own_hi{}, new_v{};
     float freq = 0.f;
     if constexpr (FRONT) {
-        freq = rope_freq<D / 2>(f.inv_freq);
-        const bf16_t *q_rows = f.q + (int64_t)b * f.q_sb + (int64_t)h0 * f.q_sh, *k_row = f.k + (int64_t)b * f.k_sb + (int64_t)g * f.k_sh;
+        const StepQkv &r = own_rows;
+        freq = rope_freq<D / 2>(r.inv_freq);
+        const bf16_t *q_rows = r.q + (int64_t)b * r.q_sb + (int64_t)h0 * r.q_sh, *k_row = r.k + (int64_t)b * r.k_sb + (int64_t)g * r.k_sh;
         asm volatile("" : "+s"(q_rows), "+s"(k_row));            // (both addresses; not that of the one to be read)
         if (is_q || is_k) {
-            const bf16_t *src = (is_q ? q_rows + (int64_t)own * f.q_sh : k_row) + own_at;
+            const bf16_t *src = (is_q ? q_rows + (int64_t)own * r.q_sh : k_row) + own_at;
             own_lo = *(const u32x4 *)src, own_hi = *(const u32x4 *)(src + D / 2);
         }
-        if (has_new) new_v = *(const u32x4 *)(f.v + (int64_t)b * f.v_sb + (int64_t)g * f.v_sh + (lane & (LPR - 1)) * 8);
+        if (has_new) new_v = *(const u32x4 *)(r.v + (int64_t)b * r.v_sb + (int64_t)g * r.v_sh + (lane & (LPR - 1)) * 8);
         asm volatile("" ::: "memory");
     }
     int q_now = -1, blk = b_lo + wave;
@@ -348,24 +373,43 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
 
     // ---- join the row groups of the wave, then the waves (m == -infinity: nothing seen yet, or logits that are no numbers, whose
     //      sums have to stay NaN)
-    float mw = fmaxf(m, __shfl_xor(m, 16, 64));
-    mw = fmaxf(mw, __shfl_xor(mw, 32, 64));
+    const float mw = wave_max32(wave_max16(m));
     const float to_mw = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mw) * scale);
     float lw = m == -INFINITY ? l : l * to_mw;
-    lw += __shfl_xor(lw, 16, 64);
-    lw += __shfl_xor(lw, 32, 64);
+    lw = wave_sum32(wave_sum16(lw));
     if (lane < NG) {
         sm[wave][lane] = mw;
         sl[wave][lane] = lw;
     }
-    const int vg = lane / LPR;                     // this lane's group of value rows: its own row group, or half of it
+    // (The row groups' sums trade places as they are added: rows of 16 lanes keep a half of the numbers at each of two steps, so that a
+    // quarter of them goes through LDS, and none more than once.)
+    constexpr int N8 = NG * 8;
+    float x[N8];
     each_head<NG>([&](auto hc) {
         constexpr int h = decltype(hc)::value;
         const float f = row_bcast<h>(to_mw);
-        float *dst = &red[wave][vg][h][(lane & (LPR - 1)) * 8];
-        *(f32x4 *)dst = f32x4{acc[h][0] * f, acc[h][1] * f, acc[h][2] * f, acc[h][3] * f};
-        *(f32x4 *)(dst + 4) = f32x4{acc[h][4] * f, acc[h][5] * f, acc[h][6] * f, acc[h][7] * f};
+#pragma unroll
+        for (int d = 0; d < 8; ++d) x[h * 8 + d] = acc[h][d] * f;
     });
+#pragma unroll
+    for (int i = 0; i < N8 / 2; ++i) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[i]), __float_as_uint(x[i + N8 / 2]), false, false);
+        x[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < N8 / 4; ++i) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[i]), __float_as_uint(x[i + N8 / 4]), false, false);
+        x[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        if (D == 64) x[i] += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x[i]), 0x128, 0xf, 0xf, true));   // the row's other half
+    }
+    if (col < LPR) {
+        const int first = rg * (N8 / 4);
+        float *dst = &red[wave][first / 8][col * 8 + first % 8];
+        if constexpr (NG == 1) *(float2 *)dst = float2{x[0], x[1]};
+        else
+#pragma unroll
+            for (int i = 0; i < N8 / 4; i += 4) *(f32x4 *)(dst + i) = f32x4{x[i], x[i + 1], x[i + 2], x[i + 3]};
+    }
     __syncthreads();
     const int64_t row0 = ((int64_t)split * j.B + b) * j.H + h0;
     for (int e = threadIdx.x * 2; e < nh * D; e += kDecWaves * kWave * 2) {
@@ -378,9 +422,7 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         for (int w = 0; w < kDecWaves; ++w) {
             const float f = sm[w][h] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((sm[w][h] - mx) * scale);
             den += sm[w][h] == -INFINITY ? sl[w][h] : sl[w][h] * f;
-            float2 ow{0.f, 0.f};
-#pragma unroll
-            for (int r = 0; r < GRP; ++r) ow.x += red[w][r][h][d], ow.y += red[w][r][h][d + 1];
+            const float2 ow = *(const float2 *)&red[w][h][d];
             o.x += ow.x * f, o.y += ow.y * f;
         }
         const f16x2 part{(_Float16)(den == 0.f ? 0.f : o.x / den), (_Float16)(den == 0.f ? 0.f : o.y / den)};
@@ -400,28 +442,33 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
         //      write its L2 back.  Wave w takes every fourth split, a lane one head's 8 elements (merge_piece's arithmetic).
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        int &last = *(int *)&sm[0][0];
-        uint32_t *ticket = j.ticket + (int64_t)b * gridDim.y + blockIdx.y;
+        __shared__ int last;
+        uint32_t *ticket = j.ticket + (int64_t)b * (j.Hkv * chunks) + blockIdx.y;
         if (threadIdx.x == 0) last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)n_split - 1;
         __syncthreads();
         if (!last) return;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        asm volatile("" ::: "memory");
         if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();                           // (the word is sm's)
         const int h = lane / LPR, at = (lane & (LPR - 1)) * 8;                 // (heads of 64: four of them are 32 lanes)
         const bool on = h < nh;
-        const int64_t step = (int64_t)j.B * j.H, row = (int64_t)b * j.H + h0 + (on ? h : 0);
+        // (a scalar address for each split, one offset for the lane)
+        const int64_t rows = (int64_t)j.B * j.H, lead_row = wave * rows + (int64_t)b * j.H + h0;
+        const uint32_t lane_l = (on ? h : 0) * 4, lane_o = (on ? h : 0) * (D * 2) + at * 2;
+        const char *from_l = (const char *)(j.lse_part + lead_row), *from_o = (const char *)(j.o_part + lead_row * D);
         float mx = -INFINITY, den = 0.f, o[8] = {};
-        constexpr int kBatch = 8;                  // splits whose rows are requested together
+        constexpr int kBatch = 8;                  // splits whose rows are requested together: all of a wave's, up to 64 splits
         for (int s0 = wave; s0 < n_split; s0 += kBatch * kDecWaves) {
             float l8[kBatch];
-            f16x8 o8[kBatch];
+            uint64_t lo[kBatch], hi[kBatch];
 #pragma unroll
             for (int i = 0; i < kBatch; ++i) {
-                const int s = s0 + i * kDecWaves;
-                const bool in = on && s < n_split;
-                l8[i] = in ? j.lse_part[s * step + row] : -INFINITY;
-                o8[i] = in ? *(const f16x8 *)((const _Float16 *)j.o_part + (s * step + row) * D + at) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+                l8[i] = -INFINITY, lo[i] = hi[i] = 0;
+                if (s0 + i * kDecWaves < n_split) {
+                    l8[i] = __hip_atomic_load((const float *)(from_l + lane_l), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    lo[i] = __hip_atomic_load((const uint64_t *)(from_o + lane_o), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    hi[i] = __hip_atomic_load((const uint64_t *)(from_o + lane_o + 8), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    from_l += rows * (kDecWaves * 4), from_o += rows * (kDecWaves * D * 2);
+                }
             }
             float mn = mx;
 #pragma unroll
@@ -434,37 +481,40 @@ __global__ __launch_bounds__(kDecWaves * kWave, 3) void decode_attn_kernel(Decod
             }
 #pragma unroll
             for (int i = 0; i < kBatch; ++i) {     // exp2(-inf) = 0: empty splits hold zeros, those with a logit that was no number NaN
+                if (s0 + i * kDecWaves >= n_split) break;
                 const float w = __builtin_amdgcn_exp2f(l8[i] - base);
+                const f16x4 x = __builtin_bit_cast(f16x4, lo[i]), y = __builtin_bit_cast(f16x4, hi[i]);
 #pragma unroll
-                for (int d = 0; d < 8; ++d) o[d] += (float)o8[i][d] * w;
+                for (int d = 0; d < 4; ++d) o[d] += (float)x[d] * w, o[4 + d] += (float)y[d] * w;
                 den += w;
             }
             mx = mn;
         }
-        float *mine = red_room + (wave * 64 + lane) * kJoin;                   // 8 sums, the maximum, the weight
-#pragma unroll
-        for (int d = 0; d < 8; ++d) mine[d] = o[d];
-        mine[8] = mx, mine[9] = den;
-        __syncthreads();
-        if (wave != 0 || !on) return;
-        mx = -INFINITY, den = 0.f;
-#pragma unroll
-        for (int d = 0; d < 8; ++d) o[d] = 0.f;
-#pragma unroll
-        for (int w = 0; w < kDecWaves; ++w) mx = fmaxf(mx, red_room[(w * 64 + lane) * kJoin + 8]);
-        const float base = mx == -INFINITY ? 0.f : mx;
-#pragma unroll
-        for (int w = 0; w < kDecWaves; ++w) {
-            const float *part = red_room + (w * 64 + lane) * kJoin;
-            const float f = __builtin_amdgcn_exp2f(part[8] - base);
-            // (a wave whose splits are all empty or no numbers: its sums are zeros or NaN, taken with weight 0)
-#pragma unroll
-            for (int d = 0; d < 8; ++d) o[d] += part[d] * f;
-            den += part[9] * f;
+        if (on) {
+            float *mine = &red[wave][h][at];
+            *(f32x4 *)mine = f32x4{o[0], o[1], o[2], o[3]};
+            *(f32x4 *)(mine + 4) = f32x4{o[4], o[5], o[6], o[7]};
+            if (at == 0) sm[wave][h] = mx, sl[wave][h] = den;
         }
-        const float inv = den > 0.f ? 1.f / den : 0.f;
-        *(u32x4 *)(j.out + (int64_t)b * j.out_sb + (int64_t)(h0 + h) * j.out_sh + at) =
-            u32x4{pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv), pack_bf16x2(o[4] * inv, o[5] * inv), pack_bf16x2(o[6] * inv, o[7] * inv)};
+        __syncthreads();
+        for (int e = threadIdx.x * 2; e < nh * D; e += kDecWaves * kWave * 2) {
+            const int eh = e / D, d = e % D;
+            float most = -INFINITY, all = 0.f;
+            float2 x{0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < kDecWaves; ++w) most = fmaxf(most, sm[w][eh]);
+            const float base = most == -INFINITY ? 0.f : most;
+#pragma unroll
+            for (int w = 0; w < kDecWaves; ++w) {
+                // (a wave whose splits are all empty or no numbers: its sums are zeros or NaN, taken with weight 0)
+                const float f = __builtin_amdgcn_exp2f(sm[w][eh] - base);
+                const float2 xw = *(const float2 *)&red[w][eh][d];
+                x.x += xw.x * f, x.y += xw.y * f;
+                all += sl[w][eh] * f;
+            }
+            const float inv = all > 0.f ? 1.f / all : 0.f;
+            *(uint32_t *)(j.out + (int64_t)b * j.out_sb + (int64_t)(h0 + eh) * j.out_sh + d) = pack_bf16x2(x.x * inv, x.y * inv);
+        }
     }
 }
 
@@ -477,6 +527,7 @@ DecodePlan plan_of(const DecodeJob *job, int NG) {
         if (s < job->n_seg) n += (job->seg[s].rows + kDecodeBlock - 1) / kDecodeBlock * (job->seg[s].n_ids > 0 ? job->seg[s].n_ids : 1);
         p.end[s] = s < job->n_seg ? n : INT32_MAX;
     }
+    p.blocks = n;
     return p;
 }
 
@@ -496,12 +547,11 @@ template <int D>
 int launch_step(const DecodeJob *job, const StepRows *rows, void *stream) {
     const int G = job->H / job->Hkv, NG = G >= 3 ? 4 : G;
     const int y = job->Hkv * ((G + NG - 1) / NG);
-    // The workgroups that write the cache come behind all splits, in batch rows of their own.  In the grid's first dimension, behind
-    // the splits of every head, they took places among the 512 that the chip has at two workgroups a CU and left again, so that some
-    // CUs got three splits and some one, and a row of 65 spread the heads of a group, which read the same keys, over the XCDs: causal
-    // steps of 8 key heads over 24,000 / 32,768 / 49,152 tokens 31.8 / 39.3 / 52.1 us so, 29.3 / 33.2 / 42.4 now, 32.5 / 36.5 / 45.7 as two
-    // launches; of 2 key heads with 16 query heads each over 65,536 / 98,304 60.9 / 88.2, 38.1 / 54.1 and 47.2 / 63.1; of 36 heads of 64
-    // over 10,000 26.7, 26.7 and 32.2.
+    // The workgroups that write the cache come behind all splits, in batch rows of their own.  In the grid's first dimension, behind the
+    // splits of every head, they take places of splits and leave again, so that some CUs get two splits and some none, and a row of
+    // them spreads the heads of a group, which read the same keys, over the XCDs.  (With workgroups of four waves: causal steps of 8 key heads
+    // over 24,000 / 32,768 / 49,152 tokens 31.8 / 39.3 / 52.1 us so, 29.3 / 33.2 / 42.4 behind all, 32.5 / 36.5 / 45.7 as two launches; of 2 key
+    // heads with 16 query heads each over 65,536 / 98,304 60.9 / 88.2, 38.1 / 54.1 and 47.2 / 63.1.)
     const int64_t extra = (int64_t)(1 + rows->pieces) * job->Hkv * job->B, planes = (extra + (int64_t)job->nsplit * y - 1) / ((int64_t)job->nsplit * y);
     if (job->B + planes > 65535 || extra >= (1ll << 30)) return 1;
     const dim3 grid(job->nsplit, y, (unsigned)(job->B + planes));
@@ -532,15 +582,22 @@ int launch_memory_step(const DecodeJob *job, const infllm_ingest_args *in, void 
 
 }  // namespace
 
-// Key splits of a decode step over `blocks` blocks of 16 keys: two workgroups per CU where there are blocks for them (a
-// wave then has one or two blocks of its own in flight), never fewer than one block per wave, at most max_splits.
-int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int64_t blocks, int32_t max_splits) {
+// Key splits of a decode step over `blocks` blocks of 16 keys: as many as have a block for each of their waves and a CU of their own (heads
+// of 64: half of one), of which `others` are for the workgroups beside the splits; at most max_splits.  Where the heads alone are about as
+// many, workgroups come in rounds, and the splits are those whose rounds take least, a round being its blocks and four blocks' time to begin
+// and end.  (Heads of 64 with a CU to each, 72 heads with a window of 2,048: 28.6 us a step, so 21.7.)
+int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int32_t dim, int64_t blocks, int32_t max_splits, int64_t others) {
     const int G = H / Hkv, NG = G >= 3 ? 4 : G;
-    const int64_t wgs = (int64_t)B * Hkv * ((G + NG - 1) / NG);
-    int64_t s = (2 * 256 + wgs - 1) / wgs;
-    if (s > blocks / kDecWaves) s = blocks / kDecWaves;
-    if (s > max_splits) s = max_splits;
-    return s < 1 ? 1 : (int)s;
+    const int64_t wgs = (int64_t)B * Hkv * ((G + NG - 1) / NG), places = (dim == 64 ? 512 : 256) - std::min<int64_t>(others, 128);
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>((blocks + kDecWaves - 1) / kDecWaves, max_splits));
+    if (wgs * 4 <= places) return (int)std::min(places / wgs, most);
+    int best = 1;
+    int64_t best_time = INT64_MAX;
+    for (int s = 1; s <= std::min<int64_t>(most, 8); ++s) {
+        const int64_t time = (wgs * s + places - 1) / places * (4 + (blocks + s * kDecWaves - 1) / (s * kDecWaves));
+        if (time < best_time) best = s, best_time = time;
+    }
+    return best;
 }
 
 static int check_job(const DecodeJob *job, int32_t dim) {
@@ -583,7 +640,7 @@ int infllm_decode_memory_step(const DecodeJob *job, const infllm_ingest_args *in
 }
 
 // How many of a launch's splits the ranges get that wait for a selection (lead_blocks of 16 keys) so that they end with the others: the
-// selection is taken for as long as three blocks of a wave.  It reads all scores twice and lasts the longer the more there are, but the
+// selection is taken for as long as three blocks of a wave (measured with workgroups of four).  It reads all scores twice and lasts the longer the more there are, but the
 // launch depends little on where between two and six the line lies.  (The kernel alone, 32 / 8 heads of 128, 16 of 20 / 479 / 4,096 /
 // 16,384 units, taken for 1, 2, 3, 6 and 9 blocks: 13.2 11.9 12.1 12.2 11.9 / 14.3 12.4 12.3 12.4 12.1 / 15.8 13.2 13.6 13.5 13.4 /
 // 23.2 20.7 20.7 20.6 20.6 us; 64 of 16,384: 36.9 36.1 36.5 36.8 36.1; 36 heads of 64, 15 splits each, 16 of

@@ -315,23 +315,23 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         if (far_rows > 0)
             d.seg[d.n_seg++] = a->kind == 2 ? DecodeSeg{(const bf16_t *)raw_from, ov, raw_from_sh * a->Hkv, raw_from_sh, a->ov_sb, a->ov_sh, (int32_t)far_rows, 1, 0, nullptr, -1}
                                             : DecodeSeg{ok, ov, a->ok_sb, a->ok_sh, a->ov_sb, a->ov_sh, (int32_t)far_rows, 1, 0, nullptr, -1};
-        d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, (near_old + kDecodeBlock - 1) / kDecodeBlock + (far_rows + kDecodeBlock - 1) / kDecodeBlock, max_parts);
+        StepRows f{};
+        for (int i = 0; i < kCopies; ++i) {
+            f.copy[i] = j.copy[i];
+            f.pieces += (j.copy[i].n + kStepCopyRows - 1) / kStepCopyRows;
+        }
+        d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, D, (near_old + kDecodeBlock - 1) / kDecodeBlock + (far_rows + kDecodeBlock - 1) / kDecodeBlock + 1, max_parts,
+                                        (int64_t)(1 + f.pieces) * a->Hkv * a->B);
         d.o_part = (uint16_t *)((char *)a->d_work + q_bytes);
         d.lse_part = (float *)((char *)a->d_work + q_bytes + part_rows * 2 * D);
         d.out = (bf16_t *)a->d_out; d.out_sb = a->o_sb; d.out_sh = a->o_sh;
         d.ticket = (uint32_t *)a->d_ticket;
-        StepRows f{};
         f.q = j.q; f.k = j.k; f.v = j.v;
         f.q_sb = a->q_sb; f.q_sh = a->q_sh; f.k_sb = a->k_sb; f.k_sh = a->k_sh; f.v_sb = a->v_sb; f.v_sh = a->v_sh;
         f.pos = a->seen; f.glb_pos = j.glb_pos;
         f.inv_freq = a->d_inv_freq; f.distance_scale = a->distance_scale;
         f.dk = j.dk; f.dv = j.dv; f.dk_sb = j.dk_sb; f.dk_sh = j.dk_sh; f.dv_sb = j.dv_sb; f.dv_sh = j.dv_sh;
         if (j.n_raw > 0) f.raw = j.raw, f.raw_sb = j.raw_sb, f.raw_sh = j.raw_sh;
-        const int piece_rows = D == 128 ? kStepCopyRows<128> : kStepCopyRows<64>;
-        for (int i = 0; i < kCopies; ++i) {
-            f.copy[i] = j.copy[i];
-            f.pieces += (j.copy[i].n + piece_rows - 1) / piece_rows;
-        }
         rc = infllm_decode_step(&d, &f, D, stream);
         if (rc != 1) return rc;
     }
@@ -380,7 +380,7 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         const int64_t far = far_rows;
         if (far > 0) d.seg[d.n_seg++] = DecodeSeg{sk, bv, sk_sb, sk_sh, bv_sb, bv_sh, (int32_t)far, 1, 0, nullptr, -1};
         const int64_t blocks = (near + kDecodeBlock - 1) / kDecodeBlock + (far > 0 ? (far + kDecodeBlock - 1) / kDecodeBlock : 0);
-        d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, blocks, max_parts);
+        d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, D, blocks, max_parts);
         d.o_part = (uint16_t *)((char *)a->d_work + q_bytes);
         d.lse_part = (float *)((char *)a->d_work + q_bytes + part_rows * 2 * D);
         d.out = (bf16_t *)a->d_out; d.out_sb = a->o_sb; d.out_sh = a->o_sh;
