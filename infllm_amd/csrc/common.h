@@ -82,10 +82,27 @@ __device__ __forceinline__ void load_to_lds4(const float *base, uint32_t lane_of
 __device__ __forceinline__ void load_to_lds16(const bf16_t *base, uint32_t lane_off, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(lane_off), "s"(base) : "memory");
 }
+__device__ __forceinline__ void load_to_lds16_at(const bf16_t *src, uint32_t lds) {                       // every lane from an address of its own
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory");
+}
 __device__ __forceinline__ uint32_t lds_address(const char *p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p; }
 
 __device__ __forceinline__ float wave_xor32(float x) {
     return __shfl_xor(x, 32, 64);
+}
+
+// A word of every line of the kernel's arguments (the first BYTES of them, a number of lines up to 16), in one trip: what is read of them
+// where it is needed is then a trip to the scalar cache and not to memory.
+template <int BYTES>
+__device__ __forceinline__ void touch_arguments() {
+    constexpr int kLines = (BYTES + 63) / 64;
+    static_assert(kLines <= 16);
+    auto *p = (const __attribute__((address_space(4))) uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
+    uint32_t w[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) w[i] = i < kLines ? p[min(16 * i, BYTES / 4 - 1)] : 0;
+    asm volatile("" : : "s"(w[0]), "s"(w[1]), "s"(w[2]), "s"(w[3]), "s"(w[4]), "s"(w[5]), "s"(w[6]), "s"(w[7]), "s"(w[8]), "s"(w[9]), "s"(w[10]), "s"(w[11]),
+                 "s"(w[12]), "s"(w[13]), "s"(w[14]), "s"(w[15]));
 }
 
 // the larger of a lane's value and that of the lane 32 away, in both: vector instructions (a shuffle is a trip through LDS)

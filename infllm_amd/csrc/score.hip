@@ -310,7 +310,7 @@ struct BlockEnd {
 // that such a query sees infinite or NaN.
 //
 // A wave's exponentials and MFMAs overlap (half a sub-tile of 32 queries apart), so the loop runs at the rate of the vector unit
-// (768 cycles of a sub-tile of 32 queries x 64 keys); what is left is a launch of one or two rounds of workgroups whose first 7
+// (768 cycles of a sub-tile of 32 queries x 64 keys); what is left is a launch of one or two rounds of workgroups whose first 5
 // of 20 us are the wait for their keys.  So registers and LDS are kept to a third of a CU: all carving and scoring workgroups of
 // 512 queries x 4,096 keys x 32 heads are in flight at once, one's wait beside another's loop.  The queries go from memory
 // straight into LDS (64 rows a stage, three stages in turn, no registers on the way), and a wave's two accumulators are the halves
@@ -381,22 +381,45 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
         asm volatile("" ::: "memory");
     }
     if (st_lo < st_hi) load_stage(st_lo, 0);
-    if (NB > 2 && st_lo + 1 < st_hi) load_stage(st_lo + 1, 1);
 
-    // ---- this wave's keys as the B operand (lane = key column)
+    // ---- this wave's keys as the B operand (lane = key column), by way of the stages that are not on their way yet: 32 keys of every wave
+    //      at a time, whole rows in order.  (Keys that do not count: one that does again, its sums are not used.)  Straight into registers,
+    //      by lanes that fetch their own key's pieces, they are 64 lines an instruction, and the 12 waves of a CU asked for 6 us: keys in
+    //      registers 7.2 us behind the launch's start, 5.5 so.  Prompts of 16,001 / 131,072 tokens 2,521 -> 2,505 / 24,210 -> 23,937 us,
+    //      operator over 512 x (4,608 + 2,624) keys 93.2 -> 92.2.
+    constexpr int kKeyLds = 32 / QG / kRowsPerLd;
+    static_assert((NB - 1) * kStage >= 128 * kRow && (KS == 1 || QG == 1), "room for 128 keys behind the first stage");
+    const bf16_t *kbase = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh;
+    const uint32_t k_lds = lds_address(lds) + kStage;
+    auto ask_keys = [&](int ks) {
+        if (hi > lo)
+#pragma unroll
+            for (int i = 0; i < kKeyLds; ++i) {
+                const int r = kRowsPerLd * (kKeyLds * any_wave + i) + lane / (D / 8);
+                int row = slot + min(max((r >> 5) * kWaveKeys + ks * 32 + (r & 31), lo), hi - 1);
+                row = row < cap ? row : row - cap;
+                load_to_lds16_at(kbase + (int64_t)row * a.k_sl + ((lane & (D / 8 - 1)) ^ swz<D>(r)) * 8, k_lds + (kKeyLds * any_wave + i) * 1024);
+            }
+    };
     bf16x8 kreg[KS][D / 16];
+    auto take_keys = [&](int ks) {                                  // (a wave's rows are its own, or of it and the other group's)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if constexpr (QG > 1) asm volatile("s_barrier" ::: "memory");
+        const uint32_t at = k_lds + (wave * 32 + col) * kRow + ((grp ^ swz<D>(col)) * 16);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        const int r = wave * kWaveKeys + ks * 32 + col;
-        int row = slot + r;
-        row = row < cap ? row : row - cap;
-        const bf16_t *krow = (const bf16_t *)a.d_k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh + (int64_t)row * a.k_sl + grp * 8;
+        for (int kk = 0; kk < D / 16; ++kk) kreg[ks][kk] = __builtin_bit_cast(bf16x8, *(const __attribute__((address_space(3))) u32x4 *)(uintptr_t)(at ^ (kk * 32)));
 #pragma unroll
-        for (int kk = 0; kk < D / 16; ++kk) {
-            const u32x4 raw = r >= lo && r < hi ? *(const u32x4 *)(krow + kk * 16) : u32x4{0, 0, 0, 0};
-            kreg[ks][kk] = __builtin_bit_cast(bf16x8, raw);
-        }
+        for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(kreg[ks][kk]));         // (read before the rows are overwritten)
+    };
+    ask_keys(0);
+    take_keys(0);
+    if constexpr (kSumsFirst) {                                     // (they have come; the compiler's wait for them belongs here)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int p = 0; p < 8; ++p) asm volatile("" : "+v"(l8[e][p]));
     }
+    if constexpr (KS > 1) ask_keys(1);
     // ---- joined log-sum-exps of all queries
     if constexpr (JOIN) {
         const int padded = (Lq + QR - 1) / QR * QR;
@@ -414,8 +437,10 @@ __device__ __forceinline__ void key_sums(const infllm_score_args &a, const PartS
                 if (i0 + e * kThreads < padded) Ls[i0 + e * kThreads] = den > 0.f ? m8 + log2f(den) : empty;
             }
         }
-        __syncthreads();
     }
+    if constexpr (KS > 1) take_keys(1);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");                 // the sums are there, and the keys' place is free
+    if (NB > 2 && st_lo + 1 < st_hi) load_stage(st_lo + 1, 1);
 
     // (the keys' wait belongs here: in front of their first use, inside the loop, it would be one for the stages on their way)
 #pragma unroll
@@ -629,6 +654,7 @@ __global__ __launch_bounds__(256, (D == 64 ? 4 : 3)) void block_end_kernel(Block
         asm volatile("" : "+s"(p));
         return *(const BlockEnd *)p;
     };
+    touch_arguments<sizeof(BlockEnd)>();                          // (prompts of 16,001 / 131,072 tokens 0.7 / 0.4 %)
     int x = blockIdx.x;
     const int n_carve = arguments().n_carve;
     if (x < n_carve) {
