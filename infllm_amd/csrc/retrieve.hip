@@ -462,32 +462,34 @@ int ticket_slot(hipStream_t st) {
     return -1;
 }
 
-// the selection by one workgroup of kRetrThreads threads over N <= NB * 16 * kRetrThreads scores; a thread keeps its
-// keys (units tid, tid + kRetrThreads, ...) in registers
-template <int NB>
+// the selection by one workgroup of kRetrThreads threads over N <= R * kRetrThreads scores; a thread keeps its
+// keys (units tid, tid + kRetrThreads, ...) in registers.  (With 16 keys a thread however few units there are, and a release and an acquire
+// around the ticket, which what crosses workgroups here - stores performed, loads past the L2 - does not need: 8 best of 64 units with
+// rows of 512 6.5 -> 5.2 us, 16 of 300 / 2,000 7.4 / 10.6 -> 6.0 / 9.2, 16 of 8,192 with rows of 4,096 19.7 -> 19.0.)
+template <int R>
 __device__ __forceinline__ void select_topk_block(const float *scores, int N, int k, int32_t *idx_out, int32_t *idx_out2) {
     __shared__ uint64_t surv[kSurvivorCap + 8];
     __shared__ uint32_t gmax[kRetrThreads / 64][64];
     __shared__ int wave_cnt[kRetrThreads / 64];
     __shared__ int s_count;
-    constexpr int R = NB * 16;                                   // 16 loads in flight per thread and round trip
+    constexpr int kBatch = R < 16 ? R : 16;                      // loads in flight per thread and round trip
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     uint32_t key[R];
     uint32_t best = 0;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        float sc[16];
+    for (int b = 0; b < R / kBatch; ++b) {
+        float sc[kBatch];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int n = tid + (b * 16 + j) * kRetrThreads;
+        for (int j = 0; j < kBatch; ++j) {
+            const int n = tid + (b * kBatch + j) * kRetrThreads;
             // an agent-scope load: it is served from where the other workgroups' agent-scope stores went
             sc[j] = n < N ? __hip_atomic_load(scores + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
         }
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int n = tid + (b * 16 + j) * kRetrThreads;
-            key[b * 16 + j] = n < N ? order_key(sc[j]) : 0u;
-            best = key[b * 16 + j] > best ? key[b * 16 + j] : best;
+        for (int j = 0; j < kBatch; ++j) {
+            const int n = tid + (b * kBatch + j) * kRetrThreads;
+            key[b * kBatch + j] = n < N ? order_key(sc[j]) : 0u;
+            best = key[b * kBatch + j] > best ? key[b * kBatch + j] : best;
         }
     }
     auto composite = [&](int j) { return ((uint64_t)key[j] << 32) | (uint32_t)(0xffffffffu - (uint32_t)(tid + j * kRetrThreads)); };
@@ -497,21 +499,38 @@ __device__ __forceinline__ void select_topk_block(const float *scores, int N, in
     // counting made the launch 17.7 us instead of 11).  The threshold is on the score's key alone: units that tie with it all
     // pass, and are told apart by the composites afterwards.
     const int groups = k <= 16 ? 16 : k <= 32 ? 32 : 64;
-    for (int o = 32; o >= groups; o >>= 1) {
-        const uint32_t other = __shfl_xor(best, o, 64);
-        best = other > best ? other : best;
-    }
-    gmax[wave][lane] = best;                                     // lane: its group's maximum, lane mod groups
+    gmax[wave][lane] = best;
     __syncthreads();
-    uint32_t tau = 0;
+    uint32_t bests[kRetrThreads / 64], tau = 0;
 #pragma unroll
-    for (int w = 0; w < kRetrThreads / 64; ++w) tau = max(tau, gmax[w][lane]);
+    for (int w = 0; w < kRetrThreads / 64; ++w) bests[w] = gmax[w][lane], tau = max(tau, bests[w]);
+    for (int o = 32; o >= groups; o >>= 1) tau = max(tau, (uint32_t)__shfl_xor(tau, o, 64));        // lane: its group's maximum, lane mod groups
+    const uint32_t top = tau;
     // the smallest of them: rows of 16 lanes by rotation, which is the whole of it when the rows are copies of each other
     tau = min(tau, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)tau, 0x121, 0xf, 0xf, false));
     tau = min(tau, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)tau, 0x122, 0xf, 0xf, false));
     tau = min(tau, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)tau, 0x124, 0xf, 0xf, false));
     tau = min(tau, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)tau, 0x128, 0xf, 0xf, false));
     for (int o = 16; o < groups; o <<= 1) tau = min(tau, (uint32_t)__shfl_xor(tau, o, 64));
+    // Of 64 groups that lets five times k units pass, and their ranking by counting is longer than all else: every wave halves the way
+    // up to the largest, until k of the threads' best are above and at most an eighth more.  (64 best of 1,000 / 16,384 units with rows of
+    // 4,096: 17.3 / 34.1 -> 11.9 / 30.1 us; of 64 units, where nothing is to be gained, 10.3 -> 11.5, so not of a few.)
+    if (k > 16 && N > 2 * groups) {
+        uint32_t lo = __builtin_amdgcn_readfirstlane(tau), hi = top;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) hi = max(hi, (uint32_t)__shfl_xor(hi, o, 64));
+        hi = __builtin_amdgcn_readfirstlane(hi);
+        for (int i = 0; i < 12 && hi - lo > 1; ++i) {            // (lo: k of them reach it; hi: fewer than k, or it was not tried)
+            const uint32_t mid = lo + (hi - lo) / 2;
+            int c = 0;
+#pragma unroll
+            for (int w = 0; w < kRetrThreads / 64; ++w) c += __popcll(__builtin_amdgcn_ballot_w64(bests[w] >= mid));
+            if (c >= k) lo = mid;
+            else hi = mid;
+            if (c >= k && c <= k + k / 8) break;
+        }
+        tau = lo;
+    }
     auto collect = [&](uint64_t thr) {                           // composites >= thr into surv[]; s_count = how many there are
 #pragma unroll
         for (int j = 0; j < R; ++j) {
@@ -690,15 +709,16 @@ __device__ __forceinline__ void score_rows(const bf16_t *reps, int64_t rep_strid
         __syncthreads();
         unsigned int *const ticket = job.ticket ? job.ticket : &retrieval_tickets[job.slot];
         if (threadIdx.x == 0) {
-            const unsigned int drawn = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned int drawn = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             is_last = drawn == (unsigned int)n_wgs - 1;
         }
         __syncthreads();
         if (!is_last) return;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        asm volatile("" ::: "memory");
         if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (N <= 16 * kRetrThreads) select_topk_block<1>(scores, N, job.k, job.idx, job.idx2);
-        else select_topk_block<2>(scores, N, job.k, job.idx, job.idx2);
+        if (N <= 4 * kRetrThreads) select_topk_block<4>(scores, N, job.k, job.idx, job.idx2);
+        else if (N <= 16 * kRetrThreads) select_topk_block<16>(scores, N, job.k, job.idx, job.idx2);
+        else select_topk_block<32>(scores, N, job.k, job.idx, job.idx2);
         publish(job.flag, job.flag_value);
     }
 }
@@ -1014,10 +1034,10 @@ int infllm_call_rank_room() { return kCallRankEntries; }
 
 // select_topk_block over several tables, one workgroup each (table t at scores + t * scores_xs, its ids to
 // idx_out + t * idx_xs)
-template <int NB>
+template <int R>
 __global__ __launch_bounds__(kRetrThreads) void select_rows_kernel(const float *scores, int N, int k, int32_t *idx_out, int64_t scores_xs,
                                                                    int64_t idx_xs) {
-    select_topk_block<NB>(scores + blockIdx.x * scores_xs, N, k, idx_out + blockIdx.x * idx_xs, nullptr);
+    select_topk_block<R>(scores + blockIdx.x * scores_xs, N, k, idx_out + blockIdx.x * idx_xs, nullptr);
 }
 
 // Scores of the same N rows under several queries, every row read once per group of QG queries: the group's queries
@@ -1137,9 +1157,9 @@ extern "C" int infllm_score_topk_queries(const void *d_reps, int64_t rep_stride,
     INFLLM_CHECK_LAUNCH("score_topk_queries");
     if (N > 32 * kRetrThreads || k > 64) return launch_topk(d_scores, N, k, d_idx, nullptr, nullptr, 0, n_queries, scores_qs, idx_qs, stream);
     if (N <= 16 * kRetrThreads)
-        hipLaunchKernelGGL(select_rows_kernel<1>, dim3(n_queries), dim3(kRetrThreads), 0, (hipStream_t)stream, d_scores, N, k, d_idx, scores_qs, idx_qs);
+        hipLaunchKernelGGL(select_rows_kernel<16>, dim3(n_queries), dim3(kRetrThreads), 0, (hipStream_t)stream, d_scores, N, k, d_idx, scores_qs, idx_qs);
     else
-        hipLaunchKernelGGL(select_rows_kernel<2>, dim3(n_queries), dim3(kRetrThreads), 0, (hipStream_t)stream, d_scores, N, k, d_idx, scores_qs, idx_qs);
+        hipLaunchKernelGGL(select_rows_kernel<32>, dim3(n_queries), dim3(kRetrThreads), 0, (hipStream_t)stream, d_scores, N, k, d_idx, scores_qs, idx_qs);
     INFLLM_CHECK_LAUNCH("score_topk_queries (selection)");
     return 0;
 }
