@@ -514,8 +514,9 @@ __device__ __forceinline__ void select_topk_block(const float *scores, int N, in
     for (int o = 16; o < groups; o <<= 1) tau = min(tau, (uint32_t)__shfl_xor(tau, o, 64));
     // Of 64 groups that lets five times k units pass, and their ranking by counting is longer than all else: every wave halves the way
     // up to the largest, until k of the threads' best are above and at most an eighth more.  (64 best of 1,000 / 16,384 units with rows of
-    // 4,096: 17.3 / 34.1 -> 11.9 / 30.1 us; of 64 units, where nothing is to be gained, 10.3 -> 11.5, so not of a few.)
-    if (k > 16 && N > 2 * groups) {
+    // 4,096: 17.3 / 34.1 -> 11.9 / 30.1 us.  With and without, rows of 512: 64 best of 146 / 256 / 512 / 3,000 units 7.1 and 6.2, 7.3 and 7.4,
+    // 6.9 and 7.7, 10.1 and 12.9; 32 of 256 / 800 / 1,500 / 3,000 6.4 and 5.6, 7.2 and 6.8, 8.3 and 8.3, 9.6 and 10.6.)
+    if (k > 16 && N > (groups == 64 ? 256 : 1024)) {
         uint32_t lo = __builtin_amdgcn_readfirstlane(tau), hi = top;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) hi = max(hi, (uint32_t)__shfl_xor(hi, o, 64));
