@@ -171,7 +171,8 @@ PyObject *py_step(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     if (!q || !old_k || old_k->dim() != 4) Py_RETURN_NONE;
     const int64_t rows_old = old_k->size(2), seen = PyLong_AsLongLong(PyTuple_GET_ITEM(past, 2)), rows_all = rows_old + 1, len_k = seen + 1;
     if (PyErr_Occurred()) return nullptr;
-    if (rows_old < 1 || rows_old >= INT32_MAX || !rows_of(q, *q, batch, heads * dim) || !rows_of(k, *q, batch, kv_heads * dim) || !rows_of(v, *q, batch, kv_heads * dim) ||
+    if (n_init < 0 || n_init > INT32_MAX || rows_old < 1 || rows_old >= INT32_MAX || !rows_of(q, *q, batch, heads * dim) ||
+        !rows_of(k, *q, batch, kv_heads * dim) || !rows_of(v, *q, batch, kv_heads * dim) ||
         !cached_of(old_k, *q, batch, kv_heads, rows_old, dim) || !cached_of(old_v, *q, batch, kv_heads, rows_old, dim))
         Py_RETURN_NONE;
     if (!freq || freq->device() != q->device() || freq->scalar_type() != at::kFloat || freq->numel() != dim / 2 || !freq->is_contiguous()) Py_RETURN_NONE;
@@ -186,11 +187,7 @@ PyObject *py_step(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     bool fits = words && PyTuple_CheckExact(words) && PyTuple_GET_SIZE(words) == 6;
     for (int i = 0; fits && i < 4; ++i) held[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(words, i + 2));
     fits = fits && !PyErr_Occurred() && held[0] >= batch * heads && held[1] == stream && held[3] >= step_bytes;
-    at::Tensor new_k, new_v;
-    if (fits && !cut) {
-        fits = claim(*old_k, *old_v, 1, stream);
-        if (fits) std::tie(new_k, new_v) = grown(*old_k, *old_v, 1);
-    }
+    if (fits && !cut) fits = claim(*old_k, *old_v, 1, stream);
     if (!fits) {
         Py_DECREF(dict);
         if (PyErr_Occurred()) return nullptr;
@@ -204,6 +201,7 @@ PyObject *py_step(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
         ~Held() { Py_DECREF(o); }
     } words_held{words};
     if (bad) return nullptr;
+    // (behind this point other threads may run: views and tensors are made by torch's dispatcher, which can be a Python mode's)
     PyObject *address = PyObject_CallFunctionObjArgs(args[16], words, nullptr);
     if (!address) return nullptr;
     void *const ticket = PyLong_AsVoidPtr(address);
@@ -212,7 +210,9 @@ PyObject *py_step(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
 
     const auto options = at::TensorOptions().dtype(at::kBFloat16).device(q->device());
     const int64_t rows_new = cut ? n_init + n_local : rows_all;
-    if (cut) {
+    at::Tensor new_k, new_v;
+    if (!cut) std::tie(new_k, new_v) = grown(*old_k, *old_v, 1);
+    else {
         const at::Tensor cache = at::empty({2, batch, kv_heads, rows_new, dim}, options);
         new_k = cache.select(0, 0);
         new_v = cache.select(0, 1);

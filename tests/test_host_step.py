@@ -92,3 +92,42 @@ def test_failures_and_other_inputs():
         host.claim(None, None, 1, 0)
     t = torch.zeros((1, 2, 3, 4))
     assert host.claim(t, t, 1, 0) is None
+
+
+class Other(torch.utils._python_dispatch.TorchDispatchMode):
+    """runs `work` at the first view or tensor that a call makes"""
+    def __init__(self, work):
+        super().__init__()
+        self.work = work
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        work, self.work = self.work, lambda: None
+        work()
+        return func(*args, **(kwargs or {}))
+
+
+def plain_step(n_init, mode=None):
+    """one native step behind three tokens: (what it returns, its native calls, the storage of its cache)"""
+    host, H, D, calls = _lib.host(), 2, 64, []
+    both = torch.zeros((2, 1, H, 8, D), dtype=torch.bfloat16)
+    host.make_room(both, 3, 0)
+    k, v = both.narrow(3, 0, 3).unbind(0)
+    storage = k.untyped_storage()
+    storage._infllm_words = (torch.zeros(64, dtype=torch.int32), 64, H, 0, 128, 1 << 20)
+    rows = [torch.zeros((1, 1, H * D), dtype=torch.bfloat16) for _ in range(3)]
+    args = (1, 40, n_init, *rows, (k, v, 3, None), ROPE[D].inv_freq, 1.0, 1, H, H, D, 1 << 10, 0, lambda a, s: calls.append(a) or 0, lambda words: words[1])
+    with mode(storage) if mode else torch.no_grad():
+        return host.step(*args), calls, storage
+
+
+def test_sizes_that_the_argument_block_does_not_hold():
+    assert plain_step(8)[0] is not None
+    for n in (-1, 1 << 31, 1 << 40):
+        got, calls, storage = plain_step(n)
+        assert got is None and not calls and storage._infllm_words is not None      # (the general way refuses it)
+
+
+def test_words_are_taken_before_other_code_runs():
+    seen = []
+    got, calls, _ = plain_step(8, lambda storage: Other(lambda: seen.append("_infllm_words" in storage.__dict__)))
+    assert seen == [False] and got is not None and len(calls) == 1
