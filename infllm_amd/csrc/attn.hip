@@ -150,9 +150,11 @@ struct KernargLayout {                     // the arguments as the launch lays t
 // Heads of 64 leave room for two workgroups on a CU: half the accumulators and operands fit 128 registers (four waves per
 // SIMD), the tiles 64 KB.  Their arithmetic per tile is bound by the exponentials (32 of 16 cycles a wave against 512 cycles
 // of MFMA), and within one wave the two only add up; with four waves one's MFMAs run under another's exponentials (36 heads,
-// prompt of 24,300 tokens, with the scores' smaller workgroups: 4474 -> 3550 us a pass).
-template <int D, int MODE>
-constexpr int kWgsPerCu = D == 64 && (MODE == kLinear || MODE == kPaged) ? 2 : 1;
+// prompt of 24,300 tokens, with the scores' smaller workgroups: 4474 -> 3550 us a pass).  The sinks' form, which took 129 registers when
+// it was given more, fits as well: sinks + window of 2,048 over 16,001 tokens 773 -> 649 us, of 512 over 7,596 172 -> 147, 4 batch rows of
+// 4,096 in a window of 4,000 667 -> 543.
+template <int D>
+constexpr int kWgsPerCu = D == 64 ? 2 : 1;
 
 // BASE2: the queries come with the softmax scale and log2(e) in them (types with a window, heads of 128), multiplied in where they are
 // rotated, ahead of their one rounding to bf16: their products with keys are logits to base 2.  The linear form starts the products
@@ -161,7 +163,7 @@ constexpr int kWgsPerCu = D == 64 && (MODE == kLinear || MODE == kPaged) ? 2 : 1
 // max and adds it.  Causal prompt of 8,001 tokens, 32 / 8 heads: 533 -> 521.5 us, sinks + window of 4,096 over 16,001 1,037.5 -> 1,026.5.
 // (The streaming memory's queries stay as they are: 128K tokens 1.5 % faster so, 24,300 of 36 heads of 64 0.5 %.)
 template <int D, int MODE, bool INLINE = false, bool BASE2 = false>
-__global__ __launch_bounds__(kThreads, (2 * kWgsPerCu<D, MODE>)) void attn_stage_kernel(infllm_attn_args a, infllm_attn_args a2, StageGeom geo,
+__global__ __launch_bounds__(kThreads, 2 * kWgsPerCu<D>) void attn_stage_kernel(infllm_attn_args a, infllm_attn_args a2, StageGeom geo,
                                                                  std::conditional_t<INLINE, InlinePages, NoInlinePages>) {
     constexpr bool HAS_LIN = MODE != kPaged, HAS_PAG = MODE != kLinear, SINKS = MODE == kSinks || MODE == kSinksStaged, TWO = MODE == kBoth || SINKS;
     constexpr int kRow = D * 2, kTB = kTileBytes<D>;                     // bytes of a row, of a tile
