@@ -161,7 +161,8 @@ constexpr int kWgsPerCu = D == 64 ? 2 : 1;
 // from less the running max (kFromMax), and a probability is an exponential and nothing else: the multiply-add that every score took
 // went into the power of the card, which lowers its clock under this loop.  The sinks' form has no registers for the 16 that hold the
 // max and adds it.  Causal prompt of 8,001 tokens, 32 / 8 heads: 533 -> 521.5 us, sinks + window of 4,096 over 16,001 1,037.5 -> 1,026.5.
-// (The streaming memory's queries stay as they are: 128K tokens 1.5 % faster so, 24,300 of 36 heads of 64 0.5 %.)
+// (The streaming memory's queries do not take it along, though 128K tokens would be 1.5 % faster with it, 24,300 of 36 heads of 64 0.5 %:
+// they would round otherwise than those of its steps, which the same cache is selected and scored by.)
 template <int D, int MODE, bool INLINE = false, bool BASE2 = false>
 __global__ __launch_bounds__(kThreads, 2 * kWgsPerCu<D>) void attn_stage_kernel(infllm_attn_args a, infllm_attn_args a2, StageGeom geo,
                                                                  std::conditional_t<INLINE, InlinePages, NoInlinePages>) {
