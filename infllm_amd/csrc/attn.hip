@@ -156,19 +156,15 @@ struct KernargLayout {                     // the arguments as the launch lays t
 template <int D>
 constexpr int kWgsPerCu = D == 64 ? 2 : 1;
 
-// BASE2: the queries come with the softmax scale and log2(e) in them (types with a window, heads of 128), multiplied in where they are
-// rotated, ahead of their one rounding to bf16: their products with keys are logits to base 2.  The linear form starts the products
-// from less the running max (kFromMax), and a probability is an exponential and nothing else: the multiply-add that every score took
-// went into the power of the card, which lowers its clock under this loop.  The sinks' form has no registers for the 16 that hold the
-// max and adds it.  Causal prompt of 8,001 tokens, 32 / 8 heads: 533 -> 521.5 us, sinks + window of 4,096 over 16,001 1,037.5 -> 1,026.5.
-// (The streaming memory's queries do not take it along, though 128K tokens would be 1.5 % faster with it, 24,300 of 36 heads of 64 0.5 %:
-// they would round otherwise than those of its steps, which the same cache is selected and scored by.)
-template <int D, int MODE, bool INLINE = false, bool BASE2 = false>
+// The softmax scale is applied to products, in 32 bits.  In the queries, ahead of their rounding, it saves a score its multiply-add (causal,
+// 8,001 tokens, 526 us, 518 so; sinks + window of 4,096 over 16,001 1,022 and 1,014) and costs exactness: pairs that are hardly turned lose
+// little as they are rounded, and would as much as all others.  N(0, 1) rows, 1,500 tokens, base 1e6: outputs 2.69e-3 off 64 bits, 2.78e-3
+// so; hardly any pair turned 2.16e-3 and 2.52e-3, and with logits up to 70 4.0e-3 and 6.4e-3.
+template <int D, int MODE, bool INLINE = false>
 __global__ __launch_bounds__(kThreads, 2 * kWgsPerCu<D>) void attn_stage_kernel(infllm_attn_args a, infllm_attn_args a2, StageGeom geo,
                                                                  std::conditional_t<INLINE, InlinePages, NoInlinePages>) {
     constexpr bool HAS_LIN = MODE != kPaged, HAS_PAG = MODE != kLinear, SINKS = MODE == kSinks || MODE == kSinksStaged, TWO = MODE == kBoth || SINKS;
     constexpr int kRow = D * 2, kTB = kTileBytes<D>;                     // bytes of a row, of a tile
-    constexpr bool kFromMax = BASE2 && D == 128 && !TWO;
     constexpr bool PING = D == 128, kTurns = D == 128 && (MODE == kLinear || MODE == kSinks);
     const infllm_attn_args &ap = TWO ? a2 : a;                 // the paged stage's arguments
     extern __shared__ __attribute__((aligned(1024))) char lds_dyn[];    // kStages K tiles, then kStages V tiles
@@ -401,16 +397,13 @@ __global__ __launch_bounds__(kThreads, 2 * kWgsPerCu<D>) void attn_stage_kernel(
 
     // ---- running softmax state of this lane's query (max kept in raw logit units, allowed to lag)
     float m_run = -INFINITY, m_limit = -INFINITY, l_run = 0.f, neg_ms = 0.f;
-    [[maybe_unused]] f32x16 from_max;         // kFromMax: what scores are taken from, 16 times less the max; 0 as long as there is none
-#pragma unroll
-    for (int r = 0; r < 16; ++r) from_max[r] = 0.f;
     f32x16 oacc[D / 32];
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
 
-    const float scale = BASE2 ? 1.f : geo.scale, lazy = kLazyLog2 / scale;
+    const float scale = geo.scale, lazy = kLazyLog2 / scale;
     typedef short s16x8 __attribute__((ext_vector_type(8)));
     // kb / vb: k_off / v_off in the tile's buffer
     auto k_operand = [&](uint32_t kb, int kk, int ks) {
@@ -506,20 +499,7 @@ __global__ __launch_bounds__(kThreads, 2 * kWgsPerCu<D>) void attn_stage_kernel(
         // lazy running max: it only moves when a score would exceed it by more than 2^kLazyLog2 after scaling,
         // so the rescale of the output accumulators is rare; probabilities stay below 2^kLazyLog2
         const bool moved = tmax > m_limit;
-        if constexpr (kFromMax) {                // (scores are less the max already)
-            if (__builtin_amdgcn_ballot_w64(moved) != 0) {
-                const float by = moved ? tmax : 0.f;
-                const float al = !moved ? 1.f : m_limit == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(-by);
-                m_limit = moved ? kLazyLog2 : m_limit;
-                l_run *= al;
-#pragma unroll
-                for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) oacc[dt][r] *= al;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) from_max[r] -= by, s[0][r] -= by, s[1][r] -= by;
-            }
-        } else if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+        if (__builtin_amdgcn_ballot_w64(moved) != 0) {
             const float m_new = moved ? tmax : m_run;
             const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale);      // exp2(-inf) = 0 on the first move
             const float al = moved ? alpha : 1.f;
@@ -710,8 +690,8 @@ __global__ __launch_bounds__(kThreads, 2 * kWgsPerCu<D>) void attn_stage_kernel(
     auto exps = [&](int ks, int r0, int r1) {
 #pragma unroll
         for (int r = r0; r < r1; r += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(kFromMax ? s[ks][r] : __builtin_fmaf(s[ks][r], scale, neg_ms));
-            const float p1 = __builtin_amdgcn_exp2f(kFromMax ? s[ks][r + 1] : __builtin_fmaf(s[ks][r + 1], scale, neg_ms));
+            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[ks][r], scale, neg_ms));
+            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[ks][r + 1], scale, neg_ms));
             pw[ks][r >> 1] = pack_bf16x2(p0, p1);
             asm volatile("" : "+v"(pw[ks][r >> 1]));                                // formed here, not where it is read
         }
@@ -744,19 +724,17 @@ __global__ __launch_bounds__(kThreads, 2 * kWgsPerCu<D>) void attn_stage_kernel(
     };
     // S = K.Q of this tile; its first 8 operands are on their way
     auto qk_mul = [&](uint32_t kb) {
-        if constexpr (!kFromMax)
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
+        for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[ks][r] = 0.f;
+            for (int r = 0; r < 16; ++r) s[ks][r] = 0.f;
 #pragma unroll
         for (int g = 4; g < 8; ++g) {
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int i = 4 * g + j;
-                s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, op[i & 7]), qreg[((i - 16) >> 1) % (D / 16)],
-                                                                   kFromMax && i < 18 ? from_max : s[i & 1], 0, 0, 0);
+                s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, op[i & 7]), qreg[((i - 16) >> 1) % (D / 16)], s[i & 1], 0, 0, 0);
                 if (i + 8 < 32) request(i + 8, 0, kb);
             }
             if (g < 6) {
@@ -1015,7 +993,7 @@ __global__ __launch_bounds__(kThreads, 2 * kWgsPerCu<D>) void attn_stage_kernel(
         }
     }
     if (qi >= a.Lq) return;
-    if (grp == 0) a.d_lse_part[row] = l_tot > 0.f ? (kFromMax ? -from_max[0] : m_run * scale) + log2f(l_tot) : -INFINITY;
+    if (grp == 0) a.d_lse_part[row] = l_tot > 0.f ? m_run * scale + log2f(l_tot) : -INFINITY;
 }
 
 // one thread per (row, 8 dims): P fp16 partials -> bf16 output row + final lse (merge_piece, common.h)
@@ -1182,16 +1160,16 @@ struct StageOut {
     const float2 *q_angles = nullptr, *sink_angle = nullptr;
 };
 
-template <int D, int MODE, bool INLINE, bool BASE2, typename Pages>
+template <int D, int MODE, bool INLINE, typename Pages>
 int launch_mode(dim3 grid, const infllm_attn_args &a, const infllm_attn_args &a2, const StageGeom &geo, const Pages &pages, void *stream) {
     constexpr size_t lds_bytes = 2 * kStages * kTileBytes<D>;
     static std::atomic<bool> lds_set{false};                  // dynamic LDS above 64 KiB must be enabled once per kernel
     if (!lds_set.load(std::memory_order_acquire)) {
-        const hipError_t e = hipFuncSetAttribute((const void *)attn_stage_kernel<D, MODE, INLINE, BASE2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+        const hipError_t e = hipFuncSetAttribute((const void *)attn_stage_kernel<D, MODE, INLINE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
         if (e != hipSuccess) return infllm_fail(-2, "attn_stage: %s", hipGetErrorString(e));
         lds_set.store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL((attn_stage_kernel<D, MODE, INLINE, BASE2>), grid, dim3(kThreads), lds_bytes, (hipStream_t)stream, a, a2, geo, pages);
+    hipLaunchKernelGGL((attn_stage_kernel<D, MODE, INLINE>), grid, dim3(kThreads), lds_bytes, (hipStream_t)stream, a, a2, geo, pages);
     INFLLM_CHECK_LAUNCH("attn_stage");
     return 0;
 }
@@ -1212,26 +1190,22 @@ int launch_stage(int mode, const infllm_attn_args *a, const infllm_attn_args *a2
     // tile indices stay below 2^30, so any ring of 2^31 tiles or more never wraps: one divisor stands for all of them
     if (mode != kPaged) geo.cap_tiles = fast_div((uint32_t)std::min<int64_t>(a->cap / kTile, 1ll << 31));
     const infllm_attn_args &second = a2 ? *a2 : *a;
-    const bool base2 = geo.scale == 1.f;
     if (h_pages) {
         const infllm_attn_args &pg = mode == kBoth ? second : *a;
         INFLLM_REQUIRE((mode == kPaged || mode == kBoth) && pg.n_pages >= 0 && (int64_t)pg.B * pg.n_pages <= kInlinePages,
                        "attn_stage: %d x %d pages do not fit a launch", pg.B, pg.n_pages);
         InlinePages table;
         memcpy(table.p, h_pages, sizeof(infllm_page) * pg.B * pg.n_pages);
-        if (mode == kBoth) return launch_mode<D, kBoth, true, false>(grid, *a, second, geo, table, stream);
-        return launch_mode<D, kPaged, true, false>(grid, *a, second, geo, table, stream);
+        return mode == kPaged ? launch_mode<D, kPaged, true>(grid, *a, second, geo, table, stream)
+                              : launch_mode<D, kBoth, true>(grid, *a, second, geo, table, stream);
     }
     constexpr NoInlinePages none{};
-    constexpr bool kForms = D == 128;                // (of heads of 64 the types with a window scale their scores too)
-    INFLLM_REQUIRE(!kForms || base2 || (mode != kSinks && mode != kSinksStaged), "attn_stage: sinks of queries without the softmax scale");
     switch (mode) {
-        case kLinear: return kForms && base2 ? launch_mode<D, kLinear, false, kForms>(grid, *a, second, geo, none, stream)
-                                             : launch_mode<D, kLinear, false, false>(grid, *a, second, geo, none, stream);
-        case kPaged: return launch_mode<D, kPaged, false, false>(grid, *a, second, geo, none, stream);
-        case kBoth: return launch_mode<D, kBoth, false, false>(grid, *a, second, geo, none, stream);
-        case kSinks: return launch_mode<D, kSinks, false, kForms>(grid, *a, second, geo, none, stream);
-        default: return launch_mode<D, kSinksStaged, false, kForms>(grid, *a, second, geo, none, stream);
+        case kLinear: return launch_mode<D, kLinear, false>(grid, *a, second, geo, none, stream);
+        case kPaged: return launch_mode<D, kPaged, false>(grid, *a, second, geo, none, stream);
+        case kBoth: return launch_mode<D, kBoth, false>(grid, *a, second, geo, none, stream);
+        case kSinks: return launch_mode<D, kSinks, false>(grid, *a, second, geo, none, stream);
+        default: return launch_mode<D, kSinksStaged, false>(grid, *a, second, geo, none, stream);
     }
 }
 

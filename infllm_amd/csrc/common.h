@@ -23,10 +23,6 @@ constexpr int kTile = INFLLM_KEY_TILE;    // keys per tile
 constexpr int kInlinePages = 64;          // page table entries that a launch of the paged stage can carry
 constexpr int kWave = 64;
 constexpr float kLog2e = 1.4426950408889634f;
-// The softmax scale that goes with queries that were rounded with their scale and log2(e) in them, whose products with keys are logits
-// to base 2 (the attention kernel has forms without the multiplication).
-constexpr float kBase2Scale = 0.69314718055994531f;
-static_assert(kBase2Scale * kLog2e == 1.f, "log2(e) times log(2)");
 
 // thread-local error text, returned by infllm_last_error()
 char *infllm_err_buf();

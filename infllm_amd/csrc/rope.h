@@ -9,8 +9,8 @@ struct Rot8 {
 };
 
 // rotate 8 pairs (lo[i], hi[i]) by (c[i], s[i]); fp32 math, one rounding to bf16.  `raw` (optional) receives the 16
-// rotated values before that rounding: lo pairs first, then hi pairs.  `by`: what the rounded ones are multiplied with ahead of it.
-__device__ __forceinline__ Rot8 rotate8(u32x4 xlo, u32x4 xhi, const float2 *cs, float *raw = nullptr, float by = 1.f) {
+// rotated values before that rounding: lo pairs first, then hi pairs.
+__device__ __forceinline__ Rot8 rotate8(u32x4 xlo, u32x4 xhi, const float2 *cs, float *raw = nullptr) {
     Rot8 r;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
@@ -20,8 +20,8 @@ __device__ __forceinline__ Rot8 rotate8(u32x4 xlo, u32x4 xhi, const float2 *cs, 
         // x*cos + rotate_half(x)*sin, rotate_half = (-hi, lo)
         const float l0 = a0 * c0.x - b0 * c0.y, l1 = a1 * c1.x - b1 * c1.y;
         const float h0 = b0 * c0.x + a0 * c0.y, h1 = b1 * c1.x + a1 * c1.y;
-        r.lo[w] = pack_bf16x2(l0 * by, l1 * by);
-        r.hi[w] = pack_bf16x2(h0 * by, h1 * by);
+        r.lo[w] = pack_bf16x2(l0, l1);
+        r.hi[w] = pack_bf16x2(h0, h1);
         if (raw) {
             raw[2 * w] = l0, raw[2 * w + 1] = l1;
             raw[8 + 2 * w] = h0, raw[8 + 2 * w + 1] = h1;

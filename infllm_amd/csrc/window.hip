@@ -20,7 +20,6 @@ struct StageJob {
     const float *inv_freq;
     double distance_scale;
     bf16_t *q_loc, *q_glb;                     // [B, H, n, D]; q_glb NULL: not wanted
-    float q_scale;                             // what rotated queries (or the angles by which they will be) are multiplied with
     float2 *pos_cs;                            // [n, D / 2] cosine and sine of every position and frequency (NULL: not wanted)
     float2 *glb_cs;                            // cosine and sine of every frequency at the sinks' angle (NULL: not wanted)
     bf16_t *dk, *dv;                           // where row 0 of head 0 goes, rotated / as it is
@@ -92,8 +91,8 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
     rope_angles<HALF>(j.pos0 + p0, np, j.glb_pos, j.distance_scale, freq, cs_pos, cs_glb);
     __syncthreads();
     if (j.pos_cs && b == 0 && g0 == 0)
-        for (int i = tid; i < np * HALF; i += 256) j.pos_cs[(int64_t)p0 * HALF + i] = make_float2(cs_pos[0][i].x * j.q_scale, cs_pos[0][i].y * j.q_scale);
-    if (j.glb_cs && blockIdx.x == 0 && b == 0 && g0 == 0 && tid < HALF) j.glb_cs[tid] = make_float2(cs_glb[tid].x * j.q_scale, cs_glb[tid].y * j.q_scale);
+        for (int i = tid; i < np * HALF; i += 256) j.pos_cs[(int64_t)p0 * HALF + i] = cs_pos[0][i];
+    if (j.glb_cs && blockIdx.x == 0 && b == 0 && g0 == 0 && tid < HALF) j.glb_cs[tid] = cs_glb[tid];
     if (j.do_q) {
         for (int hg0 = 0; hg0 < n_heads; hg0 += 4) {
 #pragma unroll
@@ -106,11 +105,11 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(StageJob j) {
                     lo = *(const u32x4 *)(src + qc * 8), hi = *(const u32x4 *)(src + HALF + qc * 8);
                 }
                 const int64_t o = (((int64_t)b * j.H + h0 + hl) * j.n + p0 + qp) * D;
-                Rot8 r = rotate8(lo, hi, &cs_pos[qp][qc * 8], nullptr, j.q_scale);
+                Rot8 r = rotate8(lo, hi, &cs_pos[qp][qc * 8]);
                 *(u32x4 *)(j.q_loc + o + qc * 8) = r.lo;
                 *(u32x4 *)(j.q_loc + o + HALF + qc * 8) = r.hi;
                 if (j.q_glb) {
-                    r = rotate8(lo, hi, &cs_glb[qc * 8], nullptr, j.q_scale);
+                    r = rotate8(lo, hi, &cs_glb[qc * 8]);
                     *(u32x4 *)(j.q_glb + o + qc * 8) = r.lo;
                     *(u32x4 *)(j.q_glb + o + HALF + qc * 8) = r.hi;
                 }
@@ -249,9 +248,6 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     j.glb_pos = a->kind == 2 ? a->n_local - 1 : a->n_local + a->n_init - 1;
     j.inv_freq = a->d_inv_freq; j.distance_scale = a->distance_scale;
     j.q_loc = q_loc;
-    // Several queries of heads of 128 take the softmax scale along, and their logits are to base 2 (BASE2, attn.hip); a step scales its own.
-    const bool base2 = D == 128 && !step;
-    j.q_scale = base2 ? a->softmax_scale * kLog2e : 1.f;
     // Queries are rotated to the sinks' angle where they are attended, by a table of it in their place, which two rows fill and one
     // row does not hold.
     const bool sink_turns = sink_stage && !step && rows_q >= 2;
@@ -405,7 +401,7 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
     l.window = causal ? rows_base : a->n_local;
     l.j_lo = std::max<int64_t>(0, rows_base - a->n_q - l.window + 1);
     l.j_hi = rows_base;
-    l.softmax_scale = base2 ? kBase2Scale : scale;
+    l.softmax_scale = scale;
     if (sink_stage) {
         s = l;
         if (sink_turns) {

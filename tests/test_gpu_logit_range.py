@@ -1,8 +1,9 @@
-"""Logits far from zero: scores start from less the running max, which moves by hundreds of powers of two - rows whose keys' logits all lie
+"""Logits far from zero: the running max moves by hundreds of powers of two - rows whose keys' logits all lie
 high or low, keys whose logits rise or fall by more than the range of an exponent behind each other, one key above or below all others.
 
 Against a dense softmax in 64 bits over the same bf16 inputs, or the oracle's in 32 bits, max-abs 2e-2 / mean-abs 2e-3 as in the other
-tests: products of up to 300 are summed in 32 bits to 300 x 2^-22 at worst, 1e-4 of a probability."""
+tests: products of up to 300 are summed in 32 bits by 8 MFMAs in a row (of 16 elements), whose sums round by
+300 x 2^-24 each: 1.4e-4 of a probability at worst."""
 import pytest
 import torch
 
