@@ -251,21 +251,22 @@ class InfLLMHipError(RuntimeError):
 
 
 def host():
-    """The extension module of csrc/host.cpp: the host side of a step of the attention types with a plain cache."""
+    """The extension module of csrc/host.cpp: the host side of a step of the attention types with a plain cache.  Nothing else needs it."""
     global _host
     if _host is None:
-        import torch  # noqa: F401  (whose libraries the module is linked against)
+        lib = load()                       # (which imports torch, whose libraries the module is linked against)
         try:
             from . import _host as module
         except ImportError as e:
             raise InfLLMHipError(f"infllm_amd/_host.so cannot be loaded ({e}): build it with `python -m infllm_amd.build`") from e
+        module.bind(lib.infllm_window_forward, C.cast(lib.infllm_window_forward, c_vp).value)
         _host = module
     return _host
 
 
 def load():
     """Load the shared library once; raise if it is absent or incomplete."""
-    global _lib
+    global _lib, _host
     if _lib is not None:
         return _lib
     # One HIP runtime (and one ROCr) per process: PyTorch bundles its own and every device pointer handed to the library
@@ -284,8 +285,7 @@ def load():
         fn.restype, fn.argtypes = restype, argtypes
     if lib.infllm_version() != ABI_VERSION:
         raise InfLLMHipError(f"ABI version {lib.infllm_version()} != expected {ABI_VERSION}; rebuild the library")
-    host().bind(lib.infllm_window_forward, C.cast(lib.infllm_window_forward, c_vp).value)
-    _lib = lib
+    _lib, _host = lib, None                # (the extension module is bound to this library's functions when it is asked for)
     return lib
 
 
