@@ -254,12 +254,13 @@ def host():
     """The extension module of csrc/host.cpp: the host side of a step of the attention types with a plain cache.  Nothing else needs it."""
     global _host
     if _host is None:
-        lib = load()                       # (which imports torch, whose libraries the module is linked against)
+        import torch                       # (whose libraries the module is linked against)
+        lib = load()
         try:
             from . import _host as module
-        except ImportError as e:
-            raise InfLLMHipError(f"infllm_amd/_host.so cannot be loaded ({e}): build it with `python -m infllm_amd.build`") from e
-        module.bind(lib.infllm_window_forward, C.cast(lib.infllm_window_forward, c_vp).value)
+            module.bind(lib.infllm_window_forward, C.cast(lib.infllm_window_forward, c_vp).value, ABI_VERSION, C.sizeof(WindowArgs), torch.__version__)
+        except (ImportError, TypeError) as e:              # (TypeError: one from before it compared anything)
+            raise InfLLMHipError(f"infllm_amd/_host.so cannot be used ({e}): build it with `python -m infllm_amd.build`") from e
         _host = module
     return _host
 

@@ -51,7 +51,8 @@ def build_host(verbose=True):
     if not cxx:
         raise RuntimeError("no C++ compiler found (set CXX)")
     include = [sysconfig.get_paths()["include"], *cpp_extension.include_paths()]
-    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-I{p}" for p in include],
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          f'-DINFLLM_TORCH_VERSION="{torch.__version__}"', *[f"-I{p}" for p in include],
           os.path.join(CSRC, "host.cpp"), "-o", HOST_PATH, *[f"-L{p}" for p in cpp_extension.library_paths()], "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"],
          verbose)
     return HOST_PATH

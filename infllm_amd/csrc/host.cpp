@@ -131,14 +131,21 @@ PyObject *py_claim(PyObject *, PyObject *const *args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// bind(infllm_window_forward, its address): what step calls by itself when it is given this object
+// bind(infllm_window_forward, its address, ABI version, size of its argument block, torch's version): what step calls by itself when it is
+// given this object.  The block is filled here as this file was compiled with it, and torch's objects are read as that torch lays them out:
+// a module of another build is refused.
 PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
-    if (n != 2) {
-        PyErr_SetString(PyExc_TypeError, "bind(function, address)");
+    if (n != 5) {
+        PyErr_SetString(PyExc_TypeError, "bind(function, address, ABI version, size of the argument block, torch's version)");
         return nullptr;
     }
     void *address = PyLong_AsVoidPtr(args[1]);
-    if (PyErr_Occurred()) return nullptr;
+    const long long version = PyLong_AsLongLong(args[2]), bytes = PyLong_AsLongLong(args[3]);
+    const char *torch_version = PyErr_Occurred() ? nullptr : PyUnicode_AsUTF8(args[4]);
+    if (!torch_version) return nullptr;
+    if (version != INFLLM_ABI_VERSION || bytes != (long long)sizeof(infllm_window_args) || std::strcmp(torch_version, INFLLM_TORCH_VERSION) != 0)
+        return PyErr_Format(PyExc_ImportError, "built for ABI version %d with blocks of %zu bytes and torch %s, not for %lld, %lld and %s", INFLLM_ABI_VERSION,
+                            sizeof(infllm_window_args), INFLLM_TORCH_VERSION, version, bytes, torch_version);
     Py_INCREF(args[0]);
     Py_XDECREF(forward_object);
     forward_object = args[0];
@@ -275,6 +282,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 }  // namespace
 
 PyMODINIT_FUNC PyInit__host() {
+    constexpr size_t kMinor = sizeof("3.1") - 1 + (PY_MINOR_VERSION >= 10);             // of "3.10.12"; the file's name names no interpreter
+    if (std::strncmp(Py_GetVersion(), PY_VERSION, kMinor + 1) != 0)
+        return PyErr_Format(PyExc_ImportError, "built for Python %s, not for %s", PY_VERSION, Py_GetVersion());
     room_name = PyUnicode_InternFromString("_infllm_room");
     words_name = PyUnicode_InternFromString("_infllm_words");
     return room_name && words_name ? PyModule_Create(&module) : nullptr;

@@ -34,3 +34,25 @@ def test_it_is_given_the_library_that_is_loaded(fresh):
         lib = _lib.load()
         assert _lib.host() is Module and _lib.host() is Module
         assert seen.pop()[0] is lib.infllm_window_forward and not seen
+
+
+def test_a_module_of_another_build_is_refused(fresh):
+    import torch
+    module, lib, block = _lib.host(), _lib.load(), _lib.C.sizeof(_lib.WindowArgs)
+    told = [lib.infllm_window_forward, 1, _lib.ABI_VERSION, block, torch.__version__]
+    for i, other in ((2, _lib.ABI_VERSION + 1), (3, block + 8), (4, torch.__version__ + "1")):
+        with pytest.raises(ImportError, match="built"):
+            module.bind(*told[:i], other, *told[i + 1:])
+    fresh.setattr(_lib, "_host", None)
+    with fresh.context() as m:                                         # a header that has moved on
+        m.setattr(_lib, "ABI_VERSION", _lib.ABI_VERSION + 1)
+        with pytest.raises(_lib.InfLLMHipError, match="_host.*built"):
+            _lib.host()
+
+    class Older:
+        bind = staticmethod(lambda function, address: None)
+    with fresh.context() as m:
+        m.setattr(infllm_amd, "_host", Older)
+        with pytest.raises(_lib.InfLLMHipError, match="_host"):
+            _lib.host()
+    assert _lib.host() is module
