@@ -43,7 +43,13 @@ def _run(cmd, verbose):
         print(err, file=sys.stderr)
 
 
-def build_host(verbose=True):
+def _library(out, verbose, extra_flags):
+    # ROCr (libhsa-runtime64) is linked for the DMA-engine copy of carved units; in a process it is the copy the HIP
+    # runtime already loaded
+    _run([hipcc_path(), *HIPCC_FLAGS, *extra_flags, *[os.path.join(CSRC, s) for s in SOURCES], "-o", out, "-lhsa-runtime64"], verbose)
+
+
+def _host_module(out, verbose):
     """csrc/host.cpp against the installed torch.  (Its libraries are in the process when the module is imported: no path to them.)"""
     import torch
     from torch.utils import cpp_extension
@@ -53,17 +59,22 @@ def build_host(verbose=True):
     include = [sysconfig.get_paths()["include"], *cpp_extension.include_paths()]
     _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
           f'-DINFLLM_TORCH_VERSION="{torch.__version__}"', *[f"-I{p}" for p in include],
-          os.path.join(CSRC, "host.cpp"), "-o", HOST_PATH, *[f"-L{p}" for p in cpp_extension.library_paths()], "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"],
+          os.path.join(CSRC, "host.cpp"), "-o", out, *[f"-L{p}" for p in cpp_extension.library_paths()], "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"],
          verbose)
-    return HOST_PATH
 
 
 def build(verbose=True, extra_flags=()):
-    # ROCr (libhsa-runtime64) is linked for the DMA-engine copy of carved units; in a process it is the copy the HIP
-    # runtime already loaded
-    cmd = [hipcc_path(), *HIPCC_FLAGS, *extra_flags, *[os.path.join(CSRC, s) for s in SOURCES], "-o", LIB_PATH, "-lhsa-runtime64"]
-    _run(cmd, verbose)
-    build_host(verbose)
+    """Both, or neither: they share include/infllm_hip.h, and one that failed leaves the pair that was there."""
+    new = {path: path[:-len(".so")] + ".new.so" for path in (LIB_PATH, HOST_PATH)}
+    try:
+        _library(new[LIB_PATH], verbose, extra_flags)
+        _host_module(new[HOST_PATH], verbose)
+        for path, made in new.items():
+            os.replace(made, path)
+    finally:
+        for made in new.values():
+            if os.path.exists(made):
+                os.remove(made)
     return LIB_PATH
 
 

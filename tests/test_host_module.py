@@ -56,3 +56,30 @@ def test_a_module_of_another_build_is_refused(fresh):
         with pytest.raises(_lib.InfLLMHipError, match="_host"):
             _lib.host()
     assert _lib.host() is module
+
+
+@pytest.mark.parametrize("broken", ["libinfllm_hip", "_host"])
+def test_a_build_that_fails_leaves_both_as_they_were(broken, tmp_path, monkeypatch):
+    from infllm_amd import build
+    lib, host = tmp_path / "libinfllm_hip.so", tmp_path / "_host.so"
+    monkeypatch.setattr(build, "LIB_PATH", str(lib))
+    monkeypatch.setattr(build, "HOST_PATH", str(host))
+    monkeypatch.setattr(build, "hipcc_path", lambda: "hipcc")
+
+    def run(fail, text):
+        def step(cmd, verbose):
+            out = cmd[cmd.index("-o") + 1]
+            with open(out, "w") as f:
+                f.write(text)
+            if fail and fail in out:
+                raise RuntimeError("no compiler")
+        return step
+    monkeypatch.setattr(build, "_run", run(None, "old"))
+    assert build.build(False) == str(lib)
+    monkeypatch.setattr(build, "_run", run(broken, "new"))
+    with pytest.raises(RuntimeError):
+        build.build(False)
+    assert lib.read_text() == host.read_text() == "old" and len(list(tmp_path.iterdir())) == 2
+    monkeypatch.setattr(build, "_run", run(None, "new"))
+    build.build(False)
+    assert lib.read_text() == host.read_text() == "new" and len(list(tmp_path.iterdir())) == 2
