@@ -1254,7 +1254,7 @@ extern "C" int infllm_attn_stage_splits(const infllm_attn_args *a, int32_t max_s
     int64_t keys = a->d_pages ? (int64_t)a->n_pages * kTile : a->j_hi - a->j_lo;
     if (!a->d_pages && a->mask == INFLLM_MASK_WINDOW) keys = std::min<int64_t>(keys, a->window + kTile);
     keys = std::max<int64_t>(keys, 1);
-    if (a->Lq == 1 && !a->d_pages) return infllm_decode_splits(a->B, a->H, a->Hkv, kD, (keys + kDecodeBlock - 1) / kDecodeBlock, std::min(max_splits, 64));
+    if (a->Lq == 1 && !a->d_pages) return infllm_decode_splits(a->B, a->H, a->Hkv, kD, (keys + kDecodeBlock - 1) / kDecodeBlock, std::min(max_splits, 64), 0, 0);
     const int64_t wgs = ((int64_t)((a->Lq + kQTile - 1) / kQTile) * (a->H / a->Hkv) + kWaves - 1) / kWaves * a->Hkv * a->B;
     const int64_t tiles = (keys + kTile - 1) / kTile;
     return infllm_attn_splits(wgs, tiles, std::min(max_splits, 64), (double)tiles);

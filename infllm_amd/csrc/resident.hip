@@ -480,7 +480,7 @@ int decode_step(Resident *R, const infllm_resident_call *a, int64_t st0, hipStre
     const int far_segs = j.n_seg;
     j.new_logit = (int32_t)(b0 - j_lo);
     ring(d.d_ring_k_rot, j_lo, rides ? b0 : b1, 0, true);
-    j.nsplit = infllm_decode_splits(B, d.H, d.Hkv, d.dim, blocks, j.nsplit, rides ? (int64_t)B * d.Hkv : 0);
+    j.nsplit = infllm_decode_splits(B, d.H, d.Hkv, d.dim, blocks, j.nsplit, rides ? (int64_t)B * d.Hkv : 0, 0);
     j.o_part = a->d_o_part; j.lse_part = a->d_lse_part;
     j.logits = a->d_logits; j.logit_stride = d.n_local;
     if (selects) {

@@ -317,7 +317,7 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
             f.pieces += (j.copy[i].n + kStepCopyRows - 1) / kStepCopyRows;
         }
         d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, D, (near_old + kDecodeBlock - 1) / kDecodeBlock + (far_rows + kDecodeBlock - 1) / kDecodeBlock + 1, max_parts,
-                                        (int64_t)(1 + f.pieces) * a->Hkv * a->B);
+                                        (int64_t)a->Hkv * a->B, (int64_t)f.pieces * a->Hkv * a->B);
         d.o_part = (uint16_t *)((char *)a->d_work + q_bytes);
         d.lse_part = (float *)((char *)a->d_work + q_bytes + part_rows * 2 * D);
         d.out = (bf16_t *)a->d_out; d.out_sb = a->o_sb; d.out_sh = a->o_sh;
@@ -376,7 +376,7 @@ extern "C" int infllm_window_forward(const infllm_window_args *a, void *stream) 
         const int64_t far = far_rows;
         if (far > 0) d.seg[d.n_seg++] = DecodeSeg{sk, bv, sk_sb, sk_sh, bv_sb, bv_sh, (int32_t)far, 1, 0, nullptr, -1};
         const int64_t blocks = (near + kDecodeBlock - 1) / kDecodeBlock + (far > 0 ? (far + kDecodeBlock - 1) / kDecodeBlock : 0);
-        d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, D, blocks, max_parts);
+        d.nsplit = infllm_decode_splits(a->B, a->H, a->Hkv, D, blocks, max_parts, 0, 0);
         d.o_part = (uint16_t *)((char *)a->d_work + q_bytes);
         d.lse_part = (float *)((char *)a->d_work + q_bytes + part_rows * 2 * D);
         d.out = (bf16_t *)a->d_out; d.out_sb = a->o_sb; d.out_sh = a->o_sh;
