@@ -106,4 +106,4 @@ int infllm_decode_step(const DecodeJob *job, const StepRows *rows, int32_t dim, 
 extern "C" int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int32_t dim, int64_t blocks, int32_t max_splits, int64_t rows, int64_t copies);
 int infllm_decode_memory_step(const DecodeJob *job, const infllm_ingest_args *in, int32_t dim, void *stream);
 int infllm_decode_attn(const DecodeJob *job, int32_t dim, void *stream);
-int infllm_decode_lead_splits(int32_t nsplit, int64_t lead_blocks, int64_t blocks);
+extern "C" int infllm_decode_lead_splits(int32_t nsplit, int64_t lead_blocks, int64_t blocks);

@@ -440,7 +440,7 @@ __global__ __launch_bounds__(kDecWaves * kWave, 2) void decode_attn_kernel(Decod
     if constexpr (JOIN) {
         // ---- The split that ends last joins them: a launch of its own is 4.8 us, of which next to nothing is work.  Every split's
         //      stores have been performed before its ticket is drawn, and nothing else crosses workgroups, so that none has to
-        //      write its L2 back.  Wave w takes every fourth split, a lane one head's 8 elements (merge_piece's arithmetic).
+        //      write its L2 back.  Wave w takes every eighth split, a lane one head's 8 elements (merge_piece's arithmetic).
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         __shared__ int last;
@@ -594,7 +594,7 @@ int launch_memory_step(const DecodeJob *job, const infllm_ingest_args *in, void 
 // free by then.  (They were taken off the places before, and nobody counted XCDs: 32 / 8 heads of 128, 16 batch rows behind 2,000 / 4,000 /
 // 16,000 tokens 41.9 / 74.5 / 265 us a step, one split on half of the chip, now 28.9 / 49.6 / 171; 40 / 40 heads, 3 rows behind 8,000 131 and 84;
 // 16 heads of one key head, 8 rows behind 16,000 51.6 with 7 splits, 36.1 with 8; 64 / 8 heads, 6 rows of a full window of 4,096 91.6 and 65.6.
-// Against all counts of splits tried one by one over 1,006 such steps, the estimate takes 2 % longer than the best, 18 % at worst.)
+// Against all counts of splits tried one by one, over 1,006 steps of 13 geometries, the rule takes 2 % longer than the best: 1 % for heads of 128.)
 extern "C" int infllm_decode_splits(int32_t B, int32_t H, int32_t Hkv, int32_t dim, int64_t blocks, int32_t max_splits, int64_t rows, int64_t copies) {
     const int G = H / Hkv, NG = G >= 3 ? 4 : G, chunks = (G + NG - 1) / NG;
     const int64_t wgs = (int64_t)B * Hkv * chunks, places = (dim == 64 ? 512 : 256) - std::min<int64_t>(rows + copies, 128);
@@ -651,16 +651,16 @@ int infllm_decode_memory_step(const DecodeJob *job, const infllm_ingest_args *in
 }
 
 // How many of a launch's splits the ranges get that wait for a selection (lead_blocks of 16 keys) so that they end with the others: the
-// selection is taken for as long as three blocks of a wave (measured with workgroups of four).  It reads all scores twice and lasts the longer the more there are, but the
-// launch depends little on where between two and six the line lies.  (The kernel alone, 32 / 8 heads of 128, 16 of 20 / 479 / 4,096 /
-// 16,384 units, taken for 1, 2, 3, 6 and 9 blocks: 13.2 11.9 12.1 12.2 11.9 / 14.3 12.4 12.3 12.4 12.1 / 15.8 13.2 13.6 13.5 13.4 /
-// 23.2 20.7 20.7 20.6 20.6 us; 64 of 16,384: 36.9 36.1 36.5 36.8 36.1; 36 heads of 64, 15 splits each, 16 of
-// 512: 17.6 16.2 16.4 15.9 21.8.)
-int infllm_decode_lead_splits(int32_t nsplit, int64_t lead_blocks, int64_t blocks) {
+// selection is taken for as long as two blocks of a wave.  It reads all scores twice and lasts the longer the more there are, but with many
+// splits the launch depends little on where between two and nine the line lies; few splits are cut differently.  (The kernel alone, us, taken for
+// 1, 2, 3, 6 and 9 blocks.  32 / 8 heads of 128, 32 splits, 16 of 20 / 479 / 4,096 / 16,000 units: 13.8 11.1 11.2 11.3 11.1 / 13.3 11.6 11.4 11.9
+// 11.8 / 14.0 11.8 12.0 11.8 12.0 / 17.1 14.8 14.8 14.8 14.6; 64 of 4,096: 20.6 20.5 21.0 20.6 20.6.  32 / 32 heads, 8 splits, 16 of 20 / 479:
+// 21.6 21.7 24.8 24.8 30.5 / 22.4 22.5 22.7 25.0 30.3.  36 heads of 64, 14 splits, 16 of 512: 14.9 14.1 14.0 14.0 14.0.)
+extern "C" int infllm_decode_lead_splits(int32_t nsplit, int64_t lead_blocks, int64_t blocks) {
     int best = 1;
     int64_t best_time = INT64_MAX;
     for (int s = 1; s < nsplit; ++s) {
-        const int64_t lead = kDecWaves * s, rest = kDecWaves * (nsplit - s), time = std::max((lead_blocks + lead - 1) / lead + 3, (blocks + rest - 1) / rest);
+        const int64_t lead = kDecWaves * s, rest = kDecWaves * (nsplit - s), time = std::max((lead_blocks + lead - 1) / lead + 2, (blocks + rest - 1) / rest);
         if (time < best_time) best = s, best_time = time;
     }
     return best;

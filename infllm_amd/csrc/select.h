@@ -18,7 +18,7 @@ struct SelectLds {
 // smallest of the groups' largest is a threshold that at least k units reach, and few more do.  Those are ranked against each other
 // by counting.  Where more than fit reach it (equal scores, say) the k-th largest composite is found digit by digit instead.
 // (select_topk_block of retrieve.hip is the same method for one workgroup behind a launch's last score, which fetches the scores once,
-// from where other XCDs stored them, and keeps them in registers; here four waves have neither the registers nor that need.)
+// from where other XCDs stored them, and keeps them in registers; here the kernel has neither the registers nor that need.)
 // ids: the k, best first; a barrier has followed when the function returns.
 template <int THREADS>
 __device__ __forceinline__ void select_units(const float *scores, int N, int k, int32_t *ids, SelectLds<THREADS> &lds) {

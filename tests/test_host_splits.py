@@ -31,6 +31,17 @@ def test_workgroups_that_read_the_same_keys_meet_behind_one_l2(H, Hkv):
         assert splits(B, H, Hkv, 128, 2000, B * Hkv, 0) % 8 == 0, B
 
 
+def test_a_selection_is_two_blocks_of_a_wave():
+    """8 splits of 136 blocks behind a selection and 256 others: the selection and 6 blocks a wave beside 7, not 5 beside 8"""
+    f = _lib.load().infllm_decode_lead_splits
+    f.restype, f.argtypes = C.c_int, [C.c_int32, C.c_int64, C.c_int64]
+    assert f(8, 136, 256) == 3
+    for n in (2, 3, 8, 32, 64):
+        for lead in (1, 136, 100000):
+            for rest in (1, 256, 100000):
+                assert 1 <= f(n, lead, rest) < n
+
+
 def test_bounds():
     for H, Hkv in ((32, 8), (40, 40), (16, 1)):
         for blocks in (0, 1, 7, 8, 9, 64, 100000):
