@@ -148,7 +148,7 @@ def call_lists_entry(dev, n_units=8192, tables=8, queries=15, launches=40):
     idx = torch.empty((queries, k), dtype=torch.int32, device=dev)
     us = _event_time_us(lambda i: ops.score_topk_queries(reps[i % tables], n_units, qbars, k, scores, idx), launches, 2 * tables)
     nbytes = n_units * C * 2 + 2 * queries * n_units * 4
-    return _hbm_entry("unit_scores_queries_kernel<8> + select_rows_kernel<1>",
+    return _hbm_entry("unit_scores_queries_kernel<8> + select_rows_kernel<16>",
                       f"lists of a call: {queries} mean queries over {n_units} x {C} bf16 representatives, top-{k} each, two launches "
                       f"({tables} tables in rotation; the same by one retrieval per block: {queries} x {n_units * C * 2 / 2 ** 20:.0f} MiB)",
                       nbytes, us, launches)
